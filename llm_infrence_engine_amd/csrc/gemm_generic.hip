@@ -1,6 +1,6 @@
 // C[M,N] (+)= A[M,K] . W[N,K]^T (+ bias[N]) with float accumulation on the vector ALUs.
-// This is the true 32-bit matrix product of the float path (no reduced-precision matrix mode) and the
-// any-shape fallback of the bfloat16 path.  Every output element sums its K products in the same
+// The any-shape fallback: bfloat16 sizes that no matrix-core kernel takes, and float operands whose rows do not come in
+// 16-byte pieces (the others go to csrc/gemm_f32.hip).  Every output element sums its K products in the same
 // order whatever M is, so a token's result does not depend on what else is in the batch.
 #include "common.h"
 #include "api.h"
@@ -85,6 +85,13 @@ gemm_generic_kernel(const TA* __restrict__ A, const TA* __restrict__ W, const fl
   }
 }
 
+}  // namespace
+
+int ms_gemm_f32_launch(const float* A, const float* W, const float* bias, float* C, int M, int N, int K, size_t lda,
+                       size_t ldw, size_t ldc, int accumulate, hipStream_t stream);     // csrc/gemm_f32.hip
+
+namespace {
+
 template <typename TA, typename TC>
 int launch(const void* A, const void* W, const float* bias, void* C, int M, int N, int K, size_t lda, size_t ldw,
            size_t ldc, int accumulate, hipStream_t stream) {
@@ -92,6 +99,11 @@ int launch(const void* A, const void* W, const float* bias, void* C, int M, int 
   const size_t vec_bytes = 4 * sizeof(TA);
   const bool vec = (K % 4 == 0) && (lda % 4 == 0) && (ldw % 4 == 0) && ((uintptr_t)A % vec_bytes == 0) &&
                    ((uintptr_t)W % vec_bytes == 0);
+  if constexpr (sizeof(TA) == 4) {
+    if (vec) return ms_gemm_f32_launch((const float*)A, (const float*)W, bias, (float*)C, M, N, K, lda, ldw, ldc, accumulate, stream);
+    gemm_generic_kernel<TA, TC, false><<<grid, block, 0, stream>>>((const TA*)A, (const TA*)W, bias, (TC*)C, M, N, K, lda, ldw, ldc, accumulate);
+    return ms_launch_status();
+  }
   if (vec)
     gemm_generic_kernel<TA, TC, true><<<grid, block, 0, stream>>>((const TA*)A, (const TA*)W, bias, (TC*)C, M, N, K, lda, ldw, ldc, accumulate);
   else

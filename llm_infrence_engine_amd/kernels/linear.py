@@ -1,6 +1,7 @@
 """Matrix products of the model: out = a @ w.T (+ bias).  Picks the kernel by type and shape.
 
-float32          the vector-ALU kernel: a true 32-bit product, whatever the shape.
+float32          a true 32-bit product on the matrix cores' float instruction (rows that do not come in 16-byte
+                 pieces: on the vector ALUs); a row's sums do not depend on how many rows there are.
 bfloat16, few rows (a decode step)   the weight-streaming matrix-core kernel, with the bias, the gated
                  activation or split-K partial sums as its epilogue.
 bfloat16, many rows (prompt portions)  the library's matrix product (hipBLASLt through torch.mm), as the

@@ -454,7 +454,8 @@ def rope_store(qkv: torch.Tensor, num_heads: int, num_kv_heads: int, head_dim: i
 
 def gemm_generic(a: torch.Tensor, w: torch.Tensor, out: torch.Tensor, bias: Optional[torch.Tensor] = None,
                  accumulate: bool = False) -> torch.Tensor:
-    """out (+)= a @ w.T (+ bias), float accumulation on the vector ALUs.  a [M, K] and out [M, N] may be row
+    """out (+)= a @ w.T (+ bias), accumulated in float: 32-bit operands on the matrix cores' float instruction where their rows
+    come in 16-byte pieces, anything else on the vector ALUs.  a [M, K] and out [M, N] may be row
     slices of wider matrices (unit stride in the last dimension)."""
     for t, name in ((a, "a"), (w, "w"), (out, "out")):
         _check(t, name, contiguous=False)

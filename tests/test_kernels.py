@@ -117,6 +117,28 @@ def test_gemm_row_does_not_depend_on_the_batch(ops):
     assert torch.equal(full[40:41], one)
 
 
+@pytest.mark.parametrize("N,K", [(16, 4), (33, 20), (64, 64), (200, 300), (896, 1028), (9728, 896)])
+def test_float_product_in_the_same_order_for_any_number_of_rows(ops, N, K):
+    """Both kernels of the 32-bit product and both of the tiled one's tiles, at the edges of their tiles, as rows of wider
+    matrices: within float rounding of 64 bits, and bit for bit the same row whatever is beside it."""
+    g = torch.Generator().manual_seed(31)
+    M = 700 if N > 9000 else 130
+    a = torch.randn(M, K + 8, generator=g).to(DEV)[:, 4:4 + K]
+    w = (torch.randn(N, K, generator=g) / math.sqrt(K)).to(DEV)
+    bias = torch.randn(N, generator=g).to(DEV)
+    want = a.double() @ w.double().T + bias.double()
+    # a slice is one chain of at most 16 ceil(K / 256) or 64 sums, then come at most 16 slices and the bias
+    chain = max(64, 16 * -(-K // 256)) + 18
+    bound = chain * 2.0 ** -24 * (a.double().abs() @ w.double().abs().T + bias.double().abs())
+    full = torch.empty(M, N, device=DEV)
+    ops.gemm_generic(a, w, full, bias=bias)
+    assert ((full.double() - want).abs() <= bound).all()
+    for lo, hi in ((0, 1), (3, 19), (5, 22), (0, 33), (2, 66), (0, 65), (1, 98), (M - 1, M)):
+        out = torch.empty(hi - lo, N, device=DEV)
+        ops.gemm_generic(a[lo:hi], w, out, bias=bias)
+        assert torch.equal(out, full[lo:hi]), (lo, hi)
+
+
 def rope_reference(x, pos, rot, inv):
     ang = pos.double()[:, None] * inv[None]
     cos, sin = torch.cat((ang, ang), -1).cos()[:, None], torch.cat((ang, ang), -1).sin()[:, None]
@@ -190,12 +212,14 @@ def attention_reference(q, k, v, scale, window=None):
 
 @pytest.mark.parametrize("dtype", DTYPES)
 @pytest.mark.parametrize("nh,nkv,d,page_size,window", [(4, 2, 16, 4, None), (6, 2, 32, 8, None), (5, 1, 48, 16, None),
-                                                        (3, 3, 80, 4, 7), (8, 2, 128, 16, 40)])
+                                                        (3, 3, 80, 4, 7), (8, 2, 128, 16, 40), (2, 1, 18, 4, None),
+                                                        (4, 2, 64, 16, 1100)])
 def test_paged_attention_generic(ops, dtype, nh, nkv, d, page_size, window):
     """Three requests in one batch: a whole prompt, a portion after a cached prefix, one decoded token;
     pages handed out in shuffled order and the pool pre-filled with large values that must never be read."""
     g = torch.Generator().manual_seed(6)
-    ctx = [70, 133, 201]       # keys each request holds after this step
+    # keys each request holds after this step; behind the widest window so many that every wave has several blocks of 64
+    ctx = [70, 513, 1300] if window == 1100 else [70, 133, 201]
     qlen = [70, 9, 1]          # its new tokens
     pages_per = [-(-c // page_size) for c in ctx]
     P = sum(pages_per) + 5
