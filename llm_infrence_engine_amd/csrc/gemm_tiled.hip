@@ -3,13 +3,18 @@
 // interleaved gate/up weight never goes to memory, which saves the write of [M, 2I], its read and a kernel.
 //
 // A block of 8 waves owns a tile of BN features by BM tokens, as large as registers allow (256 x 256: a byte
-// loaded does 128 multiply-adds; a CU draws 100 GB/s and more from its XCD's L2 but 27 GB/s from beyond it, some
-// 40 GB/s in this kernel, where a fifth of the requests miss).  Per step of 64 columns the tile's rows of W
-// and A go from memory straight to LDS (global_load_lds, 16 bytes a lane: no registers, no LDS write
-// instructions) into one of two buffers, a step before they are multiplied.  LDS rows are 128 bytes with their
-// eight 16-byte pieces permuted by the row number (piece c at place c ^ (row & 7)): fragment reads then run at
-// the full LDS rate (measured 237 bytes a clock; rows 144 bytes apart give 116).  A step has one barrier, in
-// its middle, and the matrix pipe has work on both sides of it (see the main loop).
+// loaded does 128 multiply-adds).  Per step of 64 columns the tile's rows of W and A go from memory straight to LDS
+// (global_load_lds, 16 bytes a lane: no registers, no LDS write instructions), A one step and W two steps before they are
+// multiplied; the 256 x 256 tile's three slots for W and two for A are all of the CU's 160 KB.  LDS rows are 128 bytes
+// with their eight 16-byte pieces permuted by the row number (piece c at place c ^ (row & 7)): fragment reads then run at
+// the full LDS rate (measured 237 bytes a clock; rows 144 bytes apart give 116).
+//
+// What bounds it: with all CUs at work the matrix pipes are busy 60 % of the time at 1.8 GHz (8,192 cubed: 1.36
+// PFLOP/s), where the library's kernel has them busy 86 % of the time and the chip then runs at 1.54 GHz (1.57): the power
+// the chip may draw is close.  A step of the 256 x 256 tile takes 1.6 us then, 1.15 us with a third of the CUs at work, and
+// its products 0.85 us at 2.4 GHz.  One barrier a step with everything drained at it, and reads from LDS that the compiler
+// had moved next to their use, took 1.70 and 1.38 us (7B gate/up, 2,048 tokens 525 -> 480 us and 4,096 951 -> 864; 0.5B
+// gate/up, 2,048 tokens 47.3 -> 43.0; 8,192 cubed 877 -> 811).
 //
 // W is the A operand of the MFMA and the tokens the B operand, so a lane ends up with 4 output features of one
 // token per tile.  Which 16 features make up a tile is free: tile i of a wave takes, for q = 0..3, the four
@@ -17,6 +22,7 @@
 // features of its token over its FT tiles and stores them as one run.
 #include "common.h"
 #include "api.h"
+#include <type_traits>
 
 namespace {
 
@@ -74,22 +80,6 @@ __device__ __forceinline__ int feature_of_row(int l) {
   return wf * (FT * 16) + (rr >> 2) * (4 * FT) + i * 4 + (rr & 3);
 }
 
-// The instruction order of a step's first half, told to the scheduler: before the TT products of tile I the reads
-// that the source has there (the next tile of W but for the last, tile I of the second half, token fragment I
-// of the second half while there are any).  0x100: reads from LDS, 0x008: matrix instructions.
-template <int I, int FT, int TT>
-struct FirstHalfOrder {
-  static __device__ __forceinline__ void apply() {
-    __builtin_amdgcn_sched_group_barrier(0x100, (I + 1 < FT ? 1 : 0) + 1 + (I < TT ? 1 : 0), 0);
-    __builtin_amdgcn_sched_group_barrier(0x008, TT, 0);
-    FirstHalfOrder<I + 1, FT, TT>::apply();
-  }
-};
-template <int FT, int TT>
-struct FirstHalfOrder<FT, FT, TT> {
-  static __device__ __forceinline__ void apply() {}
-};
-
 // A lane's run of RUN consecutive results goes to memory in the widest pieces that RUN allows (16 bytes for a
 // multiple of 8 bfloat16, else 8 or 4), when the row starts at such an address.
 template <int RUN>
@@ -127,12 +117,13 @@ gemm_tiled_kernel(const bf16* __restrict__ A, size_t lda, const bf16* __restrict
                   TO* __restrict__ out, size_t ldo, int M, int N, int K, int m_tiles, int n_tiles, int xm, QkvEpilogue qkv,
                   GroupedRows grp) {
   constexpr int NWAVES = WF * WT, THREADS = NWAVES * MS_WAVE;
-  constexpr int BN = WF * FT * 16, BM = WT * TT * 16, ROWS = BN + BM;
-  constexpr int LOADS = (ROWS / 8 + NWAVES - 1) / NWAVES;   // loads of 8 rows (1 KB) a wave makes per step at most
-  static_assert(ROWS % 8 == 0, "a load brings eight rows");
-  static_assert(TT < FT, "the main loop reads the token fragments beside the first TT + 1 tiles of W");
+  constexpr int BN = WF * FT * 16, BM = WT * TT * 16;
+  static_assert(BN % 8 == 0 && BM % 8 == 0, "a load brings eight rows");
+  // loads of 8 rows (1 KB) a wave makes per step at most, of W and of A
+  constexpr int LOADS_W = (BN / 8 + NWAVES - 1) / NWAVES, LOADS_A = (BM / 8 + NWAVES - 1) / NWAVES;
+  constexpr int SLOT_W = BN * PITCH, SLOT_A = BM * PITCH;
   extern __shared__ __align__(16) unsigned char lds_raw[];
-  bf16* lds = reinterpret_cast<bf16*>(lds_raw);          // two buffers of ROWS x PITCH
+  bf16* lds = reinterpret_cast<bf16*>(lds_raw);          // three slots of BN rows of W, two of BM rows of A
 
   // Blocks with consecutive ids go to consecutive XCDs, each with an L2 of its own.  The 8 XCDs are laid over the
   // tiles as xm x (8 / xm): an XCD takes every xm-th token tile and every (8 / xm)-th tile of W, its token tiles
@@ -154,30 +145,36 @@ gemm_tiled_kernel(const bf16* __restrict__ A, size_t lda, const bf16* __restrict
   const int wf = wave % WF, wt = wave / WF;
   const int col = lane & 15, kq = lane >> 4;
 
-  // Load p of a wave fills LDS rows (wave + p * NWAVES) * 8 .. + 7: lane l's 16 bytes land at l * 16 of that 1 KB,
-  // which is place l & 7 of row l >> 3, so the lane asks memory for the piece that belongs there.  Rows past the
+  // Load p of a wave fills LDS rows (wave + p * NWAVES) * 8 .. + 7 of a slot: lane l's 16 bytes land at l * 16 of that
+  // 1 KB, which is place l & 7 of row l >> 3, so the lane asks memory for the piece that belongs there.  Rows past the
   // end of W or A repeat the last row (their results are not stored).
-  const bf16* src[LOADS];
+  const bf16 *src_w[LOADS_W], *src_a[LOADS_A];
 #pragma unroll
-  for (int p = 0; p < LOADS; ++p) {
-    const int l = min((wave + p * NWAVES) * 8 + (lane >> 3), ROWS - 1);   // (past the tile's rows: not loaded)
-    const int piece = (lane & 7) ^ (l & 7);
-    if (l < BN) src[p] = W + (size_t)min(n0 + feature_of_row<FT>(l), N - 1) * ldw + piece * 8;
-    else {
-      int r = min(m0 + l - BN, M - 1);
-      if (EPI == EPI_GROUPED && grp.in_div > 0) r = max(grp.rows[r], 0) / grp.in_div;   // (a row without an item: any row)
-      src[p] = A + (size_t)r * lda + piece * 8;
-    }
+  for (int p = 0; p < LOADS_W; ++p) {
+    const int l = min((wave + p * NWAVES) * 8 + (lane >> 3), BN - 1);   // (past the tile's rows: not loaded)
+    src_w[p] = W + (size_t)min(n0 + feature_of_row<FT>(l), N - 1) * ldw + ((lane & 7) ^ (l & 7)) * 8;
+  }
+#pragma unroll
+  for (int p = 0; p < LOADS_A; ++p) {
+    const int l = min((wave + p * NWAVES) * 8 + (lane >> 3), BM - 1);
+    int r = min(m0 + l, M - 1);
+    if (EPI == EPI_GROUPED && grp.in_div > 0) r = max(grp.rows[r], 0) / grp.in_div;   // (a row without an item: any row)
+    src_a[p] = A + (size_t)r * lda + ((lane & 7) ^ (l & 7)) * 8;
   }
   typedef __attribute__((address_space(3))) void lds_void;
   typedef const __attribute__((address_space(1))) void global_void;
-  auto load_rows = [&](int k, int buffer) {
-#pragma unroll
-    for (int p = 0; p < LOADS; ++p)
-      if ((p + 1) * NWAVES * 8 <= ROWS || (wave + p * NWAVES) * 8 < ROWS)   // the last round may be for some waves only
-        __builtin_amdgcn_global_load_lds((global_void*)(src[p] + k),
-                                         (lds_void*)(lds + buffer + (wave + p * NWAVES) * 8 * PITCH), 16, 0, 0);
+  // the wave's p-th load of a step's rows of W, or of A, into the slot whose first value in LDS is `slot`
+  auto load_w = [&](int p, int step, int slot) {
+    if ((p + 1) * NWAVES * 8 <= BN || (wave + p * NWAVES) * 8 < BN)   // the last round may be for some waves only
+      __builtin_amdgcn_global_load_lds((global_void*)(src_w[p] + step * BK),
+                                       (lds_void*)(lds + slot + (wave + p * NWAVES) * 8 * PITCH), 16, 0, 0);
   };
+  auto load_a = [&](int p, int step, int slot) {
+    if ((p + 1) * NWAVES * 8 <= BM || (wave + p * NWAVES) * 8 < BM)
+      __builtin_amdgcn_global_load_lds((global_void*)(src_a[p] + step * BK),
+                                       (lds_void*)(lds + 3 * SLOT_W + slot + (wave + p * NWAVES) * 8 * PITCH), 16, 0, 0);
+  };
+  constexpr int FEWEST_W = BN / 8 / NWAVES, FEWEST_A = BM / 8 / NWAVES;   // loads every wave makes
 
   f32x4 acc[FT][TT];
 #pragma unroll
@@ -190,50 +187,93 @@ gemm_tiled_kernel(const bf16* __restrict__ A, size_t lda, const bf16* __restrict
   static_assert(BK == 64, "a step is two products of 32 columns deep");
   const int place0 = (kq ^ (col & 7)) * 8, place1 = ((kq + 4) ^ (col & 7)) * 8;
   const bf16* w_frag = lds + (wf * FT * 16 + col) * PITCH;
-  const bf16* a_frag = lds + (BN + wt * TT * 16 + col) * PITCH;
+  const bf16* a_frag = lds + 3 * SLOT_W + (wt * TT * 16 + col) * PITCH;
 
-  // A step has one barrier, in its middle.  First half: the products of the first 32 columns, whose token
-  // fragments are in registers already and whose tiles of W are read one ahead; meanwhile every fragment of the
-  // second 32 columns is read too.  Then nothing of this step is left in its buffer: the wave waits for the rows
-  // of the next step (asked for a step ago), the barrier makes them visible to all and says that all are done
-  // with this buffer, and the rows of the step after next are asked for into it.  Second half: the products of
-  // the second 32 columns from registers, meanwhile the first fragments of the next step are read.  So no read
-  // from LDS and no load from memory is waited for with the matrix pipe idle, except at the barrier itself.
-  const int steps = K / BK;
-  load_rows(0, 0);
-  if (steps > 1) load_rows(BK, ROWS * PITCH);
-  __builtin_amdgcn_s_waitcnt(0x0F70);   // vmcnt(0): the loads to LDS have landed
-  __syncthreads();
-  bf16x8 a0[TT], a1[TT], w1[FT];
+  // A step is four blocks of products, two to each half of its columns; a block's fragments of W (a half's FT lie in a ring
+  // of FT registers) and, before a half, its TT fragments of the tokens are read beside the first products of the block
+  // before it, and waited for at its start only.  The barrier stands before the last block: by then every fragment of the
+  // step is in registers, so the wave waits for its share of the next step's rows, the barrier makes all shares visible and
+  // says that everybody is done with this step's slots, into which go the step after next of A, during the last block, and
+  // the one after that of W, during the next step's first: W, which mostly comes from beyond the L2, has the longer way.
+  // The loads are asked for one by one between the products (eight in a row hold up those behind them).  So no read from
+  // LDS and no load from memory is waited for with the matrix pipe idle.  The order of the instructions is the written one (sched_barrier), and a step is one straight piece
+  // of code: left to itself the compiler moved the reads for the next step behind the branch to it and waited for each on
+  // the spot, and a step took twice the time of its products.
+  constexpr int HALF = (FT + 1) / 2;      // tiles of W in the first block of a half; the second has the others
+  bf16x8 wr[FT], a[2][TT];
+  auto read_w = [&](int half, int i, int slot) {
+    wr[i] = *reinterpret_cast<const bf16x8*>(w_frag + slot + i * 16 * PITCH + (half ? place1 : place0));
+  };
+  auto read_a = [&](int half, int j, int slot) {
+    a[half][j] = *reinterpret_cast<const bf16x8*>(a_frag + slot + j * 16 * PITCH + (half ? place1 : place0));
+  };
+  // mode 2: the step after next is asked for; 1: there is none; 0: the last step, nothing follows
+  auto step = [&](auto mode_c, int s, int slot_w, int next_w, int free_w, int slot_a, int next_a) {
+    constexpr int MODE = decltype(mode_c)::value;
 #pragma unroll
-  for (int j = 0; j < TT; ++j) a0[j] = *reinterpret_cast<const bf16x8*>(a_frag + j * 16 * PITCH + place0);
-  bf16x8 w_next = *reinterpret_cast<const bf16x8*>(w_frag + place0);
-  for (int s = 0; s < steps; ++s) {
-    const int buf = (s & 1) * ROWS * PITCH, other = ((s + 1) & 1) * ROWS * PITCH;
+    for (int block = 0; block < 4; ++block) {
+      const int half = block >> 1, i0 = block & 1 ? HALF : 0, i1 = block & 1 ? FT : HALF;
+      if (MODE > 0 && block == 3) {
+        // (of the loads under way, only those of the step after next of W may still be)
+        if (MODE == 2) asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"(FEWEST_W) : "memory");
+        else asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");
+      }
+      // what the next block needs: tiles r0 .. r1 - 1 of W and, when it begins a half, the tokens' fragments
+      const int r0 = block & 1 ? 0 : HALF, r1 = block & 1 ? HALF : FT, of_a = block & 1 ? TT : 0;
+      const int reads = block == 3 && MODE == 0 ? 0 : r1 - r0 + of_a, spread = i1 - i0 > 2 ? 2 : 1;
 #pragma unroll
-    for (int i = 0; i < FT; ++i) {
-      const bf16x8 w_cur = w_next;
-      if (i + 1 < FT) w_next = *reinterpret_cast<const bf16x8*>(w_frag + buf + (i + 1) * 16 * PITCH + place0);
-      w1[i] = *reinterpret_cast<const bf16x8*>(w_frag + buf + i * 16 * PITCH + place1);
-      if (i < TT) a1[i] = *reinterpret_cast<const bf16x8*>(a_frag + buf + i * 16 * PITCH + place1);
+      for (int i = i0; i < i1; ++i) {
 #pragma unroll
-      for (int j = 0; j < TT; ++j) acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(w_cur, a0[j], acc[i][j], 0, 0, 0);
+        for (int r = 0; r < reads; ++r) {
+          if (r * spread / reads != i - i0) continue;
+          const int to = block == 1 ? 1 : block == 3 ? 0 : half;
+          if (r < of_a) read_a(to, r, block == 3 ? next_a : slot_a);
+          else read_w(to, r0 + r - of_a, block == 3 ? next_w : slot_w);
+        }
+#pragma unroll
+        for (int j = 0; j < TT; ++j)
+          acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wr[i], a[half][j], acc[i][j], 0, 0, 0);
+        if (MODE == 2 && block == 0) {
+#pragma unroll
+          for (int p = 0; p < LOADS_W; ++p) if (p * (i1 - i0) / LOADS_W == i - i0) load_w(p, s + 2, free_w);
+        }
+        if (MODE == 2 && block == 3) {
+#pragma unroll
+          for (int p = 0; p < LOADS_A; ++p) if (p * (i1 - i0) / LOADS_A == i - i0) load_a(p, s + 2, slot_a);
+        }
+        __builtin_amdgcn_sched_barrier(0);
+      }
     }
-    // the order of the instructions (left to itself the compiler reads a fragment right before its products and
-    // waits for it): the reads written before each group of TT products stay there
-    FirstHalfOrder<0, FT, TT>::apply();
-    __builtin_amdgcn_s_waitcnt(0x0070);   // vmcnt(0) and lgkmcnt(0): the next step's rows have landed, this step's are read
-    __syncthreads();
-    if (s + 2 < steps) load_rows((s + 2) * BK, buf);
-    // (after the last step these reads bring what nobody uses)
+  };
+  const int steps = K / BK;
 #pragma unroll
-    for (int i = 0; i < FT; ++i) {
-      if (i < TT) a0[i] = *reinterpret_cast<const bf16x8*>(a_frag + other + i * 16 * PITCH + place0);
-      if (i == TT) w_next = *reinterpret_cast<const bf16x8*>(w_frag + other + place0);
+  for (int first = 0; first < 2; ++first) {
+    if (first < steps) {
 #pragma unroll
-      for (int j = 0; j < TT; ++j) acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(w1[i], a1[j], acc[i][j], 0, 0, 0);
+      for (int p = 0; p < LOADS_W; ++p) load_w(p, first, first * SLOT_W);
+#pragma unroll
+      for (int p = 0; p < LOADS_A; ++p) load_a(p, first, first * SLOT_A);
     }
   }
+  if (steps > 1) asm volatile("s_waitcnt vmcnt(%0)\n\ts_barrier" ::"n"(FEWEST_W + FEWEST_A) : "memory");
+  else asm volatile("s_waitcnt vmcnt(0)\n\ts_barrier" ::: "memory");
+#pragma unroll
+  for (int j = 0; j < TT; ++j) read_a(0, j, 0);
+#pragma unroll
+  for (int i = 0; i < HALF; ++i) read_w(0, i, 0);
+  int sw = 0, sa = 0;      // the current step's slots
+  auto after_w = [&](int slot) { return slot == 2 * SLOT_W ? 0 : slot + SLOT_W; };
+  for (int s = 0; s + 2 < steps; ++s) {
+    step(std::integral_constant<int, 2>{}, s, sw, after_w(sw), after_w(after_w(sw)), sa, SLOT_A - sa);
+    sw = after_w(sw);
+    sa = SLOT_A - sa;
+  }
+  if (steps > 1) {
+    step(std::integral_constant<int, 1>{}, 0, sw, after_w(sw), 0, sa, SLOT_A - sa);
+    sw = after_w(sw);
+    sa = SLOT_A - sa;
+  }
+  step(std::integral_constant<int, 0>{}, 0, sw, 0, 0, sa, 0);
 
   // the lane's run of 4 FT features of token m (tile j): acc[i][j][r] is feature f0 + i * 4 + r
   const int f0 = n0 + wf * (FT * 16) + kq * (4 * FT);
@@ -357,7 +397,7 @@ template <int WF, int WT, int FT, int TT, int EPI, typename TO>
 int launch(const bf16* A, size_t lda, const bf16* W, size_t ldw, TO* out, size_t ldo, int M, int N, int K,
            hipStream_t stream, const QkvEpilogue& qkv = QkvEpilogue{}, const GroupedRows& grp = GroupedRows{}) {
   constexpr int BN = WF * FT * 16, BM = WT * TT * 16;
-  constexpr size_t lds = 2 * (size_t)(BN + BM) * PITCH * sizeof(bf16);
+  constexpr size_t lds = (size_t)(3 * BN + 2 * BM) * PITCH * sizeof(bf16);
   static bool raised = false;   // once per instantiation: allow more dynamic LDS than the default 64 KB
   if (!raised) {
     if (hipFuncSetAttribute(reinterpret_cast<const void*>(&gemm_tiled_kernel<WF, WT, FT, TT, EPI, TO>),
@@ -383,7 +423,7 @@ int launch_grouped(const bf16* A, size_t lda, const bf16* W, TO* out, size_t ldo
                    const GroupedRows& grp, hipStream_t stream) {
   constexpr int WF = 2, WT = 4, FT = 8;
   constexpr int BN = WF * FT * 16, BM = WT * TT * 16;
-  constexpr size_t lds = 2 * (size_t)(BN + BM) * PITCH * sizeof(bf16);
+  constexpr size_t lds = (size_t)(3 * BN + 2 * BM) * PITCH * sizeof(bf16);
   static bool raised = false;
   if (!raised) {
     if (hipFuncSetAttribute(reinterpret_cast<const void*>(&gemm_tiled_kernel<WF, WT, FT, TT, EPI_GROUPED, TO>),
@@ -402,13 +442,12 @@ int launch_grouped(const bf16* A, size_t lda, const bf16* W, TO* out, size_t ldo
 int g_tile = 0;   // measurements: 0 leaves the choice of tile; 1 to 5 force one (256, 128, 64, 192, 160 features wide)
 
 // The tile that takes the least time by a model of the measurements.  A block of 256 tokens by 256, 192 or 160
-// features has a CU to itself; its time is what the CU needs to draw its rows (some 40 GB/s whatever the tile), so
-// a step of 64 columns takes 1.70, 1.44 or 1.32 us, a tile 3 us more for its start and end, and the tiles run in
-// whole rounds over the CUs: the narrower tiles pay where they fill the rounds better (2,048 tokens of the 0.5B
-// gate/up shape: 304 tiles of 256 features take two rounds, 51.7 us; 488 of 160 take two shorter ones, 45.0;
-// 1,024 tokens: 28.2 -> 22.6 in one round).  Tiles of 128 x 128 go two to a CU, 1.26 us a step each; they end at
-// different times, so their rounds are counted as they come, plus 0.3 for the last.  Within 5 % of the measured
-// times at 256 to 4,096 tokens of the 0.5B and 1.5B gate/up shapes.
+// features has a CU to itself; a step of 64 columns takes 1.6, 1.3 or 1.3 us with all CUs at work, a tile 3 us more for
+// its start and end, and the tiles run in whole rounds over the CUs: the narrower tiles pay where they fill the rounds
+// better (2,048 tokens of the 0.5B gate/up shape: 304 tiles of 256 features take two rounds, 48.6 us; 408 of 192 two
+// shorter ones, 43.0; 1,024 tokens: 25.0 -> 21.9 in one round).  Tiles of 128 x 128 go two to a CU, 1.15 us a step each;
+// they end at different times, so their rounds are counted as they come, plus 0.3 for the last.  Within a tenth of the
+// measured times at 1,024 to 4,096 tokens of the 0.5B and 7B gate/up shapes.
 struct TileChoice { int tile; double us; long long tiles, slots; };
 
 TileChoice choose_tile(int M, int N, int K) {
@@ -417,13 +456,14 @@ TileChoice choose_tile(int M, int N, int K) {
   const long long small = (long long)((N + 127) / 128) * ((M + 127) / 128);
   // fewer tiles of 128 x 128 than CUs: tiles of 64 x 64 (four waves) put four times as many CUs to work, and a
   // tile's time is the time its CU needs to draw its rows (q/k/v of the 0.5B shape, 512 tokens: 11.3 -> 8.7 us;
-  // gate/up at 128 tokens 16.6 -> 12.9, at 256 tokens 16.0 -> 14.9; from 512 tokens on 20.4 against 25.5)
+  // gate/up at 128 tokens 16.6 -> 12.9, at 256 tokens 16.0 -> 14.9; from 512 tokens on 20.4 against 25.5, all measured
+  // with two buffers)
   if (small < cus) {
     const long long tiny = (long long)((N + 63) / 64) * ((M + 63) / 64);
     return {3, 0.0, tiny, (tiny + 5 * cus - 1) / (5 * cus) * 5 * cus};
   }
-  TileChoice best{2, ((double)small / (double)(2 * cus) + 0.3) * 1.26 * steps, small, (small + 2 * cus - 1) / (2 * cus) * 2 * cus};
-  const struct { int tile, features; double step_us; } wide[] = {{1, 256, 1.70}, {4, 192, 1.44}, {5, 160, 1.32}};
+  TileChoice best{2, ((double)small / (double)(2 * cus) + 0.3) * 1.15 * steps, small, (small + 2 * cus - 1) / (2 * cus) * 2 * cus};
+  const struct { int tile, features; double step_us; } wide[] = {{1, 256, 1.60}, {4, 192, 1.30}, {5, 160, 1.30}};
   for (const auto& w : wide) {
     const long long tiles = (long long)((N + w.features - 1) / w.features) * ((M + 255) / 256);
     const long long rounds = (tiles + cus - 1) / cus;
