@@ -27,7 +27,7 @@
 // requests, surplus tiles leave at once; a decode-only batch is the case of one tile per request) and
 // split (every request has one token and a long context: the keys are also split over several blocks which
 // write unnormalised partial results, and a second kernel combines them).
-#include "common.h"
+#include "attention_tiles.h"
 #include "api.h"
 #include <algorithm>
 
@@ -37,13 +37,9 @@ typedef __attribute__((ext_vector_type(8))) __bf16 bf16x8;
 typedef __attribute__((ext_vector_type(4))) __bf16 bf16x4;
 typedef __attribute__((ext_vector_type(4))) float f32x4;
 
-__device__ __forceinline__ float fast_exp2(float x) { return __builtin_amdgcn_exp2f(x); }
-
 __device__ __forceinline__ float fast_sigmoid(float x) {
   return __builtin_amdgcn_rcpf(1.0f + fast_exp2(-1.4426950408889634f * x));
 }
-
-constexpr float REF_SLACK = 8.0f;   // log2 units by which a column's maximum may run ahead of its reference
 
 template <int D>
 struct KeyBlock {          // one block of 32 keys as this lane sees it
@@ -184,10 +180,7 @@ attention_mfma_kernel(const bf16* __restrict__ q, size_t q_stride, const bf16* _
   const int bx = SPLIT ? blockIdx.x : blockIdx.z;
   const int rep = nh / nkv;
   const PageGeom pg = {page_size, page_shift};
-  // Which request, and which of its tiles.  A request owns ceil(columns / tile width) tiles, requests in order,
-  // so the launch needs to know only how many tokens and requests a step has, not how the tokens are dealt out
-  // (a captured graph serves every mix).  The waves of a block find their place alike: a lane per request
-  // works out its tiles, a prefix sum over the wave and a vote say where this block's tile falls.
+  // which request, and which of its tiles
   int r, rank, n_tiles;
   if (SPLIT) {
     r = blockIdx.z; rank = 0; n_tiles = 1;
@@ -198,33 +191,8 @@ attention_mfma_kernel(const bf16* __restrict__ q, size_t q_stride, const bf16* _
     n_tiles = ((q_start[1] - q_start[0]) * rep + 16 * NT - 1) / (16 * NT);
     if (rank >= n_tiles) return;
   } else {
-    const int flat = blockIdx.y;
-    int before = 0;
-    r = -1; rank = 0; n_tiles = 0;
-    for (int base = 0; base < n_splits; base += MS_WAVE) {
-      const int i = base + lane;
-      int mine = 0;
-      if (i < n_splits) mine = ((q_start[i + 1] - q_start[i]) * rep + 16 * NT - 1) / (16 * NT);
-      int upto = mine;   // tiles of the requests base..i
-#pragma unroll
-      for (int o = 1; o < MS_WAVE; o <<= 1) {
-        const int v = __shfl_up(upto, o, MS_WAVE);
-        if (lane >= o) upto += v;
-      }
-      const unsigned long long hit = __builtin_amdgcn_ballot_w64(flat < before + upto);
-      if (hit) {
-        const int first = __builtin_ctzll(hit);
-        r = base + first;
-        n_tiles = __shfl(mine, first, MS_WAVE);
-        rank = flat - before - (__shfl(upto, first, MS_WAVE) - n_tiles);
-        break;
-      }
-      before += __shfl(upto, MS_WAVE - 1, MS_WAVE);
-    }
-    if (r < 0) return;   // the grid has room for a partial tile of every request; this block is surplus
-    r = __builtin_amdgcn_readfirstlane(r);
-    rank = __builtin_amdgcn_readfirstlane(rank);
-    n_tiles = __builtin_amdgcn_readfirstlane(n_tiles);
+    find_tile(q_start, n_splits, rep, 16 * NT, blockIdx.y, lane, r, rank, n_tiles);
+    if (r < 0) return;
   }
   const int row = table_rows ? table_rows[r] : r;
   const int* table = block_table + (size_t)row * table_stride;
@@ -412,8 +380,8 @@ attention_mfma_kernel(const bf16* __restrict__ q, size_t q_stride, const bf16* _
     bf16x8 p[NT];
     float m_safe[NT];
     if constexpr (EXTRA != BOUNDED) {
-      float corr[NT], bmax[NT];
-      bool moved = false;
+      float bmax[NT];
+      bool ahead = false;      // some score of this lane's runs ahead of its column's reference
       // the block's maxima of the raw scores (the scale is positive, so they are the maxima of the scaled ones
       // too); one branch for the whole tile, so that what follows is straight-line code for all its columns
       if (unmasked) {
@@ -443,31 +411,32 @@ attention_mfma_kernel(const bf16* __restrict__ q, size_t q_stride, const bf16* _
           bmax[t] = bm;
         }
       }
+      // m is the reference that the exponents are taken against, not necessarily the maximum: it follows the
+      // maximum only when that has run ahead by more than REF_SLACK (a factor 2^REF_SLACK in the terms, far
+      // inside float's range), so that the accumulators are rescaled rarely.  Any reference gives the same
+      // softmax; all lanes of a column decide alike because the block's maximum is the same in all of them.  Whether any
+      // reference has to move is seen from each lane's own scores: the exchanges between the lanes of a column, eight
+      // trips to LDS one after the other, are made only then.
 #pragma unroll
-      for (int t = 0; t < NT; ++t) {
-        float bm = bmax[t];
-        bm = fmaxf(bm, __shfl_xor(bm, 16, MS_WAVE));
-        bm = fmaxf(bm, __shfl_xor(bm, 32, MS_WAVE));
-        bm *= sl2;
-        // m is the reference that the exponents are taken against, not necessarily the maximum: it follows the
-        // maximum only when that has run ahead by more than REF_SLACK (a factor 2^REF_SLACK in the terms, far
-        // inside float's range), so that the accumulators are rescaled rarely.  Any reference gives the same
-        // softmax; all lanes of a column decide alike because bm is the same in all of them.
-        const bool step = bm > m[t] + REF_SLACK;
-        const float m_new = step ? bm : m[t];
-        corr[t] = step ? fast_exp2(m[t] - m_new) : 1.0f;   // m = -inf: 0
-        moved |= step;
-        m[t] = m_new;
-        m_safe[t] = m_new == -INFINITY ? 0.f : m_new;
-      }
-      if (NT == 1 || __builtin_amdgcn_ballot_w64(moved) != 0) {   // the same branch for the whole wave
+      for (int t = 0; t < NT; ++t) ahead |= bmax[t] * sl2 > m[t] + REF_SLACK;
+      if (__builtin_amdgcn_ballot_w64(ahead) != 0) {   // the same branch for the whole wave
 #pragma unroll
         for (int t = 0; t < NT; ++t) {
-          if (SUMS_BY_MATRIX) lsum[t] *= corr[t]; else lvec[t] *= corr[t];
+          float bm = bmax[t];
+          bm = fmaxf(bm, __shfl_xor(bm, 16, MS_WAVE));
+          bm = fmaxf(bm, __shfl_xor(bm, 32, MS_WAVE));
+          bm *= sl2;
+          const bool step = bm > m[t] + REF_SLACK;
+          const float m_new = step ? bm : m[t];
+          const float corr = step ? fast_exp2(m[t] - m_new) : 1.0f;   // m = -inf: 0
+          m[t] = m_new;
+          if (SUMS_BY_MATRIX) lsum[t] *= corr; else lvec[t] *= corr;
 #pragma unroll
-          for (int c = 0; c < CT; ++c) o[c][t] *= corr[t];
+          for (int c = 0; c < CT; ++c) o[c][t] *= corr;
         }
       }
+#pragma unroll
+      for (int t = 0; t < NT; ++t) m_safe[t] = m[t] == -INFINITY ? 0.f : m[t];
     }
     // column by column, so that the products of one column run on the matrix cores while the next column's
     // exponentials are taken

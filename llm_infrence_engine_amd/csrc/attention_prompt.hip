@@ -1,0 +1,377 @@
+// Paged causal attention of prompt portions on the matrix cores (v_mfma_f32_16x16x32_bf16), bfloat16 in, float softmax:
+// the columns, score and value products and the lazily moving reference of csrc/attention_mfma.hip, with the keys and
+// values staged in LDS.
+//
+// Why: a wave of the unstaged kernel draws 16 KB for 32 keys of 128 dims and does 0.2 us of products with them, and eight
+// waves on a CU ask for more than the 45 bytes a clock that a CU gets from its L2 (320 to 400 TFLOP/s at 128 dims).  Here
+// the four waves of a block own neighbouring tiles of 32 columns and walk the same keys, 64 at a time: those go from the
+// pages straight to LDS (global_load_lds), a tile of keys ahead of their use, and every wave reads all of them there.  Two
+// blocks share a CU (64 KB of LDS each), one barrier a tile.  What is left is the softmax on the vector pipe (16
+// exponentials of 16 clocks per 32 x 32 scores) beside the products: 930 TFLOP/s at 4,096 tokens of 28 heads of 128 dims,
+// 1,020 behind 4,096 more, where the unstaged kernel has 380 and 400.
+//
+// A unit is 32 keys.  Row r of the u-th score product of a unit is its key 8 (r / 4) + 4 u + r % 4, so that a lane (quarter
+// kq) has the scores of the eight consecutive keys 8 kq .. + 7, which it needs as one 16-byte read of a value's row.
+// LDS: keys in rows of D, their 16-byte pieces permuted so that the 16 rows of a product meet every bank once (piece p of
+// key k at place p ^ f(k)); values as they lie in a page of 16, [dim][16 keys], the two halves of a row swapped for every
+// other eight dims.
+#include "attention_tiles.h"
+#include "api.h"
+#include <algorithm>
+
+namespace {
+
+typedef __attribute__((ext_vector_type(8))) __bf16 bf16x8;
+typedef __attribute__((ext_vector_type(4))) __bf16 bf16x4;
+typedef __attribute__((ext_vector_type(4))) float f32x4;
+typedef __attribute__((address_space(3))) void lds_void;
+typedef const __attribute__((address_space(1))) void global_void;
+
+constexpr int GROUP = 4;              // waves that walk the same keys
+constexpr int NT = 2;                 // tiles of 16 columns a wave
+constexpr int COLS = GROUP * NT * 16; // columns a block
+constexpr int KEYS = 64;              // keys a tile: one chunk of 16 for every wave to bring
+
+template <int D> __device__ __forceinline__ int permute(int key) {     // f of a key's number in its unit
+  return D == 128 ? (key & 3) | ((key >> 1) & 12) : ((key >> 1) & 1) | ((key >> 2) & 6);
+}
+
+// KG groups of waves own the same columns and take the tiles of keys in turn, each with its own place in LDS; at the end
+// they merge what they have, each for its share of the dims.
+template <int D, int KG>
+__global__ void __launch_bounds__(KG * GROUP * MS_WAVE, 2 * KG)
+attention_prompt_kernel(const bf16* __restrict__ q, size_t q_stride, const bf16* __restrict__ k_pages,
+                        const bf16* __restrict__ vt_pages, const int* __restrict__ block_table, int table_stride,
+                        const int* __restrict__ table_rows, const int* __restrict__ q_start,
+                        const int* __restrict__ context_lens, bf16* __restrict__ out, size_t out_stride, int nh, int nkv,
+                        int page_size, float scale_log2e, int window, int n_requests, int pair_order) {
+  constexpr int CT = D / 16, PIECES = D / 8;
+  constexpr int CHUNK = 16 * D;                       // values of a chunk of 16 keys, of keys as of values
+  constexpr int STAGE = 2 * 4 * CHUNK;                // a tile: four chunks of keys, four of values
+  constexpr int LOADS = CHUNK * 2 / 1024;             // wave loads of 1 KB a chunk
+  extern __shared__ __align__(16) unsigned char lds_raw[];
+  bf16* lds = reinterpret_cast<bf16*>(lds_raw);       // [KG][2 tiles][STAGE]
+  static_assert(CT % KG == 0, "the groups share the dims out");
+  const int lane = threadIdx.x & (MS_WAVE - 1);
+  const int kg = __builtin_amdgcn_readfirstlane(threadIdx.x / (GROUP * MS_WAVE));
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / MS_WAVE) - kg * GROUP;   // in its group
+  const int col16 = lane & 15, kq = lane >> 4;
+  const int g = blockIdx.x, rep = nh / nkv;
+
+  int r, rank, n_tiles;
+  find_tile(q_start, n_requests, rep, COLS, blockIdx.y, lane, r, rank, n_tiles);
+  if (r < 0) return;
+  const int* table = block_table + (size_t)(table_rows ? table_rows[r] : r) * table_stride;
+  const int q0 = q_start[r], qlen = q_start[r + 1] - q0, start_pos = context_lens[r] - qlen, ncols = qlen * rep;
+  // Late tiles see the most keys: they go first, and where all blocks fit on the chip at once the later half goes first,
+  // latest tile first, then the earlier half, earliest first, so that a long tile's companion on its CU is a short one.
+  const int half = pair_order ? (n_tiles + 1) / 2 : n_tiles;
+  const int tile = rank < half ? n_tiles - 1 - rank : rank - half;
+  const int b0 = tile * COLS, c0 = b0 + wave * NT * 16;       // first column of the block, of the wave
+  const int key_hi = start_pos + (min(ncols, b0 + COLS) - 1) / rep;
+  const int key_lo = window > 0 ? max(0, start_pos + b0 / rep - window + 1) : 0;
+  const int t_begin = key_lo / KEYS, t_end = key_hi / KEYS + 1;
+  // the wave's own columns; without any it still brings its chunks
+  const bool works = c0 < ncols;
+  const int first_pos = start_pos + min(c0, ncols - 1) / rep, last_pos = start_pos + (min(ncols, c0 + NT * 16) - 1) / rep;
+  const bool full = c0 + NT * 16 <= ncols;
+
+  // ---- bringing a tile: the wave's chunk of keys and of values
+  const int k_lane = lane * 8;                                 // this lane's first value in a load's 1 KB
+  int k_src[LOADS], v_src[LOADS];                              // what it asks for, from the chunk's first value in the page
+#pragma unroll
+  for (int j = 0; j < LOADS; ++j) {
+    const int at = j * 512 + k_lane, key = at / D, place = (at % D) / 8;
+    k_src[j] = key * D + (place ^ permute<D>((wave & 1) * 16 + key)) * 8;
+    const int dim = at / 16, vh = (at >> 3) & 1;
+    v_src[j] = dim * page_size + (vh ^ ((dim >> 3) & 1)) * 8;
+  }
+  auto page_of = [&](int t) {        // the page of the wave's chunk of tile t; past the context: the null page
+    const int key = t * KEYS + wave * 16;
+    return key <= key_hi ? __builtin_amdgcn_readfirstlane(table[key / page_size]) : 0;
+  };
+  auto bring = [&](int t, int page, int stage) {
+    const int off = (t * KEYS + wave * 16) % page_size;
+    const size_t head = ((size_t)page * nkv + g) * page_size * D;
+    const bf16* kp = k_pages + head + (size_t)off * D;
+    const bf16* vp = vt_pages + head + off;
+    bf16* to = lds + (kg * 2 + stage) * STAGE + wave * CHUNK;
+#pragma unroll
+    for (int j = 0; j < LOADS; ++j) __builtin_amdgcn_global_load_lds((global_void*)(kp + k_src[j]), (lds_void*)(to + j * 512), 16, 0, 0);
+#pragma unroll
+    for (int j = 0; j < LOADS; ++j) __builtin_amdgcn_global_load_lds((global_void*)(vp + v_src[j]), (lds_void*)(to + 4 * CHUNK + j * 512), 16, 0, 0);
+  };
+  if (t_begin + kg < t_end) bring(t_begin + kg, page_of(t_begin + kg), 0);
+  int page_next = t_begin + kg + KG < t_end ? page_of(t_begin + kg + KG) : 0;
+
+  // ---- this lane's columns
+  int pos[NT];      // -1: an idle column (sees no key; its result is not written)
+  bf16x8 qv[NT][D / 32];
+#pragma unroll
+  for (int t = 0; t < NT; ++t) {
+    const int c = c0 + t * 16 + col16, cc = min(c, ncols - 1);
+    pos[t] = c < ncols ? start_pos + cc / rep : -1;
+    const bf16* qp = q + (size_t)(q0 + cc / rep) * q_stride + (size_t)(g * rep + cc % rep) * D + kq * 8;
+#pragma unroll
+    for (int s = 0; s < D / 32; ++s) qv[t][s] = *reinterpret_cast<const bf16x8*>(qp + s * 32);
+  }
+  // The sums of the exponentials: at 128 dims one more product, of P^T with ones (the matrix pipe has the time there), at 64
+  // added up in float on the vector pipe, a lane's share at a time, as the other kernel's tile at either size has them.
+  constexpr bool SUMS_BY_MATRIX = D == 128;
+  float m[NT], lvec[NT] = {};
+  f32x4 o[CT][NT] = {}, lsum[SUMS_BY_MATRIX ? NT : 1] = {};
+#pragma unroll
+  for (int t = 0; t < NT; ++t) m[t] = -INFINITY;
+  bf16x8 ones;
+#pragma unroll
+  for (int i = 0; i < 8; ++i) ones[i] = (__bf16)1.0f;
+
+  // where a lane's fragments lie: key rows of the u-th product of a unit, value rows of 16 dims
+  int k_row[2], k_perm[2];
+#pragma unroll
+  for (int u = 0; u < 2; ++u) {
+    const int key = (col16 >> 2) * 8 + u * 4 + (col16 & 3);
+    k_row[u] = (key >> 4) * CHUNK + (key & 15) * D;
+    k_perm[u] = permute<D>(key);
+  }
+  const int v_row = 4 * CHUNK + (kq >> 1) * CHUNK + col16 * 16 + (((kq & 1) ^ (col16 >> 3)) * 8);
+
+  // the queries have arrived (said here, where the compiler sees it: otherwise it waits for them, and with them for the
+  // loads to LDS, before the first product of every turn)
+  __builtin_amdgcn_s_waitcnt(0x0F70);
+  const int turns = (t_end - t_begin + KG - 1) / KG;
+  for (int turn = 0; turn < turns; ++turn) {
+    const int t = t_begin + turn * KG + kg, stage = turn & 1;
+    asm volatile("s_waitcnt vmcnt(0)\n\ts_barrier" ::: "memory");   // this tile has landed; nobody reads the one before it
+    if (t + KG < t_end) {
+      bring(t + KG, page_next, stage ^ 1);
+      page_next = t + 2 * KG < t_end ? page_of(t + 2 * KG) : 0;
+    }
+    if (!works || t >= t_end) continue;      // the same for the whole wave
+    // two units at a time, or one where the registers (128 a lane with two groups) hold no more scores
+    constexpr int UNITS = KG == 1 ? 2 : 1, SPAN = UNITS * 32;
+#pragma unroll
+    for (int unit = 0; unit < 2; unit += UNITS) {
+      const int base = t * KEYS + unit * 32;
+      if (base > last_pos) break;
+      const bf16* st = lds + (kg * 2 + stage) * STAGE + unit * 2 * CHUNK;
+
+      // scores: s[n][u][t] holds keys base + n*32 + kq*8 + u*4 + (0..3) of column t*16 + col16
+      f32x4 s[UNITS][2][NT];
+#pragma unroll
+      for (int n = 0; n < UNITS; ++n)
+#pragma unroll
+        for (int u = 0; u < 2; ++u) {
+#pragma unroll
+          for (int t2 = 0; t2 < NT; ++t2) s[n][u][t2] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+          for (int ks = 0; ks < D / 32; ++ks) {
+            const bf16x8 kf = *reinterpret_cast<const bf16x8*>(st + n * 2 * CHUNK + k_row[u] + (((ks * 4 + kq) ^ k_perm[u]) & (PIECES - 1)) * 8);
+#pragma unroll
+            for (int t2 = 0; t2 < NT; ++t2) s[n][u][t2] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(kf, qv[t2][ks], s[n][u][t2], 0, 0, 0);
+          }
+        }
+
+      const bool unmasked = full && base + SPAN - 1 <= first_pos && (window <= 0 || base > last_pos - window);
+      if (!unmasked) {
+#pragma unroll
+        for (int n = 0; n < UNITS; ++n)
+#pragma unroll
+          for (int u = 0; u < 2; ++u)
+#pragma unroll
+            for (int t2 = 0; t2 < NT; ++t2)
+#pragma unroll
+              for (int i = 0; i < 4; ++i) {
+                const int key = base + n * 32 + kq * 8 + u * 4 + i;
+                if (key > pos[t2] || (window > 0 && key <= pos[t2] - window)) s[n][u][t2][i] = -INFINITY;
+              }
+      }
+      float bmax[NT];
+      bool ahead = false;
+#pragma unroll
+      for (int t2 = 0; t2 < NT; ++t2) {
+        float bm = -INFINITY;
+#pragma unroll
+        for (int n = 0; n < UNITS; ++n)
+#pragma unroll
+          for (int u = 0; u < 2; ++u)
+#pragma unroll
+            for (int i = 0; i < 4; ++i) bm = fmaxf(bm, s[n][u][t2][i]);
+        bmax[t2] = bm;
+        ahead |= bm * scale_log2e > m[t2] + REF_SLACK;
+      }
+      if (__builtin_amdgcn_ballot_w64(ahead) != 0) {      // some column's reference moves: rare
+#pragma unroll
+        for (int t2 = 0; t2 < NT; ++t2) {
+          float bm = bmax[t2];
+          bm = fmaxf(bm, __shfl_xor(bm, 16, MS_WAVE));
+          bm = fmaxf(bm, __shfl_xor(bm, 32, MS_WAVE));
+          bm *= scale_log2e;
+          const bool step = bm > m[t2] + REF_SLACK;
+          const float corr = step ? fast_exp2(m[t2] - bm) : 1.0f;      // m = -inf: 0
+          if (step) m[t2] = bm;
+          if (SUMS_BY_MATRIX) lsum[t2] *= corr; else lvec[t2] *= corr;
+#pragma unroll
+          for (int c = 0; c < CT; ++c) o[c][t2] *= corr;
+        }
+      }
+      float ref[NT];
+#pragma unroll
+      for (int t2 = 0; t2 < NT; ++t2) ref[t2] = m[t2] == -INFINITY ? 0.f : m[t2];
+      // values past the wave's last visible key may be anything a reused page still holds: they count as zeros
+      const bool clean = base + SPAN - 1 <= last_pos;
+#pragma unroll
+      for (int n = 0; n < UNITS; ++n) {
+        bf16x8 p[NT];
+#pragma unroll
+        for (int t2 = 0; t2 < NT; ++t2) {
+#pragma unroll
+          for (int u = 0; u < 2; ++u)
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+              const float e = fast_exp2(fmaf(s[n][u][t2][i], scale_log2e, -ref[t2]));
+              if (!SUMS_BY_MATRIX) lvec[t2] += e;
+              p[t2][u * 4 + i] = (__bf16)e;
+            }
+          if (SUMS_BY_MATRIX) lsum[t2] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ones, p[t2], lsum[t2], 0, 0, 0);
+        }
+#pragma unroll
+        for (int c4 = 0; c4 < CT; c4 += 4) {
+          bf16x8 v[4];
+#pragma unroll
+          for (int c = 0; c < 4; ++c) v[c] = *reinterpret_cast<const bf16x8*>(st + n * 2 * CHUNK + v_row + (c4 + c) * 256);
+          if (!clean) {
+#pragma unroll
+            for (int i = 0; i < 8; ++i)
+              if (base + n * 32 + kq * 8 + i > last_pos) {
+#pragma unroll
+                for (int c = 0; c < 4; ++c) v[c][i] = (__bf16)0.0f;
+              }
+          }
+#pragma unroll
+          for (int c = 0; c < 4; ++c)
+#pragma unroll
+            for (int t2 = 0; t2 < NT; ++t2) o[c4 + c][t2] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(v[c], p[t2], o[c4 + c][t2], 0, 0, 0);
+        }
+      }
+    }
+  }
+
+  constexpr int OWN = CT / KG;
+  float l[NT];
+#pragma unroll
+  for (int t = 0; t < NT; ++t) {
+    if (SUMS_BY_MATRIX) {
+      l[t] = lsum[t][0];      // every row of the product of ones is the column's sum
+    } else {                  // a column's sum is spread over the four lane groups
+      l[t] = lvec[t] + __shfl_xor(lvec[t], 16, MS_WAVE);
+      l[t] += __shfl_xor(l[t], 32, MS_WAVE);
+    }
+  }
+  if constexpr (KG > 1) {
+    __shared__ float sm_m[KG][COLS], sm_l[KG][COLS];
+    f32x4* sm_o = reinterpret_cast<f32x4*>(lds);        // [group of the sums][wave][dims' tile of the other group][NT][64]
+    static_assert(KG == 2 && (size_t)KG * GROUP * OWN * NT * MS_WAVE * 16 <= (size_t)KG * 2 * STAGE * 2, "the other group's share fits");
+    __syncthreads();                                    // nobody reads keys or values any more
+#pragma unroll
+    for (int t = 0; t < NT; ++t) {
+      const int c = (wave * NT + t) * 16 + col16;
+      if (kq == 0) { sm_m[kg][c] = m[t]; sm_l[kg][c] = l[t]; }
+#pragma unroll
+      for (int d = 0; d < OWN; ++d) sm_o[(((kg * GROUP + wave) * OWN + d) * NT + t) * MS_WAVE + lane] = kg == 0 ? o[OWN + d][t] : o[d][t];
+    }
+    __syncthreads();
+#pragma unroll
+    for (int t = 0; t < NT; ++t) {
+      const int c = (wave * NT + t) * 16 + col16;
+      const float other_m = sm_m[kg ^ 1][c], big = fmaxf(m[t], other_m), safe = big == -INFINITY ? 0.f : big;
+      const float mine = fast_exp2(m[t] - safe), theirs = fast_exp2(other_m - safe);
+      l[t] = l[t] * mine + sm_l[kg ^ 1][c] * theirs;
+#pragma unroll
+      for (int d = 0; d < OWN; ++d) {
+        const f32x4 part = sm_o[((((kg ^ 1) * GROUP + wave) * OWN + d) * NT + t) * MS_WAVE + lane];
+        if (kg == 0) o[d][t] = o[d][t] * mine + part * theirs;
+        else o[OWN + d][t] = o[OWN + d][t] * mine + part * theirs;
+      }
+    }
+  }
+#pragma unroll
+  for (int t = 0; t < NT; ++t) {
+    if (pos[t] < 0) continue;
+    const int c = c0 + t * 16 + col16;
+    const float inv = 1.0f / l[t];
+    bf16* op = out + (size_t)(q0 + c / rep) * out_stride + (size_t)(g * rep + c % rep) * D + kq * 4;
+#pragma unroll
+    for (int d = 0; d < CT; ++d) {
+      if (KG > 1 && d / OWN != kg) continue;
+      bf16x4 w;
+#pragma unroll
+      for (int i = 0; i < 4; ++i) w[i] = (__bf16)(o[d][t][i] * inv);
+      *reinterpret_cast<bf16x4*>(op + d * 16) = w;
+    }
+  }
+}
+
+template <int D, int KG>
+int launch(dim3 grid, dim3 block, const bf16* q, size_t q_stride, const bf16* k, const bf16* vt, const int* table, int table_stride,
+           const int* table_rows, const int* q_start, const int* ctx, bf16* out, size_t out_stride, int nh, int nkv, int page_size,
+           float scale_log2e, int window, int n_requests, int pair_order, hipStream_t stream) {
+  constexpr size_t bytes = (size_t)KG * 2 * 2 * KEYS * D * sizeof(bf16);
+  static bool raised = false;   // once per instantiation: allow more dynamic LDS than the default 64 KB
+  if (!raised) {
+    if (hipFuncSetAttribute(reinterpret_cast<const void*>(&attention_prompt_kernel<D, KG>),
+                            hipFuncAttributeMaxDynamicSharedMemorySize, (int)bytes) != hipSuccess)
+      return MS_LAUNCH_FAILED;
+    raised = true;
+  }
+  attention_prompt_kernel<D, KG><<<grid, block, bytes, stream>>>(q, q_stride, k, vt, table, table_stride, table_rows, q_start, ctx, out, out_stride, nh, nkv, page_size, scale_log2e, window, n_requests, pair_order);
+  return ms_launch_status();
+}
+
+}  // namespace
+
+// Whether a step's attention is the faster way here than on ms_paged_attention_mfma (a launch's constants: a captured
+// graph's are its capacities).  A block's time is a chain of tiles of 64 keys, 1.7 us each (two groups at 64 dims: half as
+// many), where the other kernel spreads a tile's keys over four waves: so this one pays once its blocks fill the chip, at
+// 64 dims, where a tile draws half as much, for chains that are short beside the step or contexts that are long.
+// Measured, us, other kernel / this one: 28 heads on 4 of 128 dims, 700 tokens 20.1 / 25.6, 1,024 33 / 30, 2,048 91 / 54,
+// 4,096 318 / 130 (and behind 4,096 more 903 / 353), 4 x 512 41.8 / 25.1, 16 x 100 23.6 / 14.8; 14 heads on 2 of 64 dims,
+// 2,048 tokens 24.3 / 30.9, 3,500 55.1 / 60.1, 4,096 57.9 / 56.4 (behind 4,096 more 143 / 120), 2 x 2,048 39.4 / 42.1,
+// 4 x 512 14.9 / 12.7, 8 x 512 23.5 / 16.3, 16 x 100 11.1 / 8.2.  A single token behind a long context is one block with the
+// whole chain (nine requests with 2,040 tokens and eight of one behind 4,000 keys: 132 / 130 at 128 dims), so in a step of
+// several requests the contexts may be no longer than twice the step.
+extern "C" int ms_attention_prompt_pays(int n_requests, int n_tokens, int max_q_len, int max_context_len, int num_heads,
+                                        int num_kv_heads, int head_dim, int page_size) {
+  if ((head_dim != 64 && head_dim != 128) || page_size % 16 || num_kv_heads <= 0) return 0;
+  if (n_requests > 1 && (long long)max_context_len > 2LL * n_tokens) return 0;
+  const long long blocks = (long long)n_tokens * (num_heads / num_kv_heads) / COLS * num_kv_heads, cus = ms_compute_units();
+  if (head_dim == 128) return blocks * 8 >= cus * 7;
+  if (n_requests == 1) return blocks * 10 >= cus * 17 && max_context_len >= 4096;
+  return blocks * 16 >= cus * 7 && (long long)max_q_len * 3 <= n_tokens;
+}
+
+// The arguments of ms_paged_attention_mfma's general shape, for plain scores (no sink, cap, slopes, gate; values of the
+// keys' size).  MS_UNSUPPORTED for what it does not take.
+extern "C" int ms_attention_prompt(const void* q, long long q_stride, const void* k_pages, const void* vt_pages,
+                                   const int* block_table, int table_stride, const int* table_rows, const int* q_start,
+                                   const int* context_lens, void* out, long long out_stride, int n_requests, int n_tokens,
+                                   int max_q_len, int num_heads, int num_kv_heads, int head_dim, int page_size, float scale,
+                                   int window, hipStream_t stream) {
+  if (n_requests <= 0 || max_q_len <= 0 || n_tokens <= 0) return MS_OK;
+  if (num_heads <= 0 || num_kv_heads <= 0 || num_heads % num_kv_heads || table_stride <= 0) return MS_BAD_ARG;
+  if (!(scale > 0.f)) return MS_BAD_ARG;   // maxima are taken of the raw scores
+  if (q_stride % 8 || out_stride % 4 || ((uintptr_t)q % 16) || ((uintptr_t)out % 8)) return MS_UNSUPPORTED;
+  if (num_kv_heads > 65535 || page_size <= 0) return MS_UNSUPPORTED;
+  if (head_dim != 64 && head_dim != 128) return MS_UNSUPPORTED;
+  if (page_size % 16 || ((uintptr_t)k_pages | (uintptr_t)vt_pages) % 16) return MS_UNSUPPORTED;
+  const int rep = num_heads / num_kv_heads;
+  long long tiles = (long long)n_tokens * rep / COLS + n_requests;
+  tiles = std::min(tiles, (((long long)max_q_len * rep + COLS - 1) / COLS) * n_requests);
+  if (tiles > 65535 || (long long)max_q_len * rep > 0x7fffffffLL) return MS_UNSUPPORTED;
+  const int pair_order = tiles * num_kv_heads <= 2LL * ms_compute_units() ? 1 : 0;
+  dim3 grid(num_kv_heads, (unsigned)tiles), block((head_dim == 64 ? 2 : 1) * GROUP * MS_WAVE);
+#define GO(D, KG) return launch<D, KG>(grid, block, (const bf16*)q, (size_t)q_stride, (const bf16*)k_pages, (const bf16*)vt_pages, block_table, table_stride, table_rows, q_start, context_lens, (bf16*)out, (size_t)out_stride, num_heads, num_kv_heads, page_size, scale * 1.4426950408889634f, window, n_requests, pair_order, stream)
+  if (head_dim == 64) GO(64, 2);
+  GO(128, 1);
+#undef GO
+}

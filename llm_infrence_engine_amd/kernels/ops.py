@@ -67,6 +67,9 @@ _SIGNATURES = {
     "ms_paged_attention_mfma": [_c_ptr, _c_ll, _c_ptr, _c_ptr, _c_ptr, _c_int, _c_ptr, _c_ptr, _c_ptr, _c_ptr, _c_ll,
                                 _c_int, _c_int, _c_int, _c_int, _c_int, _c_int, _c_int, _c_int, _c_float, _c_int, _c_ptr,
                                 _c_float, _c_ptr, _c_ptr, _c_ll, _c_int, _c_float, _c_ptr],
+    "ms_attention_prompt": [_c_ptr, _c_ll, _c_ptr, _c_ptr, _c_ptr, _c_int, _c_ptr, _c_ptr, _c_ptr, _c_ptr, _c_ll, _c_int, _c_int,
+                            _c_int, _c_int, _c_int, _c_int, _c_int, _c_float, _c_int, _c_ptr],
+    "ms_attention_prompt_pays": [_c_int, _c_int, _c_int, _c_int, _c_int, _c_int, _c_int, _c_int],
     "ms_paged_attention_mfma_decode": [_c_ptr, _c_ll, _c_ptr, _c_ptr, _c_ptr, _c_int, _c_ptr, _c_ptr, _c_ptr, _c_ptr,
                                        _c_ll, _c_ptr, _c_ptr, _c_int, _c_int, _c_int, _c_int, _c_int, _c_int, _c_float,
                                        _c_int, _c_int, _c_int, _c_ptr, _c_float, _c_ptr, _c_ptr, _c_ll, _c_int, _c_float,
@@ -903,6 +906,7 @@ def paged_attention_mfma(q: torch.Tensor, k_pages: torch.Tensor, vt_pages: torch
         raise ValueError(f"max_q_len {max_q_len} / max_context_len {max_context_len} do not fit a table of "
                          f"{block_table.shape[1]} pages of {page_size}")
     q_stride = q.stride(0) if N > 1 else q.shape[1]
+    plain = sink is None and not softcap and slopes is None and gate is None and out_scale == 1.0 and dv == d
     if attention_splits_keys(R, nkv, num_heads // nkv, max_q_len, max_context_len):
         # a launch constant of the batch size and of the longest context the step is made for (in a captured
         # graph: the cache's capacity, so that the graph stays valid as contexts grow): every request spreads
@@ -919,6 +923,12 @@ def paged_attention_mfma(q: torch.Tensor, k_pages: torch.Tensor, vt_pages: torch
               block_table.data_ptr(), block_table.shape[1], _ptr(table_rows), q_start.data_ptr(), context_lens.data_ptr(),
               out.data_ptr(), num_heads * dv, part_o.data_ptr(), part_ml.data_ptr(), R, num_heads, nkv, d, dv, page_size, float(scale),
               int(window or 0), MIN_BLOCKS_PER_SPLIT, n_splits, _ptr(sink), *more, _stream())
+    elif (plain and k_pages.data_ptr() % 16 == 0 and vt_pages.data_ptr() % 16 == 0
+          and _get("ms_attention_prompt_pays")(R, N, max_q_len, max_context_len, num_heads, nkv, d, page_size)):
+        # many prompt tokens: keys and values staged in LDS for four neighbouring tiles
+        _call("ms_attention_prompt", q.data_ptr(), q_stride, k_pages.data_ptr(), vt_pages.data_ptr(), block_table.data_ptr(),
+              block_table.shape[1], _ptr(table_rows), q_start.data_ptr(), context_lens.data_ptr(), out.data_ptr(), num_heads * dv,
+              R, N, max_q_len, num_heads, nkv, d, page_size, float(scale), int(window or 0), _stream())
     else:
         _call("ms_paged_attention_mfma", q.data_ptr(), q_stride, k_pages.data_ptr(), vt_pages.data_ptr(),
               block_table.data_ptr(), block_table.shape[1], _ptr(table_rows), q_start.data_ptr(), context_lens.data_ptr(),

@@ -984,6 +984,38 @@ def test_attention_mfma_tile_shapes(ops, d, shape):
     torch.testing.assert_close(got, want, **tol(torch.bfloat16))
 
 
+@pytest.mark.parametrize("nh,nkv,d,page_size,window", [(14, 2, 64, 16, None), (8, 8, 128, 32, None), (4, 1, 64, 16, 40),
+                                                        (28, 4, 128, 16, None), (6, 2, 64, 48, 130), (20, 1, 128, 16, 65)])
+def test_attention_of_staged_prompts(ops, nh, nkv, d, page_size, window):
+    """The prompt kernel that stages keys and values in LDS: single tokens, portions behind cached keys, prompts whose columns
+    fill no tile, a request without a token, rows of the table in no order, at the edges of its tiles of 64 keys; what no
+    request owns is NaN.  Against the oracle, and against the kernel that shares nothing."""
+    g = torch.Generator().manual_seed(nh * 10 + d)
+    ctx, qlen = [70, 133, 64, 65, 300, 1, 500], [70, 9, 64, 1, 150, 1, 257]
+    c = _paged_case(g, torch.bfloat16, nh, nkv, d, page_size, ctx, qlen, float("nan"))
+    scale = 1.0 / math.sqrt(d)
+    want = torch.cat([attention_reference(q.double(), k.double(), v.double(), scale, window).transpose(0, 1).reshape(-1, nh * d)
+                      for q, k, v in zip(c["qs"], c["ks"], c["vs"])])
+    N, R = c["q"].shape[0], len(ctx) + 1
+    wide = torch.zeros(N + 5, (nh + 2 * nkv) * d, dtype=torch.bfloat16, device=DEV)      # five tokens of nobody at the end
+    wide[:N, :nh * d] = c["q"].to(DEV)
+    perm = torch.randperm(R, generator=g)
+    table = torch.zeros(R, c["table"].shape[1], dtype=torch.int32)
+    table[perm[:R - 1]] = c["table"]
+    kp, vt, table, rows = c["kp"].to(DEV), c["vt"].to(DEV), table.to(DEV), perm.to(torch.int32).to(DEV)
+    q_start = torch.tensor([0] + list(np.cumsum(qlen)) + [N], dtype=torch.int32, device=DEV)
+    lens = torch.tensor(ctx + [7], dtype=torch.int32, device=DEV)
+    out = torch.full((N + 5, nh * d), 3.0, dtype=torch.bfloat16, device=DEV)
+    ops._call("ms_attention_prompt", wide.data_ptr(), wide.stride(0), kp.data_ptr(), vt.data_ptr(), table.data_ptr(),
+              table.shape[1], rows.data_ptr(), q_start.data_ptr(), lens.data_ptr(), out.data_ptr(), nh * d, R, N + 5, 257, nh,
+              nkv, d, page_size, scale, window or 0, ops._stream())
+    torch.testing.assert_close(out[:N].double().cpu(), want, **tol(torch.bfloat16))
+    assert (out[N:] == 3.0).all()
+    other = torch.empty(N, nh * d, dtype=torch.bfloat16, device=DEV)
+    ops.paged_attention_mfma(wide[:N], kp, vt, table, q_start, lens, other, nh, scale, 257, 500, window, table_rows=rows)
+    torch.testing.assert_close(out[:N].double(), other.double(), **tol(torch.bfloat16))
+
+
 @pytest.mark.parametrize("ramp", [0.5, 6.0, 60.0])
 def test_attention_mfma_when_the_maximum_keeps_rising(ops, ramp):
     """Scores that grow along the context by ``ramp`` log2 units in all: the running reference of the softmax
