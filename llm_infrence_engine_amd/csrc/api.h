@@ -63,6 +63,9 @@ void ms_attention_mfma_force(int nt, int waves, int dim_shares);
 int ms_gemm_stream(const void* A, long long lda, const int* rows, const float* norm_w, float eps, const void* W,
                    long long ldw, const float* bias, void* out, long long ldo, int M, int N, int K, int epilogue,
                    int out_dtype, int norm, int any_shape, hipStream_t stream);
+int ms_gemm_quads(const void* A, long long lda, const int* rows, const float* norm_w, float eps, const void* W,
+                   long long ldw, const float* bias, void* out, long long ldo, int M, int N, int K, int epilogue,
+                   int out_dtype, int norm, hipStream_t stream);
 
 int ms_gemm_panel(const void* A, long long lda, const int* rows, const float* norm_w, float eps, const void* W,
                    long long ldw, const float* bias, void* out, long long ldo, int M, int N, int K, int epilogue,

@@ -7,6 +7,7 @@
 // dimension to be the whole head and d/2 a multiple of 16.
 #include "common.h"
 #include "api.h"
+#include "quads.h"
 
 namespace {
 
@@ -192,7 +193,85 @@ qkv_rope_store_kernel(const float* __restrict__ X, size_t ldx, const float* __re
   }
 }
 
-int g_qkv_pair8 = -1;   // measurements: 0 / 1 force whole tiles / tiles of 8 + 8 rows, -1 leaves the choice
+// Few tokens: a block owns two units of four rows (quads.h), each of two lower features of a head and their partners half
+// a head above.  G tokens; the same sums in the same order as above, to the bit.  The blocks above are 18 to 36 here, each a
+// chain of dependent loads; these are one to two for every two CUs, and a wave's whole share is in flight at once.  0.5B
+// shape (1152 x 896): 5.2 -> 4.2 us at one token, 5.5 -> 5.0 at 8 (the launch alone is 1.6).
+template <int WAVES, int G>
+__global__ void __launch_bounds__(WAVES * MS_WAVE)
+qkv_rope_store_few_kernel(const float* __restrict__ X, size_t ldx, const float* __restrict__ norm_w, float eps,
+                          const bf16* __restrict__ W, const float* __restrict__ bias, const int* __restrict__ positions,
+                          const float* __restrict__ inv_freq, const int* __restrict__ slot_mapping,
+                          bf16* __restrict__ q_out, bf16* __restrict__ k_pages, bf16* __restrict__ v_pages, int M, int K,
+                          int nh, int nkv, int d, int page_size, int v_transposed) {
+  constexpr int U = 2;
+  __shared__ f32x4 part[U][WAVES][G];
+  __shared__ float part_ss[WAVES][G];
+  const int lane = threadIdx.x & (MS_WAVE - 1);
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / MS_WAVE);   // the same for the whole wave
+  const int head = blockIdx.y, half = d / 2, j0 = blockIdx.x * (2 * U);
+
+  const bf16* wrow[U];
+#pragma unroll
+  for (int u = 0; u < U; ++u)
+    wrow[u] = W + ((size_t)head * d + j0 + 2 * u + (lane & 1) + ((lane >> 1) & 1) * half) * K;
+  const int m = lane & (G - 1), mc = min(m, M - 1);
+  const float* x = X + (size_t)mc * ldx;
+  QuadProduct<U, G, 1, true> product(lane, wave, WAVES, K);
+  product.ask(0, wrow, x, norm_w);
+  // What the epilogue needs from memory arrives under the products: wave u finishes unit u, lane r G + m stores its row r
+  // for token m (r = 0, 1: the lower features, r = 2, 3: their partners).
+  const int r = (lane / G) & 3, j = j0 + 2 * min(wave, U - 1) + (r & 1);
+  const float b_lo = bias ? bias[head * d + j] : 0.f, b_hi = bias ? bias[head * d + half + j] : 0.f;
+  const float freq = inv_freq[j];
+  const int pos = positions[mc];
+  const long long slot = slot_mapping[mc];
+  product.run(wrow, x, norm_w);
+
+  const float squares = quad_sum_rows(product.ss);
+  if (lane < G) {
+#pragma unroll
+    for (int u = 0; u < U; ++u) part[u][wave][lane] = product.acc[u];
+    part_ss[wave][lane] = squares;
+  }
+  __syncthreads();
+  if (wave >= U || m >= M || lane >= 4 * G) return;
+  float total = 0.f, lo = 0.f, hi = 0.f;
+#pragma unroll
+  for (int w = 0; w < WAVES; ++w) {
+    const f32x4 v = part[wave][w][m];
+    total += part_ss[w][m];
+    lo += r & 1 ? v[1] : v[0];
+    hi += r & 1 ? v[3] : v[2];
+  }
+  const float inv = 1.0f / sqrtf(total / (float)K + eps);
+  lo = lo * inv + b_lo;
+  hi = hi * inv + b_hi;
+  if (head < nh + nkv) {   // q and k heads turn by position * inv_freq[j]
+    float sn, cs;
+    ms_sincos_rot((float)pos * freq, &sn, &cs);
+    const float x1 = lo, x2 = hi;
+    lo = x1 * cs - x2 * sn;
+    hi = x2 * cs + x1 * sn;
+  }
+  const bf16 v = __float2bfloat16(r < 2 ? lo : hi);
+  const int f = r < 2 ? j : j + half;   // this lane's feature within the head
+  if (head < nh) {
+    q_out[((size_t)m * nh + head) * d + f] = v;
+    return;
+  }
+  if (slot < 0) return;
+  // a page of a power of two (the usual case) needs no division
+  const bool pow2 = (page_size & (page_size - 1)) == 0;
+  const long long page = pow2 ? slot >> (31 - __builtin_clz(page_size)) : slot / page_size;
+  const int off = pow2 ? (int)(slot & (page_size - 1)) : (int)(slot % page_size);
+  if (head < nh + nkv) k_pages[(((size_t)page * nkv + (head - nh)) * page_size + off) * d + f] = v;
+  else if (v_transposed) v_pages[(((size_t)page * nkv + (head - nh - nkv)) * d + f) * page_size + off] = v;
+  else v_pages[(((size_t)page * nkv + (head - nh - nkv)) * page_size + off) * d + f] = v;
+}
+
+int g_qkv_pair8 = -1;   // measurements: 0 / 1 / 2 force whole tiles / tiles of 8 + 8 rows / units of four rows (up to 8
+                        // tokens), -1 leaves the choice
 
 template <int MT>
 int launch(const float* X, size_t ldx, const float* norm_w, float eps, const bf16* W, const float* bias,
@@ -204,12 +283,23 @@ int launch(const float* X, size_t ldx, const float* norm_w, float eps, const bf1
   // time is what its CU can draw.  With more blocks than CUs every block reading all the activations costs
   // more than the shorter stream of weights saves.
   const int pair_blocks = (nh + 2 * nkv) * (d / 16) * token_groups;
-  const bool pair8 = g_qkv_pair8 >= 0 ? g_qkv_pair8 != 0 : pair_blocks <= ms_compute_units();
+  const bool pair8 = g_qkv_pair8 == 0 || g_qkv_pair8 == 1 ? g_qkv_pair8 != 0 : pair_blocks <= ms_compute_units();
   const int blocks = pair8 ? pair_blocks : pair_blocks / 2;
   // LDS holds (waves - 1) * 2 * MT KB.  (Measured at the 0.5B and 7B shapes: 8 waves are 0.4 to 1 us faster than
   // 16; tiles of 8 or 4 rows on more CUs are slower, by up to 2x, because every block reads all activations.)
   int waves = 4;
   while (waves < 8 && blocks * waves < 1024 && steps >= waves * 2) waves *= 2;
+  // Units of four rows while one round of loads holds a wave's share (K <= 1024) and there is a CU for every block: the
+  // norm reads the activations as floats, once per block.  (At 3584 columns a product of 4608 rows took 14.7 us against
+  // 14.5, at 8 tokens 22 against 15.)
+  const int few_blocks = (nh + 2 * nkv) * (d / 8);
+  if (M <= 8 && (g_qkv_pair8 == 2 || (g_qkv_pair8 < 0 && K <= 1024 && few_blocks <= ms_compute_units()))) {
+#define GO(WV, G) qkv_rope_store_few_kernel<WV, G><<<dim3(d / 8, nh + 2 * nkv), dim3(WV * MS_WAVE), 0, stream>>>(X, ldx, norm_w, eps, W, bias, positions, inv_freq, slot_mapping, q_out, k_pages, v_pages, M, K, nh, nkv, d, page_size, v_transposed)
+    if (M <= 4) { if (waves == 4) GO(4, 4); else GO(8, 4); }
+    else { if (waves == 4) GO(4, 8); else GO(8, 8); }
+#undef GO
+    return ms_launch_status();
+  }
 #define GO(WV, P8) qkv_rope_store_kernel<MT, WV, P8><<<dim3(d / (P8 ? 16 : 32), nh + 2 * nkv, token_groups), dim3(WV * MS_WAVE), 0, stream>>>(X, ldx, norm_w, eps, W, bias, positions, inv_freq, slot_mapping, q_out, k_pages, v_pages, M, K, nh, nkv, d, page_size, v_transposed)
   if (pair8) { if (waves == 4) GO(4, true); else GO(8, true); }
   else { if (waves == 4) GO(4, false); else GO(8, false); }

@@ -589,6 +589,33 @@ def test_gemm_stream(ops, M, N, K):
     torch.testing.assert_close(gated.double(), torch.nn.functional.silu(hw[:, 0::2]) * hw[:, 1::2], **tol(torch.bfloat16))
 
 
+@pytest.mark.parametrize("M", [1, 3, 7, 16])
+@pytest.mark.parametrize("N,K", [(898, 6136), (898, 2056), (1030, 264), (2040, 1032), (4100, 1000)])
+def test_products_in_units_of_four_rows(ops, M, N, K):
+    """Few rows and a narrow matrix: one or two units of four rows to a block, one to three loads of four k-steps, steps
+    that fill a load in part, a last step that K fills in part, rows that run out inside a unit, strided activations.  A
+    row has the same bits alone and among the rows that go to the tiled kernel; an infinite activation stays in its row.
+    Tolerance: float sums of K products of unit variance over another order."""
+    g = torch.Generator().manual_seed(M * 1000 + N + K)
+    a = torch.randn(16, K + 8, generator=g).bfloat16().to(DEV)[:, :K]
+    w = (torch.randn(N, K, generator=g) / math.sqrt(K)).bfloat16().to(DEV)
+    bias = torch.randn(N, generator=g).to(DEV)
+    want = a.double() @ w.double().T
+    got = ops.gemm_skinny(a[:M], w, out_dtype=torch.float32)
+    torch.testing.assert_close(got.double(), want[:M], atol=3e-5, rtol=3e-5)
+    assert torch.equal(got, ops.gemm_skinny(a, w, out_dtype=torch.float32)[:M])
+    x = torch.randn(16, K, generator=g).to(DEV)
+    nw = (1 + 0.1 * torch.randn(K, generator=g)).to(DEV)
+    h = (x.double() * nw.double()).float().bfloat16().double() * torch.rsqrt((x.double() ** 2).mean(-1, keepdim=True) + 1e-6)
+    got = ops.gemm_skinny_norm(x[:M], nw, 1e-6, w, bias, out_dtype=torch.float32)
+    torch.testing.assert_close(got.double(), (h @ w.double().T + bias.double())[:M], atol=2e-4, rtol=2e-4)
+    if K < 2048:   # (longer rows with a norm are staged, by as many columns as the rows leave room for)
+        assert torch.equal(got, ops.gemm_skinny_norm(x, nw, 1e-6, w, bias, out_dtype=torch.float32)[:M])
+    b = a[:M].clone()
+    b[0, K - 1] = float("inf")
+    torch.testing.assert_close(ops.gemm_skinny(b, w, out_dtype=torch.float32)[1:].double(), want[1:M], atol=3e-5, rtol=3e-5)
+
+
 def test_gemm_stream_refuses_what_it_cannot_take(ops):
     w = torch.zeros(64, 64, dtype=torch.bfloat16, device=DEV)
     with pytest.raises(RuntimeError, match="unsupported"):
@@ -1088,6 +1115,21 @@ def test_qkv_rope_store_fused_equals_the_separate_kernels(ops, M, nh, nkv, d, K,
 
     lib = build.load()
     lib.ms_qkv_rope_store_force(0 if tiles == "whole" else 1)
+    try:
+        _qkv_fused_case(ops, M, nh, nkv, d, K, v_transposed)
+    finally:
+        lib.ms_qkv_rope_store_force(-1)
+
+
+@pytest.mark.parametrize("M", [1, 4, 5, 8])
+@pytest.mark.parametrize("nh,nkv,d,K,v_transposed", [(14, 2, 64, 896, True), (6, 3, 32, 72, False), (4, 1, 128, 2568, True)])
+def test_qkv_rope_store_in_units_of_four_rows(ops, M, nh, nkv, d, K, v_transposed):
+    """The blocks of few tokens: two units of two rotary pairs, one or two groups of four tokens, a last group that is
+    not full, columns of one piece, of one round and of two."""
+    from llm_infrence_engine_amd.kernels import build
+
+    lib = build.load()
+    lib.ms_qkv_rope_store_force(2)
     try:
         _qkv_fused_case(ops, M, nh, nkv, d, K, v_transposed)
     finally:
