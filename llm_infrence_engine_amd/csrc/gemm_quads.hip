@@ -94,7 +94,7 @@ gemm_quads_kernel(const void* __restrict__ A, size_t lda, const bf16* __restrict
 // wider ones of one round of loads (7296 x 896: 6.3 | 5.4).  Every block reads all the activations, so more tokens pay for
 // less: 5 to 8 of them lose with a long K (896 x 4864: 6.8 | 7.1; ms_gemm_stream, which shares them out through LDS, keeps
 // those), 3 or 4 where a wave needs a second round (896 x 7296: 7.4 | 8.0), and the folded norm, which reads twice the bytes,
-// beyond one round or a wide W (9728 x 896 at 4 tokens: 7.9 | 8.4; 512 x 3584: 5.5 | 8.0).
+// beyond one round or a wide W (9728 x 896 at 4 tokens: 7.9 | 8.4; 512 x 3584 at 8: 7.6 | 8.1).
 bool pays(int M, int units, int K, bool norm, int cus) {
   if (K < 256) return false;
   if (K <= 1024) return units <= (M > 8 ? 1 : norm || M > 4 ? 2 : 8) * cus && !(norm && M > 8);

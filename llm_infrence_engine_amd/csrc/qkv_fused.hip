@@ -291,7 +291,7 @@ int launch(const float* X, size_t ldx, const float* norm_w, float eps, const bf1
   while (waves < 8 && blocks * waves < 1024 && steps >= waves * 2) waves *= 2;
   // Units of four rows while one round of loads holds a wave's share (K <= 1024) and there is a CU for every block: the
   // norm reads the activations as floats, once per block.  (At 3584 columns a product of 4608 rows took 14.7 us against
-  // 14.5, at 8 tokens 22 against 15.)
+  // 14.5 at one token, and more tokens cost these blocks more.)
   const int few_blocks = (nh + 2 * nkv) * (d / 8);
   if (M <= 8 && (g_qkv_pair8 == 2 || (g_qkv_pair8 < 0 && K <= 1024 && few_blocks <= ms_compute_units()))) {
 #define GO(WV, G) qkv_rope_store_few_kernel<WV, G><<<dim3(d / 8, nh + 2 * nkv), dim3(WV * MS_WAVE), 0, stream>>>(X, ldx, norm_w, eps, W, bias, positions, inv_freq, slot_mapping, q_out, k_pages, v_pages, M, K, nh, nkv, d, page_size, v_transposed)
