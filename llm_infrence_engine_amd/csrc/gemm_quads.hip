@@ -11,7 +11,6 @@
 #include "common.h"
 #include "api.h"
 #include "quads.h"
-#include <algorithm>
 
 namespace {
 

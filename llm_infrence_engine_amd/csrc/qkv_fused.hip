@@ -194,9 +194,9 @@ qkv_rope_store_kernel(const float* __restrict__ X, size_t ldx, const float* __re
 }
 
 // Few tokens: a block owns two units of four rows (quads.h), each of two lower features of a head and their partners half
-// a head above.  G tokens; the same sums in the same order as above, to the bit.  The blocks above are 18 to 36 here, each a
-// chain of dependent loads; these are one to two for every two CUs, and a wave's whole share is in flight at once.  0.5B
-// shape (1152 x 896): 5.2 -> 4.2 us at one token, 5.5 -> 5.0 at 8 (the launch alone is 1.6).
+// a head above.  G tokens; the same sums in the same order as above, to the bit.  The 0.5B shape (1152 x 896) has 72
+// of the blocks above, each wave of which waits for a chain of dependent loads; there are 144 of these, and a wave's whole
+// share is in flight at once: 5.2 -> 4.2 us at one token, 5.5 -> 5.0 at 8 (the launch alone is 1.6).
 template <int WAVES, int G>
 __global__ void __launch_bounds__(WAVES * MS_WAVE)
 qkv_rope_store_few_kernel(const float* __restrict__ X, size_t ldx, const float* __restrict__ norm_w, float eps,
