@@ -7,11 +7,19 @@
 // the four waves of a block own neighbouring tiles of 32 columns and walk the same keys, 64 at a time: those go from the
 // pages straight to LDS (global_load_lds), a tile of keys ahead of their use, and every wave reads all of them there.  Two
 // blocks share a CU (64 KB of LDS each), one barrier a tile.  What is left is the softmax on the vector pipe (16
-// exponentials of 16 clocks per 32 x 32 scores) beside the products: 930 TFLOP/s at 4,096 tokens of 28 heads of 128 dims,
-// 1,020 behind 4,096 more, where the unstaged kernel has 380 and 400.
+// exponentials of 16 clocks per 32 x 32 scores) beside the products: 870 TFLOP/s at 4,096 tokens of 28 heads of 128 dims,
+// 990 behind 4,096 more, where the unstaged kernel has 380 and 400.
 //
 // A unit is 32 keys.  Row r of the u-th score product of a unit is its key 8 (r / 4) + 4 u + r % 4, so that a lane (quarter
 // kq) has the scores of the eight consecutive keys 8 kq .. + 7, which it needs as one 16-byte read of a value's row.
+// Rounding: the probabilities meet the values as bfloat16, and those that are powers of two lose nothing by it.  The four
+// waves that share a tile in the other kernel have a reference each, the largest score of their first 32 keys; a column here
+// has one (two at 64 dims), and where that stayed with its first 64 keys the result lay 2 to 9 % farther from 64 bits (28
+// heads of 128 dims, 16 x 130 tokens, scores of spread 2: 0.00180 of the norm for 0.00175; 14 of 64 dims: 0.00189 for
+// 0.00176).  So over the wave's first 128 keys the reference goes with the maximum of every unit of 32, down too, and later
+// it moves at a smaller distance than there: 0.00175 and 0.00176, and no farther than the other kernel from 64 to 8,192 keys
+// at spreads of 1 to 5.  Price: 1 to 6 % of a long prompt's time (2,048 tokens of 28 heads of 128 dims 58.5 -> 61.2 us),
+// while short ones gain as much from the exchange of maxima without LDS (16 x 100: 13.9 -> 13.3).
 // LDS: keys in rows of D, their 16-byte pieces permuted so that the 16 rows of a product meet every bank once (piece p of
 // key k at place p ^ f(k)); values as they lie in a page of 16, [dim][16 keys], the two halves of a row swapped for every
 // other eight dims.
@@ -32,8 +40,22 @@ constexpr int NT = 2;                 // tiles of 16 columns a wave
 constexpr int COLS = GROUP * NT * 16; // columns a block
 constexpr int KEYS = 64;              // keys a tile: one chunk of 16 for every wave to bring
 
+constexpr int FOLLOWED = 128;         // keys over which the reference goes with every unit's maximum ..
+constexpr float FOLLOW_DOWN = 4.f;    // .. unless that is further below it: sums grow by 2^16 at most on the way down
+// log2 units by which a maximum may run ahead of its reference afterwards (64 dims: two references a column)
+template <int D> constexpr float SLACK = D == 64 ? 4.f : 3.f;
+
 template <int D> __device__ __forceinline__ int permute(int key) {     // f of a key's number in its unit
   return D == 128 ? (key & 3) | ((key >> 1) & 12) : ((key >> 1) & 1) | ((key >> 2) & 6);
+}
+
+// The maximum over the four lanes, 16 apart, that share a column.
+__device__ __forceinline__ float column_max(float x) {
+  const unsigned u = __float_as_uint(x);
+  const auto a = __builtin_amdgcn_permlane16_swap(u, u, false, false);
+  const unsigned w = __float_as_uint(fmaxf(__uint_as_float(a[0]), __uint_as_float(a[1])));
+  const auto b = __builtin_amdgcn_permlane32_swap(w, w, false, false);
+  return fmaxf(__uint_as_float(b[0]), __uint_as_float(b[1]));
 }
 
 // KG groups of waves own the same columns and take the tiles of keys in turn, each with its own place in LDS; at the end
@@ -75,6 +97,7 @@ attention_prompt_kernel(const bf16* __restrict__ q, size_t q_stride, const bf16*
   const bool works = c0 < ncols;
   const int first_pos = start_pos + min(c0, ncols - 1) / rep, last_pos = start_pos + (min(ncols, c0 + NT * 16) - 1) / rep;
   const bool full = c0 + NT * 16 <= ncols;
+  const int wave_lo = window > 0 ? max(0, first_pos - window + 1) : 0, follow_end = (wave_lo + FOLLOWED - 1) / KEYS + 1;
 
   // ---- bringing a tile: the wave's chunk of keys and of values
   const int k_lane = lane * 8;                                 // this lane's first value in a load's 1 KB
@@ -148,43 +171,38 @@ attention_prompt_kernel(const bf16* __restrict__ q, size_t q_stride, const bf16*
       page_next = t + 2 * KG < t_end ? page_of(t + 2 * KG) : 0;
     }
     if (!works || t >= t_end) continue;      // the same for the whole wave
-    // two units at a time, or one where the registers (128 a lane with two groups) hold no more scores
-    constexpr int UNITS = KG == 1 ? 2 : 1, SPAN = UNITS * 32;
+    const float slack = t < follow_end ? -FOLLOW_DOWN : SLACK<D>;
 #pragma unroll
-    for (int unit = 0; unit < 2; unit += UNITS) {
+    for (int unit = 0; unit < 2; ++unit) {
       const int base = t * KEYS + unit * 32;
       if (base > last_pos) break;
       const bf16* st = lds + (kg * 2 + stage) * STAGE + unit * 2 * CHUNK;
 
-      // scores: s[n][u][t] holds keys base + n*32 + kq*8 + u*4 + (0..3) of column t*16 + col16
-      f32x4 s[UNITS][2][NT];
+      // scores: s[u][t] holds keys base + kq*8 + u*4 + (0..3) of column t*16 + col16
+      f32x4 s[2][NT];
 #pragma unroll
-      for (int n = 0; n < UNITS; ++n)
+      for (int u = 0; u < 2; ++u) {
 #pragma unroll
-        for (int u = 0; u < 2; ++u) {
+        for (int t2 = 0; t2 < NT; ++t2) s[u][t2] = f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-          for (int t2 = 0; t2 < NT; ++t2) s[n][u][t2] = f32x4{0.f, 0.f, 0.f, 0.f};
+        for (int ks = 0; ks < D / 32; ++ks) {
+          const bf16x8 kf = *reinterpret_cast<const bf16x8*>(st + k_row[u] + (((ks * 4 + kq) ^ k_perm[u]) & (PIECES - 1)) * 8);
 #pragma unroll
-          for (int ks = 0; ks < D / 32; ++ks) {
-            const bf16x8 kf = *reinterpret_cast<const bf16x8*>(st + n * 2 * CHUNK + k_row[u] + (((ks * 4 + kq) ^ k_perm[u]) & (PIECES - 1)) * 8);
-#pragma unroll
-            for (int t2 = 0; t2 < NT; ++t2) s[n][u][t2] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(kf, qv[t2][ks], s[n][u][t2], 0, 0, 0);
-          }
+          for (int t2 = 0; t2 < NT; ++t2) s[u][t2] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(kf, qv[t2][ks], s[u][t2], 0, 0, 0);
         }
+      }
 
-      const bool unmasked = full && base + SPAN - 1 <= first_pos && (window <= 0 || base > last_pos - window);
+      const bool unmasked = full && base + 31 <= first_pos && (window <= 0 || base > last_pos - window);
       if (!unmasked) {
 #pragma unroll
-        for (int n = 0; n < UNITS; ++n)
+        for (int u = 0; u < 2; ++u)
 #pragma unroll
-          for (int u = 0; u < 2; ++u)
+          for (int t2 = 0; t2 < NT; ++t2)
 #pragma unroll
-            for (int t2 = 0; t2 < NT; ++t2)
-#pragma unroll
-              for (int i = 0; i < 4; ++i) {
-                const int key = base + n * 32 + kq * 8 + u * 4 + i;
-                if (key > pos[t2] || (window > 0 && key <= pos[t2] - window)) s[n][u][t2][i] = -INFINITY;
-              }
+            for (int i = 0; i < 4; ++i) {
+              const int key = base + kq * 8 + u * 4 + i;
+              if (key > pos[t2] || (window > 0 && key <= pos[t2] - window)) s[u][t2][i] = -INFINITY;
+            }
       }
       float bmax[NT];
       bool ahead = false;
@@ -192,22 +210,17 @@ attention_prompt_kernel(const bf16* __restrict__ q, size_t q_stride, const bf16*
       for (int t2 = 0; t2 < NT; ++t2) {
         float bm = -INFINITY;
 #pragma unroll
-        for (int n = 0; n < UNITS; ++n)
+        for (int u = 0; u < 2; ++u)
 #pragma unroll
-          for (int u = 0; u < 2; ++u)
-#pragma unroll
-            for (int i = 0; i < 4; ++i) bm = fmaxf(bm, s[n][u][t2][i]);
+          for (int i = 0; i < 4; ++i) bm = fmaxf(bm, s[u][t2][i]);
         bmax[t2] = bm;
-        ahead |= bm * scale_log2e > m[t2] + REF_SLACK;
+        ahead |= bm * scale_log2e > m[t2] + slack;
       }
-      if (__builtin_amdgcn_ballot_w64(ahead) != 0) {      // some column's reference moves: rare
+      if (__builtin_amdgcn_ballot_w64(ahead) != 0) {      // some column's reference moves: rare once the first keys are past
 #pragma unroll
         for (int t2 = 0; t2 < NT; ++t2) {
-          float bm = bmax[t2];
-          bm = fmaxf(bm, __shfl_xor(bm, 16, MS_WAVE));
-          bm = fmaxf(bm, __shfl_xor(bm, 32, MS_WAVE));
-          bm *= scale_log2e;
-          const bool step = bm > m[t2] + REF_SLACK;
+          const float bm = column_max(bmax[t2]) * scale_log2e;
+          const bool step = bm > m[t2] + slack;
           const float corr = step ? fast_exp2(m[t2] - bm) : 1.0f;      // m = -inf: 0
           if (step) m[t2] = bm;
           if (SUMS_BY_MATRIX) lsum[t2] *= corr; else lvec[t2] *= corr;
@@ -219,40 +232,37 @@ attention_prompt_kernel(const bf16* __restrict__ q, size_t q_stride, const bf16*
 #pragma unroll
       for (int t2 = 0; t2 < NT; ++t2) ref[t2] = m[t2] == -INFINITY ? 0.f : m[t2];
       // values past the wave's last visible key may be anything a reused page still holds: they count as zeros
-      const bool clean = base + SPAN - 1 <= last_pos;
+      const bool clean = base + 31 <= last_pos;
+      bf16x8 p[NT];
 #pragma unroll
-      for (int n = 0; n < UNITS; ++n) {
-        bf16x8 p[NT];
+      for (int t2 = 0; t2 < NT; ++t2) {
 #pragma unroll
-        for (int t2 = 0; t2 < NT; ++t2) {
+        for (int u = 0; u < 2; ++u)
 #pragma unroll
-          for (int u = 0; u < 2; ++u)
-#pragma unroll
-            for (int i = 0; i < 4; ++i) {
-              const float e = fast_exp2(fmaf(s[n][u][t2][i], scale_log2e, -ref[t2]));
-              if (!SUMS_BY_MATRIX) lvec[t2] += e;
-              p[t2][u * 4 + i] = (__bf16)e;
-            }
-          if (SUMS_BY_MATRIX) lsum[t2] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ones, p[t2], lsum[t2], 0, 0, 0);
-        }
-#pragma unroll
-        for (int c4 = 0; c4 < CT; c4 += 4) {
-          bf16x8 v[4];
-#pragma unroll
-          for (int c = 0; c < 4; ++c) v[c] = *reinterpret_cast<const bf16x8*>(st + n * 2 * CHUNK + v_row + (c4 + c) * 256);
-          if (!clean) {
-#pragma unroll
-            for (int i = 0; i < 8; ++i)
-              if (base + n * 32 + kq * 8 + i > last_pos) {
-#pragma unroll
-                for (int c = 0; c < 4; ++c) v[c][i] = (__bf16)0.0f;
-              }
+          for (int i = 0; i < 4; ++i) {
+            const float e = fast_exp2(fmaf(s[u][t2][i], scale_log2e, -ref[t2]));
+            if (!SUMS_BY_MATRIX) lvec[t2] += e;
+            p[t2][u * 4 + i] = (__bf16)e;
           }
+        if (SUMS_BY_MATRIX) lsum[t2] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ones, p[t2], lsum[t2], 0, 0, 0);
+      }
 #pragma unroll
-          for (int c = 0; c < 4; ++c)
+      for (int c4 = 0; c4 < CT; c4 += 4) {
+        bf16x8 v[4];
 #pragma unroll
-            for (int t2 = 0; t2 < NT; ++t2) o[c4 + c][t2] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(v[c], p[t2], o[c4 + c][t2], 0, 0, 0);
+        for (int c = 0; c < 4; ++c) v[c] = *reinterpret_cast<const bf16x8*>(st + v_row + (c4 + c) * 256);
+        if (!clean) {
+#pragma unroll
+          for (int i = 0; i < 8; ++i)
+            if (base + kq * 8 + i > last_pos) {
+#pragma unroll
+              for (int c = 0; c < 4; ++c) v[c][i] = (__bf16)0.0f;
+            }
         }
+#pragma unroll
+        for (int c = 0; c < 4; ++c)
+#pragma unroll
+          for (int t2 = 0; t2 < NT; ++t2) o[c4 + c][t2] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(v[c], p[t2], o[c4 + c][t2], 0, 0, 0);
       }
     }
   }
