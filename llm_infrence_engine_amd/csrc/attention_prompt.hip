@@ -165,7 +165,9 @@ attention_prompt_kernel(const bf16* __restrict__ q, size_t q_stride, const bf16*
   const int turns = (t_end - t_begin + KG - 1) / KG;
   for (int turn = 0; turn < turns; ++turn) {
     const int t = t_begin + turn * KG + kg, stage = turn & 1;
-    asm volatile("s_waitcnt vmcnt(0)\n\ts_barrier" ::: "memory");   // this tile has landed; nobody reads the one before it
+    // This tile has landed (vmcnt), and the wave's reads of the one before it have ended (lgkmcnt: what uses them need not
+    // stand before this), so that its place may be filled again.
+    asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");
     if (t + KG < t_end) {
       bring(t + KG, page_next, stage ^ 1);
       page_next = t + 2 * KG < t_end ? page_of(t + 2 * KG) : 0;

@@ -255,8 +255,8 @@ gemm_tiled_kernel(const bf16* __restrict__ A, size_t lda, const bf16* __restrict
       for (int p = 0; p < LOADS_A; ++p) load_a(p, first, first * SLOT_A);
     }
   }
-  if (steps > 1) asm volatile("s_waitcnt vmcnt(%0)\n\ts_barrier" ::"n"(FEWEST_W + FEWEST_A) : "memory");
-  else asm volatile("s_waitcnt vmcnt(0)\n\ts_barrier" ::: "memory");
+  if (steps > 1) asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"(FEWEST_W + FEWEST_A) : "memory");
+  else asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");
 #pragma unroll
   for (int j = 0; j < TT; ++j) read_a(0, j, 0);
 #pragma unroll

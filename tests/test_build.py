@@ -38,6 +38,18 @@ def test_no_kernel_spills_registers_to_memory():
     assert all(v.get("lds", 0) <= 64 * 1024 for v in usage.values())
 
 
+def test_a_written_barrier_waits_for_the_reads_before_it():
+    """A barrier written in assembly, unlike ``__syncthreads``, waits for nothing by itself.  Behind it other waves load into
+    the part of LDS that was read before it, so it has to name the reads (lgkmcnt) beside the loads (vmcnt): the products that
+    use what was read, and the compiler's wait with them, may stand on either side of it."""
+    found = []
+    for src in build.sources():
+        found += [(src.name, text) for text in re.findall(r'asm volatile\("([^"]*)"', src.read_text()) if "s_barrier" in text]
+    assert found
+    for name, text in found:
+        assert re.search(r"s_waitcnt vmcnt\([^)]*\) lgkmcnt\(0\)\\n\\ts_barrier", text), (name, text)
+
+
 def test_a_library_older_than_its_sources_is_built_again_not_loaded(tmp_path, monkeypatch):
     """``load()`` with a stamp that names other sources calls ``build()`` and loads what that returns."""
     import ctypes
