@@ -149,10 +149,15 @@ constexpr bool extra_variant() {
   return !(NT == 1 && WAVES == 16) && !(D == 128 && NT == 1 && WAVES == 8 && VS == 1) && !(NT > 1 && WAVES == 8);
 }
 
+// The narrow tile of the largest head over four waves serves launches of more blocks than CUs, two blocks on a CU: with 260
+// registers a lane in place of 252 there was one (64 tokens of 8 key/value heads behind 30 keys 5.2 -> 8.3 us, behind 150
+// 11.6 -> 15.0), so the number is asked for.
+constexpr bool four_waves_many_tiles(int d, int nt, int waves, int extra) { return d == 128 && nt == 1 && waves == 4 && extra == PLAIN; }
+
 // NARROW: values have fewer dims than keys (a multiple of 16); the tiles of 16 dims past them are neither read nor
 // multiplied, which a branch that is the same for the whole launch decides.
 template <int D, int NT, int WAVES, bool SPLIT, int VS, bool SINK, int EXTRA = PLAIN, bool NARROW = false>
-__global__ void __launch_bounds__(WAVES * MS_WAVE, (NT > 1 && EXTRA != CHANGED && !(NARROW && D == 128) ? 2 : 1))
+__global__ void __launch_bounds__(WAVES * MS_WAVE, ((NT > 1 && EXTRA != CHANGED && !(NARROW && D == 128)) || four_waves_many_tiles(D, NT, WAVES, EXTRA) ? 2 : 1))
 attention_mfma_kernel(const bf16* __restrict__ q, size_t q_stride, const bf16* __restrict__ k_pages,
                       const bf16* __restrict__ vt_pages, const int* __restrict__ block_table, int table_stride,
                       const int* __restrict__ table_rows, const int* __restrict__ q_start,

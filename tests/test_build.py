@@ -36,6 +36,9 @@ def test_no_kernel_spills_registers_to_memory():
     spills = {k: v["scratch"] for k, v in usage.items() if v.get("scratch", 0) > 0}
     assert not spills, f"kernels that spill registers: {spills}"
     assert all(v.get("lds", 0) <= 64 * 1024 for v in usage.values())
+    # launches of more blocks than CUs, of four waves each, that count on a CU holding two of them
+    pairs = {k: v["occupancy"] for k, v in usage.items() if re.search(r"attention_mfma_kernelILi128ELi1ELi4ELb0ELi1ELb[01]ELi0ELb0E", k)}
+    assert len(pairs) == 2 and min(pairs.values()) >= 2, pairs
 
 
 def test_a_written_barrier_waits_for_the_reads_before_it():
