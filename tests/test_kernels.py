@@ -820,6 +820,49 @@ def test_linear_picks_a_kernel_for_every_shape(ops):
             torch.testing.assert_close(got.double(), want, **tol(dtype))
 
 
+@pytest.mark.parametrize("dtype", DTYPES)
+@pytest.mark.parametrize("nh,nkv,d,dv,window,transposed", [(3, 1, 20, 20, None, False), (4, 2, 64, 64, None, True), (2, 2, 18, 70, 150, False),
+                                                           (2, 1, 128, 256, None, True)])
+def test_generic_attention_has_the_same_bits_with_one_wave_and_with_four(ops, dtype, nh, nkv, d, dv, window, transposed):
+    """One wave to a (token, head) or four, as the step's size decides: the same runs of keys merged in the same order, at the
+    edges of a run's blocks of 64 keys and of the four runs; alone in the step and beside others; against 64 bits."""
+    from llm_infrence_engine_amd.kernels import build
+
+    lib = build.load()
+    g = torch.Generator().manual_seed(d + dv)
+    seen, page = [1, 2, 5, 63, 64, 65, 128, 129, 192, 256, 257, 320, 700], 4
+    pages = [-(-n // page) for n in seen]
+    N, P = len(seen), sum(pages) + 1
+    k, v = torch.randn(P, nkv, page, d, generator=g).to(dtype), torch.randn(P, nkv, page, dv, generator=g).to(dtype)
+    k[0] = v[0] = float("nan")
+    table = torch.zeros(N, max(pages), dtype=torch.int32)
+    q = (torch.randn(N, nh * d, generator=g) * 2).to(dtype)
+    want = torch.empty(N, nh, dv, dtype=torch.float64)
+    for r, n in enumerate(seen):
+        at = torch.arange(pages[r]) + 1 + sum(pages[:r])
+        table[r, :pages[r]] = at
+        kk, vv = (x[at].transpose(0, 1).reshape(nkv, -1, x.shape[3])[:, :n].double() for x in (k, v))
+        want[r] = attention_reference(q[r].reshape(nh, 1, d).double(), kk, vv, d ** -0.5, window)[:, 0]
+    vp = (v.transpose(2, 3).contiguous() if transposed else v).to(DEV)
+    rows, pos = torch.arange(N, dtype=torch.int32, device=DEV), torch.tensor(seen, dtype=torch.int32, device=DEV) - 1
+    q, kp, table = q.to(DEV), k.to(DEV), table.to(DEV)
+
+    def run(waves, lo=0, hi=N):
+        out = torch.empty(hi - lo, nh * dv, dtype=dtype, device=DEV)
+        lib.ms_attention_generic_force(waves)
+        try:
+            return ops.paged_attention_generic(q[lo:hi], kp, vp, table, rows[lo:hi], pos[lo:hi], out, nh, d ** -0.5, window,
+                                               v_transposed=transposed)
+        finally:
+            lib.ms_attention_generic_force(0)
+
+    one = run(1)
+    torch.testing.assert_close(one.double().cpu(), want.reshape(N, -1), **tol(dtype))
+    assert torch.equal(one, run(4)) and torch.equal(one, run(0))
+    for r in (0, 4, 9, N - 1):
+        assert torch.equal(one[r:r + 1], run(1, r, r + 1)) and torch.equal(one[r:r + 1], run(4, r, r + 1))
+
+
 def _paged_case(g, dtype, nh, nkv, d, page_size, ctx, qlen, fill):
     """Random requests laid out in shuffled pages (values transposed); returns what the kernels take and
     the plain answer.  Unused slots, the tails of last pages and the null page hold ``fill``."""
