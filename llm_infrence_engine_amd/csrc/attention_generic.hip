@@ -34,7 +34,7 @@ __device__ __forceinline__ void dot4(const float* q, const bf16* k, float& dot) 
 // step.  W = 4, a run to a wave, is for steps that would leave the chip idle: a decode step waits for one token's keys (3 x
 // 14 items behind 135 keys at a head size of 64: 74 us with one wave that kept one run, 9.1 with four).  With W = 1 a wave
 // works its item's runs off by itself and waits for nothing but its own loads: for steps that fill the chip (8 prompts of 64
-// tokens, 14 heads of 64 dims, float: 61.5 us while every item had four waves, 18.3 so; 24 before either).
+// tokens, 14 heads of 64 dims: float 61.5 us while every item had four waves, 23.6 so, bfloat16 86 and 19.3).
 // What bounds it is the latency of a wave's loads: a lane reads its own key's row, the wave one row of values after another.
 // Values are asked for R rows at a time and never behind a condition (each load would be waited for by itself, which was 3
 // of the 7 us of a token with one key): lanes past the value size read its last entry, places past the keys the last row.
