@@ -1,4 +1,4 @@
-// out[M,N] = A[M,K] . W[N,K]^T for up to 16 rows and a narrow W (decode steps: the output and down projections, the
+// out[M,N] = A[M,K] . W[N,K]^T for up to 8 rows and a narrow W (decode steps: the output and down projections, the
 // pieces of the latent and recurrent layers), bfloat16 in, float accumulation (v_mfma_f32_16x16x32_bf16).
 //
 // What bounds these is latency, not memory: a launch is 1.6 us, 224 blocks that read 4 MB, pass one barrier and store take
@@ -87,19 +87,36 @@ gemm_quads_kernel(const void* __restrict__ A, size_t lda, const bf16* __restrict
   }
 }
 
-// Where this kernel is the faster one (us, before against with it, at the 0.5B shapes unless said): a narrow W, whose
-// blocks elsewhere are few and each a chain of four or five dependent loads (896 x 896: 3.9 | 2.8 at one token, 4.0 | 3.4 at
-// 8; 896 x 4864: 6.1 | 5.1, 10.3 | 9.5 at 16; 1792 x 896: 3.9 | 3.0; 2048 x 2048: 5.5 | 4.2), and for up to four tokens
-// wider ones of one round of loads (7296 x 896: 6.3 | 5.4).  Every block reads all the activations, so more tokens pay for
-// less: 5 to 8 of them lose with a long K (896 x 4864: 6.8 | 7.1; ms_gemm_stream, which shares them out through LDS, keeps
-// those), 3 or 4 where a wave needs a second round (896 x 7296: 7.4 | 8.0), and the folded norm, which reads twice the bytes,
-// beyond one round or a wide W (9728 x 896 at 4 tokens: 7.9 | 8.4; 512 x 3584 at 8: 7.6 | 8.1).
-bool pays(int M, int units, int K, bool norm, int cus) {
-  if (K < 256) return false;
-  if (K <= 1024) return units <= (M > 8 ? 1 : norm || M > 4 ? 2 : 8) * cus && !(norm && M > 8);
-  if (norm) return false;
-  if (M <= 4) return units <= 2 * cus && (M <= 2 || K <= 6144);
-  return units <= cus && (M > 8 || K <= 4096);
+// Where this kernel is the faster one (us, before against with it, unless said as before/with).  Narrow matrices gain because
+// their blocks elsewhere are few and each a chain of dependent loads; what costs here is that a wave's load of W takes four
+// k-steps whether it has four or not, and that every block reads all the activations.  `full`: a wave's steps in sixteenths
+// of what its loads could take.
+//   One unit a block (a CU for every block): always but for the shortest rows.  896 x 896 at one token 3.9 | 2.8, at 8 4.0 |
+//     3.4; 896 x 4864 6.1 | 5.1; 256 columns are even to 5 % worse, 264 even to 6 % better; with the norm, which reads twice the
+//     bytes of activations, up to 384 columns 3 to 9 % worse, from 416 on better.
+//   Two units a block: rows whose loads are full enough.  1344 x 512 0.97 to 1.02, x 576 1.04 to 1.15, x 896 1.16 to 1.27,
+//     x 1024 (half full: two steps to each of 16 waves) 0.92 to 1.01, x 2048 1.12 to 1.23, x 2560 0.93 to 1.03, from 3072 on
+//     1.0 to 1.4; where K fills the last step in part, which costs the others more, x 1000 and x 1032 1.05 to 1.15.  5 to 8
+//     tokens pay for one round of loads only (896 x 4864: 6.8 | 7.1), 3 or 4 up to 6144 columns (896 x 7296: 7.4 | 8.0).
+//     With the norm x 576 1.03 to 1.10 at two tokens, at 4 0.96 to 1.03 (x 640 0.98 to 1.06), at 8 from 896 columns on 1.0
+//     to 1.06.
+//   Wider ones, measured up to 8 units a CU: full loads of up to 4 tokens (7296 x 896 6.3 | 5.4; 4100 x 992 1.1 to 1.2, x 640
+//     0.91 to 1.05, x 1000, where 16 waves have two steps each, 0.84 to 0.93; 8192 x 1024 0.6 to 0.7).
+// (9 to 16 tokens stay with ms_gemm_stream and ms_gemm_skinny.)
+bool pays(int M, int units, int K, int waves, int loads, bool norm, int cus) {
+  if (M > 8) return false;
+  const int full = 4 * ((K + 31) / 32) / (waves * loads);
+  if (units <= cus) {
+    if (norm) return K > 384 && K <= 1024;
+    return K > 256 && (M <= 2 || K <= (M <= 4 ? 6144 : 4096));
+  }
+  if (units <= 2 * cus) {
+    const bool part = K % 32 != 0;
+    if (waves == 8) return full >= (norm && M > 4 ? 14 : norm && M > 2 ? 10 : 9);
+    if (K <= 1024) return part || (norm && M > 4);
+    return !norm && M <= 4 && (M <= 2 || K <= 6144) && (part || loads >= 3 || full >= (M > 2 ? 12 : 11));
+  }
+  return units <= 8 * cus && !norm && M <= 4 && waves == 8 && full >= 13;
 }
 
 template <int EPI, typename TO, bool NORM>
@@ -107,11 +124,11 @@ int plan(const void* A, size_t lda, const bf16* W, size_t ldw, const float* bias
          int K, const float* norm_w, float eps, const int* rows, hipStream_t stream) {
   const int cus = ms_compute_units();
   const int units = (N + 3) / 4;
-  if (!pays(M, units, K, NORM, cus)) return MS_UNSUPPORTED;
   // waves as ms_gemm_skinny would take for the shape: the order of the sums goes by them
   const int tiles = (N + 15) / 16, skinny_blocks = tiles <= cus ? tiles : cus * ((tiles + 4 * cus - 1) / (4 * cus));
   const int waves = (tiles + skinny_blocks - 1) / skinny_blocks >= 3 || K <= 992 ? 8 : 16;
   const int loads = ((K + 31) / 32 + 4 * waves - 1) / (4 * waves);   // of W to a wave and unit
+  if (!pays(M, units, K, waves, loads, NORM, cus)) return MS_UNSUPPORTED;
   const int u = units <= cus ? 1 : 2;
   const int rounds = (loads + (u == 1 ? 2 : 1)) / (u == 1 ? 3 : 2);
   const int c = NORM ? 1 : (loads + rounds - 1) / rounds;
@@ -121,16 +138,14 @@ int plan(const void* A, size_t lda, const bf16* W, size_t ldw, const float* bias
         A, lda, W, ldw, bias, out, ldo, M, N, K, norm_w, eps, rows); \
     return ms_launch_status(); \
   }
-#define GO2(CV, UV, GV) GO(8, CV, UV, GV) GO(16, CV, UV, GV)
-  if (M <= 4) { GO2(1, 1, 4) GO2(1, 2, 4) }
-  else if (M <= 8) { GO2(1, 1, 8) GO2(1, 2, 8) }
+  // (those that `pays` can ask for)
+#define ONE(GV) GO(8, 1, 1, GV) GO(16, 1, 1, GV) GO(8, 1, 2, GV) GO(16, 1, 2, GV)
+  if (M <= 4) { ONE(4) } else { ONE(8) }
   if constexpr (!NORM) {
-    if (M <= 4) { GO(16, 2, 1, 4) GO(16, 2, 2, 4) GO(16, 3, 1, 4) }
-    else if (M <= 8) GO(16, 2, 1, 8)
-    else { GO2(1, 1, 16) GO(16, 2, 1, 16) GO(16, 3, 1, 16) }
+    if (M <= 4) { GO(16, 2, 1, 4) GO(16, 3, 1, 4) GO(16, 2, 2, 4) } else { GO(16, 2, 1, 8) }
   }
+#undef ONE
 #undef GO
-#undef GO2
   return MS_UNSUPPORTED;
 }
 
@@ -141,7 +156,6 @@ extern "C" int ms_gemm_quads(const void* A, long long lda, const int* rows, cons
                               const void* W, long long ldw, const float* bias, void* out, long long ldo, int M, int N,
                               int K, int epilogue, int out_dtype, int norm, hipStream_t stream) {
   if (M <= 0 || N <= 0) return MS_OK;
-  if (M > 16) return MS_UNSUPPORTED;
   if (K <= 0 || K % 8 || ldw % 8 || lda < K || ldw < K || lda % (norm ? 4 : 8)) return MS_UNSUPPORTED;
   if (((uintptr_t)A | (uintptr_t)W) % 16 || (norm && ((uintptr_t)norm_w % 16))) return MS_UNSUPPORTED;
   if (norm && !norm_w) return MS_BAD_ARG;

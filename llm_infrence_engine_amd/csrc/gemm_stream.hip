@@ -279,8 +279,8 @@ int plan(const void* A, size_t lda, const bf16* W, size_t ldw, const float* bias
   // stage between the loads and the matrix cores): few rows of W per CU and many columns: the down projection
   // of the 0.5B shape, 896 x 4864, at 8 tokens: 6.8 us against 9.5.  There a block of the other kernel spends its time
   // on the activations, which it reads as MFMA operands, one load a k-step.  Wider or shorter matrices were slower
-  // here by 5 to 30 %.  (ms_gemm_quads is asked first and takes what is left of these but for 5 to 8 tokens beyond 4096
-  // columns, 3 or 4 beyond 6144 and the folded norm: 896 x 4864 at 8 tokens 7.1 there, 512 x 3584 with norm 7.6 here, 8.1 there.)
+  // here by 5 to 30 %.  (ms_gemm_quads is asked first; left here are 5 to 8 tokens beyond 4096 columns, 3 or 4 beyond 6144,
+  // more than 8, and the folded norm: 896 x 4864 at 8 tokens 7.1 there, 512 x 3584 with norm 7.6 here, 8.1 there.)
   if (!any_shape && (units > cus || K < 2048)) return MS_UNSUPPORTED;
   if (units > 16 * cus) return MS_UNSUPPORTED;   // more than 64 rows to a block
   const int blocks = units < cus ? units : cus;

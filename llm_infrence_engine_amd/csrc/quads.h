@@ -5,7 +5,7 @@
 // come: a tile of 16 rows has only four that count, so one load of 64 lanes takes the four rows of FOUR steps (lane
 // 16 kq + 4 i + r: row r, step i, piece kq), and step i's operand is that register turned by 4 i lanes within the rows of
 // 16 lanes: rows 0 to 3 of the tile are the unit's, the others are other steps' values whose products nobody reads.
-// The activations of G = 4, 8 or 16 tokens come in the same way, 16 / G steps to a load.
+// The activations of G = 4 or 8 tokens come in the same way, 16 / G steps to a load.
 #pragma once
 #include "common.h"
 
@@ -84,7 +84,7 @@ struct QuadProduct {
 
   template <int I>
   __device__ __forceinline__ void step(const quad_u32 (&w)[U], const quad_u32 (&x)[XL], const quad_f32 (&f)[XL][2]) {
-    constexpr int J = I / XS, BY = G == 16 ? 0 : (I % XS) * G;
+    constexpr int J = I / XS, BY = (I % XS) * G;
     if constexpr (NORM) {
 #pragma unroll
       for (int e = 0; e < 4; ++e) {

@@ -590,10 +590,11 @@ def test_gemm_stream(ops, M, N, K):
 
 
 @pytest.mark.parametrize("M", [1, 3, 7, 16])
-@pytest.mark.parametrize("N,K", [(898, 6136), (898, 2056), (1030, 264), (2040, 1032), (4100, 1000)])
+@pytest.mark.parametrize("N,K", [(898, 6136), (898, 2056), (1030, 264), (2040, 1032), (4100, 1000), (898, 1000), (514, 424),
+                                 (1030, 584), (2040, 904), (1030, 3080), (2046, 1000), (4100, 904)])
 def test_products_in_units_of_four_rows(ops, M, N, K):
-    """Few rows and a narrow matrix: one or two units of four rows to a block, one to three loads of four k-steps, steps
-    that fill a load in part, a last step that K fills in part, rows that run out inside a unit, strided activations.  A
+    """Few rows and a narrow matrix, on both sides of where it is worth it: one or two units of four rows to a block, 8 and 16
+    waves, one to three loads of four k-steps, steps that fill a load in part, a last step that K fills in part, rows that run out inside a unit, strided activations.  A
     row has the same bits alone and among the rows that go to the tiled kernel; an infinite activation stays in its row.
     Tolerance: float sums of K products of unit variance over another order."""
     g = torch.Generator().manual_seed(M * 1000 + N + K)
