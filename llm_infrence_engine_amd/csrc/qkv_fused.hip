@@ -291,9 +291,13 @@ int launch(const float* X, size_t ldx, const float* norm_w, float eps, const bf1
   while (waves < 8 && blocks * waves < 1024 && steps >= waves * 2) waves *= 2;
   // Units of four rows while one round of loads holds a wave's share (K <= 1024) and there is a CU for every block: the
   // norm reads the activations as floats, once per block.  (At 3584 columns a product of 4608 rows took 14.7 us against
-  // 14.5 at one token, and more tokens cost these blocks more.)
+  // 14.5 at one token, and more tokens cost these blocks more.)  A wave's load takes four k-steps whether it has them or not,
+  // so short rows lose (heads of 32 to 128 dims, 128 to 2048 rows of W, old time / new): 128 columns 0.91 to 0.97, 256 0.85
+  // to 0.98, 384 0.91 to 1.03, 448 0.94 to 1.03 up to 4 tokens and 1.02 to 1.08 beyond, 512 0.98 to 1.11, 640 1.02 to 1.15,
+  // 896 1.09 to 1.28.  Where K fills its last step in part the other blocks pay more: 200 columns 0.99 to 1.17.
   const int few_blocks = (nh + 2 * nkv) * (d / 8);
-  if (M <= 8 && (g_qkv_pair8 == 2 || (g_qkv_pair8 < 0 && K <= 1024 && few_blocks <= ms_compute_units()))) {
+  const bool few_pays = K <= 1024 && few_blocks <= ms_compute_units() && (K >= (M > 4 ? 448 : 512) || (K % 32 && K >= 200));
+  if (M <= 8 && (g_qkv_pair8 == 2 || (g_qkv_pair8 < 0 && few_pays))) {
 #define GO(WV, G) qkv_rope_store_few_kernel<WV, G><<<dim3(d / 8, nh + 2 * nkv), dim3(WV * MS_WAVE), 0, stream>>>(X, ldx, norm_w, eps, W, bias, positions, inv_freq, slot_mapping, q_out, k_pages, v_pages, M, K, nh, nkv, d, page_size, v_transposed)
     if (M <= 4) { if (waves == 4) GO(4, 4); else GO(8, 4); }
     else { if (waves == 4) GO(4, 8); else GO(8, 8); }
