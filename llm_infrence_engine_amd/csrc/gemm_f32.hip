@@ -4,14 +4,15 @@
 // The order of a sum is the same whatever M is, so a token's result does not depend on what else is in the batch: K is
 // cut into at most 16 slices (from K alone, `slice_steps`), a slice is summed 16 values at a time from its start, and the
 // slices are added in order.  Two kernels keep that order:
-//   rows     M <= 64 (a decode step): all waves of a block on the same 4 to 16 rows of W, the slices dealt out over them
-//            and added through LDS.  Bound by reading W.
-//   tiled    more rows: 64 x 64 or 32 x 32 tiles staged through LDS four steps ahead, 4 waves; 32 x 32 where the larger
-//            tiles would be fewer than two a CU.  Bound by the float matrix rate (157 TFLOP/s nominal).
+//   rows     up to 64 rows (a decode step; against very many rows of W up to 16): all waves of a block on the same 4 to 16
+//            rows of W, the slices dealt out over them and added through LDS.  Bound by reading W.
+//   tiled    the others: 64 x 64 or 32 x 32 tiles staged through LDS four steps ahead, 4 waves; 32 x 32 where the larger
+//            tiles would be fewer than two a CU.  Bound by the float matrix rate (157 TFLOP/s nominal), short K by writing C.
 // Measured with the 0.5B sizes against the 64 x 64 vector-ALU tile that ran them before (one MI355X): of 3 rows the down
 // product (896 x 4,864) 319 -> 17 us, gate/up (9,728 x 896) 63 -> 12 us, q/k/v (1,152 x 896) 63 -> 6.3 us, the head
-// (151,936 x 896) 221 -> 100 us; of 338 rows down 316 -> 84 us, gate/up 108 -> 88 us.  Down is bound by the steps a CU
-// works off (16 waves, 19 steps each), whatever its rows; the tiled steps by the way from one barrier to the next.
+// (151,936 x 896) 221 -> 100 us, of 64 rows 252 -> 220; of 338 rows down 316 -> 84 us, gate/up 108 -> 88 us.  Down is bound
+// by the steps a CU works off (16 waves, 19 steps each), whatever its rows; the tiled steps by the way from one barrier to
+// the next.  C leaves a tile through LDS in whole rows (4,096 x 32,000 x 64: 440 us as the fragments lie, 270 so, 261 before).
 #include "common.h"
 #include "api.h"
 
@@ -55,7 +56,8 @@ template <int R, int NT>
 __global__ void __launch_bounds__(MAX_SLICES * MS_WAVE)
 gemm_f32_rows_kernel(const float* __restrict__ A, const float* __restrict__ W, const float* __restrict__ bias,
                      float* C, int M, int N, int K, size_t lda, size_t ldw, size_t ldc, int accumulate) {
-  __shared__ float part[MAX_SLICES][NT * 256];      // [slice][token][row of W]
+  extern __shared__ __align__(16) float part[];      // [slice][token][row of W]
+  constexpr int PART = NT * 256;                     // of a slice
   constexpr int AHEAD = NT == 4 ? 2 : 4;            // steps whose operands are asked for before they are used
   const int lane = threadIdx.x & (MS_WAVE - 1), wave = __builtin_amdgcn_readfirstlane(threadIdx.x / MS_WAVE);
   const int r = lane & 15, g = lane >> 4;
@@ -96,14 +98,14 @@ gemm_f32_rows_kernel(const float* __restrict__ A, const float* __restrict__ W, c
     }
     // the accumulators hold W's row 4 g + i and the token r
 #pragma unroll
-    for (int t = 0; t < NT; ++t) *reinterpret_cast<f32x4*>(&part[slice][(t * 16 + r) * 16 + 4 * g]) = acc[t];
+    for (int t = 0; t < NT; ++t) *reinterpret_cast<f32x4*>(&part[slice * PART + (t * 16 + r) * 16 + 4 * g]) = acc[t];
   }
   __syncthreads();
   for (int e = threadIdx.x; e < NT * 16 * R; e += blockDim.x) {
     const int m = e / R, n = n0 + e % R, at = m * 16 + e % R;
     if (m >= M || n >= N) continue;
-    float v = part[0][at];
-    for (int s = 1; s < slices; ++s) v += part[s][at];
+    float v = part[at];
+    for (int s = 1; s < slices; ++s) v += part[s * PART + at];
     store(C, (size_t)m * ldc + n, v, bias, n, accumulate);
   }
 }
@@ -112,7 +114,7 @@ gemm_f32_rows_kernel(const float* __restrict__ A, const float* __restrict__ W, c
 template <int T>
 __global__ void __launch_bounds__(256)
 gemm_f32_tiled_kernel(const float* __restrict__ A, const float* __restrict__ W, const float* __restrict__ bias,
-                      float* C, int M, int N, int K, size_t lda, size_t ldw, size_t ldc, int accumulate) {
+                      float* C, int M, int N, int K, size_t lda, size_t ldw, size_t ldc, int accumulate, int runs) {
   constexpr int BK = 32, LD = BK + 4;               // rows 36 floats apart: 16 rows' 16-byte reads meet every bank once
   constexpr int F = T / 32, L = T / 32;             // fragments a wave and side, 16-byte loads a thread and operand
   constexpr int AHEAD = 4;                          // steps asked for ahead: one step is 0.1 us of products, a load takes longer
@@ -124,7 +126,7 @@ gemm_f32_tiled_kernel(const float* __restrict__ A, const float* __restrict__ W, 
   const int per = slice_steps(K);
   const int srow = tid >> 3, sk = (tid & 7) * 4;    // what this thread stages: rows srow + 32 i
   f32x4 total[F][F] = {}, acc[F][F] = {};
-  f32x4 wreg[AHEAD][L], areg[AHEAD][L];
+  f32x4 wreg[AHEAD][L] = {}, areg[AHEAD][L] = {};
 
   const float *wrow[L], *arow[L];
 #pragma unroll
@@ -148,7 +150,8 @@ gemm_f32_tiled_kernel(const float* __restrict__ A, const float* __restrict__ W, 
   };
 
 #pragma unroll
-  for (int u = 0; u < AHEAD; ++u) fetch(u, u * BK);
+  for (int u = 0; u < AHEAD; ++u)
+    if (u * BK < K) fetch(u, u * BK);
   put(0, 0, 0);
   __syncthreads();
   int left = per;
@@ -183,36 +186,63 @@ gemm_f32_tiled_kernel(const float* __restrict__ A, const float* __restrict__ W, 
       }
     }
   }
+  // C goes out in rows of the tile (a wave's fragments are 64 bytes of 16 rows each): short K is bound by writing it
+  constexpr int LC = T + 4;
+  float* tile = &lds[0][0][0][0];                   // (nobody reads operands any more)
+  static_assert(T * LC <= 2 * 2 * T * LD, "the tile of C fits where the operands lay");
 #pragma unroll
   for (int i = 0; i < F; ++i)
 #pragma unroll
-    for (int j = 0; j < F; ++j) {
-      total[i][j] += acc[i][j];
-      const int m = m0 + wm + 16 * j + r;
+    for (int j = 0; j < F; ++j)
+      *reinterpret_cast<f32x4*>(&tile[(wm + 16 * j + r) * LC + wn + 16 * i + 4 * g]) = total[i][j] + acc[i][j];
+  __syncthreads();
+  const int c = tid % (T / 4) * 4, n = n0 + c;
 #pragma unroll
-      for (int e = 0; e < 4; ++e) {
-        const int n = n0 + wn + 16 * i + 4 * g + e;
-        if (m < M && n < N) store(C, (size_t)m * ldc + n, total[i][j][e], bias, n, accumulate);
+  for (int p = 0; p < T * T / 1024; ++p) {
+    const int row = tid / (T / 4) + p * (1024 / T), m = m0 + row;
+    if (m >= M) break;
+    f32x4 v = *reinterpret_cast<const f32x4*>(&tile[row * LC + c]);
+    const size_t at = (size_t)m * ldc + n;
+    if (runs && n + 3 < N) {
+      if (bias) {
+#pragma unroll
+        for (int e = 0; e < 4; ++e) v[e] += bias[n + e];
       }
+      if (accumulate) v += *reinterpret_cast<const f32x4*>(C + at);
+      *reinterpret_cast<f32x4*>(C + at) = v;
+    } else {
+#pragma unroll
+      for (int e = 0; e < 4; ++e)
+        if (n + e < N) store(C, at + e, v[e], bias, n + e, accumulate);
     }
+  }
 }
 
+int g_kernel = 0;      // measurements: 1 the kernel of few rows, 2 and 3 the tiled one with tiles of 64 and 32; 0 leaves the choice
+
 }  // namespace
+
+extern "C" void ms_gemm_f32_force(int kernel) { g_kernel = kernel; }
 
 // The caller has checked sizes; K, lda and ldw are multiples of 4 and A and W lie on 16 bytes.
 int ms_gemm_f32_launch(const float* A, const float* W, const float* bias, float* C, int M, int N, int K, size_t lda,
                        size_t ldw, size_t ldc, int accumulate, hipStream_t stream) {
-  if (M <= 64) {
+  const int cus = ms_compute_units();
+  // More than 16 rows against many: every block of the first kernel reads all of A, a tile its part once through LDS.  17 to 32
+  // rows from 64 features a CU on (24 rows of 20,000 x 512 17.2 us there, 15.3 in tiles; 32 of 152,064 x 3,584 1,010 and 519;
+  // of 9,728 x 896 19.3 and 19.1), 33 to 64 from 32 a CU on (64 of 9,728 x 896 33 and 24, of 151,936 x 896 405 and 220, of
+  // 6,144 x 2,048 43 and 40, but 33 of them 33 and 40).
+  const bool few = M <= 16 || (M <= 32 ? N < 64 * cus : M <= 64 && N < 32 * cus);
+  if (g_kernel == 1 ? M <= 64 : g_kernel == 0 && few) {
     // Rows a block: as few as keep the blocks within the CUs, because a CU reads at a rate of its own and 16 bytes a lane
     // fill 64-byte pieces from 4 rows as from 16 (3 rows of 896 x 4,864: 18.3 us as 56 blocks of 16, 17.2 as 224 of 4;
     // q/k/v 6.5 and 6.3).  More tiles than CUs: blocks of four waves, several of them on a CU, instead of one that has a
     // wave for every slice (9,728 x 896: 19.6 us, now 11.9; the head 161, now 100).
-    const int cus = ms_compute_units();
     const int R = (N + 3) / 4 <= cus ? 4 : (N + 7) / 8 <= cus ? 8 : 16;
     const int steps = (K + STEP - 1) / STEP, per = slice_steps(K), slices = (steps + per - 1) / per;
     const int waves = (N + R - 1) / R > cus && slices > 4 ? 4 : slices;
     dim3 grid((N + R - 1) / R), block(waves * MS_WAVE);
-#define ROWS2(R_, NT) gemm_f32_rows_kernel<R_, NT><<<grid, block, 0, stream>>>(A, W, bias, C, M, N, K, lda, ldw, ldc, accumulate)
+#define ROWS2(R_, NT) gemm_f32_rows_kernel<R_, NT><<<grid, block, (size_t)slices * NT * 256 * sizeof(float), stream>>>(A, W, bias, C, M, N, K, lda, ldw, ldc, accumulate)
 #define ROWS(NT) do { if (R == 4) ROWS2(4, NT); else if (R == 8) ROWS2(8, NT); else ROWS2(16, NT); } while (0)
     if (M <= 16) ROWS(1);
     else if (M <= 32) ROWS(2);
@@ -222,9 +252,10 @@ int ms_gemm_f32_launch(const float* A, const float* W, const float* bias, float*
     return ms_launch_status();
   }
   const long long big = (long long)((N + 63) / 64) * ((M + 63) / 64);
-  if (big >= 2 * ms_compute_units())
-    gemm_f32_tiled_kernel<64><<<dim3((N + 63) / 64, (M + 63) / 64), 256, 0, stream>>>(A, W, bias, C, M, N, K, lda, ldw, ldc, accumulate);
+  const int runs = ldc % 4 == 0 && (uintptr_t)C % 16 == 0;
+  if (g_kernel == 2 || (g_kernel != 3 && M > 32 && big >= 2 * cus))
+    gemm_f32_tiled_kernel<64><<<dim3((N + 63) / 64, (M + 63) / 64), 256, 0, stream>>>(A, W, bias, C, M, N, K, lda, ldw, ldc, accumulate, runs);
   else
-    gemm_f32_tiled_kernel<32><<<dim3((N + 31) / 32, (M + 31) / 32), 256, 0, stream>>>(A, W, bias, C, M, N, K, lda, ldw, ldc, accumulate);
+    gemm_f32_tiled_kernel<32><<<dim3((N + 31) / 32, (M + 31) / 32), 256, 0, stream>>>(A, W, bias, C, M, N, K, lda, ldw, ldc, accumulate, runs);
   return ms_launch_status();
 }

@@ -117,7 +117,7 @@ def test_gemm_row_does_not_depend_on_the_batch(ops):
     assert torch.equal(full[40:41], one)
 
 
-@pytest.mark.parametrize("N,K", [(16, 4), (33, 20), (64, 64), (200, 300), (896, 1028), (9728, 896)])
+@pytest.mark.parametrize("N,K", [(16, 4), (33, 20), (64, 64), (200, 300), (896, 1028), (9728, 896), (16500, 64), (32801, 36)])
 def test_float_product_in_the_same_order_for_any_number_of_rows(ops, N, K):
     """Both kernels of the 32-bit product and both of the tiled one's tiles, at the edges of their tiles, as rows of wider
     matrices: within float rounding of 64 bits, and bit for bit the same row whatever is beside it."""
@@ -137,6 +137,8 @@ def test_float_product_in_the_same_order_for_any_number_of_rows(ops, N, K):
         out = torch.empty(hi - lo, N, device=DEV)
         ops.gemm_generic(a[lo:hi], w, out, bias=bias)
         assert torch.equal(out, full[lo:hi]), (lo, hi)
+        ops.gemm_generic(a[lo:hi], w, out, bias=bias, accumulate=True)
+        assert torch.equal(out, 2 * full[lo:hi]), (lo, hi)
 
 
 def rope_reference(x, pos, rot, inv):
