@@ -9,23 +9,18 @@ namespace {
 
 constexpr int BM = 64, BN = 64, BK = 16, PAD = 4;
 
-template <typename T> struct Vec4;
-template <> struct Vec4<float> { typedef float4 type; };
-template <> struct Vec4<bf16> { typedef uint2 type; };
-
-__device__ __forceinline__ void unpack4(const float4& v, float* o) { o[0] = v.x; o[1] = v.y; o[2] = v.z; o[3] = v.w; }
 __device__ __forceinline__ void unpack4(const uint2& v, float* o) {
   o[0] = __uint_as_float(v.x << 16); o[1] = __uint_as_float(v.x & 0xffff0000u);
   o[2] = __uint_as_float(v.y << 16); o[3] = __uint_as_float(v.y & 0xffff0000u);
 }
 
-// Loads 4 consecutive k values of one row into o (zeros outside the matrix).
+// Loads 4 consecutive k values of one row into o (zeros outside the matrix).  VEC: bfloat16 rows in pieces of four.
 template <typename T, bool VEC>
 __device__ __forceinline__ void load4(const T* __restrict__ base, int row, int n_rows, size_t ld, int k, int K, float* o) {
   if (row >= n_rows || k >= K) { o[0] = o[1] = o[2] = o[3] = 0.f; return; }
   const T* p = base + (size_t)row * ld + k;
-  if (VEC) {
-    unpack4(*reinterpret_cast<const typename Vec4<T>::type*>(p), o);
+  if constexpr (VEC) {
+    unpack4(*reinterpret_cast<const uint2*>(p), o);
   } else {
 #pragma unroll
     for (int i = 0; i < 4; ++i) o[i] = (k + i < K) ? to_float(p[i]) : 0.f;
@@ -102,12 +97,11 @@ int launch(const void* A, const void* W, const float* bias, void* C, int M, int 
   if constexpr (sizeof(TA) == 4) {
     if (vec) return ms_gemm_f32_launch((const float*)A, (const float*)W, bias, (float*)C, M, N, K, lda, ldw, ldc, accumulate, stream);
     gemm_generic_kernel<TA, TC, false><<<grid, block, 0, stream>>>((const TA*)A, (const TA*)W, bias, (TC*)C, M, N, K, lda, ldw, ldc, accumulate);
-    return ms_launch_status();
-  }
-  if (vec)
+  } else if (vec) {
     gemm_generic_kernel<TA, TC, true><<<grid, block, 0, stream>>>((const TA*)A, (const TA*)W, bias, (TC*)C, M, N, K, lda, ldw, ldc, accumulate);
-  else
+  } else {
     gemm_generic_kernel<TA, TC, false><<<grid, block, 0, stream>>>((const TA*)A, (const TA*)W, bias, (TC*)C, M, N, K, lda, ldw, ldc, accumulate);
+  }
   return ms_launch_status();
 }
 
