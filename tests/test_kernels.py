@@ -1159,6 +1159,90 @@ def test_attention_mfma_when_the_maximum_keeps_rising(ops, ramp):
     torch.testing.assert_close(got, want, **tol(torch.bfloat16))
 
 
+@pytest.mark.parametrize("nh,nkv,d", [(7, 1, 64), (4, 2, 64), (3, 1, 128), (4, 4, 128)])
+@pytest.mark.parametrize("ramp", [0.5, 6.0, 60.0, -6.0, -60.0])
+def test_attention_of_staged_prompts_when_scores_rise_or_fall(ops, nh, nkv, d, ramp):
+    """Scores that rise or fall along the context by ``ramp`` log2 units in all: the staged kernel's reference follows its first
+    keys up and down, stays, or moves at almost every unit of 32, after several tiles of 64 keys to each group of waves; at 64
+    dims the two groups end with references apart, late keys dwarf the early ones or the other way round."""
+    g = torch.Generator().manual_seed(int(abs(ramp) * 10) + d + nh)
+    ctx, qlen, page = [900, 333, 40], [200, 70, 40], 16
+    c = _paged_case(g, torch.bfloat16, nh, nkv, d, page, ctx, qlen, float("nan"))
+    scale = 1.0 / math.sqrt(d)
+    u = torch.zeros(d); u[5] = 1.0
+    for r in range(len(ctx)):
+        c["qs"][r] = (c["qs"][r].float() * 0.05 + u).to(torch.bfloat16)
+        steps = torch.arange(ctx[r]).float() / ctx[r] * ramp * math.log(2.0) / scale
+        c["ks"][r] = (c["ks"][r].float() * 0.05 + steps[None, :, None] * u).to(torch.bfloat16)
+        for j in range(ctx[r]):
+            c["kp"][c["table"][r, j // page].item(), :, j % page] = c["ks"][r][:, j]
+    want = torch.cat([attention_reference(q.double(), k.double(), v.double(), scale, None).transpose(0, 1).reshape(-1, nh * d)
+                      for q, k, v in zip(c["qs"], c["ks"], c["vs"])])
+    q = torch.cat([x.transpose(0, 1).reshape(-1, nh * d) for x in c["qs"]]).to(DEV)
+    kp, vt, table = c["kp"].to(DEV), c["vt"].to(DEV), c["table"].to(DEV)
+    q_start = torch.tensor([0] + list(np.cumsum(qlen)), dtype=torch.int32, device=DEV)
+    lens, out = torch.tensor(ctx, dtype=torch.int32, device=DEV), torch.empty_like(q)
+    ops._call("ms_attention_prompt", q.data_ptr(), nh * d, kp.data_ptr(), vt.data_ptr(), table.data_ptr(), table.shape[1], None,
+              q_start.data_ptr(), lens.data_ptr(), out.data_ptr(), nh * d, len(ctx), q.shape[0], max(qlen), nh, nkv, d, page,
+              scale, 0, ops._stream())
+    torch.testing.assert_close(out.double().cpu(), want, **tol(torch.bfloat16))
+
+
+@pytest.mark.parametrize("d", [64, 128])
+@pytest.mark.parametrize("R,nkv", [(40, 8), (80, 8)])
+def test_the_choice_of_the_staged_prompt_kernel(ops, d, R, nkv):
+    """Through the call that chooses: prompts beside single tokens, with the most tokens of a request given as a capacity (as
+    a captured step has it) and tokens of nobody behind them; as many blocks as the chip holds at once (40 requests) and more
+    (80).  Eagerly, and captured and replayed with other lengths of the same capacity."""
+    g = torch.Generator().manual_seed(d + R)
+    N, most, nh = 100 * R, 128, nkv
+    assert ops._get("ms_attention_prompt_pays")(R, N, most, 160, nh, nkv, d, 16) == 1
+    scale = 1.0 / math.sqrt(d)
+    cases = []
+    for turn in range(2):
+        qlen = [1 if r % 5 == turn else 60 + (r * 17 + turn * 11) % 40 for r in range(R)]
+        ctx = [n + (r * 7) % 50 for r, n in enumerate(qlen)]
+        c = _paged_case(g, torch.bfloat16, nh, nkv, d, 16, ctx, qlen, float("nan"))
+        want = torch.cat([attention_reference(q.double(), k.double(), v.double(), scale, None).transpose(0, 1).reshape(-1, nh * d)
+                          for q, k, v in zip(c["qs"], c["ks"], c["vs"])])
+        cases.append((qlen, ctx, c, want))
+    P, T = max(c["kp"].shape[0] for *_, c, _ in cases), 160 // 16
+    q, out = torch.zeros(N, nh * d, dtype=torch.bfloat16, device=DEV), torch.zeros(N, nh * d, dtype=torch.bfloat16, device=DEV)
+    kp = torch.zeros(P, nkv, 16, d, dtype=torch.bfloat16, device=DEV)
+    vt = torch.zeros(P, nkv, d, 16, dtype=torch.bfloat16, device=DEV)
+    table = torch.zeros(R, T, dtype=torch.int32, device=DEV)
+    q_start, lens = torch.zeros(R + 1, dtype=torch.int32, device=DEV), torch.zeros(R, dtype=torch.int32, device=DEV)
+
+    def put(qlen, ctx, c):
+        n = sum(qlen)
+        q[:n].copy_(c["q"])
+        kp[:c["kp"].shape[0]].copy_(c["kp"])
+        vt[:c["vt"].shape[0]].copy_(c["vt"])
+        table[:, :c["table"].shape[1]].copy_(c["table"])
+        q_start.copy_(torch.tensor([0] + list(np.cumsum(qlen)), dtype=torch.int32))
+        lens.copy_(torch.tensor(ctx, dtype=torch.int32))
+        out.fill_(3.0)
+        return n
+
+    def run():
+        ops.paged_attention_mfma(q, kp, vt, table, q_start, lens, out, nh, scale, most, 160)
+
+    eager = []
+    for qlen, ctx, c, want in cases:
+        n = put(qlen, ctx, c)
+        run()
+        torch.testing.assert_close(out[:n].double().cpu(), want, **tol(torch.bfloat16))
+        assert (out[n:] == 3.0).all()
+        eager.append(out.clone())
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        run()
+    for turn in (0, 1, 0, 1):
+        put(*cases[turn][:3])
+        graph.replay()
+        assert torch.equal(out, eager[turn])
+
+
 def test_attention_mfma_support_matrix(ops):
     assert ops.attention_mfma_supported(64, 16) and ops.attention_mfma_supported(128, 32)
     assert not ops.attention_mfma_supported(48, 16) and not ops.attention_mfma_supported(64, 8)
