@@ -444,24 +444,25 @@ int g_tile = 0;   // measurements: 0 leaves the choice of tile; 1 to 5 force one
 // The tile that takes the least time by a model of the measurements.  A block of 256 tokens by 256, 192 or 160
 // features has a CU to itself; a step of 64 columns takes 1.6, 1.3 or 1.3 us with all CUs at work, a tile 3 us more for
 // its start and end, and the tiles run in whole rounds over the CUs: the narrower tiles pay where they fill the rounds
-// better (2,048 tokens of the 0.5B gate/up shape: 304 tiles of 256 features take two rounds, 48.6 us; 408 of 192 two
-// shorter ones, 43.0; 1,024 tokens: 25.0 -> 21.9 in one round).  Tiles of 128 x 128 go two to a CU, 1.15 us a step each;
-// they end at different times, so their rounds are counted as they come, plus 0.3 for the last.  Within a tenth of the
-// measured times at 1,024 to 4,096 tokens of the 0.5B and 7B gate/up shapes.
+// better (2,048 tokens of the 0.5B gate/up shape: 304 tiles of 256 features take two rounds, 44.5 us; 408 of 192 two
+// shorter ones, 38.0; 1,024 tokens: 23.2 -> 20.8 in one round).  Tiles of 128 x 128 go two to a CU, 1.15 us a step each;
+// they end at different times, so their rounds are counted as they come, plus 0.3 for the last.  What counts is the order it
+// puts the tiles in: over 83 sizes (128 to 4,096 tokens, 1,024 to 55,296 features, 128 to 5,120 columns) its times run from 28 %
+// below the measured ones (128 columns 63 %) to 40 % above (a round that leaves CUs idle runs at a higher clock), most of them
+// 0 to 17 % above, and the tile it takes is within 5 % of the best one but for five sizes, 23 % behind at worst.
 struct TileChoice { int tile; double us; long long tiles, slots; };
 
 TileChoice choose_tile(int M, int N, int K) {
   const long long cus = ms_compute_units();
   const double steps = (double)((K + BK - 1) / BK);
   const long long small = (long long)((N + 127) / 128) * ((M + 127) / 128);
-  // fewer tiles of 128 x 128 than CUs: tiles of 64 x 64 (four waves) put four times as many CUs to work, and a
-  // tile's time is the time its CU needs to draw its rows (q/k/v of the 0.5B shape, 512 tokens: 11.3 -> 8.7 us;
-  // gate/up at 128 tokens 16.6 -> 12.9, at 256 tokens 16.0 -> 14.9; from 512 tokens on 20.4 against 25.5, all measured
-  // with two buffers)
-  if (small < cus) {
-    const long long tiny = (long long)((N + 63) / 64) * ((M + 63) / 64);
-    return {3, 0.0, tiny, (tiny + 5 * cus - 1) / (5 * cus) * 5 * cus};
-  }
+  // Fewer tiles of 128 x 128 than CUs: tiles of 64 x 64 (four waves) put four times as many CUs to work, and a tile's time is
+  // the time its CU needs to draw its rows; four of them fit a CU (40 KB of LDS each).  Time with 128 over time with 64, at 270
+  // sizes: 0.99 to 1.39 up to two tiles of 64 a CU (gate/up of the 0.5B shape at 160 tokens 9.9 and 8.6 us, 4,096 x 1,024 at
+  // 512 tokens 10.3 and 9.3), and either way from there to four (6,144 x 768 at 640 tokens 10.4 and 12.8, 2,560 x 1,024 at
+  // 1,534 tokens 15.4 and 14.1; 0.88 to 1.28 up to 512 columns, 0.78 to 1.13 up to 1,024, 0.67 to 1.05 beyond).  From the CUs on:
+  // 512 tokens of gate/up 14.6 and 17.1.
+  if (small < cus) return {3, 0.0, (long long)((N + 63) / 64) * ((M + 63) / 64), 4 * cus};
   TileChoice best{2, ((double)small / (double)(2 * cus) + 0.3) * 1.15 * steps, small, (small + 2 * cus - 1) / (2 * cus) * 2 * cus};
   const struct { int tile, features; double step_us; } wide[] = {{1, 256, 1.60}, {4, 192, 1.30}, {5, 160, 1.30}};
   for (const auto& w : wide) {
@@ -480,14 +481,17 @@ extern "C" void ms_gemm_tiled_force_xcd_split(int xm) { g_xcd_split = xm; }
 
 // Whether the gated product of M tokens is faster here than as the library's product and an activation kernel
 // (measured with a different W every call, 65 to 8,192 tokens): up to 1,536 columns always (0.5 to 0.98 of the
-// library's time); beyond that the two are within 15 % of each other either way, and this kernel is taken where it
-// won throughout: up to 2,048 tokens whose tiles fill at least 9/10 of their rounds over the CUs.
+// library's time); beyond that up to 2,048 tokens whose tiles fill at least 9/10 of their rounds over the CUs.  That line is
+// where this kernel won throughout with one barrier and everything drained at it a step; as it is now it takes 0.76 to 0.86 of
+// the library's time there (7B gate/up, 2,048 tokens 413 and 546 us; one row of 55,296 x 5,120, at 1,300 tokens, 1.03), and 0.73
+// to 1.2 on the other side (7B gate/up: 256 tokens 72 and 87, 1,024 tokens 239 and 315, 4,096 tokens 822 and 864; 14,336 x
+// 4,096: 256 tokens 65 and 55, 1,024 tokens 92 and 103).  Tiles of 64 x 64 never.
 extern "C" int ms_gemm_tiled_pays(int M, int N, int K) {
   if (M <= 0 || N <= 0 || K <= 0 || K % BK) return 0;
   if (K <= 1536) return 1;
   if (M > 2048) return 0;
   const TileChoice c = choose_tile(M, N, K);
-  return c.tiles * 10 >= c.slots * 9;
+  return c.tile != 3 && c.tiles * 10 >= c.slots * 9;
 }
 
 // A bfloat16 [M, lda], W bfloat16 [N, ldw] (rows of K, K a multiple of 64), out bfloat16.
@@ -587,6 +591,8 @@ extern "C" int ms_gemm_tiled_qkv(const void* A, long long lda, const void* W, lo
   const size_t ldo = (size_t)nh * head_dim;
   // heads of 128: tiles of 256 features by 128 tokens (with 256 tokens the epilogue no longer fits the registers)
   if (head_dim == 128) return launch<2, 4, 8, 2, EPI_QKV, bf16>(a, lda, w, ldw, o, ldo, M, N, K, stream, e);
+  // (128 x 128, whose epilogue takes longer here, over 64 x 64: 2.0 to 1.08 of the time up to 3 tiles of 64 a CU (1,152 x 896: 1,024
+  // tokens 18.4 and 11.2 us, 2,600 tokens 22.6 and 20.5), 0.81 to 1.23 from there to 4, and 0.78 to 1.05 beyond)
   int tile = g_tile;
   if (tile == 0) tile = choose_tile(M, N, K).tile;
   if (tile == 3) return launch<1, 4, 4, 1, EPI_QKV, bf16>(a, lda, w, ldw, o, ldo, M, N, K, stream, e);

@@ -772,6 +772,31 @@ def test_gemm_tiled(ops, M, N, K, tile):
     assert torch.equal(ops.gemm_tiled(a[M - 70:], w), out[M - 70:])
 
 
+@pytest.mark.parametrize("M,N,K", [(640, 6528, 576), (640, 6530, 576), (65, 32640, 64), (129, 16386, 128)])
+def test_gemm_tiled_on_both_sides_of_its_small_tiles(ops, M, N, K):
+    """Where the choice goes from tiles of 64 x 64 to wider ones (as many tiles of 128 x 128 as CUs): the same bits as with either."""
+    force = ops._get("ms_gemm_tiled_force")
+    force.restype = None
+    g = torch.Generator().manual_seed(M + N)
+    a = torch.randn(M, K, generator=g).bfloat16().to(DEV)
+    w = (torch.randn(N, K, generator=g) / math.sqrt(K)).bfloat16().to(DEV)
+    out, act = ops.gemm_tiled(a, w), ops.gemm_tiled(a, w, ops.EPI_SWIGLU)
+    torch.testing.assert_close(out.double(), a.double() @ w.double().T, **tol(torch.bfloat16))
+    for tile in (2, 3):
+        force(tile)
+        try:
+            assert torch.equal(out, ops.gemm_tiled(a, w)) and torch.equal(act, ops.gemm_tiled(a, w, ops.EPI_SWIGLU))
+        finally:
+            force(0)
+
+
+def test_gemm_tiled_of_long_rows_is_not_taken_for_small_tiles(ops):
+    """Four tiles of 64 x 64 to nearly every CU, which the library's product is faster than: rows that begin on 8 bytes and
+    rows that do not."""
+    for n in (15360, 15362):
+        assert ops._get("ms_gemm_tiled_pays")(256, n, 4096) == 0
+
+
 def test_gemm_tiled_refuses_what_it_cannot_take_and_linear_goes_on(ops):
     from llm_infrence_engine_amd.kernels import linear
 
