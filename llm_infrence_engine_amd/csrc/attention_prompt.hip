@@ -343,23 +343,34 @@ int launch(dim3 grid, dim3 block, const bf16* q, size_t q_stride, const bf16* k,
 }  // namespace
 
 // Whether a step's attention is the faster way here than on ms_paged_attention_mfma (a launch's constants: a captured
-// graph's are its capacities).  A block's time is a chain of tiles of 64 keys, 1.7 us each (two groups at 64 dims: half as
-// many), where the other kernel spreads a tile's keys over four waves: so this one pays once its blocks fill the chip, at
-// 64 dims, where a tile draws half as much, for chains that are short beside the step or contexts that are long.
-// Measured, us, other kernel / this one: 28 heads on 4 of 128 dims, 700 tokens 20.1 / 25.6, 1,024 33 / 30, 2,048 91 / 54,
-// 4,096 318 / 130 (and behind 4,096 more 903 / 353), 4 x 512 41.8 / 25.1, 16 x 100 23.6 / 14.8; 14 heads on 2 of 64 dims,
-// 2,048 tokens 24.3 / 30.9, 3,500 55.1 / 60.1, 4,096 57.9 / 56.4 (behind 4,096 more 143 / 120), 2 x 2,048 39.4 / 42.1,
-// 4 x 512 14.9 / 12.7, 8 x 512 23.5 / 16.3, 16 x 100 11.1 / 8.2.  A single token behind a long context is one block with the
-// whole chain (nine requests with 2,040 tokens and eight of one behind 4,000 keys: 132 / 130 at 128 dims), so in a step of
-// several requests the contexts may be no longer than twice the step.
+// graph's are its capacities).  A block's time is a chain of tiles of 64 keys, 1.9 us each (two groups at 64 dims: half as
+// many), where the other kernel spreads a tile's keys over four waves.  So this one pays once its blocks fill the chip and
+// the step is long beside its longest chain: the last tile of a portion has twice the keys of the mean one where nothing lies
+// before it, fewer than that behind cached keys, so what counts is the blocks a CU times (2 - portion / context), `fills`.
+// A single token behind a long context is one block with the whole chain: in a step of several requests the contexts may be
+// no longer than twice the step.  Time of the other kernel over this one's, at 1,500 steps with 1 to 64 query heads a
+// key/value head times 1 to 16 of those, 1 to 64 requests, contexts up to 14,000 keys (most gain; the ends of each range):
+//   128 dims, from 7/8 of a block a CU on.  One request: 1.0 to 2.4 from fills 1.35 on (28 heads on 4: 2,048 tokens 91 us / 54)
+//     or with at most 400 keys; 0.74 to 1.4 else (4 on 4, 7,777 tokens 183 / 237; 16 on 8, 1,880 tokens 52 / 65).  Several: 0.94
+//     to 2.3 from 1.6 on or with at most 600 keys (400 where one portion has a third of the tokens); 0.70 to 1.5 else.
+//   64 dims, where a tile draws half as much.  One request: 1.06 to 1.54 from 4,096 keys, 1.7 blocks a CU and fills 2.3 on (14 on
+//     2, 4,096 tokens behind 4,096: 143 / 120); 0.94 to 1.3 below.  Several, no portion over a third of the tokens: 0.93 to 1.5
+//     from 7/16 of a block a CU on with contexts of at most 288 keys or 9/8 of the portion, 0.8 to 1.4 with longer ones up to
+//     1.5 blocks a CU (13 requests of up to 307 tokens behind up to 2,577 keys, 16 on 16: 58 / 72), 0.94 to 1.6 above.
 extern "C" int ms_attention_prompt_pays(int n_requests, int n_tokens, int max_q_len, int max_context_len, int num_heads,
                                         int num_kv_heads, int head_dim, int page_size) {
   if ((head_dim != 64 && head_dim != 128) || page_size % 16 || num_kv_heads <= 0) return 0;
   if (n_requests > 1 && (long long)max_context_len > 2LL * n_tokens) return 0;
   const long long blocks = (long long)n_tokens * (num_heads / num_kv_heads) / COLS * num_kv_heads, cus = ms_compute_units();
-  if (head_dim == 128) return blocks * 8 >= cus * 7;
-  if (n_requests == 1) return blocks * 10 >= cus * 17 && max_context_len >= 4096;
-  return blocks * 16 >= cus * 7 && (long long)max_q_len * 3 <= n_tokens;
+  const bool uneven = n_requests == 1 || 3LL * max_q_len > n_tokens;
+  const auto fills = [&](long long twentieths) {
+    return blocks * (2LL * max_context_len - max_q_len) * 20 >= twentieths * cus * max_context_len;
+  };
+  if (head_dim == 128)
+    return blocks * 8 >= cus * 7 && (max_context_len <= (uneven ? 400 : 600) || fills(n_requests == 1 ? 27 : 32));
+  if (n_requests == 1) return blocks * 10 >= cus * 17 && max_context_len >= 4096 && fills(46);
+  const bool short_chains = max_context_len <= 288 || 8LL * max_context_len <= 9LL * max_q_len;
+  return !uneven && blocks * 16 >= cus * (short_chains ? 7 : 24);
 }
 
 // The arguments of ms_paged_attention_mfma's general shape, for plain scores (no sink, cap, slopes, gate; values of the
