@@ -112,7 +112,7 @@ int ms_attention_prompt(const void* q, long long q_stride, const void* k_pages, 
                         long long out_stride, int n_requests, int n_tokens, int max_q_len, int num_heads, int num_kv_heads,
                         int head_dim, int page_size, float scale, int window, hipStream_t stream);
 int ms_attention_prompt_pays(int n_requests, int n_tokens, int max_q_len, int max_context_len, int num_heads, int num_kv_heads,
-                             int head_dim, int page_size);
+                             int head_dim, int page_size, int window);
 int ms_paged_attention_generic(const void* q, long long q_stride, const void* k_pages, const void* v_pages,
                                const int* block_table, int table_stride, const int* table_rows,
                                const int* n_live_tokens, const int* token_req, const int* positions,

@@ -346,7 +346,8 @@ int launch(dim3 grid, dim3 block, const bf16* q, size_t q_stride, const bf16* k,
 // graph's are its capacities).  A block's time is a chain of tiles of 64 keys, 1.9 us each (two groups at 64 dims: half as
 // many), where the other kernel spreads a tile's keys over four waves.  So this one pays once its blocks fill the chip and
 // the step is long beside its longest chain: the last tile of a portion has twice the keys of the mean one where nothing lies
-// before it, fewer than that behind cached keys, so what counts is the blocks a CU times (2 - portion / context), `fills`.
+// before it, fewer than that behind cached keys, so what counts is the blocks a CU times (2 - portion / context), `fills`; with a
+// window all tiles have about its keys.
 // A single token behind a long context is one block with the whole chain: in a step of several requests the contexts may be
 // no longer than twice the step.  Time of the other kernel over this one's, at 1,500 steps with 1 to 64 query heads a
 // key/value head times 1 to 16 of those, 1 to 64 requests, contexts up to 14,000 keys (most gain; the ends of each range):
@@ -358,18 +359,21 @@ int launch(dim3 grid, dim3 block, const bf16* q, size_t q_stride, const bf16* k,
 //     from 7/16 of a block a CU on with contexts of at most 288 keys or 9/8 of the portion, 0.8 to 1.4 with longer ones up to
 //     1.5 blocks a CU (13 requests of up to 307 tokens behind up to 2,577 keys, 16 on 16: 58 / 72), 0.94 to 1.6 above.
 extern "C" int ms_attention_prompt_pays(int n_requests, int n_tokens, int max_q_len, int max_context_len, int num_heads,
-                                        int num_kv_heads, int head_dim, int page_size) {
+                                        int num_kv_heads, int head_dim, int page_size, int window) {
   if ((head_dim != 64 && head_dim != 128) || page_size % 16 || num_kv_heads <= 0) return 0;
   if (n_requests > 1 && (long long)max_context_len > 2LL * n_tokens) return 0;
   const long long blocks = (long long)n_tokens * (num_heads / num_kv_heads) / COLS * num_kv_heads, cus = ms_compute_units();
   const bool uneven = n_requests == 1 || 3LL * max_q_len > n_tokens;
-  const auto fills = [&](long long twentieths) {
-    return blocks * (2LL * max_context_len - max_q_len) * 20 >= twentieths * cus * max_context_len;
-  };
+  long long chain = max_context_len, keys = 2LL * max_context_len - max_q_len;    // of the last tile, of a mean one twice
+  if (window > 0) {
+    chain = std::min<long long>(chain, (long long)window + COLS / std::max(1, num_heads / num_kv_heads));
+    keys = std::min(keys, 2 * std::min<long long>(window, chain));
+  }
+  const auto fills = [&](long long twentieths) { return blocks * keys * 20 >= twentieths * cus * chain; };
   if (head_dim == 128)
-    return blocks * 8 >= cus * 7 && (max_context_len <= (uneven ? 400 : 600) || fills(n_requests == 1 ? 27 : 32));
+    return blocks * 8 >= cus * 7 && (chain <= (uneven ? 400 : 600) || fills(n_requests == 1 ? 27 : 32));
   if (n_requests == 1) return blocks * 10 >= cus * 17 && max_context_len >= 4096 && fills(46);
-  const bool short_chains = max_context_len <= 288 || 8LL * max_context_len <= 9LL * max_q_len;
+  const bool short_chains = chain <= 288 || 8LL * max_context_len <= 9LL * max_q_len;
   return !uneven && blocks * 16 >= cus * (short_chains ? 7 : 24);
 }
 

@@ -1221,7 +1221,7 @@ def test_the_choice_of_the_staged_prompt_kernel(ops, d, R, nkv):
     (80).  Eagerly, and captured and replayed with other lengths of the same capacity."""
     g = torch.Generator().manual_seed(d + R)
     N, most, nh = 100 * R, 128, nkv
-    assert ops._get("ms_attention_prompt_pays")(R, N, most, 160, nh, nkv, d, 16) == 1
+    assert ops._get("ms_attention_prompt_pays")(R, N, most, 160, nh, nkv, d, 16, 0) == 1
     scale = 1.0 / math.sqrt(d)
     cases = []
     for turn in range(2):
@@ -1268,17 +1268,18 @@ def test_the_choice_of_the_staged_prompt_kernel(ops, d, R, nkv):
         assert torch.equal(out, eager[turn])
 
 
-@pytest.mark.parametrize("R,N,most,longest,nh,nkv,d,pays", [
-    (13, 1900, 307, 2884, 16, 16, 64, 0), (57, 2143, 69, 839, 8, 8, 64, 0), (16, 1787, 248, 1171, 16, 8, 64, 0),
-    (8, 1520, 474, 564, 10, 2, 64, 0), (47, 959, 86, 1191, 16, 16, 64, 0), (1, 7571, 7571, 7571, 8, 2, 64, 0),
-    (1, 7777, 7777, 7777, 4, 4, 128, 0), (1, 1880, 1880, 1880, 16, 8, 128, 0), (4, 1902, 1004, 1010, 16, 4, 128, 0),
-    (3, 786, 678, 678, 40, 8, 128, 0),
-    (42, 1919, 88, 88, 8, 8, 64, 1), (32, 1601, 124, 125, 20, 4, 64, 1), (33, 864, 113, 273, 32, 8, 64, 1),
-    (33, 1941, 122, 778, 32, 4, 64, 1), (1, 4096, 4096, 8192, 14, 2, 64, 1), (1, 2048, 2048, 2048, 28, 4, 128, 1),
-    (16, 1600, 100, 100, 28, 4, 128, 1), (4, 2048, 512, 512, 28, 4, 128, 1)])
-def test_staged_prompts_are_taken_where_the_step_is_long_beside_its_longest_chain(ops, R, N, most, longest, nh, nkv, d, pays):
+@pytest.mark.parametrize("R,N,most,longest,nh,nkv,d,window,pays", [
+    (13, 1900, 307, 2884, 16, 16, 64, 0, 0), (57, 2143, 69, 839, 8, 8, 64, 0, 0), (16, 1787, 248, 1171, 16, 8, 64, 0, 0),
+    (8, 1520, 474, 564, 10, 2, 64, 0, 0), (47, 959, 86, 1191, 16, 16, 64, 0, 0), (1, 7571, 7571, 7571, 8, 2, 64, 0, 0),
+    (1, 7777, 7777, 7777, 4, 4, 128, 0, 0), (1, 1880, 1880, 1880, 16, 8, 128, 0, 0), (4, 1902, 1004, 1010, 16, 4, 128, 0, 0),
+    (3, 786, 678, 678, 40, 8, 128, 0, 0),
+    (42, 1919, 88, 88, 8, 8, 64, 0, 1), (32, 1601, 124, 125, 20, 4, 64, 0, 1), (33, 864, 113, 273, 32, 8, 64, 0, 1),
+    (33, 1941, 122, 778, 32, 4, 64, 0, 1), (1, 4096, 4096, 8192, 14, 2, 64, 0, 1), (1, 2048, 2048, 2048, 28, 4, 128, 0, 1),
+    (16, 1600, 100, 100, 28, 4, 128, 0, 1), (4, 2048, 512, 512, 28, 4, 128, 0, 1),
+    (1, 1880, 1880, 1880, 16, 8, 128, 300, 1), (1, 4319, 4319, 4319, 14, 2, 64, 300, 1), (16, 1787, 248, 1171, 16, 8, 64, 500, 0)])
+def test_staged_prompts_are_taken_where_the_step_is_long_beside_its_longest_chain(ops, R, N, most, longest, nh, nkv, d, pays, window):
     """Sizes that the staged kernel was measured on both sides of: those at 0 take 1.05 to 1.3 times as long there."""
-    assert ops._get("ms_attention_prompt_pays")(R, N, most, longest, nh, nkv, d, 16) == pays
+    assert ops._get("ms_attention_prompt_pays")(R, N, most, longest, nh, nkv, d, 16, window) == pays
 
 
 def test_attention_mfma_support_matrix(ops):
