@@ -1260,7 +1260,7 @@ def test_the_choice_of_the_staged_prompt_kernel(ops, d, R, nkv):
         assert (out[n:] == 3.0).all()
         eager.append(out.clone())
     graph = torch.cuda.CUDAGraph()
-    with torch.cuda.graph(graph):
+    with torch.inference_mode(), torch.cuda.graph(graph):     # (as the engine captures: the generator keeps the first mode)
         run()
     for turn in (0, 1, 0, 1):
         put(*cases[turn][:3])
