@@ -417,6 +417,9 @@ int launch(const bf16* A, size_t lda, const bf16* W, size_t ldw, TO* out, size_t
 // The grouped product: tiles of 256 features by 256 rows (TT = 4) or 128 rows (TT = 2), the rows' tiles those of
 // ms_moe_align.  The XCDs are laid over the tiles of W alone (xm = 1), row tiles running fastest on an XCD:
 // neighbouring row tiles mostly belong to one expert and then share its slab of W in that XCD's L2 at the same time.
+// With the loads waited for by count 128 sizes (1 to 100 tiles, 512 to 5,632 features, 256 to 3,584 columns) take 0.72 to 0.94 of
+// the time that everything drained at a barrier a step took: 16 experts of 5,632 x 2,048, 100 tiles of 256 rows 590.8 -> 526.7 us,
+// 2,048 x 2,816, 32 tiles of 128 rows 72.5 -> 61.6.
 constexpr int GROUPED_TT = 4;
 template <typename TO, int TT>
 int launch_grouped(const bf16* A, size_t lda, const bf16* W, TO* out, size_t ldo, int tiles, int N, int K,
