@@ -69,6 +69,14 @@ int ms_gemm_quads(const void* A, long long lda, const int* rows, const float* no
                    long long ldw, const float* bias, void* out, long long ldo, int M, int N, int K, int epilogue,
                    int out_dtype, int norm, hipStream_t stream);
 
+int ms_gemm_ring_pays(int M, int N, int K);
+int ms_gemm_ring(const void* A, long long lda, const int* rows, const float* norm_w, float eps, const void* W,
+                 long long ldw, const float* bias, void* out, long long ldo, int M, int N, int K, int epilogue,
+                 int out_dtype, int norm, int any_shape, hipStream_t stream);
+int ms_gemm_ring_qkv(const float* x, long long ldx, const float* norm_w, float eps, const void* W, const float* bias,
+                     const int* positions, const float* inv_freq, const int* slot_mapping, void* q_out, void* k_pages,
+                     void* v_pages, int M, int K, int num_heads, int num_kv_heads, int head_dim, int page_size,
+                     int v_transposed, hipStream_t stream);
 int ms_gemm_panel(const void* A, long long lda, const int* rows, const float* norm_w, float eps, const void* W,
                    long long ldw, const float* bias, void* out, long long ldo, int M, int N, int K, int epilogue,
                    int out_dtype, int norm, int any_shape, hipStream_t stream);

@@ -253,7 +253,7 @@ int launch_mt(const void* A, size_t lda, const bf16* W, size_t ldw, const float*
 // Tuning knob for measurements: force the block shape (tiles per block, waves) out of (4,4) (4,8) (3,4) (3,8) (2,8)
 // (2,16) (1,8) (1,16), and the 16-token groups per block (1, 2 or 4; further groups go to further blocks), for
 // every later ms_gemm_skinny* launch; zeros give the choice back to the heuristic.  While anything is forced,
-// products of up to 16 rows stay in this kernel instead of going to ms_gemm_quads or ms_gemm_stream.
+// products of up to 16 rows stay in this kernel instead of going to ms_gemm_ring, ms_gemm_quads or ms_gemm_stream.
 extern "C" void ms_gemm_skinny_force(int ntile, int waves, int token_groups) {
   g_force_ntile = ntile;
   g_force_waves = waves;
@@ -268,8 +268,10 @@ extern "C" int ms_gemm_skinny(const void* A, long long lda, const void* W, long 
                               long long ldo, int M, int N, int K, int epilogue, int out_dtype, hipStream_t stream) {
   if (M <= 0 || N <= 0) return MS_OK;
   if (M > 64) return MS_UNSUPPORTED;
-  if (M <= 16 && !forced()) {   // one token group: units of four rows or the streaming kernel, where they take the shape
-    int rc = ms_gemm_quads(A, lda, nullptr, nullptr, 0.f, W, ldw, bias, out, ldo, M, N, K, epilogue, out_dtype, 0, stream);
+  if (M <= 16 && !forced()) {   // one token group: a ring through LDS for a large W, units of four rows or the streaming kernel
+    int rc = ms_gemm_ring(A, lda, nullptr, nullptr, 0.f, W, ldw, bias, out, ldo, M, N, K, epilogue, out_dtype, 0, 0, stream);
+    if (rc != MS_UNSUPPORTED) return rc;
+    rc = ms_gemm_quads(A, lda, nullptr, nullptr, 0.f, W, ldw, bias, out, ldo, M, N, K, epilogue, out_dtype, 0, stream);
     if (rc != MS_UNSUPPORTED) return rc;
     rc = ms_gemm_stream(A, lda, nullptr, nullptr, 0.f, W, ldw, bias, out, ldo, M, N, K, epilogue, out_dtype, 0, 0, stream);
     if (rc != MS_UNSUPPORTED) return rc;
@@ -315,7 +317,9 @@ extern "C" int ms_gemm_skinny_norm(const float* x, long long ldx, const int* row
   if (M <= 0 || N <= 0) return MS_OK;
   if (M > 64) return MS_UNSUPPORTED;
   if (M <= 16 && !forced()) {
-    int rc = ms_gemm_quads(x, ldx, rows, norm_w, eps, W, ldw, bias, out, ldo, M, N, K, epilogue, out_dtype, 1, stream);
+    int rc = ms_gemm_ring(x, ldx, rows, norm_w, eps, W, ldw, bias, out, ldo, M, N, K, epilogue, out_dtype, 1, 0, stream);
+    if (rc != MS_UNSUPPORTED) return rc;
+    rc = ms_gemm_quads(x, ldx, rows, norm_w, eps, W, ldw, bias, out, ldo, M, N, K, epilogue, out_dtype, 1, stream);
     if (rc != MS_UNSUPPORTED) return rc;
     rc = ms_gemm_stream(x, ldx, rows, norm_w, eps, W, ldw, bias, out, ldo, M, N, K, epilogue, out_dtype, 1, 0, stream);
     if (rc != MS_UNSUPPORTED) return rc;

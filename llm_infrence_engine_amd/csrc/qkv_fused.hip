@@ -330,6 +330,11 @@ extern "C" int ms_qkv_rope_store(const float* x, long long ldx, const float* nor
   if (num_heads <= 0 || num_kv_heads <= 0 || page_size <= 0 || !positions || !inv_freq || !slot_mapping || !q_out ||
       !k_pages || !v_pages)
     return MS_BAD_ARG;
+  if (g_qkv_pair8 < 0) {   // a large W: the kernel that rings its rows through LDS
+    const int rc = ms_gemm_ring_qkv(x, ldx, norm_w, eps, W, bias, positions, inv_freq, slot_mapping, q_out, k_pages, v_pages, M, K,
+                                    num_heads, num_kv_heads, head_dim, page_size, v_transposed, stream);
+    if (rc != MS_UNSUPPORTED) return rc;
+  }
 #define GO(MT) return launch<MT>(x, ldx, norm_w, eps, (const bf16*)W, bias, positions, inv_freq, slot_mapping, (bf16*)q_out, (bf16*)k_pages, (bf16*)v_pages, M, K, num_heads, num_kv_heads, head_dim, page_size, v_transposed, stream)
   // the packed projection is narrow (few tile pairs): every 16-token group gets blocks of its own
   GO(1);

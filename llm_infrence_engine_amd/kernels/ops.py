@@ -38,6 +38,9 @@ _SIGNATURES = {
                        _c_ptr],
     "ms_gemm_stream": [_c_ptr, _c_ll, _c_ptr, _c_ptr, _c_float, _c_ptr, _c_ll, _c_ptr, _c_ptr, _c_ll, _c_int, _c_int,
                        _c_int, _c_int, _c_int, _c_int, _c_int, _c_ptr],
+    "ms_gemm_ring": [_c_ptr, _c_ll, _c_ptr, _c_ptr, _c_float, _c_ptr, _c_ll, _c_ptr, _c_ptr, _c_ll, _c_int, _c_int,
+                     _c_int, _c_int, _c_int, _c_int, _c_int, _c_ptr],
+    "ms_gemm_ring_pays": [_c_int, _c_int, _c_int],
     "ms_gemm_panel": [_c_ptr, _c_ll, _c_ptr, _c_ptr, _c_float, _c_ptr, _c_ll, _c_ptr, _c_ptr, _c_ll, _c_int, _c_int,
                       _c_int, _c_int, _c_int, _c_int, _c_int, _c_ptr],
     "ms_gemm_panel_splitk_parts": [_c_int, _c_int, _c_int],
@@ -530,7 +533,7 @@ def gemm_skinny(a: torch.Tensor, w: torch.Tensor, bias: Optional[torch.Tensor] =
     if not gated and epilogue != EPI_RELU2 and split_columns:
         # long rows against few of them (a down projection): the columns are split over blocks too, and the
         # partial sums are added up in a fixed order by a second kernel
-        parts = _get("ms_gemm_panel_splitk_parts")(M, N, K)
+        parts = 0 if _rings(M, N, K) else _get("ms_gemm_panel_splitk_parts")(M, N, K)
         if parts > 1:
             partial = torch.empty((parts, M, N), dtype=torch.float32, device=a.device)
             _call("ms_gemm_panel_splitk", a.data_ptr(), lda, w.data_ptr(), K, _ptr(bias), out.data_ptr(), ldo, M, N, K,
@@ -541,9 +544,15 @@ def gemm_skinny(a: torch.Tensor, w: torch.Tensor, bias: Optional[torch.Tensor] =
     return out
 
 
+def _rings(M: int, N: int, K: int) -> bool:
+    """Whether ``gemm_skinny`` and ``gemm_skinny_norm`` go to the kernel that rings a large matrix through LDS."""
+    return M <= STREAM_MAX_ROWS and bool(_get("ms_gemm_ring_pays")(M, N, K))
+
+
 def splits_columns(a: torch.Tensor, w: torch.Tensor) -> bool:
     """Whether ``gemm_skinny`` spreads the columns of this product over blocks (its sums then pass a second kernel)."""
-    return _get("ms_gemm_panel_splitk_parts")(a.shape[0], w.shape[0], w.shape[1]) > 1
+    (M, K), N = a.shape, w.shape[0]
+    return not _rings(M, N, K) and _get("ms_gemm_panel_splitk_parts")(M, N, K) > 1
 
 
 def gemm_tiled_pays(a: torch.Tensor, w: torch.Tensor) -> bool:
@@ -706,6 +715,16 @@ def gemm_stream(a: torch.Tensor, w: torch.Tensor, bias: Optional[torch.Tensor] =
     residual stream whose RMS norm is folded in.  With ``any_shape`` every shape it can compute is taken;
     a shape it cannot raises."""
     return _gemm_by_name("ms_gemm_stream", a, w, bias, epilogue, out_dtype, residual, norm_weight, eps, rows, any_shape)
+
+
+def gemm_ring(a: torch.Tensor, w: torch.Tensor, bias: Optional[torch.Tensor] = None, epilogue: int = EPI_STORE,
+              out_dtype: torch.dtype = torch.bfloat16, residual: Optional[torch.Tensor] = None,
+              norm_weight: Optional[torch.Tensor] = None, eps: float = 0.0,
+              rows: Optional[torch.Tensor] = None, any_shape: bool = True) -> torch.Tensor:
+    """The kernel that rings a large matrix through LDS past up to 16 rows, called by name (``gemm_skinny`` and
+    ``gemm_skinny_norm`` go to it by themselves for the shapes it is faster on).  Arguments as for ``gemm_stream``; a shape it
+    cannot compute (long rows with a norm that do not fit LDS) raises."""
+    return _gemm_by_name("ms_gemm_ring", a, w, bias, epilogue, out_dtype, residual, norm_weight, eps, rows, any_shape)
 
 
 PANEL_MAX_ROWS = 64

@@ -619,6 +619,72 @@ def test_products_in_units_of_four_rows(ops, M, N, K):
     torch.testing.assert_close(ops.gemm_skinny(b, w, out_dtype=torch.float32)[1:].double(), want[1:M], atol=3e-5, rtol=3e-5)
 
 
+@pytest.mark.parametrize("M", [1, 4, 5, 16])
+@pytest.mark.parametrize("N,K", [(2, 64), (898, 4872), (1030, 264), (5120, 2056), (9728, 904), (4100, 1000), (16 * 256 * 9 + 6, 136),
+                                 (3000, 128), (7168, 2560)])
+def test_gemm_ring(ops, M, N, K):
+    """W ringed through LDS: blocks of two rows and of 146, tiles of 4, 8, 12 and 16 rows, fewer items than waves, tiles that
+    several waves share and waves that hold several tiles, columns that end inside a strip, one strip; every epilogue, the
+    folded norm with gathered rows, strided activations; a row's numbers do not depend on the rest of the batch, and what is
+    not a number stays in its row.  Tolerances: float sums of K products of unit variance over another order."""
+    g = torch.Generator().manual_seed(M * 1000 + N + K)
+    a = torch.randn(M, K + 8, generator=g).bfloat16().to(DEV)[:, :K]
+    w = (torch.randn(N, K, generator=g) / math.sqrt(K)).bfloat16().to(DEV)
+    bias = torch.randn(N, generator=g).to(DEV)
+    want = a.double() @ w.double().T
+    out = ops.gemm_ring(a, w, bias)
+    torch.testing.assert_close(out.double(), want + bias.double(), **tol(torch.bfloat16))
+    f = ops.gemm_ring(a, w, None, out_dtype=torch.float32)
+    torch.testing.assert_close(f.double(), want, atol=3e-5, rtol=3e-5)
+    x = torch.randn(M, N, generator=g).to(DEV)
+    x0 = x.clone()
+    ops.gemm_ring(a, w, bias, ops.EPI_RESIDUAL, residual=x)
+    torch.testing.assert_close(x.double(), x0.double() + want + bias.double(), atol=3e-5, rtol=3e-5)
+    act = ops.gemm_ring(a, w, None, ops.EPI_SWIGLU)
+    torch.testing.assert_close(act.double(), torch.nn.functional.silu(want[:, 0::2]) * want[:, 1::2], **tol(torch.bfloat16))
+    assert torch.equal(ops.gemm_ring(a[M - 1:], w, bias), out[M - 1:])
+    if M > 1:
+        b = a.clone()
+        b[0, K - 1] = float("nan")
+        assert torch.equal(ops.gemm_ring(b, w, bias)[1:], out[1:])
+    xs = torch.randn(M + 3, K, generator=g).to(DEV)
+    nw = (1 + 0.1 * torch.randn(K, generator=g)).to(DEV)
+    rows = torch.randperm(M + 3, generator=g)[:M].to(torch.int32).to(DEV)
+    xr = xs[rows.long()].double()
+    h = (xr * nw.double()).float().bfloat16().double() * torch.rsqrt((xr * xr).mean(-1, keepdim=True) + 1e-5)
+    if M * K > 46000:
+        with pytest.raises(RuntimeError, match="unsupported"):
+            ops.gemm_ring(xs, w, bias, norm_weight=nw, eps=1e-5, rows=rows)
+        return
+    got = ops.gemm_ring(xs, w, bias, out_dtype=torch.float32, norm_weight=nw, eps=1e-5, rows=rows)
+    torch.testing.assert_close(got.double(), h @ w.double().T + bias.double(), atol=2e-4, rtol=2e-4)
+    gated = ops.gemm_ring(xs, w, None, ops.EPI_SWIGLU, norm_weight=nw, eps=1e-5, rows=rows)
+    hw = h @ w.double().T
+    torch.testing.assert_close(gated.double(), torch.nn.functional.silu(hw[:, 0::2]) * hw[:, 1::2], **tol(torch.bfloat16))
+
+
+@pytest.mark.parametrize("M", [1, 4, 9, 16])
+def test_a_large_matrix_goes_to_the_ring(ops, M):
+    """Both sides of the line on values of W, the activations that only these products have, and the front of an attention
+    layer of that size against the separate kernels (values transposed and not)."""
+    g = torch.Generator().manual_seed(M)
+    for N, K in ((12000, 2000), (11990, 2000)):
+        a = torch.randn(M, K, generator=g).bfloat16().to(DEV)
+        w = (torch.randn(N, K, generator=g) / math.sqrt(K)).bfloat16().to(DEV)
+        f = ops.gemm_skinny(a, w, out_dtype=torch.float32)
+        assert torch.equal(f, ops.gemm_ring(a, w, out_dtype=torch.float32)) == (N * K >= 24000000)
+        want = a.double() @ w.double().T
+        torch.testing.assert_close(f.double(), want, atol=3e-5, rtol=3e-5)
+        torch.testing.assert_close(ops.gemm_skinny(a, w, None, ops.EPI_RELU2).double(), want.clamp(min=0) ** 2, **tol(torch.bfloat16))
+        numbers = torch.tensor([1.5, 1.702], device=DEV)
+        gate, up = want[:, 0::2].clamp(max=1.5), want[:, 1::2].clamp(-1.5, 1.5)
+        torch.testing.assert_close(ops.gemm_skinny(a, w, numbers, ops.EPI_CLAMPED).double(), gate * torch.sigmoid(1.702 * gate) * (up + 1),
+                                   **tol(torch.bfloat16))
+    if M * 4608 <= 46000:
+        _qkv_fused_case(ops, M, 32, 5, 128, 4608, True)
+        _qkv_fused_case(ops, M, 72, 5, 64, 4616, False)
+
+
 def test_gemm_stream_refuses_what_it_cannot_take(ops):
     w = torch.zeros(64, 64, dtype=torch.bfloat16, device=DEV)
     with pytest.raises(RuntimeError, match="unsupported"):
