@@ -34,8 +34,11 @@ extern "C" int ms_embed(const int* ids, const void* table, float* out, int n_tok
 // ------------------------------------------------------------------------------------------------
 // Row r of the output is the norm of row rows[r] (or r) of x.  With `delta`, x[row] += delta[row]
 // first (written back), which is the residual sum of the layer before; delta may come as n_partials
-// partial sums [n_partials, N, H], added in order.
+// partial sums [n_partials, N, H], added in order (64 rows with four of them: 896 wide 6.9 -> 3.0 us, 3,584 wide 19.9 -> 4.5, by
+// reading four values at a time and by a thread for each four; the sum into x alone and the norm were 6.3 and 6.4).
 // y = w * (x * rsqrt(mean(x^2) + eps)), all in float, rounded once on store.
+template <typename T> struct alignas(sizeof(T) * 4) Four { T v[4]; };
+
 template <typename T, typename TD>
 __global__ void rms_norm_kernel(float* __restrict__ x, const TD* __restrict__ delta, int n_partials,
                                 size_t partial_stride, const float* __restrict__ w,
@@ -48,12 +51,16 @@ __global__ void rms_norm_kernel(float* __restrict__ x, const TD* __restrict__ de
   float* xr = x + (size_t)src * H;
   T* o = out + (size_t)r * H;
   float ss = 0.f;
-  if (H % 4 == 0 && n_partials == 1 && staged) {  // four values at a time (rows start 16-byte aligned when H % 4 == 0)
+  if (H % 4 == 0 && staged) {  // four values at a time (rows start 16-byte aligned when H % 4 == 0)
     const TD* dr = delta ? delta + (size_t)src * H : nullptr;
     for (int i = threadIdx.x * 4; i < H; i += blockDim.x * 4) {
       float4 v = *reinterpret_cast<const float4*>(xr + i);
       if (dr) {
-        v.x += to_float(dr[i]); v.y += to_float(dr[i + 1]); v.z += to_float(dr[i + 2]); v.w += to_float(dr[i + 3]);
+#pragma unroll 4
+        for (int p = 0; p < n_partials; ++p) {
+          const Four<TD> d = *reinterpret_cast<const Four<TD>*>(dr + p * partial_stride + i);
+          v.x += to_float(d.v[0]); v.y += to_float(d.v[1]); v.z += to_float(d.v[2]); v.w += to_float(d.v[3]);
+        }
         if (write_back) *reinterpret_cast<float4*>(xr + i) = v;
       }
       *reinterpret_cast<float4*>(buf + i) = v;
@@ -64,10 +71,8 @@ __global__ void rms_norm_kernel(float* __restrict__ x, const TD* __restrict__ de
     for (int i = threadIdx.x * 4; i < H; i += blockDim.x * 4) {
       const float4 v = *reinterpret_cast<const float4*>(buf + i);
       const float4 g = *reinterpret_cast<const float4*>(w + i);
-      o[i] = from_float<T>(g.x * (v.x * inv));
-      o[i + 1] = from_float<T>(g.y * (v.y * inv));
-      o[i + 2] = from_float<T>(g.z * (v.z * inv));
-      o[i + 3] = from_float<T>(g.w * (v.w * inv));
+      *reinterpret_cast<Four<T>*>(o + i) = Four<T>{{from_float<T>(g.x * (v.x * inv)), from_float<T>(g.y * (v.y * inv)),
+                                                   from_float<T>(g.z * (v.z * inv)), from_float<T>(g.w * (v.w * inv))}};
     }
     return;
   }
@@ -101,6 +106,7 @@ extern "C" int ms_rms_norm(float* x, const void* delta, int delta_dtype, int n_p
   if (delta && (n_partials < 1 || partial_stride < 0)) return MS_BAD_ARG;
   if (hidden <= 0) return MS_BAD_ARG;
   dim3 grid(n_rows), block(hidden >= 1024 ? 256 : 128);
+  if (n_partials > 1 && hidden % 4 == 0) block = dim3(std::min(1024, (hidden / 4 + 63) / 64 * 64));   // few rows: one round of loads
   // the row is staged in LDS while it fits what a launch may ask for without more ado (64 KB with the 64 bytes
   // of the reduction); a wider row is read from memory a second time instead
   const int staged = (size_t)hidden * sizeof(float) + 64 <= 65536 ? 1 : 0;

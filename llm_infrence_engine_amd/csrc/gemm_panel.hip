@@ -629,3 +629,19 @@ extern "C" int ms_gemm_panel_splitk(const void* A, long long lda, const void* W,
     return run_splitk<EPI_RESIDUAL, float>(a, lda, w, ldw, bias, (float*)out, ldo, M, N, K, (float*)partial, parts, stream);
   return MS_BAD_ARG;
 }
+
+// out (=, +=) the sum of partial sums float [parts, M, N] in part order, + bias: epilogue 0 (out_dtype float or bfloat16) or 3
+// (out float +=).
+extern "C" int ms_add_partials(const float* partial, int parts, const float* bias, void* out, long long ldo, int M, int N,
+                               int epilogue, int out_dtype, hipStream_t stream) {
+  if (M <= 0 || N <= 0) return MS_OK;
+  if (parts < 1 || !partial || ldo < N || (uintptr_t)partial % 16) return MS_BAD_ARG;
+  const dim3 grid((M * ((N + 3) / 4) + 255) / 256), block(256);
+#define GO(EPI, TO) splitk_reduce_kernel<EPI, TO><<<grid, block, 0, stream>>>(partial, parts, bias, (TO*)out, ldo, M, N)
+  if (epilogue == EPI_STORE && out_dtype == MS_BF16) GO(EPI_STORE, bf16);
+  else if (epilogue == EPI_STORE && out_dtype == MS_F32) GO(EPI_STORE, float);
+  else if (epilogue == EPI_RESIDUAL && out_dtype == MS_F32) GO(EPI_RESIDUAL, float);
+  else return MS_BAD_ARG;
+#undef GO
+  return ms_launch_status();
+}

@@ -276,6 +276,10 @@ extern "C" int ms_gemm_skinny(const void* A, long long lda, const void* W, long 
     rc = ms_gemm_stream(A, lda, nullptr, nullptr, 0.f, W, ldw, bias, out, ldo, M, N, K, epilogue, out_dtype, 0, 0, stream);
     if (rc != MS_UNSUPPORTED) return rc;
   }
+  if (!forced() && ms_gemm_slab_parts(M, N, K, 0)) {   // 17 to 64 rows and a W that has to be read from memory
+    const int rc = ms_gemm_slab(A, lda, W, ldw, bias, out, ldo, M, N, K, epilogue, out_dtype, 1, stream);
+    if (rc != MS_UNSUPPORTED) return rc;
+  }
   if (!forced()) {    // the kernel that holds the activations in LDS, where it takes the shape
     const int rc = ms_gemm_panel(A, lda, nullptr, nullptr, 0.f, W, ldw, bias, out, ldo, M, N, K, epilogue, out_dtype, 0, 0, stream);
     if (rc != MS_UNSUPPORTED) return rc;

@@ -88,7 +88,7 @@ def linear(a: torch.Tensor, w: torch.Tensor, bias: Optional[torch.Tensor] = None
            out_dtype: Optional[torch.dtype] = None) -> torch.Tensor:
     """[M, K] x [N, K] -> [M, N] in ``out_dtype`` (default: a's type).  ``a`` may be a ``LazyNorm``."""
     if isinstance(a, LazyNorm):
-        if ops.skinny_norm_ok(a.x, w, a.num_rows) and ops.fold_norm_pays(a.num_rows, a.x.shape[1]):
+        if ops.skinny_norm_ok(a.x, w, a.num_rows) and ops.fold_norm_pays(a.num_rows, a.x.shape[1]) and not ops.slab_pays(a.num_rows, w):
             try:
                 return ops.gemm_skinny_norm(a.x, a.weight, a.eps, w, bias, ops.EPI_STORE, out_dtype or a.out_dtype, a.rows)
             except ops.UnsupportedShape:
@@ -116,10 +116,14 @@ def linear(a: torch.Tensor, w: torch.Tensor, bias: Optional[torch.Tensor] = None
 
 
 def linear_residual(a: torch.Tensor, w: torch.Tensor, bias: Optional[torch.Tensor] = None,
-                    residual: Optional[torch.Tensor] = None) -> Optional[torch.Tensor]:
+                    residual: Optional[torch.Tensor] = None, sums: bool = False) -> Optional[torch.Tensor]:
     """A product that is to be added to the float residual stream.  With few rows the kernel adds it into
     ``residual`` itself (each element by one lane, no atomics) and None is returned; otherwise the product
-    [M, N] is returned for the next norm to add."""
+    [M, N] is returned for the next norm to add; with ``sums`` it may also be float partial sums [parts, M, N]."""
+    if sums and residual is not None and bias is None and a.dtype == torch.bfloat16:
+        partial = ops.gemm_sums(a, w)
+        if partial is not None:
+            return partial
     if residual is not None and a.dtype == torch.bfloat16 and ops.skinny_ok(a, w):
         try:
             ops.gemm_skinny(a, w, bias, ops.EPI_RESIDUAL, residual=residual)
@@ -154,7 +158,8 @@ def linear_swiglu(a: torch.Tensor, w_gate_up: torch.Tensor) -> torch.Tensor:
     """silu(a @ gate.T) * (a @ up.T) for ``w_gate_up`` = interleave_rows(gate, up): [M, I].  ``a`` may be a
     ``LazyNorm``."""
     if isinstance(a, LazyNorm):
-        if ops.skinny_norm_ok(a.x, w_gate_up, a.num_rows) and ops.fold_norm_pays(a.num_rows, a.x.shape[1]):
+        if (ops.skinny_norm_ok(a.x, w_gate_up, a.num_rows) and ops.fold_norm_pays(a.num_rows, a.x.shape[1])
+                and not ops.slab_pays(a.num_rows, w_gate_up)):
             try:
                 return ops.gemm_skinny_norm(a.x, a.weight, a.eps, w_gate_up, None, ops.EPI_SWIGLU, rows=a.rows)
             except ops.UnsupportedShape:

@@ -41,6 +41,11 @@ _SIGNATURES = {
     "ms_gemm_ring": [_c_ptr, _c_ll, _c_ptr, _c_ptr, _c_float, _c_ptr, _c_ll, _c_ptr, _c_ptr, _c_ll, _c_int, _c_int,
                      _c_int, _c_int, _c_int, _c_int, _c_int, _c_ptr],
     "ms_gemm_ring_pays": [_c_int, _c_int, _c_int],
+    "ms_gemm_slab": [_c_ptr, _c_ll, _c_ptr, _c_ll, _c_ptr, _c_ptr, _c_ll, _c_int, _c_int, _c_int, _c_int, _c_int, _c_int, _c_ptr],
+    "ms_gemm_slab_parts": [_c_int, _c_int, _c_int, _c_int],
+    "ms_gemm_slab_qkv": [_c_ptr, _c_ll, _c_ptr, _c_ll, _c_ptr, _c_ptr, _c_ptr, _c_ptr, _c_ptr, _c_ptr, _c_ptr, _c_int, _c_int,
+                         _c_int, _c_int, _c_int, _c_int, _c_int, _c_ptr],
+    "ms_add_partials": [_c_ptr, _c_int, _c_ptr, _c_ptr, _c_ll, _c_int, _c_int, _c_int, _c_int, _c_ptr],
     "ms_gemm_panel": [_c_ptr, _c_ll, _c_ptr, _c_ptr, _c_float, _c_ptr, _c_ll, _c_ptr, _c_ptr, _c_ll, _c_int, _c_int,
                       _c_int, _c_int, _c_int, _c_int, _c_int, _c_ptr],
     "ms_gemm_panel_splitk_parts": [_c_int, _c_int, _c_int],
@@ -533,7 +538,13 @@ def gemm_skinny(a: torch.Tensor, w: torch.Tensor, bias: Optional[torch.Tensor] =
     if not gated and epilogue != EPI_RELU2 and split_columns:
         # long rows against few of them (a down projection): the columns are split over blocks too, and the
         # partial sums are added up in a fixed order by a second kernel
-        parts = 0 if _rings(M, N, K) else _get("ms_gemm_panel_splitk_parts")(M, N, K)
+        parts = _get("ms_gemm_slab_parts")(M, N, K, 0)
+        if parts > 1:
+            partial = _slab_sums(a, w, lda, parts)
+            _call("ms_add_partials", partial.data_ptr(), parts, _ptr(bias), out.data_ptr(), ldo, M, N, epilogue, _code(out_dtype),
+                  _stream())
+            return out
+        parts = 0 if parts or _rings(M, N, K) else _get("ms_gemm_panel_splitk_parts")(M, N, K)
         if parts > 1:
             partial = torch.empty((parts, M, N), dtype=torch.float32, device=a.device)
             _call("ms_gemm_panel_splitk", a.data_ptr(), lda, w.data_ptr(), K, _ptr(bias), out.data_ptr(), ldo, M, N, K,
@@ -552,7 +563,86 @@ def _rings(M: int, N: int, K: int) -> bool:
 def splits_columns(a: torch.Tensor, w: torch.Tensor) -> bool:
     """Whether ``gemm_skinny`` spreads the columns of this product over blocks (its sums then pass a second kernel)."""
     (M, K), N = a.shape, w.shape[0]
-    return not _rings(M, N, K) and _get("ms_gemm_panel_splitk_parts")(M, N, K) > 1
+    parts = _get("ms_gemm_slab_parts")(M, N, K, 0)
+    return parts > 1 if parts else not _rings(M, N, K) and _get("ms_gemm_panel_splitk_parts")(M, N, K) > 1
+
+
+def _slab_sums(a: torch.Tensor, w: torch.Tensor, lda: int, parts: int) -> torch.Tensor:
+    (M, K), N = a.shape, w.shape[0]
+    partial = torch.empty((parts, M, N), dtype=torch.float32, device=a.device)
+    _call("ms_gemm_slab", a.data_ptr(), lda, w.data_ptr(), K, None, partial.data_ptr(), N, M, N, K, EPI_STORE, F32, parts, _stream())
+    return partial
+
+
+def slab_pays(n_rows: int, w: torch.Tensor) -> bool:
+    """Whether a product of so many bfloat16 rows goes to the kernel that takes slabs of a matrix through LDS."""
+    return _get("ms_gemm_slab_parts")(n_rows, w.shape[0], w.shape[1], 0) > 0
+
+
+def gemm_sums(a: torch.Tensor, w: torch.Tensor) -> Optional[torch.Tensor]:
+    """a @ w.T as float partial sums [parts, M, N] over runs of the columns, for a reader that adds them up on its way
+    (``rms_norm``'s ``delta``), where that is the faster way to the product; None: it is not."""
+    if not skinny_ok(a, w):
+        return None
+    (M, K), N = a.shape, w.shape[0]
+    parts = _get("ms_gemm_slab_parts")(M, N, K, 1)
+    if parts <= 1:
+        return None
+    _check(a, "a", torch.bfloat16, contiguous=False)
+    _check(w, "w", torch.bfloat16, (N, a.shape[1]))
+    return _slab_sums(a, w, a.stride(0) if M > 1 else K, parts)
+
+
+def gemm_slab(a: torch.Tensor, w: torch.Tensor, bias: Optional[torch.Tensor] = None, epilogue: int = EPI_STORE,
+              out_dtype: torch.dtype = torch.bfloat16, residual: Optional[torch.Tensor] = None) -> torch.Tensor:
+    """The kernel that takes slabs of a matrix through LDS past up to 64 rows, called by name (``gemm_skinny`` goes to it by
+    itself for the shapes it is faster on).  Arguments as for ``gemm_skinny``."""
+    _check(a, "a", torch.bfloat16, contiguous=False)
+    _check(w, "w", torch.bfloat16)
+    if a.dim() != 2 or a.stride(1) != 1 or w.shape[1] != a.shape[1]:
+        raise ValueError(f"shapes do not fit: a {list(a.shape)} (stride {a.stride()}), w {list(w.shape)}")
+    (M, K), N = a.shape, w.shape[0]
+    gated = epilogue in (EPI_SWIGLU, EPI_CLAMPED)
+    if bias is not None:
+        _check(bias, "bias", torch.float32, (2,) if epilogue == EPI_CLAMPED else (N,))
+    if epilogue == EPI_RESIDUAL:
+        _check(residual, "residual", torch.float32, (M, N))
+        out = residual
+    else:
+        out = torch.empty((M, N // 2 if gated else N), dtype=out_dtype, device=a.device)
+    _call("ms_gemm_slab", a.data_ptr(), a.stride(0) if M > 1 else K, w.data_ptr(), K, _ptr(bias), out.data_ptr(), out.shape[1], M, N,
+          K, epilogue, _code(out.dtype), 1, _stream())
+    return out
+
+
+def gemm_slab_qkv_pays(a, w_qkv: torch.Tensor, head_dim: int, rot_dim: int, k_pages: torch.Tensor) -> bool:
+    """Whether ``gemm_slab_qkv`` takes these normed rows (17 to 64, heads rotated whole): it spares the rotation's launch."""
+    return (isinstance(a, torch.Tensor) and a.dtype == torch.bfloat16 and STREAM_MAX_ROWS < a.shape[0] <= SKINNY_MAX_ROWS
+            and skinny_ok(a, w_qkv) and rot_dim == head_dim and head_dim % 2 == 0 and k_pages.dtype == torch.bfloat16
+            and w_qkv.shape[0] <= 0xffff and w_qkv.numel() < 1 << 31 and max(w_qkv.shape[1], a.stride(0)) <= 1 << 22)
+
+
+def gemm_slab_qkv(a: torch.Tensor, w_qkv: torch.Tensor, bias: Optional[torch.Tensor], num_heads: int, num_kv_heads: int,
+                  head_dim: int, positions: torch.Tensor, inv_freq: torch.Tensor, slot_mapping: torch.Tensor,
+                  k_pages: torch.Tensor, v_pages: torch.Tensor, v_transposed: bool = False) -> torch.Tensor:
+    """a [M <= 64, K] @ w_qkv.T (+ bias), q and k rotated (whole heads, half-split pairs), k and v stored into their pages;
+    returns q [M, num_heads head_dim].  ``qkv_rope_store`` for rows that are normed already."""
+    _check(a, "a", torch.bfloat16, contiguous=False)
+    M, K = a.shape
+    n = num_heads + 2 * num_kv_heads
+    _check(w_qkv, "w_qkv", torch.bfloat16, (n * head_dim, K))
+    _check(positions, "positions", torch.int32, (M,))
+    _check(inv_freq, "inv_freq", torch.float32, (head_dim // 2,))
+    _check(slot_mapping, "slot_mapping", torch.int32, (M,))
+    if bias is not None:
+        _check(bias, "bias", torch.float32, (n * head_dim,))
+    _check(k_pages, "k_pages", torch.bfloat16, (None, num_kv_heads, None, head_dim))
+    _check(v_pages, "v_pages", torch.bfloat16, _v_shape(k_pages, v_transposed))
+    q = torch.empty((M, num_heads * head_dim), dtype=torch.bfloat16, device=a.device)
+    _call("ms_gemm_slab_qkv", a.data_ptr(), a.stride(0) if M > 1 else K, w_qkv.data_ptr(), K, _ptr(bias), positions.data_ptr(),
+          inv_freq.data_ptr(), slot_mapping.data_ptr(), q.data_ptr(), k_pages.data_ptr(), v_pages.data_ptr(), M, K, num_heads,
+          num_kv_heads, head_dim, k_pages.shape[2], int(bool(v_transposed)), _stream())
+    return q
 
 
 def gemm_tiled_pays(a: torch.Tensor, w: torch.Tensor) -> bool:

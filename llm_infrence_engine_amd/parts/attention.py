@@ -174,7 +174,7 @@ class GQAttention(Mixer):
         out = self.rt.empty(ctx.num_tokens, nh * dv)
         ops.paged_attention(q, kv, ctx, out, nh, self.scale, self.window, self.sink_w, self.softcap, self.slopes, None,
                             self.out_scale)
-        return linear.linear_residual(out, self.w_o, self.b_o, x)
+        return linear.linear_residual(out, self.w_o, self.b_o, x, self.hands_on_sums)
 
     def _blending(self, qkv, ctx):
         """{} or the keyword that has the position encoding blend the values with the first such layer's."""

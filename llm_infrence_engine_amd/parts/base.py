@@ -210,6 +210,7 @@ class Norm(Part):
     # ``bias`` (None: none), with ``eps``, and a kernel that has the row at hand may take it itself.  None: only ``forward``.
     statistic: Optional[str] = None
     settles_writes = False      # as ``Block.settles_writes``, of ``forward``'s delta
+    takes_sums = False          # True: the delta of ``forward`` and ``lazy`` may be float partial sums [parts, N, H]
 
     def lazy(self, x: torch.Tensor, delta: Optional[torch.Tensor] = None, rows: Optional[torch.Tensor] = None,
              write_back: bool = True):
@@ -242,6 +243,7 @@ class PositionEncoding(Part):
 
 class Mixer(Part):
     accepts_lazy_norm = False   # True: h may be a LazyNorm that the part hands to kernels.linear
+    hands_on_sums = False       # set by a block whose next norm takes them: ``forward_residual`` may return partial sums
 
     @property
     def graph_safe(self):
@@ -282,6 +284,7 @@ class SequenceFilter(Part):
 
 class FeedForward(Part):
     accepts_lazy_norm = False
+    hands_on_sums = False       # as ``Mixer.hands_on_sums``
 
     def forward(self, h: torch.Tensor, ctx: StepContext) -> torch.Tensor:
         raise NotImplementedError
@@ -308,6 +311,7 @@ class Block(Part):
     # True: ``pending`` may be an object with ``add_into(x)``, a write that is more than an addend (a normed sum, a write into
     # several streams), and the block carries it out with whatever pass it makes; else the model does so first
     settles_writes = False
+    takes_sums = False          # as ``Norm.takes_sums``, of ``pending``; else the model adds them into x first
 
     def __init__(self, **built):
         unknown = set(built) - set(self.takes)

@@ -18,6 +18,12 @@ class PreNormResidual(Block):
              "feed_forward": "feed_forward"}
     optional = ("position",)
 
+    def __init__(self, **built):
+        super().__init__(**built)
+        self.takes_sums = self.mixer_norm.takes_sums
+        self.mixer.hands_on_sums = self.feed_forward_norm.takes_sums
+        self.feed_forward.hands_on_sums = True
+
     def forward(self, x, pending, ctx, kv, state):
         norm = self.mixer_norm.lazy if self.mixer.accepts_lazy_norm else self.mixer_norm.forward
         a = self.mixer.forward_residual(norm(x, delta=pending), ctx, kv, state, x)

@@ -31,7 +31,7 @@ class SwiGLU(FeedForward):
         return self.forward_residual(h, ctx, None)
 
     def forward_residual(self, h, ctx, x):
-        return linear.linear_residual(linear.linear_swiglu(h, self.w_gate_up), self.w_down, None, x)
+        return linear.linear_residual(linear.linear_swiglu(h, self.w_gate_up), self.w_down, None, x, self.hands_on_sums)
 
 
 class DenseAct(FeedForward):

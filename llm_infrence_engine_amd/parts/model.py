@@ -102,7 +102,9 @@ class Model:
                 if pending is not None:      # the pass's addends go into the sum itself
                     from ..kernels import ops
 
-                    pending.add_into(x) if hasattr(pending, "add_into") else ops.residual_add(x, pending)
+                    pending = self._settled(x, pending, None)
+                    if pending is not None:
+                        ops.residual_add(x, pending)
                     pending = None
                 new = self.pass_entry.forward(x, kept, run.opens_pass)
                 x = x if new is None else new
@@ -113,10 +115,18 @@ class Model:
 
     @staticmethod
     def _settled(x, pending, reader):
-        """``pending`` as ``reader`` (a block or the final norm) takes it: a write that is more than an addend is carried out
-        now if the reader does not do that itself."""
-        if hasattr(pending, "add_into") and not reader.settles_writes:
+        """``pending`` as ``reader`` (a block, the final norm, None: somebody who takes one addend) takes it: a write that is
+        more than an addend, or partial sums [parts, *x.shape], are carried out now if the reader does not do that itself."""
+        if hasattr(pending, "add_into"):
+            if reader is not None and reader.settles_writes:
+                return pending
             pending.add_into(x)
+            return None
+        if pending is not None and pending.dim() > x.dim() and not (reader is not None and reader.takes_sums):
+            from ..kernels import ops
+
+            for part in pending:
+                ops.residual_add(x, part)
             return None
         return pending
 

@@ -18,6 +18,7 @@ from .base import Norm, register_part
 
 class RMSNorm(Norm):
     statistic = "rms"
+    takes_sums = True
     bias = None
 
     def __init__(self, prefix: str, size: int, eps: float, offset: float = 0.0, name: str = "weight", gain: float = 1.0):
@@ -73,7 +74,8 @@ class RMSNorm(Norm):
         """As ``forward``, for a consumer that can fold the norm into its first product: with few rows in
         bfloat16 the addend is summed into x now and the normalisation is left to that product."""
         n = x.shape[0] if rows is None else rows.numel()
-        if self.rt.dtype != torch.bfloat16 or n > ops.SKINNY_MAX_ROWS or self.size % 8 or (delta is not None and not write_back):
+        if (self.rt.dtype != torch.bfloat16 or n > ops.SKINNY_MAX_ROWS or self.size % 8
+                or (delta is not None and (not write_back or delta.dim() == 3))):
             return self.forward(x, delta, rows, write_back)
         if delta is not None:
             ops.residual_add(x, delta)

@@ -29,6 +29,9 @@ class RotaryHalf(PositionEncoding):
         self.inv_freq = (1.0 / (self.theta ** (j / self.rotary_dim))).to(torch.float32).to(rt.device)
 
     def project_encode_store(self, h, w_qkv, bias, num_heads, num_kv_heads, head_dim, ctx, kv):
+        if kv is not None and kv.store and ops.gemm_slab_qkv_pays(h, w_qkv, head_dim, self.rotary_dim, kv.k_pages):
+            return ops.gemm_slab_qkv(h, w_qkv, bias, num_heads, num_kv_heads, head_dim, ctx.positions, self.inv_freq,
+                                     kv.slot_mapping, kv.k_pages, kv.v_pages, kv.v_transposed)
         if (kv is not None and kv.store
                 and ops.gemm_tiled_qkv_pays(h, w_qkv, head_dim, self.rotary_dim, kv.k_pages)):
             # a portion of a prompt: rotation and cache store are the product's epilogue; the cosines and sines of

@@ -685,6 +685,108 @@ def test_a_large_matrix_goes_to_the_ring(ops, M):
         _qkv_fused_case(ops, M, 72, 5, 64, 4616, False)
 
 
+@pytest.mark.parametrize("M", [17, 33, 64])
+@pytest.mark.parametrize("N,K", [(2, 64), (6, 8), (898, 1032), (1030, 264), (5120, 520), (16 * 256 * 10 + 6, 136), (2560, 9000),
+                                 (16 * 256 * 10 * 2 + 20, 72)])
+def test_gemm_slab(ops, M, N, K):
+    """Slabs of W through LDS: blocks of fewer rows than a unit and of ten tiles, one slab and three to a CU, fewer items than
+    waves, waves that begin and end inside a slice, columns that end inside a slice; every epilogue, strided activations;
+    a row's numbers do not depend on the rest of the batch, and what is not a number stays in its row.  Tolerances: float sums
+    of K products of unit variance over another order."""
+    g = torch.Generator().manual_seed(M * 1000 + N + K)
+    a = torch.randn(M, K + 8, generator=g).bfloat16().to(DEV)[:, :K]
+    w = (torch.randn(N, K, generator=g) / math.sqrt(K)).bfloat16().to(DEV)
+    bias = torch.randn(N, generator=g).to(DEV)
+    want = a.double() @ w.double().T
+    out = ops.gemm_slab(a, w, bias)
+    torch.testing.assert_close(out.double(), want + bias.double(), **tol(torch.bfloat16))
+    f = ops.gemm_slab(a, w, None, out_dtype=torch.float32)
+    torch.testing.assert_close(f.double(), want, atol=3e-5, rtol=3e-5)
+    x = torch.randn(M, N, generator=g).to(DEV)
+    x0 = x.clone()
+    ops.gemm_slab(a, w, bias, ops.EPI_RESIDUAL, residual=x)
+    torch.testing.assert_close(x.double(), x0.double() + want + bias.double(), atol=3e-5, rtol=3e-5)
+    act = ops.gemm_slab(a, w, None, ops.EPI_SWIGLU)
+    torch.testing.assert_close(act.double(), torch.nn.functional.silu(want[:, 0::2]) * want[:, 1::2], **tol(torch.bfloat16))
+    torch.testing.assert_close(ops.gemm_slab(a, w, None, ops.EPI_RELU2).double(), want.clamp(min=0) ** 2, **tol(torch.bfloat16))
+    numbers = torch.tensor([1.5, 1.702], device=DEV)
+    gate, up = want[:, 0::2].clamp(max=1.5), want[:, 1::2].clamp(-1.5, 1.5)
+    torch.testing.assert_close(ops.gemm_slab(a, w, numbers, ops.EPI_CLAMPED).double(), gate * torch.sigmoid(1.702 * gate) * (up + 1),
+                               **tol(torch.bfloat16))
+    assert torch.equal(ops.gemm_slab(a[M - 17:], w, bias), out[M - 17:])
+    b = a.clone()
+    b[0, K - 1] = float("nan")
+    assert torch.equal(ops.gemm_slab(b, w, bias)[1:], out[1:])
+
+
+@pytest.mark.parametrize("M", [17, 40, 64])
+@pytest.mark.parametrize("N,K", [(896, 896), (900, 1000), (3584, 776), (640, 9000), (10240, 768), (10248, 768), (512, 8192)])
+def test_few_rows_by_a_large_matrix_go_to_slabs(ops, M, N, K):
+    """Both sides of the lines on the size of W and on its rows: partial sums for a reader that adds them up (the RMS norm,
+    against the sum and the norm in double), the plain product and the sum into the residual stream."""
+    g = torch.Generator().manual_seed(M + N + K)
+    a = torch.randn(M, K, generator=g).bfloat16().to(DEV)
+    w = (torch.randn(N, K, generator=g) / math.sqrt(K)).bfloat16().to(DEV)
+    want = a.double() @ w.double().T
+    torch.testing.assert_close(ops.gemm_skinny(a, w, out_dtype=torch.float32).double(), want, atol=3e-5, rtol=3e-5)
+    x = torch.randn(M, N, generator=g).to(DEV)
+    x0 = x.double()
+    ops.gemm_skinny(a, w, None, ops.EPI_RESIDUAL, residual=x)
+    torch.testing.assert_close(x.double(), x0 + want, atol=3e-5, rtol=3e-5)
+    parts = ops.gemm_sums(a, w)
+    assert (parts is not None) == (750000 <= N * K and N <= 10240)
+    if parts is None:
+        return
+    assert parts.shape == (4, M, N)
+    torch.testing.assert_close(parts.double().sum(0), want, atol=3e-5, rtol=3e-5)
+    x = x0.float()
+    nw = (1 + 0.1 * torch.randn(N, generator=g)).to(DEV)
+    rows = torch.randperm(M, generator=g)[:M - 3].to(torch.int32).to(DEV)
+    total = x0 + want
+    normed = total * torch.rsqrt((total * total).mean(-1, keepdim=True) + 1e-6) * nw.double()
+    some = ops.rms_norm(x, nw, 1e-6, torch.empty(M - 3, N, dtype=torch.bfloat16, device=DEV), delta=parts, rows=rows, write_back=False)
+    torch.testing.assert_close(some.double(), normed[rows.long()], **tol(torch.bfloat16))
+    assert torch.equal(x, x0.float())
+    h = ops.rms_norm(x, nw, 1e-6, torch.empty(M, N, dtype=torch.bfloat16, device=DEV), delta=parts)
+    torch.testing.assert_close(h.double(), normed, **tol(torch.bfloat16))
+    torch.testing.assert_close(x.double(), total, atol=3e-5, rtol=3e-5)
+
+
+@pytest.mark.parametrize("M", [17, 48, 64])
+@pytest.mark.parametrize("nh,nkv,d,K,v_transposed", [(14, 2, 64, 896, True), (5, 1, 128, 520, False), (3, 3, 6, 72, False), (70, 5, 64, 136, True)])
+def test_gemm_slab_qkv_equals_product_rotation_and_store(ops, M, nh, nkv, d, K, v_transposed):
+    """The front of an attention layer of 17 to 64 normed rows against a double product and the plain rotation: heads that
+    straddle a unit of four rows and blocks, a token that is not stored, pages plain and transposed."""
+    g = torch.Generator().manual_seed(M + d + K)
+    page_size, pages = 16, 6
+    n = nh + 2 * nkv
+    a = torch.randn(M, K, generator=g).bfloat16().to(DEV)
+    w = (torch.randn(n * d, K, generator=g) / math.sqrt(K)).bfloat16().to(DEV)
+    bias = torch.randn(n * d, generator=g).to(DEV)
+    pos = torch.randint(0, 3000, (M,), generator=g).to(torch.int32).to(DEV)
+    slots = torch.randperm(pages * page_size, generator=g)[:M].to(torch.int32)
+    slots[2] = -1
+    slots = slots.to(DEV)
+    inv_freq = (1.0 / (1e6 ** (torch.arange(0, d, 2, dtype=torch.float64) / d))).float().to(DEV)
+    kp = torch.zeros(pages, nkv, page_size, d, dtype=torch.bfloat16, device=DEV)
+    vp = torch.zeros((pages, nkv, d, page_size) if v_transposed else (pages, nkv, page_size, d), dtype=torch.bfloat16, device=DEV)
+    q = ops.gemm_slab_qkv(a, w, bias, nh, nkv, d, pos, inv_freq, slots, kp, vp, v_transposed)
+    exact = (a.double() @ w.double().T + bias.double()).view(M, n, d).cpu()
+    rot = rope_reference(exact[:, :nh + nkv], pos.cpu(), d, inv_freq.double().cpu())
+    torch.testing.assert_close(q.double().cpu().view(M, nh, d), rot[:, :nh], atol=3e-2, rtol=1.6e-2)
+    for t in range(M):
+        s = int(slots[t])
+        if s < 0:
+            continue
+        p, o = divmod(s, page_size)
+        torch.testing.assert_close(kp[p, :, o].double().cpu(), rot[t, nh:], atol=3e-2, rtol=1.6e-2)
+        v = vp[p, :, :, o] if v_transposed else vp[p, :, o]
+        torch.testing.assert_close(v.double().cpu(), exact[t, nh + nkv:], atol=3e-2, rtol=1.6e-2)
+    untouched = torch.ones(pages * page_size, dtype=torch.bool)
+    untouched[slots[slots >= 0].long().cpu()] = False
+    assert (kp.permute(0, 2, 1, 3).reshape(pages * page_size, -1)[untouched.to(DEV)] == 0).all()
+
+
 def test_gemm_stream_refuses_what_it_cannot_take(ops):
     w = torch.zeros(64, 64, dtype=torch.bfloat16, device=DEV)
     with pytest.raises(RuntimeError, match="unsupported"):
