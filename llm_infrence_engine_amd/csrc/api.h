@@ -103,6 +103,9 @@ int ms_gemm_tiled(const void* A, long long lda, const void* W, long long ldw, vo
                   int K, int epilogue, float limit, float alpha, hipStream_t stream);
 void ms_gemm_tiled_force(int tile);
 void ms_gemm_tiled_force_xcd_split(int xm);   // measurements: rows of XCDs over the tiles (1, 2, 4, 8); 0 leaves the choice
+int ms_gemm_tiled_sums_parts(int M, int N, int K);   // partial sums over runs of the columns: float [parts, M, N]; 0: not for it
+int ms_gemm_tiled_sums(const void* A, long long lda, const void* W, long long ldw, float* partial, int M, int N, int K, int parts,
+                       hipStream_t stream);
 int ms_gemm_tiled_pays(int M, int N, int K);
 int ms_gemm_tiled_plain_pays(int M, int N, int K);   // the same question for a plain product (epilogue 0)
 

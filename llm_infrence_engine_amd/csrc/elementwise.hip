@@ -106,7 +106,8 @@ extern "C" int ms_rms_norm(float* x, const void* delta, int delta_dtype, int n_p
   if (delta && (n_partials < 1 || partial_stride < 0)) return MS_BAD_ARG;
   if (hidden <= 0) return MS_BAD_ARG;
   dim3 grid(n_rows), block(hidden >= 1024 ? 256 : 128);
-  if (n_partials > 1 && hidden % 4 == 0) block = dim3(std::min(1024, (hidden / 4 + 63) / 64 * 64));   // few rows: one round of loads
+  // a thread for every four values where every row has a CU of its own and several sums are read: one round of loads
+  if (n_partials > 1 && hidden % 4 == 0 && n_rows <= ms_compute_units()) block = dim3(std::min(1024, (hidden / 4 + 63) / 64 * 64));
   // the row is staged in LDS while it fits what a launch may ask for without more ado (64 KB with the 64 bytes
   // of the reduction); a wider row is read from memory a second time instead
   const int staged = (size_t)hidden * sizeof(float) + 64 <= 65536 ? 1 : 0;

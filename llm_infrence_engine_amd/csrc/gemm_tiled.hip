@@ -31,7 +31,7 @@ typedef __attribute__((ext_vector_type(4))) float f32x4;
 
 // beside the epilogues of common.h (without EPI_RESIDUAL): the q/k/v product's, the grouped product's, and EPI_SWIGLU with
 // the tanh form of the gelu for the silu
-enum { EPI_QKV = 2, EPI_GROUPED = 7, EPI_GEGLU = 4 };
+enum { EPI_QKV = 2, EPI_GROUPED = 7, EPI_GEGLU = 4, EPI_SUMS = 8 };
 
 // the gate's activation of a gated epilogue: g * sigmoid(g), or the tanh form of the gelu with the tanh as
 // 1 - 2 / (2^(2 y log2 e) + 1) through the hardware's exp2 and reciprocal (the result is rounded to bfloat16)
@@ -114,8 +114,8 @@ __device__ __forceinline__ void store_run_f32(float* o, const float* v, int run,
 template <int WF, int WT, int FT, int TT, int EPI, typename TO>
 __global__ void __launch_bounds__(WF * WT * MS_WAVE)
 gemm_tiled_kernel(const bf16* __restrict__ A, size_t lda, const bf16* __restrict__ W, size_t ldw,
-                  TO* __restrict__ out, size_t ldo, int M, int N, int K, int m_tiles, int n_tiles, int xm, QkvEpilogue qkv,
-                  GroupedRows grp) {
+                  TO* __restrict__ out, size_t ldo, int M, int N, int K, int m_tiles, int n_tiles, int xm, int parts,
+                  QkvEpilogue qkv, GroupedRows grp) {
   constexpr int NWAVES = WF * WT, THREADS = NWAVES * MS_WAVE;
   constexpr int BN = WF * FT * 16, BM = WT * TT * 16;
   static_assert(BN % 8 == 0 && BM % 8 == 0, "a load brings eight rows");
@@ -130,10 +130,29 @@ gemm_tiled_kernel(const bf16* __restrict__ A, size_t lda, const bf16* __restrict
   // running fastest (they share a tile of W at the same time).  With xm = 1 a tile of W is read from memory by
   // one XCD only and every XCD reads all of A; a larger xm leaves an XCD 1 / xm of A to keep in its L2.  The host
   // launches 8 * ceil(m_tiles / xm) * ceil(n_tiles / (8 / xm)) blocks; one without a tile leaves.
-  const int xcd = blockIdx.x & 7, local = (int)(blockIdx.x >> 3);
+  const int xcd = blockIdx.x & 7;
+  const int local = (int)(blockIdx.x >> 3);
   const int xn = 8 / xm, mi = (m_tiles + xm - 1) / xm;
-  const int nt = (local / mi) * xn + xcd / xm;
-  const int mt = (local % mi) * xm + xcd % xm;
+  int steps = K / BK;
+  int nt = 0, mt = 0;
+  if (EPI == EPI_SUMS) {
+    // a run of the columns: the parts one after the other, each with all tiles, dealt out over the XCDs in equal runs (there is
+    // about a block for every CU: by rows of tiles, 14 over 8 XCDs, some CUs would get two and others none)
+    const int all = m_tiles * n_tiles * parts, per = (all + 7) / 8, id = xcd * per + local;
+    if (local >= per || id >= all) return;
+    const int part = id / (m_tiles * n_tiles), tile = id - part * (m_tiles * n_tiles);
+    nt = tile / m_tiles;
+    mt = tile - nt * m_tiles;
+    const int from = (int)((long long)steps * part / parts), to = (int)((long long)steps * (part + 1) / parts);
+    steps = to - from;
+    A += (size_t)from * BK;
+    W += (size_t)from * BK;
+    out += (size_t)part * M * N;
+  }
+  if (EPI != EPI_SUMS) {
+    nt = (local / mi) * xn + xcd / xm;
+    mt = (local % mi) * xm + xcd % xm;
+  }
   if (nt >= n_tiles || mt >= m_tiles) return;
   const int n0 = nt * BN, m0 = mt * BM;
   if (EPI == EPI_GROUPED) {     // the token tile is a tile of one expert's rows: its matrix is the W of this block
@@ -245,7 +264,6 @@ gemm_tiled_kernel(const bf16* __restrict__ A, size_t lda, const bf16* __restrict
       }
     }
   };
-  const int steps = K / BK;
 #pragma unroll
   for (int first = 0; first < 2; ++first) {
     if (first < steps) {
@@ -373,6 +391,11 @@ gemm_tiled_kernel(const bf16* __restrict__ A, size_t lda, const bf16* __restrict
       for (int g = 0; g < 4 * FT; ++g) v[g] = grp.act ? tiled_gelu_erf(acc[g >> 2][j][g & 3]) : acc[g >> 2][j][g & 3];
       if (sizeof(TO) == 4) store_run_f32(reinterpret_cast<float*>(out) + row * ldo + f0, v, 4 * FT, N - f0);
       else store_run<4 * FT>(reinterpret_cast<bf16*>(out) + row * ldo + f0, v, N - f0);
+    } else if (EPI == EPI_SUMS) {
+      float v[4 * FT];
+#pragma unroll
+      for (int g = 0; g < 4 * FT; ++g) v[g] = acc[g >> 2][j][g & 3];
+      store_run_f32(reinterpret_cast<float*>(out) + (size_t)m * ldo + f0, v, 4 * FT, N - f0);
     } else {
       float v[4 * FT];
 #pragma unroll
@@ -395,7 +418,7 @@ int choose_xcd_split(int M) {
 
 template <int WF, int WT, int FT, int TT, int EPI, typename TO>
 int launch(const bf16* A, size_t lda, const bf16* W, size_t ldw, TO* out, size_t ldo, int M, int N, int K,
-           hipStream_t stream, const QkvEpilogue& qkv = QkvEpilogue{}, const GroupedRows& grp = GroupedRows{}) {
+           hipStream_t stream, const QkvEpilogue& qkv = QkvEpilogue{}, const GroupedRows& grp = GroupedRows{}, int parts = 1) {
   constexpr int BN = WF * FT * 16, BM = WT * TT * 16;
   constexpr size_t lds = (size_t)(3 * BN + 2 * BM) * PITCH * sizeof(bf16);
   static bool raised = false;   // once per instantiation: allow more dynamic LDS than the default 64 KB
@@ -407,10 +430,11 @@ int launch(const bf16* A, size_t lda, const bf16* W, size_t ldw, TO* out, size_t
   }
   const int n_tiles = (N + BN - 1) / BN, m_tiles = (M + BM - 1) / BM;
   const int xm = choose_xcd_split(M);
-  const long long blocks = 8LL * ((m_tiles + xm - 1) / xm) * ((n_tiles + 8 / xm - 1) / (8 / xm));
+  const long long blocks = EPI == EPI_SUMS ? ((long long)m_tiles * n_tiles * parts + 7) / 8 * 8
+                                           : 8LL * ((m_tiles + xm - 1) / xm) * ((n_tiles + 8 / xm - 1) / (8 / xm));
   if (blocks > 0x7fffffffLL) return MS_UNSUPPORTED;
   gemm_tiled_kernel<WF, WT, FT, TT, EPI, TO><<<dim3((unsigned)blocks), dim3(WF * WT * MS_WAVE), lds, stream>>>(
-      A, lda, W, ldw, out, ldo, M, N, K, m_tiles, n_tiles, xm, qkv, grp);
+      A, lda, W, ldw, out, ldo, M, N, K, m_tiles, n_tiles, xm, parts, qkv, grp);
   return ms_launch_status();
 }
 
@@ -438,7 +462,7 @@ int launch_grouped(const bf16* A, size_t lda, const bf16* W, TO* out, size_t ldo
   const long long blocks = 8LL * tiles * ((n_tiles + 7) / 8);
   if (blocks > 0x7fffffffLL) return MS_UNSUPPORTED;
   gemm_tiled_kernel<WF, WT, FT, TT, EPI_GROUPED, TO><<<dim3((unsigned)blocks), dim3(WF * WT * MS_WAVE), lds, stream>>>(
-      A, lda, W, (size_t)K, out, ldo, tiles * BM, N, K, tiles, n_tiles, 1, QkvEpilogue{}, grp);
+      A, lda, W, (size_t)K, out, ldo, tiles * BM, N, K, tiles, n_tiles, 1, 1, QkvEpilogue{}, grp);
   return ms_launch_status();
 }
 
@@ -475,6 +499,32 @@ TileChoice choose_tile(int M, int N, int K) {
     const long long rounds = (tiles + cus - 1) / cus;
     const double us = (double)rounds * (3.0 + steps * w.step_us);
     if (us < best.us) best = {w.tile, us, tiles, rounds * cus};
+  }
+  return best;
+}
+
+// Tile and column parts of a product in partial sums, the least time by a model of the measurements: a start and a step of 64
+// columns by how many blocks share a CU (by how many CUs are at work, for tiles of 256), rounds over the CUs, and a write and a
+// read of every sum at 5 TB/s.
+struct SumsChoice { int tile, parts; double us; long long blocks; };
+
+SumsChoice choose_sums(int M, int N, int K) {
+  const long long cus = ms_compute_units();
+  const int steps = K / BK;
+  const struct { int tile, size, to_a_cu; double start_us[4], step_us[4]; } kinds[] = {
+      {1, 256, 1, {12.}, {1.05}}, {2, 128, 2, {9., 13.}, {0.55, 1.0}}, {3, 64, 4, {7., 7., 7., 8.}, {0.30, 0.43, 0.63, 0.82}}};
+  SumsChoice best{0, 1, 1e30, 0};
+  for (const auto& k : kinds) {
+    const long long tiles = (long long)((N + k.size - 1) / k.size) * ((M + k.size - 1) / k.size), slots = cus * k.to_a_cu;
+    for (int p = 1; p <= 8 && (p == 1 || p * 4 <= steps); ++p) {
+      const long long blocks = tiles * p;
+      const int at = (int)(blocks >= slots ? k.to_a_cu : (blocks + cus - 1) / cus) - 1;
+      double rounds = (double)((blocks + slots - 1) / slots);
+      if (k.to_a_cu > 1 && rounds > 1) rounds = (double)blocks / (double)slots + 0.3;
+      const double step = k.step_us[at] + (k.to_a_cu == 1 ? 0.5 * (double)(blocks < cus ? blocks : cus) / (double)cus : 0.);
+      const double us = rounds * (k.start_us[at] + (steps + p - 1) / p * step) + (double)p * M * N * 8 / 5e6;
+      if (us < best.us) best = {k.tile, p, us, blocks};
+    }
   }
   return best;
 }
@@ -528,6 +578,43 @@ extern "C" int ms_gemm_tiled(const void* A, long long lda, const void* W, long l
   if (tile == 4) GO(2, 4, 6, 4);   // 192 features x 256 tokens
   if (tile == 5) GO(2, 4, 5, 4);   // 160 features x 256 tokens
   GO(2, 4, 4, 2);                  // 128 x 128
+#undef GO
+}
+
+// Column parts for a product whose reader adds partial sums up itself (the norm that follows a down projection), 0 where the
+// library's product, or this kernel's whole one, is the faster way.  Few features leave a product of whole columns fewer
+// tiles than CUs: 2,048 tokens by 3,584 x 18,944 are 112 tiles of 256 for 256 CUs; in two parts 235 us + 30 for the norm that adds
+// them up, the library 363 + 17.  Time of the library and its norm over this, 65 to 4,096 tokens, 14 sizes of W (896 x 896 to
+// 5,120 x 27,648):
+//   up to 128 tokens 1.06 to 2.7;
+//   up to 512 tokens by rows of 4,096 columns and more 0.97 to 2.6 (896 x 4,864 at 390 tokens 21.4 and 18.8 us), by rows of up to
+//   1,024 1.1 to 1.25, between these 0.89 to 1.6;
+//   up to 1,024 tokens by 8,192 columns and more 0.98 to 1.55, by fewer 0.84 to 1.15;
+//   beyond, by 16,384 columns and more where one round of blocks in parts fills 5/6 of the CUs, 1.4 to 1.57 (4,096 x 28,672 at
+//   2,048 tokens, all CUs, 0.96); elsewhere the library mostly wins (0.65 to 1.54).
+extern "C" int ms_gemm_tiled_sums_parts(int M, int N, int K) {
+  if (M <= 64 || N <= 0 || K < 768 || K % BK || N > 8192) return 0;
+  const SumsChoice c = choose_sums(M, N, K);
+  if (M <= 128 || (M <= 512 && (K >= 4096 || K <= 1024)) || (M <= 1024 && K >= 8192)) return c.parts;
+  const int cus = ms_compute_units();
+  return K >= 16384 && c.tile == 1 && c.parts > 1 && c.blocks < cus && c.blocks * 6 >= cus * 5 ? c.parts : 0;
+}
+
+// Partial sums of the plain product over `parts` runs of the columns: float [parts, M, N].
+extern "C" int ms_gemm_tiled_sums(const void* A, long long lda, const void* W, long long ldw, float* partial, int M, int N, int K,
+                                  int parts, hipStream_t stream) {
+  if (M <= 0 || N <= 0) return MS_OK;
+  if (K <= 0 || K % BK || lda % 8 || ldw % 8 || lda < K || ldw < K) return MS_UNSUPPORTED;
+  if (((uintptr_t)A | (uintptr_t)W | (uintptr_t)partial) % 16) return MS_UNSUPPORTED;
+  if (parts < 1 || parts > K / BK) return MS_BAD_ARG;
+  const bf16* a = (const bf16*)A;
+  const bf16* w = (const bf16*)W;
+  int tile = g_tile;
+  if (tile == 0) tile = choose_sums(M, N, K).tile;
+#define GO(WF, WT, FT, TT) return launch<WF, WT, FT, TT, EPI_SUMS, float>(a, lda, w, ldw, partial, (size_t)N, M, N, K, stream, QkvEpilogue{}, GroupedRows{}, parts)
+  if (tile == 1) GO(2, 4, 8, 4);
+  if (tile == 3) GO(1, 4, 4, 1);
+  GO(2, 4, 4, 2);
 #undef GO
 }
 

@@ -52,6 +52,8 @@ _SIGNATURES = {
     "ms_gemm_panel_splitk": [_c_ptr, _c_ll, _c_ptr, _c_ll, _c_ptr, _c_ptr, _c_ll, _c_int, _c_int, _c_int, _c_int, _c_int,
                              _c_ptr, _c_int, _c_ptr],
     "ms_gemm_tiled": [_c_ptr, _c_ll, _c_ptr, _c_ll, _c_ptr, _c_ll, _c_int, _c_int, _c_int, _c_int, _c_float, _c_float, _c_ptr],
+    "ms_gemm_tiled_sums_parts": [_c_int, _c_int, _c_int],
+    "ms_gemm_tiled_sums": [_c_ptr, _c_ll, _c_ptr, _c_ll, _c_ptr, _c_int, _c_int, _c_int, _c_int, _c_ptr],
     "ms_gemm_tiled_force": [_c_int],
     "ms_gemm_tiled_force_xcd_split": [_c_int],
     "ms_gemm_tiled_pays": [_c_int, _c_int, _c_int],
@@ -582,15 +584,32 @@ def slab_pays(n_rows: int, w: torch.Tensor) -> bool:
 def gemm_sums(a: torch.Tensor, w: torch.Tensor) -> Optional[torch.Tensor]:
     """a @ w.T as float partial sums [parts, M, N] over runs of the columns, for a reader that adds them up on its way
     (``rms_norm``'s ``delta``), where that is the faster way to the product; None: it is not."""
+    (M, K), N = a.shape, w.shape[0]
+    if M > SKINNY_MAX_ROWS:
+        if not (a.dtype == w.dtype == torch.bfloat16 and a.is_contiguous() and w.is_contiguous() and a.data_ptr() % 16 == 0
+                and w.data_ptr() % 16 == 0):
+            return None
+        parts = _get("ms_gemm_tiled_sums_parts")(M, N, K)
+        return gemm_tiled_sums(a, w, parts) if parts else None
     if not skinny_ok(a, w):
         return None
-    (M, K), N = a.shape, w.shape[0]
     parts = _get("ms_gemm_slab_parts")(M, N, K, 1)
     if parts <= 1:
         return None
     _check(a, "a", torch.bfloat16, contiguous=False)
     _check(w, "w", torch.bfloat16, (N, a.shape[1]))
     return _slab_sums(a, w, a.stride(0) if M > 1 else K, parts)
+
+
+def gemm_tiled_sums(a: torch.Tensor, w: torch.Tensor, parts: int) -> torch.Tensor:
+    """Float partial sums [parts, M, N] of a @ w.T over runs of the columns, for many rows (the tiled product; K a multiple of
+    64, at least one step of that to a part)."""
+    _check(a, "a", torch.bfloat16)
+    M, K = a.shape
+    _check(w, "w", torch.bfloat16, (None, K))
+    partial = torch.empty((parts, M, w.shape[0]), dtype=torch.float32, device=a.device)
+    _call("ms_gemm_tiled_sums", a.data_ptr(), K, w.data_ptr(), K, partial.data_ptr(), M, w.shape[0], K, parts, _stream())
+    return partial
 
 
 def gemm_slab(a: torch.Tensor, w: torch.Tensor, bias: Optional[torch.Tensor] = None, epilogue: int = EPI_STORE,

@@ -787,6 +787,35 @@ def test_gemm_slab_qkv_equals_product_rotation_and_store(ops, M, nh, nkv, d, K, 
     assert (kp.permute(0, 2, 1, 3).reshape(pages * page_size, -1)[untouched.to(DEV)] == 0).all()
 
 
+@pytest.mark.parametrize("tile", [0, 1, 2, 3])
+@pytest.mark.parametrize("M,N,K,parts", [(65, 896, 896, 3), (390, 900, 4864, 5), (1, 2, 64, 1), (257, 258, 192, 3), (700, 2304, 448, 7),
+                                         (1025, 130, 1024, 8)])
+def test_gemm_tiled_sums(ops, M, N, K, parts, tile):
+    """The tiled product in runs of its columns: every tile, runs of different lengths and of one and two steps, blocks that
+    deal out unevenly over the XCDs, features and tokens that fill no whole tile; each part against its own columns in double,
+    and the norm that adds them up (one part too)."""
+    g = torch.Generator().manual_seed(M + N + K)
+    a = torch.randn(M, K, generator=g).bfloat16().to(DEV)
+    w = (torch.randn(N, K, generator=g) / math.sqrt(K)).bfloat16().to(DEV)
+    force = ops._get("ms_gemm_tiled_force")
+    force(tile)
+    try:
+        got = ops.gemm_tiled_sums(a, w, parts)
+    finally:
+        force(0)
+    edges = [K // 64 * p // parts * 64 for p in range(parts + 1)]
+    for p in range(parts):
+        want = a[:, edges[p]:edges[p + 1]].double() @ w[:, edges[p]:edges[p + 1]].double().T
+        torch.testing.assert_close(got[p].double(), want, atol=3e-5, rtol=3e-5)
+    x = torch.randn(M, N, generator=g).to(DEV)
+    nw = (1 + 0.1 * torch.randn(N, generator=g)).to(DEV)
+    total = x.double() + got.double().sum(0)
+    normed = total * torch.rsqrt((total * total).mean(-1, keepdim=True) + 1e-6) * nw.double()
+    h = ops.rms_norm(x, nw, 1e-6, torch.empty(M, N, dtype=torch.bfloat16, device=DEV), delta=got)
+    torch.testing.assert_close(h.double(), normed, **tol(torch.bfloat16))
+    torch.testing.assert_close(x.double(), total, atol=3e-5, rtol=3e-5)
+
+
 def test_gemm_stream_refuses_what_it_cannot_take(ops):
     w = torch.zeros(64, 64, dtype=torch.bfloat16, device=DEV)
     with pytest.raises(RuntimeError, match="unsupported"):
