@@ -534,19 +534,22 @@ SumsChoice choose_sums(int M, int N, int K) {
 extern "C" void ms_gemm_tiled_force(int tile) { g_tile = tile; }
 extern "C" void ms_gemm_tiled_force_xcd_split(int xm) { g_xcd_split = xm; }
 
-// Whether the gated product of M tokens is faster here than as the library's product and an activation kernel
-// (measured with a different W every call, 65 to 8,192 tokens): up to 1,536 columns always (0.5 to 0.98 of the
-// library's time); beyond that up to 2,048 tokens whose tiles fill at least 9/10 of their rounds over the CUs.  That line is
-// where this kernel won throughout with one barrier and everything drained at it a step; as it is now it takes 0.76 to 0.86 of
-// the library's time there (7B gate/up, 2,048 tokens 413 and 546 us; one row of 55,296 x 5,120, at 1,300 tokens, 1.03), and 0.73
-// to 1.2 on the other side (7B gate/up: 256 tokens 72 and 87, 1,024 tokens 239 and 315, 4,096 tokens 822 and 864; 14,336 x
-// 4,096: 256 tokens 65 and 55, 1,024 tokens 92 and 103).  Tiles of 64 x 64 never.
+// Whether the gated product of M tokens is faster here than as the library's product and an activation kernel.  Time of these over
+// this kernel's, a different W every call:
+//   up to 1,536 columns 1.02 to 2 (65 to 8,192 tokens);
+//   2,048 to 3,584 columns, 5,632 to 37,888 rows, 130 to 8,192 tokens: 0.99 to 1.38, 1.15 on average (7B gate/up: 256 tokens 91 and
+//   79 us, 1,024 tokens 313 and 245, 2,176 tokens 566 and 532, 4,096 tokens 876 and 834; 22,016 x 2,048, 4,096 tokens 365 and 304);
+//   4,096 and 5,120 columns, 12,288 to 55,296 rows: beyond 512 tokens 0.95 to 1.28 (27,648 x 5,120, 1,024 tokens 276 and 226,
+//   3,584 tokens 766 and 804), up to 512 tokens 0.91 to 1.21;
+//   8,192 columns 0.96 to 1.03.
+// Tiles of 64 x 64 only up to 1,536 columns.
 extern "C" int ms_gemm_tiled_pays(int M, int N, int K) {
   if (M <= 0 || N <= 0 || K <= 0 || K % BK) return 0;
   if (K <= 1536) return 1;
-  if (M > 2048) return 0;
   const TileChoice c = choose_tile(M, N, K);
-  return c.tile != 3 && c.tiles * 10 >= c.slots * 9;
+  if (c.tile == 3) return 0;
+  if (K <= 3584 || (K <= 5120 && M > 512)) return 1;
+  return M <= 2048 && c.tiles * 10 >= c.slots * 9;
 }
 
 // A bfloat16 [M, lda], W bfloat16 [N, ldw] (rows of K, K a multiple of 64), out bfloat16.
