@@ -26,6 +26,7 @@
 #include "attention_tiles.h"
 #include "api.h"
 #include <algorithm>
+#include <cmath>
 
 namespace {
 
@@ -36,9 +37,11 @@ typedef __attribute__((address_space(3))) void lds_void;
 typedef const __attribute__((address_space(1))) void global_void;
 
 constexpr int GROUP = 4;              // waves that walk the same keys
-constexpr int NT = 2;                 // tiles of 16 columns a wave
-constexpr int COLS = GROUP * NT * 16; // columns a block
 constexpr int KEYS = 64;              // keys a tile: one chunk of 16 for every wave to bring
+
+constexpr int WIDE = GROUP * 2 * 16;  // columns a block of the wide kind
+// kinds: two tiles of columns a wave; one; and twice the groups of waves (two tiles at 64 dims, one at 128)
+enum { PROMPT_WIDE = 1, PROMPT_NARROW = 2, PROMPT_NARROW_GROUPS = 3 };
 
 constexpr int FOLLOWED = 128;         // keys over which the reference goes with every unit's maximum ..
 constexpr float FOLLOW_DOWN = 4.f;    // .. unless that is further below it: sums grow by 2^16 at most on the way down
@@ -59,14 +62,16 @@ __device__ __forceinline__ float column_max(float x) {
 }
 
 // KG groups of waves own the same columns and take the tiles of keys in turn, each with its own place in LDS; at the end
-// they merge what they have, each for its share of the dims.
-template <int D, int KG>
-__global__ void __launch_bounds__(KG * GROUP * MS_WAVE, 2 * KG)
+// they merge what they have, each for its share of the dims.  NT tiles of 16 columns a wave: with one, a block's columns and its
+// share of the softmax are half as many, a turn takes 0.6 of the time and twice as many blocks share the work out.
+template <int D, int KG, int NT>
+__global__ void __launch_bounds__(KG * GROUP * MS_WAVE, D == 64 ? 4 : 2)
 attention_prompt_kernel(const bf16* __restrict__ q, size_t q_stride, const bf16* __restrict__ k_pages,
                         const bf16* __restrict__ vt_pages, const int* __restrict__ block_table, int table_stride,
                         const int* __restrict__ table_rows, const int* __restrict__ q_start,
                         const int* __restrict__ context_lens, bf16* __restrict__ out, size_t out_stride, int nh, int nkv,
                         int page_size, float scale_log2e, int window, int n_requests, int pair_order) {
+  constexpr int COLS = GROUP * NT * 16;               // columns a block
   constexpr int CT = D / 16, PIECES = D / 8;
   constexpr int CHUNK = 16 * D;                       // values of a chunk of 16 keys, of keys as of values
   constexpr int STAGE = 2 * 4 * CHUNK;                // a tile: four chunks of keys, four of values
@@ -282,28 +287,37 @@ attention_prompt_kernel(const bf16* __restrict__ q, size_t q_stride, const bf16*
   }
   if constexpr (KG > 1) {
     __shared__ float sm_m[KG][COLS], sm_l[KG][COLS];
-    f32x4* sm_o = reinterpret_cast<f32x4*>(lds);        // [group of the sums][wave][dims' tile of the other group][NT][64]
-    static_assert(KG == 2 && (size_t)KG * GROUP * OWN * NT * MS_WAVE * 16 <= (size_t)KG * 2 * STAGE * 2, "the other group's share fits");
+    f32x4* sm_o = reinterpret_cast<f32x4*>(lds);        // [group of the sums][wave][tile of dims][NT][64]
+    static_assert((size_t)KG * GROUP * CT * NT * MS_WAVE * 16 <= (size_t)KG * 2 * STAGE * 2, "all sums fit");
     __syncthreads();                                    // nobody reads keys or values any more
 #pragma unroll
     for (int t = 0; t < NT; ++t) {
       const int c = (wave * NT + t) * 16 + col16;
       if (kq == 0) { sm_m[kg][c] = m[t]; sm_l[kg][c] = l[t]; }
 #pragma unroll
-      for (int d = 0; d < OWN; ++d) sm_o[(((kg * GROUP + wave) * OWN + d) * NT + t) * MS_WAVE + lane] = kg == 0 ? o[OWN + d][t] : o[d][t];
+      for (int d = 0; d < CT; ++d)
+        if (d / OWN != kg) sm_o[(((kg * GROUP + wave) * CT + d) * NT + t) * MS_WAVE + lane] = o[d][t];
     }
     __syncthreads();
 #pragma unroll
     for (int t = 0; t < NT; ++t) {
       const int c = (wave * NT + t) * 16 + col16;
-      const float other_m = sm_m[kg ^ 1][c], big = fmaxf(m[t], other_m), safe = big == -INFINITY ? 0.f : big;
-      const float mine = fast_exp2(m[t] - safe), theirs = fast_exp2(other_m - safe);
-      l[t] = l[t] * mine + sm_l[kg ^ 1][c] * theirs;
+      float big = m[t];
 #pragma unroll
-      for (int d = 0; d < OWN; ++d) {
-        const f32x4 part = sm_o[((((kg ^ 1) * GROUP + wave) * OWN + d) * NT + t) * MS_WAVE + lane];
-        if (kg == 0) o[d][t] = o[d][t] * mine + part * theirs;
-        else o[OWN + d][t] = o[OWN + d][t] * mine + part * theirs;
+      for (int k = 1; k < KG; ++k) big = fmaxf(big, sm_m[(kg + k) % KG][c]);
+      const float safe = big == -INFINITY ? 0.f : big, mine = fast_exp2(m[t] - safe);
+      l[t] *= mine;
+#pragma unroll
+      for (int d = 0; d < CT; ++d)
+        if (d / OWN == kg) o[d][t] *= mine;
+#pragma unroll
+      for (int k = 1; k < KG; ++k) {
+        const int other = (kg + k) % KG;
+        const float theirs = fast_exp2(sm_m[other][c] - safe);
+        l[t] += sm_l[other][c] * theirs;
+#pragma unroll
+        for (int d = 0; d < CT; ++d)
+          if (d / OWN == kg) o[d][t] += sm_o[(((other * GROUP + wave) * CT + d) * NT + t) * MS_WAVE + lane] * theirs;
       }
     }
   }
@@ -324,19 +338,19 @@ attention_prompt_kernel(const bf16* __restrict__ q, size_t q_stride, const bf16*
   }
 }
 
-template <int D, int KG>
+template <int D, int KG, int NT>
 int launch(dim3 grid, dim3 block, const bf16* q, size_t q_stride, const bf16* k, const bf16* vt, const int* table, int table_stride,
            const int* table_rows, const int* q_start, const int* ctx, bf16* out, size_t out_stride, int nh, int nkv, int page_size,
            float scale_log2e, int window, int n_requests, int pair_order, hipStream_t stream) {
   constexpr size_t bytes = (size_t)KG * 2 * 2 * KEYS * D * sizeof(bf16);
   static bool raised = false;   // once per instantiation: allow more dynamic LDS than the default 64 KB
   if (!raised) {
-    if (hipFuncSetAttribute(reinterpret_cast<const void*>(&attention_prompt_kernel<D, KG>),
+    if (hipFuncSetAttribute(reinterpret_cast<const void*>(&attention_prompt_kernel<D, KG, NT>),
                             hipFuncAttributeMaxDynamicSharedMemorySize, (int)bytes) != hipSuccess)
       return MS_LAUNCH_FAILED;
     raised = true;
   }
-  attention_prompt_kernel<D, KG><<<grid, block, bytes, stream>>>(q, q_stride, k, vt, table, table_stride, table_rows, q_start, ctx, out, out_stride, nh, nkv, page_size, scale_log2e, window, n_requests, pair_order);
+  attention_prompt_kernel<D, KG, NT><<<grid, block, bytes, stream>>>(q, q_stride, k, vt, table, table_stride, table_rows, q_start, ctx, out, out_stride, nh, nkv, page_size, scale_log2e, window, n_requests, pair_order);
   return ms_launch_status();
 }
 
@@ -362,11 +376,11 @@ extern "C" int ms_attention_prompt_pays(int n_requests, int n_tokens, int max_q_
                                         int num_kv_heads, int head_dim, int page_size, int window) {
   if ((head_dim != 64 && head_dim != 128) || page_size % 16 || num_kv_heads <= 0) return 0;
   if (n_requests > 1 && (long long)max_context_len > 2LL * n_tokens) return 0;
-  const long long blocks = (long long)n_tokens * (num_heads / num_kv_heads) / COLS * num_kv_heads, cus = ms_compute_units();
+  const long long blocks = (long long)n_tokens * (num_heads / num_kv_heads) / WIDE * num_kv_heads, cus = ms_compute_units();
   const bool uneven = n_requests == 1 || 3LL * max_q_len > n_tokens;
   long long chain = max_context_len, keys = 2LL * max_context_len - max_q_len;    // of the last tile, of a mean one twice
   if (window > 0) {
-    chain = std::min<long long>(chain, (long long)window + COLS / std::max(1, num_heads / num_kv_heads));
+    chain = std::min<long long>(chain, (long long)window + WIDE / std::max(1, num_heads / num_kv_heads));
     keys = std::min(keys, 2 * std::min<long long>(window, chain));
   }
   const auto fills = [&](long long twentieths) { return blocks * keys * 20 >= twentieths * cus * chain; };
@@ -377,9 +391,43 @@ extern "C" int ms_attention_prompt_pays(int n_requests, int n_tokens, int max_q_
   return !uneven && blocks * 16 >= cus * (short_chains ? 7 : 24);
 }
 
+// Which kernel a step's attention should take: 0 ms_paged_attention_mfma, else a kind of this one.  Between the other kernel and
+// the wide kind ms_attention_prompt_pays decides; one of the narrow kinds takes the step where a model of the measurements
+// puts it 6 % ahead of that.  The model, in us: a start, the cube root of the sum of cubes of the longest chain (in tiles of 64
+// keys) and of the work a CU has (blocks of 128 columns a CU times the mean tile's keys), and a little a block; its terms fitted
+// to 320 and 250 random steps (64 and 128 dims; 1 to 40 requests, portions of up to 4,096 tokens alone, behind up to 8,000 keys,
+// and beside single tokens; residuals 6 to 13 %).  There the choice takes 0.81 and 0.93 of the time of the choice between
+// the other two, at most 1.06 and 1.16 of it.  Steps of a few tokens a request stay with the other kernel (30 requests of 2 tokens 5.4
+// and 6.0 us).  14 heads on 2 of 64 dims: 386 tokens 12.1 -> 9.9 us, 1,158 23.3 -> 18.2, 2,912 tokens behind 4,688 141 -> 119; 28
+// heads on 4 of 128: 910 tokens 29.8 -> 23.3, 2,094 74.7 -> 59.2.
+extern "C" int ms_attention_prompt_kind(int n_requests, int n_tokens, int max_q_len, int max_context_len, int num_heads,
+                                        int num_kv_heads, int head_dim, int page_size, int window) {
+  if ((head_dim != 64 && head_dim != 128) || page_size % 16 || num_kv_heads <= 0 || num_heads % num_kv_heads) return 0;
+  const int plain = ms_attention_prompt_pays(n_requests, n_tokens, max_q_len, max_context_len, num_heads, num_kv_heads, head_dim, page_size, window)
+                        ? PROMPT_WIDE : 0;
+  if (max_q_len <= 16 || (long long)n_tokens * (num_heads / num_kv_heads) / (WIDE / 2) + n_requests > 65535) return plain;
+  double chain = max_context_len, mean = max_context_len - max_q_len / 2;
+  if (window > 0) {
+    chain = std::min(chain, (double)window + WIDE / std::max(1, num_heads / num_kv_heads));
+    mean = std::min(mean, (double)window);
+  }
+  const double a_cu = (double)n_tokens * num_heads / WIDE / ms_compute_units();
+  static const double terms[2][4][4] = {   // start, chain, load, blocks: of the other kernel, wide, narrow, narrow with more groups
+      {{7.1, 0.74, 0.58, 5.5}, {7.0, 0.92, 0.40, 3.0}, {5.8, 0.575, 0.65, 3.8}, {8.8, 0.69, 0.52, 5.2}},
+      {{6.0, 0.65, 2.28, 11.3}, {6.5, 1.83, 0.90, 3.9}, {5.6, 1.13, 1.27, 4.8}, {6.3, 0.74, 1.455, 10.1}}};
+  double us[4];
+  for (int k = 0; k < 4; ++k) {
+    const double* t = terms[head_dim == 128][k];
+    const double c = chain / KEYS * t[1], l = a_cu * mean / KEYS * t[2];
+    us[k] = t[0] + cbrt(c * c * c + l * l * l) + a_cu * t[3];
+  }
+  const int narrow = us[PROMPT_NARROW] <= us[PROMPT_NARROW_GROUPS] ? PROMPT_NARROW : PROMPT_NARROW_GROUPS;
+  return us[narrow] * 1.06 < us[plain] ? narrow : plain;
+}
+
 // The arguments of ms_paged_attention_mfma's general shape, for plain scores (no sink, cap, slopes, gate; values of the
-// keys' size).  MS_UNSUPPORTED for what it does not take.
-extern "C" int ms_attention_prompt(const void* q, long long q_stride, const void* k_pages, const void* vt_pages,
+// keys' size), on the kind that ms_attention_prompt_kind names.  MS_UNSUPPORTED for what it does not take.
+extern "C" int ms_attention_prompt_as(int kind, const void* q, long long q_stride, const void* k_pages, const void* vt_pages,
                                    const int* block_table, int table_stride, const int* table_rows, const int* q_start,
                                    const int* context_lens, void* out, long long out_stride, int n_requests, int n_tokens,
                                    int max_q_len, int num_heads, int num_kv_heads, int head_dim, int page_size, float scale,
@@ -392,13 +440,33 @@ extern "C" int ms_attention_prompt(const void* q, long long q_stride, const void
   if (head_dim != 64 && head_dim != 128) return MS_UNSUPPORTED;
   if (page_size % 16 || ((uintptr_t)k_pages | (uintptr_t)vt_pages) % 16) return MS_UNSUPPORTED;
   const int rep = num_heads / num_kv_heads;
-  long long tiles = (long long)n_tokens * rep / COLS + n_requests;
-  tiles = std::min(tiles, (((long long)max_q_len * rep + COLS - 1) / COLS) * n_requests);
+  if (kind < PROMPT_WIDE || kind > PROMPT_NARROW_GROUPS) return MS_BAD_ARG;
+  const int cols = kind == PROMPT_NARROW || (kind == PROMPT_NARROW_GROUPS && head_dim == 128) ? WIDE / 2 : WIDE;
+  long long tiles = (long long)n_tokens * rep / cols + n_requests;
+  tiles = std::min(tiles, (((long long)max_q_len * rep + cols - 1) / cols) * n_requests);
   if (tiles > 65535 || (long long)max_q_len * rep > 0x7fffffffLL) return MS_UNSUPPORTED;
-  const int pair_order = tiles * num_kv_heads <= 2LL * ms_compute_units() ? 1 : 0;
-  dim3 grid(num_kv_heads, (unsigned)tiles), block((head_dim == 64 ? 2 : 1) * GROUP * MS_WAVE);
-#define GO(D, KG) return launch<D, KG>(grid, block, (const bf16*)q, (size_t)q_stride, (const bf16*)k_pages, (const bf16*)vt_pages, block_table, table_stride, table_rows, q_start, context_lens, (bf16*)out, (size_t)out_stride, num_heads, num_kv_heads, page_size, scale * 1.4426950408889634f, window, n_requests, pair_order, stream)
-  if (head_dim == 64) GO(64, 2);
-  GO(128, 1);
+  const int groups = (head_dim == 64 ? 2 : 1) * (kind == PROMPT_NARROW_GROUPS ? 2 : 1);
+  // two blocks share a CU, but for the most groups, whose tiles take its LDS
+  const int pair_order = tiles * num_kv_heads <= 2LL * ms_compute_units() && kind != PROMPT_NARROW_GROUPS ? 1 : 0;
+  dim3 grid(num_kv_heads, (unsigned)tiles), block(groups * GROUP * MS_WAVE);
+#define GO(D, KG, NT) return launch<D, KG, NT>(grid, block, (const bf16*)q, (size_t)q_stride, (const bf16*)k_pages, (const bf16*)vt_pages, block_table, table_stride, table_rows, q_start, context_lens, (bf16*)out, (size_t)out_stride, num_heads, num_kv_heads, page_size, scale * 1.4426950408889634f, window, n_requests, pair_order, stream)
+  if (head_dim == 64) {
+    if (kind == PROMPT_NARROW) GO(64, 2, 1);
+    if (kind == PROMPT_NARROW_GROUPS) GO(64, 4, 2);
+    GO(64, 2, 2);
+  }
+  if (kind == PROMPT_NARROW) GO(128, 1, 1);
+  if (kind == PROMPT_NARROW_GROUPS) GO(128, 2, 1);
+  GO(128, 1, 2);
 #undef GO
+}
+
+extern "C" int ms_attention_prompt(const void* q, long long q_stride, const void* k_pages, const void* vt_pages,
+                                   const int* block_table, int table_stride, const int* table_rows, const int* q_start,
+                                   const int* context_lens, void* out, long long out_stride, int n_requests, int n_tokens,
+                                   int max_q_len, int num_heads, int num_kv_heads, int head_dim, int page_size, float scale,
+                                   int window, hipStream_t stream) {
+  return ms_attention_prompt_as(PROMPT_WIDE, q, q_stride, k_pages, vt_pages, block_table, table_stride, table_rows, q_start,
+                                context_lens, out, out_stride, n_requests, n_tokens, max_q_len, num_heads, num_kv_heads, head_dim,
+                                page_size, scale, window, stream);
 }

@@ -79,6 +79,9 @@ _SIGNATURES = {
                                 _c_float, _c_ptr, _c_ptr, _c_ll, _c_int, _c_float, _c_ptr],
     "ms_attention_prompt": [_c_ptr, _c_ll, _c_ptr, _c_ptr, _c_ptr, _c_int, _c_ptr, _c_ptr, _c_ptr, _c_ptr, _c_ll, _c_int, _c_int,
                             _c_int, _c_int, _c_int, _c_int, _c_int, _c_float, _c_int, _c_ptr],
+    "ms_attention_prompt_as": [_c_int, _c_ptr, _c_ll, _c_ptr, _c_ptr, _c_ptr, _c_int, _c_ptr, _c_ptr, _c_ptr, _c_ptr, _c_ll, _c_int, _c_int,
+                               _c_int, _c_int, _c_int, _c_int, _c_int, _c_float, _c_int, _c_ptr],
+    "ms_attention_prompt_kind": [_c_int, _c_int, _c_int, _c_int, _c_int, _c_int, _c_int, _c_int, _c_int],
     "ms_attention_prompt_pays": [_c_int, _c_int, _c_int, _c_int, _c_int, _c_int, _c_int, _c_int, _c_int],
     "ms_paged_attention_mfma_decode": [_c_ptr, _c_ll, _c_ptr, _c_ptr, _c_ptr, _c_int, _c_ptr, _c_ptr, _c_ptr, _c_ptr,
                                        _c_ll, _c_ptr, _c_ptr, _c_int, _c_int, _c_int, _c_int, _c_int, _c_int, _c_float,
@@ -1051,13 +1054,15 @@ def paged_attention_mfma(q: torch.Tensor, k_pages: torch.Tensor, vt_pages: torch
               block_table.data_ptr(), block_table.shape[1], _ptr(table_rows), q_start.data_ptr(), context_lens.data_ptr(),
               out.data_ptr(), num_heads * dv, part_o.data_ptr(), part_ml.data_ptr(), R, num_heads, nkv, d, dv, page_size, float(scale),
               int(window or 0), MIN_BLOCKS_PER_SPLIT, n_splits, _ptr(sink), *more, _stream())
-    elif (plain and k_pages.data_ptr() % 16 == 0 and vt_pages.data_ptr() % 16 == 0
-          and _get("ms_attention_prompt_pays")(R, N, max_q_len, max_context_len, num_heads, nkv, d, page_size, int(window or 0))):
-        # many prompt tokens: keys and values staged in LDS for four neighbouring tiles
-        _call("ms_attention_prompt", q.data_ptr(), q_stride, k_pages.data_ptr(), vt_pages.data_ptr(), block_table.data_ptr(),
-              block_table.shape[1], _ptr(table_rows), q_start.data_ptr(), context_lens.data_ptr(), out.data_ptr(), num_heads * dv,
-              R, N, max_q_len, num_heads, nkv, d, page_size, float(scale), int(window or 0), _stream())
     else:
+        kind = 0
+        if plain and k_pages.data_ptr() % 16 == 0 and vt_pages.data_ptr() % 16 == 0:
+            kind = _get("ms_attention_prompt_kind")(R, N, max_q_len, max_context_len, num_heads, nkv, d, page_size, int(window or 0))
+        if kind:     # keys and values staged in LDS for four neighbouring tiles
+            _call("ms_attention_prompt_as", kind, q.data_ptr(), q_stride, k_pages.data_ptr(), vt_pages.data_ptr(), block_table.data_ptr(),
+                  block_table.shape[1], _ptr(table_rows), q_start.data_ptr(), context_lens.data_ptr(), out.data_ptr(), num_heads * dv,
+                  R, N, max_q_len, num_heads, nkv, d, page_size, float(scale), int(window or 0), _stream())
+            return out
         _call("ms_paged_attention_mfma", q.data_ptr(), q_stride, k_pages.data_ptr(), vt_pages.data_ptr(),
               block_table.data_ptr(), block_table.shape[1], _ptr(table_rows), q_start.data_ptr(), context_lens.data_ptr(),
               out.data_ptr(), num_heads * dv, R, N, max_q_len, num_heads, nkv, d, dv, page_size, float(scale), int(window or 0),

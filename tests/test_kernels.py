@@ -1410,6 +1410,98 @@ def test_attention_of_staged_prompts_when_scores_rise_or_fall(ops, nh, nkv, d, r
     torch.testing.assert_close(out.double().cpu(), want, **tol(torch.bfloat16))
 
 
+def _staged(ops, kind, q, kp, vt, table, q_start, lens, nh, longest, window, rows=None, out=None):
+    (P, nkv, page, d), N, R = kp.shape, q.shape[0], lens.numel()
+    out = torch.full((N, nh * d), 3.0, dtype=torch.bfloat16, device=DEV) if out is None else out
+    ops._call("ms_attention_prompt_as", kind, q.data_ptr(), q.stride(0), kp.data_ptr(), vt.data_ptr(), table.data_ptr(), table.shape[1],
+              ops._ptr(rows), q_start.data_ptr(), lens.data_ptr(), out.data_ptr(), nh * d, R, N, longest, nh, nkv, d, page, d ** -0.5,
+              window or 0, ops._stream())
+    return out
+
+
+@pytest.mark.parametrize("kind", [2, 3])
+@pytest.mark.parametrize("nh,nkv,d,page_size,window", [(14, 2, 64, 16, None), (8, 8, 128, 32, None), (4, 1, 64, 16, 40),
+                                                        (28, 4, 128, 16, None), (6, 2, 64, 48, 130), (20, 1, 128, 16, 65)])
+def test_narrow_kinds_of_staged_prompts(ops, nh, nkv, d, page_size, window, kind):
+    """Blocks of 64 columns, and of more groups of waves that share the keys out (fewer tiles of keys than groups, one more than
+    a turn, requests of one token): against the oracle; what no request owns is NaN, and tokens of nobody stay as they are."""
+    g = torch.Generator().manual_seed(nh * 10 + d + kind)
+    ctx, qlen = [70, 133, 64, 65, 300, 1, 257, 513], [70, 9, 64, 1, 150, 1, 257, 257]
+    c = _paged_case(g, torch.bfloat16, nh, nkv, d, page_size, ctx, qlen, float("nan"))
+    want = torch.cat([attention_reference(q.double(), k.double(), v.double(), d ** -0.5, window).transpose(0, 1).reshape(-1, nh * d)
+                      for q, k, v in zip(c["qs"], c["ks"], c["vs"])])
+    N, R = c["q"].shape[0], len(ctx) + 1
+    wide = torch.zeros(N + 5, (nh + 2 * nkv) * d, dtype=torch.bfloat16, device=DEV)
+    wide[:N, :nh * d] = c["q"].to(DEV)
+    perm = torch.randperm(R, generator=g)
+    table = torch.zeros(R, c["table"].shape[1], dtype=torch.int32)
+    table[perm[:R - 1]] = c["table"]
+    q_start = torch.tensor([0] + list(np.cumsum(qlen)) + [N], dtype=torch.int32, device=DEV)
+    out = _staged(ops, kind, wide, c["kp"].to(DEV), c["vt"].to(DEV), table.to(DEV), q_start, torch.tensor(ctx + [7], dtype=torch.int32, device=DEV),
+                  nh, 257, window, perm.to(torch.int32).to(DEV))
+    torch.testing.assert_close(out[:N].double().cpu(), want, **tol(torch.bfloat16))
+    assert (out[N:] == 3.0).all()
+
+
+@pytest.mark.parametrize("kind", [2, 3])
+@pytest.mark.parametrize("nh,nkv,d", [(7, 1, 64), (4, 4, 128)])
+@pytest.mark.parametrize("ramp", [0.5, 60.0, -6.0, -60.0])
+def test_narrow_kinds_when_scores_rise_or_fall(ops, nh, nkv, d, ramp, kind):
+    """As for the wide kind: the groups of waves end with references apart, late keys dwarf the early ones or the other way."""
+    g = torch.Generator().manual_seed(int(abs(ramp) * 10) + d + nh)
+    ctx, qlen, page = [900, 333, 40], [200, 70, 40], 16
+    c = _paged_case(g, torch.bfloat16, nh, nkv, d, page, ctx, qlen, float("nan"))
+    u = torch.zeros(d); u[5] = 1.0
+    for r in range(len(ctx)):
+        c["qs"][r] = (c["qs"][r].float() * 0.05 + u).to(torch.bfloat16)
+        steps = torch.arange(ctx[r]).float() / ctx[r] * ramp * math.log(2.0) / d ** -0.5
+        c["ks"][r] = (c["ks"][r].float() * 0.05 + steps[None, :, None] * u).to(torch.bfloat16)
+        for j in range(ctx[r]):
+            c["kp"][c["table"][r, j // page].item(), :, j % page] = c["ks"][r][:, j]
+    want = torch.cat([attention_reference(q.double(), k.double(), v.double(), d ** -0.5, None).transpose(0, 1).reshape(-1, nh * d)
+                      for q, k, v in zip(c["qs"], c["ks"], c["vs"])])
+    q = torch.cat([x.transpose(0, 1).reshape(-1, nh * d) for x in c["qs"]]).to(DEV)
+    q_start = torch.tensor([0] + list(np.cumsum(qlen)), dtype=torch.int32, device=DEV)
+    out = _staged(ops, kind, q, c["kp"].to(DEV), c["vt"].to(DEV), c["table"].to(DEV), q_start, torch.tensor(ctx, dtype=torch.int32, device=DEV), nh, 200, None)
+    torch.testing.assert_close(out.double().cpu(), want, **tol(torch.bfloat16))
+
+
+@pytest.mark.parametrize("kind", [1, 2, 3])
+@pytest.mark.parametrize("nh,nkv,d,lens,past,spread", [(6, 2, 64, [130] * 8, 0, 2.0), (6, 2, 64, [512, 40], 0, 4.0), (8, 2, 128, [200] * 4, 0, 2.0),
+                                                       (4, 2, 128, [700], 900, 3.0), (4, 1, 64, [700], 900, 3.0), (4, 2, 64, [300], 2200, 1.0),
+                                                       (4, 2, 128, [300], 2200, 1.0)])
+def test_kinds_of_staged_prompts_lie_no_farther_from_64_bits_than_the_other_kernel(ops, nh, nkv, d, lens, past, spread, kind):
+    """As the test of the wide kind above, over the kinds."""
+    g = torch.Generator().manual_seed(d + past + 5)
+    R, N, ctx, page = len(lens), sum(lens), [past + n for n in lens], 16
+    pages = [-(-n // page) for n in ctx]
+    kp = torch.randn(sum(pages) + 1, nkv, page, d, generator=g).bfloat16().to(DEV)
+    vp = torch.randn(sum(pages) + 1, nkv, page, d, generator=g).bfloat16().to(DEV)
+    vt = vp.transpose(2, 3).contiguous()
+    q = (torch.randn(N, nh * d, generator=g) * spread).bfloat16().to(DEV)
+    table = torch.zeros(R, max(pages), dtype=torch.int32)
+    for r in range(R):
+        table[r, :pages[r]] = torch.arange(pages[r]) + 1 + sum(pages[:r])
+    table = table.to(DEV)
+    q_start = torch.tensor([0] + list(np.cumsum(lens)), dtype=torch.int32, device=DEV)
+    held = torch.tensor(ctx, dtype=torch.int32, device=DEV)
+    want = []
+    for r in range(R):
+        k, v = (x[table[r, :pages[r]].long()].transpose(1, 2).reshape(-1, nkv, d)[:ctx[r]].transpose(0, 1).double() for x in (kp, vp))
+        rows = q[int(q_start[r]):int(q_start[r + 1])].reshape(-1, nh, d).transpose(0, 1).double()
+        hidden = torch.arange(ctx[r], device=DEV)[None] > torch.arange(past, ctx[r], device=DEV)[:, None]
+        o = [(rows[h] @ k[h * nkv // nh].t() * d ** -0.5).masked_fill(hidden, -math.inf).softmax(-1) @ v[h * nkv // nh] for h in range(nh)]
+        want.append(torch.stack(o, 1).reshape(-1, nh * d))
+    want = torch.cat(want)
+    staged, other = _staged(ops, kind, q, kp, vt, table, q_start, held, nh, max(lens), None), torch.empty_like(q)
+    ops._call("ms_paged_attention_mfma", q.data_ptr(), nh * d, kp.data_ptr(), vt.data_ptr(), table.data_ptr(), table.shape[1], None,
+              q_start.data_ptr(), held.data_ptr(), other.data_ptr(), nh * d, R, N, max(lens), nh, nkv, d, d, page, d ** -0.5,
+              0, None, 0.0, None, None, 0, 1, 1.0, ops._stream())
+    far = [((x.double() - want).norm() / want.norm()).item() for x in (staged, other)]
+    print(kind, d, far)
+    assert far[0] <= 1.005 * far[1], far
+
+
 @pytest.mark.parametrize("d", [64, 128])
 @pytest.mark.parametrize("R,nkv", [(40, 8), (80, 8)])
 def test_the_choice_of_the_staged_prompt_kernel(ops, d, R, nkv):
