@@ -77,7 +77,7 @@ int ms_gemm_ring_qkv(const float* x, long long ldx, const float* norm_w, float e
                      const int* positions, const float* inv_freq, const int* slot_mapping, void* q_out, void* k_pages,
                      void* v_pages, int M, int K, int num_heads, int num_kv_heads, int head_dim, int page_size,
                      int v_transposed, hipStream_t stream);
-// 17 to 64 rows by a W that has to be read from memory (parts > 1: partial sums); ms_gemm_slab_parts: column parts it is to be
+// 5 to 64 rows by a W that has to be read from memory (parts > 1: partial sums); ms_gemm_slab_parts: column parts it is to be
 // called with (0: another kernel is the faster one), sums: for a reader that adds partial sums up itself.
 int ms_gemm_slab_parts(int M, int N, int K, int sums);
 int ms_gemm_slab(const void* A, long long lda, const void* W, long long ldw, const float* bias, void* out, long long ldo, int M,

@@ -268,16 +268,16 @@ extern "C" int ms_gemm_skinny(const void* A, long long lda, const void* W, long 
                               long long ldo, int M, int N, int K, int epilogue, int out_dtype, hipStream_t stream) {
   if (M <= 0 || N <= 0) return MS_OK;
   if (M > 64) return MS_UNSUPPORTED;
+  if (!forced() && ms_gemm_slab_parts(M, N, K, 0)) {   // 9 to 64 rows and a W that has to be read from memory
+    const int rc = ms_gemm_slab(A, lda, W, ldw, bias, out, ldo, M, N, K, epilogue, out_dtype, 1, stream);
+    if (rc != MS_UNSUPPORTED) return rc;
+  }
   if (M <= 16 && !forced()) {   // one token group: a ring through LDS for a large W, units of four rows or the streaming kernel
     int rc = ms_gemm_ring(A, lda, nullptr, nullptr, 0.f, W, ldw, bias, out, ldo, M, N, K, epilogue, out_dtype, 0, 0, stream);
     if (rc != MS_UNSUPPORTED) return rc;
     rc = ms_gemm_quads(A, lda, nullptr, nullptr, 0.f, W, ldw, bias, out, ldo, M, N, K, epilogue, out_dtype, 0, stream);
     if (rc != MS_UNSUPPORTED) return rc;
     rc = ms_gemm_stream(A, lda, nullptr, nullptr, 0.f, W, ldw, bias, out, ldo, M, N, K, epilogue, out_dtype, 0, 0, stream);
-    if (rc != MS_UNSUPPORTED) return rc;
-  }
-  if (!forced() && ms_gemm_slab_parts(M, N, K, 0)) {   // 17 to 64 rows and a W that has to be read from memory
-    const int rc = ms_gemm_slab(A, lda, W, ldw, bias, out, ldo, M, N, K, epilogue, out_dtype, 1, stream);
     if (rc != MS_UNSUPPORTED) return rc;
   }
   if (!forced()) {    // the kernel that holds the activations in LDS, where it takes the shape

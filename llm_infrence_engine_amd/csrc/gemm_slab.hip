@@ -1,4 +1,4 @@
-// out[M,N] = A[M,K] . W[N,K]^T for 17 to 64 tokens (a decode step of a larger batch) and a W that has to be read from memory,
+// out[M,N] = A[M,K] . W[N,K]^T for 5 to 64 tokens (a decode step of a batch) and a W that has to be read from memory,
 // bfloat16 in, float accumulation on the matrix cores (v_mfma_f32_16x16x32_bf16).
 //
 // What bounds it: reading W once.  A block owns a slab of up to 160 rows of W (or a run of their columns, where the rows are
@@ -318,16 +318,20 @@ int plan(const bf16* A, size_t lda, const bf16* W, size_t ldw, const float* bias
 }  // namespace
 
 // The column parts this kernel is to take for a product of M rows with W[N, K], 0 where another kernel is the faster one.
-// The lines go by W alone beside the 17 to 64 rows, so that a row's bits do not hang on how many there are.  The plain product from
+// With a reader that adds sums up from 9 rows on, and by rows of 8,192 columns and more from 5 (a layer's norms and four
+// products, the norms folded in and W ringed or streamed | here: 896 wide 22.3 | 25.7 us at 8 rows, 26.3 | 25.6 at 9, 29.1 | 26.0 at 16;
+// 2,048 wide 51.2 | 47.4 at 4, 59.2 | 48.8 at 16; 3,584 wide 97 | 95 at 8, 115 | 95 at 16; 5,120 wide 188 | 179 and 229 | 181); other
+// products from 17 on, and from 9 on by a W of 8 million values (9,728 x 896 7.0 us at 16 rows, 7.6 with the norm folded in).
+// The lines go by W alone beside the number of rows, so that a row's bits do not hang on how many there are.  The plain product from
 // 4 million values of W on (896 x 4,864: 8.5 against 11.3 us at 17 tokens, 12.0 against 11.6 at 64; 1,152 x 896 3.9 | 4.0 and
 // 5.0 | 5.5, 896 x 896 4.2 | 4.1 and 5.4 | 4.2), but for short rows in several slabs to a CU, whose start and end each pays for
 // (151,936 x 896: 64 to 85 against 65 to 83).  Four parts for a reader that adds sums up itself from 896 x 896 on (4.0 against
 // 4.2, and no read of the residual stream), as long as a slab of four takes the rows; rows of 8,192 columns and more
 // go in four parts even when a kernel has to add them up (3,584 x 18,944: 33.4 + 5 us against 55.8 whole).
 extern "C" int ms_gemm_slab_parts(int M, int N, int K, int sums) {
-  if (M <= 16 || M > MAX_ROWS || N <= 0 || K <= 0 || K % 8 || K > MAX_STRIDE) return 0;
+  if (M <= (sums && K >= 8192 ? 4 : 8) || M > MAX_ROWS || N <= 0 || K <= 0 || K % 8 || K > MAX_STRIDE) return 0;
   const long long values = (long long)N * K;
-  if (sums ? (values < 750000 || K < 768) : values < 4000000) return 0;
+  if (sums ? (values < 750000 || K < 768) : values < (M <= 16 ? 8000000 : 4000000)) return 0;
   const int cus = ms_compute_units();
   if (N > cus * MAX_TILES * 16 && K < 2048) return 0;
   if (N > cus * MAX_TILES * 4 || (!sums && K < 8192)) return 1;

@@ -42,9 +42,10 @@ __device__ __forceinline__ MaxIdx better(MaxIdx a, MaxIdx b) {  // larger value,
   return a;
 }
 
-__device__ MaxIdx block_argmax(const float* __restrict__ row, int V, MaxIdx* red) {
+// The first maximum of row[begin..end); index 0x7fffffff: there is none but NaN.
+__device__ MaxIdx block_argmax(const float* __restrict__ row, int begin, int end, MaxIdx* red) {
   MaxIdx best = {-INFINITY, 0x7fffffff};
-  for (int i = threadIdx.x; i < V; i += blockDim.x) best = better(best, MaxIdx{row[i], i});
+  for (int i = begin + threadIdx.x; i < end; i += blockDim.x) best = better(best, MaxIdx{row[i], i});
   for (int o = MS_WAVE / 2; o > 0; o >>= 1) {
     MaxIdx other = {__shfl_xor(best.v, o, MS_WAVE), __shfl_xor(best.i, o, MS_WAVE)};
     best = better(best, other);
@@ -55,7 +56,6 @@ __device__ MaxIdx block_argmax(const float* __restrict__ row, int V, MaxIdx* red
   __syncthreads();
   MaxIdx r = red[0];
   for (int w = 1; w < (int)(blockDim.x / MS_WAVE); ++w) r = better(r, red[w]);
-  if (r.i == 0x7fffffff) r.i = 0;  // a row of NaN or -inf only
   return r;
 }
 
@@ -80,7 +80,7 @@ constexpr int FIX_PLACES = 44;
 
 struct RowWork {                     // one per row, in the workspace the caller brings
   // Every field is written by one kernel (block 0 of the row) and read by later kernels only.
-  unsigned chunk_max[MAX_CHUNKS];    // key of the largest scaled logit of every chunk
+  unsigned chunk_max[MAX_CHUNKS];    // key of the largest scaled logit of every chunk (no temperature: the largest itself)
   unsigned k_digits[2];              // digits of the top-k key after the searches of levels 1 and 2
   unsigned p_digits[2];              // and of the top-p key
   unsigned top_k_key;                // the top-k key itself (0: top-k keeps everything)
@@ -90,7 +90,7 @@ struct RowWork {                     // one per row, in the workspace the caller
   unsigned long long k_mass_above[2];
   unsigned long long p_mass_above[2];
   unsigned long long total;          // mass of the tokens that top-k keeps
-  unsigned long long chunk_mass[MAX_CHUNKS];
+  unsigned long long chunk_mass[MAX_CHUNKS];   // (no temperature: where the largest stands)
   unsigned count[N_HIST][RADIX_BINS];
   unsigned long long mass[N_HIST][RADIX_BINS];
 };
@@ -168,11 +168,13 @@ __device__ __forceinline__ void chunk_range(int V, int n_chunks, int c, int* beg
   *end = min(V, *begin + len);
 }
 
-// Stage 0: every chunk's largest key, and the workspace made ready (histograms and sums zero).
+// Stage 0: every chunk's largest key, and the workspace made ready (histograms and sums zero).  Of a row without temperature
+// every chunk's first maximum (one block that went through the row in the last kernel took 52 us for 151,936 logits).
 __global__ void __launch_bounds__(THREADS)
 sample_max_kernel(const float* __restrict__ logits, size_t ld, int V, const float* __restrict__ temperature,
                   RowWork* __restrict__ work, int n_chunks) {
   __shared__ unsigned red[THREADS / MS_WAVE];
+  __shared__ MaxIdx red_mi[THREADS / MS_WAVE];
   const int r = blockIdx.y, c = blockIdx.x;
   RowWork& w = work[r];
   // this block's share of the row's histograms
@@ -181,11 +183,15 @@ sample_max_kernel(const float* __restrict__ logits, size_t ld, int V, const floa
   for (int i = c * THREADS + threadIdx.x; i < N_HIST * RADIX_BINS; i += n_chunks * THREADS) { zc[i] = 0u; zm[i] = 0ull; }
   if (threadIdx.x == 0) { w.chunk_mass[c] = 0ull; w.chunk_max[c] = 0u; }
   const float T = temperature[r];
-  if (!(T > 0.f)) return;
-  const float inv_t = 1.0f / T;
   const float* row = logits + (size_t)r * ld;
   int begin, end;
   chunk_range(V, n_chunks, c, &begin, &end);
+  if (!(T > 0.f)) {
+    const MaxIdx top = block_argmax(row, begin, end, red_mi);
+    if (threadIdx.x == 0) { w.chunk_max[c] = __float_as_uint(top.v); w.chunk_mass[c] = (unsigned)top.i; }
+    return;
+  }
+  const float inv_t = 1.0f / T;
   unsigned best = 0;
   for (int i = begin + threadIdx.x; i < end; i += blockDim.x) {
     const float s = row[i] * inv_t;
@@ -345,8 +351,11 @@ sample_draw_kernel(const float* __restrict__ logits, size_t ld, int V, const flo
   const float* row = logits + (size_t)r * ld;
   const float T = temperature[r];
   if (!(T > 0.f)) {
-    const MaxIdx top = block_argmax(row, V, red_mi);
-    if (threadIdx.x == 0) out[r] = top.i;
+    if (threadIdx.x == 0) {
+      MaxIdx top = {-INFINITY, 0x7fffffff};
+      for (int c = 0; c < n_chunks; ++c) top = better(top, MaxIdx{__uint_as_float(work[r].chunk_max[c]), (int)work[r].chunk_mass[c]});
+      out[r] = top.i == 0x7fffffff ? 0 : top.i;   // (a row of NaN only)
+    }
     return;
   }
   RowWork& w = work[r];
@@ -397,8 +406,8 @@ sample_draw_kernel(const float* __restrict__ logits, size_t ld, int V, const flo
     if (threadIdx.x == 0) out[r] = pick;
     return;
   }
-  const MaxIdx top = block_argmax(row, V, red_mi);   // no mass at all (a row of NaN or -inf): as the greedy choice
-  if (threadIdx.x == 0) out[r] = top.i;
+  const MaxIdx top = block_argmax(row, 0, V, red_mi);   // no mass at all (a row of NaN or -inf): as the greedy choice
+  if (threadIdx.x == 0) out[r] = top.i == 0x7fffffff ? 0 : top.i;
 }
 
 // First maximum of a row in two stages, so that a few rows still use the whole chip: stage 1 finds the best

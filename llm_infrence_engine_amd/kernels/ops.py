@@ -638,8 +638,8 @@ def gemm_slab(a: torch.Tensor, w: torch.Tensor, bias: Optional[torch.Tensor] = N
 
 
 def gemm_slab_qkv_pays(a, w_qkv: torch.Tensor, head_dim: int, rot_dim: int, k_pages: torch.Tensor) -> bool:
-    """Whether ``gemm_slab_qkv`` takes these normed rows (17 to 64, heads rotated whole): it spares the rotation's launch."""
-    return (isinstance(a, torch.Tensor) and a.dtype == torch.bfloat16 and STREAM_MAX_ROWS < a.shape[0] <= SKINNY_MAX_ROWS
+    """Whether ``gemm_slab_qkv`` takes these normed rows (5 to 64, heads rotated whole): it spares the rotation's launch."""
+    return (isinstance(a, torch.Tensor) and a.dtype == torch.bfloat16 and 4 < a.shape[0] <= SKINNY_MAX_ROWS
             and skinny_ok(a, w_qkv) and rot_dim == head_dim and head_dim % 2 == 0 and k_pages.dtype == torch.bfloat16
             and w_qkv.shape[0] <= 0xffff and w_qkv.numel() < 1 << 31 and max(w_qkv.shape[1], a.stride(0)) <= 1 << 22)
 

@@ -672,7 +672,7 @@ def test_a_large_matrix_goes_to_the_ring(ops, M):
         a = torch.randn(M, K, generator=g).bfloat16().to(DEV)
         w = (torch.randn(N, K, generator=g) / math.sqrt(K)).bfloat16().to(DEV)
         f = ops.gemm_skinny(a, w, out_dtype=torch.float32)
-        assert torch.equal(f, ops.gemm_ring(a, w, out_dtype=torch.float32)) == (N * K >= 24000000)
+        assert torch.equal(f, ops.gemm_ring(a, w, out_dtype=torch.float32)) == (N * K >= 24000000 and M <= 8)
         want = a.double() @ w.double().T
         torch.testing.assert_close(f.double(), want, atol=3e-5, rtol=3e-5)
         torch.testing.assert_close(ops.gemm_skinny(a, w, None, ops.EPI_RELU2).double(), want.clamp(min=0) ** 2, **tol(torch.bfloat16))
@@ -685,7 +685,7 @@ def test_a_large_matrix_goes_to_the_ring(ops, M):
         _qkv_fused_case(ops, M, 72, 5, 64, 4616, False)
 
 
-@pytest.mark.parametrize("M", [17, 33, 64])
+@pytest.mark.parametrize("M", [1, 9, 17, 33, 64])
 @pytest.mark.parametrize("N,K", [(2, 64), (6, 8), (898, 1032), (1030, 264), (5120, 520), (16 * 256 * 10 + 6, 136), (2560, 9000),
                                  (16 * 256 * 10 * 2 + 20, 72)])
 def test_gemm_slab(ops, M, N, K):
@@ -713,13 +713,13 @@ def test_gemm_slab(ops, M, N, K):
     gate, up = want[:, 0::2].clamp(max=1.5), want[:, 1::2].clamp(-1.5, 1.5)
     torch.testing.assert_close(ops.gemm_slab(a, w, numbers, ops.EPI_CLAMPED).double(), gate * torch.sigmoid(1.702 * gate) * (up + 1),
                                **tol(torch.bfloat16))
-    assert torch.equal(ops.gemm_slab(a[M - 17:], w, bias), out[M - 17:])
+    assert torch.equal(ops.gemm_slab(a[max(0, M - 17):], w, bias), out[max(0, M - 17):])
     b = a.clone()
     b[0, K - 1] = float("nan")
     assert torch.equal(ops.gemm_slab(b, w, bias)[1:], out[1:])
 
 
-@pytest.mark.parametrize("M", [17, 40, 64])
+@pytest.mark.parametrize("M", [5, 8, 9, 16, 17, 40, 64])
 @pytest.mark.parametrize("N,K", [(896, 896), (900, 1000), (3584, 776), (640, 9000), (10240, 768), (10248, 768), (512, 8192)])
 def test_few_rows_by_a_large_matrix_go_to_slabs(ops, M, N, K):
     """Both sides of the lines on the size of W and on its rows: partial sums for a reader that adds them up (the RMS norm,
@@ -734,7 +734,7 @@ def test_few_rows_by_a_large_matrix_go_to_slabs(ops, M, N, K):
     ops.gemm_skinny(a, w, None, ops.EPI_RESIDUAL, residual=x)
     torch.testing.assert_close(x.double(), x0 + want, atol=3e-5, rtol=3e-5)
     parts = ops.gemm_sums(a, w)
-    assert (parts is not None) == (750000 <= N * K and N <= 10240)
+    assert (parts is not None) == (750000 <= N * K and N <= 10240 and M > (4 if K >= 8192 else 8))
     if parts is None:
         return
     assert parts.shape == (4, M, N)
@@ -814,6 +814,39 @@ def test_gemm_tiled_sums(ops, M, N, K, parts, tile):
     h = ops.rms_norm(x, nw, 1e-6, torch.empty(M, N, dtype=torch.bfloat16, device=DEV), delta=got)
     torch.testing.assert_close(h.double(), normed, **tol(torch.bfloat16))
     torch.testing.assert_close(x.double(), total, atol=3e-5, rtol=3e-5)
+
+
+@pytest.mark.parametrize("V", [5, 2048, 2049, 40000, 151936])
+def test_greedy_rows_among_drawn_ones(ops, V):
+    """Rows without temperature in a call that draws others: the first of equal maxima, on either side of a chunk's edge, +0 and
+    -0 equal, NaN never, -inf only (the first) and NaN only (0); many rows and few, which are cut into other chunks."""
+    g = torch.Generator().manual_seed(V)
+    for M in (3, 40):
+        x = torch.randn(M, V, generator=g)
+        want = torch.empty(M, dtype=torch.int32)
+        for r in range(M):
+            if r % 8 == 1:
+                at = sorted(torch.randperm(V, generator=g)[:3].tolist())
+                x[r, at] = 50.0
+                x[r, (at[0] + 1) % V if V > 5 and (at[0] + 1) % V not in at else at[0]] = float("nan") if V > 5 else 50.0
+            if r % 8 == 2:
+                x[r] = -x[r].abs() - 1
+                x[r, V // 3], x[r, V // 2] = -0.0, 0.0
+            if r % 8 == 3:
+                x[r] = -math.inf
+            if r % 8 == 4:
+                x[r] = float("nan")
+            y = torch.where(torch.isnan(x[r]), torch.full_like(x[r], -math.inf), x[r])
+            first = int((y == y.max()).nonzero()[0])
+            want[r] = 0 if torch.isnan(x[r]).all() else first
+        T = torch.zeros(M)
+        T[0], T[-1] = 1.0, -1.0
+        logits = x.to(DEV)
+        out = torch.full((M,), -1, dtype=torch.int32, device=DEV)
+        top_k, top_p = torch.full((M,), 3, dtype=torch.int32, device=DEV), torch.full((M,), 0.9, device=DEV)
+        ops.sample(logits, out, T.to(DEV), top_k, top_p, torch.arange(M, device=DEV), torch.zeros(M, dtype=torch.int32, device=DEV))
+        assert torch.equal(out.cpu()[1:], want[1:])
+        assert 0 <= int(out[0]) < V
 
 
 def test_gemm_stream_refuses_what_it_cannot_take(ops):
