@@ -42,10 +42,25 @@ __device__ __forceinline__ MaxIdx better(MaxIdx a, MaxIdx b) {  // larger value,
   return a;
 }
 
+// f(i, row[i]) for this thread's share of row[begin..end), in no particular order; eight loads under way at a time (64 rows of
+// 151,936 with top-k and top-p, 19 logits a thread: 143 -> 124 us; up to 16 rows, at most 10 logits a thread, no difference).
+template <typename F>
+__device__ __forceinline__ void for_share(const float* __restrict__ row, int begin, int end, F f) {
+  constexpr int AT_ONCE = 8;
+  for (int base = begin + threadIdx.x; base < end; base += AT_ONCE * THREADS) {
+    float v[AT_ONCE];
+#pragma unroll
+    for (int j = 0; j < AT_ONCE; ++j) v[j] = row[min(base + j * THREADS, end - 1)];
+#pragma unroll
+    for (int j = 0; j < AT_ONCE; ++j)
+      if (base + j * THREADS < end) f(base + j * THREADS, v[j]);
+  }
+}
+
 // The first maximum of row[begin..end); index 0x7fffffff: there is none but NaN.
 __device__ MaxIdx block_argmax(const float* __restrict__ row, int begin, int end, MaxIdx* red) {
   MaxIdx best = {-INFINITY, 0x7fffffff};
-  for (int i = begin + threadIdx.x; i < end; i += blockDim.x) best = better(best, MaxIdx{row[i], i});
+  for_share(row, begin, end, [&](int i, float v) { best = better(best, MaxIdx{v, i}); });
   for (int o = MS_WAVE / 2; o > 0; o >>= 1) {
     MaxIdx other = {__shfl_xor(best.v, o, MS_WAVE), __shfl_xor(best.i, o, MS_WAVE)};
     best = better(best, other);
@@ -193,10 +208,10 @@ sample_max_kernel(const float* __restrict__ logits, size_t ld, int V, const floa
   }
   const float inv_t = 1.0f / T;
   unsigned best = 0;
-  for (int i = begin + threadIdx.x; i < end; i += blockDim.x) {
-    const float s = row[i] * inv_t;
+  for_share(row, begin, end, [&](int, float v) {
+    const float s = v * inv_t;
     if (s == s) best = max(best, order_key(s));     // NaN never wins
-  }
+  });
   for (int o = MS_WAVE / 2; o > 0; o >>= 1) best = max(best, (unsigned)__shfl_xor((int)best, o, MS_WAVE));
   if ((threadIdx.x & (MS_WAVE - 1)) == 0) red[threadIdx.x / MS_WAVE] = best;
   __syncthreads();
@@ -279,15 +294,15 @@ sample_level_kernel(const float* __restrict__ logits, size_t ld, int V, const fl
   const float* row = logits + (size_t)r * ld;
   int begin, end;
   chunk_range(V, n_chunks, c, &begin, &end);
-  for (int i = begin + threadIdx.x; i < end; i += blockDim.x) {
-    const float s = row[i] * inv_t;
-    if (!(s == s)) continue;
+  for_share(row, begin, end, [&](int, float v) {
+    const float s = v * inv_t;
+    if (!(s == s)) return;
     const unsigned key = order_key(s);
-    if (level > 1 && (key >> (shift + (level == 2 ? 11 : 10))) != digits) continue;
+    if (level > 1 && (key >> (shift + (level == 2 ? 11 : 10))) != digits) return;
     const int bin = (int)((key >> shift) & (unsigned)(bins - 1));
     atomicAdd(&lc[bin], 1u);
     atomicAdd(&lm[bin], fixed_mass(s, zmax));
-  }
+  });
   __syncthreads();
   for (int i = threadIdx.x; i < bins; i += blockDim.x)
     if (lc[i]) {
@@ -323,10 +338,10 @@ sample_chunk_mass_kernel(const float* __restrict__ logits, size_t ld, int V, con
   int begin, end;
   chunk_range(V, n_chunks, c, &begin, &end);
   unsigned long long mine = 0;
-  for (int i = begin + threadIdx.x; i < end; i += blockDim.x) {
-    const float s = row[i] * inv_t;
+  for_share(row, begin, end, [&](int, float v) {
+    const float s = v * inv_t;
     if (s == s && order_key(s) >= floor_key) mine += fixed_mass(s, zmax);
-  }
+  });
   for (int o = MS_WAVE / 2; o > 0; o >>= 1) mine += __shfl_xor(mine, o, MS_WAVE);
   if ((threadIdx.x & (MS_WAVE - 1)) == 0) red[threadIdx.x / MS_WAVE] = mine;
   __syncthreads();
@@ -375,9 +390,15 @@ sample_draw_kernel(const float* __restrict__ logits, size_t ld, int V, const flo
   const int per = (end - begin + (int)blockDim.x - 1) / (int)blockDim.x;
   const int lo = min(end, begin + (int)threadIdx.x * per), hi = min(end, lo + per);
   unsigned long long mine = 0;
-  for (int i = lo; i < hi; ++i) {
-    const float s = row[i] * inv_t;
-    if (s == s && order_key(s) >= floor_key) mine += fixed_mass(s, zmax);
+  for (int i0 = lo; i0 < hi; i0 += 8) {              // (eight loads under way at a time here too)
+    float v[8];
+#pragma unroll
+    for (int j = 0; j < 8; ++j) v[j] = row[min(i0 + j, hi - 1)];
+#pragma unroll
+    for (int j = 0; j < 8; ++j) {
+      const float s = v[j] * inv_t;
+      if (i0 + j < hi && s == s && order_key(s) >= floor_key) mine += fixed_mass(s, zmax);
+    }
   }
   // exclusive sums over the threads, in thread (that is, index) order
   const int lane = threadIdx.x & (MS_WAVE - 1), wave = threadIdx.x / MS_WAVE;
