@@ -43,7 +43,7 @@ template <typename T, typename TD>
 __global__ void rms_norm_kernel(float* __restrict__ x, const TD* __restrict__ delta, int n_partials,
                                 size_t partial_stride, const float* __restrict__ w,
                                 const int* __restrict__ rows, T* __restrict__ out, int H, float eps, int write_back,
-                                int staged) {
+                                int staged, int quads) {
   __shared__ float red[16];
   extern __shared__ float buf[];  // H floats: the row after the residual sum (a row too wide for it is read twice)
   const int r = blockIdx.x;
@@ -51,7 +51,7 @@ __global__ void rms_norm_kernel(float* __restrict__ x, const TD* __restrict__ de
   float* xr = x + (size_t)src * H;
   T* o = out + (size_t)r * H;
   float ss = 0.f;
-  if (H % 4 == 0 && staged) {  // four values at a time (rows start 16-byte aligned when H % 4 == 0)
+  if (quads && staged) {   // four values at a time: every row of every operand starts at an address that fits them
     const TD* dr = delta ? delta + (size_t)src * H : nullptr;
     for (int i = threadIdx.x * 4; i < H; i += blockDim.x * 4) {
       float4 v = *reinterpret_cast<const float4*>(xr + i);
@@ -107,12 +107,15 @@ extern "C" int ms_rms_norm(float* x, const void* delta, int delta_dtype, int n_p
   if (hidden <= 0) return MS_BAD_ARG;
   dim3 grid(n_rows), block(hidden >= 1024 ? 256 : 128);
   // a thread for every four values where every row has a CU of its own and several sums are read: one round of loads
-  if (n_partials > 1 && hidden % 4 == 0 && n_rows <= ms_compute_units()) block = dim3(std::min(1024, (hidden / 4 + 63) / 64 * 64));
+  const size_t out_quad = dtype == MS_BF16 ? 8 : 16, delta_quad = dtype == MS_BF16 && delta_dtype == MS_BF16 ? 8 : 16;
+  const int quads = hidden % 4 == 0 && ((uintptr_t)x | (uintptr_t)weight) % 16 == 0 && (uintptr_t)out % out_quad == 0 &&
+                    (!delta || ((uintptr_t)delta % delta_quad == 0 && (n_partials == 1 || partial_stride % 4 == 0)));
+  if (n_partials > 1 && quads && n_rows <= ms_compute_units()) block = dim3(std::min(1024, (hidden / 4 + 63) / 64 * 64));
   // the row is staged in LDS while it fits what a launch may ask for without more ado (64 KB with the 64 bytes
   // of the reduction); a wider row is read from memory a second time instead
   const int staged = (size_t)hidden * sizeof(float) + 64 <= 65536 ? 1 : 0;
   size_t lds = staged ? (size_t)hidden * sizeof(float) : 0;
-#define LAUNCH(T, TD) rms_norm_kernel<T, TD><<<grid, block, lds, stream>>>(x, (const TD*)delta, n_partials, (size_t)partial_stride, weight, rows, (T*)out, hidden, eps, write_back, staged)
+#define LAUNCH(T, TD) rms_norm_kernel<T, TD><<<grid, block, lds, stream>>>(x, (const TD*)delta, n_partials, (size_t)partial_stride, weight, rows, (T*)out, hidden, eps, write_back, staged, quads)
   if (dtype == MS_F32) {
     if (delta && delta_dtype == MS_BF16) return MS_BAD_ARG;
     LAUNCH(float, float);

@@ -849,6 +849,26 @@ def test_greedy_rows_among_drawn_ones(ops, V):
         assert 0 <= int(out[0]) < V
 
 
+@pytest.mark.parametrize("delta", [None, "bfloat16", "sums"])
+def test_rms_norm_of_rows_at_odd_addresses(ops, delta):
+    """Operands that start between two groups of four values are read one value at a time."""
+    g = torch.Generator().manual_seed(3)
+    N, H = 5, 900
+    x = torch.randn(N * H + 1, generator=g).to(DEV)[1:].view(N, H)
+    out = torch.zeros(N * H + 1, dtype=torch.bfloat16, device=DEV)[1:].view(N, H)
+    nw = (1 + 0.1 * torch.randn(H + 1, generator=g)).to(DEV)[1:]
+    d = None
+    if delta == "bfloat16":
+        d = torch.randn(N * H + 1, generator=g).bfloat16().to(DEV)[1:].view(N, H)
+    elif delta == "sums":
+        d = torch.randn(3 * N * H + 1, generator=g).to(DEV)[1:].view(3, N, H)
+    total = x.double() + (0 if d is None else d.double().view(-1, N, H).sum(0))
+    ops.rms_norm(x, nw, 1e-6, out, delta=d)
+    want = total * torch.rsqrt((total * total).mean(-1, keepdim=True) + 1e-6) * nw.double()
+    torch.testing.assert_close(out.double(), want, **tol(torch.bfloat16))
+    torch.testing.assert_close(x.double(), total, atol=3e-6, rtol=3e-6)
+
+
 def test_gemm_stream_refuses_what_it_cannot_take(ops):
     w = torch.zeros(64, 64, dtype=torch.bfloat16, device=DEV)
     with pytest.raises(RuntimeError, match="unsupported"):
