@@ -543,7 +543,7 @@ def gemm_skinny(a: torch.Tensor, w: torch.Tensor, bias: Optional[torch.Tensor] =
     if not gated and epilogue != EPI_RELU2 and split_columns:
         # long rows against few of them (a down projection): the columns are split over blocks too, and the
         # partial sums are added up in a fixed order by a second kernel
-        parts = _get("ms_gemm_slab_parts")(M, N, K, 0)
+        parts = _slab_parts(a, w)
         if parts > 1:
             partial = _slab_sums(a, w, lda, parts)
             _call("ms_add_partials", partial.data_ptr(), parts, _ptr(bias), out.data_ptr(), ldo, M, N, epilogue, _code(out_dtype),
@@ -568,8 +568,19 @@ def _rings(M: int, N: int, K: int) -> bool:
 def splits_columns(a: torch.Tensor, w: torch.Tensor) -> bool:
     """Whether ``gemm_skinny`` spreads the columns of this product over blocks (its sums then pass a second kernel)."""
     (M, K), N = a.shape, w.shape[0]
-    parts = _get("ms_gemm_slab_parts")(M, N, K, 0)
+    parts = _slab_parts(a, w)
     return parts > 1 if parts else not _rings(M, N, K) and _get("ms_gemm_panel_splitk_parts")(M, N, K) > 1
+
+
+SLAB_MAX_STRIDE = 1 << 22     # values between two rows that the slabs' kernel reaches over
+
+
+def _slab_parts(a: torch.Tensor, w: torch.Tensor, sums: bool = False) -> int:
+    """Column parts the slabs' kernel is to be called with (``sums``: for a reader that adds them up itself), 0: it is not the
+    faster one, or does not take rows as far apart as these."""
+    if a.shape[0] > 1 and a.stride(0) > SLAB_MAX_STRIDE:
+        return 0
+    return _get("ms_gemm_slab_parts")(a.shape[0], w.shape[0], w.shape[1], int(sums))
 
 
 def _slab_sums(a: torch.Tensor, w: torch.Tensor, lda: int, parts: int) -> torch.Tensor:
@@ -596,7 +607,7 @@ def gemm_sums(a: torch.Tensor, w: torch.Tensor) -> Optional[torch.Tensor]:
         return gemm_tiled_sums(a, w, parts) if parts else None
     if not skinny_ok(a, w):
         return None
-    parts = _get("ms_gemm_slab_parts")(M, N, K, 1)
+    parts = _slab_parts(a, w, True)
     if parts <= 1:
         return None
     _check(a, "a", torch.bfloat16, contiguous=False)
@@ -641,7 +652,7 @@ def gemm_slab_qkv_pays(a, w_qkv: torch.Tensor, head_dim: int, rot_dim: int, k_pa
     """Whether ``gemm_slab_qkv`` takes these normed rows (5 to 64, heads rotated whole): it spares the rotation's launch."""
     return (isinstance(a, torch.Tensor) and a.dtype == torch.bfloat16 and 4 < a.shape[0] <= SKINNY_MAX_ROWS
             and skinny_ok(a, w_qkv) and rot_dim == head_dim and head_dim % 2 == 0 and k_pages.dtype == torch.bfloat16
-            and w_qkv.shape[0] <= 0xffff and w_qkv.numel() < 1 << 31 and max(w_qkv.shape[1], a.stride(0)) <= 1 << 22)
+            and w_qkv.shape[0] <= 0xffff and w_qkv.numel() < 1 << 31 and max(w_qkv.shape[1], a.stride(0)) <= SLAB_MAX_STRIDE)
 
 
 def gemm_slab_qkv(a: torch.Tensor, w_qkv: torch.Tensor, bias: Optional[torch.Tensor], num_heads: int, num_kv_heads: int,

@@ -752,6 +752,28 @@ def test_few_rows_by_a_large_matrix_go_to_slabs(ops, M, N, K):
     torch.testing.assert_close(x.double(), total, atol=3e-5, rtol=3e-5)
 
 
+@pytest.mark.parametrize("M", [9, 17])
+def test_rows_too_far_apart_for_slabs_go_to_the_other_kernels(ops, M):
+    """Rows up to 4,194,304 values apart go through slabs, farther ones as before: long rows in partial sums (plain, into the
+    residual stream, and for a reader that would have added them up) and a plain product."""
+    from llm_infrence_engine_amd.kernels import linear
+
+    far = (1 << 22) + 8
+    flat = torch.zeros((M - 1) * far + 8200, dtype=torch.bfloat16, device=DEV)
+    g = torch.Generator().manual_seed(M)
+    for N, K in ((1040, 8200), (4200, 2000)):
+        a = flat.as_strided((M, K), (far, 1))
+        a.copy_(torch.randn(M, K, generator=g).bfloat16())
+        w = (torch.randn(N, K, generator=g) / math.sqrt(K)).bfloat16().to(DEV)
+        want = a.double() @ w.double().T
+        near = flat.as_strided((M, K), (far - 8, 1))
+        assert ops.splits_columns(near, w) == (K >= 8192) and ops.gemm_sums(a, w) is None and ops.gemm_sums(near, w) is not None
+        torch.testing.assert_close(ops.gemm_skinny(a, w, out_dtype=torch.float32).double(), want, atol=5e-5, rtol=5e-5)
+        x = torch.zeros(M, N, device=DEV)
+        assert linear.linear_residual(a, w, None, x, True) is None
+        torch.testing.assert_close(x.double(), want, atol=5e-5, rtol=5e-5)
+
+
 @pytest.mark.parametrize("M", [17, 48, 64])
 @pytest.mark.parametrize("nh,nkv,d,K,v_transposed", [(14, 2, 64, 896, True), (5, 1, 128, 520, False), (3, 3, 6, 72, False), (70, 5, 64, 136, True)])
 def test_gemm_slab_qkv_equals_product_rotation_and_store(ops, M, nh, nkv, d, K, v_transposed):
