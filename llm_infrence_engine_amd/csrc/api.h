@@ -129,7 +129,7 @@ int ms_qkv_rope_store(const float* x, long long ldx, const float* norm_w, float 
                       int page_size, int v_transposed, hipStream_t stream);
 
 int ms_attention_prompt_kind(int n_requests, int n_tokens, int max_q_len, int max_context_len, int num_heads, int num_kv_heads,
-                             int head_dim, int page_size, int window);   // 0: ms_paged_attention_mfma; 1 to 3: a kind of
+                             int head_dim, int page_size, int window, int exact);   // 0: ms_paged_attention_mfma; 1 to 3: a kind of
 int ms_attention_prompt_as(int kind, const void* q, long long q_stride, const void* k_pages, const void* vt_pages,
                            const int* block_table, int table_stride, const int* table_rows, const int* q_start,
                            const int* context_lens, void* out, long long out_stride, int n_requests, int n_tokens, int max_q_len,

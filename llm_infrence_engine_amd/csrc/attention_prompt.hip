@@ -391,38 +391,56 @@ extern "C" int ms_attention_prompt_pays(int n_requests, int n_tokens, int max_q_
   return !uneven && blocks * 16 >= cus * (short_chains ? 7 : 24);
 }
 
-// Which kernel a step's attention should take: 0 ms_paged_attention_mfma, else a kind of this one.  Between the other kernel and
-// the wide kind ms_attention_prompt_pays decides; one of the narrow kinds takes the step where a model of the measurements
-// puts it 6 % ahead of that.  The model, in us: a start, the cube root of the sum of cubes of the longest chain (in tiles of 64
-// keys) and of the work a CU has (blocks of 128 columns a CU times the mean tile's keys), and a little a block; its terms fitted
-// to 320 and 250 random steps (64 and 128 dims; 1 to 40 requests, portions of up to 4,096 tokens alone, behind up to 8,000 keys,
-// and beside single tokens; residuals 6 to 13 %).  There the choice takes 0.81 and 0.93 of the time of the choice between
-// the other two, at most 1.06 and 1.16 of it.  Steps of a few tokens a request stay with the other kernel (30 requests of 2 tokens 5.4
-// and 6.0 us).  14 heads on 2 of 64 dims: 386 tokens 12.1 -> 9.9 us, 1,158 23.3 -> 18.2, 2,912 tokens behind 4,688 141 -> 119; 28
-// heads on 4 of 128: 910 tokens 29.8 -> 23.3, 2,094 74.7 -> 59.2.
+// Which kernel a step's attention should take: 0 ms_paged_attention_mfma, else a kind of this one.  exact: the two maxima are the
+// step's own; 0: bounds, as a captured step has them, which say nothing of the requests that will be in it.  Between the other
+// kernel and the wide kind ms_attention_prompt_pays decides; the narrow kinds take what they were seen to win over that choice,
+// in 16,000 random exact steps and 6,600 with a capture's bounds (64 and 128 dims; alone, 2 to 48 even or ragged portions, beside
+// single tokens, behind up to 14,000 keys; a quarter with a window).  What decides is how far the wide kind's blocks fill the chip,
+// `fill` a CU: up to one or two all run at once and a CU waits for the longest, which blocks of half the columns cut short, while
+// beyond that they only start and stream the keys twice as often.  Time over that of the choice without:
+//   64 dims, where the other kernel would run: the narrow kind always, 0.63 to 1.05, 0.79 in the middle (with a capture's bounds
+//     0.63 to 0.98); one request that fills 1.5 with 2,048 keys a mean tile twice the groups, 0.82 to 0.98 (3,883 tokens behind
+//     7,000, 14 heads on 2: 201 us, 204 narrow, 176).
+//   64 dims, where the wide kind would: narrow up to a fill of one, 0.69 to 1.02, 0.93 in the middle; beyond 0.73 to 1.28 (8 portions
+//     of 512 tokens, 14 on 2, fill 1.75: 19.1 us wide, 22.2 narrow).
+//   128 dims, where the wide kind would: one portion with most of the tokens and few keys before it, whose tiles are short and
+//     long, up to a fill of two, 0.62 to 1.02, 0.76 in the middle (2,059 tokens of 28 heads on 4 71.9 -> 55.3 us); beyond up to 1.26, and
+//     even portions 0.64 to 1.25.
+//   128 dims, where the other kernel would, whose waves share a long chain: narrow from a fill of 7/8 or of a 512th of the longest
+//     tile's keys (even portions; 0.51 to 1.01, 0.78 in the middle, 1.11 in one of 1,155), 1.5 (one of several with most tokens; 0.57 to
+//     0.88), one (one alone; 0.58 to 0.88) or 5/8 (alone behind its own length of keys and more, or with a window; 0.53 to 0.99), and
+//     alone between 5/8 and one twice the groups (0.62 to 0.89).  Below up to 1.9.
+//   128 dims, several requests with more keys than their longest portion explains, or with bounds: as without.  A single token may
+//     hold them (40 heads on 8, 945 tokens beside 8 decoding ones with 3,535 keys: 57 us, 76 narrow; bounds 0.6 to 1.8).
+// Steps of a few tokens a request stay with the other kernel (30 requests of 2 tokens 5.4 and 6.0 us).
 extern "C" int ms_attention_prompt_kind(int n_requests, int n_tokens, int max_q_len, int max_context_len, int num_heads,
-                                        int num_kv_heads, int head_dim, int page_size, int window) {
+                                        int num_kv_heads, int head_dim, int page_size, int window, int exact) {
   if ((head_dim != 64 && head_dim != 128) || page_size % 16 || num_kv_heads <= 0 || num_heads % num_kv_heads) return 0;
   const int plain = ms_attention_prompt_pays(n_requests, n_tokens, max_q_len, max_context_len, num_heads, num_kv_heads, head_dim, page_size, window)
                         ? PROMPT_WIDE : 0;
-  if (max_q_len <= 16 || (long long)n_tokens * (num_heads / num_kv_heads) / (WIDE / 2) + n_requests > 65535) return plain;
-  double chain = max_context_len, mean = max_context_len - max_q_len / 2;
+  const double rep = num_heads / num_kv_heads;
+  if (max_q_len <= 16 || (double)n_tokens * rep / (WIDE / 2) + n_requests > 65535) return plain;
+  double chain = max_context_len, mean = max_context_len - max_q_len / 2.0;    // keys of the longest tile and of the mean one
   if (window > 0) {
-    chain = std::min(chain, (double)window + WIDE / std::max(1, num_heads / num_kv_heads));
+    chain = std::min(chain, window + WIDE / std::max(1.0, rep));
     mean = std::min(mean, (double)window);
   }
-  const double a_cu = (double)n_tokens * num_heads / WIDE / ms_compute_units();
-  static const double terms[2][4][4] = {   // start, chain, load, blocks: of the other kernel, wide, narrow, narrow with more groups
-      {{7.1, 0.74, 0.58, 5.5}, {7.0, 0.92, 0.40, 3.0}, {5.8, 0.575, 0.65, 3.8}, {8.8, 0.69, 0.52, 5.2}},
-      {{6.0, 0.65, 2.28, 11.3}, {6.5, 1.83, 0.90, 3.9}, {5.6, 1.13, 1.27, 4.8}, {6.3, 0.74, 1.455, 10.1}}};
-  double us[4];
-  for (int k = 0; k < 4; ++k) {
-    const double* t = terms[head_dim == 128][k];
-    const double c = chain / KEYS * t[1], l = a_cu * mean / KEYS * t[2];
-    us[k] = t[0] + cbrt(c * c * c + l * l * l) + a_cu * t[3];
+  const bool alone = n_requests == 1, most = alone || 2LL * n_tokens <= (long long)n_requests * max_q_len;
+  // wide blocks a CU: the portions are of one length, unless one holds most of the tokens
+  const auto blocks = [&](double tokens) { return std::ceil(tokens * rep / WIDE); };
+  const double fill = (alone ? blocks(n_tokens)
+                       : most ? blocks(max_q_len) + (n_requests - 1) * blocks((double)std::max(n_tokens - max_q_len, 1) / (n_requests - 1))
+                              : n_requests * blocks((double)n_tokens / n_requests)) * num_kv_heads / ms_compute_units();
+  if (head_dim == 64) {
+    if (plain) return exact && !alone && fill <= 1.0 ? PROMPT_NARROW : plain;
+    return exact && alone && fill >= 1.5 && mean >= 2048 ? PROMPT_NARROW_GROUPS : PROMPT_NARROW;
   }
-  const int narrow = us[PROMPT_NARROW] <= us[PROMPT_NARROW_GROUPS] ? PROMPT_NARROW : PROMPT_NARROW_GROUPS;
-  return us[narrow] * 1.06 < us[plain] ? narrow : plain;
+  if (!exact || (!alone && chain > 1.5 * max_q_len)) return plain;
+  const bool from_start = chain >= max_context_len && mean <= 0.6 * chain;
+  if (plain) return most && from_start && fill <= 2.0 ? PROMPT_NARROW : plain;
+  if (alone) return fill < 0.625 ? plain : from_start && fill < 1.0 ? PROMPT_NARROW_GROUPS : PROMPT_NARROW;
+  if (most) return from_start && fill >= 1.5 ? PROMPT_NARROW : plain;
+  return fill >= 0.875 || chain <= 512 * fill ? PROMPT_NARROW : plain;
 }
 
 // The arguments of ms_paged_attention_mfma's general shape, for plain scores (no sink, cap, slopes, gate; values of the

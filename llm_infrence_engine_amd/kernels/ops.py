@@ -81,7 +81,7 @@ _SIGNATURES = {
                             _c_int, _c_int, _c_int, _c_int, _c_int, _c_float, _c_int, _c_ptr],
     "ms_attention_prompt_as": [_c_int, _c_ptr, _c_ll, _c_ptr, _c_ptr, _c_ptr, _c_int, _c_ptr, _c_ptr, _c_ptr, _c_ptr, _c_ll, _c_int, _c_int,
                                _c_int, _c_int, _c_int, _c_int, _c_int, _c_float, _c_int, _c_ptr],
-    "ms_attention_prompt_kind": [_c_int, _c_int, _c_int, _c_int, _c_int, _c_int, _c_int, _c_int, _c_int],
+    "ms_attention_prompt_kind": [_c_int, _c_int, _c_int, _c_int, _c_int, _c_int, _c_int, _c_int, _c_int, _c_int],
     "ms_attention_prompt_pays": [_c_int, _c_int, _c_int, _c_int, _c_int, _c_int, _c_int, _c_int, _c_int],
     "ms_paged_attention_mfma_decode": [_c_ptr, _c_ll, _c_ptr, _c_ptr, _c_ptr, _c_int, _c_ptr, _c_ptr, _c_ptr, _c_ptr,
                                        _c_ll, _c_ptr, _c_ptr, _c_int, _c_int, _c_int, _c_int, _c_int, _c_int, _c_float,
@@ -1010,12 +1010,13 @@ def paged_attention_mfma(q: torch.Tensor, k_pages: torch.Tensor, vt_pages: torch
                          scale: float, max_q_len: int, max_context_len: int, window: Optional[int] = None,
                          table_rows: Optional[torch.Tensor] = None, sink: Optional[torch.Tensor] = None,
                          softcap: float = 0.0, slopes: Optional[torch.Tensor] = None,
-                         gate: Optional[torch.Tensor] = None, out_scale: float = 1.0) -> torch.Tensor:
+                         gate: Optional[torch.Tensor] = None, out_scale: float = 1.0, exact: bool = True) -> torch.Tensor:
     """Matrix-core attention, bfloat16.  k_pages [P, nkv, page_size, d], vt_pages [P, nkv, value size, page_size]
     (the key size or a smaller multiple of 16);
     request r owns tokens q_start[r]..q_start[r+1]-1, holds context_lens[r] keys after this step and has row
     ``table_rows[r]`` of ``block_table`` (row r without ``table_rows``).  ``max_q_len`` and ``max_context_len``
-    are upper bounds; tokens from q_start[R] on belong to no request, a request may have no token.  A small
+    are upper bounds (``exact``: the step's own lengths, or close to them; the choice of a kernel hangs on it); tokens from
+    q_start[R] on belong to no request, a request may have no token.  A small
     batch of single tokens with long contexts also splits the keys over blocks (and combines).  ``sink`` float [nh]:
     exp(sink[h]) joins the denominator of head h's softmax.  ``softcap``, ``slopes``, ``gate`` and ``out_scale`` as in
     ``paged_attention_generic``."""
@@ -1068,7 +1069,8 @@ def paged_attention_mfma(q: torch.Tensor, k_pages: torch.Tensor, vt_pages: torch
     else:
         kind = 0
         if plain and k_pages.data_ptr() % 16 == 0 and vt_pages.data_ptr() % 16 == 0:
-            kind = _get("ms_attention_prompt_kind")(R, N, max_q_len, max_context_len, num_heads, nkv, d, page_size, int(window or 0))
+            kind = _get("ms_attention_prompt_kind")(R, N, max_q_len, max_context_len, num_heads, nkv, d, page_size, int(window or 0),
+                                                      int(exact))
         if kind:     # keys and values staged in LDS for four neighbouring tiles
             _call("ms_attention_prompt_as", kind, q.data_ptr(), q_stride, k_pages.data_ptr(), vt_pages.data_ptr(), block_table.data_ptr(),
                   block_table.shape[1], _ptr(table_rows), q_start.data_ptr(), context_lens.data_ptr(), out.data_ptr(), num_heads * dv,
@@ -1135,7 +1137,7 @@ def paged_attention(q: torch.Tensor, kv, ctx, out: torch.Tensor, num_heads: int,
             and not (by_entry and (gate.data_ptr() % 8 or (q.shape[0] > 1 and gate.stride(0) % 4)))):
         return paged_attention_mfma(q, kv.k_pages, kv.v_pages, kv.block_table, ctx.q_start, ctx.context_lens, out,
                                     num_heads, scale, ctx.max_q_len, ctx.max_context_len, window, kv.table_rows, sink,
-                                    softcap, slopes, gate, out_scale)
+                                    softcap, slopes, gate, out_scale, ctx.n_live_tokens is None)
     return paged_attention_generic(q, kv.k_pages, kv.v_pages, kv.block_table, ctx.token_req, ctx.positions, out,
                                    num_heads, scale, window, kv.v_transposed, kv.table_rows, ctx.n_live_tokens, sink,
                                    softcap, slopes, gate, out_scale)

@@ -1,0 +1,54 @@
+"""Which kernel a call goes to, where that is a rule on sizes in the library: host code alone, so these run without a GPU (the
+library then takes the chip to have 256 compute units, as it has)."""
+from types import SimpleNamespace
+
+import pytest
+import torch
+
+
+@pytest.fixture(scope="module")
+def ops():
+    from llm_infrence_engine_amd.kernels import ops
+
+    return ops
+
+
+@pytest.mark.parametrize("R,N,most,longest,nh,nkv,d,window,exact,kind", [
+    # us of the other kernel, wide, narrow, narrow with twice the groups
+    (8, 4096, 512, 512, 14, 2, 64, 0, 1, 1),            # 25.8 19.1 22.2 27.0
+    (48, 1680, 35, 35, 16, 8, 64, 0, 1, 1),             # 14.8 9.8 11.6 17.9
+    (6, 1644, 274, 274, 32, 4, 64, 0, 1, 1),            # 21.9 15.3 16.9 22.5
+    (4, 1436, 1013, 4955, 28, 4, 128, 0, 1, 0),         # 69 160 106 74: the longest context belongs to 13 tokens
+    (9, 953, 945, 3535, 40, 8, 128, 0, 1, 0),           # 57 112 76 56: to a single token
+    (24, 456, 19, 845, 28, 4, 128, 0, 1, 0),            # 27 33 29 35
+    (8, 2048, 256, 256, 28, 4, 128, 0, 1, 1),           # 36 20.7 22.9 33
+    (64, 1536, 1536, 8192, 32, 4, 64, 0, 0, 2),         # a capture's bounds; 32 portions of 42 tokens: 16.2 11.3 12.4 18.9
+    (64, 256, 256, 8192, 14, 2, 64, 0, 0, 2),
+    (64, 512, 512, 4096, 28, 4, 128, 0, 0, 0),          # 24 portions of 20 tokens: 9.7 9.3 8.1 12.5
+    (16, 768, 768, 4096, 16, 2, 128, 0, 0, 0),          # 607 tokens beside single ones of 4,000 keys: 51 123 83 59
+    # as before
+    (1, 2048, 2048, 2048, 14, 2, 64, 0, 1, 2), (3, 396, 171, 171, 14, 2, 64, 0, 1, 2), (1, 3910, 3910, 12105, 14, 2, 64, 0, 1, 3),
+    (1, 2345, 2345, 10186, 14, 2, 64, 256, 1, 2), (1, 910, 910, 910, 28, 4, 128, 0, 1, 3), (1, 2059, 2059, 2059, 28, 4, 128, 0, 1, 2),
+    (1, 3077, 3077, 3077, 28, 4, 128, 0, 1, 1), (30, 60, 2, 2, 14, 2, 64, 0, 1, 0),
+    (1, 800, 800, 4000, 28, 4, 128, 0, 1, 2), (1, 100, 400, 400, 14, 2, 64, 0, 1, 2), (3, 100, 90, 100, 7, 2, 64, 0, 1, 0)])
+def test_kind_of_prompt_attention(ops, R, N, most, longest, nh, nkv, d, window, exact, kind):
+    """Measured on both sides of its lines: even portions that fill the chip once as they are, contexts that say nothing of the
+    longest portion, and what a captured step knows of those that will run in it."""
+    assert ops._get("ms_attention_prompt_kind")(R, N, most, longest, nh, nkv, d, 16, window, exact) == kind
+
+
+@pytest.mark.parametrize("captured", [False, True])
+def test_a_captured_step_says_that_its_lengths_are_bounds(ops, monkeypatch, captured):
+    seen = {}
+
+    def attention(*args):
+        seen["exact"] = args[17]
+
+    monkeypatch.setattr(ops, "paged_attention_mfma", attention)
+    pages = torch.zeros(2, 2, 16, 64, dtype=torch.bfloat16)
+    kv = SimpleNamespace(k_pages=pages, v_pages=pages.transpose(2, 3).contiguous(), v_transposed=True, block_table=None, table_rows=None)
+    ctx = SimpleNamespace(q_start=None, context_lens=None, max_q_len=4, max_context_len=16,
+                          n_live_tokens=torch.zeros(1, dtype=torch.int32) if captured else None)
+    q = torch.zeros(4, 4 * 64, dtype=torch.bfloat16)
+    ops.paged_attention(q, kv, ctx, torch.empty_like(q), 4, 0.125)
+    assert seen["exact"] is not captured
