@@ -107,6 +107,7 @@ int ms_gemm_tiled_sums_parts(int M, int N, int K);   // partial sums over runs o
 int ms_gemm_tiled_sums(const void* A, long long lda, const void* W, long long ldw, float* partial, int M, int N, int K, int parts,
                        hipStream_t stream);
 int ms_gemm_tiled_pays(int M, int N, int K);
+int ms_gemm_tiled_relu2_pays(int M, int N, int K);   // the same question for epilogue 5
 int ms_gemm_tiled_plain_pays(int M, int N, int K);   // the same question for a plain product (epilogue 0)
 
 // The q/k/v product of many tokens with bias, rotation (whole heads, pairs (j, j + d/2)) and the store of k and v

@@ -534,13 +534,25 @@ SumsChoice choose_sums(int M, int N, int K) {
 extern "C" void ms_gemm_tiled_force(int tile) { g_tile = tile; }
 extern "C" void ms_gemm_tiled_force_xcd_split(int xm) { g_xcd_split = xm; }
 
+// What of the tiles' places the product fills: tiles in whole rounds over the CUs, counted for the XCD with the most of them.
+static double filled(int M, int N, const TileChoice& c) {
+  const int features = c.tile == 1 ? 256 : (c.tile == 4 ? 192 : (c.tile == 5 ? 160 : 128)), tokens = c.tile == 2 ? 128 : 256;
+  const int to_a_cu = c.tile == 2 ? 2 : 1, xm = choose_xcd_split(M), xn = 8 / xm, cus = ms_compute_units();
+  const long long n_tiles = (N + features - 1) / features, m_tiles = (M + tokens - 1) / tokens;
+  const long long most = ((n_tiles + xn - 1) / xn) * ((m_tiles + xm - 1) / xm), places = (long long)(cus + 7) / 8 * to_a_cu;
+  return (double)M * N / ((double)((most + places - 1) / places) * places * 8 * features * tokens);
+}
+
 // Whether the gated product of M tokens is faster here than as the library's product and an activation kernel.  Time of these over
-// this kernel's, a different W every call:
+// this kernel's, a different W every call, with silu (the gelu and the clamped gate, whose kernels cost more: 1.08 times that):
 //   up to 1,536 columns 1.02 to 2 (65 to 8,192 tokens);
-//   2,048 to 3,584 columns, 5,632 to 37,888 rows, 130 to 8,192 tokens: 0.99 to 1.38, 1.15 on average (7B gate/up: 256 tokens 91 and
-//   79 us, 1,024 tokens 313 and 245, 2,176 tokens 566 and 532, 4,096 tokens 876 and 834; 22,016 x 2,048, 4,096 tokens 365 and 304);
-//   4,096 and 5,120 columns, 12,288 to 55,296 rows: beyond 512 tokens 0.95 to 1.28 (27,648 x 5,120, 1,024 tokens 276 and 226,
-//   3,584 tokens 766 and 804), up to 512 tokens 0.91 to 1.21;
+//   beyond, up to 2,048 tokens whose tiles fill 9/10 of their rounds: 0.99 to 1.3;
+//   687 other sizes of 1,600 to 5,120 columns (5,248 to 55,296 rows, 65 to 4,096 tokens), by what the tiles fill:
+//     up to 3,584 columns tiles of 192 or 160 features, those of 256 from 0.65 on, those of 128 from 0.7 on or up to 0.4 (one round
+//     that leaves CUs idle, as the library's does): 0.92 to 1.60, 1.15 on average, 8 of 385 below 0.97 (7B gate/up: 1,024 tokens 313 and
+//     245 us, 2,176 tokens 566 and 532); the others 0.71 to 1.38, 1.03 on average (14,336 x 3,584, 300 tokens 55 and 62);
+//     4,096 to 5,120 columns beyond 512 tokens from 0.8 on: 0.91 to 1.58, 1.12 on average, 4 of 108 below 0.97; the others 0.80 to
+//     1.30, 1.01 on average;
 //   8,192 columns 0.96 to 1.03.
 // Tiles of 64 x 64 only up to 1,536 columns.
 extern "C" int ms_gemm_tiled_pays(int M, int N, int K) {
@@ -548,8 +560,19 @@ extern "C" int ms_gemm_tiled_pays(int M, int N, int K) {
   if (K <= 1536) return 1;
   const TileChoice c = choose_tile(M, N, K);
   if (c.tile == 3) return 0;
-  if (K <= 3584 || (K <= 5120 && M > 512)) return 1;
-  return M <= 2048 && c.tiles * 10 >= c.slots * 9;
+  if (M <= 2048 && c.tiles * 10 >= c.slots * 9) return 1;
+  const double f = filled(M, N, c);
+  if (K <= 3584) return c.tile >= 4 || (c.tile == 1 ? f >= 0.65 : f >= 0.7 || f <= 0.4);
+  return K <= 5120 && M > 512 && f >= 0.8;
+}
+
+// The same question for the squared relu, whose product is written whole and whose own kernel costs little: the sizes that the
+// gated product takes beyond 2,048 tokens or with rounds not full are 0.69 to 1.4 here, a tenth of them below 0.93.
+extern "C" int ms_gemm_tiled_relu2_pays(int M, int N, int K) {
+  if (M <= 0 || N <= 0 || K <= 0 || K % BK) return 0;
+  if (K <= 1536) return 1;
+  const TileChoice c = choose_tile(M, N, K);
+  return c.tile != 3 && M <= 2048 && c.tiles * 10 >= c.slots * 9;
 }
 
 // A bfloat16 [M, lda], W bfloat16 [N, ldw] (rows of K, K a multiple of 64), out bfloat16.

@@ -147,7 +147,7 @@ def linear_act(a: torch.Tensor, w: torch.Tensor, epilogue: int, numbers: Optiona
             if epilogue == ops.EPI_RELU2 and ops.splits_columns(a, w):
                 return None
             return ops.gemm_skinny(a, w, numbers, epilogue)
-        if a.shape[0] > ops.SKINNY_MAX_ROWS and ops.gemm_tiled_pays(a, w):
+        if a.shape[0] > ops.SKINNY_MAX_ROWS and ops.gemm_tiled_pays(a, w, epilogue):
             return ops.gemm_tiled(a, w, epilogue, limit, alpha)
     except ops.UnsupportedShape:
         _fell_back(a.shape[0], w.shape[0], w.shape[1], "product + activation")

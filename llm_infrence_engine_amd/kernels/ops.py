@@ -57,6 +57,7 @@ _SIGNATURES = {
     "ms_gemm_tiled_force": [_c_int],
     "ms_gemm_tiled_force_xcd_split": [_c_int],
     "ms_gemm_tiled_pays": [_c_int, _c_int, _c_int],
+    "ms_gemm_tiled_relu2_pays": [_c_int, _c_int, _c_int],
     "ms_gemm_tiled_plain_pays": [_c_int, _c_int, _c_int],
     "ms_gemm_tiled_qkv": [_c_ptr, _c_ll, _c_ptr, _c_ll, _c_ptr, _c_ptr, _c_ptr, _c_ptr, _c_ptr, _c_ptr, _c_int,
                           _c_int, _c_int, _c_int, _c_int, _c_int, _c_int, _c_ptr],
@@ -678,11 +679,13 @@ def gemm_slab_qkv(a: torch.Tensor, w_qkv: torch.Tensor, bias: Optional[torch.Ten
     return q
 
 
-def gemm_tiled_pays(a: torch.Tensor, w: torch.Tensor) -> bool:
-    """Whether ``gemm_tiled(a, w, EPI_SWIGLU)`` takes these sizes and is the faster way to the gated product."""
+def gemm_tiled_pays(a: torch.Tensor, w: torch.Tensor, epilogue: int = EPI_SWIGLU) -> bool:
+    """Whether ``gemm_tiled(a, w, epilogue)`` takes these sizes and is the faster way to the gated product (one of the three
+    gates) or to the squared relu's."""
+    pays = _get("ms_gemm_tiled_relu2_pays" if epilogue == EPI_RELU2 else "ms_gemm_tiled_pays")
     return (a.dtype == torch.bfloat16 and w.dtype == torch.bfloat16 and a.dim() == 2 and a.is_contiguous()
             and w.is_contiguous() and a.data_ptr() % 16 == 0 and w.data_ptr() % 16 == 0
-            and bool(_get("ms_gemm_tiled_pays")(a.shape[0], w.shape[0], a.shape[1])))
+            and bool(pays(a.shape[0], w.shape[0], a.shape[1])))
 
 
 def gemm_tiled_plain_pays(a: torch.Tensor, w: torch.Tensor) -> bool:

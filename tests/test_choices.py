@@ -52,3 +52,23 @@ def test_a_captured_step_says_that_its_lengths_are_bounds(ops, monkeypatch, capt
     q = torch.zeros(4, 4 * 64, dtype=torch.bfloat16)
     ops.paged_attention(q, kv, ctx, torch.empty_like(q), 4, 0.125)
     assert seen["exact"] is not captured
+
+
+@pytest.mark.parametrize("M,N,K,gated,relu2", [
+    # times of the library and the activation's kernel over the tiled kernel's: silu, squared relu
+    (300, 14336, 3584, 0, 0),         # 0.88 0.88: tiles of 128 fill half a round
+    (305, 16384, 3072, 0, 0),         # 0.88
+    (2305, 11008, 4096, 0, 0),        # 0.93 0.88
+    (3072, 5248, 3008, 0, 0),         # 0.71 0.69: 21 tiles of features over 8 XCDs
+    (2305, 19200, 4928, 0, 0),        # 0.80 0.80
+    (1024, 37888, 3584, 1, 0), (2176, 37888, 3584, 1, 0), (4096, 22016, 2048, 1, 0), (3000, 27648, 5120, 1, 0),
+    (2048, 8192, 3072, 1, 1), (70, 37888, 3584, 1, 0), (193, 18944, 3072, 0, 0),
+    # both as ever: full rounds, short rows; rows that are no multiple of 64, long ones
+    (2048, 37888, 3584, 1, 1), (1300, 55296, 5120, 1, 1), (8192, 9728, 896, 1, 1), (65, 7296, 1536, 1, 1), (512, 8192, 2056, 0, 0),
+    (4096, 28672, 8192, 0, 0), (256, 15360, 4096, 0, 0)])
+def test_where_the_tiled_kernel_takes_products_with_an_activation(ops, M, N, K, gated, relu2):
+    assert ops._get("ms_gemm_tiled_pays")(M, N, K) == gated
+    assert ops._get("ms_gemm_tiled_relu2_pays")(M, N, K) == relu2
+    if M * max(N, K) < 1 << 24:
+        a, w = torch.empty(M, K, dtype=torch.bfloat16), torch.empty(N, K, dtype=torch.bfloat16)
+        assert ops.gemm_tiled_pays(a, w, ops.EPI_RELU2) == bool(relu2) and ops.gemm_tiled_pays(a, w, ops.EPI_GEGLU) == bool(gated)
