@@ -610,19 +610,28 @@ extern "C" int ms_gemm_tiled(const void* A, long long lda, const void* W, long l
 // Column parts for a product whose reader adds partial sums up itself (the norm that follows a down projection), 0 where the
 // library's product, or this kernel's whole one, is the faster way.  Few features leave a product of whole columns fewer
 // tiles than CUs: 2,048 tokens by 3,584 x 18,944 are 112 tiles of 256 for 256 CUs; in two parts 235 us + 30 for the norm that adds
-// them up, the library 363 + 17.  Time of the library and its norm over this, 65 to 4,096 tokens, 14 sizes of W (896 x 896 to
-// 5,120 x 27,648):
-//   up to 128 tokens 1.06 to 2.7;
-//   up to 512 tokens by rows of 4,096 columns and more 0.97 to 2.6 (896 x 4,864 at 390 tokens 21.4 and 18.8 us), by rows of up to
-//   1,024 1.1 to 1.25, between these 0.89 to 1.6;
-//   up to 1,024 tokens by 8,192 columns and more 0.98 to 1.55, by fewer 0.84 to 1.15;
-//   beyond, by 16,384 columns and more where one round of blocks in parts fills 5/6 of the CUs, 1.4 to 1.57 (4,096 x 28,672 at
-//   2,048 tokens, all CUs, 0.96); elsewhere the library mostly wins (0.65 to 1.54).
+// them up, the library 363 + 17.  Time of the other way and its norm over this, 3,700 sizes (512 to 8,192 features, 768 to
+// 28,672 columns, 65 to 4,096 tokens), and outside the lines:
+//   up to 128 tokens 0.93 to 3.8, 1.5 on average;
+//   up to 256 tokens by 4,096 columns and more 0.94 to 4.1, 1.6 on average, by up to 1,024 and up to 5,120 features 0.98 to 1.26 (more
+//     features 0.89 to 1.10);
+//   up to 512 tokens by more than 8,192 columns 0.98 to 2.8; by more than 4,096 in several parts, up to 5,120 features, 0.92 to 1.6,
+//     1.1 on average, 12 of 586 below 0.97 (896 x 4,864 at 390 tokens 1.11).  Not: tiles of 128 that take every CU once (2,048 x 5,632
+//     at 390 tokens 0.93), whole columns (0.81 to 1.02), more features (0.89 to 1.1), 1,024 columns and fewer (896 x 896 0.91 to 0.96);
+//   up to 1,024 tokens by more than 8,192 columns, up to 5,120 features, 0.93 to 2.3, 1.29 on average; with more features 0.83 to 1.8,
+//     by 8,192 columns 0.85 to 1.17;
+//   beyond, by 16,384 columns and more where one round of blocks in parts fills 5/6 of the CUs, but not all: 0.96 to 2.0, 1.4 on
+//     average (3,584 x 18,944 at 1,281 to 1,536 tokens and at 1,793 to 2,304).  With every CU taken 0.96 to 1.02 (4,096 x 28,672 at 2,048
+//     tokens); elsewhere 0.74 to 1.47 (3,584 x 18,944 1.08 at 1,600 tokens, 1.4 at 1,200 and 2,560, 0.80 at 2,816): what the library
+//     takes there changes by a factor of two from one number of tokens to the next.
 extern "C" int ms_gemm_tiled_sums_parts(int M, int N, int K) {
   if (M <= 64 || N <= 0 || K < 768 || K % BK || N > 8192) return 0;
   const SumsChoice c = choose_sums(M, N, K);
-  if (M <= 128 || (M <= 512 && (K >= 4096 || K <= 1024)) || (M <= 1024 && K >= 8192)) return c.parts;
   const int cus = ms_compute_units();
+  if (M <= 128) return c.parts;
+  if (M <= 256) return K >= 4096 || (K <= 1024 && N <= 5120) ? c.parts : 0;
+  if (M <= 512) return K > 8192 || (K > 4096 && N <= 5120 && c.parts > 1 && !(c.tile == 2 && c.blocks == cus)) ? c.parts : 0;
+  if (M <= 1024) return K > 8192 && N <= 5120 ? c.parts : 0;
   return K >= 16384 && c.tile == 1 && c.parts > 1 && c.blocks < cus && c.blocks * 6 >= cus * 5 ? c.parts : 0;
 }
 

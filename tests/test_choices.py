@@ -72,3 +72,18 @@ def test_where_the_tiled_kernel_takes_products_with_an_activation(ops, M, N, K, 
     if M * max(N, K) < 1 << 24:
         a, w = torch.empty(M, K, dtype=torch.bfloat16), torch.empty(N, K, dtype=torch.bfloat16)
         assert ops.gemm_tiled_pays(a, w, ops.EPI_RELU2) == bool(relu2) and ops.gemm_tiled_pays(a, w, ops.EPI_GEGLU) == bool(gated)
+
+
+@pytest.mark.parametrize("M,N,K,taken", [
+    # times of the other way over partial sums
+    (390, 896, 896, 0), (512, 768, 768, 0),                       # 0.96 0.91
+    (240, 8064, 896, 0),                                          # 0.90
+    (390, 2048, 5632, 0), (384, 4096, 4096, 0),                   # 0.93 0.91
+    (429, 4480, 6784, 0), (512, 7808, 7808, 0), (437, 6400, 8192, 0),   # 0.82 0.92 0.90
+    (900, 3072, 8192, 0), (791, 6080, 8448, 0), (640, 8192, 28672, 0),  # 0.85 0.85 0.86
+    (128, 8192, 2048, 1), (256, 896, 896, 1), (256, 4096, 4096, 1), (390, 896, 4864, 1), (512, 896, 4864, 1), (512, 3584, 18944, 1),
+    (384, 2048, 8192, 1), (1024, 3584, 18944, 1), (900, 5120, 13824, 1), (2048, 3584, 18944, 1), (1300, 5120, 27648, 1),
+    # as ever
+    (64, 896, 4864, 0), (200, 1536, 2048, 0), (1024, 896, 4864, 0), (1600, 3584, 18944, 0), (2048, 4096, 28672, 0), (100, 8256, 4096, 0)])
+def test_where_products_of_many_rows_leave_partial_sums(ops, M, N, K, taken):
+    assert (ops._get("ms_gemm_tiled_sums_parts")(M, N, K) > 0) == bool(taken)
