@@ -33,6 +33,7 @@ FIRST_VALUES = ("gqa_attention", "first_values")     # the key of ``StepContext.
 
 class GQAttention(Mixer):
     accepts_lazy_norm = True
+    sums_on_request = True
 
     def __init__(self, prefix: str, position, hidden_size: int, num_heads: int, num_kv_heads: int, head_dim: int,
                  scale: float, qkv_bias: bool = True, out_bias: bool = False, window: Optional[int] = None,

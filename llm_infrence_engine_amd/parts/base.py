@@ -174,6 +174,19 @@ class StepContext:
 
 
 # ------------------------------------------------------------------------------------------------ part interfaces
+def declares(part, flag: str, *methods: str) -> bool:
+    """Whether ``part`` sets ``flag``, which promises something of its ``methods``: the nearest of its classes that has either
+    decides, so that a class with a method of its own does not inherit what another's was promised to do."""
+    if flag in vars(part):
+        return bool(vars(part)[flag])
+    for c in type(part).__mro__:
+        if flag in vars(c):
+            return bool(vars(c)[flag])
+        if any(m in vars(c) for m in methods):
+            return False
+    return False
+
+
 Getter = Callable[[TensorSpec], torch.Tensor]
 
 
@@ -210,7 +223,8 @@ class Norm(Part):
     # ``bias`` (None: none), with ``eps``, and a kernel that has the row at hand may take it itself.  None: only ``forward``.
     statistic: Optional[str] = None
     settles_writes = False      # as ``Block.settles_writes``, of ``forward``'s delta
-    takes_sums = False          # True: the delta of ``forward`` and ``lazy`` may be float partial sums [parts, N, H]
+    # True: the delta of the class's ``forward`` and ``lazy`` may be float partial sums [parts, N, H]
+    takes_sums = False
 
     def lazy(self, x: torch.Tensor, delta: Optional[torch.Tensor] = None, rows: Optional[torch.Tensor] = None,
              write_back: bool = True):
@@ -243,7 +257,8 @@ class PositionEncoding(Part):
 
 class Mixer(Part):
     accepts_lazy_norm = False   # True: h may be a LazyNorm that the part hands to kernels.linear
-    hands_on_sums = False       # set by a block whose next norm takes them: ``forward_residual`` may return partial sums
+    sums_on_request = False     # True: the class's ``forward_residual`` may return partial sums where ``hands_on_sums``
+    hands_on_sums = False       # set by a block whose next norm takes them
 
     @property
     def graph_safe(self):
@@ -284,7 +299,7 @@ class SequenceFilter(Part):
 
 class FeedForward(Part):
     accepts_lazy_norm = False
-    hands_on_sums = False       # as ``Mixer.hands_on_sums``
+    sums_on_request = hands_on_sums = False     # as a ``Mixer``'s
 
     def forward(self, h: torch.Tensor, ctx: StepContext) -> torch.Tensor:
         raise NotImplementedError

@@ -10,7 +10,7 @@ from dataclasses import dataclass
 from typing import Any
 
 from ..kernels import ops
-from .base import Block, Norm, register_part
+from .base import Block, Norm, declares, register_part
 
 
 class PreNormResidual(Block):
@@ -20,9 +20,12 @@ class PreNormResidual(Block):
 
     def __init__(self, **built):
         super().__init__(**built)
-        self.takes_sums = self.mixer_norm.takes_sums
-        self.mixer.hands_on_sums = self.feed_forward_norm.takes_sums
-        self.feed_forward.hands_on_sums = True
+        if type(self).forward is not PreNormResidual.forward:
+            return
+        norms = [declares(n, "takes_sums", "forward", "lazy") for n in (self.mixer_norm, self.feed_forward_norm)]
+        self.takes_sums = norms[0]
+        self.mixer.hands_on_sums = norms[1] and declares(self.mixer, "sums_on_request", "forward_residual")
+        self.feed_forward.hands_on_sums = declares(self.feed_forward, "sums_on_request", "forward_residual")
 
     def forward(self, x, pending, ctx, kv, state):
         norm = self.mixer_norm.lazy if self.mixer.accepts_lazy_norm else self.mixer_norm.forward

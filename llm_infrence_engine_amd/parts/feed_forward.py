@@ -12,6 +12,7 @@ from .base import FeedForward, register_part
 
 class SwiGLU(FeedForward):
     accepts_lazy_norm = True
+    sums_on_request = True
 
     def __init__(self, prefix: str, hidden_size: int, intermediate_size: int):
         self.prefix, self.hidden_size, self.intermediate_size = prefix, hidden_size, intermediate_size

@@ -15,7 +15,7 @@ from ..weights.reader import CheckpointReader, place
 from ..weights.spec import TensorSpec
 from . import (attention, blocks, delta, ends, experts, feed_forward, filters, latent, linear_attention, mingru,  # noqa: F401
                norms, pooled_attention, positions, scan, side, side_by_side, streams)      # (register the built-in parts)
-from .base import KVView, Runtime, StateView, StepContext, build_part, part_class, weakest
+from .base import KVView, Runtime, StateView, StepContext, build_part, declares, part_class, weakest
 
 
 @dataclass
@@ -122,7 +122,7 @@ class Model:
                 return pending
             pending.add_into(x)
             return None
-        if pending is not None and pending.dim() > x.dim() and not (reader is not None and reader.takes_sums):
+        if pending is not None and pending.dim() > x.dim() and not (reader is not None and declares(reader, "takes_sums", "forward", "lazy")):
             from ..kernels import ops
 
             for part in pending:

@@ -87,3 +87,61 @@ def test_where_the_tiled_kernel_takes_products_with_an_activation(ops, M, N, K, 
     (64, 896, 4864, 0), (200, 1536, 2048, 0), (1024, 896, 4864, 0), (1600, 3584, 18944, 0), (2048, 4096, 28672, 0), (100, 8256, 4096, 0)])
 def test_where_products_of_many_rows_leave_partial_sums(ops, M, N, K, taken):
     assert (ops._get("ms_gemm_tiled_sums_parts")(M, N, K) > 0) == bool(taken)
+
+
+# ---------------------------------------------------------------- who may leave sums undone, and who may be given them
+def _block(ops, norm=None, mixer=None, feed_forward=None, block=None):
+    from llm_infrence_engine_amd.parts.attention import GQAttention
+    from llm_infrence_engine_amd.parts.blocks import PreNormResidual
+    from llm_infrence_engine_amd.parts.feed_forward import SwiGLU
+    from llm_infrence_engine_amd.parts.norms import RMSNorm
+
+    def of(base, body):
+        return type("Own", body if isinstance(body, tuple) else (base,), {} if body is None or isinstance(body, tuple) else body)
+
+    norms = [of(RMSNorm, norm)("", 64, 1e-5) for _ in range(2)]
+    m = of(GQAttention, mixer)("", None, 64, 2, 2, 32, 0.1)
+    f = of(SwiGLU, feed_forward)("", 64, 128)
+    return of(PreNormResidual, block)(position=None, mixer_norm=norms[0], mixer=m, feed_forward_norm=norms[1], feed_forward=f)
+
+
+def test_parts_of_a_programs_own_see_one_addend(ops):
+    """Partial sums pass between the parts that were written for them: a class derived from one of these, with a method of its
+    own (here or in a class beside it), is handed one addend and leaves one, unless it says that it knows better."""
+    from llm_infrence_engine_amd.parts.norms import RMSNorm
+
+    def flags(b):
+        return b.takes_sums, b.mixer.hands_on_sums, b.feed_forward.hands_on_sums
+
+    own = lambda self, *a, **k: None     # noqa: E731
+    beside = type("Beside", (), {"forward": own})
+    assert flags(_block(ops)) == (True, True, True)
+    assert flags(_block(ops, norm={"forward": own})) == flags(_block(ops, norm={"lazy": own})) == (False, False, True)
+    assert flags(_block(ops, norm=(beside, RMSNorm))) == (False, False, True)
+    assert flags(_block(ops, norm={"forward": own, "takes_sums": True})) == (True, True, True)
+    assert flags(_block(ops, norm={"other": own})) == (True, True, True)
+    assert flags(_block(ops, mixer={"forward_residual": own})) == (True, False, True)
+    assert flags(_block(ops, feed_forward={"forward_residual": own})) == (True, True, False)
+    assert flags(_block(ops, block={"forward": own})) == (False, False, False)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("reader", ["norm", "own norm", "layer norm", "block", "own block", None])
+def test_the_model_adds_up_sums_for_a_reader_that_takes_one_addend(ops, reader):
+    """Three partial sums of 5 rows by 64, before each kind of reader and before nobody's (an entry into another pass)."""
+    from llm_infrence_engine_amd.parts.model import Model
+    from llm_infrence_engine_amd.parts.norms import LayerNorm, RMSNorm
+
+    own = {"forward": lambda self, *a, **k: None}
+    r = {"norm": lambda: RMSNorm("", 64, 1e-5), "own norm": lambda: type("Own", (RMSNorm,), own)("", 64, 1e-5),
+         "layer norm": lambda: LayerNorm("", 64, 1e-5), "block": lambda: _block(ops), "own block": lambda: _block(ops, norm=own),
+         None: lambda: None}[reader]()
+    g = torch.Generator().manual_seed(7)
+    x0, sums = torch.randn(5, 64, generator=g), torch.randn(3, 5, 64, generator=g)
+    x, pending = x0.cuda(), sums.cuda()
+    left = Model._settled(x, pending, r)
+    if reader in ("norm", "block"):
+        assert left is pending and torch.equal(x.cpu(), x0)
+    else:
+        assert left is None
+        torch.testing.assert_close(x.cpu().double(), x0.double() + sums.double().sum(0), atol=2e-6, rtol=2e-6)
