@@ -626,13 +626,14 @@ extern "C" int ms_gemm_tiled(const void* A, long long lda, const void* W, long l
 //     takes there changes by a factor of two from one number of tokens to the next.
 extern "C" int ms_gemm_tiled_sums_parts(int M, int N, int K) {
   if (M <= 64 || N <= 0 || K < 768 || K % BK || N > 8192) return 0;
+  if (M > 128 && (M <= 256 ? K < 4096 && (K > 1024 || N > 5120)
+                  : M <= 512 ? K <= 8192 && (K <= 4096 || N > 5120)
+                  : M <= 1024 ? K <= 8192 || N > 5120 : K < 16384)) return 0;   // (asked for twice a layer: before the choice)
   const SumsChoice c = choose_sums(M, N, K);
   const int cus = ms_compute_units();
-  if (M <= 128) return c.parts;
-  if (M <= 256) return K >= 4096 || (K <= 1024 && N <= 5120) ? c.parts : 0;
-  if (M <= 512) return K > 8192 || (K > 4096 && N <= 5120 && c.parts > 1 && !(c.tile == 2 && c.blocks == cus)) ? c.parts : 0;
-  if (M <= 1024) return K > 8192 && N <= 5120 ? c.parts : 0;
-  return K >= 16384 && c.tile == 1 && c.parts > 1 && c.blocks < cus && c.blocks * 6 >= cus * 5 ? c.parts : 0;
+  if (M > 256 && M <= 512 && K <= 8192 && (c.parts == 1 || (c.tile == 2 && c.blocks == cus))) return 0;
+  if (M > 1024 && (c.tile != 1 || c.parts == 1 || c.blocks >= cus || c.blocks * 6 < cus * 5)) return 0;
+  return c.parts;
 }
 
 // Partial sums of the plain product over `parts` runs of the columns: float [parts, M, N].

@@ -601,11 +601,11 @@ def gemm_sums(a: torch.Tensor, w: torch.Tensor) -> Optional[torch.Tensor]:
     (``rms_norm``'s ``delta``), where that is the faster way to the product; None: it is not."""
     (M, K), N = a.shape, w.shape[0]
     if M > SKINNY_MAX_ROWS:
-        if not (a.dtype == w.dtype == torch.bfloat16 and a.is_contiguous() and w.is_contiguous() and a.data_ptr() % 16 == 0
-                and w.data_ptr() % 16 == 0):
-            return None
         parts = _get("ms_gemm_tiled_sums_parts")(M, N, K)
-        return gemm_tiled_sums(a, w, parts) if parts else None
+        if not (parts and a.dtype == w.dtype == torch.bfloat16 and a.is_contiguous() and w.is_contiguous()
+                and a.data_ptr() % 16 == 0 and w.data_ptr() % 16 == 0):
+            return None
+        return gemm_tiled_sums(a, w, parts)
     if not skinny_ok(a, w):
         return None
     parts = _slab_parts(a, w, True)
