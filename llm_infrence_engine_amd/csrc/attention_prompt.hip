@@ -479,6 +479,7 @@ extern "C" int ms_attention_prompt_as(int kind, const void* q, long long q_strid
 #undef GO
 }
 
+// The wide kind by name (tests, measurements).
 extern "C" int ms_attention_prompt(const void* q, long long q_stride, const void* k_pages, const void* vt_pages,
                                    const int* block_table, int table_stride, const int* table_rows, const int* q_start,
                                    const int* context_lens, void* out, long long out_stride, int n_requests, int n_tokens,

@@ -504,7 +504,9 @@ int plan(const void* A, size_t lda, const bf16* W, size_t ldw, const float* bias
 
 // Columns split over blocks as well, for a W with long rows and too few tiles to give every CU a share of
 // whole rows that is worth its loads of the activations (down projections): the number of column parts, 0 if
-// the shape is not one for it.  Every block then takes at most 16 tiles (one round of its waves).
+// the shape is not one for it.  Every block then takes at most 16 tiles (one round of its waves).  Slabs and rings are asked for
+// first (gemm_skinny in kernels/ops.py): what comes here are 17 to 64 rows by a W of fewer than 4 million values and 8,192 columns or
+// more, and the shapes below where the rows lie farther apart than slabs reach over.
 int splitk_parts(int M, int N, int K) {
   const int cus = ms_compute_units();
   const int tiles = (N + 15) / 16;

@@ -18,7 +18,8 @@
 //
 // us before | with it (before: gemm_panel, whose operands go to registers 16 rows by 64 bytes a load; at one and at 8 tokens): 55,296 x 5,120
 // 104 | 87, 107 | 93; 37,888 x 3,584 55 | 45, 57 | 49; 152,064 x 3,584 186 | 163, 192 | 179; 151,936 x 896 54 | 45, 64 | 50;
-// 5,120 x 27,648 (two kernels before) 59 | 45, 61 | 50; 3,584 x 18,944 31 | 25, 32 | 26.  6.0 to 6.8 TB/s for the largest.
+// 5,120 x 27,648 (two kernels before) 59 | 45, 61 | 50; 3,584 x 18,944 31 | 25, 32 | 26.  6.0 to 6.7 TB/s
+// for the largest at one token, 5.4 to 6.1 at 8.
 #include "common.h"
 #include "api.h"
 
@@ -353,8 +354,9 @@ int plan(const void* A, size_t lda, const bf16* W, size_t ldw, const float* bias
 }  // namespace
 
 // Whether this kernel is the faster one for a product of M rows with W[N, K] (that it can compute): from 24 million values of
-// W on.  The line goes by W alone, so that a row's bits do not hang on how many rows there are (but for folded norms of so many
-// long rows that they do not fit LDS: M K beyond about 47,000).  Time of the others over this one's, K from 512 to
+// W on.  The line goes by W alone, so that in the calls that come here first (folded norms, and up to 8 rows without: from 9 on slabs
+// are asked for before, see ms_gemm_slab_parts) a row's bits do not hang on how many rows there are, but for folded norms of so many
+// long rows that they do not fit LDS (M K beyond about 47,000).  Time of the others over this one's, K from 512 to
 // 18,944, N from 1,024 to 151,936, 1 to 16 rows, without and with the norm: 0.95 to 1.52 from 24 million on, 1.2 on average (2,048
 // x 12,288 with norm, 16 rows 0.91); between 10 and 24 million 0.99 to 1.31 at one row, but with the norm 0.79 to 1.0 at 8 and 16
 // rows, whose turn to bfloat16 every block pays for; below, its start (rings, the order of the tiles) is what counts: 896 x

@@ -15,7 +15,8 @@
 // read W as operands, 16 rows by 64 bytes a load; for narrow W with the columns split and a kernel that adds up): 37,888 x 3,584
 // 71 | 52, 59 | 48; 4,608 x 3,584 19.6 | 15.5, 17.4 | 11.7; 3,584 x 3,584 18.6 | 12.7, 14.8 | 10.0, and 11.4, 9.2 as four partial
 // sums; 3,584 x 18,944 50 | 33.4, 44 | 27.4 as four; 152,064 x 3,584 268 | 225, 212 | 193; 55,296 x 5,120 124 | 112, 119 | 95;
-// 9,728 x 896 11.6 | 8.9, 9.3 | 7.2; 896 x 4,864 11.6 | 6.4, 11.2 | 5.0 as four.  5.0 (64 tokens) to 6.0 TB/s of W for the largest.
+// 9,728 x 896 11.6 | 8.9, 9.3 | 7.2; 896 x 4,864 11.6 | 6.4, 11.2 | 5.0 as four.  4.8 to 5.2 TB/s of W (64 tokens) and 5.6 to 6.0
+// (24) for the largest three.
 // The other split, all waves on one slice with a barrier a slice, took 50 us for 37,888 x 3,584, but 29 for 3,584 x 3,584 and
 // 126 for 3,584 x 18,944 (0.45 us a step of 64 columns, whatever the slab): its fragments are read by several waves.  Asking for
 // neighbouring slices by neighbouring waves, or starting blocks at different columns, changed nothing.
@@ -322,9 +323,10 @@ int plan(const bf16* A, size_t lda, const bf16* W, size_t ldw, const float* bias
 // products, the norms folded in and W ringed or streamed | here: 896 wide 22.3 | 25.7 us at 8 rows, 26.3 | 25.6 at 9, 29.1 | 26.0 at 16;
 // 2,048 wide 51.2 | 47.4 at 4, 59.2 | 48.8 at 16; 3,584 wide 97 | 95 at 8, 115 | 95 at 16; 5,120 wide 188 | 179 and 229 | 181); other
 // products from 17 on, and from 9 on by a W of 8 million values (9,728 x 896 7.0 us at 16 rows, 7.6 with the norm folded in).
-// The lines go by W alone beside the number of rows, so that a row's bits do not hang on how many there are.  The plain product from
-// 4 million values of W on (896 x 4,864: 8.5 against 11.3 us at 17 tokens, 12.0 against 11.6 at 64; 1,152 x 896 3.9 | 4.0 and
-// 5.0 | 5.5, 896 x 896 4.2 | 4.1 and 5.4 | 4.2), but for short rows in several slabs to a CU, whose start and end each pays for
+// The lines on W change at 5, 9 and 17 rows only: between these edges a row's bits do not hang on how many others there are, across
+// them another kernel sums in another order, and a norm may be folded in or not.  The plain product from 4 million values of W on
+// (896 x 4,864: 8.5 against 11.3 us at 17 tokens, 12.0 against 11.6 at 64; 1,152 x 896 3.9 | 4.0 and 5.0 | 5.5, 896 x 896 4.2 | 4.1
+// and 5.4 | 4.2), but for short rows in several slabs to a CU, whose start and end each pays for
 // (151,936 x 896: 64 to 85 against 65 to 83).  Four parts for a reader that adds sums up itself from 896 x 896 on (4.0 against
 // 4.2, and no read of the residual stream), as long as a slab of four takes the rows; rows of 8,192 columns and more
 // go in four parts even when a kernel has to add them up (3,584 x 18,944: 33.4 + 5 us against 55.8 whole).

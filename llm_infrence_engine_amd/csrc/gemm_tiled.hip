@@ -610,28 +610,29 @@ extern "C" int ms_gemm_tiled(const void* A, long long lda, const void* W, long l
 // Column parts for a product whose reader adds partial sums up itself (the norm that follows a down projection), 0 where the
 // library's product, or this kernel's whole one, is the faster way.  Few features leave a product of whole columns fewer
 // tiles than CUs: 2,048 tokens by 3,584 x 18,944 are 112 tiles of 256 for 256 CUs; in two parts 235 us + 30 for the norm that adds
-// them up, the library 363 + 17.  Time of the other way and its norm over this, 3,700 sizes (512 to 8,192 features, 768 to
-// 28,672 columns, 65 to 4,096 tokens), and outside the lines:
-//   up to 128 tokens 0.93 to 3.8, 1.5 on average;
-//   up to 256 tokens by 4,096 columns and more 0.94 to 4.1, 1.6 on average, by up to 1,024 and up to 5,120 features 0.98 to 1.26 (more
-//     features 0.89 to 1.10);
-//   up to 512 tokens by more than 8,192 columns 0.98 to 2.8; by more than 4,096 in several parts, up to 5,120 features, 0.92 to 1.6,
-//     1.1 on average, 12 of 586 below 0.97 (896 x 4,864 at 390 tokens 1.11).  Not: tiles of 128 that take every CU once (2,048 x 5,632
-//     at 390 tokens 0.93), whole columns (0.81 to 1.02), more features (0.89 to 1.1), 1,024 columns and fewer (896 x 896 0.91 to 0.96);
-//   up to 1,024 tokens by more than 8,192 columns, up to 5,120 features, 0.93 to 2.3, 1.29 on average; with more features 0.83 to 1.8,
-//     by 8,192 columns 0.85 to 1.17;
+// them up, the library 363 + 17.  Time of the other way and its norm over this, 3,565 sizes (512 to 8,192 features, 768 to
+// 28,672 columns, 65 to 4,096 tokens; every product by a W that lies in no cache: with W at hand the whole product of a narrow
+// model looks better than it is in a model, 896 x 896 by 512 tokens 0.95 where it is 1.05), inside and outside the lines:
+//   up to 128 tokens 1.05 to 4.1, 1.6 on average;
+//   up to 256 tokens by 4,096 columns and more or up to 1,024 0.95 to 3.6, 1.5 on average;
+//   up to 512 tokens by more than 8,192 columns 1.0 to 3.1; by more than 4,096 in several parts, up to 5,120 features, 0.90 to 1.8,
+//     1.13 on average; by up to 1,024 for up to 1,024 features 0.96 to 1.11.  Not: whole columns (4,480 x 6,784 at 429 tokens 0.82), more
+//     features (0.81 to 1.2), 4,096 columns (0.93 to 1.12), 1,024 and fewer for more features (0.87 to 1.0);
+//   up to 1,024 tokens by more than 8,192 columns, up to 5,120 features or by 16,384 columns and more, 0.92 to 3.2, 1.33 on average;
+//     else 0.88 to 2.0, 1.08 on average (8,192 columns 0.89 to 1.17);
+//   in all 12 of 3,416 below 0.97;
 //   beyond, by 16,384 columns and more where one round of blocks in parts fills 5/6 of the CUs, but not all: 0.96 to 2.0, 1.4 on
 //     average (3,584 x 18,944 at 1,281 to 1,536 tokens and at 1,793 to 2,304).  With every CU taken 0.96 to 1.02 (4,096 x 28,672 at 2,048
 //     tokens); elsewhere 0.74 to 1.47 (3,584 x 18,944 1.08 at 1,600 tokens, 1.4 at 1,200 and 2,560, 0.80 at 2,816): what the library
 //     takes there changes by a factor of two from one number of tokens to the next.
 extern "C" int ms_gemm_tiled_sums_parts(int M, int N, int K) {
   if (M <= 64 || N <= 0 || K < 768 || K % BK || N > 8192) return 0;
-  if (M > 128 && (M <= 256 ? K < 4096 && (K > 1024 || N > 5120)
-                  : M <= 512 ? K <= 8192 && (K <= 4096 || N > 5120)
-                  : M <= 1024 ? K <= 8192 || N > 5120 : K < 16384)) return 0;   // (asked for twice a layer: before the choice)
+  if (M > 128 && (M <= 256 ? K > 1024 && K < 4096
+                  : M <= 512 ? K <= 8192 && (K <= 4096 || N > 5120) && (K > 1024 || N > 1024)
+                  : M <= 1024 ? K <= 8192 || (N > 5120 && K < 16384) : K < 16384)) return 0;   // (asked for twice a layer: before the choice)
   const SumsChoice c = choose_sums(M, N, K);
   const int cus = ms_compute_units();
-  if (M > 256 && M <= 512 && K <= 8192 && (c.parts == 1 || (c.tile == 2 && c.blocks == cus))) return 0;
+  if (M > 256 && M <= 512 && K > 4096 && K <= 8192 && c.parts == 1) return 0;
   if (M > 1024 && (c.tile != 1 || c.parts == 1 || c.blocks >= cus || c.blocks * 6 < cus * 5)) return 0;
   return c.parts;
 }

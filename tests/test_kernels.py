@@ -774,10 +774,10 @@ def test_rows_too_far_apart_for_slabs_go_to_the_other_kernels(ops, M):
         torch.testing.assert_close(x.double(), want, atol=5e-5, rtol=5e-5)
 
 
-@pytest.mark.parametrize("M", [17, 48, 64])
+@pytest.mark.parametrize("M", [5, 9, 16, 17, 48, 64])
 @pytest.mark.parametrize("nh,nkv,d,K,v_transposed", [(14, 2, 64, 896, True), (5, 1, 128, 520, False), (3, 3, 6, 72, False), (70, 5, 64, 136, True)])
 def test_gemm_slab_qkv_equals_product_rotation_and_store(ops, M, nh, nkv, d, K, v_transposed):
-    """The front of an attention layer of 17 to 64 normed rows against a double product and the plain rotation: heads that
+    """The front of an attention layer of 5 to 64 normed rows against a double product and the plain rotation: heads that
     straddle a unit of four rows and blocks, a token that is not stored, pages plain and transposed."""
     g = torch.Generator().manual_seed(M + d + K)
     page_size, pages = 16, 6
