@@ -548,9 +548,10 @@ static double filled(int M, int N, const TileChoice& c) {
 //   up to 1,536 columns 1.02 to 2 (65 to 8,192 tokens);
 //   beyond, up to 2,048 tokens whose tiles fill 9/10 of their rounds: 0.99 to 1.3;
 //   687 other sizes of 1,600 to 5,120 columns (5,248 to 55,296 rows, 65 to 4,096 tokens), by what the tiles fill:
-//     up to 3,584 columns tiles of 192 or 160 features, those of 256 from 0.65 on, those of 128 from 0.7 on or up to 0.4 (one round
-//     that leaves CUs idle, as the library's does): 0.92 to 1.60, 1.15 on average, 8 of 385 below 0.97 (7B gate/up: 1,024 tokens 313 and
-//     245 us, 2,176 tokens 566 and 532); the others 0.71 to 1.38, 1.03 on average (14,336 x 3,584, 300 tokens 55 and 62);
+//     up to 3,584 columns tiles of 192 or 160 features, the others from 0.65 on, and those of 128 up to 0.4 (one round that leaves CUs
+//     idle, as the library's does): 0.92 to 1.60, 1.14 on average, 12 of 409 below 0.97 (7B gate/up: 1,024 tokens 313 and 245 us, 2,176
+//     tokens 566 and 532; 256 tokens of 22,016 x 2,048 0.97, but four layers of that width 597 and 592 us); the others 0.71 to 1.38, 1.03
+//     on average (14,336 x 3,584, 300 tokens 55 and 62);
 //     4,096 to 5,120 columns beyond 512 tokens from 0.8 on: 0.91 to 1.58, 1.12 on average, 4 of 108 below 0.97; the others 0.80 to
 //     1.30, 1.01 on average;
 //   8,192 columns 0.96 to 1.03.
@@ -562,7 +563,7 @@ extern "C" int ms_gemm_tiled_pays(int M, int N, int K) {
   if (c.tile == 3) return 0;
   if (M <= 2048 && c.tiles * 10 >= c.slots * 9) return 1;
   const double f = filled(M, N, c);
-  if (K <= 3584) return c.tile >= 4 || (c.tile == 1 ? f >= 0.65 : f >= 0.7 || f <= 0.4);
+  if (K <= 3584) return c.tile >= 4 || f >= 0.65 || (c.tile == 2 && f <= 0.4);
   return K <= 5120 && M > 512 && f >= 0.8;
 }
 

@@ -61,7 +61,7 @@ def test_a_captured_step_says_that_its_lengths_are_bounds(ops, monkeypatch, capt
     (2305, 11008, 4096, 0, 0),        # 0.93 0.88
     (3072, 5248, 3008, 0, 0),         # 0.71 0.69: 21 tiles of features over 8 XCDs
     (2305, 19200, 4928, 0, 0),        # 0.80 0.80
-    (1024, 37888, 3584, 1, 0), (2176, 37888, 3584, 1, 0), (4096, 22016, 2048, 1, 0), (3000, 27648, 5120, 1, 0),
+    (1024, 37888, 3584, 1, 0), (2176, 37888, 3584, 1, 0), (4096, 22016, 2048, 1, 0), (256, 22016, 2048, 1, 0), (3000, 27648, 5120, 1, 0),
     (2048, 8192, 3072, 1, 1), (70, 37888, 3584, 1, 0), (193, 18944, 3072, 0, 0),
     # both as ever: full rounds, short rows; rows that are no multiple of 64, long ones
     (2048, 37888, 3584, 1, 1), (1300, 55296, 5120, 1, 1), (8192, 9728, 896, 1, 1), (65, 7296, 1536, 1, 1), (512, 8192, 2056, 0, 0),
