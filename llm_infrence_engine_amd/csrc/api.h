@@ -122,6 +122,18 @@ int ms_gemm_skinny_norm(const float* x, long long ldx, const int* rows, const fl
                         long long ldw, const float* bias, void* out, long long ldo, int M, int N, int K, int epilogue,
                         int out_dtype, hipStream_t stream);
 
+// The products between two attentions of a decode step as one kernel (csrc/decode_chain.hip): x += attn . w_o^T, the gated
+// feed-forward behind norm2 added to x, and (w_qkv not null) the next layer's norm1, q/k/v, rotation and cache store.  `workspace`:
+// ms_decode_chain_workspace bytes (0: sizes not taken), zeroed once, for one batch size and one stream at a time; the step's
+// launches number 0 .. launches - 1 in order.
+int ms_decode_chain_workspace(int M, int H, int num_heads, int num_kv_heads, int head_dim, int I);
+void ms_decode_chain_limit(int limit);
+int ms_decode_chain(const void* attn, long long ld_attn, const void* w_o, float* x, long long ldx, const float* norm2, float eps2,
+                    const void* w_gate_up, const void* w_down, const float* norm1, float eps1, const void* w_qkv, const float* b_qkv,
+                    const int* positions, const float* inv_freq, const int* slot_mapping, void* q_out, void* k_pages, void* v_pages,
+                    int M, int H, int I, int num_heads, int num_kv_heads, int head_dim, int page_size, int v_transposed,
+                    void* workspace, int launch, int launches, hipStream_t stream);
+
 void ms_qkv_rope_store_force(int pair8);
 
 int ms_qkv_rope_store(const float* x, long long ldx, const float* norm_w, float eps, const void* W, const float* bias,

@@ -32,6 +32,7 @@ import numpy as np
 import torch
 
 from ..kernels import ops
+from ..parts.chain import DecodeChain
 from .batch import BatchBuilder, StepBuffers, StepEntry, StepLayout
 
 PORTION_BUCKETS = (16, 32, 64, 128, 256, 384, 512, 768, 1024, 1536, 2048, 3072, 4096)
@@ -70,6 +71,7 @@ class _Bucket:
         self.fields = self.buf.views(layout)
         self.slots = [self.fields[f"slots{g}"] for g in range(layout.n_groups)]
         self.graph: Optional[torch.cuda.CUDAGraph] = None
+        self.chain = None                                 # decode: what runs the layers, with a workspace that replays use
         self.logits: Optional[torch.Tensor] = None       # decode: [rows, V] of the last step
         self.hidden = None                                # portions: (residual stream, unsummed addend)
         self.sampled = False                              # decode: False, or (top-k, top-p): tokens are drawn, not the argmax
@@ -166,6 +168,8 @@ class StepGraphs:
         runner, model = self.runner, self.runner.model
         decode = max_q_len == 1 and lay.n_tokens == lay.n_requests
         ctx = self.builder.context(f, lay.n_tokens, lay.n_requests, max_q_len, max_context_len, padded=True)
+        if decode:
+            ctx.chain = bk.chain = DecodeChain.of(model, lay.n_tokens)
         caches = runner.caches(ctx.state_slots, bk.slots)
         G = lay.n_groups
         # what the table entries of the last steps changed must be on the device before a description that is all

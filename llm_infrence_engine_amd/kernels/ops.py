@@ -30,6 +30,11 @@ _SIGNATURES = {
                           _c_int, _c_int, _c_int, _c_int, _c_int, _c_int, _c_int, _c_ptr],
     "ms_decode_advance": [_c_ptr, _c_ptr, _c_ptr, _c_ptr, _c_ptr, _c_ptr, _c_ptr, _c_ptr, _c_ptr, _c_ptr, _c_int, _c_int, _c_int,
                           _c_int, _c_ptr],
+    "ms_decode_chain_workspace": [_c_int] * 6,
+    "ms_decode_chain_limit": [_c_int],
+    "ms_decode_chain": [_c_ptr, _c_ll, _c_ptr, _c_ptr, _c_ll, _c_ptr, _c_float, _c_ptr, _c_ptr, _c_ptr, _c_float, _c_ptr, _c_ptr,
+                        _c_ptr, _c_ptr, _c_ptr, _c_ptr, _c_ptr, _c_ptr, _c_int, _c_int, _c_int, _c_int, _c_int, _c_int, _c_int,
+                        _c_int, _c_ptr, _c_int, _c_int, _c_ptr],
     "ms_max_cache_groups": [],
     "ms_table_update": [_c_ptr, _c_ptr, _c_ptr, _c_ptr, _c_int, _c_int, _c_ll, _c_ptr],
     "ms_zero_rows": [_c_ptr, _c_ll, _c_ptr, _c_ptr, _c_int, _c_ptr],
@@ -922,6 +927,59 @@ def qkv_rope_store(x: torch.Tensor, norm_weight: torch.Tensor, eps: float, w_qkv
     _call("ms_qkv_rope_store", x.data_ptr(), K, norm_weight.data_ptr(), float(eps), w_qkv.data_ptr(), _ptr(bias),
           positions.data_ptr(), inv_freq.data_ptr(), slot_mapping.data_ptr(), q.data_ptr(), k_pages.data_ptr(),
           v_pages.data_ptr(), M, K, num_heads, num_kv_heads, head_dim, k_pages.shape[2], int(v_transposed), _stream())
+    return q
+
+
+def decode_chain_workspace(n_tokens: int, hidden: int, num_heads: int, num_kv_heads: int, head_dim: int, intermediate: int) -> int:
+    """Bytes of the workspace ``decode_chain`` wants for these sizes; 0: it does not take them."""
+    return _get("ms_decode_chain_workspace")(n_tokens, hidden, num_heads, num_kv_heads, head_dim, intermediate)
+
+
+def decode_chain_limit(looks: int) -> None:
+    """Tests: how often a waiting block of ``decode_chain`` looks before it gives its item up (0: the kernel's own choice)."""
+    _get("ms_decode_chain_limit")(looks)
+
+
+def decode_chain(attn: torch.Tensor, w_o: torch.Tensor, x: torch.Tensor, norm2: torch.Tensor, eps2: float,
+                 w_gate_up: torch.Tensor, w_down: torch.Tensor, num_heads: int, num_kv_heads: int, head_dim: int,
+                 workspace: torch.Tensor, launch: int, launches: int, front=None) -> Optional[torch.Tensor]:
+    """x += attn @ w_o.T; x += (silu(g) * u) @ w_down.T for g, u = rms_norm(x, norm2) @ w_gate_up.T (interleaved rows), in
+    one kernel.  ``front``: the arguments (norm weight, eps, w_qkv, bias, positions, inv_freq, slot_mapping, k_pages, v_pages,
+    v_transposed) of ``qkv_rope_store`` for the new x, which then runs in the same kernel; returns its q.  ``workspace``: uint8,
+    zeroed once, of one batch size; ``launch`` numbers the step's chains 0 .. launches - 1, in order, one stream at a time."""
+    _check(attn, "attn", torch.bfloat16)
+    _check(x, "x", torch.float32)
+    M, H = x.shape
+    _check(attn, "attn", torch.bfloat16, (M, num_heads * head_dim))
+    _check(w_o, "w_o", torch.bfloat16, (H, num_heads * head_dim))
+    _check(norm2, "norm2", torch.float32, (H,))
+    _check(w_gate_up, "w_gate_up", torch.bfloat16, (None, H))
+    I = w_gate_up.shape[0] // 2
+    _check(w_gate_up, "w_gate_up", torch.bfloat16, (2 * I, H))
+    _check(w_down, "w_down", torch.bfloat16, (H, I))
+    _check(workspace, "workspace", torch.uint8)
+    if 0 < workspace.numel() < decode_chain_workspace(M, H, num_heads, num_kv_heads, head_dim, I):
+        raise ValueError("the workspace is too small")
+    q, tail = None, (None, 0.0) + (None,) * 8
+    page_size, v_transposed = 1, False
+    if front is not None:
+        norm1, eps1, w_qkv, bias, positions, inv_freq, slot_mapping, k_pages, v_pages, v_transposed = front
+        _check(norm1, "norm1", torch.float32, (H,))
+        _check(w_qkv, "w_qkv", torch.bfloat16, ((num_heads + 2 * num_kv_heads) * head_dim, H))
+        if bias is not None:
+            _check(bias, "bias", torch.float32, (w_qkv.shape[0],))
+        _check(positions, "positions", torch.int32, (M,))
+        _check(inv_freq, "inv_freq", torch.float32, (head_dim // 2,))
+        _check(slot_mapping, "slot_mapping", torch.int32, (M,))
+        _check(k_pages, "k_pages", torch.bfloat16, (None, num_kv_heads, None, head_dim))
+        _check(v_pages, "v_pages", torch.bfloat16, _v_shape(k_pages, v_transposed))
+        q = torch.empty((M, num_heads * head_dim), dtype=torch.bfloat16, device=x.device)
+        page_size = k_pages.shape[2]
+        tail = (norm1.data_ptr(), float(eps1), w_qkv.data_ptr(), _ptr(bias), positions.data_ptr(), inv_freq.data_ptr(),
+                slot_mapping.data_ptr(), q.data_ptr(), k_pages.data_ptr(), v_pages.data_ptr())
+    _call("ms_decode_chain", attn.data_ptr(), attn.shape[1], w_o.data_ptr(), x.data_ptr(), H, norm2.data_ptr(), float(eps2),
+          w_gate_up.data_ptr(), w_down.data_ptr(), *tail, M, H, I, num_heads, num_kv_heads, head_dim, page_size,
+          int(v_transposed), workspace.data_ptr(), launch, launches, _stream())
     return q
 
 

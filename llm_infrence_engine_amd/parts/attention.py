@@ -152,9 +152,14 @@ class GQAttention(Mixer):
     def forward_residual(self, h, ctx, kv, state, x):
         if kv is None:
             raise RuntimeError("attention needs a key/value cache view")
-        nh, nkv, d, dv = self.num_heads, self.num_kv_heads, self.head_dim, self.value_dim
         if self.gate or self.value_blend:
             return self._forward_packed(h, ctx, kv, x)
+        out = self.attend(self.project_and_store(h, ctx, kv), ctx, kv)
+        return linear.linear_residual(out, self.w_o, self.b_o, x, self.hands_on_sums)
+
+    def project_and_store(self, h, ctx, kv):
+        """q [N, nh d] (or the packed projection, of which the attention reads the first columns); k and v go into the pages."""
+        nh, nkv, d, dv = self.num_heads, self.num_kv_heads, self.head_dim, self.value_dim
         q = None
         if self.position is not None and dv == d:
             q = self.position.project_encode_store(h, self.w_qkv, self.b_qkv, nh, nkv, d, ctx, kv)
@@ -172,10 +177,14 @@ class GQAttention(Mixer):
                 self.position.encode_and_store(q, nh, nkv, d, ctx, kv)
             elif kv.store:
                 ops.rope_store(q, nh, nkv, d, 0, None, None, kv.slot_mapping, kv.k_pages, kv.v_pages, kv.v_transposed)
-        out = self.rt.empty(ctx.num_tokens, nh * dv)
-        ops.paged_attention(q, kv, ctx, out, nh, self.scale, self.window, self.sink_w, self.softcap, self.slopes, None,
-                            self.out_scale)
-        return linear.linear_residual(out, self.w_o, self.b_o, x, self.hands_on_sums)
+        return q
+
+    def attend(self, q, ctx, kv):
+        """The heads' results [N, nh dv] for what ``project_and_store`` left."""
+        out = self.rt.empty(ctx.num_tokens, self.num_heads * self.value_dim)
+        ops.paged_attention(q, kv, ctx, out, self.num_heads, self.scale, self.window, self.sink_w, self.softcap, self.slopes,
+                            None, self.out_scale)
+        return out
 
     def _blending(self, qkv, ctx):
         """{} or the keyword that has the position encoding blend the values with the first such layer's."""

@@ -95,6 +95,8 @@ class Model:
         copies of it) and what the last run has still to write into it (an addend, a write that the final norm carries out
         itself, or None)."""
         x = self.embedding.forward(ctx)
+        if ctx.chain is not None and ctx.chain.takes(caches):
+            return ctx.chain.forward(self, x, ctx, caches), None
         kept = x.clone() if self.pass_entry is not None and self.pass_entry.keeps_embedding else None
         pending = None
         for i, run in enumerate(self.spec.order):

@@ -79,3 +79,18 @@ def test_a_library_older_than_its_sources_is_built_again_not_loaded(tmp_path, mo
     build.load()
     assert calls == [1] and loaded[-1] == str(old)
     monkeypatch.setattr(build, "_lib", None)
+
+
+def test_loads_written_in_assembly_wait_for_their_bases():
+    """A memory instruction may read a scalar register five wait states after a vector instruction (the compiler's v_readlane)
+    wrote it, which the compiler does not see to for assembly; and a load's registers are taken as written where its block
+    ends.  So a block with loads begins with the wait states and ends with the wait for the loads."""
+    for src in build.sources():
+        text = src.read_text()
+        for name, body in re.findall(r'#define (\w+)[^\n]*?("[^"\n]*(?:global|buffer|flat)_load[^\n]*)', text):
+            blocks = [b for b in re.findall(r"asm volatile\((.*?)\s*:", text, re.S) if re.search(rf"\b{name}\(", b)]
+            assert blocks, (src.name, name)
+            for b in blocks:
+                assert b.startswith("SGPRS_READY") and b.endswith('"s_waitcnt vmcnt(0)"'), (src.name, b)
+            assert '#define SGPRS_READY "s_nop 4' in text
+        assert not re.search(r'asm volatile\(\s*"[^"]*_(load|store)', text), src.name     # none beside those

@@ -96,6 +96,8 @@ def _block(ops, norm=None, mixer=None, feed_forward=None, block=None):
     from llm_infrence_engine_amd.parts.norms import RMSNorm
 
     def of(base, body):
+        if body is True:
+            return base
         return type("Own", body if isinstance(body, tuple) else (base,), {} if body is None or isinstance(body, tuple) else body)
 
     norms = [of(RMSNorm, norm)("", 64, 1e-5) for _ in range(2)]
@@ -144,3 +146,38 @@ def test_the_model_adds_up_sums_for_a_reader_that_takes_one_addend(ops, reader):
     else:
         assert left is None
         torch.testing.assert_close(x.cpu().double(), x0.double() + sums.double().sum(0), atol=2e-6, rtol=2e-6)
+
+
+def test_chains_take_the_parts_whose_arithmetic_they_have(ops):
+    """Layers of exactly the parts that the kernel of a decode step's products stands in for, and no class derived from one;
+    whatever it has no place for (a bias behind the heads, gates, blended values, heads turned in part) goes layer by layer."""
+    from llm_infrence_engine_amd.parts import chain
+    from llm_infrence_engine_amd.parts.attention import GQAttention
+    from llm_infrence_engine_amd.parts.positions import RotaryHalf
+
+    exact = dict(norm=True, mixer=True, feed_forward=True, block=True)
+
+    def sizes(turned=32, **attention):
+        b = _block(ops, **exact)
+        b.mixer = GQAttention("", RotaryHalf("", 32, turned, 1e4), 64, 2, 2, 32, 0.1, **attention)
+        return chain._sizes(b)
+
+    assert sizes() == sizes(qkv_bias=False) == sizes(window=8, sink=True) == (2, 2, 32, 64, 128)
+    assert sizes(turned=16) is sizes(out_bias=True) is sizes(gate=True) is sizes(value_blend="first") is None
+    own = {"other": lambda self: None}
+    for part in ("norm", "mixer", "feed_forward", "block"):
+        b = _block(ops, **dict(exact, **{part: own}))
+        b.mixer.position = RotaryHalf("", 32, 32, 1e4)
+        assert chain._sizes(b) is None
+    assert chain._sizes(_block(ops, **exact)) is None      # no position encoding
+
+    def model(runs=2, opens=None, dtype=torch.bfloat16, entry=None):
+        b = _block(ops, **exact)
+        b.mixer.position = RotaryHalf("", 32, 32, 1e4)
+        return SimpleNamespace(spec=SimpleNamespace(order=[SimpleNamespace(layer=0, opens_pass=opens)] * runs), layers=[b],
+                               rt=SimpleNamespace(dtype=dtype, device="cpu"), pass_entry=entry)
+
+    made = chain.DecodeChain.of(model(), 8)
+    assert made.launches == 2 and not made.workspace.any()
+    assert chain.DecodeChain.of(model(), 9) is chain.DecodeChain.of(model(runs=1), 1) is chain.DecodeChain.of(model(opens=0), 1) is None
+    assert chain.DecodeChain.of(model(dtype=torch.float32), 1) is chain.DecodeChain.of(model(entry=b""), 1) is None

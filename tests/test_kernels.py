@@ -1899,3 +1899,89 @@ def test_read_probe_reads_everything_once(ops):
         assert got == np.bitwise_xor.reduce(t[:n].cpu().numpy().view(np.uint32))
     with pytest.raises(ValueError, match="16 bytes"):
         ops.read_probe(t[:3])
+
+
+def _chain_reference(attn, w_o, x, n2, w_gu, w_down, eps):
+    """x after the output projection and the gated feed-forward, in double, rounded to bfloat16 where the kernel rounds, and how
+    far float sums may lie from it: a product of the middle whose sum falls to the other side of a rounding boundary moves by
+    one step of its size, 2^-8 of it at most, and takes w_down's column with it; two of the largest at once, and 1e-4 for the
+    float sums of values up to about 5."""
+    x = x.double() + attn.double() @ w_o.double().T
+    inv = 1 / torch.sqrt((x * x).mean(1, keepdim=True) + eps)
+    gu = ((x * n2.double()).bfloat16().double() @ w_gu.double().T) * inv
+    act = (torch.nn.functional.silu(gu[:, 0::2]) * gu[:, 1::2]).bfloat16().double()
+    return x + act @ w_down.double().T, 2 * act.abs().max().item() / 256 * w_down.abs().max().item() + 1e-4
+
+
+@pytest.mark.parametrize("limit", [0, 1])
+@pytest.mark.parametrize("M", [1, 3, 4, 5, 8])
+@pytest.mark.parametrize("H,I,nh,nkv,d,v_transposed", [(896, 4864, 14, 2, 64, True), (1024, 6144, 8, 8, 128, False),
+                                                       (64, 32, 2, 1, 32, True), (288, 544, 3, 1, 96, True)])
+def test_decode_chain(ops, M, H, I, nh, nkv, d, v_transposed, limit):
+    """Two steps of three chains on one workspace, each against double: full and short rows (waves and runs without a
+    k-step), tokens that fill a group and not, a token that is not stored, a last chain without a front.  With a limit of one
+    look the blocks that wait give their items up and one of them works off the list: the same results to the bit."""
+    page_size, pages, eps, n = 16, 8, 1e-6, nh + 2 * nkv
+
+    def run(limit):
+        g = torch.Generator().manual_seed(M + H + I)
+        x = torch.randn(M, H, generator=g).to(DEV)
+        inv_freq = (1.0 / (1e6 ** (torch.arange(0, d, 2, dtype=torch.float64) / d))).float().to(DEV)
+        ws = torch.zeros(ops.decode_chain_workspace(M, H, nh, nkv, d, I), dtype=torch.uint8, device=DEV)
+        kept = []
+        ops.decode_chain_limit(limit)
+        try:
+            for call in range(6):
+                attn = torch.randn(M, nh * d, generator=g).bfloat16().to(DEV)
+                w_o = (torch.randn(H, nh * d, generator=g) / math.sqrt(nh * d)).bfloat16().to(DEV)
+                n1, n2 = ((1 + 0.1 * torch.randn(H, generator=g)).to(DEV) for _ in range(2))
+                w_gu = (torch.randn(2 * I, H, generator=g) / math.sqrt(H)).bfloat16().to(DEV)
+                w_down = (torch.randn(H, I, generator=g) / math.sqrt(I)).bfloat16().to(DEV)
+                w_qkv = (torch.randn(n * d, H, generator=g) / math.sqrt(H)).bfloat16().to(DEV)
+                bias = torch.randn(n * d, generator=g).to(DEV) if call % 2 else None
+                pos = torch.randint(0, 3000, (M,), generator=g).to(torch.int32).to(DEV)
+                slots = torch.randperm(pages * page_size, generator=g)[:M].to(torch.int32)
+                slots[M // 2] = -1 if M > 1 else slots[0]
+                slots = slots.to(DEV)
+                kp = torch.zeros(pages, nkv, page_size, d, dtype=torch.bfloat16, device=DEV)
+                vp = torch.zeros((pages, nkv, d, page_size) if v_transposed else (pages, nkv, page_size, d), dtype=torch.bfloat16, device=DEV)
+                want, apart = _chain_reference(attn, w_o, x, n2, w_gu, w_down, eps)
+                front = (n1, eps, w_qkv, bias, pos, inv_freq, slots, kp, vp, v_transposed) if call % 3 < 2 else None
+                q = ops.decode_chain(attn, w_o, x, n2, eps, w_gu, w_down, nh, nkv, d, ws, call % 3, 3, front)
+                assert (x.double() - want).abs().max().item() <= apart
+                assert (x.double() - want).square().mean().sqrt().item() <= apart / 8     # (most do not move)
+                kept.append(x.clone())
+                if front is None:
+                    assert q is None
+                    continue
+                y = ((want * n1.double()) / torch.sqrt((want * want).mean(1, keepdim=True) + eps)) @ w_qkv.double().T
+                y = (y + (bias.double() if bias is not None else 0)).view(M, n, d).cpu()
+                rot = rope_reference(y[:, :nh + nkv], pos.cpu(), d, inv_freq.double().cpu())
+                torch.testing.assert_close(q.double().cpu().view(M, nh, d), rot[:, :nh], atol=4e-2, rtol=1.6e-2)
+                for t in range(M):
+                    s = int(slots[t])
+                    if s < 0:
+                        continue
+                    p, o = divmod(s, page_size)
+                    torch.testing.assert_close(kp[p, :, o].double().cpu(), rot[t, nh:], atol=4e-2, rtol=1.6e-2)
+                    v = vp[p, :, :, o] if v_transposed else vp[p, :, o]
+                    torch.testing.assert_close(v.double().cpu(), y[t, nh + nkv:], atol=4e-2, rtol=1.6e-2)
+                untouched = torch.ones(pages * page_size, dtype=torch.bool)
+                untouched[slots[slots >= 0].long().cpu()] = False
+                assert (kp.permute(0, 2, 1, 3).reshape(pages * page_size, -1)[untouched.to(DEV)] == 0).all()
+                kept += [q, kp, vp]
+            assert not ws[:4 * 1152].any()      # nothing is left on the list
+        finally:
+            ops.decode_chain_limit(0)
+        return kept
+
+    got = run(limit)
+    if limit:
+        assert all(torch.equal(a, b) for a, b in zip(got, run(0)))
+
+
+def test_decode_chain_refuses_what_it_cannot_take(ops):
+    for sizes in [(9, 896, 14, 2, 64, 4864), (0, 896, 14, 2, 64, 4864), (1, 1056, 14, 2, 64, 4864), (1, 896, 17, 1, 64, 4864),
+                  (1, 896, 14, 2, 64, 6176), (1, 896, 14, 2, 64, 4880), (1, 880, 14, 2, 64, 4864), (1, 896, 14, 2, 60, 4864)]:
+        assert ops.decode_chain_workspace(*sizes) == 0
+    assert ops.decode_chain_workspace(8, 896, 14, 2, 64, 4864) > 0
