@@ -168,9 +168,9 @@ class StepGraphs:
         runner, model = self.runner, self.runner.model
         decode = max_q_len == 1 and lay.n_tokens == lay.n_requests
         ctx = self.builder.context(f, lay.n_tokens, lay.n_requests, max_q_len, max_context_len, padded=True)
-        if decode:
-            ctx.chain = bk.chain = DecodeChain.of(model, lay.n_tokens)
         caches = runner.caches(ctx.state_slots, bk.slots)
+        if decode:
+            ctx.chain = bk.chain = DecodeChain.of(model, ctx, caches)
         G = lay.n_groups
         # what the table entries of the last steps changed must be on the device before a description that is all
         # padding stands in for a step

@@ -40,7 +40,7 @@ class ModelRunner:
         self.pools = CachePools(self.layout, page_size, num_pages, max_requests, self.rt,
                                 self.manager.max_pages_per_request)
         self.builder = BatchBuilder(self.manager, self.pools, model.spec.vocab_size, self.rt.device)
-        self.chains = {}         # for steps of single tokens launched kernel by kernel: tokens -> DecodeChain, or None
+        self.chains = {}         # for steps of single tokens launched kernel by kernel: (tokens, long contexts) -> DecodeChain, or None
         self.graphs = None
         # a part that cannot be captured (it walks the requests on the host, as a mixer with state usually does)
         # keeps the whole model out of graphs
@@ -95,12 +95,13 @@ class ModelRunner:
             logits = self.graphs.run_portions(entries)
         else:
             built = self.builder.build(entries)
+            caches = self.caches(built.ctx.state_slots, built.slots)
             if built.ctx.decode_only:
-                n = built.ctx.num_tokens
-                if n not in self.chains:
-                    self.chains[n] = DecodeChain.of(self.model, n)
-                built.ctx.chain = self.chains[n]
-            logits = self.model.forward(built.ctx, self.caches(built.ctx.state_slots, built.slots))
+                key = (built.ctx.num_tokens, built.ctx.max_context_len > ops.DECODE_KEYS)
+                if key not in self.chains:
+                    self.chains[key] = DecodeChain.of(self.model, built.ctx, caches)
+                built.ctx.chain = self.chains[key]
+            logits = self.model.forward(built.ctx, caches)
         for e in entries:
             m.advance(e.req_id, m.computed(e.req_id) + len(e.tokens))
         return logits

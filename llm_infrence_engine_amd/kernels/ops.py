@@ -7,6 +7,7 @@ missing library, raises.
 from __future__ import annotations
 
 import ctypes
+import struct
 import sys
 from typing import Optional
 
@@ -30,7 +31,12 @@ _SIGNATURES = {
                           _c_int, _c_int, _c_int, _c_int, _c_int, _c_int, _c_int, _c_ptr],
     "ms_decode_advance": [_c_ptr, _c_ptr, _c_ptr, _c_ptr, _c_ptr, _c_ptr, _c_ptr, _c_ptr, _c_ptr, _c_ptr, _c_int, _c_int, _c_int,
                           _c_int, _c_ptr],
-    "ms_decode_chain_workspace": [_c_int] * 6,
+    "ms_decode_chain_workspace": [_c_int] * 7,
+    "ms_decode_layer_bytes": [],
+    "ms_decode_first": [_c_ptr, _c_ll, _c_ptr, _c_float, _c_ptr, _c_ptr, _c_ptr, _c_ptr, _c_ptr, _c_ptr, _c_ptr, _c_int, _c_int,
+                        _c_int, _c_int, _c_int, _c_int, _c_int, _c_int, _c_ptr, _c_ptr],
+    "ms_decode_layers": [_c_ptr, _c_ptr, _c_ll, _c_ptr, _c_ptr, _c_ptr, _c_ptr, _c_ptr, _c_int, _c_float, _c_int, _c_int, _c_int,
+                         _c_int, _c_int, _c_int, _c_int, _c_int, _c_ptr, _c_ptr],
     "ms_decode_chain_limit": [_c_int],
     "ms_decode_chain": [_c_ptr, _c_ll, _c_ptr, _c_ptr, _c_ll, _c_ptr, _c_float, _c_ptr, _c_ptr, _c_ptr, _c_float, _c_ptr, _c_ptr,
                         _c_ptr, _c_ptr, _c_ptr, _c_ptr, _c_ptr, _c_ptr, _c_int, _c_int, _c_int, _c_int, _c_int, _c_int, _c_int,
@@ -930,9 +936,73 @@ def qkv_rope_store(x: torch.Tensor, norm_weight: torch.Tensor, eps: float, w_qkv
     return q
 
 
-def decode_chain_workspace(n_tokens: int, hidden: int, num_heads: int, num_kv_heads: int, head_dim: int, intermediate: int) -> int:
-    """Bytes of the workspace ``decode_chain`` wants for these sizes; 0: it does not take them."""
-    return _get("ms_decode_chain_workspace")(n_tokens, hidden, num_heads, num_kv_heads, head_dim, intermediate)
+def decode_chain_workspace(n_tokens: int, hidden: int, num_heads: int, num_kv_heads: int, head_dim: int, intermediate: int,
+                           n_layers: int = 0) -> int:
+    """Bytes of the workspace ``decode_chain`` wants for these sizes, or with ``n_layers`` ``decode_first`` and
+    ``decode_layers``; 0: they do not take them."""
+    return _get("ms_decode_chain_workspace")(n_tokens, hidden, num_heads, num_kv_heads, head_dim, intermediate, n_layers)
+
+
+DECODE_KEYS = 1024      # keys of a context, with the step's own, that ``decode_layers`` reads at most
+
+
+def decode_layer_table(layers, device) -> torch.Tensor:
+    """The records of ``decode_layers``: for each layer a dict of its tensors w_o, w_gate_up, w_down, norm2, k_pages, v_pages
+    and eps2, and of the layer after it (not of the last one) w_front, norm1, b_front (may be None), inv_freq, front_k, front_v
+    and eps1.  The tensors have to outlive the table; it does not keep them."""
+    names = ("w_o", "w_gate_up", "w_down", "w_front", "norm2", "norm1", "b_front", "inv_freq", "k_pages", "v_pages", "front_k", "front_v")
+    rows = b"".join(struct.pack("<12Q2f", *(_ptr(l.get(n)) or 0 for n in names), l["eps2"], l.get("eps1", 0.0)) for l in layers)
+    if len(rows) != len(layers) * _get("ms_decode_layer_bytes")():
+        raise build.KernelLibraryError("the library's record of a layer has another size than this module's")
+    return torch.frombuffer(bytearray(rows), dtype=torch.uint8).to(device)
+
+
+def decode_first(x: torch.Tensor, norm_weight: torch.Tensor, eps: float, w_qkv: torch.Tensor, bias: Optional[torch.Tensor],
+                 positions: torch.Tensor, inv_freq: torch.Tensor, slot_mapping: torch.Tensor, k_pages: torch.Tensor,
+                 v_pages: torch.Tensor, num_heads: int, num_kv_heads: int, head_dim: int, intermediate: int, n_layers: int,
+                 workspace: torch.Tensor) -> None:
+    """rms_norm(x) @ w_qkv.T + bias of the first layer, q and k rotated; k and v go into the pages, all three into the
+    workspace, for the ``decode_layers`` that has to follow on the same one."""
+    _check(x, "x", torch.float32)
+    M, H = x.shape
+    _check(norm_weight, "norm_weight", torch.float32, (H,))
+    _check(w_qkv, "w_qkv", torch.bfloat16, ((num_heads + 2 * num_kv_heads) * head_dim, H))
+    if bias is not None:
+        _check(bias, "bias", torch.float32, (w_qkv.shape[0],))
+    _check(positions, "positions", torch.int32, (M,))
+    _check(inv_freq, "inv_freq", torch.float32, (head_dim // 2,))
+    _check(slot_mapping, "slot_mapping", torch.int32, (M,))
+    _check(k_pages, "k_pages", torch.bfloat16, (None, num_kv_heads, None, head_dim))
+    _check(v_pages, "v_pages", torch.bfloat16, _v_shape(k_pages, True))
+    _check(workspace, "workspace", torch.uint8)
+    if workspace.numel() < decode_chain_workspace(M, H, num_heads, num_kv_heads, head_dim, intermediate, n_layers):
+        raise ValueError("the workspace is too small")
+    _call("ms_decode_first", x.data_ptr(), H, norm_weight.data_ptr(), float(eps), w_qkv.data_ptr(), _ptr(bias),
+          positions.data_ptr(), inv_freq.data_ptr(), slot_mapping.data_ptr(), k_pages.data_ptr(), v_pages.data_ptr(), M, H,
+          intermediate, num_heads, num_kv_heads, head_dim, k_pages.shape[2], n_layers, workspace.data_ptr(), _stream())
+
+
+def decode_layers(table: torch.Tensor, x: torch.Tensor, positions: torch.Tensor, slot_mapping: torch.Tensor,
+                  context_lens: torch.Tensor, block_table: torch.Tensor, table_rows: Optional[torch.Tensor], scale: float,
+                  num_heads: int, num_kv_heads: int, head_dim: int, intermediate: int, page_size: int, n_layers: int,
+                  workspace: torch.Tensor) -> torch.Tensor:
+    """Every layer of a step of single tokens from the first one's attention on, behind ``decode_first``: x in place.
+    ``table``: ``decode_layer_table``; contexts of at most ``DECODE_KEYS`` keys."""
+    _check(x, "x", torch.float32)
+    M, H = x.shape
+    _check(table, "table", torch.uint8, (n_layers * _get("ms_decode_layer_bytes")(),))
+    for name, t in (("positions", positions), ("slot_mapping", slot_mapping), ("context_lens", context_lens)):
+        _check(t, name, torch.int32, (M,))
+    _check(block_table, "block_table", torch.int32, (None, None))
+    if table_rows is not None:
+        _check(table_rows, "table_rows", torch.int32, (M,))
+    _check(workspace, "workspace", torch.uint8)
+    if workspace.numel() < decode_chain_workspace(M, H, num_heads, num_kv_heads, head_dim, intermediate, n_layers):
+        raise ValueError("the workspace is too small")
+    _call("ms_decode_layers", table.data_ptr(), x.data_ptr(), H, positions.data_ptr(), slot_mapping.data_ptr(),
+          context_lens.data_ptr(), block_table.data_ptr(), _ptr(table_rows), block_table.shape[1], float(scale), M, H,
+          intermediate, num_heads, num_kv_heads, head_dim, page_size, n_layers, workspace.data_ptr(), _stream())
+    return x
 
 
 def decode_chain_limit(looks: int) -> None:

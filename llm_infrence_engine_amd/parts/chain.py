@@ -1,10 +1,12 @@
-"""A decode step of a narrow model as attentions and the chains between them.
+"""A decode step of a narrow model in few launches.
 
 Between two attentions lie four products (output projection, gate/up, down, the next layer's q/k/v) with two norms.  For up to
 8 tokens each is over in a few microseconds, most of which are a launch and the wait for weights, so one kernel runs all four
-(``ops.decode_chain``): a layer takes two launches instead of five.  It needs a workspace that outlives the step and belongs
-to one batch size: every captured decode graph has its own (``engine/graph.py``), and a runner one for every batch size of
-the steps that it launches kernel by kernel (``engine/runner.py``).
+(``ops.decode_chain``): a layer takes two launches instead of five.  Where contexts are short and the attention is the plain one
+(heads of 64, no window, sink, cap or slopes, one cache group), that is in the kernel too, and all layers of the step are two launches
+(``ops.decode_first``, ``ops.decode_layers``).  Either needs a workspace that outlives the step and belongs to one batch size:
+every captured decode graph has its own (``engine/graph.py``), and a runner one for every batch size of the steps that it
+launches kernel by kernel (``engine/runner.py``).
 """
 from __future__ import annotations
 
@@ -37,42 +39,102 @@ def _sizes(layer) -> Optional[tuple]:
     return m.num_heads, m.num_kv_heads, m.head_dim, m.hidden_size, f.intermediate_size
 
 
-class DecodeChain:
-    """The chains of one batch size, with their workspace."""
+def _plain_attention(m) -> bool:
+    return m.window is None and m.sink_w is None and not m.softcap and m.slopes is None and m.out_scale == 1.0
 
-    def __init__(self, sizes: tuple, launches: int, n_bytes: int, device):
-        self.sizes, self.launches = sizes, launches
-        self.workspace = torch.zeros(n_bytes, dtype=torch.uint8, device=device)
+
+class DecodeChain:
+    """The chains of one batch size, with their workspace; ``table``: what ``ops.decode_layers`` reads, where the step's layers
+    go in two launches, else None."""
+
+    def __init__(self, model, sizes: tuple, n_bytes: int):
+        self.sizes, self.runs = sizes, len(model.spec.order)
+        self.layers = [model.layers[run.layer] for run in model.spec.order]
+        self.workspace = torch.zeros(n_bytes, dtype=torch.uint8, device=model.rt.device)
+        self.table, self.pages = None, []
         self.broken_off = False      # a step ended with an exception between its launches
 
     @classmethod
-    def of(cls, model, n_tokens: int) -> Optional["DecodeChain"]:
-        """For decode steps of ``n_tokens`` tokens; None where the kernel does not take the model or the size."""
-        runs = model.spec.order
-        if model.rt.dtype != torch.bfloat16 or model.pass_entry is not None or not 2 <= len(runs) <= 1024:
+    def of(cls, model, ctx, caches) -> Optional["DecodeChain"]:
+        """For decode steps like ``ctx``, of as many tokens and of contexts on the same side of ``ops.DECODE_KEYS``, from
+        ``caches``; None where the kernels do not take the model or the size."""
+        runs, n = model.spec.order, ctx.num_tokens
+        if model.rt.dtype != torch.bfloat16 or model.pass_entry is not None or not 2 <= len(runs) <= 1024 or n != ctx.num_requests:
             return None
         if any(run.opens_pass is not None for run in runs):
             return None
         sizes = {_sizes(model.layers[run.layer]) for run in runs}
-        if len(sizes) != 1 or None in sizes:
+        if len(sizes) != 1 or None in sizes or not cls._stores(caches):
             return None
         sizes = sizes.pop()
         nh, nkv, d, H, I = sizes
-        n_bytes = ops.decode_chain_workspace(n_tokens, H, nh, nkv, d, I)
-        return cls(sizes, len(runs), n_bytes, model.rt.device) if n_bytes else None
+        if ctx.max_context_len <= ops.DECODE_KEYS and cls._one_group(model, caches):
+            n_bytes = ops.decode_chain_workspace(n, H, nh, nkv, d, I, len(runs))
+            if n_bytes:
+                chain = cls(model, sizes, n_bytes)
+                chain._lay_out(caches)
+                return chain
+        n_bytes = ops.decode_chain_workspace(n, H, nh, nkv, d, I)
+        return cls(model, sizes, n_bytes) if n_bytes else None
+
+    @staticmethod
+    def _stores(caches) -> bool:
+        """Whether every run stores its keys and values in bfloat16 pages of its own."""
+        return all(c.kv is not None and c.kv.store and c.kv.k_pages.dtype == torch.bfloat16 for c in caches)
+
+    @staticmethod
+    def _one_group(model, caches) -> bool:
+        """Whether all runs have plain attention of one scale over one group's pages, laid out as the kernel reads them."""
+        kv = caches[0].kv
+        mixers = [model.layers[run.layer].mixer for run in model.spec.order]
+        page_size = kv.k_pages.shape[2]
+        return (all(_plain_attention(m) and m.scale == mixers[0].scale for m in mixers) and page_size >= 16
+                and page_size & (page_size - 1) == 0
+                and all(c.kv.block_table is kv.block_table and c.kv.slot_mapping is kv.slot_mapping and c.kv.v_transposed
+                        and c.kv.window is None and c.kv.stride == 1 for c in caches))
+
+    def _lay_out(self, caches):
+        rows = []
+        for i, (layer, c) in enumerate(zip(self.layers, caches)):
+            m, f = layer.mixer, layer.feed_forward
+            row = dict(w_o=m.w_o, w_gate_up=f.w_gate_up, w_down=f.w_down, norm2=layer.feed_forward_norm.weight,
+                       eps2=layer.feed_forward_norm.eps, k_pages=c.kv.k_pages, v_pages=c.kv.v_pages)
+            if i + 1 < len(self.layers):
+                then, kv = self.layers[i + 1], caches[i + 1].kv
+                row.update(w_front=then.mixer.w_qkv, norm1=then.mixer_norm.weight, eps1=then.mixer_norm.eps, b_front=then.mixer.b_qkv,
+                           inv_freq=then.mixer.position.inv_freq, front_k=kv.k_pages, front_v=kv.v_pages)
+            rows.append(row)
+        self.pages = [t for c in caches for t in (c.kv.k_pages, c.kv.v_pages)]
+        self.table = ops.decode_layer_table(rows, self.workspace.device)
 
     def takes(self, caches) -> bool:
-        """Whether every run stores its keys and values in bfloat16 pages of its own."""
-        return len(caches) == self.launches and all(c.kv is not None and c.kv.store and c.kv.k_pages.dtype == torch.bfloat16
-                                                    for c in caches)
+        """Whether these are the caches that the chain was made for (or, where it reads no table of them, any like them)."""
+        if len(caches) != self.runs or not self._stores(caches):
+            return False
+        return self.table is None or all(a.data_ptr() == b.data_ptr() for a, b in
+                                         zip(self.pages, (t for c in caches for t in (c.kv.k_pages, c.kv.v_pages))))
 
-    def forward(self, model, x, ctx, caches):
+    def forward(self, x, ctx, caches):
         """All runs of the order on the embedded tokens ``x`` [N, H], in place; returns x."""
         if self.broken_off:          # its launches did not count each other up: start over
             self.workspace.zero_()
         self.broken_off = True
+        (self._layer_by_layer if self.table is None else self._whole)(x, ctx, caches)
+        self.broken_off = False
+        return x
+
+    def _whole(self, x, ctx, caches):
+        nh, nkv, d, _, I = self.sizes
+        first, kv = self.layers[0], caches[0].kv
+        m, norm = first.mixer, first.mixer_norm
+        ops.decode_first(x, norm.weight, norm.eps, m.w_qkv, m.b_qkv, ctx.positions, m.position.inv_freq, kv.slot_mapping,
+                         kv.k_pages, kv.v_pages, nh, nkv, d, I, self.runs, self.workspace)
+        ops.decode_layers(self.table, x, ctx.positions, kv.slot_mapping, ctx.context_lens, kv.block_table, kv.table_rows, m.scale,
+                          nh, nkv, d, I, kv.k_pages.shape[2], self.runs, self.workspace)
+
+    def _layer_by_layer(self, x, ctx, caches):
         nh, nkv, d, _, _ = self.sizes
-        layers = [model.layers[run.layer] for run in model.spec.order]
+        layers = self.layers
         q = layers[0].mixer.project_and_store(layers[0].mixer_norm.lazy(x), ctx, caches[0].kv)
         for i, layer in enumerate(layers):
             m, f = layer.mixer, layer.feed_forward
@@ -83,6 +145,4 @@ class DecodeChain:
                 front = (then.mixer_norm.weight, then.mixer_norm.eps, then.mixer.w_qkv, then.mixer.b_qkv, ctx.positions,
                          then.mixer.position.inv_freq, kv.slot_mapping, kv.k_pages, kv.v_pages, kv.v_transposed)
             q = ops.decode_chain(out, m.w_o, x, layer.feed_forward_norm.weight, layer.feed_forward_norm.eps, f.w_gate_up,
-                                 f.w_down, nh, nkv, d, self.workspace, i, self.launches, front)
-        self.broken_off = False
-        return x
+                                 f.w_down, nh, nkv, d, self.workspace, i, self.runs, front)

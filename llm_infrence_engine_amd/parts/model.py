@@ -96,7 +96,7 @@ class Model:
         itself, or None)."""
         x = self.embedding.forward(ctx)
         if ctx.chain is not None and ctx.chain.takes(caches):
-            return ctx.chain.forward(self, x, ctx, caches), None
+            return ctx.chain.forward(x, ctx, caches), None
         kept = x.clone() if self.pass_entry is not None and self.pass_entry.keeps_embedding else None
         pending = None
         for i, run in enumerate(self.spec.order):

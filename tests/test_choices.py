@@ -171,13 +171,25 @@ def test_chains_take_the_parts_whose_arithmetic_they_have(ops):
         assert chain._sizes(b) is None
     assert chain._sizes(_block(ops, **exact)) is None      # no position encoding
 
-    def model(runs=2, opens=None, dtype=torch.bfloat16, entry=None):
+    def of(n=8, runs=2, opens=None, dtype=torch.bfloat16, entry=None, keys=64, store=True, page=16, transposed=True, **attention):
         b = _block(ops, **exact)
-        b.mixer.position = RotaryHalf("", 32, 32, 1e4)
-        return SimpleNamespace(spec=SimpleNamespace(order=[SimpleNamespace(layer=0, opens_pass=opens)] * runs), layers=[b],
-                               rt=SimpleNamespace(dtype=dtype, device="cpu"), pass_entry=entry)
+        b.mixer = GQAttention("", RotaryHalf("", 64, 64, 1e4), 64, 2, 1, 64, 0.1, **attention)
+        b.load = None
+        for part, names in ((b.mixer, ("w_o", "w_qkv", "b_qkv", "sink_w")), (b.feed_forward, ("w_gate_up", "w_down")),
+                            (b.mixer_norm, ("weight",)), (b.feed_forward_norm, ("weight",)), (b.mixer.position, ("inv_freq",))):
+            for name in names:
+                setattr(part, name, torch.zeros(1))
+        b.mixer.sink_w = torch.zeros(1) if b.mixer.sink else None
+        m = SimpleNamespace(spec=SimpleNamespace(order=[SimpleNamespace(layer=0, opens_pass=opens)] * runs), layers=[b],
+                            rt=SimpleNamespace(dtype=dtype, device="cpu"), pass_entry=entry)
+        table, slots, pages = torch.zeros(1), torch.zeros(1), torch.zeros(1, 1, page, 64, dtype=torch.bfloat16)
+        caches = [SimpleNamespace(kv=SimpleNamespace(k_pages=pages.clone(), v_pages=pages.clone(), block_table=table, slot_mapping=slots,
+                                                     v_transposed=transposed, window=b.mixer.window, stride=1, store=store))
+                  for _ in range(runs)]
+        made = chain.DecodeChain.of(m, SimpleNamespace(num_tokens=n, num_requests=n, max_context_len=keys), caches)
+        assert made is None or made.takes(caches) and not made.workspace.any()
+        return None if made is None else "layers" if made.table is None else "step"
 
-    made = chain.DecodeChain.of(model(), 8)
-    assert made.launches == 2 and not made.workspace.any()
-    assert chain.DecodeChain.of(model(), 9) is chain.DecodeChain.of(model(runs=1), 1) is chain.DecodeChain.of(model(opens=0), 1) is None
-    assert chain.DecodeChain.of(model(dtype=torch.float32), 1) is chain.DecodeChain.of(model(entry=b""), 1) is None
+    assert of() == of(keys=1024) == of(page=32) == "step"
+    assert of(keys=1025) == of(window=8) == of(sink=True) == of(softcap=9.0) == of(page=48) == of(transposed=False) == of(out_scale=2.0) == "layers"
+    assert of(9) is of(runs=1) is of(opens=0) is of(dtype=torch.float32) is of(entry=b"") is of(store=False) is None

@@ -1970,7 +1970,7 @@ def test_decode_chain(ops, M, H, I, nh, nkv, d, v_transposed, limit):
                 untouched[slots[slots >= 0].long().cpu()] = False
                 assert (kp.permute(0, 2, 1, 3).reshape(pages * page_size, -1)[untouched.to(DEV)] == 0).all()
                 kept += [q, kp, vp]
-            assert not ws[:4 * 1152].any()      # nothing is left on the list
+            assert not ws[:4 * 32768].any()      # nothing is left on the list
         finally:
             ops.decode_chain_limit(0)
         return kept
@@ -1980,8 +1980,108 @@ def test_decode_chain(ops, M, H, I, nh, nkv, d, v_transposed, limit):
         assert all(torch.equal(a, b) for a, b in zip(got, run(0)))
 
 
+@pytest.mark.parametrize("limit", [0, 1])
+@pytest.mark.parametrize("contexts", [(1,), (1024,), (17, 600), (32, 33, 2), (513, 64, 1, 1000), (1, 97, 128, 577, 31)])
+@pytest.mark.parametrize("H,I,nh,nkv,page_size", [(896, 4864, 14, 2, 16), (96, 64, 16, 1, 64)])
+def test_decode_layers(ops, H, I, nh, nkv, page_size, contexts, limit):
+    """Three steps of three layers in two launches each against double on what lies in the pages: contexts of one key, of whole
+    and of part blocks of 32, of all 1,024; a token that is not stored; pages in no order, with NaN behind the last key.  With
+    a limit of one look every waiting block gives its item up, to the same bits."""
+    M, d, L, eps, scale, n = len(contexts), 64, 3, 1e-6, 0.125, nh + 2 * nkv
+    width = -(-1030 // page_size)
+
+    def run(limit):
+        g = torch.Generator().manual_seed(M + H)
+        rand = lambda *shape, std=1.0: (torch.randn(*shape, generator=g) * std)     # noqa: E731
+        pages = M * width + 1
+        table = (torch.randperm(M * width, generator=g) + 1).view(M, width).to(torch.int32)
+        rows = torch.randperm(M, generator=g).to(torch.int32)
+        inv_freq = (1.0 / (1e6 ** (torch.arange(0, d, 2, dtype=torch.float64) / d))).float().to(DEV)
+        layers = []
+        for _ in range(L):
+            l = dict(w_o=rand(H, nh * d, std=(nh * d) ** -0.5), w_gate_up=rand(2 * I, H, std=H ** -0.5), w_down=rand(H, I, std=I ** -0.5),
+                     w_qkv=rand(n * d, H, std=H ** -0.5))
+            l = {k: v.bfloat16().to(DEV) for k, v in l.items()}
+            l.update(norm1=(1 + rand(H, std=0.1)).to(DEV), norm2=(1 + rand(H, std=0.1)).to(DEV), bias=rand(n * d).to(DEV),
+                     k=torch.full((pages, nkv, page_size, d), float("nan"), dtype=torch.bfloat16, device=DEV),
+                     v=torch.full((pages, nkv, d, page_size), float("nan"), dtype=torch.bfloat16, device=DEV))
+            for m, c in enumerate(contexts):
+                for t in range(0, c - 1, page_size):
+                    p, w = int(table[rows[m], t // page_size]), min(page_size, c - 1 - t)
+                    l["k"][p, :, :w], l["v"][p, :, :, :w] = rand(nkv, w, d).bfloat16().to(DEV), rand(nkv, d, w).bfloat16().to(DEV)
+            layers.append(l)
+        recs = []
+        for i, l in enumerate(layers):
+            rec = dict(w_o=l["w_o"], w_gate_up=l["w_gate_up"], w_down=l["w_down"], norm2=l["norm2"], eps2=eps, k_pages=l["k"], v_pages=l["v"])
+            if i + 1 < L:
+                t = layers[i + 1]
+                rec.update(w_front=t["w_qkv"], norm1=t["norm1"], eps1=eps, b_front=t["bias"], inv_freq=inv_freq, front_k=t["k"], front_v=t["v"])
+            recs.append(rec)
+        records = ops.decode_layer_table(recs, DEV)
+        ws = torch.zeros(ops.decode_chain_workspace(M, H, nh, nkv, d, I, L), dtype=torch.uint8, device=DEV)
+        kept = []
+        ops.decode_chain_limit(limit)
+        try:
+            for step in range(3):
+                lens = [min(c + step, 1024) for c in contexts]
+                pos = torch.tensor([c - 1 for c in lens], dtype=torch.int32)
+                slot = torch.tensor([int(table[rows[m], (c - 1) // page_size]) * page_size + (c - 1) % page_size for m, c in enumerate(lens)])
+                if M > 2 and step == 2:
+                    slot[2] = -1
+                x = rand(M, H).to(DEV)
+                x0 = x.double()
+                before = [(l["k"].clone(), l["v"].clone()) for l in layers]
+                pos_d, slot_d = pos.to(DEV), slot.to(torch.int32).to(DEV)
+                a = layers[0]
+                ops.decode_first(x, a["norm1"], eps, a["w_qkv"], a["bias"], pos_d, inv_freq, slot_d, a["k"], a["v"], nh, nkv, d, I, L, ws)
+                ops.decode_layers(records, x, pos_d, slot_d, (pos + 1).to(DEV), table.to(DEV), rows.to(DEV), scale, nh, nkv, d, I,
+                                  page_size, L, ws)
+                y = x0
+                for l, (bk, bv) in zip(layers, before):
+                    z = ((y * l["norm1"].double()) / torch.sqrt((y * y).mean(1, keepdim=True) + eps)) @ l["w_qkv"].double().T + l["bias"].double()
+                    z = z.view(M, n, d).cpu()
+                    rot = rope_reference(z[:, :nh + nkv], pos, d, inv_freq.double().cpu())
+                    heads = torch.empty(M, nh * d, dtype=torch.float64)
+                    for m, c in enumerate(lens):
+                        at = [(int(table[rows[m], t // page_size]), t % page_size) for t in range(c - 1)]
+                        p, o = [q[0] for q in at], [q[1] for q in at]
+                        new_k, new_v = rot[m, nh:], z[m, nh + nkv:]
+                        if int(slot[m]) >= 0:      # what was stored is what it should be, and counts as it was rounded
+                            sp, so = divmod(int(slot[m]), page_size)
+                            torch.testing.assert_close(l["k"][sp, :, so].double().cpu(), new_k, atol=6e-2, rtol=2e-2)
+                            torch.testing.assert_close(l["v"][sp, :, :, so].double().cpu(), new_v, atol=6e-2, rtol=2e-2)
+                            new_k, new_v = l["k"][sp, :, so].double().cpu(), l["v"][sp, :, :, so].double().cpu()
+                        keys = torch.cat([bk[p, :, o].double().cpu(), new_k[None]]).repeat_interleave(nh // nkv, 1)     # [c, nh, d]
+                        vals = torch.cat([bv[p, :, :, o].double().cpu(), new_v[None]]).repeat_interleave(nh // nkv, 1)
+                        w = (scale * torch.einsum("hd,chd->hc", rot[m, :nh], keys)).softmax(1)
+                        heads[m] = torch.einsum("hc,chd->hd", w, vals).reshape(-1)
+                    y, _ = _chain_reference(heads.to(DEV), l["w_o"], y, l["norm2"], l["w_gate_up"], l["w_down"], eps)
+                # queries, heads, probabilities and the middle are rounded to bfloat16 (2^-9 each) three layers deep
+                assert (x.double() - y).norm() < 1.2e-2 * (y - x0).norm()
+                for l, (bk, bv) in zip(layers, before):      # nothing else was written
+                    for now, was in ((l["k"].permute(0, 2, 1, 3), bk.permute(0, 2, 1, 3)), (l["v"].permute(0, 3, 1, 2), bv.permute(0, 3, 1, 2))):
+                        rest = torch.ones(pages * page_size, dtype=torch.bool)
+                        rest[slot[slot >= 0]] = False
+                        rest = rest.to(DEV)
+                        assert torch.equal(now.reshape(pages * page_size, -1)[rest].view(torch.int16), was.reshape(pages * page_size, -1)[rest].view(torch.int16))
+                kept += [x.clone()] + [l["k"].clone() for l in layers]
+            assert not ws[:4 * 32768].any()
+        finally:
+            ops.decode_chain_limit(0)
+        return kept
+
+    got = run(limit)
+    if limit:
+        assert all(torch.equal(a.view(torch.int16 if a.dtype == torch.bfloat16 else torch.int32), b.view(torch.int16 if b.dtype == torch.bfloat16 else torch.int32))
+                   for a, b in zip(got, run(0)))
+
+
 def test_decode_chain_refuses_what_it_cannot_take(ops):
     for sizes in [(9, 896, 14, 2, 64, 4864), (0, 896, 14, 2, 64, 4864), (1, 1056, 14, 2, 64, 4864), (1, 896, 17, 1, 64, 4864),
                   (1, 896, 14, 2, 64, 6176), (1, 896, 14, 2, 64, 4880), (1, 880, 14, 2, 64, 4864), (1, 896, 14, 2, 60, 4864)]:
         assert ops.decode_chain_workspace(*sizes) == 0
     assert ops.decode_chain_workspace(8, 896, 14, 2, 64, 4864) > 0
+    for sizes in [(1, 896, 7, 2, 64, 4864, 24), (1, 896, 7, 1, 128, 4864, 24), (1, 1024, 16, 0, 64, 4864, 24), (1, 1024, 32, 1, 32, 64, 2),
+                  (1, 896, 14, 2, 64, 4864, 60)]:
+        assert ops.decode_chain_workspace(*sizes) == 0
+    assert ops.decode_chain_workspace(8, 896, 14, 2, 64, 4864, 24) > 0
