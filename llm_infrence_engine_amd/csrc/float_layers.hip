@@ -1,0 +1,60 @@
+// All layers of a 32-bit step by one call: the same nine kernels a layer as when every one is asked for by itself, from the host
+// side of the library.  A decode step of the 32-bit path is as slow as its launches are made: 219 of them took 2.62 ms from
+// Python (12 us each, of which the launch itself is 4) where the GPU has 1.7 ms of work.
+#include "common.h"
+#include "api.h"
+
+namespace {
+
+// Device addresses of one layer's weights and pages; in host memory.
+struct FloatLayer {
+  const float *norm1, *w_qkv, *b_qkv, *inv_freq, *w_o, *norm2, *w_gate_up, *w_down;
+  float *k_pages, *v_pages;
+  float eps1, eps2;
+};
+
+}  // namespace
+
+extern "C" int ms_float_layer_bytes() { return (int)sizeof(FloatLayer); }
+
+// Floats of `work` for n_tokens tokens.
+extern "C" long long ms_float_layers_work(int n_tokens, int H, int num_heads, int num_kv_heads, int head_dim, int I) {
+  return (long long)n_tokens * (2ll * H + (2ll * num_heads + 2ll * num_kv_heads) * head_dim + 3ll * I);
+}
+
+// x float [N, H] in place, but for the last down projection, which is left in work's first [N, H] for whoever adds it.  w_gate_up's
+// rows interleaved, heads turned whole, pages as ms_rope_store has them; n_live may be null.
+extern "C" int ms_float_layers(const void* layers, int n_layers, float* x, float* work, const int* positions, const int* token_req,
+                               const int* slot_mapping, const int* block_table, int table_width, const int* table_rows,
+                               const int* n_live, int n_tokens, int H, int I, int num_heads, int num_kv_heads, int head_dim,
+                               int page_size, long long num_pages, int v_transposed, float scale, hipStream_t stream) {
+  if (n_tokens <= 0) return MS_OK;
+  if (!layers || n_layers < 1 || !x || !work || !positions || !token_req || !slot_mapping || !block_table || H <= 0 || I <= 0 ||
+      num_heads <= 0 || num_kv_heads <= 0 || head_dim <= 0 || page_size <= 0)
+    return MS_BAD_ARG;
+  const long long N = n_tokens;
+  const int Ko = num_heads * head_dim, Q = (num_heads + 2 * num_kv_heads) * head_dim;
+  float *sum = work, *h = sum + N * H, *qkv = h + N * H, *heads = qkv + N * Q, *gate_up = heads + N * Ko, *act = gate_up + N * 2 * I;
+  auto product = [&](const float* a, const float* w, const float* bias, float* out, int n, int k) {
+    return ms_gemm_generic(a, w, bias, out, n_tokens, n, k, k, k, n, MS_F32, MS_F32, 0, stream);
+  };
+  for (int i = 0; i < n_layers; ++i) {
+    const FloatLayer& l = static_cast<const FloatLayer*>(layers)[i];
+    int rc = ms_rms_norm(x, i ? sum : nullptr, MS_F32, 1, N * H, l.norm1, nullptr, h, n_tokens, H, l.eps1, 1, MS_F32, stream);
+    if (rc == MS_OK) rc = product(h, l.w_qkv, l.b_qkv, qkv, Q, H);
+    if (rc == MS_OK)
+      rc = ms_rope_store(qkv, nullptr, positions, l.inv_freq, slot_mapping, l.k_pages, l.v_pages, n_tokens, num_heads, num_kv_heads,
+                         head_dim, head_dim, page_size, v_transposed, MS_F32, stream);
+    if (rc == MS_OK)
+      rc = ms_paged_attention_generic(qkv, Q, l.k_pages, l.v_pages, block_table, table_width, table_rows, n_live, token_req, positions,
+                                      heads, Ko, n_tokens, num_heads, num_kv_heads, head_dim, head_dim, page_size, num_pages, scale, 0,
+                                      v_transposed, nullptr, 0.f, nullptr, nullptr, 0, 1, 1.f, MS_F32, stream);
+    if (rc == MS_OK) rc = product(heads, l.w_o, nullptr, sum, H, Ko);
+    if (rc == MS_OK) rc = ms_rms_norm(x, sum, MS_F32, 1, N * H, l.norm2, nullptr, h, n_tokens, H, l.eps2, 1, MS_F32, stream);
+    if (rc == MS_OK) rc = product(h, l.w_gate_up, nullptr, gate_up, 2 * I, H);
+    if (rc == MS_OK) rc = ms_silu_mul(gate_up, act, n_tokens, I, MS_F32, stream);
+    if (rc == MS_OK) rc = product(act, l.w_down, nullptr, sum, H, I);
+    if (rc != MS_OK) return rc;
+  }
+  return MS_OK;
+}

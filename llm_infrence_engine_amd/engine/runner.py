@@ -14,7 +14,7 @@ import torch
 
 from ..cache import CacheLayout, CacheManager, CachePools
 from ..kernels import ops
-from ..parts.chain import DecodeChain
+from ..parts.chain import DecodeChain, FloatLayers
 from ..parts.model import Model, RunCache
 from .batch import BatchBuilder, StepEntry
 
@@ -40,7 +40,9 @@ class ModelRunner:
         self.pools = CachePools(self.layout, page_size, num_pages, max_requests, self.rt,
                                 self.manager.max_pages_per_request)
         self.builder = BatchBuilder(self.manager, self.pools, model.spec.vocab_size, self.rt.device)
-        self.chains = {}         # for steps of single tokens launched kernel by kernel: (tokens, long contexts) -> DecodeChain, or None
+        # for steps launched kernel by kernel: (tokens, long contexts) -> DecodeChain of steps of single tokens, "float" -> FloatLayers;
+        # None where there is none
+        self.chains = {}
         self.graphs = None
         # a part that cannot be captured (it walks the requests on the host, as a mixer with state usually does)
         # keeps the whole model out of graphs
@@ -101,6 +103,10 @@ class ModelRunner:
                 if key not in self.chains:
                     self.chains[key] = DecodeChain.of(self.model, built.ctx, caches)
                 built.ctx.chain = self.chains[key]
+            if built.ctx.chain is None:
+                if "float" not in self.chains:
+                    self.chains["float"] = FloatLayers.of(self.model, caches)
+                built.ctx.chain = self.chains["float"]
             logits = self.model.forward(built.ctx, caches)
         for e in entries:
             m.advance(e.req_id, m.computed(e.req_id) + len(e.tokens))

@@ -31,6 +31,9 @@ _SIGNATURES = {
                           _c_int, _c_int, _c_int, _c_int, _c_int, _c_int, _c_int, _c_ptr],
     "ms_decode_advance": [_c_ptr, _c_ptr, _c_ptr, _c_ptr, _c_ptr, _c_ptr, _c_ptr, _c_ptr, _c_ptr, _c_ptr, _c_int, _c_int, _c_int,
                           _c_int, _c_ptr],
+    "ms_float_layer_bytes": [],
+    "ms_float_layers": [_c_ptr, _c_int, _c_ptr, _c_ptr, _c_ptr, _c_ptr, _c_ptr, _c_ptr, _c_int, _c_ptr, _c_ptr, _c_int, _c_int, _c_int,
+                        _c_int, _c_int, _c_int, _c_int, _c_ll, _c_int, _c_float, _c_ptr],
     "ms_decode_chain_workspace": [_c_int] * 7,
     "ms_decode_layer_bytes": [],
     "ms_decode_first": [_c_ptr, _c_ll, _c_ptr, _c_float, _c_ptr, _c_ptr, _c_ptr, _c_ptr, _c_ptr, _c_ptr, _c_ptr, _c_int, _c_int,
@@ -1051,6 +1054,47 @@ def decode_chain(attn: torch.Tensor, w_o: torch.Tensor, x: torch.Tensor, norm2: 
           w_gate_up.data_ptr(), w_down.data_ptr(), *tail, M, H, I, num_heads, num_kv_heads, head_dim, page_size,
           int(v_transposed), workspace.data_ptr(), launch, launches, _stream())
     return q
+
+
+def float_layer_records(layers, num_heads: int, num_kv_heads: int, head_dim: int) -> bytes:
+    """What ``float_layers`` reads of its layers: for each a dict of its float tensors norm1, w_qkv, b_qkv (may be None), inv_freq,
+    w_o, norm2, w_gate_up (rows interleaved), w_down, k_pages and v_pages, and of eps1 and eps2.  The tensors have to outlive the
+    records."""
+    names = ("norm1", "w_qkv", "b_qkv", "inv_freq", "w_o", "norm2", "w_gate_up", "w_down", "k_pages", "v_pages")
+    out = []
+    for l in layers:
+        H, I = l["w_down"].shape
+        width = (num_heads + 2 * num_kv_heads) * head_dim
+        for name, shape in (("norm1", (H,)), ("w_qkv", (width, H)), ("b_qkv", (width,)), ("inv_freq", (head_dim // 2,)),
+                            ("w_o", (H, num_heads * head_dim)), ("norm2", (H,)), ("w_gate_up", (2 * I, H)), ("w_down", (H, I)),
+                            ("k_pages", (None, num_kv_heads, None, head_dim)), ("v_pages", (None, num_kv_heads, None, None))):
+            if name != "b_qkv" or l[name] is not None:
+                _check(l[name], name, torch.float32, shape)
+        out.append(struct.pack("<10Q2f", *(_ptr(l[n]) or 0 for n in names), l["eps1"], l["eps2"]))
+    if len(out[0]) != _get("ms_float_layer_bytes")():
+        raise build.KernelLibraryError("the library's record of a layer has another size than this module's")
+    return b"".join(out)
+
+
+def float_layers(records: bytes, n_layers: int, x: torch.Tensor, positions: torch.Tensor, token_req: torch.Tensor,
+                 slot_mapping: torch.Tensor, block_table: torch.Tensor, table_rows: Optional[torch.Tensor],
+                 n_live_tokens: Optional[torch.Tensor], k_pages: torch.Tensor, v_transposed: bool, num_heads: int, num_kv_heads: int,
+                 intermediate: int, scale: float) -> torch.Tensor:
+    """All layers of a 32-bit step: x float [N, H] in place but for the last down projection, which is returned [N, H]."""
+    _check(x, "x", torch.float32)
+    N, H = x.shape
+    for name, t in (("positions", positions), ("token_req", token_req), ("slot_mapping", slot_mapping)):
+        _check(t, name, torch.int32, (N,))
+    _check(block_table, "block_table", torch.int32, (None, None))
+    for name, t in (("table_rows", table_rows), ("n_live_tokens", n_live_tokens)):
+        if t is not None:
+            _check(t, name, torch.int32)
+    P, _, page_size, d = k_pages.shape
+    work = torch.empty(N * (2 * H + (2 * num_heads + 2 * num_kv_heads) * d + 3 * intermediate), dtype=torch.float32, device=x.device)
+    _call("ms_float_layers", records, n_layers, x.data_ptr(), work.data_ptr(), positions.data_ptr(), token_req.data_ptr(),
+          slot_mapping.data_ptr(), block_table.data_ptr(), block_table.shape[1], _ptr(table_rows), _ptr(n_live_tokens), N, H,
+          intermediate, num_heads, num_kv_heads, d, page_size, P, int(v_transposed), float(scale), _stream())
+    return work[:N * H].view(N, H)
 
 
 def _gate_of(gate: Optional[torch.Tensor], q: torch.Tensor, num_heads: int, dv: int):

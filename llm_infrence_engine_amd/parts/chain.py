@@ -43,6 +43,61 @@ def _plain_attention(m) -> bool:
     return m.window is None and m.sink_w is None and not m.softcap and m.slopes is None and m.out_scale == 1.0
 
 
+def _own_pages(caches, dtype) -> bool:
+    """Whether every run stores its keys and values in pages of its own, of ``dtype``."""
+    return all(c.kv is not None and c.kv.store and c.kv.k_pages.dtype == dtype for c in caches)
+
+
+def _plain_layers(model, caches) -> bool:
+    """Whether all runs have plain attention of one scale over one group's pages."""
+    kv = caches[0].kv
+    mixers = [model.layers[run.layer].mixer for run in model.spec.order]
+    return (all(_plain_attention(m) and m.scale == mixers[0].scale for m in mixers)
+            and all(c.kv.block_table is kv.block_table and c.kv.slot_mapping is kv.slot_mapping and c.kv.window is None
+                    and c.kv.v_transposed == kv.v_transposed and c.kv.stride == 1 for c in caches))
+
+
+def _same_pages(pages, caches) -> bool:
+    return all(a.data_ptr() == b.data_ptr() for a, b in zip(pages, (t for c in caches for t in (c.kv.k_pages, c.kv.v_pages))))
+
+
+class FloatLayers:
+    """The layers of a step in float32, launched kernel by kernel, by one call (``ops.float_layers``): the kernels that the parts
+    would launch one by one, in their order."""
+
+    def __init__(self, model, sizes: tuple, caches):
+        self.sizes, self.layers = sizes, [model.layers[run.layer] for run in model.spec.order]
+        self.pages = [t for c in caches for t in (c.kv.k_pages, c.kv.v_pages)]
+        nh, nkv, d, _, _ = sizes
+        self.records = ops.float_layer_records(
+            [dict(norm1=l.mixer_norm.weight, eps1=l.mixer_norm.eps, w_qkv=l.mixer.w_qkv, b_qkv=l.mixer.b_qkv,
+                  inv_freq=l.mixer.position.inv_freq, w_o=l.mixer.w_o, norm2=l.feed_forward_norm.weight, eps2=l.feed_forward_norm.eps,
+                  w_gate_up=l.feed_forward.w_gate_up, w_down=l.feed_forward.w_down, k_pages=c.kv.k_pages, v_pages=c.kv.v_pages)
+             for l, c in zip(self.layers, caches)], nh, nkv, d)
+
+    @classmethod
+    def of(cls, model, caches) -> Optional["FloatLayers"]:
+        """None where a layer is not of the parts whose kernels these are."""
+        runs = model.spec.order
+        if model.rt.dtype != torch.float32 or model.pass_entry is not None or any(run.opens_pass is not None for run in runs):
+            return None
+        sizes = {_sizes(model.layers[run.layer]) for run in runs}
+        if len(sizes) != 1 or None in sizes or not _own_pages(caches, torch.float32) or not _plain_layers(model, caches):
+            return None
+        return cls(model, sizes.pop(), caches)
+
+    def takes(self, caches) -> bool:
+        """Whether these are the caches that the records were made of."""
+        return (len(caches) == len(self.layers) and _own_pages(caches, torch.float32) and _same_pages(self.pages, caches)
+                and all(c.kv.slot_mapping is caches[0].kv.slot_mapping for c in caches))
+
+    def forward(self, x, ctx, caches):
+        nh, nkv, _, _, I = self.sizes
+        kv = caches[0].kv
+        return x, ops.float_layers(self.records, len(self.layers), x, ctx.positions, ctx.token_req, kv.slot_mapping, kv.block_table,
+                                   kv.table_rows, ctx.n_live_tokens, kv.k_pages, kv.v_transposed, nh, nkv, I, self.layers[0].mixer.scale)
+
+
 class DecodeChain:
     """The chains of one batch size, with their workspace; ``table``: what ``ops.decode_layers`` reads, where the step's layers
     go in two launches, else None."""
@@ -77,21 +132,15 @@ class DecodeChain:
         n_bytes = ops.decode_chain_workspace(n, H, nh, nkv, d, I)
         return cls(model, sizes, n_bytes) if n_bytes else None
 
-    @staticmethod
-    def _stores(caches) -> bool:
-        """Whether every run stores its keys and values in bfloat16 pages of its own."""
-        return all(c.kv is not None and c.kv.store and c.kv.k_pages.dtype == torch.bfloat16 for c in caches)
+    @classmethod
+    def _stores(cls, caches) -> bool:
+        return _own_pages(caches, torch.bfloat16)
 
     @staticmethod
     def _one_group(model, caches) -> bool:
-        """Whether all runs have plain attention of one scale over one group's pages, laid out as the kernel reads them."""
-        kv = caches[0].kv
-        mixers = [model.layers[run.layer].mixer for run in model.spec.order]
-        page_size = kv.k_pages.shape[2]
-        return (all(_plain_attention(m) and m.scale == mixers[0].scale for m in mixers) and page_size >= 16
-                and page_size & (page_size - 1) == 0
-                and all(c.kv.block_table is kv.block_table and c.kv.slot_mapping is kv.slot_mapping and c.kv.v_transposed
-                        and c.kv.window is None and c.kv.stride == 1 for c in caches))
+        """Whether the pages are laid out as the kernel reads them, beside ``_plain_layers``."""
+        page_size = caches[0].kv.k_pages.shape[2]
+        return _plain_layers(model, caches) and caches[0].kv.v_transposed and page_size >= 16 and page_size & (page_size - 1) == 0
 
     def _lay_out(self, caches):
         rows = []
@@ -111,17 +160,16 @@ class DecodeChain:
         """Whether these are the caches that the chain was made for (or, where it reads no table of them, any like them)."""
         if len(caches) != self.runs or not self._stores(caches):
             return False
-        return self.table is None or all(a.data_ptr() == b.data_ptr() for a, b in
-                                         zip(self.pages, (t for c in caches for t in (c.kv.k_pages, c.kv.v_pages))))
+        return self.table is None or _same_pages(self.pages, caches)
 
     def forward(self, x, ctx, caches):
-        """All runs of the order on the embedded tokens ``x`` [N, H], in place; returns x."""
+        """All runs of the order on the embedded tokens ``x`` [N, H], in place; returns x and what is left to add to it (nothing)."""
         if self.broken_off:          # its launches did not count each other up: start over
             self.workspace.zero_()
         self.broken_off = True
         (self._layer_by_layer if self.table is None else self._whole)(x, ctx, caches)
         self.broken_off = False
-        return x
+        return x, None
 
     def _whole(self, x, ctx, caches):
         nh, nkv, d, _, I = self.sizes

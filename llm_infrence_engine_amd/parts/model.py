@@ -96,7 +96,8 @@ class Model:
         itself, or None)."""
         x = self.embedding.forward(ctx)
         if ctx.chain is not None and ctx.chain.takes(caches):
-            return ctx.chain.forward(x, ctx, caches), None
+            x, pending = ctx.chain.forward(x, ctx, caches)
+            return x, self._settled(x, pending, self.final_norm)
         kept = x.clone() if self.pass_entry is not None and self.pass_entry.keeps_embedding else None
         pending = None
         for i, run in enumerate(self.spec.order):

@@ -193,3 +193,45 @@ def test_chains_take_the_parts_whose_arithmetic_they_have(ops):
     assert of() == of(keys=1024) == of(page=32) == "step"
     assert of(keys=1025) == of(window=8) == of(sink=True) == of(softcap=9.0) == of(page=48) == of(transposed=False) == of(out_scale=2.0) == "layers"
     assert of(9) is of(runs=1) is of(opens=0) is of(dtype=torch.float32) is of(entry=b"") is of(store=False) is None
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("tokens", [[1, 1, 1], [1, 40, 3]])
+def test_float_layers_are_the_parts_one_by_one(ops, tokens):
+    """Two layers of a 32-bit step by one call and part by part: the same kernels, so the same bits, in x, in what is left to
+    add and in the pages; decoding and portions, a request further on, pages plain."""
+    from llm_infrence_engine_amd.engine.batch import StepEntry
+    from llm_infrence_engine_amd.config import config_from_dict
+    from llm_infrence_engine_amd.engine import ModelRunner
+    from llm_infrence_engine_amd.parts import chain
+    from llm_infrence_engine_amd.parts.base import Runtime
+    from llm_infrence_engine_amd.parts.model import Model
+
+    cfg = config_from_dict({"model_type": "qwen2", "hidden_size": 96, "intermediate_size": 160, "num_hidden_layers": 2,
+                            "num_attention_heads": 6, "num_key_value_heads": 2, "vocab_size": 64, "rms_norm_eps": 1e-6,
+                            "rope_theta": 10000.0, "tie_word_embeddings": True, "max_position_embeddings": 128})
+    g = torch.Generator().manual_seed(3)
+
+    class Weights:
+        def check(self, wanted, ignorable=()):
+            self.shapes = {s.name: s.shape for s in wanted}
+
+        def get(self, name):
+            return torch.randn(self.shapes[name], generator=g).cuda() / 8
+
+        def close(self):
+            pass
+
+    model = Model(cfg.to_spec())
+    model.config = cfg
+    model.load(Weights(), Runtime(torch.device("cuda:0"), torch.float32))
+    got = []
+    for whole in (True, False):
+        r = ModelRunner(model, 16, 24, 4, 96)
+        if not whole:
+            r.chains["float"] = None
+        r.step([StepEntry(0, list(range(20)), [19])])
+        out = [r.step([StepEntry(i, [7 + i] * n, [n - 1]) for i, n in enumerate(tokens)]).cpu() for _ in range(2)]
+        assert isinstance(r.chains["float"], chain.FloatLayers) == whole
+        got.append(out + [t.cpu() for pages in r.pools.pages for t in pages.values()])
+    assert all(torch.equal(a, b) for a, b in zip(*got))
