@@ -6,15 +6,18 @@
 // slices are added in order.  Two kernels keep that order:
 //   rows     up to 64 rows (a decode step; against very many rows of W up to 16): all waves of a block on the same 4 to 16
 //            rows of W, the slices dealt out over them and added through LDS.  Bound by reading W.
+//   few      up to 8 rows, of these: loads that take four steps at a time.
 //   tiled    the others: 64 x 64 or 32 x 32 tiles staged through LDS four steps ahead, 4 waves; 32 x 32 where the larger
 //            tiles would be fewer than two a CU.  Bound by the float matrix rate (157 TFLOP/s nominal), short K by writing C.
 // Measured with the 0.5B sizes against the 64 x 64 vector-ALU tile that ran them before (one MI355X): of 3 rows the down
-// product (896 x 4,864) 319 -> 17 us, gate/up (9,728 x 896) 63 -> 12 us, q/k/v (1,152 x 896) 63 -> 6.3 us, the head
+// product (896 x 4,864) 319 -> 16 us (12 with grouped loads), gate/up (9,728 x 896) 63 -> 12 us, q/k/v (1,152 x 896) 63 -> 4.5 us, the head
 // (151,936 x 896) 221 -> 100 us, of 64 rows 252 -> 220; of 338 rows down 316 -> 84 us, gate/up 108 -> 88 us.  Down is bound
 // by the steps a CU works off (16 waves, 19 steps each), whatever its rows; the tiled steps by the way from one barrier to
 // the next.  C leaves a tile through LDS in whole rows (4,096 x 32,000 x 64: 440 us as the fragments lie, 270 so, 261 before).
 #include "common.h"
 #include "api.h"
+#include "quads.h"
+#include <type_traits>
 
 namespace {
 
@@ -106,6 +109,91 @@ gemm_f32_rows_kernel(const float* __restrict__ A, const float* __restrict__ W, c
     if (m >= M || n >= N) continue;
     float v = part[at];
     for (int s = 1; s < slices; ++s) v += part[s * PART + at];
+    store(C, (size_t)m * ldc + n, v, bias, n, accumulate);
+  }
+}
+
+// Up to G = 4 or 8 tokens: the same products in the same order, with fewer loads.  A block of the kernel above spends its time on
+// issuing loads (some 70 cycles of its CU each, 38 of them to a wave for 19 steps), and most lanes of these repeat others: 4 rows
+// of W and 3 of A fill a quarter of the lanes.  Here one load takes FOUR steps of four rows (of eight rows two steps, of 16 one;
+// lane 16 g + X i + r: row r, step i, piece g), and the operand of a step is that register turned by X i lanes within the
+// rows of 16; the instruction's other rows and columns hold other steps' values, whose products nobody reads.
+template <int X>
+struct StepRows {
+  static constexpr int LOADS = X / 4, STEPS = 16 / X;      // loads to four steps, steps to a load
+  f32x4 v[LOADS];
+  __device__ __forceinline__ void fetch(const float* row, int step, int last, int lane, int K) {
+#pragma unroll
+    for (int j = 0; j < LOADS; ++j) {
+      const int k = min(step + j * STEPS + (lane & 15) / X, last) * STEP + 4 * (lane >> 4);
+      v[j] = load4(row, k, K);
+      if (k >= K) v[j] = f32x4{0.f, 0.f, 0.f, 0.f};
+    }
+  }
+  template <int I> __device__ __forceinline__ f32x4 at() const {
+    return __builtin_bit_cast(f32x4, quad_turn<(I % STEPS) * X>(__builtin_bit_cast(quad_u32, v[I / STEPS])));
+  }
+};
+
+template <int R, int G>
+__global__ void __launch_bounds__(MAX_SLICES * MS_WAVE)
+gemm_f32_few_kernel(const float* __restrict__ A, const float* __restrict__ W, const float* __restrict__ bias,
+                    float* C, int M, int N, int K, size_t lda, size_t ldw, size_t ldc, int accumulate) {
+  extern __shared__ __align__(16) float part[];      // [slice][token][row of W]
+  constexpr int PART = G * R, AHEAD = 2;             // groups of four steps asked for before they are used
+  const int lane = threadIdx.x & (MS_WAVE - 1), wave = __builtin_amdgcn_readfirstlane(threadIdx.x / MS_WAVE);
+  const int waves = blockDim.x / MS_WAVE;
+  const int per = slice_steps(K), steps = (K + STEP - 1) / STEP, slices = (steps + per - 1) / per, groups = (per + 3) / 4;
+  const int n0 = blockIdx.x * R;
+  const float* wrow = W + (size_t)min(n0 + (lane & (R - 1)), N - 1) * ldw;
+  const float* arow = A + (size_t)min(lane & (G - 1), M - 1) * lda;
+  StepRows<R> w[AHEAD];
+  StepRows<G> a[AHEAD];
+  // the groups of the wave's slices in one row
+  const int mine = (slices - wave + waves - 1) / waves * groups;
+  int ahead = wave, ahead_at = 0;                    // slice and group of the next loads
+  auto fetch = [&](int u) {
+    const int step = ahead * per + 4 * ahead_at;
+    w[u].fetch(wrow, step, steps - 1, lane, K);
+    a[u].fetch(arow, step, steps - 1, lane, K);
+    if (++ahead_at == groups) { ahead_at = 0; ahead += waves; }
+  };
+#pragma unroll
+  for (int u = 0; u < AHEAD; ++u)
+    if (u < mine) fetch(u);
+  f32x4 acc = {0.f, 0.f, 0.f, 0.f};
+  int slice = wave, at = 0;
+  for (int s = 0; s < mine; s += AHEAD) {
+#pragma unroll
+    for (int u = 0; u < AHEAD; ++u) {
+      if (s + u >= mine) break;
+      const StepRows<R> wu = w[u];
+      const StepRows<G> au = a[u];
+      if (s + u + AHEAD < mine) fetch(u);
+      const int left = min(per, steps - slice * per) - 4 * at;      // steps of this group and the slice's later ones
+      auto step = [&](auto index) {
+        constexpr int I = decltype(index)::value;
+        if (I < left) acc = step16(wu.template at<I>(), au.template at<I>(), acc);
+      };
+      step(std::integral_constant<int, 0>{});
+      step(std::integral_constant<int, 1>{});
+      step(std::integral_constant<int, 2>{});
+      step(std::integral_constant<int, 3>{});
+      if (++at == groups) {
+        // lane 16 g + token holds W's rows 4 g .. + 3
+        if ((lane & 15) < G && (lane >> 4) * 4 < R) *reinterpret_cast<f32x4*>(&part[slice * PART + (lane & 15) * R + (lane >> 4) * 4]) = acc;
+        acc = f32x4{0.f, 0.f, 0.f, 0.f};
+        at = 0;
+        slice += waves;
+      }
+    }
+  }
+  __syncthreads();
+  for (int e = threadIdx.x; e < M * R; e += blockDim.x) {
+    const int m = e / R, n = n0 + e % R;
+    if (n >= N) continue;
+    float v = part[e];
+    for (int t = 1; t < slices; ++t) v += part[t * PART + e];
     store(C, (size_t)m * ldc + n, v, bias, n, accumulate);
   }
 }
@@ -244,10 +332,20 @@ int ms_gemm_f32_launch(const float* A, const float* W, const float* bias, float*
     dim3 grid((N + R - 1) / R), block(waves * MS_WAVE);
 #define ROWS2(R_, NT) gemm_f32_rows_kernel<R_, NT><<<grid, block, (size_t)slices * NT * 256 * sizeof(float), stream>>>(A, W, bias, C, M, N, K, lda, ldw, ldc, accumulate)
 #define ROWS(NT) do { if (R == 4) ROWS2(4, NT); else if (R == 8) ROWS2(8, NT); else ROWS2(16, NT); } while (0)
-    if (M <= 16) ROWS(1);
+    // Loads of four steps (up to 8 tokens): always where a block has 4 or 8 rows of W (3 tokens: 896 x 896 5.4 -> 4.3 us, 896 x 4,864
+    // 15.9 -> 11.8, 2,048 x 2,048 9.1 -> 7.7), with 16 rows, whose loads were full, from more than four steps to a slice on
+    // (6,144 x 1,536 16.4 -> 15.0, 64,000 x 1,536 99 -> 85; with four 9,728 x 896 11.8 and 12.4, x 1,024 12.9 and 13.7, others even).
+    const bool grouped = M <= 8 && (R < 16 || per > 4);
+#define FEW2(R_, G_) gemm_f32_few_kernel<R_, G_><<<grid, block, (size_t)slices * R_ * G_ * sizeof(float), stream>>>(A, W, bias, C, M, N, K, lda, ldw, ldc, accumulate)
+#define FEW(G_) do { if (R == 4) FEW2(4, G_); else if (R == 8) FEW2(8, G_); else FEW2(16, G_); } while (0)
+    if (grouped && M <= 4) FEW(4);
+    else if (grouped) FEW(8);
+    else if (M <= 16) ROWS(1);
     else if (M <= 32) ROWS(2);
     else ROWS(4);
 #undef ROWS2
+#undef FEW2
+#undef FEW
 #undef ROWS
     return ms_launch_status();
   }

@@ -2085,3 +2085,27 @@ def test_decode_chain_refuses_what_it_cannot_take(ops):
                   (1, 896, 14, 2, 64, 4864, 60)]:
         assert ops.decode_chain_workspace(*sizes) == 0
     assert ops.decode_chain_workspace(8, 896, 14, 2, 64, 4864, 24) > 0
+
+
+@pytest.mark.parametrize("M", [1, 3, 4, 5, 8])
+@pytest.mark.parametrize("N,K", [(7, 4), (10, 36), (896, 4864), (1024, 64), (1025, 1040), (2050, 1100), (5001, 1028), (4100, 9000)])
+def test_float_products_of_up_to_8_rows_are_those_of_more(ops, M, N, K):
+    """Loads that take four k-steps of 4, 8 and 16 rows of W and of up to 4 and 8 tokens: the same bits as the same rows among 16,
+    which go one step at a time; slices of one to 36 steps, a last one that is short, a last step that is, rows and columns of
+    zeros, infinities and NaN beside others, a bias and a sum in place."""
+    g = torch.Generator().manual_seed(N + K)
+    a, w = torch.randn(16, K, generator=g), torch.randn(N, K, generator=g)
+    a[min(2, M - 1)], w[N // 2] = 0.0, 0.0
+    if M > 3:
+        a[3, K // 2] = float("inf")
+        w[N - 1, K - 1] = float("nan")
+    a, w, bias = a.to(DEV), w.to(DEV), torch.randn(N, generator=g).to(DEV)
+    base = torch.randn(16, N, generator=g).to(DEV)
+    for accumulate in (False, True):
+        want = ops.gemm_generic(a, w, base.clone(), bias, accumulate)
+        got = ops.gemm_generic(a[:M], w, base[:M].clone(), bias, accumulate)
+        assert torch.equal(got.isnan(), want[:M].isnan()) and torch.equal(got.nan_to_num(7.0), want[:M].nan_to_num(7.0))
+    exact = a.double() @ w.double().T + bias.double()
+    ok = exact[:M].isfinite()
+    got = ops.gemm_generic(a[:M], w, torch.empty(M, N, device=DEV), bias)
+    assert ((got.double() - exact[:M])[ok].abs() <= 4e-6 * math.sqrt(K) * 4).all()
