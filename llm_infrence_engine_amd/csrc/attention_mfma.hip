@@ -632,51 +632,89 @@ attention_mfma_kernel(const bf16* __restrict__ q, size_t q_stride, const bf16* _
 }
 
 // out[r, h, :] = sum_s 2^(m_s - M) O_s / sum_s 2^(m_s - M) l_s over the splits that request r used.
-// One block per (request, head): the splits' maxima and sums are fetched side by side, the
-// weights are worked out once into LDS, then a thread per dim adds the weighted partial results in split order.
-constexpr int COMBINE_MAX_SPLITS = 128;
+// One block per (request, head).  It is bound by latency, a launch and trips to memory one after another: so everything is asked
+// for at once, also of splits that turn out not to be used, every wave works the weights out for itself (a split to a lane) and adds
+// up every fourth split, and one barrier later the four sums are added in order (with the split attention in front of it, 2 requests
+// of 1,100 keys 10.0 -> 8.8 us, one of 4,352 keys and 128 dims 11.5 -> 10.8).
+constexpr int COMBINE_MAX_SPLITS = 128, COMBINE_WAVES = 4;
 
 template <int D>
-__global__ void __launch_bounds__(D < 64 ? 64 : D)
+__global__ void __launch_bounds__(COMBINE_WAVES * MS_WAVE)
 attention_combine_kernel(const float* __restrict__ part_o, const float* __restrict__ part_ml,
                          const int* __restrict__ q_start, const int* __restrict__ context_lens,
                          bf16* __restrict__ out, size_t out_stride, int nh, int dv, int window, int min_blocks,
                          int n_splits, const bf16* __restrict__ gate, size_t gate_stride, int gate_width, float out_scale) {
-  __shared__ float sm_m[COMBINE_MAX_SPLITS], sm_w[COMBINE_MAX_SPLITS];
-  const int r = blockIdx.x / nh, h = blockIdx.x % nh;
-  if (q_start[r + 1] == q_start[r]) return;   // a row that pads a captured batch: no token, nothing to write
-  const int key_hi = context_lens[r] - 1;
+  constexpr int DL = (D + MS_WAVE - 1) / MS_WAVE;    // dims to a lane
+  constexpr int AHEAD = 8;                           // splits of a wave asked for before anything is known of them
+  __shared__ float sums[COMBINE_WAVES][DL * MS_WAVE];
+  const int r = blockIdx.x / nh, h = blockIdx.x % nh, lane = threadIdx.x & (MS_WAVE - 1), wave = threadIdx.x / MS_WAVE;
+  const size_t slot0 = ((size_t)r * nh + h) * n_splits;
+  const int q0 = q_start[r], q1 = q_start[r + 1], context = context_lens[r];
+  float m[2], l[2], o[AHEAD][DL];                    // lane s and s - 64 have split s's reference and sum
+#pragma unroll
+  for (int i = 0; i < 2; ++i) {
+    const size_t at = 2 * (slot0 + min(lane + i * MS_WAVE, n_splits - 1));
+    m[i] = part_ml[at];
+    l[i] = part_ml[at + 1];
+  }
+  auto value = [&](int split, int e) { return part_o[(slot0 + min(split, n_splits - 1)) * dv + min(lane + e * MS_WAVE, dv - 1)]; };
+#pragma unroll
+  for (int a = 0; a < AHEAD; ++a)
+#pragma unroll
+    for (int e = 0; e < DL; ++e) o[a][e] = value(wave + a * COMBINE_WAVES, e);
+  if (q1 == q0) return;   // a row that pads a captured batch: no token, nothing to write
+  const int key_hi = context - 1;
   const int key_lo = window > 0 ? max(0, key_hi - window + 1) : 0;
   const int blocks = key_hi / 32 + 1 - key_lo / 32;
   const int per = max(min_blocks, (blocks + n_splits - 1) / n_splits);
   const int used = (blocks + per - 1) / per;
-  const size_t slot0 = ((size_t)r * nh + h) * n_splits;
-  const int t = threadIdx.x;
-  for (int s = t; s < used; s += blockDim.x) sm_m[s] = part_ml[(slot0 + s) * 2];
-  __syncthreads();
-  float big = -INFINITY;
-  for (int s = 0; s < used; ++s) big = fmaxf(big, sm_m[s]);
-  __syncthreads();
-  // the weights, and in sm_m (no longer needed) the splits' weighted sums for the denominator in split order
-  for (int s = t; s < used; s += blockDim.x) {
-    const float w = fast_exp2(sm_m[s] - big);
-    sm_w[s] = w;
-    sm_m[s] = w * part_ml[(slot0 + s) * 2 + 1];
+  // what lies behind the splits that were used may be anything
+  float w[2], top = -INFINITY, den = 0.f;
+#pragma unroll
+  for (int i = 0; i < 2; ++i) top = fmaxf(top, lane + i * MS_WAVE < used ? m[i] : -INFINITY);
+  top = wave_max(top);
+#pragma unroll
+  for (int i = 0; i < 2; ++i) {
+    const bool in = lane + i * MS_WAVE < used;
+    w[i] = in ? fast_exp2(m[i] - top) : 0.f;
+    den += in ? w[i] * l[i] : 0.f;
   }
+  den = wave_sum(den);
+  auto weight = [&](int split) {      // the same for the whole wave
+    return __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, split < MS_WAVE ? w[0] : w[1]), split & (MS_WAVE - 1)));
+  };
+  float acc[DL] = {};
+  const int first = __builtin_amdgcn_readfirstlane(wave);
+#pragma unroll
+  for (int a = 0; a < AHEAD; ++a) {
+    const int split = first + a * COMBINE_WAVES;
+    if (split < used) {
+#pragma unroll
+      for (int e = 0; e < DL; ++e) acc[e] += weight(split) * o[a][e];
+    }
+  }
+  for (int split = first + AHEAD * COMBINE_WAVES; split < used; split += COMBINE_WAVES) {
+#pragma unroll
+    for (int e = 0; e < DL; ++e) acc[e] += weight(split) * value(split, e);
+  }
+#pragma unroll
+  for (int e = 0; e < DL; ++e) sums[wave][lane + e * MS_WAVE] = acc[e];
   __syncthreads();
-  float den = 0.f;
-  for (int s = 0; s < used; ++s) den += sm_m[s];
+  if (wave > 0) return;
   float inv = out_scale / den;
-  const bf16* gp = gate ? gate + (size_t)q_start[r] * gate_stride + (size_t)h * gate_width : nullptr;
+  const bf16* gp = gate ? gate + (size_t)q0 * gate_stride + (size_t)h * gate_width : nullptr;
   if (gate && gate_width == 1) inv *= 1.0f / (1.0f + expf(-__bfloat162float(*gp)));
-  bf16* op = out + (size_t)q_start[r] * out_stride + (size_t)h * dv;
-  for (int d = t; d < dv; d += blockDim.x) {
-    float acc = 0.f;
-#pragma unroll 8
-    for (int s = 0; s < used; ++s) acc += sm_w[s] * part_o[(slot0 + s) * dv + d];
-    acc *= inv;
-    if (gate && gate_width != 1) acc /= 1.0f + expf(-__bfloat162float(gp[d]));
-    op[d] = __float2bfloat16(acc);
+  bf16* op = out + (size_t)q0 * out_stride + (size_t)h * dv;
+#pragma unroll
+  for (int e = 0; e < DL; ++e) {
+    const int d = lane + e * MS_WAVE;
+    if (d >= dv) continue;
+    float v = sums[0][d];
+#pragma unroll
+    for (int t = 1; t < COMBINE_WAVES; ++t) v += sums[t][d];
+    v *= inv;
+    if (gate && gate_width != 1) v /= 1.0f + expf(-__bfloat162float(gp[d]));
+    op[d] = __float2bfloat16(v);
   }
 }
 
@@ -750,7 +788,7 @@ int launch_split(const bf16* q, size_t q_stride, const bf16* k, const bf16* vt, 
     attention_mfma_kernel<D, 1, 4, true, 1, true><<<grid, block, 0, stream>>>(q, q_stride, k, vt, table, table_stride, table_rows, q_start, ctx, out, out_stride, part_o, part_ml, nh, nkv, page_size, page_shift_of(page_size), scale * 1.4426950408889634f, window, min_blocks, n_splits, sink);
   else
     attention_mfma_kernel<D, 1, 4, true, 1, false><<<grid, block, 0, stream>>>(q, q_stride, k, vt, table, table_stride, table_rows, q_start, ctx, out, out_stride, part_o, part_ml, nh, nkv, page_size, page_shift_of(page_size), scale * 1.4426950408889634f, window, min_blocks, n_splits, nullptr);
-  attention_combine_kernel<D><<<dim3(n_requests * nh), dim3(D < 64 ? 64 : D), 0, stream>>>(part_o, part_ml, q_start, ctx, out, out_stride, nh, extras ? extras->value_dim : D, window, min_blocks, n_splits, extras ? extras->gate : nullptr, extras ? extras->gate_stride : 0, extras ? extras->gate_width : 1, extras ? extras->out_scale : 1.0f);
+  attention_combine_kernel<D><<<dim3(n_requests * nh), dim3(COMBINE_WAVES * MS_WAVE), 0, stream>>>(part_o, part_ml, q_start, ctx, out, out_stride, nh, extras ? extras->value_dim : D, window, min_blocks, n_splits, extras ? extras->gate : nullptr, extras ? extras->gate_stride : 0, extras ? extras->gate_width : 1, extras ? extras->out_scale : 1.0f);
   return ms_launch_status();
 }
 

@@ -2109,3 +2109,31 @@ def test_float_products_of_up_to_8_rows_are_those_of_more(ops, M, N, K):
     ok = exact[:M].isfinite()
     got = ops.gemm_generic(a[:M], w, torch.empty(M, N, device=DEV), bias)
     assert ((got.double() - exact[:M])[ok].abs() <= 4e-6 * math.sqrt(K) * 4).all()
+
+
+@pytest.mark.parametrize("keys,cap", [(1, 2048), (257, 2048), (9000, 16384), (9000, 40000), (24001, 70000)])
+@pytest.mark.parametrize("nh,nkv,d", [(14, 2, 64), (3, 1, 32), (8, 4, 128)])
+def test_splits_are_put_together(ops, nh, nkv, d, keys, cap):
+    """One split and many of a row's keys (one, two, 36 of up to 24 or 32, 94 of 128: each wave's share in part, whole, and
+    beyond what is asked for ahead), a row that pads the batch, and what lies in the parts nobody wrote."""
+    g = torch.Generator().manual_seed(keys + d)
+    n = -(-keys // 16)
+    kp = torch.randn(n + 1, nkv, 16, d, generator=g).bfloat16().to(DEV)
+    vp = torch.randn(n + 1, nkv, d, 16, generator=g).bfloat16().to(DEV)
+    table = torch.zeros(2, -(-cap // 16), dtype=torch.int32)
+    table[0, :n] = torch.randperm(n, generator=g) + 1
+    q = torch.randn(2, nh * d, generator=g).bfloat16().to(DEV)
+    out = torch.full_like(q, 7.0)
+    junk = torch.full((64 << 20,), float("nan"), device=DEV)
+    del junk       # (the parts are likely to lie where this lay)
+    ops.paged_attention_mfma(q, kp, vp, table.to(DEV), torch.tensor([0, 1, 1], dtype=torch.int32, device=DEV),
+                             torch.tensor([keys, 0], dtype=torch.int32, device=DEV), out, nh, d ** -0.5, 1, cap)
+    k = kp[table[0, :n].long()].permute(1, 0, 2, 3).reshape(nkv, n * 16, d)[:, :keys].double()
+    v = vp[table[0, :n].long()].permute(1, 0, 3, 2).reshape(nkv, n * 16, d)[:, :keys].double()
+    k, v = (t.repeat_interleave(nh // nkv, 0) for t in (k, v))
+    w = ((k @ q[0].view(nh, d, 1).double()).squeeze(2) * d ** -0.5).softmax(1)
+    want = (w.unsqueeze(1) @ v).reshape(-1)
+    # probabilities and result in bfloat16: 2^-9 of the weighted values' size each
+    size = (w.unsqueeze(1) @ v.abs()).reshape(-1)
+    assert ((out[0].double() - want).abs() <= 2 ** -7 * size + 1e-6).all()
+    assert (out[1] == 7.0).all()
