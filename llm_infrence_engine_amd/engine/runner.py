@@ -100,17 +100,19 @@ class ModelRunner:
             caches = self.caches(built.ctx.state_slots, built.slots)
             if built.ctx.decode_only:
                 key = (built.ctx.num_tokens, built.ctx.max_context_len > ops.DECODE_KEYS)
-                if key not in self.chains:
-                    self.chains[key] = DecodeChain.of(self.model, built.ctx, caches)
-                built.ctx.chain = self.chains[key]
+                built.ctx.chain = self._chain(key, caches, lambda: DecodeChain.of(self.model, built.ctx, caches))
             if built.ctx.chain is None:
-                if "float" not in self.chains:
-                    self.chains["float"] = FloatLayers.of(self.model, caches)
-                built.ctx.chain = self.chains["float"]
+                built.ctx.chain = self._chain("float", caches, lambda: FloatLayers.of(self.model, caches))
             logits = self.model.forward(built.ctx, caches)
         for e in entries:
             m.advance(e.req_id, m.computed(e.req_id) + len(e.tokens))
         return logits
+
+    def _chain(self, key, caches, make):
+        """What runs the layers of steps like ``key``, made once and again when weights or pages are others."""
+        if key not in self.chains or (self.chains[key] is not None and not self.chains[key].takes(self.model, caches)):
+            self.chains[key] = make()
+        return self.chains[key]
 
     @torch.inference_mode()
     def decode_steps(self, entries: List[StepEntry], steps: int, sampling=None) -> List[List[int]]:

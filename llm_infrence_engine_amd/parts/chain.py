@@ -57,8 +57,30 @@ def _plain_layers(model, caches) -> bool:
                     and c.kv.v_transposed == kv.v_transposed and c.kv.stride == 1 for c in caches))
 
 
-def _same_pages(pages, caches) -> bool:
-    return all(a.data_ptr() == b.data_ptr() for a, b in zip(pages, (t for c in caches for t in (c.kv.k_pages, c.kv.v_pages))))
+def _pages(caches):
+    return [t for c in caches for t in (c.kv.k_pages, c.kv.v_pages)]
+
+
+def _weights(model):
+    out = []
+    for run in model.spec.order:
+        l = model.layers[run.layer]
+        m, f = l.mixer, l.feed_forward
+        out += (l.mixer_norm.weight, m.w_qkv, m.b_qkv, m.position.inv_freq, m.w_o, l.feed_forward_norm.weight, f.w_gate_up, f.w_down)
+    return out
+
+
+class _Addresses:
+    """The tensors whose addresses a record of the layers holds: kept alive, and compared with the model's and the caches' own
+    before the record is read again, so that weights loaded anew are not missed."""
+
+    def __init__(self, model, caches):
+        self.weights, self.pages = _weights(model), _pages(caches)
+
+    def hold(self, model, caches) -> bool:
+        now = _weights(model)
+        return (len(now) == len(self.weights) and all(a is b for a, b in zip(self.weights, now))
+                and all(a.data_ptr() == b.data_ptr() and a.shape == b.shape for a, b in zip(self.pages, _pages(caches))))
 
 
 class FloatLayers:
@@ -67,7 +89,7 @@ class FloatLayers:
 
     def __init__(self, model, sizes: tuple, caches):
         self.sizes, self.layers = sizes, [model.layers[run.layer] for run in model.spec.order]
-        self.pages = [t for c in caches for t in (c.kv.k_pages, c.kv.v_pages)]
+        self.addresses = _Addresses(model, caches)
         nh, nkv, d, _, _ = sizes
         self.records = ops.float_layer_records(
             [dict(norm1=l.mixer_norm.weight, eps1=l.mixer_norm.eps, w_qkv=l.mixer.w_qkv, b_qkv=l.mixer.b_qkv,
@@ -86,9 +108,9 @@ class FloatLayers:
             return None
         return cls(model, sizes.pop(), caches)
 
-    def takes(self, caches) -> bool:
-        """Whether these are the caches that the records were made of."""
-        return (len(caches) == len(self.layers) and _own_pages(caches, torch.float32) and _same_pages(self.pages, caches)
+    def takes(self, model, caches) -> bool:
+        """Whether these are the weights and the caches that the records were made of."""
+        return (len(caches) == len(self.layers) and _own_pages(caches, torch.float32) and self.addresses.hold(model, caches)
                 and all(c.kv.slot_mapping is caches[0].kv.slot_mapping for c in caches))
 
     def forward(self, x, ctx, caches):
@@ -106,7 +128,7 @@ class DecodeChain:
         self.sizes, self.runs = sizes, len(model.spec.order)
         self.layers = [model.layers[run.layer] for run in model.spec.order]
         self.workspace = torch.zeros(n_bytes, dtype=torch.uint8, device=model.rt.device)
-        self.table, self.pages = None, []
+        self.table, self.addresses = None, None
         self.broken_off = False      # a step ended with an exception between its launches
 
     @classmethod
@@ -127,7 +149,7 @@ class DecodeChain:
             n_bytes = ops.decode_chain_workspace(n, H, nh, nkv, d, I, len(runs))
             if n_bytes:
                 chain = cls(model, sizes, n_bytes)
-                chain._lay_out(caches)
+                chain._lay_out(model, caches)
                 return chain
         n_bytes = ops.decode_chain_workspace(n, H, nh, nkv, d, I)
         return cls(model, sizes, n_bytes) if n_bytes else None
@@ -142,7 +164,7 @@ class DecodeChain:
         page_size = caches[0].kv.k_pages.shape[2]
         return _plain_layers(model, caches) and caches[0].kv.v_transposed and page_size >= 16 and page_size & (page_size - 1) == 0
 
-    def _lay_out(self, caches):
+    def _lay_out(self, model, caches):
         rows = []
         for i, (layer, c) in enumerate(zip(self.layers, caches)):
             m, f = layer.mixer, layer.feed_forward
@@ -153,14 +175,15 @@ class DecodeChain:
                 row.update(w_front=then.mixer.w_qkv, norm1=then.mixer_norm.weight, eps1=then.mixer_norm.eps, b_front=then.mixer.b_qkv,
                            inv_freq=then.mixer.position.inv_freq, front_k=kv.k_pages, front_v=kv.v_pages)
             rows.append(row)
-        self.pages = [t for c in caches for t in (c.kv.k_pages, c.kv.v_pages)]
+        self.addresses = _Addresses(model, caches)
         self.table = ops.decode_layer_table(rows, self.workspace.device)
 
-    def takes(self, caches) -> bool:
-        """Whether these are the caches that the chain was made for (or, where it reads no table of them, any like them)."""
+    def takes(self, model, caches) -> bool:
+        """Whether these are the weights and the caches that the chain was made for (or, where it reads no table of them, any like
+        them)."""
         if len(caches) != self.runs or not self._stores(caches):
             return False
-        return self.table is None or _same_pages(self.pages, caches)
+        return self.table is None or self.addresses.hold(model, caches)
 
     def forward(self, x, ctx, caches):
         """All runs of the order on the embedded tokens ``x`` [N, H], in place; returns x and what is left to add to it (nothing)."""

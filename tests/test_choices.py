@@ -187,7 +187,13 @@ def test_chains_take_the_parts_whose_arithmetic_they_have(ops):
                                                      v_transposed=transposed, window=b.mixer.window, stride=1, store=store))
                   for _ in range(runs)]
         made = chain.DecodeChain.of(m, SimpleNamespace(num_tokens=n, num_requests=n, max_context_len=keys), caches)
-        assert made is None or made.takes(caches) and not made.workspace.any()
+        assert made is None or made.takes(m, caches) and not made.workspace.any()
+        if made is not None and made.table is not None:      # weights loaded anew, pages elsewhere
+            b.feed_forward.w_down = b.feed_forward.w_down.clone()
+            assert not made.takes(m, caches)
+            b.feed_forward.w_down = made.addresses.weights[-1]
+            caches[-1].kv.k_pages = caches[-1].kv.k_pages.clone()
+            assert not made.takes(m, caches)
         return None if made is None else "layers" if made.table is None else "step"
 
     assert of() == of(keys=1024) == of(page=32) == "step"
@@ -231,7 +237,13 @@ def test_float_layers_are_the_parts_one_by_one(ops, tokens):
         if not whole:
             r.chains["float"] = None
         r.step([StepEntry(0, list(range(20)), [19])])
+        before, ff = r.chains["float"], model.layers[0].feed_forward      # weights loaded anew are not missed
+        kept, ff.w_down = ff.w_down, ff.w_down * 2
+        anew = r.step([StepEntry(1, [3], [0])]).cpu()
+        assert (r.chains["float"] is not before) == whole
+        ff.w_down = kept
+        r.free_request(1)
         out = [r.step([StepEntry(i, [7 + i] * n, [n - 1]) for i, n in enumerate(tokens)]).cpu() for _ in range(2)]
         assert isinstance(r.chains["float"], chain.FloatLayers) == whole
-        got.append(out + [t.cpu() for pages in r.pools.pages for t in pages.values()])
+        got.append([anew] + out + [t.cpu() for pages in r.pools.pages for t in pages.values()])
     assert all(torch.equal(a, b) for a, b in zip(*got))
