@@ -223,13 +223,15 @@ __device__ __forceinline__ bool has_own_step(int lane) { return ((lane & 15) / G
 struct Shared {
   quad_f32 part[NT * WAVES * 4 * 8];   // gate: [tile][wave][row group * G + token]; else [unit][token][wave * 4 + step]
   float part_ss[8][WAVES];              // [token]
-  int late[2];                          // somebody gave up: waiting for the first word, for the others
+  int late[3];                          // somebody gave up: waiting for the first word, for the others, for a phase before the one before
   int next, position;
   unsigned done[(LIST + 32) / 32];
 };
 
 // One word of the phase before, by one wave, so that blocks far ahead of their inputs disturb nobody.  Whole block; false: not
-// within `limit` looks.
+// within `limit` looks.  VERDICT: the word of sh.late, another for each wait of an item: no barrier lies between a wave's read of it
+// and the store of the wait that follows.
+template <int VERDICT = 0>
 __device__ __forceinline__ bool wait_first(Shared& sh, const u64* word, unsigned tag, unsigned limit) {
   if (threadIdx.x < MS_WAVE) {
     int late = 1;
@@ -237,10 +239,10 @@ __device__ __forceinline__ bool wait_first(Shared& sh, const u64* word, unsigned
       if ((unsigned)(look(word) >> 32) == tag) { late = 0; break; }
       __builtin_amdgcn_s_sleep(1);
     }
-    if (threadIdx.x == 0) { sh.late[0] = late; sh.late[1] = 0; }
+    if (threadIdx.x == 0) { sh.late[VERDICT] = late; sh.late[1] = 0; }
   }
   __syncthreads();
-  return sh.late[0] == 0;
+  return sh.late[VERDICT] == 0;
 }
 
 // A wave's share of the float stream's rows (one load's worth of four k-steps, G tokens), with the norm's weights.
@@ -643,7 +645,7 @@ __device__ __forceinline__ bool run_down(Args& a, Shared& sh, LayerArgs& L, bool
   // Where there are as many blocks as CUs, their weights would come ahead of x1 on the way to gate's blocks: they wait for x1 (one
   // token 13.5 -> 13.1 us; half as many blocks lose 0.3).
   if constexpr (UD == 1 && MODE == CHAIN) {
-    if (!wait_first(sh, a.x1 + stream_word((b * 8) % a.H, 0, a.M), tag, limit)) return false;
+    if (!wait_first<2>(sh, a.x1 + stream_word((b * 8) % a.H, 0, a.M), tag, limit)) return false;
   }
   // runs `wave` and `wave` + 8 of the 16, C loads of four steps each
   quad_u32 w[2][C][UD];

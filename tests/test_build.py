@@ -94,3 +94,15 @@ def test_loads_written_in_assembly_wait_for_their_bases():
                 assert b.startswith("SGPRS_READY") and b.endswith('"s_waitcnt vmcnt(0)"'), (src.name, b)
             assert '#define SGPRS_READY "s_nop 4' in text
         assert not re.search(r'asm volatile\(\s*"[^"]*_(load|store)', text), src.name     # none beside those
+
+
+def test_waits_of_one_item_keep_their_verdicts_apart():
+    """A wave reads the verdict of a wait behind the wait's barrier, and nothing holds it up against the next wait's store: so
+    the waits of one item of a decode chain have a word each, and none the one for waits that are the waves' own."""
+    text = next(s for s in build.sources() if s.name == "decode_chain.hip").read_text()
+    items = re.split(r"\n__device__ __forceinline__ bool run_", text)[1:]
+    verdicts = [[int(v or 0) for v in re.findall(r"wait_first(?:<(\d+)>)?\(", i)] for i in items]
+    assert sum(map(len, verdicts)) >= 6
+    for v in verdicts:
+        assert len(set(v)) == len(v) and 1 not in v
+    assert f"int late[{max(map(max, filter(None, verdicts))) + 1}];" in text
