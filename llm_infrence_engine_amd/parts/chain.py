@@ -70,6 +70,20 @@ def _weights(model):
     return out
 
 
+def _readable(model, align: int) -> bool:
+    """Whether the weights are whole rows, and on ``align`` bytes those that are read in pieces (all but biases and frequencies).
+    Weights may be views of a larger buffer; the parts' own kernels take them as they come."""
+    for run in model.spec.order:
+        l = model.layers[run.layer]
+        m, f = l.mixer, l.feed_forward
+        if any(not t.is_contiguous() or t.data_ptr() % align for t in (m.w_qkv, m.w_o, f.w_gate_up, f.w_down, l.mixer_norm.weight,
+                                                                         l.feed_forward_norm.weight)):
+            return False
+        if not m.position.inv_freq.is_contiguous() or m.b_qkv is not None and not m.b_qkv.is_contiguous():
+            return False
+    return True
+
+
 class _Addresses:
     """The tensors whose addresses a record of the layers holds: kept alive, and compared with the model's and the caches' own
     before the record is read again, so that weights loaded anew are not missed."""
@@ -106,6 +120,8 @@ class FloatLayers:
         sizes = {_sizes(model.layers[run.layer]) for run in runs}
         if len(sizes) != 1 or None in sizes or not _own_pages(caches, torch.float32) or not _plain_layers(model, caches):
             return None
+        if not _readable(model, 4):
+            return None
         return cls(model, sizes.pop(), caches)
 
     def takes(self, model, caches) -> bool:
@@ -141,7 +157,7 @@ class DecodeChain:
         if any(run.opens_pass is not None for run in runs):
             return None
         sizes = {_sizes(model.layers[run.layer]) for run in runs}
-        if len(sizes) != 1 or None in sizes or not cls._stores(caches):
+        if len(sizes) != 1 or None in sizes or not cls._stores(caches) or not _readable(model, 16):
             return None
         sizes = sizes.pop()
         nh, nkv, d, H, I = sizes

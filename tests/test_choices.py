@@ -201,6 +201,56 @@ def test_chains_take_the_parts_whose_arithmetic_they_have(ops):
     assert of(9) is of(runs=1) is of(opens=0) is of(dtype=torch.float32) is of(entry=b"") is of(store=False) is None
 
 
+def _decode_stand_in(ops, keys=64, runs=2):
+    """(model, its one layer, caches, what DecodeChain.of says of them now) of parts that chains take; weights are stand-ins."""
+    from llm_infrence_engine_amd.parts import chain
+    from llm_infrence_engine_amd.parts.attention import GQAttention
+    from llm_infrence_engine_amd.parts.positions import RotaryHalf
+
+    b = _block(ops, norm=True, mixer=True, feed_forward=True, block=True)
+    b.mixer = GQAttention("", RotaryHalf("", 64, 64, 1e4), 64, 2, 1, 64, 0.1)
+    for part, names in ((b.mixer, ("w_o", "w_qkv", "b_qkv")), (b.feed_forward, ("w_gate_up", "w_down")),
+                        (b.mixer_norm, ("weight",)), (b.feed_forward_norm, ("weight",)), (b.mixer.position, ("inv_freq",))):
+        for name in names:
+            setattr(part, name, torch.zeros(4, 4))
+    b.mixer.sink_w = None
+    m = SimpleNamespace(spec=SimpleNamespace(order=[SimpleNamespace(layer=0, opens_pass=None)] * runs), layers=[b],
+                        rt=SimpleNamespace(dtype=torch.bfloat16, device="cpu"), pass_entry=None)
+    table, slots, pages = torch.zeros(1), torch.zeros(1), torch.zeros(1, 1, 16, 64, dtype=torch.bfloat16)
+    caches = [SimpleNamespace(kv=SimpleNamespace(k_pages=pages.clone(), v_pages=pages.clone(), block_table=table, slot_mapping=slots,
+                                                 v_transposed=True, window=None, stride=1, store=True)) for _ in range(runs)]
+    return m, b, caches, lambda: chain.DecodeChain.of(m, SimpleNamespace(num_tokens=8, num_requests=8, max_context_len=keys), caches)
+
+
+@pytest.mark.parametrize("keys", [64, 2000])
+def test_chains_leave_weights_they_cannot_read_to_the_parts(ops, keys):
+    """Views of a larger buffer, as a reader of weights may hand out: the products have a kernel for any address and any row
+    stride, the chains only for whole rows on 16 bytes.  Biases and frequencies are read one by one."""
+    from llm_infrence_engine_amd.parts import chain
+
+    m, b, caches, of = _decode_stand_in(ops, keys)
+    aside, strided = torch.zeros(17)[1:].view(4, 4), torch.zeros(4, 8)[:, :4]
+    assert aside.data_ptr() % 16 and not strided.is_contiguous() and of() is not None
+    for part, name in ((b.mixer, "w_o"), (b.mixer, "w_qkv"), (b.feed_forward, "w_gate_up"), (b.feed_forward, "w_down"),
+                       (b.mixer_norm, "weight"), (b.feed_forward_norm, "weight")):
+        kept = getattr(part, name)
+        for other in (aside, strided):
+            setattr(part, name, other)
+            assert of() is None
+        m.rt.dtype = torch.float32      # all layers of a 32-bit step by one call: any address, whole rows
+        for c in caches:
+            c.kv.k_pages, c.kv.v_pages = c.kv.k_pages.float(), c.kv.v_pages.float()
+        assert chain.FloatLayers.of(m, caches) is None
+        m.rt.dtype = torch.bfloat16
+        for c in caches:
+            c.kv.k_pages, c.kv.v_pages = c.kv.k_pages.bfloat16(), c.kv.v_pages.bfloat16()
+        setattr(part, name, kept)
+    b.mixer.b_qkv = b.mixer.position.inv_freq = aside
+    assert of() is not None
+    b.mixer.b_qkv = None
+    assert of() is not None
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("tokens", [[1, 1, 1], [1, 40, 3]])
 def test_float_layers_are_the_parts_one_by_one(ops, tokens):
