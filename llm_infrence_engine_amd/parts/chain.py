@@ -61,13 +61,13 @@ def _pages(caches):
     return [t for c in caches for t in (c.kv.k_pages, c.kv.v_pages)]
 
 
-def _weights(model):
-    out = []
-    for run in model.spec.order:
-        l = model.layers[run.layer]
-        m, f = l.mixer, l.feed_forward
-        out += (l.mixer_norm.weight, m.w_qkv, m.b_qkv, m.position.inv_freq, m.w_o, l.feed_forward_norm.weight, f.w_gate_up, f.w_down)
-    return out
+def _parts(l) -> tuple:
+    return l, l.mixer, l.mixer.position, l.feed_forward, l.mixer_norm, l.feed_forward_norm
+
+
+def _weights(l) -> tuple:
+    m, f = l.mixer, l.feed_forward
+    return l.mixer_norm.weight, m.w_qkv, m.b_qkv, m.position.inv_freq, m.w_o, l.feed_forward_norm.weight, f.w_gate_up, f.w_down
 
 
 def _readable(model, align: int) -> bool:
@@ -85,16 +85,32 @@ def _readable(model, align: int) -> bool:
 
 
 class _Addresses:
-    """The tensors whose addresses a record of the layers holds: kept alive, and compared with the model's and the caches' own
-    before the record is read again, so that weights loaded anew are not missed."""
+    """The parts that a chain runs and the tensors whose addresses a record of them holds: kept alive, and compared with the
+    model's and the caches' own before the chain runs again, so that weights loaded anew and layers put in are not missed."""
 
     def __init__(self, model, caches):
-        self.weights, self.pages = _weights(model), _pages(caches)
+        layers = [model.layers[run.layer] for run in model.spec.order]
+        self.parts = [_parts(l) for l in layers]
+        self.weights = [t for l in layers for t in _weights(l)]
+        self.places = [0 if t is None else t.data_ptr() for t in self.weights]
+        self.pages = _pages(caches)
+
+    def hold_weights(self, model) -> bool:
+        order, layers = model.spec.order, model.layers
+        if len(order) != len(self.parts):
+            return False
+        now = []
+        for run, (layer, mixer, position, feed_forward, mixer_norm, feed_forward_norm) in zip(order, self.parts):
+            l = layers[run.layer]
+            if (l is not layer or l.mixer is not mixer or mixer.position is not position or l.feed_forward is not feed_forward
+                    or l.mixer_norm is not mixer_norm or l.feed_forward_norm is not feed_forward_norm):
+                return False
+            now += _weights(l)
+        return all(a is b and (a is None or a.data_ptr() == place) for a, b, place in zip(now, self.weights, self.places))
 
     def hold(self, model, caches) -> bool:
-        now = _weights(model)
-        return (len(now) == len(self.weights) and all(a is b for a, b in zip(self.weights, now))
-                and all(a.data_ptr() == b.data_ptr() and a.shape == b.shape for a, b in zip(self.pages, _pages(caches))))
+        return self.hold_weights(model) and all(a.data_ptr() == b.data_ptr() and a.shape == b.shape
+                                                for a, b in zip(self.pages, _pages(caches)))
 
 
 class FloatLayers:
@@ -140,11 +156,11 @@ class DecodeChain:
     """The chains of one batch size, with their workspace; ``table``: what ``ops.decode_layers`` reads, where the step's layers
     go in two launches, else None."""
 
-    def __init__(self, model, sizes: tuple, n_bytes: int):
+    def __init__(self, model, sizes: tuple, n_bytes: int, caches):
         self.sizes, self.runs = sizes, len(model.spec.order)
         self.layers = [model.layers[run.layer] for run in model.spec.order]
         self.workspace = torch.zeros(n_bytes, dtype=torch.uint8, device=model.rt.device)
-        self.table, self.addresses = None, None
+        self.table, self.addresses = None, _Addresses(model, caches)
         self.broken_off = False      # a step ended with an exception between its launches
 
     @classmethod
@@ -164,11 +180,11 @@ class DecodeChain:
         if ctx.max_context_len <= ops.DECODE_KEYS and cls._one_group(model, caches):
             n_bytes = ops.decode_chain_workspace(n, H, nh, nkv, d, I, len(runs))
             if n_bytes:
-                chain = cls(model, sizes, n_bytes)
-                chain._lay_out(model, caches)
+                chain = cls(model, sizes, n_bytes, caches)
+                chain._lay_out(caches)
                 return chain
         n_bytes = ops.decode_chain_workspace(n, H, nh, nkv, d, I)
-        return cls(model, sizes, n_bytes) if n_bytes else None
+        return cls(model, sizes, n_bytes, caches) if n_bytes else None
 
     @classmethod
     def _stores(cls, caches) -> bool:
@@ -180,7 +196,7 @@ class DecodeChain:
         page_size = caches[0].kv.k_pages.shape[2]
         return _plain_layers(model, caches) and caches[0].kv.v_transposed and page_size >= 16 and page_size & (page_size - 1) == 0
 
-    def _lay_out(self, model, caches):
+    def _lay_out(self, caches):
         rows = []
         for i, (layer, c) in enumerate(zip(self.layers, caches)):
             m, f = layer.mixer, layer.feed_forward
@@ -191,15 +207,14 @@ class DecodeChain:
                 row.update(w_front=then.mixer.w_qkv, norm1=then.mixer_norm.weight, eps1=then.mixer_norm.eps, b_front=then.mixer.b_qkv,
                            inv_freq=then.mixer.position.inv_freq, front_k=kv.k_pages, front_v=kv.v_pages)
             rows.append(row)
-        self.addresses = _Addresses(model, caches)
         self.table = ops.decode_layer_table(rows, self.workspace.device)
 
     def takes(self, model, caches) -> bool:
-        """Whether these are the weights and the caches that the chain was made for (or, where it reads no table of them, any like
-        them)."""
+        """Whether these are the layers, the weights and the caches that the chain was made for (or, where it reads no table of
+        their pages, any caches like them)."""
         if len(caches) != self.runs or not self._stores(caches):
             return False
-        return self.table is None or self.addresses.hold(model, caches)
+        return self.addresses.hold_weights(model) if self.table is None else self.addresses.hold(model, caches)
 
     def forward(self, x, ctx, caches):
         """All runs of the order on the embedded tokens ``x`` [N, H], in place; returns x and what is left to add to it (nothing)."""

@@ -251,6 +251,35 @@ def test_chains_leave_weights_they_cannot_read_to_the_parts(ops, keys):
     assert of() is not None
 
 
+@pytest.mark.parametrize("keys", [64, 2000])
+def test_a_chain_holds_for_the_layers_and_weights_it_was_made_of(ops, keys):
+    """With or without a table of addresses: another storage under the same tensor, another tensor, another part and another
+    layer in a model's place are all seen before the chain runs again."""
+    m, b, caches, of = _decode_stand_in(ops, keys)
+    made = of()
+    assert made.takes(m, caches) and (made.table is None) == (keys == 2000)
+    kept = b.mixer.w_o.data
+    b.mixer.w_o.data = kept.clone()
+    assert not made.takes(m, caches)
+    b.mixer.w_o.data = kept
+    assert made.takes(m, caches)
+    other = _decode_stand_in(ops, keys)[1]
+    for part in ("mixer", "feed_forward", "mixer_norm", "feed_forward_norm"):
+        kept = getattr(b, part)
+        setattr(b, part, SimpleNamespace(weight=getattr(kept, "weight", None)))      # (without what the chain reads of it)
+        assert not made.takes(m, caches)
+        setattr(b, part, kept)
+    kept, b.mixer.position = b.mixer.position, other.mixer.position
+    assert not made.takes(m, caches)
+    b.mixer.position = kept
+    m.layers[0] = other
+    assert not made.takes(m, caches)
+    m.layers[0] = b
+    assert made.takes(m, caches)
+    m.spec.order = m.spec.order[:1]
+    assert not made.takes(m, caches)
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("tokens", [[1, 1, 1], [1, 40, 3]])
 def test_float_layers_are_the_parts_one_by_one(ops, tokens):
