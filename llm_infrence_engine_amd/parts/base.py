@@ -167,7 +167,7 @@ class StepContext:
     # what a part derives from the step's tensors once for all layers that hold a part like it (key: the part's
     # choice); whoever changes ``positions`` in place empties it
     shared: dict = field(default_factory=dict)
-    # what runs all layers of the step at once (``parts.chain``); None: layer by layer
+    # what runs all layers of the step at once (``parts.chain``) and takes this model and the step's caches; None: layer by layer
     chain: Optional[object] = None
 
     @property

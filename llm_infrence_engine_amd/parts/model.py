@@ -95,7 +95,7 @@ class Model:
         copies of it) and what the last run has still to write into it (an addend, a write that the final norm carries out
         itself, or None)."""
         x = self.embedding.forward(ctx)
-        if ctx.chain is not None and ctx.chain.takes(self, caches):
+        if ctx.chain is not None:      # (whoever put it there has asked it whether it takes this model and these caches)
             x, pending = ctx.chain.forward(x, ctx, caches)
             return x, self._settled(x, pending, self.final_norm)
         kept = x.clone() if self.pass_entry is not None and self.pass_entry.keeps_embedding else None

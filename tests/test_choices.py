@@ -280,6 +280,45 @@ def test_a_chain_holds_for_the_layers_and_weights_it_was_made_of(ops, keys):
     assert not made.takes(m, caches)
 
 
+@pytest.mark.parametrize("dtype,chains", [(torch.bfloat16, True), (torch.float32, True), (torch.float32, False)])
+def test_a_step_compares_a_chains_weights_once(ops, monkeypatch, dtype, chains):
+    """The host looks through the layers' weights and pages before a step's first launch, while the GPU waits: once a step."""
+    from llm_infrence_engine_amd.engine import ModelRunner, runner
+    from llm_infrence_engine_amd.parts.model import Model
+
+    looked, made, ran = [], [], []
+
+    class Chain:
+        def takes(self, model, caches):
+            looked.append(self)
+            return True
+
+        def forward(self, x, ctx, caches):
+            ran.append(self)
+            return x, None
+
+    def of(kind):
+        return classmethod(lambda cls, *args: made.append(kind) or (Chain() if chains and (kind == "float") == (dtype == torch.float32) else None))
+
+    monkeypatch.setattr(runner.DecodeChain, "of", of("decode"))
+    monkeypatch.setattr(runner.FloatLayers, "of", of("float"))
+    x = torch.zeros(1, 4)
+    layer = SimpleNamespace(forward=lambda x, pending, *a: pending, takes_sums=False, settles_writes=False)
+    model = SimpleNamespace(embedding=SimpleNamespace(forward=lambda ctx: x), pass_entry=None, layers=[layer], final_norm=None,
+                            spec=SimpleNamespace(order=[SimpleNamespace(layer=0, opens_pass=None)]), _settled=Model._settled)
+    model.forward = lambda ctx, caches: Model.forward_hidden(model, ctx, caches)[0]
+    r = ModelRunner.__new__(ModelRunner)
+    ctx = lambda: SimpleNamespace(decode_only=True, num_tokens=1, max_context_len=5, chain=None, state_slots=None)     # noqa: E731
+    r.model, r.graphs, r.chains = model, None, {}
+    r.manager = SimpleNamespace(has=lambda i: True, grow=lambda *a: None, computed=lambda i: 4, advance=lambda *a: None)
+    r.builder = SimpleNamespace(build=lambda entries: SimpleNamespace(ctx=ctx(), slots=[]))
+    r.caches = lambda rows, slots: [SimpleNamespace(kv=None, state=None)]
+    for _ in range(3):
+        r.step([SimpleNamespace(req_id=0, tokens=[1])])
+    assert len(looked) == (2 if chains else 0) and len(ran) == (3 if chains else 0)      # (not in the step that makes it)
+    assert made == (["decode"] if dtype == torch.bfloat16 else ["decode", "float"])
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("tokens", [[1, 1, 1], [1, 40, 3]])
 def test_float_layers_are_the_parts_one_by_one(ops, tokens):
