@@ -147,7 +147,7 @@ int ms_decode_chain(const void* attn, long long ld_attn, const void* w_o, float*
 // All layers of a 32-bit step by one call, with the kernels of this header (csrc/float_layers.hip); layers: records in host memory.
 int ms_float_layer_bytes();
 long long ms_float_layers_work(int n_tokens, int H, int num_heads, int num_kv_heads, int head_dim, int I);
-int ms_float_layers(const void* layers, int n_layers, float* x, float* work, const int* positions, const int* token_req,
+int ms_float_layers(const void* layers, int n_layers, float* x, float* work, long long work_floats, const int* positions, const int* token_req,
                     const int* slot_mapping, const int* block_table, int table_width, const int* table_rows, const int* n_live,
                     int n_tokens, int H, int I, int num_heads, int num_kv_heads, int head_dim, int page_size, long long num_pages,
                     int v_transposed, float scale, hipStream_t stream);

@@ -13,18 +13,37 @@ struct FloatLayer {
   float eps1, eps2;
 };
 
+// Where the pieces of the scratch begin, in floats, and where the last one ends.  Each on 256 bytes, as an allocation of its own
+// would be: which kernel a product takes goes by its rows' addresses, too.
+struct Pieces {
+  long long sum, h, qkv, heads, gate_up, act, end;
+};
+Pieces pieces_of(long long N, int H, int num_heads, int num_kv_heads, int head_dim, int I) {
+  auto behind = [](long long at, long long floats) { return at + (floats + 63) / 64 * 64; };
+  Pieces p;
+  p.sum = 0;
+  p.h = behind(p.sum, N * H);
+  p.qkv = behind(p.h, N * H);
+  p.heads = behind(p.qkv, N * (num_heads + 2 * num_kv_heads) * head_dim);
+  p.gate_up = behind(p.heads, N * num_heads * head_dim);
+  p.act = behind(p.gate_up, N * 2 * I);
+  p.end = behind(p.act, N * I);
+  return p;
+}
+
 }  // namespace
 
 extern "C" int ms_float_layer_bytes() { return (int)sizeof(FloatLayer); }
 
 // Floats of `work` for n_tokens tokens.
 extern "C" long long ms_float_layers_work(int n_tokens, int H, int num_heads, int num_kv_heads, int head_dim, int I) {
-  return (long long)n_tokens * (2ll * H + (2ll * num_heads + 2ll * num_kv_heads) * head_dim + 3ll * I);
+  return pieces_of(n_tokens, H, num_heads, num_kv_heads, head_dim, I).end;
 }
 
-// x float [N, H] in place, but for the last down projection, which is left in work's first [N, H] for whoever adds it.  w_gate_up's
-// rows interleaved, heads turned whole, pages as ms_rope_store has them; n_live may be null.
-extern "C" int ms_float_layers(const void* layers, int n_layers, float* x, float* work, const int* positions, const int* token_req,
+// x float [N, H] in place, but for the last down projection, which is left in work's first [N, H] for whoever adds it.  `work`:
+// work_floats floats, at least ms_float_layers_work.  w_gate_up's rows interleaved, heads turned whole, pages as ms_rope_store has
+// them; n_live may be null.
+extern "C" int ms_float_layers(const void* layers, int n_layers, float* x, float* work, long long work_floats, const int* positions, const int* token_req,
                                const int* slot_mapping, const int* block_table, int table_width, const int* table_rows,
                                const int* n_live, int n_tokens, int H, int I, int num_heads, int num_kv_heads, int head_dim,
                                int page_size, long long num_pages, int v_transposed, float scale, hipStream_t stream) {
@@ -34,7 +53,9 @@ extern "C" int ms_float_layers(const void* layers, int n_layers, float* x, float
     return MS_BAD_ARG;
   const long long N = n_tokens;
   const int Ko = num_heads * head_dim, Q = (num_heads + 2 * num_kv_heads) * head_dim;
-  float *sum = work, *h = sum + N * H, *qkv = h + N * H, *heads = qkv + N * Q, *gate_up = heads + N * Ko, *act = gate_up + N * 2 * I;
+  const Pieces at = pieces_of(N, H, num_heads, num_kv_heads, head_dim, I);
+  if (work_floats < at.end) return MS_BAD_ARG;
+  float *sum = work + at.sum, *h = work + at.h, *qkv = work + at.qkv, *heads = work + at.heads, *gate_up = work + at.gate_up, *act = work + at.act;
   auto product = [&](const float* a, const float* w, const float* bias, float* out, int n, int k) {
     return ms_gemm_generic(a, w, bias, out, n_tokens, n, k, k, k, n, MS_F32, MS_F32, 0, stream);
   };

@@ -32,7 +32,8 @@ _SIGNATURES = {
     "ms_decode_advance": [_c_ptr, _c_ptr, _c_ptr, _c_ptr, _c_ptr, _c_ptr, _c_ptr, _c_ptr, _c_ptr, _c_ptr, _c_int, _c_int, _c_int,
                           _c_int, _c_ptr],
     "ms_float_layer_bytes": [],
-    "ms_float_layers": [_c_ptr, _c_int, _c_ptr, _c_ptr, _c_ptr, _c_ptr, _c_ptr, _c_ptr, _c_int, _c_ptr, _c_ptr, _c_int, _c_int, _c_int,
+    "ms_float_layers_work": [_c_int] * 6,
+    "ms_float_layers": [_c_ptr, _c_int, _c_ptr, _c_ptr, _c_ll, _c_ptr, _c_ptr, _c_ptr, _c_ptr, _c_int, _c_ptr, _c_ptr, _c_int, _c_int, _c_int,
                         _c_int, _c_int, _c_int, _c_int, _c_ll, _c_int, _c_float, _c_ptr],
     "ms_decode_chain_workspace": [_c_int] * 7,
     "ms_decode_layer_bytes": [],
@@ -180,6 +181,8 @@ _SIGNATURES = {
                        _c_int, _c_int, _c_ptr],
 }
 
+_RETURNS_LL = ("ms_sample_workspace_bytes", "ms_float_layers_work")     # the others return an int
+
 _fn = {}
 
 
@@ -193,7 +196,7 @@ def _get(name):
             raise build.KernelLibraryError(
                 f"{name} is not in {build.library_path()}; the library is older than its sources, build it again") from e
         f.argtypes = _SIGNATURES[name]
-        f.restype = _c_int
+        f.restype = _c_ll if name in _RETURNS_LL else _c_int
         _fn[name] = f
     return f
 
@@ -1090,8 +1093,8 @@ def float_layers(records: bytes, n_layers: int, x: torch.Tensor, positions: torc
         if t is not None:
             _check(t, name, torch.int32)
     P, _, page_size, d = k_pages.shape
-    work = torch.empty(N * (2 * H + (2 * num_heads + 2 * num_kv_heads) * d + 3 * intermediate), dtype=torch.float32, device=x.device)
-    _call("ms_float_layers", records, n_layers, x.data_ptr(), work.data_ptr(), positions.data_ptr(), token_req.data_ptr(),
+    work = torch.empty(_get("ms_float_layers_work")(N, H, num_heads, num_kv_heads, d, intermediate), dtype=torch.float32, device=x.device)
+    _call("ms_float_layers", records, n_layers, x.data_ptr(), work.data_ptr(), work.numel(), positions.data_ptr(), token_req.data_ptr(),
           slot_mapping.data_ptr(), block_table.data_ptr(), block_table.shape[1], _ptr(table_rows), _ptr(n_live_tokens), N, H,
           intermediate, num_heads, num_kv_heads, d, page_size, P, int(v_transposed), float(scale), _stream())
     return work[:N * H].view(N, H)
@@ -1285,9 +1288,7 @@ def sample(logits: torch.Tensor, out: torch.Tensor, temperature: Optional[torch.
                         (draw_index, "draw_index", torch.int32)):
         if t is not None:
             _check(t, name, dt, (M,))
-    f = _get("ms_sample_workspace_bytes")
-    f.restype = _c_ll
-    work = torch.empty(int(f(M)), dtype=torch.uint8, device=logits.device)
+    work = torch.empty(int(_get("ms_sample_workspace_bytes")(M)), dtype=torch.uint8, device=logits.device)
     _call("ms_sample", logits.data_ptr(), V, M, V, temperature.data_ptr(), _ptr(top_k), _ptr(top_p), _ptr(seeds),
           _ptr(draw_index), out.data_ptr(), work.data_ptr(), int(use_top_k and top_k is not None),
           int(use_top_p and top_p is not None), _stream())

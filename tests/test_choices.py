@@ -365,3 +365,66 @@ def test_float_layers_are_the_parts_one_by_one(ops, tokens):
         assert isinstance(r.chains["float"], chain.FloatLayers) == whole
         got.append([anew] + out + [t.cpu() for pages in r.pools.pages for t in pages.values()])
     assert all(torch.equal(a, b) for a, b in zip(*got))
+
+
+def _small_model(dtype, seed=3, std=None, **sizes):
+    """A model of the plain parts on the GPU, with random weights: matrices of ``std`` (None: 1/8)."""
+    from llm_infrence_engine_amd.config import config_from_dict
+    from llm_infrence_engine_amd.parts.base import Runtime
+    from llm_infrence_engine_amd.parts.model import Model
+
+    cfg = config_from_dict(dict({"model_type": "qwen2", "vocab_size": 64, "rms_norm_eps": 1e-6, "rope_theta": 10000.0,
+                                 "tie_word_embeddings": True}, **sizes))
+    g = torch.Generator().manual_seed(seed)
+
+    class Weights:
+        def check(self, wanted, ignorable=()):
+            self.specs = {s.name: s for s in wanted}
+
+        def get(self, name):
+            s = self.specs[name]
+            w = torch.randn(s.shape, generator=g) * (std or 1 / 8)
+            return (1 + w if std and s.role == "norm" else w).cuda()
+
+        def close(self):
+            pass
+
+    model = Model(cfg.to_spec())
+    model.config = cfg
+    model.load(Weights(), Runtime(torch.device("cuda:0"), dtype))
+    return model
+
+
+def test_the_scratch_of_32_bit_layers_is_sized_in_one_place(ops):
+    """What the library carves up is what it says it needs, every piece from a boundary of 256 bytes on (the products look at
+    addresses), and a scratch that is too small is refused before anything is launched."""
+    need = lambda *sizes: ops._get("ms_float_layers_work")(*sizes)     # noqa: E731
+    N, H, nh, nkv, d, I = 3, 65, 4, 2, 16, 36
+    pieces = (N * H, N * H, N * (nh + 2 * nkv) * d, N * nh * d, N * 2 * I, N * I)
+    assert need(N, H, nh, nkv, d, I) == sum(-(-p // 64) * 64 for p in pieces)
+    assert need(100000, 8192, 64, 8, 128, 28672) > 1 << 31
+    there = torch.zeros(64).data_ptr()
+    call = lambda floats: ops._get("ms_float_layers")(there, 1, there, there, floats, there, there, there, there, 1, None, None, N, H, I,     # noqa: E731
+                                                      nh, nkv, d, 16, 8, 0, 0.25, None)
+    assert call(need(N, H, nh, nkv, d, I) - 1) == call(0) == 1
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("tokens", [[1], [1, 1, 1], [2, 7]])
+def test_float_layers_of_an_odd_width_are_the_parts_one_by_one(ops, tokens):
+    """The scratch's pieces lie where an allocation of their own would: a width that is no multiple of four leaves the other
+    products' kernels, and so their bits, as they are."""
+    from llm_infrence_engine_amd.engine import ModelRunner
+    from llm_infrence_engine_amd.engine.batch import StepEntry
+    from llm_infrence_engine_amd.parts import chain
+
+    model = _small_model(torch.float32, hidden_size=65, intermediate_size=132, num_hidden_layers=2, num_attention_heads=4,
+                         num_key_value_heads=2, head_dim=48, max_position_embeddings=64)
+    got = []
+    for whole in (True, False):
+        r = ModelRunner(model, 16, 24, 4, 64)
+        if not whole:
+            r.chains["float"] = None
+        got.append([r.step([StepEntry(i, [7 + i] * n, [n - 1]) for i, n in enumerate(tokens)]).cpu() for _ in range(3)])
+        assert isinstance(r.chains["float"], chain.FloatLayers) == whole
+    assert all(torch.equal(a, b) for a, b in zip(*got))
