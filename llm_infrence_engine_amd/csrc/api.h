@@ -125,7 +125,8 @@ int ms_gemm_skinny_norm(const float* x, long long ldx, const int* rows, const fl
 // The products between two attentions of a decode step as one kernel (csrc/decode_chain.hip): x += attn . w_o^T, the gated
 // feed-forward behind norm2 added to x, and (w_qkv not null) the next layer's norm1, q/k/v, rotation and cache store.  `workspace`:
 // ms_decode_chain_workspace bytes (0: sizes not taken), zeroed once, for one batch size and one stream at a time; the step's
-// launches number 0 .. launches - 1 in order.  With n_layers: for a whole step's layers in two launches, ms_decode_first (the
+// launches number 0 .. launches - 1 in order.  `told` (null: nobody): an int in host memory that becomes 1 where a launch was broken
+// off because what it waited for did not come; results are void from then on until the workspace is zeroed.  With n_layers: for a whole step's layers in two launches, ms_decode_first (the
 // first layer's norm, q/k/v, rotation, cache store) and ms_decode_layers (all the rest up to the last layer's down projection).
 int ms_decode_chain_workspace(int M, int H, int num_heads, int num_kv_heads, int head_dim, int I, int n_layers);
 int ms_decode_first(const float* x, long long ldx, const float* norm1, float eps1, const void* w_qkv, const float* b_qkv,
@@ -136,13 +137,14 @@ int ms_decode_layer_bytes();
 int ms_decode_layers(const void* layers, float* x, long long ldx, const int* positions, const int* slot_mapping,
                      const int* context_lens, const int* table, const int* table_rows, int table_width, float scale, int M, int H,
                      int I, int num_heads, int num_kv_heads, int head_dim, int page_size, int n_layers, void* workspace,
-                     hipStream_t stream);
+                     int* told, hipStream_t stream);
 void ms_decode_chain_limit(int limit);
+void ms_decode_chain_patience(int tries);
 int ms_decode_chain(const void* attn, long long ld_attn, const void* w_o, float* x, long long ldx, const float* norm2, float eps2,
                     const void* w_gate_up, const void* w_down, const float* norm1, float eps1, const void* w_qkv, const float* b_qkv,
                     const int* positions, const float* inv_freq, const int* slot_mapping, void* q_out, void* k_pages, void* v_pages,
                     int M, int H, int I, int num_heads, int num_kv_heads, int head_dim, int page_size, int v_transposed,
-                    void* workspace, int launch, int launches, hipStream_t stream);
+                    void* workspace, int* told, int launch, int launches, hipStream_t stream);
 
 // All layers of a 32-bit step by one call, with the kernels of this header (csrc/float_layers.hip); layers: records in host memory.
 int ms_float_layer_bytes();

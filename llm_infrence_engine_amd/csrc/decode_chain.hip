@@ -24,7 +24,9 @@
 // Waiting.  Blocks are dispatched in order, so those that a block waits for run already or will run as soon as there is
 // room; but other waiting kernels (another engine's, on another stream) may hold that room.  So no block waits for ever: one that has
 // polled `limit` times in vain gives its item up and ends, unless it is the only one that has given up: that one stays and
-// works off, as their inputs come in, the items that others gave up.  So a launch needs room for one block to end.
+// works off, as their inputs come in, the items that others gave up.  So a launch needs room for one block to end.  Words that never
+// come (a launch out of its turn left them out) end the one that stays, too: after `patience` tries in a row of which none got on, it
+// says so behind the list and to the host, and from then on nobody stays.
 //
 // A row's sums are the same whatever else is in the batch: k-step s belongs to wave s % 8, where it stands decides which lanes
 // hold its products, and lanes and waves are added in a fixed order.
@@ -47,7 +49,7 @@ constexpr int UO = 2, UF = 2;         // units of four rows to a block in o and 
 constexpr int HEAD = 64;              // dims of a head in WHOLE, two k-steps
 constexpr int SHARES = HEAD / 16;     // blocks of attention to a token and key/value head: each has all keys and 16 dims of the values
 constexpr int KEYS = 4;               // blocks of 32 keys to a wave: contexts up to 1,024
-constexpr int LIST = 32767;           // items that can be given up, the blocks of a launch
+constexpr int LIST = 32767;           // items that can be given up, the blocks of a launch (the first has no place: it stays)
 constexpr int MAX_LAUNCHES = 1024;    // of a step
 
 // What a kernel holds: one layer's chain (its attention before it, the next layer's after it, as kernels of their own), the front
@@ -68,7 +70,8 @@ struct ChainArgs {
   float* x;
   const int *positions, *slots, *contexts, *table, *table_rows;
   u64 *x1, *x2, *act, *heads, *qkv;   // words
-  unsigned *given_up;                 // how many items, then the items
+  unsigned *given_up;                 // how many items, then the items; [LIST]: not 0 if a launch was broken off
+  int *told;                          // that, in host memory (or null)
   unsigned *epoch;
   long long ld_attn, ldx;
   float inv_H, scale_log2;
@@ -77,7 +80,7 @@ struct ChainArgs {
   int gate_units, gate_more;          // units of four gate/up rows to a block of gate, and how many blocks have one more
   int per_head;                       // blocks of front to a head
   int launch, launches;
-  unsigned limit;
+  unsigned limit, patience;
 };
 
 template <typename T>
@@ -225,6 +228,7 @@ struct Shared {
   float part_ss[8][WAVES];              // [token]
   int late[3];                          // somebody gave up: waiting for the first word, for the others, for a phase before the one before
   int next, position;
+  unsigned in_vain;                     // tries in a row
   unsigned done[(LIST + 32) / 32];
 };
 
@@ -894,12 +898,16 @@ decode_chain_kernel(ChainArgs a) {
   if (blockIdx.x == 0 && threadIdx.x == 0) a.epoch[a.launch == 0 ? a.launches - 1 : a.launch - 1] += 1;
   if (run_item<G, UD, 6, MODE>(sh, blockIdx.x, tag, a.limit)) return;
   if constexpr (MODE != FIRST) {      // (which waits for nothing)
-    // given up: end, or stay if nobody has yet
+    // given up: end, or stay if nobody has yet (and no launch was broken off: then nothing is listed any more, either)
     if (threadIdx.x == 0) {
-      const unsigned before = __hip_atomic_fetch_add(a.given_up, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-      if (before > 0) __hip_atomic_store(a.given_up + before, blockIdx.x + 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      unsigned before = 1;
+      if (!__hip_atomic_load(a.given_up + LIST, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) {
+        before = __hip_atomic_fetch_add(a.given_up, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        if (before > 0) __hip_atomic_store(a.given_up + before, blockIdx.x + 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      }
       for (unsigned& d : sh.done) d = 0;
       sh.position = 0;
+      sh.in_vain = 0;
       sh.next = before > 0 ? -1 : (int)blockIdx.x;
     }
     __syncthreads();
@@ -907,10 +915,17 @@ decode_chain_kernel(ChainArgs a) {
       const bool ok = run_item<G, UD, 3, MODE>(sh, sh.next, tag, 64);
       __syncthreads();
       if (threadIdx.x == 0) {
-        if (ok) sh.done[sh.position / 32] |= 1u << (sh.position % 32);
-        sh.next = next_given_up(a.given_up, sh, (int)blockIdx.x);
+        if (ok) {
+          sh.done[sh.position / 32] |= 1u << (sh.position % 32);
+          sh.in_vain = 0;
+        }
+        sh.next = ++sh.in_vain > a.patience ? -1 : next_given_up(a.given_up, sh, (int)blockIdx.x);
       }
       __syncthreads();
+    }
+    if (threadIdx.x == 0 && sh.in_vain > a.patience) {      // (the list stays as it is: at most this launch's other blocks are on it)
+      __hip_atomic_store(a.given_up + LIST, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      if (a.told) __hip_atomic_store(a.told, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
     }
   }
 }
@@ -922,7 +937,8 @@ size_t heads_bytes(int M) { return round_up((size_t)WAVES * STEPS * 16 * M * 8);
 size_t qkv_bytes(int M, int heads) { return round_up((size_t)M * heads * (HEAD / 2) * 8); }
 constexpr size_t LIST_BYTES = 4 * (1 + LIST), EPOCH_BYTES = 4 * MAX_LAUNCHES;
 
-unsigned g_limit = 2048;   // looks of a waiting block, each about 0.8 us
+unsigned g_limit = 2048;         // looks of a waiting block, each about 0.8 us
+unsigned g_patience = 400000;    // tries of the block that stays, of 64 looks or more each: 20 s in which no block of the launch ended
 
 int down_units(int M, bool whole) { return M <= 2 && !whole ? 1 : 2; }
 
@@ -946,7 +962,7 @@ bool sizes_into(ChainArgs& a, int M, int H, int I, int nh, int nkv, int d, int n
   a.inv_H = 1.0f / (float)H;
   return (long long)a.n_layers * (a.n_attn + a.n_o + a.n_gate + a.n_down + a.n_front) <= LIST;
 }
-void workspace_into(ChainArgs& a, void* workspace) {
+void workspace_into(ChainArgs& a, void* workspace, int* told) {
   char* ws = (char*)workspace;
   a.given_up = (unsigned*)ws; ws += LIST_BYTES;
   a.epoch = (unsigned*)ws; ws += EPOCH_BYTES;
@@ -955,7 +971,9 @@ void workspace_into(ChainArgs& a, void* workspace) {
   a.act = (u64*)ws; ws += act_bytes(a.M);
   a.heads = (u64*)ws; ws += heads_bytes(a.M);
   a.qkv = (u64*)ws;
+  a.told = told;
   a.limit = g_limit;
+  a.patience = g_patience;
 }
 template <int MODE>
 int launch_chain(const ChainArgs& a, int blocks, hipStream_t stream) {
@@ -976,6 +994,8 @@ int shift_of(int page_size) { return page_size > 0 && (page_size & (page_size - 
 
 // Tests: how many times a waiting block looks before it gives its item up; 0 restores the choice.
 extern "C" void ms_decode_chain_limit(int limit) { g_limit = limit > 0 ? (unsigned)limit : 2048u; }
+// And how many tries in a row may be in vain before the block that stays breaks the launch off; 0 restores the choice.
+extern "C" void ms_decode_chain_patience(int tries) { g_patience = tries > 0 ? (unsigned)tries : 400000u; }
 
 // Bytes of a workspace, to be zeroed once and then left to launches of ONE batch size, one step after the other, 0 where the
 // kernels do not take the sizes: for ms_decode_chain (n_layers 0), or for ms_decode_first and ms_decode_layers of n_layers layers.
@@ -994,7 +1014,7 @@ extern "C" int ms_decode_chain(const void* attn, long long ld_attn, const void* 
                                const void* w_qkv, const float* b_qkv, const int* positions, const float* inv_freq,
                                const int* slot_mapping, void* q_out, void* k_pages, void* v_pages, int M, int H, int I,
                                int num_heads, int num_kv_heads, int head_dim, int page_size, int v_transposed, void* workspace,
-                               int launch, int launches, hipStream_t stream) {
+                               int* told, int launch, int launches, hipStream_t stream) {
   if (M <= 0) return MS_OK;
   ChainArgs a = {};
   if (!sizes_into(a, M, H, I, num_heads, num_kv_heads, head_dim, 0)) return MS_UNSUPPORTED;
@@ -1017,7 +1037,7 @@ extern "C" int ms_decode_chain(const void* attn, long long ld_attn, const void* 
   a.positions = positions; a.slots = slot_mapping; a.q_out = (bf16*)q_out;
   a.page_size = page_size; a.v_transposed = v_transposed;
   a.launch = launch; a.launches = launches;
-  workspace_into(a, workspace);
+  workspace_into(a, workspace, told);
   return launch_chain<CHAIN>(a, a.n_o + a.n_gate + a.n_down + a.n_front, stream);
 }
 
@@ -1039,7 +1059,7 @@ extern "C" int ms_decode_first(const float* x, long long ldx, const float* norm1
   a.positions = positions; a.slots = slot_mapping;
   a.page_size = page_size; a.page_shift = shift_of(page_size); a.v_transposed = 1;
   a.launch = 0; a.launches = 2;
-  workspace_into(a, workspace);
+  workspace_into(a, workspace, nullptr);
   return launch_chain<FIRST>(a, a.n_front, stream);
 }
 
@@ -1049,7 +1069,7 @@ extern "C" int ms_decode_layer_bytes() { return (int)sizeof(Layer); }
 extern "C" int ms_decode_layers(const void* layers, float* x, long long ldx, const int* positions, const int* slot_mapping,
                                 const int* context_lens, const int* table, const int* table_rows, int table_width, float scale,
                                 int M, int H, int I, int num_heads, int num_kv_heads, int head_dim, int page_size, int n_layers,
-                                void* workspace, hipStream_t stream) {
+                                void* workspace, int* told, hipStream_t stream) {
   if (M <= 0) return MS_OK;
   ChainArgs a = {};
   if (n_layers < 1 || !sizes_into(a, M, H, I, num_heads, num_kv_heads, head_dim, n_layers)) return MS_UNSUPPORTED;
@@ -1062,6 +1082,6 @@ extern "C" int ms_decode_layers(const void* layers, float* x, long long ldx, con
   a.scale_log2 = scale * 1.4426950408889634f;
   a.page_size = page_size; a.page_shift = shift_of(page_size); a.v_transposed = 1;
   a.launch = 1; a.launches = 2;
-  workspace_into(a, workspace);
+  workspace_into(a, workspace, told);
   return launch_chain<WHOLE>(a, n_layers * (a.n_attn + a.n_o + a.n_gate + a.n_down + a.n_front) - a.n_front, stream);
 }

@@ -206,6 +206,7 @@ class Engine:
                 chosen = greedy.tolist()       # the captured graph has already taken the argmax
             else:
                 chosen = self.sampler.sample(logits, rows)
+            self.runner.check()
             useful = self.scheduler.commit(sched, chosen)
         n_decode = sum(1 for s in sched if s.count == 1 and s.start > 0)
         n_prefill = sum(s.count for s in sched) - n_decode

@@ -96,6 +96,7 @@ class StepGraphs:
         self.buckets: Dict[tuple, _Bucket] = {}            # decode: (rows, long contexts, steps)
         self.portion_buckets: Dict[int, _Bucket] = {}      # steps with portions: tokens
         self.pool = None   # one memory pool for all graphs: they never run at the same time
+        self.chain = None  # of the last step, if it had one
         # what launching costs the host: seconds spent filling the buffers and enqueuing, and launches so far
         # (the reference separates a launch-bound from a GPU-bound step the same way, benchmarks/diag_gpu_launch.py:1-8)
         self.enqueue_seconds = 0.0
@@ -250,6 +251,9 @@ class StepGraphs:
         bk.buf.wait_until_sent()
         self.builder.write(d, bk.layout, bk.buf.np)
         bk.buf.send()
+        self.chain = bk.chain
+        if bk.chain is not None:
+            bk.chain.ready()
         bk.graph.replay()
         return d
 

@@ -43,6 +43,7 @@ class ModelRunner:
         # for steps launched kernel by kernel: (tokens, long contexts) -> DecodeChain of steps of single tokens, "float" -> FloatLayers;
         # None where there is none
         self.chains = {}
+        self.chain = None      # of the last step, if it had one
         self.graphs = None
         # a part that cannot be captured (it walks the requests on the host, as a mixer with state usually does)
         # keeps the whole model out of graphs
@@ -103,10 +104,19 @@ class ModelRunner:
                 built.ctx.chain = self._chain(key, caches, lambda: DecodeChain.of(self.model, built.ctx, caches))
             if built.ctx.chain is None:
                 built.ctx.chain = self._chain("float", caches, lambda: FloatLayers.of(self.model, caches))
+            self.chain = built.ctx.chain
             logits = self.model.forward(built.ctx, caches)
+        if kind is not None:
+            self.chain = self.graphs.chain
         for e in entries:
             m.advance(e.req_id, m.computed(e.req_id) + len(e.tokens))
         return logits
+
+    def check(self) -> None:
+        """To be asked when the last step's results have come: raises if they are void (``DecodeChain.check``).  The next step
+        asks, too, before it is launched."""
+        if self.chain is not None:
+            self.chain.check()
 
     def _chain(self, key, caches, make):
         """What runs the layers of steps like ``key``, made once and again when weights or pages are others."""
@@ -129,6 +139,8 @@ class ModelRunner:
             m.grow(e.req_id, m.computed(e.req_id) + steps)
         _, tokens = self.graphs.run(entries, steps, sampling)
         out = tokens.tolist()
+        self.chain = self.graphs.chain
+        self.check()
         for e in entries:
             m.advance(e.req_id, m.computed(e.req_id) + steps)
         self.greedy_tokens = None

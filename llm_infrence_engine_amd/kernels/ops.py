@@ -40,11 +40,12 @@ _SIGNATURES = {
     "ms_decode_first": [_c_ptr, _c_ll, _c_ptr, _c_float, _c_ptr, _c_ptr, _c_ptr, _c_ptr, _c_ptr, _c_ptr, _c_ptr, _c_int, _c_int,
                         _c_int, _c_int, _c_int, _c_int, _c_int, _c_int, _c_ptr, _c_ptr],
     "ms_decode_layers": [_c_ptr, _c_ptr, _c_ll, _c_ptr, _c_ptr, _c_ptr, _c_ptr, _c_ptr, _c_int, _c_float, _c_int, _c_int, _c_int,
-                         _c_int, _c_int, _c_int, _c_int, _c_int, _c_ptr, _c_ptr],
+                         _c_int, _c_int, _c_int, _c_int, _c_int, _c_ptr, _c_ptr, _c_ptr],
     "ms_decode_chain_limit": [_c_int],
+    "ms_decode_chain_patience": [_c_int],
     "ms_decode_chain": [_c_ptr, _c_ll, _c_ptr, _c_ptr, _c_ll, _c_ptr, _c_float, _c_ptr, _c_ptr, _c_ptr, _c_float, _c_ptr, _c_ptr,
                         _c_ptr, _c_ptr, _c_ptr, _c_ptr, _c_ptr, _c_ptr, _c_int, _c_int, _c_int, _c_int, _c_int, _c_int, _c_int,
-                        _c_int, _c_ptr, _c_int, _c_int, _c_ptr],
+                        _c_int, _c_ptr, _c_ptr, _c_int, _c_int, _c_ptr],
     "ms_max_cache_groups": [],
     "ms_table_update": [_c_ptr, _c_ptr, _c_ptr, _c_ptr, _c_int, _c_int, _c_ll, _c_ptr],
     "ms_zero_rows": [_c_ptr, _c_ll, _c_ptr, _c_ptr, _c_int, _c_ptr],
@@ -991,9 +992,9 @@ def decode_first(x: torch.Tensor, norm_weight: torch.Tensor, eps: float, w_qkv: 
 def decode_layers(table: torch.Tensor, x: torch.Tensor, positions: torch.Tensor, slot_mapping: torch.Tensor,
                   context_lens: torch.Tensor, block_table: torch.Tensor, table_rows: Optional[torch.Tensor], scale: float,
                   num_heads: int, num_kv_heads: int, head_dim: int, intermediate: int, page_size: int, n_layers: int,
-                  workspace: torch.Tensor) -> torch.Tensor:
+                  workspace: torch.Tensor, told: Optional[torch.Tensor] = None) -> torch.Tensor:
     """Every layer of a step of single tokens from the first one's attention on, behind ``decode_first``: x in place.
-    ``table``: ``decode_layer_table``; contexts of at most ``DECODE_KEYS`` keys."""
+    ``table``: ``decode_layer_table``; contexts of at most ``DECODE_KEYS`` keys; ``told``: as ``decode_chain`` has it."""
     _check(x, "x", torch.float32)
     M, H = x.shape
     _check(table, "table", torch.uint8, (n_layers * _get("ms_decode_layer_bytes")(),))
@@ -1007,22 +1008,33 @@ def decode_layers(table: torch.Tensor, x: torch.Tensor, positions: torch.Tensor,
         raise ValueError("the workspace is too small")
     _call("ms_decode_layers", table.data_ptr(), x.data_ptr(), H, positions.data_ptr(), slot_mapping.data_ptr(),
           context_lens.data_ptr(), block_table.data_ptr(), _ptr(table_rows), block_table.shape[1], float(scale), M, H,
-          intermediate, num_heads, num_kv_heads, head_dim, page_size, n_layers, workspace.data_ptr(), _stream())
+          intermediate, num_heads, num_kv_heads, head_dim, page_size, n_layers, workspace.data_ptr(), _told(told), _stream())
     return x
 
 
-def decode_chain_limit(looks: int) -> None:
-    """Tests: how often a waiting block of ``decode_chain`` looks before it gives its item up (0: the kernel's own choice)."""
+def _told(told: Optional[torch.Tensor]):
+    if told is not None and (told.dtype != torch.int32 or told.numel() < 1 or not told.is_pinned()):
+        raise ValueError("told must be an int32 tensor in pinned host memory")
+    return _ptr(told)
+
+
+def decode_chain_limit(looks: int, tries: int = 0) -> None:
+    """Tests: how often a waiting block of ``decode_chain`` looks before it gives its item up, and how many tries of the one that
+    stays may be in vain before it breaks the launch off (0: the kernel's own choice)."""
     _get("ms_decode_chain_limit")(looks)
+    _get("ms_decode_chain_patience")(tries)
 
 
 def decode_chain(attn: torch.Tensor, w_o: torch.Tensor, x: torch.Tensor, norm2: torch.Tensor, eps2: float,
                  w_gate_up: torch.Tensor, w_down: torch.Tensor, num_heads: int, num_kv_heads: int, head_dim: int,
-                 workspace: torch.Tensor, launch: int, launches: int, front=None) -> Optional[torch.Tensor]:
+                 workspace: torch.Tensor, launch: int, launches: int, front=None,
+                 told: Optional[torch.Tensor] = None) -> Optional[torch.Tensor]:
     """x += attn @ w_o.T; x += (silu(g) * u) @ w_down.T for g, u = rms_norm(x, norm2) @ w_gate_up.T (interleaved rows), in
     one kernel.  ``front``: the arguments (norm weight, eps, w_qkv, bias, positions, inv_freq, slot_mapping, k_pages, v_pages,
     v_transposed) of ``qkv_rope_store`` for the new x, which then runs in the same kernel; returns its q.  ``workspace``: uint8,
-    zeroed once, of one batch size; ``launch`` numbers the step's chains 0 .. launches - 1, in order, one stream at a time."""
+    zeroed once, of one batch size; ``launch`` numbers the step's chains 0 .. launches - 1, in order, one stream at a time.
+    ``told``: int32 [1] in pinned host memory, 0, which becomes 1 if the launch waited in vain for what it needs and was broken
+    off: results are void from then on, until the workspace is zeroed."""
     _check(attn, "attn", torch.bfloat16)
     _check(x, "x", torch.float32)
     M, H = x.shape
@@ -1055,7 +1067,7 @@ def decode_chain(attn: torch.Tensor, w_o: torch.Tensor, x: torch.Tensor, norm2: 
                 slot_mapping.data_ptr(), q.data_ptr(), k_pages.data_ptr(), v_pages.data_ptr())
     _call("ms_decode_chain", attn.data_ptr(), attn.shape[1], w_o.data_ptr(), x.data_ptr(), H, norm2.data_ptr(), float(eps2),
           w_gate_up.data_ptr(), w_down.data_ptr(), *tail, M, H, I, num_heads, num_kv_heads, head_dim, page_size,
-          int(v_transposed), workspace.data_ptr(), launch, launches, _stream())
+          int(v_transposed), workspace.data_ptr(), _told(told), launch, launches, _stream())
     return q
 
 

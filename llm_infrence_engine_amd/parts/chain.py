@@ -145,6 +145,9 @@ class FloatLayers:
         return (len(caches) == len(self.layers) and _own_pages(caches, torch.float32) and self.addresses.hold(model, caches)
                 and all(c.kv.slot_mapping is caches[0].kv.slot_mapping for c in caches))
 
+    def check(self) -> None:
+        """(Its kernels wait for nothing.)"""
+
     def forward(self, x, ctx, caches):
         nh, nkv, _, _, I = self.sizes
         kv = caches[0].kv
@@ -161,7 +164,11 @@ class DecodeChain:
         self.layers = [model.layers[run.layer] for run in model.spec.order]
         self.workspace = torch.zeros(n_bytes, dtype=torch.uint8, device=model.rt.device)
         self.table, self.addresses = None, _Addresses(model, caches)
-        self.broken_off = False      # a step ended with an exception between its launches
+        self.told = torch.zeros(1, dtype=torch.int32)      # not 0: a launch waited in vain (the GPU writes it)
+        if self.workspace.is_cuda:
+            self.told = self.told.pin_memory()
+        self._told = self.told.numpy()
+        self.broken_off = False      # a step ended with an exception between its launches, or a launch waited in vain
 
     @classmethod
     def of(cls, model, ctx, caches) -> Optional["DecodeChain"]:
@@ -216,10 +223,24 @@ class DecodeChain:
             return False
         return self.addresses.hold_weights(model) if self.table is None else self.addresses.hold(model, caches)
 
+    def check(self) -> None:
+        """Raises if a step's launch waited in vain, on the GPU, for what another one should have left: its results are void.  To
+        be asked when a step's results have come."""
+        if self._told[0]:
+            self._told[0], self.broken_off = 0, True
+            raise RuntimeError("a decode step's launch waited in vain for its inputs and was broken off; the step's results are void")
+
+    def ready(self) -> None:
+        """Before a step's first launch, also a replayed one: its launches count each other up, so behind a step that did not run
+        to its end they start over."""
+        self.check()
+        if self.broken_off:
+            self.workspace.zero_()
+            self.broken_off = False
+
     def forward(self, x, ctx, caches):
         """All runs of the order on the embedded tokens ``x`` [N, H], in place; returns x and what is left to add to it (nothing)."""
-        if self.broken_off:          # its launches did not count each other up: start over
-            self.workspace.zero_()
+        self.ready()
         self.broken_off = True
         (self._layer_by_layer if self.table is None else self._whole)(x, ctx, caches)
         self.broken_off = False
@@ -232,7 +253,7 @@ class DecodeChain:
         ops.decode_first(x, norm.weight, norm.eps, m.w_qkv, m.b_qkv, ctx.positions, m.position.inv_freq, kv.slot_mapping,
                          kv.k_pages, kv.v_pages, nh, nkv, d, I, self.runs, self.workspace)
         ops.decode_layers(self.table, x, ctx.positions, kv.slot_mapping, ctx.context_lens, kv.block_table, kv.table_rows, m.scale,
-                          nh, nkv, d, I, kv.k_pages.shape[2], self.runs, self.workspace)
+                          nh, nkv, d, I, kv.k_pages.shape[2], self.runs, self.workspace, self.told)
 
     def _layer_by_layer(self, x, ctx, caches):
         nh, nkv, d, _, _ = self.sizes
@@ -247,4 +268,4 @@ class DecodeChain:
                 front = (then.mixer_norm.weight, then.mixer_norm.eps, then.mixer.w_qkv, then.mixer.b_qkv, ctx.positions,
                          then.mixer.position.inv_freq, kv.slot_mapping, kv.k_pages, kv.v_pages, kv.v_transposed)
             q = ops.decode_chain(out, m.w_o, x, layer.feed_forward_norm.weight, layer.feed_forward_norm.eps, f.w_gate_up,
-                                 f.w_down, nh, nkv, d, self.workspace, i, self.runs, front)
+                                 f.w_down, nh, nkv, d, self.workspace, i, self.runs, front, self.told)

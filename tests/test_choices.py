@@ -280,6 +280,43 @@ def test_a_chain_holds_for_the_layers_and_weights_it_was_made_of(ops, keys):
     assert not made.takes(m, caches)
 
 
+@pytest.mark.parametrize("keys", [64, 2000])
+def test_a_launch_that_waited_in_vain_is_an_error_and_the_next_step_starts_over(ops, keys):
+    """What the GPU writes where a launch was broken off is seen when the step's results have come, or before the next launch,
+    replayed or not; once: the workspace is zeroed for the step after it."""
+    from llm_infrence_engine_amd.engine import ModelRunner
+    from llm_infrence_engine_amd.engine.graph import StepGraphs
+
+    m, b, caches, of = _decode_stand_in(ops, keys)
+    made, r = of(), ModelRunner.__new__(ModelRunner)
+    r.chain = made
+    r.check()
+    made.told[0] = 1
+    made.workspace[:9] = 7
+    with pytest.raises(RuntimeError, match="void"):
+        r.check()
+    r.check()
+    made.ready()
+    assert not made.workspace.any() and not made.broken_off
+
+    replays = []
+    g = StepGraphs.__new__(StepGraphs)
+    g.manager = SimpleNamespace(pending_updates=lambda: 0)
+    g.builder = SimpleNamespace(describe=lambda *a: SimpleNamespace(), write=lambda *a: None)
+    bk = SimpleNamespace(layout=SimpleNamespace(n_updates=1), chain=made, graph=SimpleNamespace(replay=lambda: replays.append(made.workspace.any().item())),
+                         buf=SimpleNamespace(wait_until_sent=lambda: None, send=lambda: None, np=None))
+    g._fill_and_replay(bk, [], 1)
+    assert g.chain is made
+    made.told[0] = 1
+    made.workspace[:9] = 7
+    with pytest.raises(RuntimeError, match="void"):
+        g._fill_and_replay(bk, [], 1)
+    g._fill_and_replay(bk, [], 1)
+    assert replays == [False, False]
+    r.chain = None
+    r.check()
+
+
 @pytest.mark.parametrize("dtype,chains", [(torch.bfloat16, True), (torch.float32, True), (torch.float32, False)])
 def test_a_step_compares_a_chains_weights_once(ops, monkeypatch, dtype, chains):
     """The host looks through the layers' weights and pages before a step's first launch, while the GPU waits: once a step."""

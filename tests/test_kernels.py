@@ -2076,6 +2076,53 @@ def test_decode_layers(ops, H, I, nh, nkv, page_size, contexts, limit):
                    for a, b in zip(got, run(0)))
 
 
+def test_a_launch_whose_inputs_never_come_ends(ops):
+    """All layers without the launch that goes before them, with the library's own bounds made short: the blocks give up, the one
+    that stays stops trying, says so behind the list and to the host, and a launch after it ends, too, with nobody staying.
+    Zeroed, the workspace is as good as new."""
+    M, H, I, nh, nkv, d, L, page_size = 2, 96, 64, 4, 2, 64, 2, 16
+    g = torch.Generator().manual_seed(11)
+    n, eps = nh + 2 * nkv, 1e-6
+    w = lambda *shape: (torch.randn(*shape, generator=g) / 8).bfloat16().to(DEV)     # noqa: E731
+    ones, inv_freq = torch.ones(H, device=DEV), torch.ones(d // 2, device=DEV)
+    kv = [torch.zeros(4, nkv, page_size, d, dtype=torch.bfloat16, device=DEV) for _ in range(2 * L)]
+    w_qkv = w(n * d, H)
+    one = dict(w_o=w(H, nh * d), w_gate_up=w(2 * I, H), w_down=w(H, I), norm2=ones, eps2=eps)
+    recs = [dict(one, k_pages=kv[2 * i], v_pages=kv[2 * i + 1].transpose(2, 3).contiguous()) for i in range(L)]
+    recs[0].update(w_front=w_qkv, norm1=ones, eps1=eps, b_front=None, inv_freq=inv_freq, front_k=recs[1]["k_pages"], front_v=recs[1]["v_pages"])
+    table = ops.decode_layer_table(recs, DEV)
+    ints = lambda *v: torch.tensor(v, dtype=torch.int32, device=DEV)     # noqa: E731
+    pos, slots, lens, blocks = ints(3, 0), ints(16 + 3, 32), ints(4, 1), ints(1, 2).view(2, 1)
+    x0 = torch.randn(M, H, generator=g).to(DEV)
+    new = lambda: torch.zeros(ops.decode_chain_workspace(M, H, nh, nkv, d, I, L), dtype=torch.uint8, device=DEV)     # noqa: E731
+    told = torch.zeros(1, dtype=torch.int32).pin_memory()
+
+    def step(ws):
+        x = x0.clone()
+        ops.decode_first(x, ones, eps, w_qkv, None, pos, inv_freq, slots, recs[0]["k_pages"], recs[0]["v_pages"], nh, nkv, d, I, L, ws)
+        return ops.decode_layers(table, x, pos, slots, lens, blocks, None, 0.125, nh, nkv, d, I, page_size, L, ws, told)
+
+    want, ws = step(new()), new()
+    x = x0.clone()
+    ops.decode_chain_limit(1, 2)
+    try:
+        for _ in range(2):
+            ops._call("ms_decode_layers", table.data_ptr(), x.data_ptr(), H, pos.data_ptr(), slots.data_ptr(), lens.data_ptr(), blocks.data_ptr(),
+                      None, 1, 0.125, M, H, I, nh, nkv, d, page_size, L, ws.data_ptr(), told.data_ptr(), ops._stream())
+            torch.cuda.synchronize()
+            words = ws[:4 * 32768].view(torch.int32)
+            assert told[0] == 1 and words[32767] == 1 and 1 < words[0] <= 32767
+            listed = int(words[0])
+            assert (words[1:listed] > 0).all() and not words[listed:32767].any()
+    finally:
+        ops.decode_chain_limit(0)
+    told.zero_()
+    ws.zero_()
+    assert torch.equal(step(ws), want) and told[0] == 0 and not ws[:4 * 32768].any()
+    with pytest.raises(ValueError, match="pinned"):
+        ops.decode_layers(table, x, pos, slots, lens, blocks, None, 0.125, nh, nkv, d, I, page_size, L, ws, torch.zeros(1, dtype=torch.int32))
+
+
 def test_decode_chain_refuses_what_it_cannot_take(ops):
     for sizes in [(9, 896, 14, 2, 64, 4864), (0, 896, 14, 2, 64, 4864), (1, 1056, 14, 2, 64, 4864), (1, 896, 17, 1, 64, 4864),
                   (1, 896, 14, 2, 64, 6176), (1, 896, 14, 2, 64, 4880), (1, 880, 14, 2, 64, 4864), (1, 896, 14, 2, 60, 4864)]:
