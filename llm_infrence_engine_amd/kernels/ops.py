@@ -950,6 +950,32 @@ def decode_chain_workspace(n_tokens: int, hidden: int, num_heads: int, num_kv_he
     return _get("ms_decode_chain_workspace")(n_tokens, hidden, num_heads, num_kv_heads, head_dim, intermediate, n_layers)
 
 
+class _Turn:
+    """Which launch is due on a workspace: the launches of a step leave words for each other, numbered by how many have run, so one
+    out of its turn or of other sizes would wait for words that never come.  Kept on the workspace tensor itself."""
+
+    def __init__(self, workspace: torch.Tensor, sizes: tuple, launch: int, launches: int):
+        self.workspace, self.after = (workspace if sizes[0] else None), (sizes, (launch + 1) % launches)
+        if self.workspace is None:      # no tokens, no launch
+            return
+        was, due = getattr(workspace, "chain_turn", (sizes, 0))
+        if was != sizes:
+            raise ValueError("the workspace belongs to launches of other sizes (decode_chain_start_over frees it)")
+        if launch != due:
+            raise ValueError(f"launch {launch} of a step's {launches} is out of its turn: {due} is due on this workspace")
+
+    def over(self) -> None:
+        if self.workspace is not None:
+            self.workspace.chain_turn = self.after
+
+
+def decode_chain_start_over(workspace: torch.Tensor) -> None:
+    """Makes a workspace new again, for launches of any sizes: behind a step that did not run to its end."""
+    workspace.zero_()
+    if hasattr(workspace, "chain_turn"):
+        del workspace.chain_turn
+
+
 DECODE_KEYS = 1024      # keys of a context, with the step's own, that ``decode_layers`` reads at most
 
 
@@ -984,9 +1010,11 @@ def decode_first(x: torch.Tensor, norm_weight: torch.Tensor, eps: float, w_qkv: 
     _check(workspace, "workspace", torch.uint8)
     if workspace.numel() < decode_chain_workspace(M, H, num_heads, num_kv_heads, head_dim, intermediate, n_layers):
         raise ValueError("the workspace is too small")
+    turn = _Turn(workspace, (M, H, num_heads, num_kv_heads, head_dim, intermediate, "layers", n_layers), 0, 2)
     _call("ms_decode_first", x.data_ptr(), H, norm_weight.data_ptr(), float(eps), w_qkv.data_ptr(), _ptr(bias),
           positions.data_ptr(), inv_freq.data_ptr(), slot_mapping.data_ptr(), k_pages.data_ptr(), v_pages.data_ptr(), M, H,
           intermediate, num_heads, num_kv_heads, head_dim, k_pages.shape[2], n_layers, workspace.data_ptr(), _stream())
+    turn.over()
 
 
 def decode_layers(table: torch.Tensor, x: torch.Tensor, positions: torch.Tensor, slot_mapping: torch.Tensor,
@@ -1006,9 +1034,11 @@ def decode_layers(table: torch.Tensor, x: torch.Tensor, positions: torch.Tensor,
     _check(workspace, "workspace", torch.uint8)
     if workspace.numel() < decode_chain_workspace(M, H, num_heads, num_kv_heads, head_dim, intermediate, n_layers):
         raise ValueError("the workspace is too small")
+    turn = _Turn(workspace, (M, H, num_heads, num_kv_heads, head_dim, intermediate, "layers", n_layers), 1, 2)
     _call("ms_decode_layers", table.data_ptr(), x.data_ptr(), H, positions.data_ptr(), slot_mapping.data_ptr(),
           context_lens.data_ptr(), block_table.data_ptr(), _ptr(table_rows), block_table.shape[1], float(scale), M, H,
           intermediate, num_heads, num_kv_heads, head_dim, page_size, n_layers, workspace.data_ptr(), _told(told), _stream())
+    turn.over()
     return x
 
 
@@ -1065,9 +1095,11 @@ def decode_chain(attn: torch.Tensor, w_o: torch.Tensor, x: torch.Tensor, norm2: 
         page_size = k_pages.shape[2]
         tail = (norm1.data_ptr(), float(eps1), w_qkv.data_ptr(), _ptr(bias), positions.data_ptr(), inv_freq.data_ptr(),
                 slot_mapping.data_ptr(), q.data_ptr(), k_pages.data_ptr(), v_pages.data_ptr())
+    turn = _Turn(workspace, (M, H, num_heads, num_kv_heads, head_dim, I, "chains", launches), launch, launches)
     _call("ms_decode_chain", attn.data_ptr(), attn.shape[1], w_o.data_ptr(), x.data_ptr(), H, norm2.data_ptr(), float(eps2),
           w_gate_up.data_ptr(), w_down.data_ptr(), *tail, M, H, I, num_heads, num_kv_heads, head_dim, page_size,
           int(v_transposed), workspace.data_ptr(), _told(told), launch, launches, _stream())
+    turn.over()
     return q
 
 

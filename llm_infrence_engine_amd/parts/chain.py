@@ -235,7 +235,7 @@ class DecodeChain:
         to its end they start over."""
         self.check()
         if self.broken_off:
-            self.workspace.zero_()
+            ops.decode_chain_start_over(self.workspace)
             self.broken_off = False
 
     def forward(self, x, ctx, caches):

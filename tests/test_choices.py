@@ -280,6 +280,82 @@ def test_a_chain_holds_for_the_layers_and_weights_it_was_made_of(ops, keys):
     assert not made.takes(m, caches)
 
 
+def test_a_chains_launches_are_refused_out_of_their_turn(ops, monkeypatch):
+    """A launch waits for words of the one before it in the step, and their numbers go by how many have run: the next one due on a
+    workspace, of the same sizes, or none.  A launch that was refused does not count; a workspace that starts over takes any."""
+    launched = []
+
+    def call(name, *args):
+        if name == broken[0]:
+            raise RuntimeError("refused")
+        launched.append(name)
+
+    broken = [None]
+    monkeypatch.setattr(ops, "_check", lambda *args, **kw: None)
+    monkeypatch.setattr(ops, "_call", call)
+    monkeypatch.setattr(ops, "_stream", lambda: 0)
+    bf = dict(dtype=torch.bfloat16)
+
+    def args(M, H=64, I=64, nh=2, nkv=1, d=64):
+        return dict(x=torch.zeros(M, H), norm=torch.ones(H), w_qkv=torch.zeros((nh + 2 * nkv) * d, H, **bf), pos=torch.zeros(M, dtype=torch.int32),
+                    f=torch.ones(d // 2), k=torch.zeros(2, nkv, 16, d, **bf), v=torch.zeros(2, nkv, d, 16, **bf), attn=torch.zeros(M, nh * d, **bf),
+                    w_o=torch.zeros(H, nh * d, **bf), w_gu=torch.zeros(2 * I, H, **bf), w_down=torch.zeros(H, I, **bf), table=torch.zeros(M, 4, dtype=torch.int32),
+                    sizes=(nh, nkv, d, I))
+
+    def first(ws, M=2, L=3):
+        a = args(M)
+        ops.decode_first(a["x"], a["norm"], 1e-6, a["w_qkv"], None, a["pos"], a["f"], a["pos"], a["k"], a["v"], *a["sizes"], L, ws)
+
+    def layers(ws, M=2, L=3):
+        a = args(M)
+        records = torch.zeros(L * ops._get("ms_decode_layer_bytes")(), dtype=torch.uint8)
+        ops.decode_layers(records, a["x"], a["pos"], a["pos"], a["pos"], a["table"], None, 1.0, *a["sizes"], 16, L, ws)
+
+    def chain(ws, launch, launches=3, M=2):
+        a = args(M)
+        ops.decode_chain(a["attn"], a["w_o"], a["x"], a["norm"], 1e-6, a["w_gu"], a["w_down"], *a["sizes"][:3], ws, launch, launches)
+
+    def refused(run, *which, **sizes):
+        n = len(launched)
+        with pytest.raises(ValueError, match="turn|sizes"):
+            run(*which, **sizes)
+        assert len(launched) == n
+
+    new = lambda: torch.zeros(ops.decode_chain_workspace(8, 64, 2, 1, 64, 64, 8), dtype=torch.uint8)     # noqa: E731
+    ws = new()
+    refused(layers, ws)
+    for _ in range(3):
+        first(ws)
+        refused(first, ws)
+        for other in (dict(M=3), dict(L=4)):
+            refused(layers, ws, **other)
+        layers(ws)
+        refused(layers, ws)
+        refused(first, ws, M=1)
+        refused(chain, ws, 0)
+    first(ws)
+    broken[0] = "ms_decode_layers"
+    with pytest.raises(RuntimeError, match="refused"):
+        layers(ws)
+    broken[0] = None
+    layers(ws)
+    first(ws)
+    ws[5] = 1
+    ops.decode_chain_start_over(ws)
+    assert not ws.any()
+    first(ws, M=5, L=2)
+
+    ws = new()
+    refused(chain, ws, 1)
+    for _ in range(2):
+        for i in range(3):
+            chain(ws, i)
+            refused(chain, ws, i)
+            refused(chain, ws, (i + 1) % 3, launches=4)
+            refused(chain, ws, (i + 1) % 3, M=1)
+    assert launched.count("ms_decode_chain") == 6
+
+
 @pytest.mark.parametrize("keys", [64, 2000])
 def test_a_launch_that_waited_in_vain_is_an_error_and_the_next_step_starts_over(ops, keys):
     """What the GPU writes where a launch was broken off is seen when the step's results have come, or before the next launch,
