@@ -1020,9 +1020,10 @@ def decode_first(x: torch.Tensor, norm_weight: torch.Tensor, eps: float, w_qkv: 
 def decode_layers(table: torch.Tensor, x: torch.Tensor, positions: torch.Tensor, slot_mapping: torch.Tensor,
                   context_lens: torch.Tensor, block_table: torch.Tensor, table_rows: Optional[torch.Tensor], scale: float,
                   num_heads: int, num_kv_heads: int, head_dim: int, intermediate: int, page_size: int, n_layers: int,
-                  workspace: torch.Tensor, told: Optional[torch.Tensor] = None) -> torch.Tensor:
+                  workspace: torch.Tensor, told: Optional[torch.Tensor] = None, max_context_len: Optional[int] = None) -> torch.Tensor:
     """Every layer of a step of single tokens from the first one's attention on, behind ``decode_first``: x in place.
-    ``table``: ``decode_layer_table``; contexts of at most ``DECODE_KEYS`` keys; ``told``: as ``decode_chain`` has it."""
+    ``table``: ``decode_layer_table``; ``told``: as ``decode_chain`` has it.  Contexts hold at most ``DECODE_KEYS`` keys;
+    ``max_context_len``: a bound of theirs (None: they are read, which waits for the GPU)."""
     _check(x, "x", torch.float32)
     M, H = x.shape
     _check(table, "table", torch.uint8, (n_layers * _get("ms_decode_layer_bytes")(),))
@@ -1034,6 +1035,10 @@ def decode_layers(table: torch.Tensor, x: torch.Tensor, positions: torch.Tensor,
     _check(workspace, "workspace", torch.uint8)
     if workspace.numel() < decode_chain_workspace(M, H, num_heads, num_kv_heads, head_dim, intermediate, n_layers):
         raise ValueError("the workspace is too small")
+    if max_context_len is None:
+        max_context_len = int(context_lens.max()) if M else 0
+    if max_context_len > DECODE_KEYS:
+        raise UnsupportedShape(f"contexts of up to {max_context_len} keys; a step's layers in two launches read {DECODE_KEYS} keys")
     turn = _Turn(workspace, (M, H, num_heads, num_kv_heads, head_dim, intermediate, "layers", n_layers), 1, 2)
     _call("ms_decode_layers", table.data_ptr(), x.data_ptr(), H, positions.data_ptr(), slot_mapping.data_ptr(),
           context_lens.data_ptr(), block_table.data_ptr(), _ptr(table_rows), block_table.shape[1], float(scale), M, H,

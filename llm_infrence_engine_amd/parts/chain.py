@@ -253,7 +253,7 @@ class DecodeChain:
         ops.decode_first(x, norm.weight, norm.eps, m.w_qkv, m.b_qkv, ctx.positions, m.position.inv_freq, kv.slot_mapping,
                          kv.k_pages, kv.v_pages, nh, nkv, d, I, self.runs, self.workspace)
         ops.decode_layers(self.table, x, ctx.positions, kv.slot_mapping, ctx.context_lens, kv.block_table, kv.table_rows, m.scale,
-                          nh, nkv, d, I, kv.k_pages.shape[2], self.runs, self.workspace, self.told)
+                          nh, nkv, d, I, kv.k_pages.shape[2], self.runs, self.workspace, self.told, ctx.max_context_len)
 
     def _layer_by_layer(self, x, ctx, caches):
         nh, nkv, d, _, _ = self.sizes

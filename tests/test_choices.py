@@ -356,6 +356,31 @@ def test_a_chains_launches_are_refused_out_of_their_turn(ops, monkeypatch):
     assert launched.count("ms_decode_chain") == 6
 
 
+def test_contexts_that_all_layers_in_two_launches_cannot_read_are_refused(ops, monkeypatch):
+    """The kernel reads 1,024 keys of a context and no more: a bound that the caller knows is held against that, else the
+    contexts themselves are."""
+    launched = []
+    monkeypatch.setattr(ops, "_check", lambda *args, **kw: None)
+    monkeypatch.setattr(ops, "_call", lambda name, *args: launched.append(name))
+    monkeypatch.setattr(ops, "_stream", lambda: 0)
+    ints = lambda *v: torch.tensor(v, dtype=torch.int32)     # noqa: E731
+
+    def layers(*contexts, **bound):
+        M = len(contexts)
+        ws = torch.zeros(ops.decode_chain_workspace(M, 64, 2, 1, 64, 64, 2), dtype=torch.uint8)
+        ws.chain_turn = ((M, 64, 2, 1, 64, 64, "layers", 2), 1)
+        records = torch.zeros(2 * ops._get("ms_decode_layer_bytes")(), dtype=torch.uint8)
+        ops.decode_layers(records, torch.zeros(M, 64), ints(*[0] * M), ints(*[0] * M), ints(*contexts), torch.zeros(M, 99, dtype=torch.int32), None,
+                          1.0, 2, 1, 64, 64, 16, 2, ws, **bound)
+        return len(launched)
+
+    assert layers(1024, 1) == 1 and layers(5, max_context_len=1024) == 2
+    for contexts, bound in (((1025,), {}), ((3, 2000, 1), {}), ((5,), dict(max_context_len=1025))):
+        with pytest.raises(ops.UnsupportedShape, match="1024 keys"):
+            layers(*contexts, **bound)
+    assert len(launched) == 2
+
+
 @pytest.mark.parametrize("keys", [64, 2000])
 def test_a_launch_that_waited_in_vain_is_an_error_and_the_next_step_starts_over(ops, keys):
     """What the GPU writes where a launch was broken off is seen when the step's results have come, or before the next launch,
