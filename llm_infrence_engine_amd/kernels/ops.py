@@ -981,13 +981,44 @@ DECODE_KEYS = 1024      # keys of a context, with the step's own, that ``decode_
 
 def decode_layer_table(layers, device) -> torch.Tensor:
     """The records of ``decode_layers``: for each layer a dict of its tensors w_o, w_gate_up, w_down, norm2, k_pages, v_pages
-    and eps2, and of the layer after it (not of the last one) w_front, norm1, b_front (may be None), inv_freq, front_k, front_v
-    and eps1.  The tensors have to outlive the table; it does not keep them."""
+    (transposed) and eps2, and of the layer after it (not of the last one) w_front, norm1, b_front (may be None), inv_freq, front_k,
+    front_v and eps1.  The tensors have to outlive the table; it does not keep them.  What a kernel on ``device`` will read is
+    looked at here: nobody sees more of it than addresses later on."""
     names = ("w_o", "w_gate_up", "w_down", "w_front", "norm2", "norm1", "b_front", "inv_freq", "k_pages", "v_pages", "front_k", "front_v")
+    sizes = None
+    if torch.device(device).type != "cpu":
+        sizes = _layer_sizes(layers[0])
+        for i, l in enumerate(layers):
+            _check_layer(l, sizes, i + 1 == len(layers))
     rows = b"".join(struct.pack("<12Q2f", *(_ptr(l.get(n)) or 0 for n in names), l["eps2"], l.get("eps1", 0.0)) for l in layers)
     if len(rows) != len(layers) * _get("ms_decode_layer_bytes")():
         raise build.KernelLibraryError("the library's record of a layer has another size than this module's")
-    return torch.frombuffer(bytearray(rows), dtype=torch.uint8).to(device)
+    table = torch.frombuffer(bytearray(rows), dtype=torch.uint8).to(device)
+    table.layer_sizes = sizes
+    return table
+
+
+def _layer_sizes(l: dict) -> tuple:
+    """(heads, key/value heads, head size, width, intermediate size, page size) that a record's tensors say."""
+    _, nkv, page_size, d = l["k_pages"].shape
+    (H, width), I = l["w_o"].shape, l["w_down"].shape[1]
+    return width // d, nkv, d, H, I, page_size
+
+
+def _check_layer(l: dict, sizes: tuple, last: bool) -> None:
+    nh, nkv, d, H, I, page_size = sizes
+    bf16, f32, width = torch.bfloat16, torch.float32, (nh + 2 * nkv) * d
+    wanted = [("w_o", bf16, (H, nh * d), 16), ("w_gate_up", bf16, (2 * I, H), 16), ("w_down", bf16, (H, I), 16), ("norm2", f32, (H,), 16),
+              ("k_pages", bf16, (None, nkv, page_size, d), 16), ("v_pages", bf16, (l["k_pages"].shape[0], nkv, d, page_size), 16)]
+    if not last:
+        wanted += [("w_front", bf16, (width, H), 16), ("norm1", f32, (H,), 16), ("inv_freq", f32, (d // 2,), 4),
+                   ("front_k", bf16, (None, nkv, page_size, d), 16), ("front_v", bf16, (l["front_k"].shape[0], nkv, d, page_size), 16)]
+        if l["b_front"] is not None:
+            wanted.append(("b_front", f32, (width,), 4))
+    for name, dtype, shape, align in wanted:
+        _check(l[name], name, dtype, shape)
+        if l[name].data_ptr() % align:
+            raise ValueError(f"{name} must lie on {align} bytes")
 
 
 def decode_first(x: torch.Tensor, norm_weight: torch.Tensor, eps: float, w_qkv: torch.Tensor, bias: Optional[torch.Tensor],
@@ -1035,14 +1066,17 @@ def decode_layers(table: torch.Tensor, x: torch.Tensor, positions: torch.Tensor,
     _check(workspace, "workspace", torch.uint8)
     if workspace.numel() < decode_chain_workspace(M, H, num_heads, num_kv_heads, head_dim, intermediate, n_layers):
         raise ValueError("the workspace is too small")
+    if getattr(table, "layer_sizes", None) != (num_heads, num_kv_heads, head_dim, H, intermediate, page_size):
+        raise ValueError("the table is of layers of other sizes, or none that decode_layer_table made for the GPU")
     if max_context_len is None:
         max_context_len = int(context_lens.max()) if M else 0
     if max_context_len > DECODE_KEYS:
         raise UnsupportedShape(f"contexts of up to {max_context_len} keys; a step's layers in two launches read {DECODE_KEYS} keys")
+    told = _told(told)
     turn = _Turn(workspace, (M, H, num_heads, num_kv_heads, head_dim, intermediate, "layers", n_layers), 1, 2)
     _call("ms_decode_layers", table.data_ptr(), x.data_ptr(), H, positions.data_ptr(), slot_mapping.data_ptr(),
           context_lens.data_ptr(), block_table.data_ptr(), _ptr(table_rows), block_table.shape[1], float(scale), M, H,
-          intermediate, num_heads, num_kv_heads, head_dim, page_size, n_layers, workspace.data_ptr(), _told(told), _stream())
+          intermediate, num_heads, num_kv_heads, head_dim, page_size, n_layers, workspace.data_ptr(), told, _stream())
     turn.over()
     return x
 
@@ -1100,10 +1134,11 @@ def decode_chain(attn: torch.Tensor, w_o: torch.Tensor, x: torch.Tensor, norm2: 
         page_size = k_pages.shape[2]
         tail = (norm1.data_ptr(), float(eps1), w_qkv.data_ptr(), _ptr(bias), positions.data_ptr(), inv_freq.data_ptr(),
                 slot_mapping.data_ptr(), q.data_ptr(), k_pages.data_ptr(), v_pages.data_ptr())
+    told = _told(told)
     turn = _Turn(workspace, (M, H, num_heads, num_kv_heads, head_dim, I, "chains", launches), launch, launches)
     _call("ms_decode_chain", attn.data_ptr(), attn.shape[1], w_o.data_ptr(), x.data_ptr(), H, norm2.data_ptr(), float(eps2),
           w_gate_up.data_ptr(), w_down.data_ptr(), *tail, M, H, I, num_heads, num_kv_heads, head_dim, page_size,
-          int(v_transposed), workspace.data_ptr(), _told(told), launch, launches, _stream())
+          int(v_transposed), workspace.data_ptr(), told, launch, launches, _stream())
     turn.over()
     return q
 

@@ -309,6 +309,7 @@ def test_a_chains_launches_are_refused_out_of_their_turn(ops, monkeypatch):
     def layers(ws, M=2, L=3):
         a = args(M)
         records = torch.zeros(L * ops._get("ms_decode_layer_bytes")(), dtype=torch.uint8)
+        records.layer_sizes = (2, 1, 64, 64, 64, 16)
         ops.decode_layers(records, a["x"], a["pos"], a["pos"], a["pos"], a["table"], None, 1.0, *a["sizes"], 16, L, ws)
 
     def chain(ws, launch, launches=3, M=2):
@@ -370,6 +371,7 @@ def test_contexts_that_all_layers_in_two_launches_cannot_read_are_refused(ops, m
         ws = torch.zeros(ops.decode_chain_workspace(M, 64, 2, 1, 64, 64, 2), dtype=torch.uint8)
         ws.chain_turn = ((M, 64, 2, 1, 64, 64, "layers", 2), 1)
         records = torch.zeros(2 * ops._get("ms_decode_layer_bytes")(), dtype=torch.uint8)
+        records.layer_sizes = (2, 1, 64, 64, 64, 16)
         ops.decode_layers(records, torch.zeros(M, 64), ints(*[0] * M), ints(*[0] * M), ints(*contexts), torch.zeros(M, 99, dtype=torch.int32), None,
                           1.0, 2, 1, 64, 64, 16, 2, ws, **bound)
         return len(launched)

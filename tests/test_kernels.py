@@ -2123,6 +2123,70 @@ def test_a_launch_whose_inputs_never_come_ends(ops):
         ops.decode_layers(table, x, pos, slots, lens, blocks, None, 0.125, nh, nkv, d, I, page_size, L, ws, torch.zeros(1, dtype=torch.int32))
 
 
+def test_a_table_of_layers_holds_what_the_kernel_can_read(ops):
+    """The kernel reads addresses out of the table and cannot look at them any more: type, shape, layout, device and alignment of
+    every tensor are looked at when the table is made, and its sizes when it is used."""
+    H, I, nh, nkv, d, page_size = 96, 64, 4, 2, 64, 16
+    bf = lambda *shape: torch.zeros(*shape, dtype=torch.bfloat16, device=DEV)     # noqa: E731
+    f = lambda *shape: torch.zeros(*shape, device=DEV)     # noqa: E731
+    pages = lambda: (bf(3, nkv, page_size, d), bf(3, nkv, d, page_size))     # noqa: E731
+    kv = [pages(), pages()]
+
+    def rows():
+        one = dict(w_o=bf(H, nh * d), w_gate_up=bf(2 * I, H), w_down=bf(H, I), norm2=f(H), eps2=1e-6)
+        two = dict(one, k_pages=kv[1][0], v_pages=kv[1][1])
+        return [dict(one, k_pages=kv[0][0], v_pages=kv[0][1], w_front=bf((nh + 2 * nkv) * d, H), norm1=f(H), eps1=1e-6, b_front=f((nh + 2 * nkv) * d),
+                     inv_freq=f(d // 2), front_k=kv[1][0], front_v=kv[1][1]), two]
+
+    table = ops.decode_layer_table(rows(), DEV)
+    assert table.numel() == 2 * ops._get("ms_decode_layer_bytes")()
+    r = rows()
+    r[0]["b_front"] = None
+    ops.decode_layer_table(r, DEV)
+
+    def refused(layer, name, bad, error=(ValueError, TypeError, RuntimeError, KeyError)):
+        r = rows()
+        if bad is None:
+            del r[layer][name]
+        else:
+            r[layer][name] = bad(r[layer][name])
+        with pytest.raises(error):
+            ops.decode_layer_table(r, DEV)
+
+    aside = lambda t: torch.zeros(t.numel() + 2, dtype=t.dtype, device=DEV)[2:].view(t.shape)      # 4 or 8 bytes off     # noqa: E731
+    strided = lambda t: torch.stack([t, t], -1)[..., 0]     # noqa: E731
+    for layer, names in ((0, ("w_o", "w_gate_up", "w_down", "norm2", "w_front", "norm1", "k_pages", "v_pages", "front_k", "front_v")),
+                         (1, ("w_o", "w_gate_up", "w_down", "norm2", "k_pages", "v_pages"))):
+        for name in names:
+            refused(layer, name, lambda t: t.cpu(), RuntimeError)
+            refused(layer, name, lambda t: t.half(), TypeError)
+            refused(layer, name, strided, ValueError)
+            refused(layer, name, lambda t: torch.cat([t, t]) if "pages" not in name and "front_" not in name else t[:, :1].contiguous(), ValueError)
+            refused(layer, name, aside, ValueError)
+            refused(layer, name, None)
+    for name in ("inv_freq", "b_front"):
+        refused(0, name, lambda t: t.bfloat16(), TypeError)
+        refused(0, name, lambda t: t[1:].clone(), ValueError)
+    refused(0, "inv_freq", None)
+    refused(0, "v_pages", lambda t: t.transpose(2, 3).contiguous(), ValueError)
+    refused(1, "k_pages", lambda t: bf(3, nkv, 2 * page_size, d), ValueError)
+
+    M = 2
+    ints = lambda *v: torch.tensor(v, dtype=torch.int32, device=DEV)     # noqa: E731
+    x, blocks = f(M, H), ints(1, 2).view(2, 1)
+
+    def layers(table, nh=nh, nkv=nkv, page_size=page_size, x=x, I=I):
+        ws = torch.zeros(ops.decode_chain_workspace(M, x.shape[1], nh, nkv, d, I, 2), dtype=torch.uint8, device=DEV)
+        ws.chain_turn = ((M, x.shape[1], nh, nkv, d, I, "layers", 2), 1)
+        ops.decode_layers(table, x, ints(3, 0), ints(19, 32), ints(4, 1), blocks, None, 0.125, nh, nkv, d, I, page_size, 2, ws, max_context_len=4)
+
+    for other in (dict(nh=2), dict(nkv=1), dict(page_size=32), dict(x=f(M, 128)), dict(I=32)):
+        with pytest.raises(ValueError, match="table"):
+            layers(table, **other)
+    with pytest.raises(ValueError, match="table"):
+        layers(table.clone())
+
+
 def test_decode_chain_refuses_what_it_cannot_take(ops):
     for sizes in [(9, 896, 14, 2, 64, 4864), (0, 896, 14, 2, 64, 4864), (1, 1056, 14, 2, 64, 4864), (1, 896, 17, 1, 64, 4864),
                   (1, 896, 14, 2, 64, 6176), (1, 896, 14, 2, 64, 4880), (1, 880, 14, 2, 64, 4864), (1, 896, 14, 2, 60, 4864)]:
