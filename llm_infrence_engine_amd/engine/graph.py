@@ -171,7 +171,7 @@ class StepGraphs:
         ctx = self.builder.context(f, lay.n_tokens, lay.n_requests, max_q_len, max_context_len, padded=True)
         caches = runner.caches(ctx.state_slots, bk.slots)
         if decode:
-            ctx.chain = bk.chain = DecodeChain.of(model, ctx, caches)
+            ctx.chain = bk.chain = DecodeChain.where_it_pays(model, ctx, caches)
         G = lay.n_groups
         # what the table entries of the last steps changed must be on the device before a description that is all
         # padding stands in for a step

@@ -101,7 +101,7 @@ class ModelRunner:
             caches = self.caches(built.ctx.state_slots, built.slots)
             if built.ctx.decode_only:
                 key = (built.ctx.num_tokens, built.ctx.max_context_len > ops.DECODE_KEYS)
-                built.ctx.chain = self._chain(key, caches, lambda: DecodeChain.of(self.model, built.ctx, caches))
+                built.ctx.chain = self._chain(key, caches, lambda: DecodeChain.where_it_pays(self.model, built.ctx, caches))
             if built.ctx.chain is None:
                 built.ctx.chain = self._chain("float", caches, lambda: FloatLayers.of(self.model, caches))
             self.chain = built.ctx.chain

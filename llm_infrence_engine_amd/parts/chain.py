@@ -43,6 +43,29 @@ def _plain_attention(m) -> bool:
     return m.window is None and m.sink_w is None and not m.softcap and m.slopes is None and m.out_scale == 1.0
 
 
+def _pays(n_tokens: int, sizes: tuple, whole: bool) -> bool:
+    """Whether a chain of ``n_tokens`` tokens (``whole``: all layers in two launches) beats the parts one by one.  It saves launches
+    and waits, and reads its inputs' words once for every block; of narrow layers that outweighs it from 5 tokens on, whose words are
+    twice as many.  The lines are drawn from captured steps of 24 layers of 41 sizes, 64 to 1,024 wide, 33 to 1,100 keys (the chain's
+    time over the parts'; values: the weights of a layer):
+
+    chain, up to 4 tokens   0.4M to 0.84M values 0.96 to 1.04; 1.05M 0.94 to 0.98; 4.6M 0.89 to 0.94; 15M 0.75 to 0.85
+    chain, 5 to 8           0.4M to 0.84M 1.07 to 1.22; 2.3M 1.03 to 1.09; 3.8M 1.03 to 1.12; 5.77M 0.96 to 1.07; 5.9M to 6.3M 0.92 to
+                            1.00 (6.9M and 7.3M up to 1.03 and 1.02, once each); 13M 0.89 to 0.96; 15M 0.81 to 0.85
+    whole, up to 4          0.07M 0.77 to 0.87; 1M 0.66 to 0.73; 15M 0.57 to 0.64
+    whole, 5 to 8           0.07M 0.85 to 1.02; 0.25M 0.86 to 1.05; 0.44M 0.82 to 0.91; 15M 0.66 to 0.73
+    whole, 5 to 8, by tokens x key/value heads, of which each is four blocks that read its keys, beyond 64 more than the CUs: up to 64
+                            0.68 to 0.93 at 33 keys, 0.62 to 0.97 at 1,000; 65 to 128 0.77 to 1.02 and 0.92 to 1.10
+
+    A captured step is told no bound of its contexts below 1,024 keys, so what loses at 1,000 is left to the chain.  With these lines no
+    measured step takes more than 1.03 of the parts' time (1,128 of them, 0.84 on average)."""
+    nh, nkv, d, H, I = sizes
+    values = 3 * H * I + 2 * H * d * (nh + nkv)
+    if whole:
+        return n_tokens * nkv <= 64 and (n_tokens <= 4 or values >= 400_000)
+    return values >= (1_000_000 if n_tokens <= 4 else 5_800_000)
+
+
 def _own_pages(caches, dtype) -> bool:
     """Whether every run stores its keys and values in pages of its own, of ``dtype``."""
     return all(c.kv is not None and c.kv.store and c.kv.k_pages.dtype == dtype for c in caches)
@@ -171,9 +194,14 @@ class DecodeChain:
         self.broken_off = False      # a step ended with an exception between its launches, or a launch waited in vain
 
     @classmethod
-    def of(cls, model, ctx, caches) -> Optional["DecodeChain"]:
+    def where_it_pays(cls, model, ctx, caches) -> Optional["DecodeChain"]:
+        """``of``, and None also where the parts one by one are as fast or faster (``_pays``)."""
+        return cls.of(model, ctx, caches, _pays)
+
+    @classmethod
+    def of(cls, model, ctx, caches, pays=lambda n_tokens, sizes, whole: True) -> Optional["DecodeChain"]:
         """For decode steps like ``ctx``, of as many tokens and of contexts on the same side of ``ops.DECODE_KEYS``, from
-        ``caches``; None where the kernels do not take the model or the size."""
+        ``caches``; None where the kernels do not take the model or the size, or it does not pay."""
         runs, n = model.spec.order, ctx.num_tokens
         if model.rt.dtype != torch.bfloat16 or model.pass_entry is not None or not 2 <= len(runs) <= 1024 or n != ctx.num_requests:
             return None
@@ -184,12 +212,14 @@ class DecodeChain:
             return None
         sizes = sizes.pop()
         nh, nkv, d, H, I = sizes
-        if ctx.max_context_len <= ops.DECODE_KEYS and cls._one_group(model, caches):
+        if ctx.max_context_len <= ops.DECODE_KEYS and cls._one_group(model, caches) and pays(n, sizes, True):
             n_bytes = ops.decode_chain_workspace(n, H, nh, nkv, d, I, len(runs))
             if n_bytes:
                 chain = cls(model, sizes, n_bytes, caches)
                 chain._lay_out(caches)
                 return chain
+        if not pays(n, sizes, False):
+            return None
         n_bytes = ops.decode_chain_workspace(n, H, nh, nkv, d, I)
         return cls(model, sizes, n_bytes, caches) if n_bytes else None
 

@@ -280,6 +280,46 @@ def test_a_chain_holds_for_the_layers_and_weights_it_was_made_of(ops, keys):
     assert not made.takes(m, caches)
 
 
+@pytest.mark.parametrize("tokens,sizes,keys,kind", [
+    # time of a decode step of 24 such layers over the parts' own: layer by layer, all layers in two launches (at 33, 577, 1,000 keys)
+    (1, (14, 2, 64, 896, 4864), 1000, "step"),       # 0.85; 0.62 0.59 0.58
+    (8, (14, 2, 64, 896, 4864), 1000, "step"),       # 0.84; 0.73 0.70 0.68
+    (8, (14, 2, 64, 896, 4864), 2000, "layers"),     # 0.84
+    (4, (2, 1, 64, 128, 512), 64, "step"),           # 1.02; 0.79 0.71
+    (4, (2, 1, 64, 128, 512), 2000, None),           # 1.02
+    (8, (2, 1, 64, 128, 512), 64, None),             # 1.26; 1.05 0.93
+    (1, (4, 2, 64, 256, 768), 2000, None),           # 0.99
+    (4, (4, 4, 64, 256, 1024), 2000, "layers"),      # 0.97
+    (8, (3, 3, 64, 192, 512), 64, "step"),           # 1.22; 0.91 0.82
+    (8, (8, 8, 64, 512, 1536), 64, "step"),          # 1.04; 0.84 0.85 0.89
+    (8, (8, 8, 64, 512, 1536), 2000, None),          # 1.04
+    (8, (4, 4, 128, 512, 1536), 64, None),           # 1.07, heads of 128
+    (4, (4, 4, 128, 512, 1536), 64, "layers"),       # 0.97
+    (7, (16, 16, 64, 1024, 512), 2000, None),        # 1.06
+    (5, (5, 1, 128, 640, 2560), 64, "layers"),       # 0.98
+    (4, (16, 16, 64, 1024, 2048), 64, "step"),       # 0.91; 0.76 0.86 0.93
+    (7, (16, 16, 64, 1024, 2048), 64, "layers"),     # 1.00; 0.92 1.01 1.09
+    (8, (12, 12, 64, 768, 2048), 64, "layers"),      # 0.97; 0.88 0.93 1.04
+    (8, (16, 8, 64, 1024, 4096), 64, "step"),        # 0.90; 0.79 0.82 0.88
+    (8, (16, 16, 64, 1024, 512), 64, None)])         # 1.01
+def test_chains_run_where_they_pay(ops, tokens, sizes, keys, kind):
+    """Measured on both sides of the lines, at which the parts' own launches are as fast or faster."""
+    from llm_infrence_engine_amd.parts import chain
+    from llm_infrence_engine_amd.parts.attention import GQAttention
+    from llm_infrence_engine_amd.parts.positions import RotaryHalf
+
+    nh, nkv, d, H, I = sizes
+    m, b, caches, of = _decode_stand_in(ops, keys)
+    kept = b.mixer
+    b.mixer = GQAttention("", RotaryHalf("", d, d, 1e4), H, nh, nkv, d, 0.1)
+    b.mixer.w_o, b.mixer.w_qkv, b.mixer.b_qkv, b.mixer.sink_w = kept.w_o, kept.w_qkv, kept.b_qkv, None
+    b.mixer.position.inv_freq = kept.position.inv_freq
+    b.mixer_norm.size = b.feed_forward_norm.size = b.feed_forward.hidden_size = H
+    b.feed_forward.intermediate_size = I
+    made = chain.DecodeChain.where_it_pays(m, SimpleNamespace(num_tokens=tokens, num_requests=tokens, max_context_len=keys), caches)
+    assert (None if made is None else "layers" if made.table is None else "step") == kind
+
+
 def test_a_chains_launches_are_refused_out_of_their_turn(ops, monkeypatch):
     """A launch waits for words of the one before it in the step, and their numbers go by how many have run: the next one due on a
     workspace, of the same sizes, or none.  A launch that was refused does not count; a workspace that starts over takes any."""
@@ -440,7 +480,7 @@ def test_a_step_compares_a_chains_weights_once(ops, monkeypatch, dtype, chains):
     def of(kind):
         return classmethod(lambda cls, *args: made.append(kind) or (Chain() if chains and (kind == "float") == (dtype == torch.float32) else None))
 
-    monkeypatch.setattr(runner.DecodeChain, "of", of("decode"))
+    monkeypatch.setattr(runner.DecodeChain, "where_it_pays", of("decode"))
     monkeypatch.setattr(runner.FloatLayers, "of", of("float"))
     x = torch.zeros(1, 4)
     layer = SimpleNamespace(forward=lambda x, pending, *a: pending, takes_sums=False, settles_writes=False)
