@@ -608,3 +608,119 @@ def test_float_layers_of_an_odd_width_are_the_parts_one_by_one(ops, tokens):
         got.append([r.step([StepEntry(i, [7 + i] * n, [n - 1]) for i, n in enumerate(tokens)]).cpu() for _ in range(3)])
         assert isinstance(r.chains["float"], chain.FloatLayers) == whole
     assert all(torch.equal(a, b) for a, b in zip(*got))
+
+
+@pytest.fixture(scope="module")
+def chained_model():
+    return _small_model(torch.bfloat16, seed=5, std=0.05, hidden_size=768, intermediate_size=2048, num_hidden_layers=3, num_attention_heads=12,
+                        num_key_value_heads=4, max_position_embeddings=2048)
+
+
+def _prompts(r, lengths):
+    from llm_infrence_engine_amd.engine.batch import StepEntry
+
+    for i, n in enumerate(lengths):
+        r.step([StepEntry(i, [(5 * j + i) % 64 for j in range(n)], [n - 1])])
+
+
+def _like(got, want):
+    # three layers, each of the two within 1.2e-2 of doubles (queries, heads, probabilities and the middle are rounded to bfloat16)
+    assert got.shape == want.shape and got.isfinite().all()
+    assert (got.double() - want.double()).norm() <= 2.4e-2 * want.double().norm()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("graphs", [False, True])
+@pytest.mark.parametrize("lengths", [[40], [1022, 7, 300], [3, 1, 16, 511, 64, 200, 33, 1023]])
+def test_a_models_chains_are_its_parts_one_by_one(ops, chained_model, monkeypatch, lengths, graphs):
+    """Decode steps of a model through its chains and part by part, logits of every step: one request, three (in a graph a row of
+    padding) and eight; a context that grows past 1,024 keys, from two launches for all layers to one a layer; steps launched,
+    replayed, and replayed several at a time."""
+    from llm_infrence_engine_amd.engine import ModelRunner
+    from llm_infrence_engine_amd.engine.batch import StepEntry
+    from llm_infrence_engine_amd.parts import chain
+
+    make = lambda graphs: ModelRunner(chained_model, 16, 200, 8, 1100, hip_graphs=graphs, graph_portion_tokens=0)     # noqa: E731
+    kinds = set()
+
+    def step(r, t):
+        out = r.step([StepEntry(i, [(11 * t + i) % 64], [0]) for i in range(len(lengths))]).clone()
+        r.check()
+        kinds.add(None if r.chain is None else r.chain.table is not None)
+        return out
+
+    a = make(graphs)
+    _prompts(a, lengths)
+    got = [step(a, t) for t in range(4)]
+    assert kinds == ({True, False} if max(lengths) > 1000 else {True})
+    tokens = a.decode_steps([StepEntry(i, [9 + i]) for i in range(len(lengths))], 4) if graphs else []
+    got.append(step(a, 5))
+    kinds.clear()
+    monkeypatch.setattr(chain.DecodeChain, "where_it_pays", classmethod(lambda *args: None))
+    b = make(False)
+    _prompts(b, lengths)
+    want = [step(b, t) for t in range(4)]
+    for row in [[9 + i for i in range(len(lengths))]] + tokens[:-1] if graphs else []:
+        b.step([StepEntry(i, [t], [0]) for i, t in enumerate(row)])
+    want.append(step(b, 5))
+    assert kinds == {None}
+    for g, w in zip(got, want):
+        _like(g, w)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("length,name,at", [(40, "decode_first", 0), (40, "decode_layers", 0), (1100, "decode_chain", 0), (1100, "decode_chain", 2)])
+def test_a_chain_starts_over_behind_a_step_that_broke_off(ops, chained_model, monkeypatch, length, name, at):
+    """An exception between a step's launches: the same step again, and those after it, are as they would have been."""
+    from llm_infrence_engine_amd.engine import ModelRunner
+    from llm_infrence_engine_amd.engine.batch import StepEntry
+
+    got, call = [], getattr(ops, name)
+    for breaks in (False, True):
+        r = ModelRunner(chained_model, 16, 200, 4, 1200)
+        _prompts(r, [length, 5])
+        for t in range(3):
+            entries = [StepEntry(i, [(7 * t + i) % 64], [0]) for i in range(2)]
+            if breaks and t == 1:
+                left = [at]
+
+                def broken(*args, **kw):
+                    left[0] -= 1
+                    if left[0] < 0:
+                        raise RuntimeError("broken off here")
+                    return call(*args, **kw)
+
+                monkeypatch.setattr(ops, name, broken)
+                with pytest.raises(RuntimeError, match="broken off here"):
+                    r.step(entries)
+                monkeypatch.setattr(ops, name, call)
+            got.append(r.step(entries).cpu())
+            r.check()
+            assert (r.chain.table is not None) == (length < 1000)
+    assert all(torch.equal(x, y) for x, y in zip(got[:3], got[3:]))
+
+
+@pytest.mark.gpu
+def test_a_model_whose_weights_lie_anywhere_steps_as_one_whose_do_not(ops):
+    """Weights that are views of one buffer, 4 bytes off 16 (as a reader may hand them out on the GPU): no chain, and the logits of
+    the same weights in places of their own."""
+    from llm_infrence_engine_amd.engine import ModelRunner
+    from llm_infrence_engine_amd.engine.batch import StepEntry
+
+    got = []
+    for aside in (False, True):
+        model = _small_model(torch.bfloat16, seed=6, std=0.05, hidden_size=768, intermediate_size=2048, num_hidden_layers=2,
+                             num_attention_heads=12, num_key_value_heads=4, max_position_embeddings=128)
+        for l in model.layers if aside else ():
+            for part, names in ((l.mixer, ("w_qkv", "w_o")), (l.feed_forward, ("w_gate_up", "w_down"))):
+                for n in names:
+                    w = getattr(part, n)
+                    there = torch.empty(w.numel() + 2, dtype=w.dtype, device=w.device)[2:].view(w.shape)
+                    assert there.copy_(w).data_ptr() % 16 == 4
+                    setattr(part, n, there)
+        r = ModelRunner(model, 16, 24, 4, 96)
+        _prompts(r, [20, 3])
+        got.append([r.step([StepEntry(i, [7 + i], [0]) for i in range(2)]) for _ in range(2)])
+        assert (r.chain is None) == aside
+    for a, b in zip(*got):
+        _like(b, a)
