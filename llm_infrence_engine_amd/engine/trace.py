@@ -53,6 +53,7 @@ def replay(model_dir, dtype: str, out_dir, max_tokens: int, lines, log=sys.stdou
             logits = runner.step(entries)
             if logits.shape[0]:
                 arr = logits.to("cpu").numpy().astype("<f4", copy=False)
+                runner.check()
                 np.ascontiguousarray(arr).tofile(out / f"{step}.f32")
         for rid in rec.get("end", ()):
             if runner.manager.has(rid):
