@@ -242,6 +242,8 @@ class StepGraphs:
 
     def _fill_and_replay(self, bk: _Bucket, entries: List[StepEntry], steps: int, every_row: bool = False,
                          sampling=None):
+        if bk.chain is not None:      # before anything is taken that this replay is to bring to the device
+            bk.chain.ready()
         if self.manager.pending_updates() > bk.layout.n_updates:
             self.builder.flush_updates()
         d = self.builder.describe(entries, steps)
@@ -252,8 +254,6 @@ class StepGraphs:
         self.builder.write(d, bk.layout, bk.buf.np)
         bk.buf.send()
         self.chain = bk.chain
-        if bk.chain is not None:
-            bk.chain.ready()
         bk.graph.replay()
         return d
 

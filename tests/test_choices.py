@@ -442,10 +442,10 @@ def test_a_launch_that_waited_in_vain_is_an_error_and_the_next_step_starts_over(
     made.ready()
     assert not made.workspace.any() and not made.broken_off
 
-    replays = []
+    replays, written = [], []
     g = StepGraphs.__new__(StepGraphs)
     g.manager = SimpleNamespace(pending_updates=lambda: 0)
-    g.builder = SimpleNamespace(describe=lambda *a: SimpleNamespace(), write=lambda *a: None)
+    g.builder = SimpleNamespace(describe=lambda *a: SimpleNamespace(), write=lambda *a: written.append(1))
     bk = SimpleNamespace(layout=SimpleNamespace(n_updates=1), chain=made, graph=SimpleNamespace(replay=lambda: replays.append(made.workspace.any().item())),
                          buf=SimpleNamespace(wait_until_sent=lambda: None, send=lambda: None, np=None))
     g._fill_and_replay(bk, [], 1)
@@ -454,10 +454,12 @@ def test_a_launch_that_waited_in_vain_is_an_error_and_the_next_step_starts_over(
     made.workspace[:9] = 7
     with pytest.raises(RuntimeError, match="void"):
         g._fill_and_replay(bk, [], 1)
+    assert len(written) == 1      # (what it takes from the manager, the block tables' changes, is the next replay's to bring)
     g._fill_and_replay(bk, [], 1)
-    assert replays == [False, False]
+    assert replays == [False, False] and len(written) == 2
     r.chain = None
     r.check()
+
 
 
 @pytest.mark.parametrize("dtype,chains", [(torch.bfloat16, True), (torch.float32, True), (torch.float32, False)])
