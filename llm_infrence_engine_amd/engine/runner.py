@@ -75,6 +75,7 @@ class ModelRunner:
     @torch.inference_mode()
     def step(self, entries: List[StepEntry]) -> torch.Tensor:
         """Float logits [wanted places, vocabulary], in the order of the entries and of their ``want``."""
+        self.check()
         m = self.manager
         seen = set()
         for e in entries:
@@ -114,7 +115,7 @@ class ModelRunner:
 
     def check(self) -> None:
         """To be asked when the last step's results have come: raises if they are void (``DecodeChain.check``).  The next step
-        asks, too, before it is launched."""
+        asks, too, before it takes anything."""
         if self.chain is not None:
             self.chain.check()
 
@@ -132,6 +133,7 @@ class ModelRunner:
         request's own rule, seed and count of draws.  Returns the chosen tokens, [steps][len(entries)]."""
         if self.graphs is None:
             raise RuntimeError("several decode steps per launch need hip_graphs")
+        self.check()
         m = self.manager
         for e in entries:
             if len(e.tokens) != 1:

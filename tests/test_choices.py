@@ -461,6 +461,20 @@ def test_a_launch_that_waited_in_vain_is_an_error_and_the_next_step_starts_over(
     r.check()
 
 
+def test_a_step_asks_for_the_last_ones_results_before_it_takes_anything(ops):
+    """A program that reads its logits without asking hears of void ones from the next step, whichever way that goes, while
+    requests and pages are still as they were."""
+    from llm_infrence_engine_amd.engine import ModelRunner
+
+    made = _decode_stand_in(ops)[3]()
+    r = ModelRunner.__new__(ModelRunner)
+    r.chain, r.graphs, r.manager = made, SimpleNamespace(chain=None), None      # (nothing to grow: it is not to be reached)
+    for step in (lambda: r.step([SimpleNamespace(req_id=0, tokens=[1])]), lambda: r.decode_steps([SimpleNamespace(req_id=0, tokens=[1])], 2)):
+        made.told[0] = 1
+        with pytest.raises(RuntimeError, match="void"):
+            step()
+        assert made.broken_off and not made.told[0]
+
 
 @pytest.mark.parametrize("dtype,chains", [(torch.bfloat16, True), (torch.float32, True), (torch.float32, False)])
 def test_a_step_compares_a_chains_weights_once(ops, monkeypatch, dtype, chains):
@@ -474,6 +488,9 @@ def test_a_step_compares_a_chains_weights_once(ops, monkeypatch, dtype, chains):
         def takes(self, model, caches):
             looked.append(self)
             return True
+
+        def check(self):
+            pass
 
         def forward(self, x, ctx, caches):
             ran.append(self)
@@ -491,7 +508,7 @@ def test_a_step_compares_a_chains_weights_once(ops, monkeypatch, dtype, chains):
     model.forward = lambda ctx, caches: Model.forward_hidden(model, ctx, caches)[0]
     r = ModelRunner.__new__(ModelRunner)
     ctx = lambda: SimpleNamespace(decode_only=True, num_tokens=1, max_context_len=5, chain=None, state_slots=None)     # noqa: E731
-    r.model, r.graphs, r.chains = model, None, {}
+    r.model, r.graphs, r.chains, r.chain = model, None, {}, None
     r.manager = SimpleNamespace(has=lambda i: True, grow=lambda *a: None, computed=lambda i: 4, advance=lambda *a: None)
     r.builder = SimpleNamespace(build=lambda entries: SimpleNamespace(ctx=ctx(), slots=[]))
     r.caches = lambda rows, slots: [SimpleNamespace(kv=None, state=None)]
