@@ -233,9 +233,9 @@ struct Shared {
 };
 
 // One word of the phase before, by one wave, so that blocks far ahead of their inputs disturb nobody.  Whole block; false: not
-// within `limit` looks.  VERDICT: the word of sh.late, another for each wait of an item: no barrier lies between a wave's read of it
+// within `limit` looks.  SLOT: the word of sh.late, another for each wait of an item: no barrier lies between a wave's read of it
 // and the store of the wait that follows.
-template <int VERDICT = 0>
+template <int SLOT = 0>
 __device__ __forceinline__ bool wait_first(Shared& sh, const u64* word, unsigned tag, unsigned limit) {
   if (threadIdx.x < MS_WAVE) {
     int late = 1;
@@ -243,10 +243,10 @@ __device__ __forceinline__ bool wait_first(Shared& sh, const u64* word, unsigned
       if ((unsigned)(look(word) >> 32) == tag) { late = 0; break; }
       __builtin_amdgcn_s_sleep(1);
     }
-    if (threadIdx.x == 0) { sh.late[VERDICT] = late; sh.late[1] = 0; }
+    if (threadIdx.x == 0) { sh.late[SLOT] = late; sh.late[1] = 0; }
   }
   __syncthreads();
-  return sh.late[VERDICT] == 0;
+  return sh.late[SLOT] == 0;
 }
 
 // A wave's share of the float stream's rows (one load's worth of four k-steps, G tokens), with the norm's weights.
