@@ -19,10 +19,10 @@ namespace {
 constexpr int WAVES = 4, STREAMS = 4;
 constexpr int MAX_D = 256;
 
-__device__ __forceinline__ void dot4(const float* q, const float* k, float& dot) {
-  const float4 v = *reinterpret_cast<const float4*>(k);
+__device__ __forceinline__ void dot4(const float* q, const float4 v, float& dot) {
   dot = fmaf(q[0], v.x, dot); dot = fmaf(q[1], v.y, dot); dot = fmaf(q[2], v.z, dot); dot = fmaf(q[3], v.w, dot);
 }
+__device__ __forceinline__ void dot4(const float* q, const float* k, float& dot) { dot4(q, *reinterpret_cast<const float4*>(k), dot); }
 __device__ __forceinline__ void dot4(const float* q, const bf16* k, float& dot) {
   const uint2 v = *reinterpret_cast<const uint2*>(k);
   dot = fmaf(q[0], __uint_as_float(v.x << 16), dot); dot = fmaf(q[1], __uint_as_float(v.x & 0xffff0000u), dot);
@@ -38,7 +38,11 @@ __device__ __forceinline__ void dot4(const float* q, const bf16* k, float& dot) 
 // What bounds it is the latency of a wave's loads: a lane reads its own key's row, the wave one row of values after another.
 // Values are asked for R rows at a time and never behind a condition (each load would be waited for by itself, which was 3
 // of the 7 us of a token with one key): lanes past the value size read its last entry, places past the keys the last row.
-template <typename T, int C, int W>     // C: values a lane, dv <= 64 C
+//
+// ONCE (float, heads of 64 dims, few items): a lane's key and the block's values are asked for together, one trip to memory where
+// the key and four times 16 rows of values were five: 8 tokens behind 1,000 keys, 14 heads 32.4 -> 26.9 us, 3 behind 135 9.2 -> 8.1.  Up to an
+// item a CU: its registers leave room for three blocks, 64 tokens behind 200 keys 20.5 -> 24.2, 140 tokens of a prompt 17.6 -> 21.7.
+template <typename T, int C, int W, bool ONCE>     // C: values a lane, dv <= 64 C
 __global__ void __launch_bounds__(WAVES * MS_WAVE, W == 1 ? 4 : 1)
 paged_attention_generic_kernel(const T* __restrict__ q, size_t q_stride, const T* __restrict__ k_pages,
                                const T* __restrict__ v_pages, const int* __restrict__ block_table, int table_stride,
@@ -101,7 +105,35 @@ paged_attention_generic_kernel(const T* __restrict__ q, size_t q_stride, const T
       const bool valid = j <= pos;
       size_t row = 0, vrow = 0;       // of the key among the rows of keys, of its first value
       float score = -INFINITY;
-      if (valid) {
+      const int count = min(MS_WAVE, pos - base + 1);
+      float values[ONCE ? MS_WAVE : 1];
+      if constexpr (ONCE) {
+        const int jj = min(j, pos), page = jj / page_size, off = jj - page * page_size;      // (lanes past the keys read the last one)
+        const size_t head = (size_t)table[page] * nkv + kvh;
+        row = head * page_size + off;
+        vrow = v_transposed ? head * dv * page_size + off : row * dv;
+        const float4* kp = reinterpret_cast<const float4*>(k_pages + row * 64);
+        float4 key[16];
+#pragma unroll
+        for (int i = 0; i < 16; ++i) key[i] = kp[i];
+#pragma unroll
+        for (int u0 = 0; u0 < MS_WAVE; u0 += 16) {
+          if (u0 >= count) break;
+#pragma unroll
+          for (int u = u0; u < u0 + 16; ++u) {
+            const unsigned lo = __builtin_amdgcn_readlane((unsigned)vrow, u), hi = __builtin_amdgcn_readlane((unsigned)(vrow >> 32), u);
+            values[u] = to_float((v_pages + (((size_t)hi << 32) | lo))[entry[0]]);
+          }
+        }
+        __builtin_amdgcn_sched_barrier(0);
+        float dot = 0.f;
+#pragma unroll
+        for (int i = 0; i < 16; ++i) dot4(&qs[slot][4 * i], key[i], dot);
+        score = dot;
+        if (softcap > 0.f) score = softcap * tanhf(score * inv_cap);
+        if (slopes) score -= slope * (float)(pos - j);
+        if (!valid) score = -INFINITY;
+      } else if (valid) {
         const int page = j / page_size, off = j - page * page_size;
         const size_t head = (size_t)table[page] * nkv + kvh;
         row = head * page_size + off;
@@ -128,7 +160,12 @@ paged_attention_generic_kernel(const T* __restrict__ q, size_t q_stride, const T
       m = m_new;
 #pragma unroll
       for (int c = 0; c < C; ++c) acc[c] *= corr;
-      const int count = min(MS_WAVE, pos - base + 1);
+      if constexpr (ONCE) {
+#pragma unroll
+        for (int u = 0; u < MS_WAVE; ++u)
+          if (u < count) acc[0] = fmaf(__int_as_float(__builtin_amdgcn_readlane(__float_as_int(p), u)), values[u], acc[0]);
+        continue;
+      }
       auto rows = [&](auto size, int j0) __attribute__((always_inline)) {
         constexpr int N = decltype(size)::value;
         float v[N][C], pj[N];
@@ -231,10 +268,11 @@ extern "C" int ms_paged_attention_generic(const void* q, long long q_stride, con
   const long long across = blocks < (1ll << 20) ? blocks : (1ll << 20);
   if ((blocks + across - 1) / across > 65535) return MS_UNSUPPORTED;
   dim3 grid((unsigned)across, (unsigned)((blocks + across - 1) / across)), block(WAVES * MS_WAVE);
-#define LAUNCH_W(T, C, W) paged_attention_generic_kernel<T, C, W><<<grid, block, 0, stream>>>((const T*)q, (size_t)q_stride, (const T*)k_pages, (const T*)v_pages, block_table, table_stride, table_rows, n_live_tokens, token_req, positions, (T*)out, (size_t)out_stride, n_tokens, num_heads, num_kv_heads, head_dim, value_dim, page_size, scale, window, v_transposed, vec, sink, softcap, slopes, (const T*)gate, (size_t)gate_stride, gate_width, out_scale)
-#define LAUNCH_C(T, C) do { if (waves == 4) LAUNCH_W(T, C, 4); else LAUNCH_W(T, C, 1); } while (0)
+#define LAUNCH_W(T, C, W, ONCE) paged_attention_generic_kernel<T, C, W, ONCE><<<grid, block, 0, stream>>>((const T*)q, (size_t)q_stride, (const T*)k_pages, (const T*)v_pages, block_table, table_stride, table_rows, n_live_tokens, token_req, positions, (T*)out, (size_t)out_stride, n_tokens, num_heads, num_kv_heads, head_dim, value_dim, page_size, scale, window, v_transposed, vec, sink, softcap, slopes, (const T*)gate, (size_t)gate_stride, gate_width, out_scale)
+#define LAUNCH_C(T, C) do { if (waves == 4) LAUNCH_W(T, C, 4, false); else LAUNCH_W(T, C, 1, false); } while (0)
 #define LAUNCH(T) do { if (value_dim <= 64) LAUNCH_C(T, 1); else if (value_dim <= 128) LAUNCH_C(T, 2); else LAUNCH_C(T, 4); } while (0)
-  if (dtype == MS_F32) LAUNCH(float);
+  if (dtype == MS_F32 && vec && head_dim == 64 && value_dim <= 64 && waves == 4 && items <= ms_compute_units()) LAUNCH_W(float, 1, 4, true);
+  else if (dtype == MS_F32) LAUNCH(float);
   else if (dtype == MS_BF16) LAUNCH(bf16);
   else return MS_BAD_ARG;
 #undef LAUNCH_C

@@ -1,8 +1,10 @@
-// All layers of a 32-bit step by one call: the same nine kernels a layer as when every one is asked for by itself, from the host
-// side of the library.  A decode step of the 32-bit path is as slow as its launches are made: 219 of them took 2.62 ms from
-// Python (12 us each, of which the launch itself is 4) where the GPU has 1.7 ms of work.
+// All layers of a 32-bit step by one call, to the same bits as when every part is asked for by itself: its nine kernels a layer, or,
+// up to 8 tokens, five.  A decode step of the 32-bit path was as slow as its launches were made: 219 of them took 2.62 ms from
+// Python (12 us each, of which the launch itself is 4) where the GPU has 1.7 ms of work; with five it has 1.2 (0.5B sizes, 3 tokens behind
+// 130: two norms, the rotation and the activation were 15.6 us of a layer's 70, and are 1 to 2 of the products' that took them in).
 #include "common.h"
 #include "api.h"
+#include "gemm_f32.h"
 
 namespace {
 
@@ -56,25 +58,36 @@ extern "C" int ms_float_layers(const void* layers, int n_layers, float* x, float
   const Pieces at = pieces_of(N, H, num_heads, num_kv_heads, head_dim, I);
   if (work_floats < at.end) return MS_BAD_ARG;
   float *sum = work + at.sum, *h = work + at.h, *qkv = work + at.qkv, *heads = work + at.heads, *gate_up = work + at.gate_up, *act = work + at.act;
-  auto product = [&](const float* a, const float* w, const float* bias, float* out, int n, int k) {
-    return ms_gemm_generic(a, w, bias, out, n_tokens, n, k, k, k, n, MS_F32, MS_F32, 0, stream);
+  auto product = [&](const float* a, const float* w, const float* bias, float* out, int n, int k, int accumulate) {
+    return ms_gemm_generic(a, w, bias, out, n_tokens, n, k, k, k, n, MS_F32, MS_F32, accumulate, stream);
   };
+  // (a product that does not take its norm refuses, and the rows go through the scratch one kernel after the other)
   for (int i = 0; i < n_layers; ++i) {
     const FloatLayer& l = static_cast<const FloatLayer*>(layers)[i];
-    int rc = ms_rms_norm(x, i ? sum : nullptr, MS_F32, 1, N * H, l.norm1, nullptr, h, n_tokens, H, l.eps1, 1, MS_F32, stream);
-    if (rc == MS_OK) rc = product(h, l.w_qkv, l.b_qkv, qkv, Q, H);
-    if (rc == MS_OK)
-      rc = ms_rope_store(qkv, nullptr, positions, l.inv_freq, slot_mapping, l.k_pages, l.v_pages, n_tokens, num_heads, num_kv_heads,
-                         head_dim, head_dim, page_size, v_transposed, MS_F32, stream);
+    const F32Front front{positions, slot_mapping, l.inv_freq, l.k_pages, l.v_pages, num_heads, num_kv_heads, head_dim, page_size, v_transposed};
+    int rc = ms_gemm_f32_normed(x, l.w_qkv, l.b_qkv, qkv, n_tokens, Q, H, F32Norm{l.norm1, l.eps1}, &front, stream);
+    if (rc == MS_UNSUPPORTED) {
+      rc = ms_rms_norm(x, nullptr, MS_F32, 1, N * H, l.norm1, nullptr, h, n_tokens, H, l.eps1, 1, MS_F32, stream);
+      if (rc == MS_OK) rc = product(h, l.w_qkv, l.b_qkv, qkv, Q, H, 0);
+      if (rc == MS_OK)
+        rc = ms_rope_store(qkv, nullptr, positions, l.inv_freq, slot_mapping, l.k_pages, l.v_pages, n_tokens, num_heads, num_kv_heads,
+                           head_dim, head_dim, page_size, v_transposed, MS_F32, stream);
+    }
     if (rc == MS_OK)
       rc = ms_paged_attention_generic(qkv, Q, l.k_pages, l.v_pages, block_table, table_width, table_rows, n_live, token_req, positions,
                                       heads, Ko, n_tokens, num_heads, num_kv_heads, head_dim, head_dim, page_size, num_pages, scale, 0,
                                       v_transposed, nullptr, 0.f, nullptr, nullptr, 0, 1, 1.f, MS_F32, stream);
-    if (rc == MS_OK) rc = product(heads, l.w_o, nullptr, sum, H, Ko);
-    if (rc == MS_OK) rc = ms_rms_norm(x, sum, MS_F32, 1, N * H, l.norm2, nullptr, h, n_tokens, H, l.eps2, 1, MS_F32, stream);
-    if (rc == MS_OK) rc = product(h, l.w_gate_up, nullptr, gate_up, 2 * I, H);
-    if (rc == MS_OK) rc = ms_silu_mul(gate_up, act, n_tokens, I, MS_F32, stream);
-    if (rc == MS_OK) rc = product(act, l.w_down, nullptr, sum, H, I);
+    if (rc == MS_OK) rc = product(heads, l.w_o, nullptr, x, H, Ko, 1);
+    if (rc == MS_OK) {
+      rc = ms_gemm_f32_normed(x, l.w_gate_up, nullptr, act, n_tokens, 2 * I, H, F32Norm{l.norm2, l.eps2}, nullptr, stream);
+      if (rc == MS_UNSUPPORTED) {
+        rc = ms_rms_norm(x, nullptr, MS_F32, 1, N * H, l.norm2, nullptr, h, n_tokens, H, l.eps2, 1, MS_F32, stream);
+        if (rc == MS_OK) rc = product(h, l.w_gate_up, nullptr, gate_up, 2 * I, H, 0);
+        if (rc == MS_OK) rc = ms_silu_mul(gate_up, act, n_tokens, I, MS_F32, stream);
+      }
+    }
+    const bool last = i + 1 == n_layers;
+    if (rc == MS_OK) rc = product(act, l.w_down, nullptr, last ? sum : x, H, I, !last);
     if (rc != MS_OK) return rc;
   }
   return MS_OK;

@@ -7,6 +7,8 @@
 //   rows     up to 64 rows (a decode step; against very many rows of W up to 16): all waves of a block on the same 4 to 16
 //            rows of W, the slices dealt out over them and added through LDS.  Bound by reading W.
 //   few      up to 8 rows, of these: loads that take four steps at a time.
+//   diagonal up to 8 rows: an instruction takes a step of two or four slices; also with the norm of A's rows, the gate, or the rotation
+//            and store of a q/k/v product within.
 //   tiled    the others: 64 x 64 or 32 x 32 tiles staged through LDS four steps ahead, 4 waves; 32 x 32 where the larger
 //            tiles would be fewer than two a CU.  Bound by the float matrix rate (157 TFLOP/s nominal), short K by writing C.
 // Measured with the 0.5B sizes against the 64 x 64 vector-ALU tile that ran them before (one MI355X): of 3 rows the down
@@ -16,6 +18,7 @@
 // the next.  C leaves a tile through LDS in whole rows (4,096 x 32,000 x 64: 440 us as the fragments lie, 270 so, 261 before).
 #include "common.h"
 #include "api.h"
+#include "gemm_f32.h"
 #include "quads.h"
 #include <type_traits>
 
@@ -198,6 +201,180 @@ gemm_f32_few_kernel(const float* __restrict__ A, const float* __restrict__ W, co
   }
 }
 
+// Up to X tokens (4 or 8), R rows of W a block (R <= X): the same products in the same order, S = 16 / X slices by one instruction.
+// The instruction's 16 rows are the block's rows at the same step of S slices, its 16 columns the tokens at that step of
+// these slices; rows and columns of one slice meet in the blocks on the diagonal, and what else comes out nobody reads.  So a step
+// costs 1 / S of the instructions and of the loads, and of both operands every lane's load is its own: 4 rows by 4,864 columns are 19
+// dependent steps of four waves, all asked for within the first few (sixteen waves of 76 instructions each are 4 us of the CU's
+// matrix pipes alone).
+//
+// NORM: A is the residual stream, and the rows are normed on their way (NORM pieces of 256 columns at most), by every block for
+// itself while its rows of W are on their way; the arithmetic and its order are rms_norm_kernel's.  EPI says what becomes of the sums.
+// 3 tokens: gate/up 9,728 x 896 with norm and gate 21.2 us in three kernels -> 13.3, q/k/v 1,152 x 896 with norm, rotation and store
+// 13 -> 6.9, 4 rows a block and no norm: see diagonal_rows.  What bounds it then: 64-byte pieces of 16 rows hold the CU's cache up for 70
+// cycles a load.  Whole lines through LDS and a ring a wave took 16 to 19 us for gate/up (few waves, each waiting for LDS), 9.4 against 8.4 for
+// 896 x 4,864, but 4.0 against 4.4 for 896 x 896.
+enum { F32_STORE = 0, F32_SWIGLU = 1, F32_QKV = 2 };
+
+template <int NORM>
+__device__ __forceinline__ void norm_rows(const float* __restrict__ x, const float* __restrict__ weight, float eps, float* h, int ldh, int M, int K) {
+  const int lane = threadIdx.x & (MS_WAVE - 1), wave = threadIdx.x / MS_WAVE, waves = blockDim.x / MS_WAVE;
+  const bool wide = K >= 1024;                       // rms_norm_kernel's blocks: 256 threads, else 128; a lane is two or four of them
+  for (int m = wave; m < M; m += waves) {
+    float4 v[NORM], w[NORM];
+#pragma unroll
+    for (int c = 0; c < NORM; ++c) {
+      const int i = min(c * 256 + lane * 4, K - 4);
+      v[c] = *reinterpret_cast<const float4*>(x + (size_t)m * K + i);
+      w[c] = *reinterpret_cast<const float4*>(weight + i);
+    }
+    float ss[4] = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int c = 0; c < NORM; ++c) {
+      if (c * 256 + lane * 4 >= K) continue;
+      const float t = v[c].x * v[c].x + v[c].y * v[c].y + v[c].z * v[c].z + v[c].w * v[c].w;
+      if (wide) ss[c & 3] += t;
+      else ss[c & 1] += t;
+    }
+    float total = 0.f;
+    total += wave_sum(ss[0]);
+    total += wave_sum(ss[1]);
+    if (wide) {
+      total += wave_sum(ss[2]);
+      total += wave_sum(ss[3]);
+    }
+    const float inv = 1.0f / sqrtf(total / (float)K + eps);
+#pragma unroll
+    for (int c = 0; c < NORM; ++c) {
+      const int i = c * 256 + lane * 4;
+      if (i < K)
+        *reinterpret_cast<float4*>(h + m * ldh + i) =
+            make_float4(w[c].x * (v[c].x * inv), w[c].y * (v[c].y * inv), w[c].z * (v[c].z * inv), w[c].w * (v[c].w * inv));
+    }
+  }
+}
+
+template <int R, int X, int EPI, int NORM>
+__global__ void __launch_bounds__(X * MS_WAVE, X == 4 ? 1 : NORM > 4 ? 2 : NORM ? 4 : 5)
+gemm_f32_diagonal_kernel(const float* __restrict__ A, const float* __restrict__ W, const float* __restrict__ bias,
+                    float* C, int M, int N, int K, size_t lda, size_t ldw, size_t ldc, int accumulate, F32Norm norm, F32Front front) {
+  extern __shared__ __align__(16) float part[];      // [slice][token][row of W], behind them (NORM) the normed rows
+  constexpr int S = 16 / X, AHEAD = X == 4 ? 10 : 8;
+  const int lane = threadIdx.x & (MS_WAVE - 1), wave = __builtin_amdgcn_readfirstlane(threadIdx.x / MS_WAVE);
+  const int waves = blockDim.x / MS_WAVE;
+  const int r = lane & 15, g = lane >> 4;
+  const int per = slice_steps(K), steps = (K + STEP - 1) / STEP, slices = (steps + per - 1) / per, groups = (slices + S - 1) / S;
+  const int n0 = blockIdx.x * R;
+  // the row of W that is the product's row n0 + i (q/k/v: the first halves of R / 2 rotary pairs, then the second)
+  auto row_of_w = [&](int i) {
+    if constexpr (EPI == F32_QKV) {
+      const int half = front.d / 2, p = n0 / 2 + i % (R / 2), head = p / half;
+      return head * front.d + p - head * half + (i / (R / 2)) * half;
+    }
+    return min(n0 + i, N - 1);
+  };
+  const float* wrow = W + (size_t)row_of_w(r % X % R) * ldw;
+  const float* arow = A + (size_t)min(r % X, M - 1) * lda;
+  float* h = part + slices * X * R;
+  const int ldh = K + 4;
+  const float* hrow = h + min(r % X, M - 1) * ldh;
+  const int jump = (waves * S - 1) * per * STEP + STEP;   // from a group's last step to the first of the wave's next
+  const int mine = (groups - wave + waves - 1) / waves * per;
+  f32x4 w[AHEAD], a[NORM ? 1 : AHEAD];
+  int ahead = 0, ahead_k = (wave * S + r / X) * per * STEP + 4 * g;      // step in its group and column of the next loads
+  auto fetch = [&](int u) {
+    w[u] = load4(wrow, ahead_k, K);
+    if constexpr (!NORM) a[u] = load4(arow, ahead_k, K);
+    if (++ahead == per) { ahead = 0; ahead_k += jump; }
+    else ahead_k += STEP;
+  };
+#pragma unroll
+  for (int u = 0; u < AHEAD; ++u)
+    if (u < mine) fetch(u);
+  if constexpr (NORM > 0) {
+    norm_rows<NORM>(A, norm.weight, norm.eps, h, ldh, M, K);
+    __syncthreads();
+  }
+  f32x4 acc = {0.f, 0.f, 0.f, 0.f};
+  int group = wave, at = 0, k = (wave * S + r / X) * per * STEP + 4 * g;
+  for (int s = 0; s < mine; s += AHEAD) {
+#pragma unroll
+    for (int u = 0; u < AHEAD; ++u) {
+      if (s + u >= mine) break;
+      const f32x4 wu = masked(w[u], k, K);
+      f32x4 au;
+      if constexpr (NORM > 0) au = masked(*reinterpret_cast<const f32x4*>(hrow + min(k, K - 4)), k, K);
+      else au = masked(a[u], k, K);
+      if (s + u + AHEAD < mine) fetch(u);
+      acc = step16(wu, au, acc);
+      k += STEP;
+      if (++at == per) {
+        // lane 16 g + c holds W's rows 4 g .. + 3 of the instruction (slice 4 g / X of the group) and token c % X of slice c / X
+        const int slice = group * S + r / X;
+        if (4 * g / X == r / X && 4 * g % X < R && slice < slices)
+          *reinterpret_cast<f32x4*>(&part[(slice * X + r % X) * R + 4 * g % X]) = acc;
+        acc = f32x4{0.f, 0.f, 0.f, 0.f};
+        at = 0;
+        group += waves;
+        k += jump - STEP;
+      }
+    }
+  }
+  __syncthreads();
+  auto sum = [&](int m, int i) {                     // of the product's row n0 + i
+    const int e = m * R + i;
+    float v = part[e];
+    for (int t = 1; t < slices; ++t) v += part[t * X * R + e];
+    return v;
+  };
+  if constexpr (EPI == F32_STORE) {
+    for (int e = threadIdx.x; e < M * R; e += blockDim.x) {
+      const int m = e / R, n = n0 + e % R;
+      if (n < N) store(C, (size_t)m * ldc + n, sum(m, e % R), bias, n, accumulate);
+    }
+  } else if constexpr (EPI == F32_SWIGLU) {          // rows 2 i and 2 i + 1: gate and up of feature i
+    for (int e = threadIdx.x; e < M * R / 2; e += blockDim.x) {
+      const int m = e / (R / 2), i = e % (R / 2) * 2;
+      if (n0 + i >= N) continue;
+      const float gate = sum(m, i), up = sum(m, i + 1);
+      C[(size_t)m * ldc + (n0 + i) / 2] = gate / (1.0f + expf(-gate)) * up;
+    }
+  } else {
+    for (int e = threadIdx.x; e < M * R / 2; e += blockDim.x) {
+      const int m = e / (R / 2), i = e % (R / 2), n = row_of_w(i), half = front.d / 2, head = n / front.d, j = n - head * front.d;
+      float x1 = sum(m, i), x2 = sum(m, i + R / 2);
+      if (bias) { x1 += bias[n]; x2 += bias[n + half]; }
+      if (head < front.nh + front.nkv) {
+        float sn, cs;
+        sincosf((float)front.positions[m] * front.inv_freq[j], &sn, &cs);
+        const float a1 = x1, a2 = x2;
+        x1 = a1 * cs - a2 * sn;
+        x2 = a2 * cs + a1 * sn;
+      }
+      if (head < front.nh) {
+        C[(size_t)m * ldc + n] = x1;
+        C[(size_t)m * ldc + n + half] = x2;
+        continue;
+      }
+      const long long slot = front.slots[m];
+      if (slot < 0) continue;
+      const long long page = slot / front.page_size;
+      const int off = (int)(slot - page * front.page_size);
+      const bool is_v = head >= front.nh + front.nkv;
+      const int kvh = head - front.nh - (is_v ? front.nkv : 0);
+      const size_t base = ((size_t)page * front.nkv + kvh) * front.page_size * front.d;
+      if (is_v && front.v_transposed) {
+        front.v_pages[base + (size_t)j * front.page_size + off] = x1;
+        front.v_pages[base + (size_t)(j + half) * front.page_size + off] = x2;
+      } else {
+        float* to = (is_v ? front.v_pages : front.k_pages) + base + (size_t)off * front.d + j;
+        to[0] = x1;
+        to[half] = x2;
+      }
+    }
+  }
+}
+
 // T x T tile: 4 waves of (T / 2) x (T / 2), F x F fragments each.
 template <int T>
 __global__ void __launch_bounds__(256)
@@ -306,9 +483,66 @@ gemm_f32_tiled_kernel(const float* __restrict__ A, const float* __restrict__ W, 
   }
 }
 
-int g_kernel = 0;      // measurements: 1 the kernel of few rows, 2 and 3 the tiled one with tiles of 64 and 32; 0 leaves the choice
+int g_kernel = 0;      // measurements: 1 the kernel of up to 64 rows, 2 and 3 the tiled one with tiles of 64 and 32, 4 and 5 that of up to 8 with blocks of 4 and 8 rows of W; 0 leaves the choice
+
+// Rows of W to a block of the kernel of slices side by side, for a plain product; 0: another kernel is as fast or faster.  us with four steps
+// to a load | so, at 3 and 8 tokens: 896 x 896 4.6 | 4.4 (8: 5.0 | 5.1), 896 x 4,864 11.4 | 8.5 and 12.9 | 12.3; 8 rows: 2,048 x 2,048
+// 7.5 | 7.0 and 8.0 | 7.8, 6,144 x 1,536 15.0 | 12.1 and 15.7 | 15.2, 4,608 x 3,584 26.3 | 22.3 but at 8 26.3 | 28.7; 3,584 x 18,944 62 | 71;
+// 384 x 192 3.1 | 3.3; 9,728 x 896 11.4 | 11.0 and 12.4 | 14.3.
+int diagonal_rows(int M, int N, int K) {
+  const int cus = ms_compute_units();
+  if (M > 8 || K < 512 || K > (M <= 4 ? 5120 : 4992)) return 0;
+  if ((N + 3) / 4 <= cus) return M <= 4 || K > 1024 ? 4 : 0;
+  return (N + 7) / 8 <= 3 * cus && K > 1024 && (M <= 4 || K <= 2048) ? 8 : 0;
+}
+
+// Floats of LDS.
+int diagonal_lds(int M, int K, int R, int X, bool normed) {
+  const int steps = (K + STEP - 1) / STEP, per = slice_steps(K);
+  return (steps + per - 1) / per * X * R + (normed ? M * (K + 4) : 0);
+}
+
+template <int R, int X, int EPI, int NORM>
+int launch_diagonal_as(const float* A, const float* W, const float* bias, float* C, int M, int N, int K, size_t lda, size_t ldw, size_t ldc,
+                       int accumulate, const F32Norm& norm, const F32Front& front, hipStream_t stream) {
+  const int steps = (K + STEP - 1) / STEP, per = slice_steps(K), slices = (steps + per - 1) / per;
+  const int groups = (slices + 16 / X - 1) / (16 / X), blocks = (N + R - 1) / R;
+  const int waves = groups > 4 && blocks > 2 * ms_compute_units() ? 4 : groups;
+  gemm_f32_diagonal_kernel<R, X, EPI, NORM><<<blocks, waves * MS_WAVE, diagonal_lds(M, K, R, X, NORM > 0) * sizeof(float), stream>>>(
+      A, W, bias, C, M, N, K, lda, ldw, ldc, accumulate, norm, front);
+  return ms_launch_status();
+}
+
+// M <= 8, R rows of W a block.
+template <int EPI, int NORM>
+int launch_diagonal(int R, const float* A, const float* W, const float* bias, float* C, int M, int N, int K, size_t lda, size_t ldw, size_t ldc,
+                    int accumulate, const F32Norm& norm, const F32Front& front, hipStream_t stream) {
+#define GO(R_, X_) return launch_diagonal_as<R_, X_, EPI, NORM>(A, W, bias, C, M, N, K, lda, ldw, ldc, accumulate, norm, front, stream)
+  if (R == 4 && M <= 4) GO(4, 4);
+  if (R == 4) GO(4, 8);
+  GO(8, 8);
+#undef GO
+}
 
 }  // namespace
+
+// What a decode step's layer makes of up to 8 rows of the residual stream x [M, K] with the norm of its reader, one kernel each:
+// the gated product, act [M, N / 2] = silu(gate) * up over interleaved rows of W, and q, k and v with their bias, q to q_out's rows of
+// (nh + 2 nkv) d, k and v to their pages.  The bits are those of ms_rms_norm, ms_gemm_generic and ms_silu_mul or ms_rope_store one after the other.
+// MS_UNSUPPORTED: sizes or addresses that the kernel does not take.
+int ms_gemm_f32_normed(const float* x, const float* W, const float* bias, float* out, int M, int N, int K, const F32Norm& norm,
+                       const F32Front* front, hipStream_t stream) {
+  if (M > 8 || K % 4 || K > 2048 || ((uintptr_t)x | (uintptr_t)W | (uintptr_t)norm.weight) % 16) return MS_UNSUPPORTED;
+  if (front ? front->d % 8 || N != (front->nh + 2 * front->nkv) * front->d : N % 2) return MS_UNSUPPORTED;
+  if ((long long)N * K > 32000000) return MS_UNSUPPORTED;      // (64,000 x 1,536 at 8 rows: 119 us so, 101 in the kernel of four steps to a load)
+  const int R = (N + 3) / 4 <= 2 * ms_compute_units() ? 4 : 8, X = R == 4 && M <= 4 ? 4 : 8;
+  if (diagonal_lds(M, K, R, X, true) * sizeof(float) > 65536) return MS_UNSUPPORTED;      // what a launch may ask for without more ado
+  const size_t ldc = front ? N : N / 2;
+#define GO(EPI, NORM) return launch_diagonal<EPI, NORM>(R, x, W, bias, out, M, N, K, K, K, ldc, 0, norm, front ? *front : F32Front{}, stream)
+  if (front) { if (K <= 1024) GO(F32_QKV, 4); else GO(F32_QKV, 8); }
+  if (K <= 1024) GO(F32_SWIGLU, 4); else GO(F32_SWIGLU, 8);
+#undef GO
+}
 
 extern "C" void ms_gemm_f32_force(int kernel) { g_kernel = kernel; }
 
@@ -321,6 +555,9 @@ int ms_gemm_f32_launch(const float* A, const float* W, const float* bias, float*
   // of 9,728 x 896 19.3 and 19.1), 33 to 64 from 32 a CU on (64 of 9,728 x 896 33 and 24, of 151,936 x 896 405 and 220, of
   // 6,144 x 2,048 43 and 40, but 33 of them 33 and 40).
   const bool few = M <= 16 || (M <= 32 ? N < 64 * cus : M <= 64 && N < 32 * cus);
+  const int side_by_side = M > 8 ? 0 : g_kernel == 4 ? 4 : g_kernel == 5 ? 8 : g_kernel == 0 ? diagonal_rows(M, N, K) : 0;
+  if (side_by_side)
+    return launch_diagonal<F32_STORE, 0>(side_by_side, A, W, bias, C, M, N, K, lda, ldw, ldc, accumulate, F32Norm{}, F32Front{}, stream);
   if (g_kernel == 1 ? M <= 64 : g_kernel == 0 && few) {
     // Rows a block: as few as keep the blocks within the CUs, because a CU reads at a rate of its own and 16 bytes a lane
     // fill 64-byte pieces from 4 rows as from 16 (3 rows of 896 x 4,864: 18.3 us as 56 blocks of 16, 17.2 as 224 of 4;

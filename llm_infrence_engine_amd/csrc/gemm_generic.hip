@@ -3,6 +3,7 @@
 // 16-byte pieces (the others go to csrc/gemm_f32.hip).  Every output element sums its K products in the same
 // order whatever M is, so a token's result does not depend on what else is in the batch.
 #include "common.h"
+#include "gemm_f32.h"
 #include "api.h"
 
 namespace {
@@ -81,9 +82,6 @@ gemm_generic_kernel(const TA* __restrict__ A, const TA* __restrict__ W, const fl
 }
 
 }  // namespace
-
-int ms_gemm_f32_launch(const float* A, const float* W, const float* bias, float* C, int M, int N, int K, size_t lda,
-                       size_t ldw, size_t ldc, int accumulate, hipStream_t stream);     // csrc/gemm_f32.hip
 
 namespace {
 

@@ -629,6 +629,30 @@ def test_float_layers_of_an_odd_width_are_the_parts_one_by_one(ops, tokens):
     assert all(torch.equal(a, b) for a, b in zip(*got))
 
 
+@pytest.mark.gpu
+@pytest.mark.parametrize("tokens", [[1], [1] * 4, [3, 2], [1] * 8, [1] * 9])
+@pytest.mark.parametrize("sizes", [dict(hidden_size=1280, intermediate_size=200, num_attention_heads=20, num_key_value_heads=4),
+                                   dict(hidden_size=2052, intermediate_size=36, num_attention_heads=6, num_key_value_heads=6, head_dim=16),
+                                   dict(hidden_size=96, intermediate_size=10, num_attention_heads=2, num_key_value_heads=1, head_dim=24),
+                                   dict(hidden_size=128, intermediate_size=2100, num_attention_heads=2, num_key_value_heads=2)])
+def test_norms_rotation_and_gate_within_32_bit_products_are_the_parts_one_by_one(ops, sizes, tokens):
+    """Up to 8 tokens the norms, the rotation with the cache store and the gate go with the products: the same bits as one by one,
+    for norms of more and of fewer threads, a width that the products leave to the parts (2,052), widths of W that are no whole blocks,
+    heads whose halves are a few blocks, blocks of 4 and of 8 rows, and 9 tokens, which are the parts again."""
+    from llm_infrence_engine_amd.engine import ModelRunner
+    from llm_infrence_engine_amd.engine.batch import StepEntry
+
+    model = _small_model(torch.float32, std=0.05, num_hidden_layers=2, max_position_embeddings=64, **sizes)
+    got = []
+    for whole in (True, False):
+        r = ModelRunner(model, 16, 32, 16, 64)
+        if not whole:
+            r.chains["float"] = None
+        out = [r.step([StepEntry(i, [(7 * i + j) % 64 for j in range(n)], [n - 1]) for i, n in enumerate(tokens)]).cpu() for _ in range(3)]
+        got.append(out + [t.cpu() for pages in r.pools.pages for t in pages.values()])
+    assert all(torch.equal(a, b) for a, b in zip(*got))
+
+
 @pytest.fixture(scope="module")
 def chained_model():
     return _small_model(torch.bfloat16, seed=5, std=0.05, hidden_size=768, intermediate_size=2048, num_hidden_layers=3, num_attention_heads=12,

@@ -2248,3 +2248,32 @@ def test_splits_are_put_together(ops, nh, nkv, d, keys, cap):
     size = (w.unsqueeze(1) @ v.abs()).reshape(-1)
     assert ((out[0].double() - want).abs() <= 2 ** -7 * size + 1e-6).all()
     assert (out[1] == 7.0).all()
+
+
+@pytest.mark.parametrize("N,K", [(4, 512), (90, 896), (896, 4864), (1031, 1028), (2053, 1100), (1500, 2052), (2048, 16)])
+def test_32_bit_products_of_up_to_8_rows_have_the_bits_of_the_kernel_for_64(ops, N, K):
+    """Blocks of 4 and of 8 rows of W whose instructions hold two or four slices side by side, for one to eight tokens: columns that
+    end within a slice, a step or a piece, slices that are not a whole number of instructions, rows past the last; with bias and
+    added onto what is there.  The kernel of up to 64 rows sums in the same order, and its own test holds it against 64 bits."""
+    from llm_infrence_engine_amd.kernels import build
+
+    lib = build.load()
+    g = torch.Generator(device=DEV).manual_seed(N + K)
+    a, w = (torch.randn(n, K, generator=g, device=DEV) for n in (8, N))
+    bias, there = torch.randn(N, generator=g, device=DEV), torch.randn(8, N, generator=g, device=DEV)
+
+    def run(kind, M, plain):
+        lib.ms_gemm_f32_force(kind)
+        try:
+            out = there[:M].clone()
+            return ops.gemm_generic(a[:M], w, out, bias=None if plain else bias, accumulate=not plain)
+        finally:
+            lib.ms_gemm_f32_force(0)
+
+    for plain in (True, False):
+        want = run(1, 8, plain)
+        exact = a.double() @ w.double().T + (0 if plain else bias.double() + there.double())
+        torch.testing.assert_close(want.double(), exact, atol=K ** 0.5 * 2e-6, rtol=2e-5)      # (sums of K products of about one)
+        for kind in (4, 5, 0):
+            for M in (1, 2, 3, 4, 5, 8):
+                assert torch.equal(run(kind, M, plain), want[:M]), (kind, M, plain)
