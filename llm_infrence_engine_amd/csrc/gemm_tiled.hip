@@ -22,6 +22,7 @@
 // features of its token over its FT tiles and stores them as one run.
 #include "common.h"
 #include "api.h"
+#include <algorithm>
 #include <type_traits>
 
 namespace {
@@ -111,7 +112,7 @@ __device__ __forceinline__ void store_run_f32(float* o, const float* v, int run,
 }
 
 // WF x WT waves along features and tokens, each with FT x TT tiles of 16 x 16.  K is a multiple of 64.
-template <int WF, int WT, int FT, int TT, int EPI, typename TO>
+template <int WF, int WT, int FT, int TT, int SW, int SA, int EPI, typename TO>
 __global__ void __launch_bounds__(WF * WT * MS_WAVE)
 gemm_tiled_kernel(const bf16* __restrict__ A, size_t lda, const bf16* __restrict__ W, size_t ldw,
                   TO* __restrict__ out, size_t ldo, int M, int N, int K, int m_tiles, int n_tiles, int xm, int parts,
@@ -123,33 +124,34 @@ gemm_tiled_kernel(const bf16* __restrict__ A, size_t lda, const bf16* __restrict
   constexpr int LOADS_W = (BN / 8 + NWAVES - 1) / NWAVES, LOADS_A = (BM / 8 + NWAVES - 1) / NWAVES;
   constexpr int SLOT_W = BN * PITCH, SLOT_A = BM * PITCH;
   extern __shared__ __align__(16) unsigned char lds_raw[];
-  bf16* lds = reinterpret_cast<bf16*>(lds_raw);          // three slots of BN rows of W, two of BM rows of A
+  bf16* lds = reinterpret_cast<bf16*>(lds_raw);          // SW slots of BN rows of W, SA of BM rows of A
 
-  // Blocks with consecutive ids go to consecutive XCDs, each with an L2 of its own.  The 8 XCDs are laid over the
-  // tiles as xm x (8 / xm): an XCD takes every xm-th token tile and every (8 / xm)-th tile of W, its token tiles
-  // running fastest (they share a tile of W at the same time).  With xm = 1 a tile of W is read from memory by
-  // one XCD only and every XCD reads all of A; a larger xm leaves an XCD 1 / xm of A to keep in its L2.  The host
-  // launches 8 * ceil(m_tiles / xm) * ceil(n_tiles / (8 / xm)) blocks; one without a tile leaves.
+  // Blocks with consecutive ids go to consecutive XCDs, each with an L2 of its own.  With xm = 1 the tiles, token tiles running
+  // fastest (they share a tile of W at the same time), are dealt out over the XCDs in equal runs: a tile of W is read from memory
+  // by one XCD, or by the two at a run's end, every XCD reads all of A, and no XCD has a round of its CUs more than others (by whole rows
+  // of tiles, 51 over 8 XCDs, 255 tiles took two: 23.3 us, 15.0 so).  Else the 8 XCDs are laid over the tiles as xm x (8 / xm): an XCD takes every xm-th token tile and
+  // every (8 / xm)-th tile of W, which leaves it 1 / xm of A to keep in its L2; the host launches 8 * ceil(m_tiles / xm) *
+  // ceil(n_tiles / (8 / xm)) blocks.  One without a tile leaves.
   const int xcd = blockIdx.x & 7;
   const int local = (int)(blockIdx.x >> 3);
-  const int xn = 8 / xm, mi = (m_tiles + xm - 1) / xm;
   int steps = K / BK;
   int nt = 0, mt = 0;
-  if (EPI == EPI_SUMS) {
-    // a run of the columns: the parts one after the other, each with all tiles, dealt out over the XCDs in equal runs (there is
-    // about a block for every CU: by rows of tiles, 14 over 8 XCDs, some CUs would get two and others none)
-    const int all = m_tiles * n_tiles * parts, per = (all + 7) / 8, id = xcd * per + local;
+  if (EPI == EPI_SUMS || (EPI != EPI_GROUPED && xm == 1)) {
+    // (partial sums: the runs of the columns one after the other, each with all tiles)
+    const int to_a_part = m_tiles * n_tiles, all = to_a_part * parts, per = (all + 7) / 8, id = xcd * per + local;
     if (local >= per || id >= all) return;
-    const int part = id / (m_tiles * n_tiles), tile = id - part * (m_tiles * n_tiles);
+    const int part = EPI == EPI_SUMS ? id / to_a_part : 0, tile = id - part * to_a_part;
     nt = tile / m_tiles;
     mt = tile - nt * m_tiles;
-    const int from = (int)((long long)steps * part / parts), to = (int)((long long)steps * (part + 1) / parts);
-    steps = to - from;
-    A += (size_t)from * BK;
-    W += (size_t)from * BK;
-    out += (size_t)part * M * N;
-  }
-  if (EPI != EPI_SUMS) {
+    if (EPI == EPI_SUMS) {
+      const int from = (int)((long long)steps * part / parts), to = (int)((long long)steps * (part + 1) / parts);
+      steps = to - from;
+      A += (size_t)from * BK;
+      W += (size_t)from * BK;
+      out += (size_t)part * M * N;
+    }
+  } else {
+    const int xn = 8 / xm, mi = (m_tiles + xm - 1) / xm;
     nt = (local / mi) * xn + xcd / xm;
     mt = (local % mi) * xm + xcd % xm;
   }
@@ -191,7 +193,7 @@ gemm_tiled_kernel(const bf16* __restrict__ A, size_t lda, const bf16* __restrict
   auto load_a = [&](int p, int step, int slot) {
     if ((p + 1) * NWAVES * 8 <= BM || (wave + p * NWAVES) * 8 < BM)
       __builtin_amdgcn_global_load_lds((global_void*)(src_a[p] + step * BK),
-                                       (lds_void*)(lds + 3 * SLOT_W + slot + (wave + p * NWAVES) * 8 * PITCH), 16, 0, 0);
+                                       (lds_void*)(lds + SW * SLOT_W + slot + (wave + p * NWAVES) * 8 * PITCH), 16, 0, 0);
   };
   constexpr int FEWEST_W = BN / 8 / NWAVES, FEWEST_A = BM / 8 / NWAVES;   // loads every wave makes
 
@@ -206,7 +208,7 @@ gemm_tiled_kernel(const bf16* __restrict__ A, size_t lda, const bf16* __restrict
   static_assert(BK == 64, "a step is two products of 32 columns deep");
   const int place0 = (kq ^ (col & 7)) * 8, place1 = ((kq + 4) ^ (col & 7)) * 8;
   const bf16* w_frag = lds + (wf * FT * 16 + col) * PITCH;
-  const bf16* a_frag = lds + 3 * SLOT_W + (wt * TT * 16 + col) * PITCH;
+  const bf16* a_frag = lds + SW * SLOT_W + (wt * TT * 16 + col) * PITCH;
 
   // A step is four blocks of products, two to each half of its columns; a block's fragments of W (a half's FT lie in a ring
   // of FT registers) and, before a half, its TT fragments of the tokens are read beside the first products of the block
@@ -226,20 +228,23 @@ gemm_tiled_kernel(const bf16* __restrict__ A, size_t lda, const bf16* __restrict
   auto read_a = [&](int half, int j, int slot) {
     a[half][j] = *reinterpret_cast<const bf16x8*>(a_frag + slot + j * 16 * PITCH + (half ? place1 : place0));
   };
-  // mode 2: the step after next is asked for; 1: there is none; 0: the last step, nothing follows
-  auto step = [&](auto mode_c, int s, int slot_w, int next_w, int free_w, int slot_a, int next_a) {
-    constexpr int MODE = decltype(mode_c)::value;
+  // LEFT: steps that follow, as far as it matters (AHEAD or more: of those to come, W's step SW - 1 on and A's step SA on are asked for)
+  constexpr int AHEAD = SA;
+  static_assert(SA == SW || SA == SW - 1, "which loads are under way at a barrier is counted for these");
+  auto step = [&](auto left_c, int s, int slot_w, int next_w, int free_w, int slot_a, int next_a) {
+    constexpr int LEFT = decltype(left_c)::value;
+    constexpr bool ASK_W = LEFT >= SW - 1, ASK_A = LEFT >= SA;
+    // loads under way that are newer than the next step's: of W and A for the steps behind it, and of W alone for the one asked for first
+    constexpr int BEHIND = LEFT >= SA ? SW - 3 + (SA == SW) : LEFT - 1, NEWER = BEHIND * (FEWEST_W + FEWEST_A) + (LEFT >= SA && SA < SW ? FEWEST_W : 0);
 #pragma unroll
     for (int block = 0; block < 4; ++block) {
       const int half = block >> 1, i0 = block & 1 ? HALF : 0, i1 = block & 1 ? FT : HALF;
-      if (MODE > 0 && block == 3) {
-        // (of the loads under way, only those of the step after next of W may still be)
-        if (MODE == 2) asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"(FEWEST_W) : "memory");
-        else asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");
+      if constexpr (LEFT > 0) {
+        if (block == 3) asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"(NEWER) : "memory");
       }
       // what the next block needs: tiles r0 .. r1 - 1 of W and, when it begins a half, the tokens' fragments
       const int r0 = block & 1 ? 0 : HALF, r1 = block & 1 ? HALF : FT, of_a = block & 1 ? TT : 0;
-      const int reads = block == 3 && MODE == 0 ? 0 : r1 - r0 + of_a, spread = i1 - i0 > 2 ? 2 : 1;
+      const int reads = block == 3 && LEFT == 0 ? 0 : r1 - r0 + of_a, spread = i1 - i0 > 2 ? 2 : 1;
 #pragma unroll
       for (int i = i0; i < i1; ++i) {
 #pragma unroll
@@ -252,46 +257,80 @@ gemm_tiled_kernel(const bf16* __restrict__ A, size_t lda, const bf16* __restrict
 #pragma unroll
         for (int j = 0; j < TT; ++j)
           acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wr[i], a[half][j], acc[i][j], 0, 0, 0);
-        if (MODE == 2 && block == 0) {
+        if (ASK_W && block == 0) {
 #pragma unroll
-          for (int p = 0; p < LOADS_W; ++p) if (p * (i1 - i0) / LOADS_W == i - i0) load_w(p, s + 2, free_w);
+          for (int p = 0; p < LOADS_W; ++p) if (p * (i1 - i0) / LOADS_W == i - i0) load_w(p, s + SW - 1, free_w);
         }
-        if (MODE == 2 && block == 3) {
+        if (ASK_A && block == 3) {
 #pragma unroll
-          for (int p = 0; p < LOADS_A; ++p) if (p * (i1 - i0) / LOADS_A == i - i0) load_a(p, s + 2, slot_a);
+          for (int p = 0; p < LOADS_A; ++p) if (p * (i1 - i0) / LOADS_A == i - i0) load_a(p, s + SA, slot_a);
         }
         __builtin_amdgcn_sched_barrier(0);
       }
     }
   };
+  // The q/k/v epilogue's inputs (heads of 64): asked for before the first rows of W, so that they have long come when the sums are there.
+  constexpr bool EARLY = EPI == EPI_QKV && FT == 4 && TT == 1;
+  constexpr int EJ = EARLY ? TT : 1, ER = EARLY ? 4 * FT : 1;
+  float2 turns[EJ][ER];
+  float biases[ER];
+  int slots[EJ];
+  if constexpr (EARLY) {
+    const int head = (n0 + wf * FT * 16) / (FT * 16);
+    const bool live = head < qkv.nh + 2 * qkv.nkv, rotated = head < qkv.nh + qkv.nkv;
+    if (live) {
 #pragma unroll
-  for (int first = 0; first < 2; ++first) {
-    if (first < steps) {
+      for (int g = 0; g < ER; ++g) biases[g] = qkv.bias ? qkv.bias[(size_t)head * FT * 16 + kq * ER + g] : 0.f;
+#pragma unroll
+      for (int j = 0; j < EJ; ++j) {
+        const int mm = min(m0 + wt * TT * 16 + j * 16 + col, M - 1);
+        slots[j] = head < qkv.nh ? -1 : qkv.slots[mm];
+        if (rotated) {
+          const float2* turn = qkv.table + (size_t)mm * (FT * 8) + (kq & 1) * ER;
+#pragma unroll
+          for (int g = 0; g < ER; ++g) turns[j][g] = turn[g];
+        }
+      }
+    }
+  }
+#pragma unroll
+  for (int first = 0; first < SA; ++first) {
+    if (first < SW - 1 && first < steps) {
 #pragma unroll
       for (int p = 0; p < LOADS_W; ++p) load_w(p, first, first * SLOT_W);
+    }
+    if (first < steps) {
 #pragma unroll
       for (int p = 0; p < LOADS_A; ++p) load_a(p, first, first * SLOT_A);
     }
   }
-  if (steps > 1) asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"(FEWEST_W + FEWEST_A) : "memory");
+  if (steps >= SA) asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"((SW - 2) * FEWEST_W + (SA - 1) * FEWEST_A) : "memory");
   else asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");
 #pragma unroll
   for (int j = 0; j < TT; ++j) read_a(0, j, 0);
 #pragma unroll
   for (int i = 0; i < HALF; ++i) read_w(0, i, 0);
   int sw = 0, sa = 0;      // the current step's slots
-  auto after_w = [&](int slot) { return slot == 2 * SLOT_W ? 0 : slot + SLOT_W; };
-  for (int s = 0; s + 2 < steps; ++s) {
-    step(std::integral_constant<int, 2>{}, s, sw, after_w(sw), after_w(after_w(sw)), sa, SLOT_A - sa);
+  auto after_w = [&](int slot) { return slot == (SW - 1) * SLOT_W ? 0 : slot + SLOT_W; };
+  auto after_a = [&](int slot) { return slot == (SA - 1) * SLOT_A ? 0 : slot + SLOT_A; };
+  auto before_w = [&](int slot) { return slot == 0 ? (SW - 1) * SLOT_W : slot - SLOT_W; };
+  int at = 0;
+  for (; at + AHEAD < steps; ++at) {
+    step(std::integral_constant<int, AHEAD>{}, at, sw, after_w(sw), before_w(sw), sa, after_a(sa));
     sw = after_w(sw);
-    sa = SLOT_A - sa;
+    sa = after_a(sa);
   }
-  if (steps > 1) {
-    step(std::integral_constant<int, 1>{}, 0, sw, after_w(sw), 0, sa, SLOT_A - sa);
-    sw = after_w(sw);
-    sa = SLOT_A - sa;
-  }
-  step(std::integral_constant<int, 0>{}, 0, sw, 0, 0, sa, 0);
+  auto last_steps = [&](auto self, auto left_c) -> void {
+    constexpr int LEFT = decltype(left_c)::value;
+    if (steps - at > LEFT) {      // (fewer steps than slots: the pipeline never fills)
+      step(left_c, at, sw, after_w(sw), before_w(sw), sa, after_a(sa));
+      sw = after_w(sw);
+      sa = after_a(sa);
+      ++at;
+    }
+    if constexpr (LEFT > 0) self(self, std::integral_constant<int, LEFT - 1>{});
+  };
+  last_steps(last_steps, std::integral_constant<int, AHEAD - 1>{});
 
   // the lane's run of 4 FT features of token m (tile j): acc[i][j][r] is feature f0 + i * 4 + r
   const int f0 = n0 + wf * (FT * 16) + kq * (4 * FT);
@@ -318,7 +357,7 @@ gemm_tiled_kernel(const bf16* __restrict__ A, size_t lda, const bf16* __restrict
         if (head < qkv.nh) {
           dst = reinterpret_cast<bf16*>(out) + (size_t)m * ldo + (size_t)head * D + e0;
         } else {
-          const long long slot = qkv.slots[m];
+          const long long slot = EARLY ? slots[EARLY ? j : 0] : qkv.slots[m];
           if (slot >= 0) {
             const long long page = slot / qkv.page_size;
             const int off = (int)(slot - page * qkv.page_size);
@@ -337,9 +376,9 @@ gemm_tiled_kernel(const bf16* __restrict__ A, size_t lda, const bf16* __restrict
 #pragma unroll
         for (int e = 0; e < 8; ++e) {
           const int g = g0 + e;
-          float v = acc[g >> 2][j][g & 3] + (bias ? bias[g] : 0.f);
+          float v = acc[g >> 2][j][g & 3] + (EARLY ? biases[EARLY ? g : 0] : bias ? bias[g] : 0.f);
           if (rotated) {
-            const float2 cs = turn[g];
+            const float2 cs = EARLY ? turns[EARLY ? j : 0][EARLY ? g : 0] : turn[g];
             const float other = __shfl_xor(v, 32);
             v = kq < 2 ? v * cs.x - other * cs.y : v * cs.x + other * cs.y;
           }
@@ -416,24 +455,24 @@ int choose_xcd_split(int M) {
   return M >= 6144 ? 4 : (M >= 4096 ? 2 : 1);
 }
 
-template <int WF, int WT, int FT, int TT, int EPI, typename TO>
+template <int WF, int WT, int FT, int TT, int SW, int SA, int EPI, typename TO>
 int launch(const bf16* A, size_t lda, const bf16* W, size_t ldw, TO* out, size_t ldo, int M, int N, int K,
            hipStream_t stream, const QkvEpilogue& qkv = QkvEpilogue{}, const GroupedRows& grp = GroupedRows{}, int parts = 1) {
   constexpr int BN = WF * FT * 16, BM = WT * TT * 16;
-  constexpr size_t lds = (size_t)(3 * BN + 2 * BM) * PITCH * sizeof(bf16);
+  constexpr size_t lds = (size_t)(SW * BN + SA * BM) * PITCH * sizeof(bf16);
   static bool raised = false;   // once per instantiation: allow more dynamic LDS than the default 64 KB
   if (!raised) {
-    if (hipFuncSetAttribute(reinterpret_cast<const void*>(&gemm_tiled_kernel<WF, WT, FT, TT, EPI, TO>),
+    if (hipFuncSetAttribute(reinterpret_cast<const void*>(&gemm_tiled_kernel<WF, WT, FT, TT, SW, SA, EPI, TO>),
                             hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds) != hipSuccess)
       return MS_LAUNCH_FAILED;
     raised = true;
   }
   const int n_tiles = (N + BN - 1) / BN, m_tiles = (M + BM - 1) / BM;
   const int xm = choose_xcd_split(M);
-  const long long blocks = EPI == EPI_SUMS ? ((long long)m_tiles * n_tiles * parts + 7) / 8 * 8
-                                           : 8LL * ((m_tiles + xm - 1) / xm) * ((n_tiles + 8 / xm - 1) / (8 / xm));
+  const long long blocks = EPI == EPI_SUMS || xm == 1 ? ((long long)m_tiles * n_tiles * parts + 7) / 8 * 8
+                                                      : 8LL * ((m_tiles + xm - 1) / xm) * ((n_tiles + 8 / xm - 1) / (8 / xm));
   if (blocks > 0x7fffffffLL) return MS_UNSUPPORTED;
-  gemm_tiled_kernel<WF, WT, FT, TT, EPI, TO><<<dim3((unsigned)blocks), dim3(WF * WT * MS_WAVE), lds, stream>>>(
+  gemm_tiled_kernel<WF, WT, FT, TT, SW, SA, EPI, TO><<<dim3((unsigned)blocks), dim3(WF * WT * MS_WAVE), lds, stream>>>(
       A, lda, W, ldw, out, ldo, M, N, K, m_tiles, n_tiles, xm, parts, qkv, grp);
   return ms_launch_status();
 }
@@ -453,7 +492,7 @@ int launch_grouped(const bf16* A, size_t lda, const bf16* W, TO* out, size_t ldo
   constexpr size_t lds = (size_t)(3 * BN + 2 * BM) * PITCH * sizeof(bf16);
   static bool raised = false;
   if (!raised) {
-    if (hipFuncSetAttribute(reinterpret_cast<const void*>(&gemm_tiled_kernel<WF, WT, FT, TT, EPI_GROUPED, TO>),
+    if (hipFuncSetAttribute(reinterpret_cast<const void*>(&gemm_tiled_kernel<WF, WT, FT, TT, 3, 2, EPI_GROUPED, TO>),
                             hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds) != hipSuccess)
       return MS_LAUNCH_FAILED;
     raised = true;
@@ -461,68 +500,68 @@ int launch_grouped(const bf16* A, size_t lda, const bf16* W, TO* out, size_t ldo
   const int n_tiles = (N + BN - 1) / BN;
   const long long blocks = 8LL * tiles * ((n_tiles + 7) / 8);
   if (blocks > 0x7fffffffLL) return MS_UNSUPPORTED;
-  gemm_tiled_kernel<WF, WT, FT, TT, EPI_GROUPED, TO><<<dim3((unsigned)blocks), dim3(WF * WT * MS_WAVE), lds, stream>>>(
+  gemm_tiled_kernel<WF, WT, FT, TT, 3, 2, EPI_GROUPED, TO><<<dim3((unsigned)blocks), dim3(WF * WT * MS_WAVE), lds, stream>>>(
       A, lda, W, (size_t)K, out, ldo, tiles * BM, N, K, tiles, n_tiles, 1, 1, QkvEpilogue{}, grp);
   return ms_launch_status();
 }
 
-int g_tile = 0;   // measurements: 0 leaves the choice of tile; 1 to 5 force one (256, 128, 64, 192, 160 features wide)
+// The tiles.  1 to 3 are as large as registers and LDS allow a block that has a CU to itself, two to a CU, four to a CU; 4 and 5 fill
+// rounds that 1 would not.  6 to 12 are for products that would leave CUs without a block, or one block to a CU: there a step is as long as its
+// loads take to come, so these have narrower tiles, that more CUs get one of, and as many slots as LDS holds.
+enum { T256 = 1, T128 = 2, T64 = 3, T192X256 = 4, T160X256 = 5, T64_DEEP = 6, T160X128 = 7, T192X128 = 8, T128X256 = 9, T96X128 = 10, T64X128 = 11, T128_DEEP = 12 };
 
-// The tile that takes the least time by a model of the measurements.  A block of 256 tokens by 256, 192 or 160
-// features has a CU to itself; a step of 64 columns takes 1.6, 1.3 or 1.3 us with all CUs at work, a tile 3 us more for
-// its start and end, and the tiles run in whole rounds over the CUs: the narrower tiles pay where they fill the rounds
-// better (2,048 tokens of the 0.5B gate/up shape: 304 tiles of 256 features take two rounds, 44.5 us; 408 of 192 two
-// shorter ones, 38.0; 1,024 tokens: 23.2 -> 20.8 in one round).  Tiles of 128 x 128 go two to a CU, 1.15 us a step each;
-// they end at different times, so their rounds are counted as they come, plus 0.3 for the last.  What counts is the order it
-// puts the tiles in: over 83 sizes (128 to 4,096 tokens, 1,024 to 55,296 features, 128 to 5,120 columns) its times run from 28 %
-// below the measured ones (128 columns 63 %) to 40 % above (a round that leaves CUs idle runs at a higher clock), most of them
-// 0 to 17 % above, and the tile it takes is within 5 % of the best one but for five sizes, 23 % behind at worst.  (Times here
-// and below: twelve products in a row in a graph, each with another W, which the last-level cache may hold; in a model's step,
-// between other kernels, 0.5B gate/up of 2,048 tokens takes 43 to 45 us.)
-struct TileChoice { int tile; double us; long long tiles, slots; };
+int g_tile = 0;   // measurements: 0 leaves the choice of tile, 1 to 12 force one
+
+// What takes a tile: us of a launch, of a round of tiles over the CUs, of a step of 64 columns in every round, and of a step with
+// all CUs at work beyond that.
+struct TileKind { int tile, features, tokens, to_a_cu; double fixed, round, step, busy; };
+constexpr TileKind KINDS[] = {{T256, 256, 256, 1, 0.06, 5.93, 0.98, 0.52},     {T128, 128, 128, 2, 2.02, 1.02, 0.46, 0.13},
+                              {T64, 64, 64, 4, 3.20, 0.00, 0.23, 0.01},        {T192X256, 192, 256, 1, 0.28, 5.24, 0.75, 0.44},
+                              {T160X256, 160, 256, 1, 0.58, 4.77, 0.73, 0.36}, {T64_DEEP, 64, 64, 2, 2.61, 0.25, 0.25, 0.00},
+                              {T160X128, 160, 128, 1, 1.58, 2.63, 0.49, 0.20}, {T192X128, 192, 128, 1, 1.56, 2.65, 0.51, 0.25},
+                              {T128X256, 128, 256, 1, 1.04, 3.31, 0.58, 0.31}, {T96X128, 96, 128, 1, 1.58, 2.21, 0.32, 0.16},
+                              {T64X128, 64, 128, 1, 1.62, 1.64, 0.25, 0.13}};
+
+// The tile that takes the least time by a model of the measurements: 200 sizes (65 to 4,096 tokens, 1,152 to 37,888 features,
+// 256 to 3,584 columns), every tile timed at each, every product by a W that lies in no cache.  Its times lie within 0.77 and 1.28 of the measured
+// ones (tiles with a CU to themselves 0.81 to 1.14), and the tile it takes is 0.4 % behind the best one on average, 12 % at worst; with 1 to 5 alone
+// the best is 9 % behind on average and up to 42 (0.5B gate/up, 9,728 x 896: 128 tokens 11.1 -> 9.3 us, 256 13.9 -> 10.9, 512 18.4 -> 13.6, 768 17.7 ->
+// 16.3, from 1,024 on the same; 5,632 x 2,048 at 256 tokens 20.8 -> 15.8, 37,888 x 3,584 at 128 80 -> 56).
+struct TileChoice { int tile, features, tokens; double us; long long tiles, slots; };
 
 TileChoice choose_tile(int M, int N, int K) {
   const long long cus = ms_compute_units();
   const double steps = (double)((K + BK - 1) / BK);
-  const long long small = (long long)((N + 127) / 128) * ((M + 127) / 128);
-  // Fewer tiles of 128 x 128 than CUs: tiles of 64 x 64 (four waves) put four times as many CUs to work, and a tile's time is
-  // the time its CU needs to draw its rows; four of them fit a CU (40 KB of LDS each).  Time with 128 over time with 64, at 270
-  // sizes: 0.99 to 1.39 up to two tiles of 64 a CU (gate/up of the 0.5B shape at 160 tokens 9.9 and 8.6 us, 4,096 x 1,024 at
-  // 512 tokens 10.3 and 9.3), and either way from there to four (6,144 x 768 at 640 tokens 10.4 and 12.8, 2,560 x 1,024 at
-  // 1,534 tokens 15.4 and 14.1; 0.88 to 1.28 up to 512 columns, 0.78 to 1.13 up to 1,024, 0.67 to 1.05 beyond).  From the CUs on:
-  // 512 tokens of gate/up 14.6 and 17.1.
-  if (small < cus) return {3, 0.0, (long long)((N + 63) / 64) * ((M + 63) / 64), 4 * cus};
-  TileChoice best{2, ((double)small / (double)(2 * cus) + 0.3) * 1.15 * steps, small, (small + 2 * cus - 1) / (2 * cus) * 2 * cus};
-  const struct { int tile, features; double step_us; } wide[] = {{1, 256, 1.60}, {4, 192, 1.30}, {5, 160, 1.30}};
-  for (const auto& w : wide) {
-    const long long tiles = (long long)((N + w.features - 1) / w.features) * ((M + 255) / 256);
-    const long long rounds = (tiles + cus - 1) / cus;
-    const double us = (double)rounds * (3.0 + steps * w.step_us);
-    if (us < best.us) best = {w.tile, us, tiles, rounds * cus};
+  TileChoice best{0, 0, 0, 1e30, 0, 0};
+  for (const TileKind& k : KINDS) {
+    const long long tiles = (long long)((N + k.features - 1) / k.features) * ((M + k.tokens - 1) / k.tokens), rounds = (tiles + cus - 1) / cus;
+    if (k.tile == T64 ? tiles <= 2 * cus : k.tile == T64_DEEP && tiles > 2 * cus) continue;      // (two of the deep ones share a CU)
+    const double share = (double)tiles / (double)cus;
+    const double us = k.fixed + (double)rounds * (k.round + steps * k.step) + steps * k.busy * (k.to_a_cu == 1 ? share : std::min(1.0, share));
+    const long long places = cus * k.to_a_cu;
+    if (us < best.us) best = {k.tile, k.features, k.tokens, us, tiles, (tiles + places - 1) / places * places};
   }
   return best;
 }
 
-// Tile and column parts of a product in partial sums, the least time by a model of the measurements: a start and a step of 64
-// columns by how many blocks share a CU (by how many CUs are at work, for tiles of 256), rounds over the CUs, and a write and a
-// read of every sum at 5 TB/s.
+// Tile and column parts of a product in partial sums, the least time by such a model (100 sizes, 768 to 3,584 features, 896 to 18,944
+// columns, 65 to 2,048 tokens: 2.6 % behind the best on average): a launch, a round and its steps, what a block more costs its CU, and a write and a read
+// of every sum at 5 TB/s.  With the two deep tiles 0.5B down projections take 1 to 2 us less (896 x 4,864: 65 tokens 8.3 -> 7.2, 512 17.9 -> 16.9).
 struct SumsChoice { int tile, parts; double us; long long blocks; };
 
 SumsChoice choose_sums(int M, int N, int K) {
   const long long cus = ms_compute_units();
   const int steps = K / BK;
-  const struct { int tile, size, to_a_cu; double start_us[4], step_us[4]; } kinds[] = {
-      {1, 256, 1, {12.}, {1.05}}, {2, 128, 2, {9., 13.}, {0.55, 1.0}}, {3, 64, 4, {7., 7., 7., 8.}, {0.30, 0.43, 0.63, 0.82}}};
+  const struct { int tile, size; double fixed, round, step, block; } kinds[] = {{T256, 256, 2.28, 5.20, 1.11, 17.61}, {T128, 128, 3.51, 0.00, 0.50, 5.03},
+                                                                              {T64, 64, 3.96, 0.00, 0.25, 0.59},    {T128_DEEP, 128, 2.18, 1.14, 0.47, 5.88},
+                                                                              {T64_DEEP, 64, 3.07, 0.00, 0.25, 1.08}};
   SumsChoice best{0, 1, 1e30, 0};
   for (const auto& k : kinds) {
-    const long long tiles = (long long)((N + k.size - 1) / k.size) * ((M + k.size - 1) / k.size), slots = cus * k.to_a_cu;
-    for (int p = 1; p <= 8 && (p == 1 || p * 4 <= steps); ++p) {
+    const long long tiles = (long long)((N + k.size - 1) / k.size) * ((M + k.size - 1) / k.size);
+    for (int p = 1; p <= 8 && (p == 1 || p * 2 <= steps); ++p) {
       const long long blocks = tiles * p;
-      const int at = (int)(blocks >= slots ? k.to_a_cu : (blocks + cus - 1) / cus) - 1;
-      double rounds = (double)((blocks + slots - 1) / slots);
-      if (k.to_a_cu > 1 && rounds > 1) rounds = (double)blocks / (double)slots + 0.3;
-      const double step = k.step_us[at] + (k.to_a_cu == 1 ? 0.5 * (double)(blocks < cus ? blocks : cus) / (double)cus : 0.);
-      const double us = rounds * (k.start_us[at] + (steps + p - 1) / p * step) + (double)p * M * N * 8 / 5e6;
+      const double us = k.fixed + (double)((blocks + cus - 1) / cus) * (k.round + (steps + p - 1) / p * k.step) +
+                        k.block * (double)blocks / (double)cus + (double)p * M * N * 8 / 5e6;
       if (us < best.us) best = {k.tile, p, us, blocks};
     }
   }
@@ -534,37 +573,36 @@ SumsChoice choose_sums(int M, int N, int K) {
 extern "C" void ms_gemm_tiled_force(int tile) { g_tile = tile; }
 extern "C" void ms_gemm_tiled_force_xcd_split(int xm) { g_xcd_split = xm; }
 
-// What of the tiles' places the product fills: tiles in whole rounds over the CUs, counted for the XCD with the most of them.
-static double filled(int M, int N, const TileChoice& c) {
-  const int features = c.tile == 1 ? 256 : (c.tile == 4 ? 192 : (c.tile == 5 ? 160 : 128)), tokens = c.tile == 2 ? 128 : 256;
-  const int to_a_cu = c.tile == 2 ? 2 : 1, xm = choose_xcd_split(M), xn = 8 / xm, cus = ms_compute_units();
-  const long long n_tiles = (N + features - 1) / features, m_tiles = (M + tokens - 1) / tokens;
+// What of the tiles' places the product fills: tiles in whole rounds over the CUs.
+static double full(int M, int N, const TileChoice& c) { return (double)M * N / ((double)c.slots * c.features * c.tokens); }
+// The same with the rounds counted for the XCD with the most tiles, where these are laid over the XCDs in whole rows.
+static double full_in_rows(int M, int N, const TileChoice& c) {
+  const int to_a_cu = c.tile == T128 ? 2 : c.tile == T64 ? 4 : 1, xm = choose_xcd_split(M), xn = 8 / xm, cus = ms_compute_units();
+  const long long n_tiles = (N + c.features - 1) / c.features, m_tiles = (M + c.tokens - 1) / c.tokens;
   const long long most = ((n_tiles + xn - 1) / xn) * ((m_tiles + xm - 1) / xm), places = (long long)(cus + 7) / 8 * to_a_cu;
-  return (double)M * N / ((double)((most + places - 1) / places) * places * 8 * features * tokens);
+  return (double)M * N / ((double)((most + places - 1) / places) * places * 8 * c.features * c.tokens);
 }
 
 // Whether the gated product of M tokens is faster here than as the library's product and an activation kernel.  Time of these over
-// this kernel's, a different W every call, with silu (the gelu and the clamped gate, whose kernels cost more: 1.08 times that):
+// this kernel's, a different W every call, with silu (the gelu and the clamped gate, whose kernels cost more: 1.08 times that), at 190 sizes
+// of up to 2,048 tokens (65 on, 5,632 to 55,296 rows, 1,600 to 5,120 columns) and with the larger tiles at 687 of up to 4,096:
 //   up to 1,536 columns 1.02 to 2 (65 to 8,192 tokens);
-//   beyond, up to 2,048 tokens whose tiles fill 9/10 of their rounds: 0.99 to 1.3;
-//   687 other sizes of 1,600 to 5,120 columns (5,248 to 55,296 rows, 65 to 4,096 tokens), by what the tiles fill:
-//     up to 3,584 columns tiles of 192 or 160 features, the others from 0.65 on, and those of 128 up to 0.4 (one round that leaves CUs
-//     idle, as the library's does): 0.92 to 1.60, 1.14 on average, 12 of 409 below 0.97 (7B gate/up: 1,024 tokens 313 and 245 us, 2,176
-//     tokens 566 and 532; 256 tokens of 22,016 x 2,048 0.97, but four layers of that width 597 and 592 us); the others 0.71 to 1.38, 1.03
-//     on average (14,336 x 3,584, 300 tokens 55 and 62);
-//     4,096 to 5,120 columns beyond 512 tokens from 0.8 on: 0.91 to 1.58, 1.12 on average, 4 of 108 below 0.97; the others 0.80 to
-//     1.30, 1.01 on average;
+//   up to 2,048 tokens by up to 4,096 columns, of tiles that are 0.72 and more full, 0.95 to 1.82, 1.2 on average, and up to 128 tokens by up to
+//     3,584 columns 0.99 to 1.53 (7B gate/up, 37,888 x 3,584: 128 tokens 1.34, 512 1.17, 1,024 1.30); tiles less full 0.88 to 1.45;
+//   192 to 2,048 tokens by up to 5,120 columns, tiles 0.8 and more full, 0.97 to 1.30; else 0.83 to 1.21;
+//   beyond, with the tiles counted in whole rows over the XCDs (as they lay when these were measured): up to 3,584 columns tiles of 192 or 160
+//     features, the others from 0.65 on, 0.92 to 1.60; 4,096 to 5,120 columns from 0.8 on 0.91 to 1.58;
 //   8,192 columns 0.96 to 1.03.
-// Tiles of 64 x 64 only up to 1,536 columns.
 extern "C" int ms_gemm_tiled_pays(int M, int N, int K) {
   if (M <= 0 || N <= 0 || K <= 0 || K % BK) return 0;
   if (K <= 1536) return 1;
+  if (K > 5120) return 0;
+  if (K <= 3584 && M <= 128) return 1;
   const TileChoice c = choose_tile(M, N, K);
-  if (c.tile == 3) return 0;
-  if (M <= 2048 && c.tiles * 10 >= c.slots * 9) return 1;
-  const double f = filled(M, N, c);
-  if (K <= 3584) return c.tile >= 4 || f >= 0.65 || (c.tile == 2 && f <= 0.4);
-  return K <= 5120 && M > 512 && f >= 0.8;
+  if (M <= 2048) return full(M, N, c) >= (K <= 4096 ? 0.72 : 0.8) && M >= (K <= 4096 ? 1 : 192);
+  const double f = full_in_rows(M, N, c);
+  if (K <= 3584) return c.tile == T192X256 || c.tile == T160X256 || f >= 0.65;
+  return f >= 0.8;
 }
 
 // The same question for the squared relu, whose product is written whole and whose own kernel costs little: the sizes that the
@@ -573,7 +611,7 @@ extern "C" int ms_gemm_tiled_relu2_pays(int M, int N, int K) {
   if (M <= 0 || N <= 0 || K <= 0 || K % BK) return 0;
   if (K <= 1536) return 1;
   const TileChoice c = choose_tile(M, N, K);
-  return c.tile != 3 && M <= 2048 && c.tiles * 10 >= c.slots * 9;
+  return M <= 2048 && c.tiles * 10 >= c.slots * 9 && (M > 512 || full(M, N, c) >= 0.9);
 }
 
 // A bfloat16 [M, lda], W bfloat16 [N, ldw] (rows of K, K a multiple of 64), out bfloat16.
@@ -595,16 +633,24 @@ extern "C" int ms_gemm_tiled(const void* A, long long lda, const void* W, long l
   bf16* o = (bf16*)out;
   int tile = g_tile;
   if (tile == 0) tile = choose_tile(M, N, K).tile;
-#define GO(WF, WT, FT, TT) return epilogue == EPI_SWIGLU ? launch<WF, WT, FT, TT, EPI_SWIGLU, bf16>(a, lda, w, ldw, o, ldo, M, N, K, stream) \
-                                : epilogue == EPI_GEGLU ? launch<WF, WT, FT, TT, EPI_GEGLU, bf16>(a, lda, w, ldw, o, ldo, M, N, K, stream)  \
-                                : epilogue == EPI_RELU2 ? launch<WF, WT, FT, TT, EPI_RELU2, bf16>(a, lda, w, ldw, o, ldo, M, N, K, stream)  \
-                                : epilogue == EPI_CLAMPED ? launch<WF, WT, FT, TT, EPI_CLAMPED, bf16>(a, lda, w, ldw, o, ldo, M, N, K, stream, QkvEpilogue{}, numbers)  \
-                                                        : launch<WF, WT, FT, TT, EPI_STORE, bf16>(a, lda, w, ldw, o, ldo, M, N, K, stream)
-  if (tile == 1) GO(2, 4, 8, 4);   // 256 x 256
-  if (tile == 3) GO(1, 4, 4, 1);   // 64 x 64, four waves
-  if (tile == 4) GO(2, 4, 6, 4);   // 192 features x 256 tokens
-  if (tile == 5) GO(2, 4, 5, 4);   // 160 features x 256 tokens
-  GO(2, 4, 4, 2);                  // 128 x 128
+#define GO(WF, WT, FT, TT, SW, SA) return epilogue == EPI_SWIGLU ? launch<WF, WT, FT, TT, SW, SA, EPI_SWIGLU, bf16>(a, lda, w, ldw, o, ldo, M, N, K, stream) \
+                                : epilogue == EPI_GEGLU ? launch<WF, WT, FT, TT, SW, SA, EPI_GEGLU, bf16>(a, lda, w, ldw, o, ldo, M, N, K, stream)  \
+                                : epilogue == EPI_RELU2 ? launch<WF, WT, FT, TT, SW, SA, EPI_RELU2, bf16>(a, lda, w, ldw, o, ldo, M, N, K, stream)  \
+                                : epilogue == EPI_CLAMPED ? launch<WF, WT, FT, TT, SW, SA, EPI_CLAMPED, bf16>(a, lda, w, ldw, o, ldo, M, N, K, stream, QkvEpilogue{}, numbers)  \
+                                                        : launch<WF, WT, FT, TT, SW, SA, EPI_STORE, bf16>(a, lda, w, ldw, o, ldo, M, N, K, stream)
+  switch (tile) {      // features x tokens, slots of W and of A
+    case T256: GO(2, 4, 8, 4, 3, 2);
+    case T64: GO(1, 4, 4, 1, 3, 2);
+    case T192X256: GO(2, 4, 6, 4, 3, 2);
+    case T160X256: GO(2, 4, 5, 4, 3, 2);
+    case T64_DEEP: GO(1, 4, 4, 1, 5, 4);
+    case T160X128: GO(2, 4, 5, 2, 4, 3);
+    case T192X128: GO(2, 4, 6, 2, 4, 3);
+    case T128X256: GO(2, 4, 4, 4, 4, 3);
+    case T96X128: GO(2, 4, 3, 2, 5, 5);
+    case T64X128: GO(1, 8, 4, 1, 5, 5);
+    default: GO(2, 4, 4, 2, 3, 2);
+  }
 #undef GO
 }
 
@@ -617,7 +663,7 @@ extern "C" int ms_gemm_tiled(const void* A, long long lda, const void* W, long l
 //   up to 128 tokens 1.05 to 4.1, 1.6 on average;
 //   up to 256 tokens by 4,096 columns and more or up to 1,024 0.95 to 3.6, 1.5 on average;
 //   up to 512 tokens by more than 8,192 columns 1.0 to 3.1; by more than 4,096 in several parts, up to 5,120 features, 0.90 to 1.8,
-//     1.13 on average; by up to 1,024 for up to 1,024 features 0.96 to 1.11.  Not: whole columns (4,480 x 6,784 at 429 tokens 0.82), more
+//     no more blocks than CUs, 1.13 on average; by up to 1,024 for up to 1,024 features 0.96 to 1.11.  Not: whole columns (4,480 x 6,784 at 429 tokens 0.82), more
 //     features (0.81 to 1.2), 4,096 columns (0.93 to 1.12), 1,024 and fewer for more features (0.87 to 1.0);
 //   up to 1,024 tokens by more than 8,192 columns, up to 5,120 features or by 16,384 columns and more, 0.92 to 3.2, 1.33 on average;
 //     else 0.88 to 2.0, 1.08 on average (8,192 columns 0.89 to 1.17);
@@ -633,8 +679,8 @@ extern "C" int ms_gemm_tiled_sums_parts(int M, int N, int K) {
                   : M <= 1024 ? K <= 8192 || (N > 5120 && K < 16384) : K < 16384)) return 0;   // (asked for twice a layer: before the choice)
   const SumsChoice c = choose_sums(M, N, K);
   const int cus = ms_compute_units();
-  if (M > 256 && M <= 512 && K > 4096 && K <= 8192 && c.parts == 1) return 0;
-  if (M > 1024 && (c.tile != 1 || c.parts == 1 || c.blocks >= cus || c.blocks * 6 < cus * 5)) return 0;
+  if (M > 256 && M <= 512 && K > 4096 && K <= 8192 && (c.parts == 1 || c.blocks > cus)) return 0;
+  if (M > 1024 && (c.tile != T256 || c.parts == 1 || c.blocks >= cus || c.blocks * 6 < cus * 5)) return 0;
   return c.parts;
 }
 
@@ -649,10 +695,14 @@ extern "C" int ms_gemm_tiled_sums(const void* A, long long lda, const void* W, l
   const bf16* w = (const bf16*)W;
   int tile = g_tile;
   if (tile == 0) tile = choose_sums(M, N, K).tile;
-#define GO(WF, WT, FT, TT) return launch<WF, WT, FT, TT, EPI_SUMS, float>(a, lda, w, ldw, partial, (size_t)N, M, N, K, stream, QkvEpilogue{}, GroupedRows{}, parts)
-  if (tile == 1) GO(2, 4, 8, 4);
-  if (tile == 3) GO(1, 4, 4, 1);
-  GO(2, 4, 4, 2);
+#define GO(WF, WT, FT, TT, SW, SA) return launch<WF, WT, FT, TT, SW, SA, EPI_SUMS, float>(a, lda, w, ldw, partial, (size_t)N, M, N, K, stream, QkvEpilogue{}, GroupedRows{}, parts)
+  switch (tile) {
+    case T256: GO(2, 4, 8, 4, 3, 2);
+    case T64: GO(1, 4, 4, 1, 3, 2);
+    case T64_DEEP: GO(1, 4, 4, 1, 5, 4);
+    case T128_DEEP: GO(2, 4, 4, 2, 5, 4);
+    default: GO(2, 4, 4, 2, 3, 2);
+  }
 #undef GO
 }
 
@@ -719,12 +769,23 @@ extern "C" int ms_gemm_tiled_qkv(const void* A, long long lda, const void* W, lo
   const bf16* w = (const bf16*)W;
   bf16* o = (bf16*)q_out;
   const size_t ldo = (size_t)nh * head_dim;
-  // heads of 128: tiles of 256 features by 128 tokens (with 256 tokens the epilogue no longer fits the registers)
-  if (head_dim == 128) return launch<2, 4, 8, 2, EPI_QKV, bf16>(a, lda, w, ldw, o, ldo, M, N, K, stream, e);
-  // (128 x 128, whose epilogue takes longer here, over 64 x 64: 2.0 to 1.08 of the time up to 3 tiles of 64 a CU (1,152 x 896: 1,024
-  // tokens 18.4 and 11.2 us, 2,600 tokens 22.6 and 20.5), 0.81 to 1.23 from there to 4, and 0.78 to 1.05 beyond)
+#define GO(WF, WT, FT, TT, SW, SA) return launch<WF, WT, FT, TT, SW, SA, EPI_QKV, bf16>(a, lda, w, ldw, o, ldo, M, N, K, stream, e)
+  // A wave's features are a head.  As long as a tile of 64 tokens (then of 128) to every head is not more than a CU's worth, these with
+  // as many slots as LDS holds; then tiles that share a CU.  Heads of 64 (18 of them by 896, us of the tiles of 64 | the taken one; the
+  // epilogue's inputs asked for early have taken 1 from either): 512 tokens 10.3 | 8.9, 1,024 11.5 | 10.7, 1,536 12.6 | 10.9, 2,048 19.7 in a second round, 15.3 in tiles of
+  // 64, 4,096 24.9 of 128 and 24.5 of 64.  Heads of 128 (12 by 1,024; 256 features by 128 tokens before; with 256 tokens the epilogue does not fit the
+  // registers): 100 to 1,024 tokens 32 to 34 | 16, 2,048 35 | 24, 4,096 36.
+  const long long cus = ms_compute_units(), heads = nh + 2 * nkv;
   int tile = g_tile;
-  if (tile == 0) tile = choose_tile(M, N, K).tile;
-  if (tile == 3) return launch<1, 4, 4, 1, EPI_QKV, bf16>(a, lda, w, ldw, o, ldo, M, N, K, stream, e);
-  return launch<2, 4, 4, 2, EPI_QKV, bf16>(a, lda, w, ldw, o, ldo, M, N, K, stream, e);
+  if (tile == 0) tile = heads * ((M + 63) / 64) <= cus ? T64_DEEP : heads * ((M + 127) / 128) <= cus ? T64X128 : T64;
+  if (head_dim == 128) {
+    if (tile == T64_DEEP) GO(1, 4, 8, 1, 5, 4);
+    if (tile == T64X128) GO(1, 8, 8, 1, 3, 3);
+    GO(2, 4, 8, 2, 3, 2);
+  }
+  if (tile == T64_DEEP) GO(1, 4, 4, 1, 5, 4);
+  if (tile == T64X128) GO(1, 8, 4, 1, 5, 5);
+  if (tile == T64) GO(1, 4, 4, 1, 3, 2);
+  GO(2, 4, 4, 2, 3, 2);
+#undef GO
 }

@@ -2277,3 +2277,80 @@ def test_32_bit_products_of_up_to_8_rows_have_the_bits_of_the_kernel_for_64(ops,
         for kind in (4, 5, 0):
             for M in (1, 2, 3, 4, 5, 8):
                 assert torch.equal(run(kind, M, plain), want[:M]), (kind, M, plain)
+
+
+@pytest.mark.parametrize("tile", [6, 7, 8, 9, 10, 11])
+@pytest.mark.parametrize("K", [64, 128, 192, 256, 320, 384, 448, 896])
+@pytest.mark.parametrize("M,N", [(65, 662), (300, 1028), (513, 130)])
+def test_gemm_tiled_with_deep_pipelines(ops, M, N, K, tile):
+    """The tiles that ask for three to five steps ahead: fewer steps than slots, as many, one more and many; rows and features that
+    fill no whole tile.  The same bits as with a tile of two steps ahead (a sum runs over the columns in one order with every tile), and
+    right against 64 bits."""
+    force = ops._get("ms_gemm_tiled_force")
+    force.restype = None
+    g = torch.Generator(device=DEV).manual_seed(M + N + K)
+    a = torch.randn(M, K, generator=g, device=DEV).bfloat16()
+    w = (torch.randn(N, K, generator=g, device=DEV) / math.sqrt(K)).bfloat16()
+    a[M - 1] *= 3.0
+    want = a.double() @ w.double().T
+    got = []
+    for t in (tile, 2):
+        force(t)
+        try:
+            got.append([ops.gemm_tiled(a, w, e) for e in (ops.EPI_STORE, ops.EPI_SWIGLU, ops.EPI_GEGLU, ops.EPI_RELU2)]
+                       + [ops.gemm_tiled(a, w, ops.EPI_CLAMPED, 7.0, 1.702)])
+        finally:
+            force(0)
+    torch.testing.assert_close(got[0][0].double(), want, **tol(torch.bfloat16))
+    torch.testing.assert_close(got[0][1].double(), torch.nn.functional.silu(want[:, 0::2]) * want[:, 1::2], **tol(torch.bfloat16))
+    assert all(torch.equal(x, y) for x, y in zip(*got))
+
+
+@pytest.mark.parametrize("tile", [6, 12])
+@pytest.mark.parametrize("M,N,K,parts", [(65, 70, 64, 1), (130, 896, 320, 2), (257, 200, 1216, 3), (513, 132, 4864, 8)])
+def test_gemm_tiled_sums_with_deep_pipelines(ops, M, N, K, parts, tile):
+    """Runs of one to ten steps on the tiles that ask for four ahead: the bits of the tile that asks for two."""
+    force = ops._get("ms_gemm_tiled_force")
+    force.restype = None
+    g = torch.Generator(device=DEV).manual_seed(M + N + K)
+    a = torch.randn(M, K, generator=g, device=DEV).bfloat16()
+    w = (torch.randn(N, K, generator=g, device=DEV) / math.sqrt(K)).bfloat16()
+    got = []
+    for t in (tile, 3):
+        force(t)
+        try:
+            got.append(ops.gemm_tiled_sums(a, w, parts))
+        finally:
+            force(0)
+    torch.testing.assert_close(got[0].double().sum(0), a.double() @ w.double().T, atol=3e-5, rtol=3e-5)
+    assert torch.equal(*got)
+
+
+@pytest.mark.parametrize("tile", [0, 3, 6, 11])
+@pytest.mark.parametrize("nh,nkv,d,K,M,transposed", [(14, 2, 64, 896, 70, True), (3, 1, 64, 64, 129, False), (2, 2, 128, 320, 65, True),
+                                                     (5, 1, 128, 128, 200, False), (8, 4, 64, 192, 1200, True)])
+def test_gemm_tiled_qkv_with_deep_pipelines(ops, nh, nkv, d, K, M, transposed, tile):
+    """The q/k/v product on the tiles of one head (64 and 128 tokens) and as chosen: the bits of the larger tile, whose own test holds it
+    against 64 bits; tokens that are not stored, no bias, heads that fill no whole tile."""
+    force = ops._get("ms_gemm_tiled_force")
+    force.restype = None
+    g = torch.Generator(device=DEV).manual_seed(M + K)
+    N = (nh + 2 * nkv) * d
+    a = torch.randn(M, K, generator=g, device=DEV).bfloat16()
+    w = (torch.randn(N, K, generator=g, device=DEV) / math.sqrt(K)).bfloat16()
+    pos = torch.arange(M, dtype=torch.int32, device=DEV)
+    table = ops.rope_table(pos, 1e4 ** (-torch.arange(0, d, 2, device=DEV).float() / d))
+    slots = (pos + 16).int()
+    slots[::7] = -1
+    got = []
+    for bias in (None, torch.randn(N, generator=g, device=DEV)):
+        for t in (tile, 2):
+            kp = torch.zeros(M // 16 + 3, nkv, 16, d, dtype=torch.bfloat16, device=DEV)
+            vp = torch.zeros((M // 16 + 3, nkv, d, 16) if transposed else kp.shape, dtype=torch.bfloat16, device=DEV)
+            force(t)
+            try:
+                got.append((ops.gemm_tiled_qkv(a, w, bias, nh, nkv, d, table, slots, kp, vp, transposed), kp, vp))
+            finally:
+                force(0)
+        assert all(torch.equal(x, y) for x, y in zip(got[-2], got[-1]))
+    assert not torch.equal(got[0][0], got[2][0])
