@@ -17,6 +17,12 @@ int ms_rms_norm(float* x, const void* delta, int delta_dtype, int n_partials, lo
 int ms_rms_norm_pair(float* x, const void* delta, int delta_dtype, const float* w1, const float* w2, void* out1, void* out2,
                      int n_rows, int hidden, float eps, int dtype, hipStream_t stream);
 
+// the same, and out1's rows h as h + sum_j taps_w[c][j] input(j - taps + 1) over the request's tokens (ms_short_conv's mode 1), for
+// steps whose requests have one token each; state [slots, taps - 1, hidden] in `dtype` moves on
+int ms_rms_norm_pair_conv(float* x, const void* delta, int delta_dtype, const float* w1, const float* w2, const float* taps_w, int taps,
+                          void* state, const int* token_req, const int* state_slots, const int* n_live_tokens, void* out1, void* out2,
+                          int n_rows, int hidden, float eps, int dtype, hipStream_t stream);
+
 int ms_bias_add(void* x, const float* bias, int n_rows, int width, int dtype, hipStream_t stream);
 
 // tables / slots: host arrays of n_groups device pointers (block table int32 [table rows, table_stride], slot
@@ -60,7 +66,7 @@ int ms_gemm_skinny(const void* A, long long lda, const void* W, long long ldw, c
 void ms_gemm_skinny_force(int ntile, int waves, int token_groups);
 void ms_attention_mfma_force(int nt, int waves, int dim_shares);
 void ms_attention_generic_force(int waves);      // measurements: 1 or 4 waves to a (token, query head); 0 leaves the choice
-void ms_gemm_f32_force(int kernel);              // measurements: 1 few rows, 2 and 3 tiles of 64 and 32; 0 leaves the choice
+void ms_gemm_f32_force(int kernel);              // measurements: 1 few rows, 2 and 3 tiles of 64 and 32, 4 and 5 up to 8 rows; 0 leaves the choice
 
 int ms_gemm_stream(const void* A, long long lda, const int* rows, const float* norm_w, float eps, const void* W,
                    long long ldw, const float* bias, void* out, long long ldo, int M, int N, int K, int epilogue,
@@ -246,6 +252,14 @@ int ms_gated_delta(const void* q, const void* k, const void* v, long long qkv_st
                    int decay_per_channel, const void* b, long long b_stride, const float* A_log, const float* dt_bias, float* state, const int* q_start,
                    const int* state_slots, float* out, int n_requests, int heads, int kv_heads, int dim, int vdim,
                    int single_tokens, int dtype, hipStream_t stream);
+
+// A step of single tokens in bfloat16 with the decay's and the gate's low-rank products and the read-out's norm (weight [vdim],
+// sigmoid gate) in one kernel.
+int ms_gated_delta_step_takes(int dim, int vdim, int rank_a, int rank_g);
+int ms_gated_delta_step(const void* qkv, long long qkv_stride, const void* proj, long long proj_stride, int a_at, int g_at, int b_at,
+                        const void* w_a2, int rank_a, const void* w_g2, int rank_g, const float* A_log, const float* dt_bias,
+                        const float* norm_w, float eps, float* state, const int* q_start, const int* state_slots, void* out,
+                        int n_requests, int heads, int kv_heads, int dim, int vdim, hipStream_t stream);
 
 // out[n, h, :] = o[n, h, :] / rms(o[n, h, :]) * weight * act(gate[n, h, :]), act the sigmoid or (gate_silu) z * sigmoid(z);
 // o float, gate and out in `dtype`.  weight [vdim], shared by the heads, or with weight_per_head [heads * vdim]; `scale`

@@ -4,6 +4,7 @@
 // and the activation are computed in float.
 #include "common.h"
 #include "api.h"
+#include <type_traits>
 #include <algorithm>
 
 // ------------------------------------------------------------------------------------------------
@@ -179,6 +180,116 @@ __global__ void rms_norm_pair_kernel(float* __restrict__ x, const TD* __restrict
     o1[i] = from_float<T>(w1[i] * v);
     o2[i] = from_float<T>(w2[i] * v);
   }
+}
+
+// The same in a step of single tokens, with the first norm's rows through a short causal convolution over time on their way:
+// out1 = n1 + sum_j w[c][j] input(j - taps + 1), the inputs before the token from the request's state, which moves one up.  As
+// rms_norm_pair_kernel and short_conv_kernel (mode 1) one after the other, to the bit: 8.5 us for 4 rows of 896 (both wait for memory
+// and a launch), 6.1 so.
+constexpr int PAIR_CONV_TAPS = 8;
+// CH: pieces of four channels a thread has at most.  Everything is asked for before the sum is there (asked for behind it, two bytes at a
+// time, the kernel took 9 us).
+template <typename T, typename TD, int CH>
+__global__ void __launch_bounds__(256) rms_norm_pair_conv_kernel(float* __restrict__ x, const TD* __restrict__ delta, const float* __restrict__ w1,
+                                          const float* __restrict__ w2, const float* __restrict__ taps_w, int taps, T* state,
+                                          const int* __restrict__ token_req, const int* __restrict__ state_slots,
+                                          const int* __restrict__ n_live_tokens, T* __restrict__ out1, T* __restrict__ out2, int H, float eps) {
+  __shared__ float red[16];
+  const int n = blockIdx.x;
+  if (n_live_tokens && n >= *n_live_tokens) return;      // a token that pads a captured batch
+  float* xr = x + (size_t)n * H;
+  const TD* dr = delta ? delta + (size_t)n * H : nullptr;
+  T* st = state + (size_t)state_slots[token_req[n]] * (taps - 1) * H;
+  float4 v[CH], a1[CH], a2[CH], tw[CH][PAIR_CONV_TAPS];
+  Four<T> past[CH][PAIR_CONV_TAPS];
+#pragma unroll
+  for (int c = 0; c < CH; ++c) {
+    const int i = (threadIdx.x + c * blockDim.x) * 4;
+    if (i >= H) continue;
+    v[c] = *reinterpret_cast<const float4*>(xr + i);
+    a1[c] = *reinterpret_cast<const float4*>(w1 + i);
+    a2[c] = *reinterpret_cast<const float4*>(w2 + i);
+#pragma unroll
+    for (int j = 0; j < PAIR_CONV_TAPS; ++j)      // four channels' weights: the j-th four of them
+      if (j < taps) tw[c][j] = *reinterpret_cast<const float4*>(taps_w + (size_t)i * taps + 4 * j);
+#pragma unroll
+    for (int j = 0; j < PAIR_CONV_TAPS - 1; ++j)
+      if (j < taps - 1) past[c][j] = *reinterpret_cast<const Four<T>*>(st + (size_t)j * H + i);
+  }
+  float ss = 0.f;
+#pragma unroll
+  for (int c = 0; c < CH; ++c) {
+    const int i = (threadIdx.x + c * blockDim.x) * 4;
+    if (i >= H) continue;
+    if (dr) {
+      v[c].x += to_float(dr[i]); v[c].y += to_float(dr[i + 1]); v[c].z += to_float(dr[i + 2]); v[c].w += to_float(dr[i + 3]);
+      *reinterpret_cast<float4*>(xr + i) = v[c];
+    }
+    ss += v[c].x * v[c].x + v[c].y * v[c].y + v[c].z * v[c].z + v[c].w * v[c].w;
+  }
+  ss = block_sum(ss, red);
+  const float inv = 1.0f / sqrtf(ss / (float)H + eps);
+#pragma unroll
+  for (int c = 0; c < CH; ++c) {
+    const int i = (threadIdx.x + c * blockDim.x) * 4;
+    if (i >= H) continue;
+    const float vv[4] = {v[c].x, v[c].y, v[c].z, v[c].w}, g1[4] = {a1[c].x, a1[c].y, a1[c].z, a1[c].w}, g2[4] = {a2[c].x, a2[c].y, a2[c].z, a2[c].w};
+    float flat[4 * PAIR_CONV_TAPS];      // [channel][tap], `taps` of them a channel
+#pragma unroll
+    for (int j = 0; j < PAIR_CONV_TAPS; ++j) {
+      flat[4 * j] = tw[c][j].x; flat[4 * j + 1] = tw[c][j].y; flat[4 * j + 2] = tw[c][j].z; flat[4 * j + 3] = tw[c][j].w;
+    }
+    Four<T> now, r1, r2;
+    auto rows = [&](auto count) __attribute__((always_inline)) {      // (the number of taps as a constant: the weights stay in registers)
+      constexpr int TAPS = decltype(count)::value;
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        const float u = vv[e] * inv;
+        now.v[e] = from_float<T>(g1[e] * u);
+        float in = to_float(now.v[e]), acc = 0.f;
+        asm("" : "+v"(in));      // rounded here, as where it goes through memory: not one operation with the sum
+#pragma unroll
+        for (int j = 0; j < TAPS - 1; ++j) acc = fmaf(flat[e * TAPS + j], to_float(past[c][j].v[e]), acc);
+        acc = fmaf(flat[e * TAPS + TAPS - 1], in, acc);
+        acc += in;
+        r1.v[e] = from_float<T>(acc);
+        r2.v[e] = from_float<T>(g2[e] * u);
+      }
+    };
+    switch (taps) {
+      case 1: rows(std::integral_constant<int, 1>{}); break;
+      case 2: rows(std::integral_constant<int, 2>{}); break;
+      case 3: rows(std::integral_constant<int, 3>{}); break;
+      case 4: rows(std::integral_constant<int, 4>{}); break;
+      case 5: rows(std::integral_constant<int, 5>{}); break;
+      case 6: rows(std::integral_constant<int, 6>{}); break;
+      case 7: rows(std::integral_constant<int, 7>{}); break;
+      default: rows(std::integral_constant<int, 8>{}); break;
+    }
+    *reinterpret_cast<Four<T>*>(out1 + (size_t)n * H + i) = r1;
+    *reinterpret_cast<Four<T>*>(out2 + (size_t)n * H + i) = r2;
+#pragma unroll
+    for (int j = 0; j < PAIR_CONV_TAPS - 1; ++j)
+      if (j < taps - 1) *reinterpret_cast<Four<T>*>(st + (size_t)j * H + i) = j + 1 < taps - 1 ? past[c][j + 1 < PAIR_CONV_TAPS ? j + 1 : j] : now;
+  }
+}
+
+// bfloat16, H a multiple of 4 up to 2,048, all rows on four values; taps 1 to 8.  MS_UNSUPPORTED for the others.
+extern "C" int ms_rms_norm_pair_conv(float* x, const void* delta, int delta_dtype, const float* w1, const float* w2, const float* taps_w,
+                                     int taps, void* state, const int* token_req, const int* state_slots, const int* n_live_tokens,
+                                     void* out1, void* out2, int n_rows, int hidden, float eps, int dtype, hipStream_t stream) {
+  if (n_rows <= 0) return MS_OK;
+  if (hidden <= 0 || taps < 1) return MS_BAD_ARG;
+  if (dtype != MS_BF16) return MS_UNSUPPORTED;
+  if (hidden % 4 || hidden > 2048 || taps > PAIR_CONV_TAPS || ((uintptr_t)x | (uintptr_t)w1 | (uintptr_t)w2 | (uintptr_t)taps_w) % 16 ||
+      ((uintptr_t)state | (uintptr_t)out1 | (uintptr_t)out2) % 8)
+    return MS_UNSUPPORTED;
+  dim3 grid(n_rows), block(hidden >= 1024 ? 256 : 128);      // as ms_rms_norm_pair: the order of the sum
+#define LAUNCH(T, TD) rms_norm_pair_conv_kernel<T, TD, 2><<<grid, block, 0, stream>>>(x, (const TD*)delta, w1, w2, taps_w, taps, (T*)state, token_req, state_slots, n_live_tokens, (T*)out1, (T*)out2, hidden, eps)
+  if (delta && delta_dtype == MS_F32) LAUNCH(bf16, float);
+  else LAUNCH(bf16, bf16);
+#undef LAUNCH
+  return ms_launch_status();
 }
 
 extern "C" int ms_rms_norm_pair(float* x, const void* delta, int delta_dtype, const float* w1, const float* w2, void* out1,

@@ -40,7 +40,8 @@ gemm_quads_kernel(const void* __restrict__ A, size_t lda, const bf16* __restrict
   const int m = lane & (G - 1), r = (lane / G) & 3, n0 = r0 + 4 * min(wave, U - 1);
   const int nc = min(n0 + r, N - 1);
   const float pre = EPI == EPI_RESIDUAL ? reinterpret_cast<const float*>(out)[(size_t)min(m, M - 1) * ldo + nc] : 0.f;
-  const float bv = bias && !ms_gated(EPI) ? bias[nc] : 0.f;
+  const float bv = bias && !ms_gated(EPI) && EPI != EPI_XIELU ? bias[nc] : 0.f;
+  const float numbers[2] = {EPI == EPI_XIELU ? bias[0] : 0.f, EPI == EPI_XIELU ? bias[1] : 0.f};
   product.run(wrow, x, norm_w);
 
   // rows 0 to 3 of a tile lie in lanes 0 to 15, one token to a lane
@@ -83,7 +84,7 @@ gemm_quads_kernel(const void* __restrict__ A, size_t lda, const bf16* __restrict
       v *= scale;
       asm("" : "+v"(v));   // rounded here, as in ms_gemm_skinny: not one operation with the bias
     }
-    if (lane < 4 * G && n0 + r < N) out[(size_t)m * ldo + n0 + r] = from_float<TO>(ms_store_value<EPI>(v + bv + pre));
+    if (lane < 4 * G && n0 + r < N) out[(size_t)m * ldo + n0 + r] = from_float<TO>(EPI == EPI_XIELU ? ms_xielu_value(v, numbers[0], numbers[1]) : ms_store_value<EPI>(v + bv + pre));
   }
 }
 
@@ -174,6 +175,10 @@ extern "C" int ms_gemm_quads(const void* A, long long lda, const int* rows, cons
   if (epilogue == EPI_CLAMPED) {
     if (N % 2 || ldo < N / 2 || out_dtype != MS_BF16 || norm || !bias) return MS_BAD_ARG;
     RUN(EPI_CLAMPED, bf16, false);
+  }
+  if (epilogue == EPI_XIELU) {
+    if (ldo < N || out_dtype != MS_BF16 || norm || !bias) return MS_BAD_ARG;
+    RUN(EPI_XIELU, bf16, false);
   }
   if (epilogue == EPI_RELU2) {
     if (ldo < N || out_dtype != MS_BF16 || norm) return MS_BAD_ARG;

@@ -328,6 +328,121 @@ gated_delta_kernel(const T* __restrict__ q, const T* __restrict__ k, const T* __
 }
 
 // ------------------------------------------------------------------------------------------------
+// A decode step of the delta rule with what lies around it, bfloat16, a block of 256 threads to a (request, head): the decay's
+// input a = W_a2 a1 and the read-out's gate W_g2 g1 (a1, g1 and b of the projections' row), the step of S, and the read-out's norm
+// and gate.  Six kernels before (two copies of row slices that products do not take, the two products, the step, the norm), 26 us of
+// a layer's 60 (14 heads of 64, ranks of 64, 4 requests), 6.6 so (9 with W_a2's and W_g2's rows asked for behind the barrier).  What bounds it is
+// two trips to memory, for the request's place and for all that depends on it, and a launch.
+constexpr int STEP_MAX_RANK = 128;      // of either low-rank map
+
+template <int LPC>      // lanes a column of S is spread over, 16 rows each
+__global__ void __launch_bounds__(256)
+gated_delta_step_kernel(const bf16* __restrict__ qkv, size_t qkv_stride, const bf16* __restrict__ proj, size_t proj_stride, int a_at,
+                        int g_at, int b_at, const bf16* __restrict__ w_a2, int rank_a, const bf16* __restrict__ w_g2, int rank_g,
+                        const float* __restrict__ A_log, const float* __restrict__ dt_bias, const float* __restrict__ norm_w,
+                        float eps, float* __restrict__ state, const int* __restrict__ q_start,
+                        const int* __restrict__ state_slots, bf16* __restrict__ out, int H, int G, int D, int E) {
+  constexpr int ROWS = 16, Dp = ROWS * LPC, COLS = 256 / LPC;      // E <= COLS
+  __shared__ __align__(16) float qs[Dp], ks[Dp], gs[Dp];
+  __shared__ float gate[COLS], in[2][STEP_MAX_RANK], red[16];
+  const int h = blockIdx.x, r = blockIdx.y, n = q_start[r];
+  if (q_start[r + 1] <= n) return;
+  const int tid = threadIdx.x, lane = tid & (MS_WAVE - 1), wave = tid / MS_WAVE, part = tid % LPC, col = tid / LPC;
+  const bool live = col < E;
+  const int kvh = h / (H / G);
+  float* Sg = state + (((size_t)state_slots[r] * H + h) * D) * E;
+  float S[ROWS];
+#pragma unroll
+  for (int i = 0; i < ROWS; ++i) {
+    const int row = part * ROWS + i;
+    S[i] = Sg[(size_t)min(row, D - 1) * E + min(col, E - 1)];      // (what is past either end is not used)
+  }
+  const bf16* prow = proj + (size_t)n * proj_stride;
+  const float rate = expf(A_log[h]), beta = sigmoid_f(to_float(prow[b_at + h]));
+  const bf16* row = qkv + (size_t)n * qkv_stride;
+  const float v = to_float(row[2 * G * D + (size_t)h * E + min(col, E - 1)]);
+  const float nw = norm_w[min(col, E - 1)];
+  // the first 64 rows' weights (all of them, up to heads of 64): four lanes to a row, eight columns at a time
+  constexpr int PIECES = STEP_MAX_RANK / 32;
+  uint4 pa[PIECES], pg[PIECES];
+  const int ra0 = h * D + min(tid / 4, D - 1), rg0 = h * E + min(tid / 4, E - 1);
+  auto ask = [&](const bf16* w, int rank, uint4 (&p)[PIECES]) __attribute__((always_inline)) {
+#pragma unroll
+    for (int j = 0; j < PIECES; ++j) p[j] = *reinterpret_cast<const uint4*>(w + min((tid & 3) * 8 + j * 32, rank - 8));
+  };
+  ask(w_a2 + (size_t)ra0 * rank_a, rank_a, pa);
+  ask(w_g2 + (size_t)rg0 * rank_g, rank_g, pg);
+  const float dt0 = dt_bias[ra0];
+  for (int i = tid; i < rank_a; i += 256) in[0][i] = to_float(prow[a_at + i]);
+  for (int i = tid; i < rank_g; i += 256) in[1][i] = to_float(prow[g_at + i]);
+  if (wave < 2) {                                          // q and k as unit vectors
+    const bf16* x = row + (size_t)(wave * G + kvh) * D;
+    float u[Dp > MS_WAVE ? Dp / MS_WAVE : 1], ss = 0.f;
+#pragma unroll
+    for (int e = 0; e < (Dp > MS_WAVE ? Dp / MS_WAVE : 1); ++e) {
+      const int i = lane + e * MS_WAVE;
+      u[e] = i < D ? to_float(x[i]) : 0.f;
+      ss = fmaf(u[e], u[e], ss);
+    }
+    const float inv = (wave == 0 ? 1.0f / sqrtf((float)D) : 1.0f) / sqrtf(wave_sum(ss) + 1e-6f);
+#pragma unroll
+    for (int e = 0; e < (Dp > MS_WAVE ? Dp / MS_WAVE : 1); ++e) {
+      const int i = lane + e * MS_WAVE;
+      if (i < Dp) (wave == 0 ? qs : ks)[i] = u[e] * inv;
+    }
+  }
+  __syncthreads();
+  auto product = [&](const uint4 (&p)[PIECES], const float* x, int rank) __attribute__((always_inline)) {
+    float sum = 0.f;
+#pragma unroll
+    for (int j = 0; j < PIECES; ++j) {
+      const int c = (tid & 3) * 8 + j * 32;
+      if (c >= rank) continue;
+      const unsigned u[4] = {p[j].x, p[j].y, p[j].z, p[j].w};
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        sum = fmaf(__uint_as_float(u[e] << 16), x[c + 2 * e], sum);
+        sum = fmaf(__uint_as_float(u[e] & 0xffff0000u), x[c + 2 * e + 1], sum);
+      }
+    }
+    return group_sum<4>(sum);
+  };
+  for (int i = tid / 4; i < Dp; i += 64) {
+    const int at = h * D + min(i, D - 1);
+    if (i >= 64) ask(w_a2 + (size_t)at * rank_a, rank_a, pa);
+    const float a = product(pa, in[0], rank_a) + (i >= 64 ? dt_bias[at] : dt0);
+    if ((tid & 3) == 0) gs[i] = i < D ? expf(-rate * softplus_f(a)) : 1.f;
+  }
+  for (int i = tid / 4; i < E; i += 64) {
+    if (i >= 64) ask(w_g2 + (size_t)(h * E + i) * rank_g, rank_g, pg);
+    const float z = product(pg, in[1], rank_g);
+    if ((tid & 3) == 0) gate[i] = sigmoid_f(z);
+  }
+  __syncthreads();
+  const float *q = qs + part * ROWS, *k = ks + part * ROWS, *g = gs + part * ROWS;      // (rows past D: q and k are 0)
+  float kv = 0.f, o = 0.f;
+#pragma unroll
+  for (int i = 0; i < ROWS; ++i) {
+    S[i] *= g[i];
+    kv = fmaf(S[i], k[i], kv);
+  }
+  const float u = beta * (v - group_sum<LPC>(kv));
+#pragma unroll
+  for (int i = 0; i < ROWS; ++i) {
+    S[i] = fmaf(k[i], u, S[i]);
+    o = fmaf(S[i], q[i], o);
+  }
+  o = group_sum<LPC>(o);
+#pragma unroll
+  for (int i = 0; i < ROWS; ++i) {
+    const int at = part * ROWS + i;
+    if (live && at < D) Sg[(size_t)at * E + col] = S[i];
+  }
+  const float inv = 1.0f / sqrtf(block_sum(live && part == 0 ? o * o : 0.f, red) / (float)E + eps);
+  if (live && part == 0) out[(size_t)n * H * E + (size_t)h * E + col] = from_float<bf16>(o * inv * nw * gate[col]);
+}
+
+// ------------------------------------------------------------------------------------------------
 // y[n, h, :] = o[n, h, :] / sqrt(mean(o[n, h, :]^2) + eps) * w[:] * act(gate[n, h, :]), act the sigmoid (gate_silu 0) or
 // z * sigmoid(z) (1); one wave per (token, head).
 template <typename T>
@@ -369,13 +484,13 @@ __global__ void xielu_kernel(const T* __restrict__ x, const float* __restrict__ 
 #pragma unroll
     for (int j = 0; j < V; ++j) {
       const float z = to_float(p.v[j]);
-      p.v[j] = from_float<T>(z > 0.f ? fmaf(ap * z, z, 0.5f * z) : fmaf(an, expm1f(z) - z, 0.5f * z));
+      p.v[j] = from_float<T>(ms_xielu_value(z, ap, an));
     }
     reinterpret_cast<Pack*>(out)[i] = p;
   }
   for (size_t i = packs * V + (size_t)blockIdx.x * blockDim.x + threadIdx.x; i < total; i += stride) {
     const float z = to_float(x[i]);
-    out[i] = from_float<T>(z > 0.f ? fmaf(ap * z, z, 0.5f * z) : fmaf(an, expm1f(z) - z, 0.5f * z));
+    out[i] = from_float<T>(ms_xielu_value(z, ap, an));
   }
 }
 
@@ -465,6 +580,34 @@ extern "C" int ms_gated_delta(const void* q, const void* k, const void* v, long 
 #undef BY_DPT
 #undef LAUNCH
 #undef LAUNCH1
+  return ms_launch_status();
+}
+
+// Whether ms_gated_delta_step takes these sizes (of a step of single tokens): a head's columns in one block, low ranks in pieces of eight.
+extern "C" int ms_gated_delta_step_takes(int dim, int vdim, int rank_a, int rank_g) {
+  const int lpc = dim <= 16 ? 1 : dim <= 32 ? 2 : dim <= 64 ? 4 : 8;
+  return dim > 0 && dim <= 128 && vdim > 0 && vdim * lpc <= 256 && rank_a > 0 && rank_g > 0 && rank_a % 8 == 0 && rank_g % 8 == 0 &&
+         rank_a <= STEP_MAX_RANK && rank_g <= STEP_MAX_RANK;
+}
+
+// qkv [tokens, >= 2 kv_heads dim + heads vdim] and proj [tokens, ..] bfloat16, rows their strides apart, a1 at column a_at of proj, g1 at
+// g_at, b at b_at; w_a2 [heads dim, rank_a] and w_g2 [heads vdim, rank_g] bfloat16 on 16 bytes; out bfloat16 [tokens, heads vdim].
+extern "C" int ms_gated_delta_step(const void* qkv, long long qkv_stride, const void* proj, long long proj_stride, int a_at, int g_at,
+                                   int b_at, const void* w_a2, int rank_a, const void* w_g2, int rank_g, const float* A_log,
+                                   const float* dt_bias, const float* norm_w, float eps, float* state, const int* q_start,
+                                   const int* state_slots, void* out, int n_requests, int heads, int kv_heads, int dim, int vdim,
+                                   hipStream_t stream) {
+  if (n_requests <= 0) return MS_OK;
+  if (heads <= 0 || kv_heads <= 0 || heads % kv_heads) return MS_BAD_ARG;
+  if (!ms_gated_delta_step_takes(dim, vdim, rank_a, rank_g) || n_requests > 65535) return MS_UNSUPPORTED;
+  if (((uintptr_t)w_a2 | (uintptr_t)w_g2) % 16) return MS_UNSUPPORTED;
+  dim3 grid(heads, n_requests), block(256);
+#define GO(LPC) gated_delta_step_kernel<LPC><<<grid, block, 0, stream>>>((const bf16*)qkv, (size_t)qkv_stride, (const bf16*)proj, (size_t)proj_stride, a_at, g_at, b_at, (const bf16*)w_a2, rank_a, (const bf16*)w_g2, rank_g, A_log, dt_bias, norm_w, eps, state, q_start, state_slots, (bf16*)out, heads, kv_heads, dim, vdim)
+  if (dim <= 16) GO(1);
+  else if (dim <= 32) GO(2);
+  else if (dim <= 64) GO(4);
+  else GO(8);
+#undef GO
   return ms_launch_status();
 }
 

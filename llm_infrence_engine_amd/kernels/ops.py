@@ -25,6 +25,13 @@ _SIGNATURES = {
     "ms_rms_norm": [_c_ptr, _c_ptr, _c_int, _c_int, _c_ll, _c_ptr, _c_ptr, _c_ptr, _c_int, _c_int, _c_float, _c_int,
                     _c_int, _c_ptr],
     "ms_rms_norm_pair": [_c_ptr, _c_ptr, _c_int, _c_ptr, _c_ptr, _c_ptr, _c_ptr, _c_int, _c_int, _c_float, _c_int, _c_ptr],
+    "ms_rms_norm_pair_conv": [_c_ptr, _c_ptr, _c_int, _c_ptr, _c_ptr, _c_ptr, _c_int, _c_ptr, _c_ptr, _c_ptr, _c_ptr, _c_ptr, _c_ptr,
+                              _c_int, _c_int, _c_float, _c_int, _c_ptr],
+    "ms_gated_delta_step_takes": [_c_int] * 4,
+    "ms_gated_delta_step": [_c_ptr, _c_ll, _c_ptr, _c_ll, _c_int, _c_int, _c_int, _c_ptr, _c_int, _c_ptr, _c_int, _c_ptr, _c_ptr,
+                            _c_ptr, _c_float, _c_ptr, _c_ptr, _c_ptr, _c_ptr, _c_int, _c_int, _c_int, _c_int, _c_int, _c_ptr],
+    "ms_gemm_quads": [_c_ptr, _c_ll, _c_ptr, _c_ptr, _c_float, _c_ptr, _c_ll, _c_ptr, _c_ptr, _c_ll, _c_int, _c_int, _c_int, _c_int,
+                      _c_int, _c_int, _c_ptr],
     "ms_gemm_skinny_norm": [_c_ptr, _c_ll, _c_ptr, _c_ptr, _c_float, _c_ptr, _c_ll, _c_ptr, _c_ptr, _c_ll, _c_int,
                             _c_int, _c_int, _c_int, _c_int, _c_ptr],
     "ms_qkv_rope_store": [_c_ptr, _c_ll, _c_ptr, _c_float, _c_ptr, _c_ptr, _c_ptr, _c_ptr, _c_ptr, _c_ptr, _c_ptr, _c_ptr,
@@ -329,6 +336,30 @@ def rms_norm_pair(x: torch.Tensor, w1: torch.Tensor, w2: torch.Tensor, eps: floa
     return out1, out2
 
 
+def rms_norm_pair_conv(x: torch.Tensor, w1: torch.Tensor, w2: torch.Tensor, eps: float, taps: torch.Tensor, state: torch.Tensor, ctx,
+                       out1: torch.Tensor, out2: torch.Tensor, delta: Optional[torch.Tensor] = None):
+    """``rms_norm_pair`` and, of out1's rows h, ``short_conv`` with CONV_ADD_INPUT (h + the convolution, the state moved on) in one
+    kernel, for a step whose requests have one token each: taps float [H, taps], state [slots, taps - 1, H]."""
+    _check(x, "x", torch.float32)
+    N, H = x.shape
+    _check(w1, "w1", torch.float32, (H,))
+    _check(w2, "w2", torch.float32, (H,))
+    _check(out1, "out1", None, (N, H))
+    _check(out2, "out2", out1.dtype, (N, H))
+    _check(taps, "taps", torch.float32, (H, None))
+    _check(state, "state", out1.dtype, (None, max(1, taps.shape[1] - 1), H))
+    _check(ctx.token_req, "token_req", torch.int32, (N,))
+    _check(ctx.state_slots, "state_slots", torch.int32, (ctx.num_requests,))
+    dcode = 0
+    if delta is not None:
+        _check(delta, "delta", None, (N, H))
+        dcode = _code(delta.dtype)
+    _call("ms_rms_norm_pair_conv", x.data_ptr(), _ptr(delta), dcode, w1.data_ptr(), w2.data_ptr(), taps.data_ptr(), taps.shape[1],
+          state.data_ptr(), ctx.token_req.data_ptr(), ctx.state_slots.data_ptr(), _ptr(ctx.n_live_tokens), out1.data_ptr(),
+          out2.data_ptr(), N, H, float(eps), _code(out1.dtype), _stream())
+    return out1, out2
+
+
 def bias_add(x: torch.Tensor, bias: torch.Tensor) -> torch.Tensor:
     """x[n, :] += bias, in place."""
     _check(x, "x")
@@ -515,6 +546,33 @@ EPI_STORE, EPI_SWIGLU, EPI_RESIDUAL = 0, 1, 3
 EPI_GEGLU = 4      # as EPI_SWIGLU with the tanh form of the gelu (the tiled product alone has it)
 EPI_RELU2 = 5      # max(product (+ bias), 0)^2
 EPI_CLAMPED = 6    # as EPI_SWIGLU with the clamped gate: min(g, limit) sigmoid(alpha ..) (clamp(u, -limit, limit) + 1)
+
+
+EPI_XIELU = 9      # the xIELU activation of the product, with its two numbers as ``xielu_numbers`` gives them
+
+
+def xielu_numbers(pq: torch.Tensor) -> torch.Tensor:
+    """softplus(p) and 1/2 + softplus(q) of an xIELU's learned numbers, for ``gemm_xielu``."""
+    return torch.nn.functional.softplus(pq.float()) + torch.tensor([0.0, 0.5], device=pq.device)
+
+
+def gemm_xielu(a: torch.Tensor, w: torch.Tensor, numbers: torch.Tensor) -> Optional[torch.Tensor]:
+    """xielu(a [M <= 8, K] @ w [N, K].T) in bfloat16, None where the kernel of narrow matrices, which has the activation as an
+    epilogue, is not the one for the product."""
+    if a.shape[0] > 8 or not skinny_ok(a, w):
+        return None
+    _check(a, "a", torch.bfloat16, contiguous=False)
+    (M, K), N = a.shape, w.shape[0]
+    _check(w, "w", torch.bfloat16, (N, K))
+    _check(numbers, "numbers", torch.float32, (2,))
+    out = torch.empty((M, N), dtype=torch.bfloat16, device=a.device)
+    rc = _get("ms_gemm_quads")(a.data_ptr(), a.stride(0) if M > 1 else K, None, None, 0.0, w.data_ptr(), K, numbers.data_ptr(), out.data_ptr(),
+                               N, M, N, K, EPI_XIELU, BF16, 0, _stream())
+    if rc == 2:
+        return None
+    if rc != 0:
+        raise RuntimeError(f"ms_gemm_quads refused its arguments: {_CODES.get(rc, rc)}")
+    return out
 
 
 def skinny_ok(a: torch.Tensor, w: torch.Tensor) -> bool:
@@ -1480,6 +1538,41 @@ def gated_delta(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, a: torch.Tens
           A_log.data_ptr(),
           dt_bias.data_ptr(), state.data_ptr(), ctx.q_start.data_ptr(), ctx.state_slots.data_ptr(), out.data_ptr(), R,
           heads, kv_heads, dim, vdim, int(getattr(ctx, "max_q_len", 0) == 1), _code(q.dtype), _stream())
+    return out
+
+
+def gated_delta_step_ok(proj: torch.Tensor, w_a2: torch.Tensor, w_g2: torch.Tensor, dim: int, vdim: int) -> bool:
+    """Whether ``gated_delta_step`` takes these."""
+    return (proj.dtype == w_a2.dtype == w_g2.dtype == torch.bfloat16 and w_a2.data_ptr() % 16 == 0 and w_g2.data_ptr() % 16 == 0
+            and bool(_get("ms_gated_delta_step_takes")(dim, vdim, w_a2.shape[1], w_g2.shape[1])))
+
+
+def gated_delta_step(qkv: torch.Tensor, proj: torch.Tensor, a_at: int, g_at: int, b_at: int, w_a2: torch.Tensor, w_g2: torch.Tensor,
+                     A_log: torch.Tensor, dt_bias: torch.Tensor, norm_w: torch.Tensor, eps: float, state: torch.Tensor, ctx,
+                     out: torch.Tensor, heads: int, kv_heads: int, dim: int, vdim: int) -> torch.Tensor:
+    """A step of single tokens in bfloat16, in one kernel: ``gated_delta`` with a = w_a2 a1 and then ``gated_head_norm`` with the
+    gate w_g2 g1 through the sigmoid, where a1, g1 and b are the columns of ``proj`` [N, ..] from a_at, g_at and b_at on; qkv
+    [N, 2 kv_heads * dim + heads * vdim] behind its convolution, w_a2 [heads * dim, rank], w_g2 [heads * vdim, rank]."""
+    N = qkv.shape[0]
+    sq, sp = _rows2d(qkv, "qkv", torch.bfloat16, 2 * kv_heads * dim + heads * vdim), _rows2d(proj, "proj", torch.bfloat16)
+    ra, rg = w_a2.shape[1], w_g2.shape[1]
+    if proj.shape[0] != N or min(a_at, g_at, b_at) < 0 or max(a_at + ra, g_at + rg, b_at + heads) > proj.shape[1]:
+        raise ValueError(f"proj {list(proj.shape)} does not hold a1, g1 and b of {N} tokens at columns {a_at}, {g_at} and {b_at}")
+    _check(w_a2, "w_a2", torch.bfloat16, (heads * dim, ra))
+    _check(w_g2, "w_g2", torch.bfloat16, (heads * vdim, rg))
+    _check(A_log, "A_log", torch.float32, (heads,))
+    _check(dt_bias, "dt_bias", torch.float32, (heads * dim,))
+    _check(norm_w, "norm_w", torch.float32, (vdim,))
+    _check(state, "state", torch.float32, (None, heads, dim, vdim))
+    _check(out, "out", torch.bfloat16, (N, heads * vdim))
+    R = ctx.num_requests
+    _check(ctx.q_start, "q_start", torch.int32, (R + 1,))
+    _check(ctx.state_slots, "state_slots", torch.int32, (R,))
+    if getattr(ctx, "max_q_len", 0) != 1:
+        raise ValueError("every request of the step must have one token")
+    _call("ms_gated_delta_step", qkv.data_ptr(), sq, proj.data_ptr(), sp, a_at, g_at, b_at, w_a2.data_ptr(), ra, w_g2.data_ptr(), rg,
+          A_log.data_ptr(), dt_bias.data_ptr(), norm_w.data_ptr(), float(eps), state.data_ptr(), ctx.q_start.data_ptr(),
+          ctx.state_slots.data_ptr(), out.data_ptr(), R, heads, kv_heads, dim, vdim, _stream())
     return out
 
 

@@ -11,6 +11,8 @@ from typing import Any
 
 from ..kernels import ops
 from .base import Block, Norm, declares, register_part
+from .filters import ShortConv
+from .norms import RMSNorm
 
 
 class PreNormResidual(Block):
@@ -45,15 +47,23 @@ class ParallelResidual(Block):
     optional = ("position", "input_filter", "feed_forward_norm", "feed_forward")
 
     def forward(self, x, pending, ctx, kv, state):
-        # x holds the sum both branches read before either adds to it; the two norms share their pass over x
-        if self.feed_forward is not None and self.feed_forward_norm is None:
+        # x holds the sum both branches read before either adds to it; the two norms share their pass over x, in a step of single
+        # tokens with the filter
+        both = None
+        if (type(self.mixer_norm) is RMSNorm and type(self.input_filter) is ShortConv and self.input_filter.add_input
+                and self.feed_forward is not None and self.feed_forward_norm is not None):
+            both = self.mixer_norm.forward_pair_filtered(self.feed_forward_norm, x, ctx, self.input_filter.weight,
+                                                         self.state_of("input_filter", state).slots, delta=pending)
+        if both is not None:
+            h, h2 = both
+        elif self.feed_forward is not None and self.feed_forward_norm is None:
             h = h2 = self.mixer_norm.forward(x, delta=pending)
         elif self.feed_forward is not None and hasattr(self.mixer_norm, "forward_pair"):
             h, h2 = self.mixer_norm.forward_pair(self.feed_forward_norm, x, delta=pending)
         else:
             h = self.mixer_norm.forward(x, delta=pending)
             h2 = self.feed_forward_norm.forward(x) if self.feed_forward is not None else None
-        if self.input_filter is not None:
+        if self.input_filter is not None and both is None:
             h = self.input_filter.forward(h, ctx, self.state_of("input_filter", state))
         a = self.mixer.forward_residual(h, ctx, kv, self.state_of("mixer", state), x)
         if self.feed_forward is None:

@@ -108,6 +108,11 @@ class GatedDelta(Mixer):
         b_at = g_at + (self.gate_rank if self.gate == "low_rank_sigmoid" else self.vw)
         proj = linear.linear(h, self.w_in)
         qkv = ops.short_conv(proj[:, :cw], self.conv_w, conv_state, ctx, self.rt.empty(N, cw), ops.CONV_SILU)
+        if (self.decay == "channel" and self.w_g2 is not None and getattr(ctx, "max_q_len", 0) == 1
+                and ops.gated_delta_step_ok(proj, self.w_a, self.w_g2, self.dim, self.vdim)):
+            y = ops.gated_delta_step(qkv, proj, a_at, g_at, b_at, self.w_a, self.w_g2, self.A_log, self.dt_bias, self.norm_w, self.eps,
+                                     S, ctx, self.rt.empty(N, self.vw), self.heads, self.kv_heads, self.dim, self.vdim)
+            return linear.linear_residual(y, self.w_o, None, x)
         if self.decay == "channel":
             a = linear.linear(_rows(proj, a_at, g_at), self.w_a, out_dtype=torch.float32)
         else:

@@ -70,6 +70,16 @@ class RMSNorm(Norm):
         return ops.rms_norm_pair(x, self.weight, other.weight, self.eps, self.rt.empty(n, self.size),
                                  self.rt.empty(n, self.size), delta=delta)
 
+    def forward_pair_filtered(self, other: "RMSNorm", x, ctx, weight, state, delta=None):
+        """``forward_pair`` with the first result h as h + its convolution over time, for a step of single tokens (``weight`` and
+        ``state`` of a short convolution that adds its input); None where that is not one kernel."""
+        if (not isinstance(other, RMSNorm) or other.size != self.size or other.eps != self.eps or getattr(ctx, "max_q_len", 0) != 1
+                or self.size % 4 or self.size > 2048 or self.rt.dtype != torch.bfloat16 or (delta is not None and delta.dim() != 2)):
+            return None
+        n = x.shape[0]
+        return ops.rms_norm_pair_conv(x, self.weight, other.weight, self.eps, weight, state, ctx, self.rt.empty(n, self.size),
+                                      self.rt.empty(n, self.size), delta=delta)
+
     def lazy(self, x, delta=None, rows=None, write_back=True):
         """As ``forward``, for a consumer that can fold the norm into its first product: with few rows in
         bfloat16 the addend is summed into x now and the normalisation is left to that product."""

@@ -2,6 +2,8 @@
 engine's (odd widths, head sizes in steps of 16, vocabularies that are no power of two)."""
 import math
 
+from types import SimpleNamespace
+
 import numpy as np
 
 import pytest
@@ -2354,3 +2356,87 @@ def test_gemm_tiled_qkv_with_deep_pipelines(ops, nh, nkv, d, K, M, transposed, t
                 force(0)
         assert all(torch.equal(x, y) for x, y in zip(got[-2], got[-1]))
     assert not torch.equal(got[0][0], got[2][0])
+
+
+@pytest.mark.parametrize("H,G,D,E,ra,rg,pad", [(14, 2, 64, 64, 64, 64, 0), (4, 4, 16, 200, 8, 16, 2), (3, 1, 20, 100, 128, 8, 5),
+                                               (6, 2, 100, 32, 72, 128, 0), (2, 1, 128, 7, 40, 24, 1), (2, 2, 33, 64, 8, 8, 3)])
+def test_gated_delta_step(ops, H, G, D, E, ra, rg, pad):
+    """A decode step of the delta rule in one kernel against 64 bits, with key sizes of one lane to a column and of eight, fewer columns
+    than threads, ranks of one piece and of the most, rows of any stride, requests without tokens, and states of others left alone."""
+    g = torch.Generator().manual_seed(D + E)
+    r = lambda *s: torch.randn(*s, generator=g)     # noqa: E731
+    starts = [0, 1, 1, 2, 3, 4, 4]                            # requests 1 and 5 have no token
+    N, R = starts[-1], len(starts) - 1
+    cw = 2 * G * D + H * E
+    qkv = r(N, cw + pad).bfloat16()
+    proj = r(N, 3 + ra + rg + H + pad).bfloat16()
+    a_at, g_at, b_at = 3, 3 + ra, 3 + ra + rg
+    w_a2, w_g2 = (r(H * D, ra) / ra ** 0.5).bfloat16(), (r(H * E, rg) / rg ** 0.5).bfloat16()
+    A_log, dt, nw, S = r(H) / 4, r(H * D) / 2 - 2, 1 + r(E) / 8, r(R + 1, H, D, E)
+    slots = torch.tensor([3, 0, 5, 1, 6, 2], dtype=torch.int32)
+    want_S, want = S.double().clone(), torch.zeros(N, H, E, dtype=torch.float64)
+    for q in range(R):
+        if starts[q + 1] == starts[q]:
+            continue
+        n, s = starts[q], int(slots[q])
+        x, p = qkv[n].double(), proj[n].double()
+        a = (w_a2.double() @ p[a_at:a_at + ra] + dt.double()).view(H, D)
+        gate = torch.sigmoid(w_g2.double() @ p[g_at:g_at + rg]).view(H, E)
+        for h in range(H):
+            k_at = G * D + h // (H // G) * D
+            qq, kk, vv = x[h // (H // G) * D:][:D], x[k_at:k_at + D], x[2 * G * D + h * E:][:E]
+            qq, kk = qq / torch.sqrt(qq @ qq + 1e-6) / D ** 0.5, kk / torch.sqrt(kk @ kk + 1e-6)
+            T = torch.exp(-torch.exp(A_log[h].double()) * torch.nn.functional.softplus(a[h]))[:, None] * want_S[s, h]
+            T = T + kk[:, None] * (torch.sigmoid(p[b_at + h]) * (vv - kk @ T))[None]
+            want_S[s, h] = T
+            o = qq @ T
+            want[n, h] = o / torch.sqrt((o * o).mean() + 1e-6) * nw.double() * gate[h]
+    ctx = SimpleNamespace(num_requests=R, q_start=torch.tensor(starts, dtype=torch.int32, device=DEV), state_slots=slots.to(DEV), max_q_len=1)
+    assert ops.gated_delta_step_ok(proj.to(DEV), w_a2.to(DEV), w_g2.to(DEV), D, E)
+    Sd, out = S.to(DEV), torch.empty(N, H * E, dtype=torch.bfloat16, device=DEV)
+    ops.gated_delta_step(qkv.to(DEV)[:, :cw], proj.to(DEV), a_at, g_at, b_at, w_a2.to(DEV), w_g2.to(DEV), A_log.to(DEV), dt.to(DEV), nw.to(DEV),
+                         1e-6, Sd, ctx, out, H, G, D, E)
+    torch.testing.assert_close(Sd.cpu().double(), want_S, atol=2e-5, rtol=2e-5)
+    # one rounding to bfloat16 (2^-9), and the float errors of o over its norm
+    torch.testing.assert_close(out.cpu().double(), want.view(N, -1), atol=1e-3, rtol=5e-3)
+    assert torch.equal(Sd[[0, 2, 4]].cpu(), S[[0, 2, 4]])
+    assert not ops._get("ms_gated_delta_step_takes")(130, 8, 8, 8) and not ops._get("ms_gated_delta_step_takes")(64, 65, 8, 8)
+    assert not ops._get("ms_gated_delta_step_takes")(64, 64, 12, 8) and not ops._get("ms_gated_delta_step_takes")(64, 64, 8, 136)
+
+
+@pytest.mark.parametrize("H,taps,delta", [(896, 4, None), (60, 1, "same"), (1028, 8, "same"), (2048, 2, None), (100, 3, "float")])
+def test_norm_pair_with_the_convolution_is_the_two_one_after_the_other(ops, H, taps, delta):
+    """The same bits in both results, in x and in the states; a token that pads a batch moves no state."""
+    g = torch.Generator(device=DEV).manual_seed(H)
+    r = lambda *s: torch.randn(*s, generator=g, device=DEV)     # noqa: E731
+    N, live, dtype = 5, 4, torch.bfloat16
+    x, w1, w2, tw = r(N, H), 1 + r(H) / 8, 1 + r(H) / 8, r(H, taps) / 2
+    d = None if delta is None else r(N, H).to(torch.float32 if delta == "float" else dtype)
+    state = r(7, max(1, taps - 1), H).to(dtype)
+    ctx = SimpleNamespace(num_requests=N, token_req=torch.arange(N, dtype=torch.int32, device=DEV), max_q_len=1,
+                          q_start=torch.tensor([0, 1, 2, 3, 4, 4], dtype=torch.int32, device=DEV),
+                          state_slots=torch.tensor([5, 0, 2, 6, 1], dtype=torch.int32, device=DEV),
+                          n_live_tokens=torch.tensor([live], dtype=torch.int32, device=DEV))
+    new = lambda: torch.empty(N, H, dtype=dtype, device=DEV)     # noqa: E731
+    xa, sa, h, a2 = x.clone(), state.clone(), new(), new()
+    ops.rms_norm_pair(xa, w1, w2, 1e-6, h, a2, delta=d)
+    a1 = ops.short_conv(h, tw, sa, ctx, new(), ops.CONV_ADD_INPUT)
+    xb, sb = x.clone(), state.clone()
+    b1, b2 = ops.rms_norm_pair_conv(xb, w1, w2, 1e-6, tw, sb, ctx, new(), new(), delta=d)
+    assert torch.equal(sa, sb) and torch.equal(xa[:live], xb[:live])
+    assert torch.equal(a1[:live], b1[:live]) and torch.equal(a2[:live], b2[:live])
+
+
+@pytest.mark.parametrize("M,N,K", [(1, 7296, 896), (4, 7296, 896), (3, 900, 296), (8, 512, 512), (2, 1030, 1000)])
+def test_gemm_xielu(ops, M, N, K):
+    """The xIELU as the epilogue of the narrow matrices' product, against 64 bits; sizes that another kernel is for are left to it."""
+    g = torch.Generator(device=DEV).manual_seed(M + N)
+    a = torch.randn(M, K, generator=g, device=DEV).bfloat16()
+    w = (torch.randn(N, K, generator=g, device=DEV) * 2 / math.sqrt(K)).bfloat16()
+    pq = torch.tensor([0.3, -0.4], device=DEV)
+    got = ops.gemm_xielu(a, w, ops.xielu_numbers(pq))
+    z = a.double() @ w.double().T
+    p, q = torch.nn.functional.softplus(pq.double())
+    want = torch.where(z > 0, p * z * z + z / 2, (0.5 + q) * (torch.expm1(z.clamp(max=0)) - z) + z / 2)
+    torch.testing.assert_close(got.double(), want, atol=2e-3, rtol=5e-3)     # one rounding to bfloat16; the product's float error
+    assert ops.gemm_xielu(torch.zeros(9, K, device=DEV, dtype=torch.bfloat16), w, pq) is None
