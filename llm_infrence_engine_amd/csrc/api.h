@@ -110,6 +110,9 @@ int ms_gemm_tiled(const void* A, long long lda, const void* W, long long ldw, vo
 void ms_gemm_tiled_force(int tile);
 void ms_gemm_tiled_force_xcd_split(int xm);   // measurements: rows of XCDs over the tiles (1, 2, 4, 8); 0 leaves the choice
 int ms_gemm_tiled_sums_parts(int M, int N, int K);   // partial sums over runs of the columns: float [parts, M, N]; 0: not for it
+// float [M, N] of 17 to 64 tokens by very many short rows
+int ms_gemm_tiled_logits(const void* A, long long lda, const void* W, long long ldw, float* out, long long ldo, int M, int N, int K,
+                         hipStream_t stream);
 int ms_gemm_tiled_sums(const void* A, long long lda, const void* W, long long ldw, float* partial, int M, int N, int K, int parts,
                        hipStream_t stream);
 int ms_gemm_tiled_pays(int M, int N, int K);

@@ -280,6 +280,10 @@ extern "C" int ms_gemm_skinny(const void* A, long long lda, const void* W, long 
     rc = ms_gemm_stream(A, lda, nullptr, nullptr, 0.f, W, ldw, bias, out, ldo, M, N, K, epilogue, out_dtype, 0, 0, stream);
     if (rc != MS_UNSUPPORTED) return rc;
   }
+  if (M > 16 && !forced() && epilogue == EPI_STORE && out_dtype == MS_F32 && !bias && N > ms_compute_units() * 160 && K < 2048) {
+    const int rc = ms_gemm_tiled_logits(A, lda, W, ldw, (float*)out, ldo, M, N, K, stream);      // very many short rows
+    if (rc != MS_UNSUPPORTED) return rc;
+  }
   if (!forced()) {    // the kernel that holds the activations in LDS, where it takes the shape
     const int rc = ms_gemm_panel(A, lda, nullptr, nullptr, 0.f, W, ldw, bias, out, ldo, M, N, K, epilogue, out_dtype, 0, 0, stream);
     if (rc != MS_UNSUPPORTED) return rc;

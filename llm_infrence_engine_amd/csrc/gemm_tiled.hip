@@ -32,7 +32,9 @@ typedef __attribute__((ext_vector_type(4))) float f32x4;
 
 // beside the epilogues of common.h (without EPI_RESIDUAL): the q/k/v product's, the grouped product's, and EPI_SWIGLU with
 // the tanh form of the gelu for the silu
-enum { EPI_QKV = 2, EPI_GROUPED = 7, EPI_GEGLU = 4, EPI_SUMS = 8 };
+enum { EPI_QKV = 2, EPI_GROUPED = 7, EPI_GEGLU = 4, EPI_SUMS = 8, EPI_LOGITS = 10 };
+// float results as they are; EPI_LOGITS: of one tile of tokens, so W is read once and marked as not to be kept
+constexpr bool tiled_sums(int epi) { return epi == EPI_SUMS || epi == EPI_LOGITS; }
 
 // the gate's activation of a gated epilogue: g * sigmoid(g), or the tanh form of the gelu with the tanh as
 // 1 - 2 / (2^(2 y log2 e) + 1) through the hardware's exp2 and reciprocal (the result is rounded to bfloat16)
@@ -188,7 +190,7 @@ gemm_tiled_kernel(const bf16* __restrict__ A, size_t lda, const bf16* __restrict
   auto load_w = [&](int p, int step, int slot) {
     if ((p + 1) * NWAVES * 8 <= BN || (wave + p * NWAVES) * 8 < BN)   // the last round may be for some waves only
       __builtin_amdgcn_global_load_lds((global_void*)(src_w[p] + step * BK),
-                                       (lds_void*)(lds + slot + (wave + p * NWAVES) * 8 * PITCH), 16, 0, 0);
+                                       (lds_void*)(lds + slot + (wave + p * NWAVES) * 8 * PITCH), 16, 0, EPI == EPI_LOGITS ? 2 : 0);
   };
   auto load_a = [&](int p, int step, int slot) {
     if ((p + 1) * NWAVES * 8 <= BM || (wave + p * NWAVES) * 8 < BM)
@@ -430,7 +432,7 @@ gemm_tiled_kernel(const bf16* __restrict__ A, size_t lda, const bf16* __restrict
       for (int g = 0; g < 4 * FT; ++g) v[g] = grp.act ? tiled_gelu_erf(acc[g >> 2][j][g & 3]) : acc[g >> 2][j][g & 3];
       if (sizeof(TO) == 4) store_run_f32(reinterpret_cast<float*>(out) + row * ldo + f0, v, 4 * FT, N - f0);
       else store_run<4 * FT>(reinterpret_cast<bf16*>(out) + row * ldo + f0, v, N - f0);
-    } else if (EPI == EPI_SUMS) {
+    } else if (tiled_sums(EPI)) {
       float v[4 * FT];
 #pragma unroll
       for (int g = 0; g < 4 * FT; ++g) v[g] = acc[g >> 2][j][g & 3];
@@ -704,6 +706,17 @@ extern "C" int ms_gemm_tiled_sums(const void* A, long long lda, const void* W, l
     default: GO(2, 4, 4, 2, 3, 2);
   }
 #undef GO
+}
+
+// out [M, N] float = A . W^T for 17 to 64 tokens by very many short rows (a narrow model's head), which ms_gemm_slab leaves alone: its slabs
+// pay a start and an end each.  us of ms_gemm_panel | so: 151,936 x 896 at 17 tokens 65 | 51, 32 68 | 58, 64 81 | 68 (of W 5.3 to 4.0 TB/s; the
+// results are 39 MB more); x 1,536 105 | 85, 110 | 95, 132 | 113.  MS_UNSUPPORTED for what it does not take.
+extern "C" int ms_gemm_tiled_logits(const void* A, long long lda, const void* W, long long ldw, float* out, long long ldo, int M, int N, int K,
+                                    hipStream_t stream) {
+  if (M <= 0 || N <= 0) return MS_OK;
+  if (M > 64 || K <= 0 || K % BK || lda % 8 || ldw % 8 || lda < K || ldw < K || ldo < N) return MS_UNSUPPORTED;
+  if (((uintptr_t)A | (uintptr_t)W) % 16) return MS_UNSUPPORTED;
+  return launch<1, 4, 4, 1, 5, 4, EPI_LOGITS, float>((const bf16*)A, lda, (const bf16*)W, ldw, out, ldo, M, N, K, stream);
 }
 
 // The grouped product of routed experts on this kernel: for every tile t of tile_rows rows (ms_gemm_tiled_grouped_rows()

@@ -2440,3 +2440,16 @@ def test_gemm_xielu(ops, M, N, K):
     want = torch.where(z > 0, p * z * z + z / 2, (0.5 + q) * (torch.expm1(z.clamp(max=0)) - z) + z / 2)
     torch.testing.assert_close(got.double(), want, atol=2e-3, rtol=5e-3)     # one rounding to bfloat16; the product's float error
     assert ops.gemm_xielu(torch.zeros(9, K, device=DEV, dtype=torch.bfloat16), w, pq) is None
+
+
+@pytest.mark.parametrize("M,N,K", [(17, 41024, 64), (64, 41000, 192), (33, 50001, 896), (40, 41030, 1984)])
+def test_logits_of_17_to_64_tokens_by_very_many_rows(ops, M, N, K):
+    """A narrow model's head on tiles of 64 x 64: rows that fill no whole tile, results whose rows start on no 16 bytes, one step of columns and
+    many; against 64 bits, and a row's bits do not hang on the others."""
+    g = torch.Generator(device=DEV).manual_seed(M + N)
+    a = torch.randn(64, K, generator=g, device=DEV).bfloat16()
+    w = (torch.randn(N, K, generator=g, device=DEV) / math.sqrt(K)).bfloat16()
+    got = ops.gemm_skinny(a[:M], w, out_dtype=torch.float32)
+    torch.testing.assert_close(got.double(), a[:M].double() @ w.double().T, atol=3e-5, rtol=3e-5)
+    assert torch.equal(got, ops.gemm_skinny(a, w, out_dtype=torch.float32)[:M])
+    assert torch.equal(got, ops.gemm_tiled_sums(a[:M], w, 1)[0])
