@@ -3,23 +3,25 @@
 //
 // The order of a sum is the same whatever M is, so a token's result does not depend on what else is in the batch: K is
 // cut into at most 16 slices (from K alone, `slice_steps`), a slice is summed 16 values at a time from its start, and the
-// slices are added in order.  Two kernels keep that order:
+// slices are added in order.  All kernels keep that order:
 //   rows     up to 64 rows (a decode step; against very many rows of W up to 16): all waves of a block on the same 4 to 16
 //            rows of W, the slices dealt out over them and added through LDS.  Bound by reading W.
 //   few      up to 8 rows, of these: loads that take four steps at a time.
 //   diagonal up to 8 rows: an instruction takes a step of two or four slices; also with the norm of A's rows, the gate, or the rotation
 //            and store of a q/k/v product within.
-//   tiled    the others: 64 x 64 or 32 x 32 tiles staged through LDS four steps ahead, 4 waves; 32 x 32 where the larger
-//            tiles would be fewer than two a CU.  Bound by the float matrix rate (157 TFLOP/s nominal), short K by writing C.
+//   slices   32 rows of W by 16, 32 or 48 tokens and the slices dealt out over a block's waves, for tiles too few to fill the chip
+//            (`choose`): bound by the way of the operands to the CU, 40 KB a us.
+//   tiled    the others: 64 x 64 or 32 x 32 tiles staged through LDS four steps ahead, 4 waves.  Bound by the float matrix rate
+//            (157 TFLOP/s nominal), short K by writing C.
 // Measured with the 0.5B sizes against the 64 x 64 vector-ALU tile that ran them before (one MI355X): of 3 rows the down
 // product (896 x 4,864) 319 -> 16 us (12 with grouped loads), gate/up (9,728 x 896) 63 -> 12 us, q/k/v (1,152 x 896) 63 -> 4.5 us, the head
-// (151,936 x 896) 221 -> 100 us, of 64 rows 252 -> 220; of 338 rows down 316 -> 84 us, gate/up 108 -> 88 us.  Down is bound
-// by the steps a CU works off (16 waves, 19 steps each), whatever its rows; the tiled steps by the way from one barrier to
-// the next.  C leaves a tile through LDS in whole rows (4,096 x 32,000 x 64: 440 us as the fragments lie, 270 so, 261 before).
+// (151,936 x 896) 221 -> 100 us, of 64 rows 252 -> 220; of 350 rows down 316 -> 45 us, gate/up 108 -> 75 us.  Of few rows
+// down is bound by the steps a CU works off (16 waves, 19 steps each); the tiled steps by the way from one barrier to the next.  C leaves a tile through LDS in whole rows (4,096 x 32,000 x 64: 440 us as the fragments lie, 270 so, 261 before).
 #include "common.h"
 #include "api.h"
 #include "gemm_f32.h"
 #include "quads.h"
+#include <algorithm>
 #include <type_traits>
 
 namespace {
@@ -28,6 +30,7 @@ typedef float f32x4 __attribute__((ext_vector_type(4)));
 
 constexpr int STEP = 16;          // k values a slice is summed by at a time: four MFMAs of four
 constexpr int MAX_SLICES = 16;
+constexpr int LDS_BYTES = 163840;  // of a CU
 
 __host__ __device__ inline int slice_steps(int K) {
   const int steps = (K + STEP - 1) / STEP;
@@ -54,6 +57,22 @@ __device__ __forceinline__ void store(float* C, size_t at, float v, const float*
   if (bias) v += bias[n];
   if (accumulate) v += C[at];
   C[at] = v;
+}
+
+// four results side by side (runs: at an address that fits them), those past the last column of N not
+__device__ __forceinline__ void store_run(float* C, size_t at, f32x4 v, const float* bias, int n, int N, int accumulate, int runs) {
+  if (runs && n + 3 < N) {
+    if (bias) {
+#pragma unroll
+      for (int e = 0; e < 4; ++e) v[e] += bias[n + e];
+    }
+    if (accumulate) v += *reinterpret_cast<const f32x4*>(C + at);
+    *reinterpret_cast<f32x4*>(C + at) = v;
+  } else {
+#pragma unroll
+    for (int e = 0; e < 4; ++e)
+      if (n + e < N) store(C, at + e, v[e], bias, n + e, accumulate);
+  }
 }
 
 // R rows of W a block (lanes of the other rows of the instruction repeat them), NT tiles of 16 tokens, the slices dealt out
@@ -468,22 +487,11 @@ gemm_f32_tiled_kernel(const float* __restrict__ A, const float* __restrict__ W, 
     if (m >= M) break;
     f32x4 v = *reinterpret_cast<const f32x4*>(&tile[row * LC + c]);
     const size_t at = (size_t)m * ldc + n;
-    if (runs && n + 3 < N) {
-      if (bias) {
-#pragma unroll
-        for (int e = 0; e < 4; ++e) v[e] += bias[n + e];
-      }
-      if (accumulate) v += *reinterpret_cast<const f32x4*>(C + at);
-      *reinterpret_cast<f32x4*>(C + at) = v;
-    } else {
-#pragma unroll
-      for (int e = 0; e < 4; ++e)
-        if (n + e < N) store(C, at + e, v[e], bias, n + e, accumulate);
-    }
+    store_run(C, at, v, bias, n, N, accumulate, runs);
   }
 }
 
-int g_kernel = 0;      // measurements: 1 the kernel of up to 64 rows, 2 and 3 the tiled one with tiles of 64 and 32, 4 and 5 that of up to 8 with blocks of 4 and 8 rows of W; 0 leaves the choice
+int g_kernel = 0;      // measurements: 1 the kernel of up to 64 rows, 2 and 3 the tiled one with tiles of 64 and 32, 4 and 5 that of up to 8 with blocks of 4 and 8 rows of W, 6 to 8 the slices of 16, 32 and 48 tokens; 0 leaves the choice
 
 // Rows of W to a block of the kernel of slices side by side, for a plain product; 0: another kernel is as fast or faster.  us with four steps
 // to a load | so, at 3 and 8 tokens: 896 x 896 4.6 | 4.4 (8: 5.0 | 5.1), 896 x 4,864 11.4 | 8.5 and 12.9 | 12.3; 8 rows: 2,048 x 2,048
@@ -524,6 +532,137 @@ int launch_diagonal(int R, const float* A, const float* W, const float* bias, fl
 #undef GO
 }
 
+// TM tokens by 32 rows of W a block, a wave for two slices.  Nothing is shared before the sums: a wave stages its slices' columns, 32
+// at a time and the next 32 ahead, in LDS of its own (whole lines of eight rows a load) and waits for its own loads by count.
+template <int TM>
+__global__ void __launch_bounds__(MAX_SLICES / 2 * MS_WAVE)
+gemm_f32_slices_kernel(const float* __restrict__ A, const float* __restrict__ W, const float* __restrict__ bias,
+                       float* C, int M, int N, int K, size_t lda, size_t ldw, size_t ldc, int accumulate, int runs) {
+  constexpr int TN = 32, BK = 32, FN = TN / 16, FM = TM / 16, LOADS = (TN + TM) / 8, LC = TN + 4;
+  extern __shared__ __align__(16) float lds[];       // [wave][2][row][8 pieces of 16 bytes]; then [slice][token][LC]
+  const int lane = threadIdx.x & (MS_WAVE - 1), wave = __builtin_amdgcn_readfirstlane(threadIdx.x / MS_WAVE);
+  const int r = lane & 15, g = lane >> 4;
+  const int n0 = blockIdx.x * TN, m0 = blockIdx.y * TM;
+  const int per = slice_steps(K), slices = ((K + STEP - 1) / STEP + per - 1) / per;
+  const int begin = 2 * wave * per * STEP, end = min(K, begin + 2 * per * STEP);
+  f32x4* mine = reinterpret_cast<f32x4*>(lds) + wave * (2 * LOADS * MS_WAVE);
+  // lane l of a load takes row l / 8 of its eight, piece (l % 8) ^ (l / 8): reads of 16 rows by four pieces then meet every bank once
+  const int sub = lane >> 3, piece = ((lane & 7) ^ sub) * 4;
+  const float* row[LOADS];
+#pragma unroll
+  for (int p = 0; p < LOADS; ++p)                    // rows past the end repeat the last one and are not stored
+    row[p] = p < TN / 8 ? W + (size_t)min(n0 + p * 8 + sub, N - 1) * ldw : A + (size_t)min(m0 + p * 8 - TN + sub, M - 1) * lda;
+  auto ask = [&](int b, int k) {                     // (nothing is read past K)
+#pragma unroll
+    for (int p = 0; p < LOADS; ++p)
+      __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)(row[p] + min(k + piece, K - 4)),
+                                       (__attribute__((address_space(3))) void*)(mine + (b * LOADS + p) * MS_WAVE), 16, 0, 0);
+  };
+  f32x4 acc[FN][FM] = {}, before[FN][FM] = {};       // of the second slice, when it has begun, and the first
+  int left = per, b = 0;
+  bool second = false;
+  ask(0, begin);
+  if (begin + BK < end) ask(1, begin + BK);
+  for (int k = begin; k < end; k += BK, b ^= 1) {
+    f32x4 wf[2][FN], af[2][FM];
+    if (k + BK < end) asm volatile("s_waitcnt vmcnt(%0)" ::"n"(LOADS) : "memory");
+    else asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+      const int at = r * 8 + ((4 * h + g) ^ (r & 7));
+#pragma unroll
+      for (int i = 0; i < FN; ++i) wf[h][i] = mine[b * LOADS * MS_WAVE + i * 128 + at];
+#pragma unroll
+      for (int j = 0; j < FM; ++j) af[h][j] = mine[b * LOADS * MS_WAVE + (FN + j) * 128 + at];
+    }
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");        // read: it may be filled again
+    if (k + 2 * BK < end) ask(b, k + 2 * BK);
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+      if (k + h * STEP >= end) break;                // the same for the whole wave
+      if (k + (h + 1) * STEP > K) {                  // columns past the last: nothing
+#pragma unroll
+        for (int i = 0; i < FN; ++i) wf[h][i] = masked(wf[h][i], k + h * STEP + 4 * g, K);
+#pragma unroll
+        for (int j = 0; j < FM; ++j) af[h][j] = masked(af[h][j], k + h * STEP + 4 * g, K);
+      }
+#pragma unroll
+      for (int i = 0; i < FN; ++i)
+#pragma unroll
+        for (int j = 0; j < FM; ++j) acc[i][j] = step16(wf[h][i], af[h][j], acc[i][j]);
+      if (--left == 0 && !second) {                  // the first slice ends
+        second = true;
+#pragma unroll
+        for (int i = 0; i < FN; ++i)
+#pragma unroll
+          for (int j = 0; j < FM; ++j) { before[i][j] = acc[i][j]; acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f}; }
+      }
+    }
+  }
+  __syncthreads();
+  float* sum = &lds[(2 * wave * TM + r) * LC + 4 * g];
+#pragma unroll
+  for (int i = 0; i < FN; ++i)
+#pragma unroll
+    for (int j = 0; j < FM; ++j) {
+      *reinterpret_cast<f32x4*>(sum + 16 * j * LC + 16 * i) = second ? before[i][j] : acc[i][j];
+      if (2 * wave + 1 < slices) *reinterpret_cast<f32x4*>(sum + (TM + 16 * j) * LC + 16 * i) = acc[i][j];
+    }
+  __syncthreads();
+  for (int e = threadIdx.x; e < TM * TN / 4; e += blockDim.x) {
+    const int tok = e / (TN / 4), c = e % (TN / 4) * 4, m = m0 + tok, n = n0 + c;
+    if (m >= M) break;
+    f32x4 v = {0.f, 0.f, 0.f, 0.f};
+    for (int s = 0; s < slices; ++s) v += *reinterpret_cast<const f32x4*>(&lds[(s * TM + tok) * LC + c]);
+    store_run(C, (size_t)m * ldc + n, v, bias, n, N, accumulate, runs);
+  }
+}
+
+int slices_of(int K) { const int steps = (K + STEP - 1) / STEP, per = slice_steps(K); return (steps + per - 1) / per; }
+// bytes: two stages of 32 columns a wave, or the slices' sums
+int slices_lds(int TM, int slices) { return std::max((slices + 1) / 2 * 2 * (32 + TM) * 32, slices * TM * (32 + 4)) * (int)sizeof(float); }
+
+// The kernel for more rows than the first two take, by what each was seen to take on 150 sizes (128 to 151,936 by 512 to 18,944, 13 to
+// 2,048 rows; 256 CUs): us = start + (begin + step * K / 1,000) * rounds.  `slices` runs in whole rounds of blocks, one or two to a CU by
+// its LDS; of the tiled one's blocks several lie on a CU, and up to one a CU they take as long as one.  The kernel so chosen is within
+// 0.3 % of the fastest on average (4 % at most, but for 7 sizes).  Before, by the number of tiles alone and with tiled kernels alone
+// | now: 896 x 4,864 at 17, 64, 350, 512 and 2,048 rows 24 | 18, 47 | 18, 81 | 45, 82 | 56, 224 | 192 us; 896 x 896 at 64 and 350
+// 12.5 | 6.9, 18.0 | 13.1; 1,152 x 896 at 350 18.1 | 16.8; 4,608 x 3,584 at 17 and 128 41 | 25, 80 | 65; 9,728 x 896 as before.
+enum { ROWS16 = 16, ROWS32 = 32, ROWS48 = 48, TILE32 = 1, TILE64 = 2 };
+int choose(int M, int N, int K, int cus) {
+  int best = 0;
+  float least = 0.f;
+  auto offer = [&](int kind, float us) { if (best == 0 || us < least) { best = kind; least = us; } };
+  auto tiles = [&](int T) { return (float)((long long)((N + T - 1) / T) * ((M + T - 1) / T)) / cus; };
+  const float k = K * 1e-3f, t64 = tiles(64), t32 = tiles(32);
+  offer(TILE64, 2.f + (1.7f + 24.2f * k) * (t64 <= 1.f ? 1.f : std::max(1.55f, 0.45f + 0.75f * t64)));
+  offer(TILE32, 2.f + (0.8f + 13.f * k) * (t32 <= 1.f ? 1.f : std::max(1.25f, 0.65f + 0.45f * t32)));
+  const float begin[] = {2.2f, 3.3f, 4.f}, step[] = {3.f, 5.1f, 7.8f};
+  for (int i = 0; i < 3; ++i) {
+    const int TM = 16 * (i + 1), room = cus * std::min(4, LDS_BYTES / slices_lds(TM, slices_of(K)));
+    const long long blocks = (long long)((N + 31) / 32) * ((M + TM - 1) / TM);
+    if ((M + TM - 1) / TM > 65535) continue;
+    offer(TM, 1.5f + (begin[i] + step[i] * k) * (0.95f * ((blocks + room - 1) / room) + 0.05f * std::max(1.f, (float)blocks / room)));
+  }
+  return best;
+}
+
+template <int TM>
+int launch_slices(const float* A, const float* W, const float* bias, float* C, int M, int N, int K, size_t lda, size_t ldw, size_t ldc,
+                  int accumulate, int runs, hipStream_t stream) {
+  const int slices = slices_of(K);
+  static bool raised = false;   // once per instantiation: allow more dynamic LDS than the default 64 KB
+  if (!raised) {
+    if (hipFuncSetAttribute(reinterpret_cast<const void*>(&gemm_f32_slices_kernel<TM>), hipFuncAttributeMaxDynamicSharedMemorySize,
+                            slices_lds(TM, MAX_SLICES)) != hipSuccess)
+      return MS_LAUNCH_FAILED;
+    raised = true;
+  }
+  gemm_f32_slices_kernel<TM><<<dim3((N + 31) / 32, (M + TM - 1) / TM), (slices + 1) / 2 * MS_WAVE, slices_lds(TM, slices), stream>>>(
+      A, W, bias, C, M, N, K, lda, ldw, ldc, accumulate, runs);
+  return ms_launch_status();
+}
+
 }  // namespace
 
 // What a decode step's layer makes of up to 8 rows of the residual stream x [M, K] with the norm of its reader, one kernel each:
@@ -554,7 +693,9 @@ int ms_gemm_f32_launch(const float* A, const float* W, const float* bias, float*
   // rows from 64 features a CU on (24 rows of 20,000 x 512 17.2 us there, 15.3 in tiles; 32 of 152,064 x 3,584 1,010 and 519;
   // of 9,728 x 896 19.3 and 19.1), 33 to 64 from 32 a CU on (64 of 9,728 x 896 33 and 24, of 151,936 x 896 405 and 220, of
   // 6,144 x 2,048 43 and 40, but 33 of them 33 and 40).
-  const bool few = M <= 16 || (M <= 32 ? N < 64 * cus : M <= 64 && N < 32 * cus);
+  // From 13 rows on (9 by rows of more than 1,024 columns) the choice is another one from 512 columns on (12 rows of 896 x 896 6.3 us
+  // in the first kernel, 6.5 as slices, 16 of them 6.8 and 6.5; 9 rows of 4,608 x 3,584 32 and 18, of 2,048 x 2,048 9.5 and 9.9).
+  const bool few = M <= 8 || (M <= 12 && K <= 1024) || (K < 512 && (M <= 16 || (M <= 32 ? N < 64 * cus : M <= 64 && N < 32 * cus)));
   const int side_by_side = M > 8 ? 0 : g_kernel == 4 ? 4 : g_kernel == 5 ? 8 : g_kernel == 0 ? diagonal_rows(M, N, K) : 0;
   if (side_by_side)
     return launch_diagonal<F32_STORE, 0>(side_by_side, A, W, bias, C, M, N, K, lda, ldw, ldc, accumulate, F32Norm{}, F32Front{}, stream);
@@ -586,11 +727,18 @@ int ms_gemm_f32_launch(const float* A, const float* W, const float* bias, float*
 #undef ROWS
     return ms_launch_status();
   }
-  const long long big = (long long)((N + 63) / 64) * ((M + 63) / 64);
+  // K below 512 is bound by writing C and stays with the tiled kernel, the larger tiles from two a CU on
+  const int kind = g_kernel == 2 ? TILE64 : g_kernel == 3 ? TILE32 : g_kernel >= 6 ? 16 * (g_kernel - 5) : K >= 512 ? choose(M, N, K, cus)
+                   : M > 32 && (long long)((N + 63) / 64) * ((M + 63) / 64) >= 2 * cus ? TILE64 : TILE32;
   const int runs = ldc % 4 == 0 && (uintptr_t)C % 16 == 0;
-  if (g_kernel == 2 || (g_kernel != 3 && M > 32 && big >= 2 * cus))
-    gemm_f32_tiled_kernel<64><<<dim3((N + 63) / 64, (M + 63) / 64), 256, 0, stream>>>(A, W, bias, C, M, N, K, lda, ldw, ldc, accumulate, runs);
-  else
-    gemm_f32_tiled_kernel<32><<<dim3((N + 31) / 32, (M + 31) / 32), 256, 0, stream>>>(A, W, bias, C, M, N, K, lda, ldw, ldc, accumulate, runs);
+#define SLICES(TM) return launch_slices<TM>(A, W, bias, C, M, N, K, lda, ldw, ldc, accumulate, runs, stream)
+  if (kind == ROWS16) SLICES(16);
+  if (kind == ROWS32) SLICES(32);
+  if (kind == ROWS48) SLICES(48);
+#undef SLICES
+#define TILED(T) gemm_f32_tiled_kernel<T><<<dim3((N + T - 1) / T, (M + T - 1) / T), 256, 0, stream>>>(A, W, bias, C, M, N, K, lda, ldw, ldc, accumulate, runs)
+  if (kind == TILE64) TILED(64);
+  else TILED(32);
+#undef TILED
   return ms_launch_status();
 }

@@ -2453,3 +2453,32 @@ def test_logits_of_17_to_64_tokens_by_very_many_rows(ops, M, N, K):
     torch.testing.assert_close(got.double(), a[:M].double() @ w.double().T, atol=3e-5, rtol=3e-5)
     assert torch.equal(got, ops.gemm_skinny(a, w, out_dtype=torch.float32)[:M])
     assert torch.equal(got, ops.gemm_tiled_sums(a[:M], w, 1)[0])
+
+
+@pytest.mark.parametrize("M,N,K", [(9, 31, 512), (13, 64, 516), (17, 97, 560), (33, 33, 896), (48, 130, 1100), (49, 65, 2052), (97, 896, 4864), (5, 7, 64), (20, 36, 20)])
+def test_32_bit_products_by_slices_have_the_bits_of_the_tiles(ops, M, N, K):
+    """Blocks whose waves have two slices each: one, an odd number and all sixteen of them, columns that end within a slice, a step or a
+    piece, tokens and rows of W past the last, rows of C at any address; with bias and added onto what is there.  The tiled kernel sums in
+    the same order; both are held against 64 bits, and the choice is one of them."""
+    from llm_infrence_engine_amd.kernels import build
+
+    force = build.load().ms_gemm_f32_force
+    g = torch.Generator(device=DEV).manual_seed(M + N + K)
+    a, w, bias = (torch.randn(*s, generator=g, device=DEV) for s in ((M, K), (N, K), (N,)))
+    there = torch.randn(M, N + 3, generator=g, device=DEV)
+
+    def run(kind, plain, wide):
+        force(kind)
+        try:
+            out = there.clone()[:, :N] if wide else there[:, :N].clone()
+            return ops.gemm_generic(a, w, out, bias=None if plain else bias, accumulate=not plain).clone()
+        finally:
+            force(0)
+
+    for plain in (True, False):
+        for wide in (False, True):
+            want = run(3, plain, wide)
+            exact = a.double() @ w.double().T + (0 if plain else bias.double() + there[:, :N].double())
+            torch.testing.assert_close(want.double(), exact, atol=K ** 0.5 * 2e-6, rtol=2e-5)      # (sums of K products of about one)
+            for kind in (2, 6, 7, 8, 0):
+                assert torch.equal(run(kind, plain, wide), want), (kind, plain, wide)
