@@ -202,7 +202,15 @@ class CacheManager:
         """True if every group has the pages for ``new_len`` tokens and ``reserve`` more."""
         if new_len > self.max_len:
             return False
-        return all(g.allocator.num_free() >= n + reserve for g, n in zip(self.groups, self.pages_to_grow(req_id, new_len)))
+        h = self._held[req_id]
+        for i, g in enumerate(self.groups):
+            entries, held = new_len // g.key.stride, h.next_page[i] * self.page_size
+            if entries <= held:
+                if reserve and g.allocator.num_free() < reserve:
+                    return False
+            elif g.allocator.num_free() < -(-(entries - held) // self.page_size) + reserve:
+                return False
+        return True
 
     def tokens_that_fit(self, req_id, reserve: int = 0) -> int:
         """How many more tokens than it has stored the request could hold with the free pages of every group,
@@ -220,6 +228,11 @@ class CacheManager:
         if new_len > self.max_len:
             raise ValueError(f"request {req_id!r} would hold {new_len} tokens; the tables are made for {self.max_len}")
         h = self._held[req_id]
+        for i, g in enumerate(self.groups):
+            if new_len // g.key.stride > h.next_page[i] * self.page_size:
+                break
+        else:
+            return                 # as nearly always with a decode step
         needs = self.pages_to_grow(req_id, new_len)
         for g, n in zip(self.groups, needs):
             if g.allocator.num_free() < n:
@@ -235,10 +248,13 @@ class CacheManager:
         h = self._held[req_id]
         if computed < h.computed:
             raise ValueError("a request's stored tokens cannot shrink; free it and add it again")
-        if any(self.entries(i, computed) > h.next_page[i] * self.page_size for i in range(len(self.groups))):
-            raise ValueError(f"request {req_id!r}: {computed} tokens stored but pages for fewer were allocated")
+        for i, g in enumerate(self.groups):
+            if computed // g.key.stride > h.next_page[i] * self.page_size:
+                raise ValueError(f"request {req_id!r}: {computed} tokens stored but pages for fewer were allocated")
         h.computed = computed
         for i, g in enumerate(self.groups):
+            if g.key.window is None:
+                continue
             first = min(self._first_needed(g, computed), h.next_page[i])
             if first > h.first_live[i]:
                 for p in range(h.first_live[i], first):

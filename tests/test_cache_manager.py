@@ -194,3 +194,44 @@ def test_tokens_that_fit_counts_every_group():
     assert m.tokens_that_fit("a") == 7          # two pages held (8 tokens) and one free in the small pool, 5 stored
     with pytest.raises(ValueError, match="pool sizes"):
         CacheManager(CacheLayout([full()]), 4, [3, 3], 2, 64)
+
+
+@pytest.mark.parametrize("window,stride", [(None, 1), (9, 1), (None, 4)])
+@pytest.mark.parametrize("steps", [1, 8])
+def test_steps_of_single_tokens_are_described_as_in_general(window, stride, steps):
+    """Rows, starts and wanted places drawn at random, a request at its start, contexts up to the last token the cache holds; what the
+    general way refuses (a token outside the vocabulary, no page, a context too long, a place beyond the token) is refused alike."""
+    from llm_infrence_engine_amd.engine.batch import BatchBuilder, StepEntry
+    from llm_infrence_engine_amd.parts.base import CacheNeed, PageTensor
+
+    needs = [full(), (CacheNeed((PageTensor("k", 1, 8),), window=window, stride=stride), None, None)]
+    rng = random.Random(steps)
+    for R in (1, 3, 70):
+        m = CacheManager(CacheLayout(needs), 4, 40 * R, R + 2, 64)
+        single, general = (BatchBuilder(m, None, 50, "cpu") for _ in range(2))
+        general._describe_single = lambda entries, steps: None
+        for r in rng.sample(range(R), R):
+            m.add(r)
+            at = 0 if r == 0 else 64 - steps if r == 1 else rng.randrange(0, 64 - steps + 1)
+            m.grow(r, at + steps)
+            m.advance(r, at)
+        entries = [StepEntry(r, [rng.randrange(50)], [0] * rng.randrange(3)) for r in range(R)]
+        assert (single._describe_single(entries, steps) is not None) == (stride == 1)
+        got, want = single.describe(entries, steps), general.describe(entries, steps)
+        for name in vars(want):
+            a, b = getattr(got, name), getattr(want, name)
+            for x, y in zip(a, b, strict=True) if name == "slots" else [(a, b)]:
+                assert np.array_equal(x, y) and getattr(x, "dtype", None) == getattr(y, "dtype", None), name
+        for bad in (StepEntry(0, [50]), StepEntry(0, [-1]), StepEntry(0, [1], [1]), StepEntry(0, [1], [-1])):
+            for b in (single, general):
+                with pytest.raises(ValueError):
+                    b.describe([bad] + entries[1:], steps)
+        m.free(0)
+        m.add(0)
+        for b in (single, general):
+            with pytest.raises(RuntimeError, match="no page"):
+                b.describe(entries, steps)
+        if R > 1:
+            for b in (single, general):
+                with pytest.raises(ValueError, match="made for 64"):
+                    b.describe(entries[1:], steps + 1)
