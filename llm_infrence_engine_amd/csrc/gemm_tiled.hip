@@ -669,6 +669,9 @@ extern "C" int ms_gemm_tiled(const void* A, long long lda, const void* W, long l
 //     features (0.81 to 1.2), 4,096 columns (0.93 to 1.12), 1,024 and fewer for more features (0.87 to 1.0);
 //   up to 1,024 tokens by more than 8,192 columns, up to 5,120 features or by 16,384 columns and more, 0.92 to 3.2, 1.33 on average;
 //     else 0.88 to 2.0, 1.08 on average (8,192 columns 0.89 to 1.17);
+//   up to 1,000 tokens by 4,096 to 8,192 columns for up to 2,048 features, in three parts and more or, from 5,600 columns on, in two of
+//     the tiles of 128, 0.97 to 1.38, 1.1 on average (270 sizes with the norm; 896 x 4,864 by 640 and 768 tokens 24.4 -> 21.8 and 24.4 ->
+//     22.3 us).  Not: whole columns (0.81 to 0.83), two parts of fewer columns (0.95 to 1.06) or of tiles of 64 (0.95 to 1.02);
 //   in all 12 of 3,416 below 0.97;
 //   beyond, by 16,384 columns and more where one round of blocks in parts fills 5/6 of the CUs, but not all: 0.96 to 2.0, 1.4 on
 //     average (3,584 x 18,944 at 1,281 to 1,536 tokens and at 1,793 to 2,304).  With every CU taken 0.96 to 1.02 (4,096 x 28,672 at 2,048
@@ -678,10 +681,12 @@ extern "C" int ms_gemm_tiled_sums_parts(int M, int N, int K) {
   if (M <= 64 || N <= 0 || K < 768 || K % BK || N > 8192) return 0;
   if (M > 128 && (M <= 256 ? K > 1024 && K < 4096
                   : M <= 512 ? K <= 8192 && (K <= 4096 || N > 5120) && (K > 1024 || N > 1024)
+                  : M <= 1000 && N <= 2048 && K > 4096 ? false
                   : M <= 1024 ? K <= 8192 || (N > 5120 && K < 16384) : K < 16384)) return 0;   // (asked for twice a layer: before the choice)
   const SumsChoice c = choose_sums(M, N, K);
   const int cus = ms_compute_units();
   if (M > 256 && M <= 512 && K > 4096 && K <= 8192 && (c.parts == 1 || c.blocks > cus)) return 0;
+  if (M > 512 && M <= 1024 && K <= 8192 && c.parts < 3 && (c.parts == 1 || K < 5600 || c.tile == T64 || c.tile == T64_DEEP)) return 0;
   if (M > 1024 && (c.tile != T256 || c.parts == 1 || c.blocks >= cus || c.blocks * 6 < cus * 5)) return 0;
   return c.parts;
 }

@@ -767,3 +767,12 @@ def test_a_model_whose_weights_lie_anywhere_steps_as_one_whose_do_not(ops):
         assert (r.chain is None) == aside
     for a, b in zip(*got):
         _like(b, a)
+
+
+@pytest.mark.parametrize("M,N,K,parts", [
+    # times of the library and the norm over partial sums and the norm
+    (640, 896, 4864, 4), (768, 896, 4864, 4), (1000, 896, 4864, 4), (560, 512, 4864, 3), (960, 768, 6912, 5), (700, 2048, 8192, 2),    # 1.12 1.09 1.04 1.14 1.15 1.14
+    (560, 896, 4864, 0), (770, 1152, 4352, 0), (900, 1536, 4864, 0), (900, 512, 8192, 0),        # 0.99 0.81 0.98 0.98
+    (1001, 896, 4864, 0), (768, 896, 4096, 0), (768, 2176, 8192, 0)])                            # as ever
+def test_where_products_of_narrow_models_by_long_rows_leave_partial_sums(ops, M, N, K, parts):
+    assert ops._get("ms_gemm_tiled_sums_parts")(M, N, K) == parts
