@@ -546,24 +546,31 @@ TileChoice choose_tile(int M, int N, int K) {
   return best;
 }
 
-// Tile and column parts of a product in partial sums, the least time by such a model (100 sizes, 768 to 3,584 features, 896 to 18,944
-// columns, 65 to 2,048 tokens: 2.6 % behind the best on average): a launch, a round and its steps, what a block more costs its CU, and a write and a read
-// of every sum at 5 TB/s.  With the two deep tiles 0.5B down projections take 1 to 2 us less (896 x 4,864: 65 tokens 8.3 -> 7.2, 512 17.9 -> 16.9).
+// Tile and column parts of a product in partial sums: the least time, with the norm that adds them up, by a model of 4,200 measurements (150
+// sizes, 896 to 5,120 features, 896 to 18,944 columns, 65 to 1,000 tokens, five tiles, one to eight parts): 0.8 % behind the best on average, 8 % at
+// most (a model of the three older tiles, without the norm, 2.8 % and 30): a launch and the norm; rounds of blocks, a step of one and what its
+// neighbours on the CU and the other CUs add to it; the sums and the result, written and read.  896 x 4,864 at 100 and 400 tokens 11.1 -> 10.7 and
+// 18.0 -> 17.7 us, 3,584 x 18,944 at 150 65 -> 50, 1,536 x 8,960 at 128 20.0 -> 16.7.  Few rows of a large W are read faster by two blocks to a CU
+// (5,120 x 13,824 at 65 tokens 40.5 us, 44.0 in the deep tiles).
 struct SumsChoice { int tile, parts; double us; long long blocks; };
 
 SumsChoice choose_sums(int M, int N, int K) {
   const long long cus = ms_compute_units();
   const int steps = K / BK;
-  const struct { int tile, size; double fixed, round, step, block; } kinds[] = {{T256, 256, 2.28, 5.20, 1.11, 17.61}, {T128, 128, 3.51, 0.00, 0.50, 5.03},
-                                                                              {T64, 64, 3.96, 0.00, 0.25, 0.59},    {T128_DEEP, 128, 2.18, 1.14, 0.47, 5.88},
-                                                                              {T64_DEEP, 64, 3.07, 0.00, 0.25, 1.08}};
+  const struct { int tile, size, to_a_cu; double start, round, step, beside, over, busy, sums, result; } kinds[] = {
+      {T256, 256, 1, 0.19, 5.74, 1.15, 0.00, 0.00, 0.24, 1.40, 0.33},     {T128, 128, 2, 7.16, 0.15, 0.48, 0.61, 0.20, 0.23, 1.13, 0.04},
+      {T64, 64, 4, 5.44, 0.00, 0.30, 2.24, 0.00, 0.10, 1.78, 0.02},       {T64_DEEP, 64, 2, 5.87, 0.03, 0.28, 0.48, 0.54, 0.06, 1.39, 0.04},
+      {T128_DEEP, 128, 1, 7.12, 0.37, 0.43, 0.00, 0.00, 0.09, 1.52, 0.02}};
   SumsChoice best{0, 1, 1e30, 0};
   for (const auto& k : kinds) {
-    const long long tiles = (long long)((N + k.size - 1) / k.size) * ((M + k.size - 1) / k.size);
+    if (k.tile == T128_DEEP && M <= 128 && (long long)N * K >= 40000000) continue;
+    const long long tiles = (long long)((N + k.size - 1) / k.size) * ((M + k.size - 1) / k.size), places = cus * k.to_a_cu;
     for (int p = 1; p <= 8 && (p == 1 || p * 2 <= steps); ++p) {
-      const long long blocks = tiles * p;
-      const double us = k.fixed + (double)((blocks + cus - 1) / cus) * (k.round + (steps + p - 1) / p * k.step) +
-                        k.block * (double)blocks / (double)cus + (double)p * M * N * 8 / 5e6;
+      const long long blocks = tiles * p, deep = (blocks + cus - 1) / cus;
+      const double share = (double)blocks / (double)cus;
+      const double rounds = k.to_a_cu == 1 ? (double)deep : blocks <= places ? 1. : share / k.to_a_cu + k.over;
+      const double step = k.step * (1. + k.beside * (double)(std::min<long long>(deep, k.to_a_cu) - 1)) + k.busy * std::min(1., share);
+      const double us = k.start + rounds * (k.round + (steps + p - 1) / p * step) + (k.sums * p + k.result) * M * N * 8 / 5e6;
       if (us < best.us) best = {k.tile, p, us, blocks};
     }
   }
@@ -589,9 +596,12 @@ static double full_in_rows(int M, int N, const TileChoice& c) {
 // this kernel's, a different W every call, with silu (the gelu and the clamped gate, whose kernels cost more: 1.08 times that), at 190 sizes
 // of up to 2,048 tokens (65 on, 5,632 to 55,296 rows, 1,600 to 5,120 columns) and with the larger tiles at 687 of up to 4,096:
 //   up to 1,536 columns 1.02 to 2 (65 to 8,192 tokens);
-//   up to 2,048 tokens by up to 4,096 columns, of tiles that are 0.72 and more full, 0.95 to 1.82, 1.2 on average, and up to 128 tokens by up to
-//     3,584 columns 0.99 to 1.53 (7B gate/up, 37,888 x 3,584: 128 tokens 1.34, 512 1.17, 1,024 1.30); tiles less full 0.88 to 1.45;
-//   192 to 2,048 tokens by up to 5,120 columns, tiles 0.8 and more full, 0.97 to 1.30; else 0.83 to 1.21;
+//   up to 2,048 tokens by up to 2,560 columns 0.94 to 1.8, 1.2 on average;
+//   by up to 3,584 columns up to 192 tokens 1.14 to 1.53; by up to 5,120 where the model expects 0.81
+//     PFLOP/s and more, or by up to 4,096 with tiles that are 0.72 full, 0.94 to 1.44, 1.11 on average (37,888 x 3,584 at 512 tokens 1.17, 900 1.23);
+//     not: tiles of 128 beyond 512 tokens at less than 0.92 PFLOP/s (0.84 to 1.0: what the library takes for 513 to 580 tokens is little more
+//     than for 512); beyond 1,024 tokens by more than 4,096 columns less full than 0.8 (0.95 to 1.12);
+//   in all 0.6 % behind the better way on average (250 sizes), 7 % by the tiles' fill alone;
 //   beyond, with the tiles counted in whole rows over the XCDs (as they lay when these were measured): up to 3,584 columns tiles of 192 or 160
 //     features, the others from 0.65 on, 0.92 to 1.60; 4,096 to 5,120 columns from 0.8 on 0.91 to 1.58;
 //   8,192 columns 0.96 to 1.03.
@@ -599,9 +609,14 @@ extern "C" int ms_gemm_tiled_pays(int M, int N, int K) {
   if (M <= 0 || N <= 0 || K <= 0 || K % BK) return 0;
   if (K <= 1536) return 1;
   if (K > 5120) return 0;
-  if (K <= 3584 && M <= 128) return 1;
+  if (M <= 2048 && (K <= 2560 || (K <= 3584 && M <= 192))) return 1;
   const TileChoice c = choose_tile(M, N, K);
-  if (M <= 2048) return full(M, N, c) >= (K <= 4096 ? 0.72 : 0.8) && M >= (K <= 4096 ? 1 : 192);
+  if (M <= 2048) {
+    const double rate = 2e-9 * M * N * K / c.us;       // PFLOP/s
+    if (c.tile == T128 && M > 512 && rate < 0.92) return 0;
+    if (K <= 4096) return rate >= 0.81 || full(M, N, c) >= 0.72;
+    return M <= 1024 ? rate >= 0.81 : full(M, N, c) >= 0.8;
+  }
   const double f = full_in_rows(M, N, c);
   if (K <= 3584) return c.tile == T192X256 || c.tile == T160X256 || f >= 0.65;
   return f >= 0.8;
@@ -665,13 +680,13 @@ extern "C" int ms_gemm_tiled(const void* A, long long lda, const void* W, long l
 //   up to 128 tokens 1.05 to 4.1, 1.6 on average;
 //   up to 256 tokens by 4,096 columns and more or up to 1,024 0.95 to 3.6, 1.5 on average;
 //   up to 512 tokens by more than 8,192 columns 1.0 to 3.1; by more than 4,096 in several parts, up to 5,120 features, 0.90 to 1.8,
-//     no more blocks than CUs, 1.13 on average; by up to 1,024 for up to 1,024 features 0.96 to 1.11.  Not: whole columns (4,480 x 6,784 at 429 tokens 0.82), more
+//     not two blocks of up to three parts a CU at less than 0.485 PFLOP/s, 1.13 on average; by up to 1,024 for up to 1,024 features 0.96 to 1.11.  Not: whole columns (4,480 x 6,784 at 429 tokens 0.82), more
 //     features (0.81 to 1.2), 4,096 columns (0.93 to 1.12), 1,024 and fewer for more features (0.87 to 1.0);
 //   up to 1,024 tokens by more than 8,192 columns, up to 5,120 features or by 16,384 columns and more, 0.92 to 3.2, 1.33 on average;
 //     else 0.88 to 2.0, 1.08 on average (8,192 columns 0.89 to 1.17);
 //   up to 1,000 tokens by 4,096 to 8,192 columns for up to 2,048 features, in three parts and more or, from 5,600 columns on, in two of
-//     the tiles of 128, 0.97 to 1.38, 1.1 on average (270 sizes with the norm; 896 x 4,864 by 640 and 768 tokens 24.4 -> 21.8 and 24.4 ->
-//     22.3 us).  Not: whole columns (0.81 to 0.83), two parts of fewer columns (0.95 to 1.06) or of tiles of 64 (0.95 to 1.02);
+//     the tiles of 128, 0.94 to 1.35, 1.08 on average (300 sizes with the norm; 896 x 4,864 by 640 and 768 tokens 24.3 -> 20.6 and 24.9 ->
+//     22.6 us).  Not: whole columns (0.81 to 0.83), two parts of fewer columns (0.95 to 1.06) or of tiles of 64 (0.95 to 1.02);
 //   in all 12 of 3,416 below 0.97;
 //   beyond, by 16,384 columns and more where one round of blocks in parts fills 5/6 of the CUs, but not all: 0.96 to 2.0, 1.4 on
 //     average (3,584 x 18,944 at 1,281 to 1,536 tokens and at 1,793 to 2,304).  With every CU taken 0.96 to 1.02 (4,096 x 28,672 at 2,048
@@ -685,7 +700,8 @@ extern "C" int ms_gemm_tiled_sums_parts(int M, int N, int K) {
                   : M <= 1024 ? K <= 8192 || (N > 5120 && K < 16384) : K < 16384)) return 0;   // (asked for twice a layer: before the choice)
   const SumsChoice c = choose_sums(M, N, K);
   const int cus = ms_compute_units();
-  if (M > 256 && M <= 512 && K > 4096 && K <= 8192 && (c.parts == 1 || c.blocks > cus)) return 0;
+  if (M > 256 && M <= 512 && K > 4096 && K <= 8192 &&
+      (c.parts == 1 || c.blocks > 2 * cus || (c.tile != T64_DEEP && c.blocks > cus && c.parts <= 3 && 2e-9 * M * N * K < 0.485 * c.us))) return 0;
   if (M > 512 && M <= 1024 && K <= 8192 && c.parts < 3 && (c.parts == 1 || K < 5600 || c.tile == T64 || c.tile == T64_DEEP)) return 0;
   if (M > 1024 && (c.tile != T256 || c.parts == 1 || c.blocks >= cus || c.blocks * 6 < cus * 5)) return 0;
   return c.parts;

@@ -771,8 +771,18 @@ def test_a_model_whose_weights_lie_anywhere_steps_as_one_whose_do_not(ops):
 
 @pytest.mark.parametrize("M,N,K,parts", [
     # times of the library and the norm over partial sums and the norm
-    (640, 896, 4864, 4), (768, 896, 4864, 4), (1000, 896, 4864, 4), (560, 512, 4864, 3), (960, 768, 6912, 5), (700, 2048, 8192, 2),    # 1.12 1.09 1.04 1.14 1.15 1.14
-    (560, 896, 4864, 0), (770, 1152, 4352, 0), (900, 1536, 4864, 0), (900, 512, 8192, 0),        # 0.99 0.81 0.98 0.98
+    (640, 896, 4864, 3), (768, 896, 4864, 3), (1000, 896, 4864, 4), (560, 512, 4864, 7), (960, 768, 6912, 5), (700, 2048, 8192, 2),    # 1.18 1.10 1.02 1.10 1.11 1.13
+    (900, 1536, 4864, 0), (700, 2048, 4352, 0),        # 0.98 0.97
+    # parts by the model of product and norm, times of other parts over them
+    (150, 3584, 18944, 4), (512, 3584, 18944, 8), (300, 5120, 27648, 2), (150, 2048, 5632, 5),       # 1.30 1.07 1.13 1.23
     (1001, 896, 4864, 0), (768, 896, 4096, 0), (768, 2176, 8192, 0)])                            # as ever
-def test_where_products_of_narrow_models_by_long_rows_leave_partial_sums(ops, M, N, K, parts):
+def test_where_products_leave_partial_sums_and_in_how_many_parts(ops, M, N, K, parts):
     assert ops._get("ms_gemm_tiled_sums_parts")(M, N, K) == parts
+
+
+@pytest.mark.parametrize("M,N,K,gated", [
+    # times of the library and the silu's kernel over the tiled kernel's
+    (900, 37888, 3584, 1), (150, 37888, 3584, 1), (200, 16384, 2048, 1), (850, 13824, 2560, 1), (900, 27648, 5120, 1),     # 1.23 1.16 1.30 1.13 1.15
+    (542, 37888, 3584, 0), (300, 55296, 5120, 0), (1300, 27648, 5120, 0)])                                                 # 0.86 0.84 0.95
+def test_where_the_tiled_kernel_takes_gated_products_by_what_it_is_expected_to_take(ops, M, N, K, gated):
+    assert ops._get("ms_gemm_tiled_pays")(M, N, K) == gated
