@@ -592,6 +592,67 @@ static double full_in_rows(int M, int N, const TileChoice& c) {
   return (double)M * N / ((double)((most + places - 1) / places) * places * 8 * c.features * c.tokens);
 }
 
+// Products whose result has to stay in 32 bits up to what reads it.  Where gate and up, or the addend of a norm, have been held in float by this
+// kernel, the library's product in its place would round them to bfloat16 first, which nobody asked for: so the sizes below, which the tiles
+// with two steps ahead (256, 192 or 160 features by 256 tokens, 128 x 128, 64 x 64) were given by their own measurements, stay here also where
+// the library is expected to be faster now.  Of 1.4 million sizes (65 to 8,192 tokens) that is 11 % of the gated ones, most of them by more than
+// 5,120 columns, 2 % of the squared relu's and 0.02 % of the sums'; time of the library and the next kernel over this one's at 125 of them, W in no
+// cache: 0.84 to 1.63, 1.05 on average, 0.67 to 1.30, 0.95, and 0.82 to 1.88, 1.05.
+static TileChoice choose_older(int M, int N, int K) {
+  const long long cus = ms_compute_units();
+  const double steps = (double)((K + BK - 1) / BK);
+  const long long small = (long long)((N + 127) / 128) * ((M + 127) / 128);
+  if (small < cus) return {T64, 64, 64, 0.0, (long long)((N + 63) / 64) * ((M + 63) / 64), 4 * cus};
+  TileChoice best{T128, 128, 128, ((double)small / (double)(2 * cus) + 0.3) * 1.15 * steps, small, (small + 2 * cus - 1) / (2 * cus) * 2 * cus};
+  const struct { int tile, features; double step_us; } wide[] = {{T256, 256, 1.60}, {T192X256, 192, 1.30}, {T160X256, 160, 1.30}};
+  for (const auto& w : wide) {
+    const long long tiles = (long long)((N + w.features - 1) / w.features) * ((M + 255) / 256), rounds = (tiles + cus - 1) / cus;
+    const double us = (double)rounds * (3.0 + steps * w.step_us);
+    if (us < best.us) best = {w.tile, w.features, 256, us, tiles, rounds * cus};
+  }
+  return best;
+}
+static bool rounds_full(int M, const TileChoice& older) { return older.tile != T64 && M <= 2048 && older.tiles * 10 >= older.slots * 9; }
+static bool gate_in_float(int M, int N, int K) {
+  const TileChoice c = choose_older(M, N, K);
+  if (c.tile == T64) return false;
+  if (rounds_full(M, c)) return true;
+  const double f = full_in_rows(M, N, c);
+  if (K <= 3584) return c.tile == T192X256 || c.tile == T160X256 || f >= 0.65 || (c.tile == T128 && f <= 0.4);
+  return K <= 5120 && M > 512 && f >= 0.8;
+}
+
+// Parts of a product in partial sums, by the same older tiles; 0: a bfloat16 addend, as ever.
+static SumsChoice choose_older_sums(int M, int N, int K) {
+  const long long cus = ms_compute_units();
+  const int steps = K / BK;
+  const struct { int tile, size, to_a_cu; double start_us[4], step_us[4]; } kinds[] = {
+      {T256, 256, 1, {12.}, {1.05}}, {T128, 128, 2, {9., 13.}, {0.55, 1.0}}, {T64, 64, 4, {7., 7., 7., 8.}, {0.30, 0.43, 0.63, 0.82}}};
+  SumsChoice best{0, 1, 1e30, 0};
+  for (const auto& k : kinds) {
+    const long long tiles = (long long)((N + k.size - 1) / k.size) * ((M + k.size - 1) / k.size), places = cus * k.to_a_cu;
+    for (int p = 1; p <= 8 && (p == 1 || p * 4 <= steps); ++p) {
+      const long long blocks = tiles * p;
+      const int at = (int)(blocks >= places ? k.to_a_cu : (blocks + cus - 1) / cus) - 1;
+      double rounds = (double)((blocks + places - 1) / places);
+      if (k.to_a_cu > 1 && rounds > 1) rounds = (double)blocks / (double)places + 0.3;
+      const double step = k.step_us[at] + (k.to_a_cu == 1 ? 0.5 * (double)(blocks < cus ? blocks : cus) / (double)cus : 0.);
+      const double us = rounds * (k.start_us[at] + (steps + p - 1) / p * step) + (double)p * M * N * 8 / 5e6;
+      if (us < best.us) best = {k.tile, p, us, blocks};
+    }
+  }
+  return best;
+}
+// (of sizes that ms_gemm_tiled_sums_parts considers)
+static int sums_in_float(int M, int N, int K) {
+  if (M > 512 && M <= 1024 && K <= 8192) return 0;
+  const SumsChoice c = choose_older_sums(M, N, K);
+  const int cus = ms_compute_units();
+  if (M > 256 && M <= 512 && K > 4096 && K <= 8192 && c.parts == 1) return 0;
+  if (M > 1024 && (c.tile != T256 || c.parts == 1 || c.blocks >= cus || c.blocks * 6 < cus * 5)) return 0;
+  return c.parts;
+}
+
 // Whether the gated product of M tokens is faster here than as the library's product and an activation kernel.  Time of these over
 // this kernel's, a different W every call, with silu (the gelu and the clamped gate, whose kernels cost more: 1.08 times that), at 190 sizes
 // of up to 2,048 tokens (65 on, 5,632 to 55,296 rows, 1,600 to 5,120 columns) and with the larger tiles at 687 of up to 4,096:
@@ -604,10 +665,10 @@ static double full_in_rows(int M, int N, const TileChoice& c) {
 //   in all 0.6 % behind the better way on average (250 sizes), 7 % by the tiles' fill alone;
 //   beyond, with the tiles counted in whole rows over the XCDs (as they lay when these were measured): up to 3,584 columns tiles of 192 or 160
 //     features, the others from 0.65 on, 0.92 to 1.60; 4,096 to 5,120 columns from 0.8 on 0.91 to 1.58;
-//   8,192 columns 0.96 to 1.03.
+//   8,192 columns 0.96 to 1.03, in this kernel only where gate and up have been held in float.
 extern "C" int ms_gemm_tiled_pays(int M, int N, int K) {
   if (M <= 0 || N <= 0 || K <= 0 || K % BK) return 0;
-  if (K <= 1536) return 1;
+  if (K <= 1536 || gate_in_float(M, N, K)) return 1;
   if (K > 5120) return 0;
   if (M <= 2048 && (K <= 2560 || (K <= 3584 && M <= 192))) return 1;
   const TileChoice c = choose_tile(M, N, K);
@@ -627,6 +688,7 @@ extern "C" int ms_gemm_tiled_pays(int M, int N, int K) {
 extern "C" int ms_gemm_tiled_relu2_pays(int M, int N, int K) {
   if (M <= 0 || N <= 0 || K <= 0 || K % BK) return 0;
   if (K <= 1536) return 1;
+  if (rounds_full(M, choose_older(M, N, K))) return 1;
   const TileChoice c = choose_tile(M, N, K);
   return M <= 2048 && c.tiles * 10 >= c.slots * 9 && (M > 512 || full(M, N, c) >= 0.9);
 }
@@ -700,11 +762,12 @@ extern "C" int ms_gemm_tiled_sums_parts(int M, int N, int K) {
                   : M <= 1024 ? K <= 8192 || (N > 5120 && K < 16384) : K < 16384)) return 0;   // (asked for twice a layer: before the choice)
   const SumsChoice c = choose_sums(M, N, K);
   const int cus = ms_compute_units();
-  if (M > 256 && M <= 512 && K > 4096 && K <= 8192 &&
-      (c.parts == 1 || c.blocks > 2 * cus || (c.tile != T64_DEEP && c.blocks > cus && c.parts <= 3 && 2e-9 * M * N * K < 0.485 * c.us))) return 0;
-  if (M > 512 && M <= 1024 && K <= 8192 && c.parts < 3 && (c.parts == 1 || K < 5600 || c.tile == T64 || c.tile == T64_DEEP)) return 0;
-  if (M > 1024 && (c.tile != T256 || c.parts == 1 || c.blocks >= cus || c.blocks * 6 < cus * 5)) return 0;
-  return c.parts;
+  const bool slower =
+      (M > 256 && M <= 512 && K > 4096 && K <= 8192 &&
+       (c.parts == 1 || c.blocks > 2 * cus || (c.tile != T64_DEEP && c.blocks > cus && c.parts <= 3 && 2e-9 * M * N * K < 0.485 * c.us))) ||
+      (M > 512 && M <= 1024 && K <= 8192 && c.parts < 3 && (c.parts == 1 || K < 5600 || c.tile == T64 || c.tile == T64_DEEP)) ||
+      (M > 1024 && (c.tile != T256 || c.parts == 1 || c.blocks >= cus || c.blocks * 6 < cus * 5));
+  return slower ? sums_in_float(M, N, K) : c.parts;
 }
 
 // Partial sums of the plain product over `parts` runs of the columns: float [parts, M, N].

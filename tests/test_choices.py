@@ -786,3 +786,15 @@ def test_where_products_leave_partial_sums_and_in_how_many_parts(ops, M, N, K, p
     (542, 37888, 3584, 0), (300, 55296, 5120, 0), (1300, 27648, 5120, 0)])                                                 # 0.86 0.84 0.95
 def test_where_the_tiled_kernel_takes_gated_products_by_what_it_is_expected_to_take(ops, M, N, K, gated):
     assert ops._get("ms_gemm_tiled_pays")(M, N, K) == gated
+
+
+@pytest.mark.parametrize("M,N,K,kind", [
+    (193, 37888, 3584, "gated"), (288, 37888, 3584, "gated"), (318, 37888, 3584, "gated"), (385, 37888, 3584, "gated"), (640, 22016, 4096, "gated"),
+    (1025, 55296, 5120, "gated"), (1092, 27648, 5120, "gated"), (2210, 2560, 2048, "gated"), (1031, 5632, 3072, "gated"), (2048, 57344, 8192, "gated"),
+    (415, 23560, 1600, "relu2"), (338, 23560, 2880, "relu2"), (464, 23560, 5120, "relu2"),
+    (387, 4608, 7168, "sums"), (506, 4778, 4352, "sums"), (450, 4480, 5120, "sums"), (1031, 1536, 16512, "sums"), (3727, 512, 16384, "sums")])
+def test_products_held_in_32_bits_up_to_their_reader_stay_so(ops, M, N, K, kind):
+    """Sizes whose gate and up, whose squared relu's input or whose norm's addend the tiled kernel holds in float, where the library, which rounds
+    them to bfloat16, is expected to be as fast or a little faster."""
+    rule = {"gated": "ms_gemm_tiled_pays", "relu2": "ms_gemm_tiled_relu2_pays", "sums": "ms_gemm_tiled_sums_parts"}[kind]
+    assert ops._get(rule)(M, N, K) > 0
