@@ -68,7 +68,7 @@ __device__ __forceinline__ float relu_squared(float z) { const float r = fmaxf(z
 //   EPI_RESIDUAL  out[M, N] += product (+ bias), float
 //   EPI_RELU2     out[M, N] = max(product (+ bias), 0)^2
 //   EPI_CLAMPED   as EPI_SWIGLU with the clamped gate; `bias` points at its two numbers, limit and alpha
-//   EPI_XIELU     out[M, N] = ms_xielu_value of the product; `bias` points at its two numbers (ms_gemm_quads alone has it)
+//   EPI_XIELU     out[M, N] = ms_xielu_value of the product; `bias` points at the learned p and q (ms_gemm_quads alone has it)
 enum { EPI_STORE = 0, EPI_SWIGLU = 1, EPI_RESIDUAL = 3, EPI_RELU2 = 5, EPI_CLAMPED = 6, EPI_XIELU = 9 };
 constexpr bool ms_gated(int epi) { return epi == EPI_SWIGLU || epi == EPI_CLAMPED; }
 template <int EPI> __device__ __forceinline__ float ms_gate_value(float g, float u, const float* __restrict__ numbers) {
@@ -76,7 +76,8 @@ template <int EPI> __device__ __forceinline__ float ms_gate_value(float g, float
 }
 template <int EPI> __device__ __forceinline__ float ms_store_value(float v) { return EPI == EPI_RELU2 ? relu_squared(v) : v; }
 
-// The xIELU activation with its two numbers worked out, softplus(p) and 1/2 + softplus(q).
+__device__ __forceinline__ float softplus_f(float x) { return x > 20.f ? x : log1pf(expf(x)); }
+// The xIELU activation with its two learned numbers worked out, ap = softplus(p) and an = 1/2 + softplus(q).
 __device__ __forceinline__ float ms_xielu_value(float z, float ap, float an) {
   return z > 0.f ? fmaf(ap * z, z, 0.5f * z) : fmaf(an, expm1f(z) - z, 0.5f * z);
 }

@@ -41,7 +41,7 @@ gemm_quads_kernel(const void* __restrict__ A, size_t lda, const bf16* __restrict
   const int nc = min(n0 + r, N - 1);
   const float pre = EPI == EPI_RESIDUAL ? reinterpret_cast<const float*>(out)[(size_t)min(m, M - 1) * ldo + nc] : 0.f;
   const float bv = bias && !ms_gated(EPI) && EPI != EPI_XIELU ? bias[nc] : 0.f;
-  const float numbers[2] = {EPI == EPI_XIELU ? bias[0] : 0.f, EPI == EPI_XIELU ? bias[1] : 0.f};
+  const float p = EPI == EPI_XIELU ? bias[0] : 0.f, q = EPI == EPI_XIELU ? bias[1] : 0.f;      // as they are at the time, as in ms_xielu
   product.run(wrow, x, norm_w);
 
   // rows 0 to 3 of a tile lie in lanes 0 to 15, one token to a lane
@@ -84,7 +84,7 @@ gemm_quads_kernel(const void* __restrict__ A, size_t lda, const bf16* __restrict
       v *= scale;
       asm("" : "+v"(v));   // rounded here, as in ms_gemm_skinny: not one operation with the bias
     }
-    if (lane < 4 * G && n0 + r < N) out[(size_t)m * ldo + n0 + r] = from_float<TO>(EPI == EPI_XIELU ? ms_xielu_value(v, numbers[0], numbers[1]) : ms_store_value<EPI>(v + bv + pre));
+    if (lane < 4 * G && n0 + r < N) out[(size_t)m * ldo + n0 + r] = from_float<TO>(EPI == EPI_XIELU ? ms_xielu_value(v, softplus_f(p), 0.5f + softplus_f(q)) : ms_store_value<EPI>(v + bv + pre));
   }
 }
 

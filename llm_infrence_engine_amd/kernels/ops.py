@@ -548,25 +548,20 @@ EPI_RELU2 = 5      # max(product (+ bias), 0)^2
 EPI_CLAMPED = 6    # as EPI_SWIGLU with the clamped gate: min(g, limit) sigmoid(alpha ..) (clamp(u, -limit, limit) + 1)
 
 
-EPI_XIELU = 9      # the xIELU activation of the product, with its two numbers as ``xielu_numbers`` gives them
+EPI_XIELU = 9      # the xIELU activation of the product, with its two learned numbers
 
 
-def xielu_numbers(pq: torch.Tensor) -> torch.Tensor:
-    """softplus(p) and 1/2 + softplus(q) of an xIELU's learned numbers, for ``gemm_xielu``."""
-    return torch.nn.functional.softplus(pq.float()) + torch.tensor([0.0, 0.5], device=pq.device)
-
-
-def gemm_xielu(a: torch.Tensor, w: torch.Tensor, numbers: torch.Tensor) -> Optional[torch.Tensor]:
-    """xielu(a [M <= 8, K] @ w [N, K].T) in bfloat16, None where the kernel of narrow matrices, which has the activation as an
+def gemm_xielu(a: torch.Tensor, w: torch.Tensor, pq: torch.Tensor) -> Optional[torch.Tensor]:
+    """xielu(a [M <= 8, K] @ w [N, K].T) in bfloat16 with pq = (p, q) as ``xielu`` has them, None where the kernel of narrow matrices, which has the activation as an
     epilogue, is not the one for the product."""
     if a.shape[0] > 8 or not skinny_ok(a, w):
         return None
     _check(a, "a", torch.bfloat16, contiguous=False)
     (M, K), N = a.shape, w.shape[0]
     _check(w, "w", torch.bfloat16, (N, K))
-    _check(numbers, "numbers", torch.float32, (2,))
+    _check(pq, "pq", torch.float32, (2,))
     out = torch.empty((M, N), dtype=torch.bfloat16, device=a.device)
-    rc = _get("ms_gemm_quads")(a.data_ptr(), a.stride(0) if M > 1 else K, None, None, 0.0, w.data_ptr(), K, numbers.data_ptr(), out.data_ptr(),
+    rc = _get("ms_gemm_quads")(a.data_ptr(), a.stride(0) if M > 1 else K, None, None, 0.0, w.data_ptr(), K, pq.data_ptr(), out.data_ptr(),
                                N, M, N, K, EPI_XIELU, BF16, 0, _stream())
     if rc == 2:
         return None

@@ -56,14 +56,13 @@ class DenseAct(FeedForward):
         self.rt = rt
         up, down, *act = (get(s) for s in self.tensor_specs())
         self.w_up, self.w_down, self.act = linear.prepare_weight(up), linear.prepare_weight(down), (act[0] if act else None)
-        self.numbers = ops.xielu_numbers(self.act) if act else None
 
     def forward(self, h, ctx):
         return self.forward_residual(h, ctx, None)
 
     def forward_residual(self, h, ctx, x):
         u = linear.linear_act(h, self.w_up, ops.EPI_RELU2) if self.activation == "relu2" else \
-            ops.gemm_xielu(h, self.w_up, self.numbers) if self.activation == "xielu" else None
+            ops.gemm_xielu(h, self.w_up, self.act) if self.activation == "xielu" else None
         if u is not None:
             return linear.linear_residual(u, self.w_down, None, x)
         u = linear.linear(h, self.w_up)

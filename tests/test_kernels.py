@@ -2434,12 +2434,37 @@ def test_gemm_xielu(ops, M, N, K):
     a = torch.randn(M, K, generator=g, device=DEV).bfloat16()
     w = (torch.randn(N, K, generator=g, device=DEV) * 2 / math.sqrt(K)).bfloat16()
     pq = torch.tensor([0.3, -0.4], device=DEV)
-    got = ops.gemm_xielu(a, w, ops.xielu_numbers(pq))
+    got = ops.gemm_xielu(a, w, pq)
     z = a.double() @ w.double().T
     p, q = torch.nn.functional.softplus(pq.double())
     want = torch.where(z > 0, p * z * z + z / 2, (0.5 + q) * (torch.expm1(z.clamp(max=0)) - z) + z / 2)
     torch.testing.assert_close(got.double(), want, atol=2e-3, rtol=5e-3)     # one rounding to bfloat16; the product's float error
     assert ops.gemm_xielu(torch.zeros(9, K, device=DEV, dtype=torch.bfloat16), w, pq) is None
+
+
+@pytest.mark.parametrize("change", ["in place", "another tensor"])
+def test_an_xielu_whose_numbers_change_is_the_new_one_for_any_number_of_tokens(ops, change):
+    """4 tokens, whose product has the activation as its epilogue, and 16, whose activation is a kernel of its own, before and after."""
+    from llm_infrence_engine_amd.parts.base import Runtime
+    from llm_infrence_engine_amd.parts.feed_forward import DenseAct
+
+    g = torch.Generator(device=DEV).manual_seed(3)
+    tensors = {"up": torch.randn(512, 512, generator=g, device=DEV).bfloat16() / 22, "down": torch.eye(512, device=DEV).bfloat16(),
+               "act": torch.tensor([0.3, -0.4], device=DEV)}
+    part = DenseAct("", 512, 512)
+    part.load(lambda spec: tensors[spec.name], Runtime(torch.device(DEV), torch.bfloat16))
+    h = torch.randn(16, 512, generator=g, device=DEV).bfloat16()
+    for p, q in ((0.3, -0.4), (1.5, 0.8)):
+        if p == 1.5 and change == "in place":
+            part.act.copy_(torch.tensor([p, q]))
+        elif p == 1.5:
+            part.act = torch.tensor([p, q], device=DEV)
+        z = h.double() @ tensors["up"].double().T
+        ap, an = torch.nn.functional.softplus(torch.tensor([p, q], dtype=torch.float64)) + torch.tensor([0.0, 0.5])
+        want = torch.where(z > 0, ap * z * z + z / 2, an * (torch.expm1(z.clamp(max=0)) - z) + z / 2)
+        for rows in (4, 16):      # roundings to bfloat16: of the product for 16 rows, by the slope of at most 2 ap |z| + an + 1/2, and of the result
+            got = part.forward(h[:rows], None).double()
+            assert ((got - want[:rows]).abs() <= 2 ** -8 * 1.02 * ((2 * ap * z.abs() + an + 0.5) * z.abs() + want.abs())[:rows] + 1e-5).all()
 
 
 @pytest.mark.parametrize("M,N,K", [(17, 41024, 64), (64, 41000, 192), (33, 50001, 896), (40, 41030, 1984)])
