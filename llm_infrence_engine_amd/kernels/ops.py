@@ -336,6 +336,13 @@ def rms_norm_pair(x: torch.Tensor, w1: torch.Tensor, w2: torch.Tensor, eps: floa
     return out1, out2
 
 
+def rms_norm_pair_conv_ok(x: torch.Tensor, w1: torch.Tensor, w2: torch.Tensor, taps: torch.Tensor, state: torch.Tensor, dtype) -> bool:
+    """Whether ``rms_norm_pair_conv`` takes these, with results of type ``dtype``: rows of four values on as many places."""
+    H, n = x.shape[1], taps.shape[1]
+    return (dtype == state.dtype == torch.bfloat16 and H % 4 == 0 and H <= 2048 and n <= MAX_CONV_TAPS and state.data_ptr() % 8 == 0
+            and (x.data_ptr() | w1.data_ptr() | w2.data_ptr() | taps.data_ptr()) % 16 == 0)
+
+
 def rms_norm_pair_conv(x: torch.Tensor, w1: torch.Tensor, w2: torch.Tensor, eps: float, taps: torch.Tensor, state: torch.Tensor, ctx,
                        out1: torch.Tensor, out2: torch.Tensor, delta: Optional[torch.Tensor] = None):
     """``rms_norm_pair`` and, of out1's rows h, ``short_conv`` with CONV_ADD_INPUT (h + the convolution, the state moved on) in one

@@ -74,7 +74,8 @@ class RMSNorm(Norm):
         """``forward_pair`` with the first result h as h + its convolution over time, for a step of single tokens (``weight`` and
         ``state`` of a short convolution that adds its input); None where that is not one kernel."""
         if (not isinstance(other, RMSNorm) or other.size != self.size or other.eps != self.eps or getattr(ctx, "max_q_len", 0) != 1
-                or self.size % 4 or self.size > 2048 or self.rt.dtype != torch.bfloat16 or (delta is not None and delta.dim() != 2)):
+                or (delta is not None and delta.dim() != 2)
+                or not ops.rms_norm_pair_conv_ok(x, self.weight, other.weight, weight, state, self.rt.dtype)):
             return None
         n = x.shape[0]
         return ops.rms_norm_pair_conv(x, self.weight, other.weight, self.eps, weight, state, ctx, self.rt.empty(n, self.size),

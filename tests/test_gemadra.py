@@ -694,3 +694,38 @@ def test_command_line_generates(shape):
     r = subprocess.run([sys.executable, "-m", "llm_infrence_engine_amd", "--model", str(folder), "--dtype", "float32",
                         "--prompt-ids", "5,17,3", "--max-new-tokens", "4"], cwd=ROOT, capture_output=True, text=True, timeout=300)
     assert r.returncode == 0, r.stderr[-2000:]
+
+
+def _decoded(shape, change):
+    """Logits of two decode steps of three requests in bfloat16, step by step, after ``change`` of the loaded model's layers."""
+    from llm_infrence_engine_amd.engine.batch import StepEntry
+    from llm_infrence_engine_amd.engine.runner import load_runner
+
+    name, cfg, folder, reqs, want, noise = shape
+    runner = load_runner(folder, dtype="bfloat16", page_size=PAGES[name], num_pages=64, max_requests=4, max_len=128)
+    for l in runner.model.layers:
+        change(l)
+    rids = list(reqs)[:3]
+    runner.step([StepEntry(r, reqs[r][:n], [0]) for r, n in zip(rids, (3, 1, 2))])
+    out = []
+    for t in range(2):
+        out.append(runner.step([StepEntry(r, [7 * i + t], [0]) for i, r in enumerate(rids)]).cpu())
+    return torch.stack(out)
+
+
+def _aside(part, names, offset):
+    for n in names:
+        w = getattr(part, n, None)
+        if w is not None:
+            there = torch.empty(w.numel() + offset, dtype=w.dtype, device=w.device)[offset:].view(w.shape)
+            assert there.copy_(w).data_ptr() % 16
+            setattr(part, n, there)
+
+
+@gpu
+@pytest.mark.parametrize("part,names", [("mixer_norm", ["weight"]), ("feed_forward_norm", ["weight"]), ("input_filter", ["weight"])])
+def test_decoding_with_norms_and_convolutions_at_any_place(shape, part, names):
+    """Scales and taps 4 bytes off 16, as a reader of weights may hand them out: the norms and the convolution one after the other, to the
+    same bits."""
+    moved = _decoded(shape, lambda l: getattr(l, part) is not None and _aside(getattr(l, part), names, 1))
+    assert torch.equal(moved, _decoded(shape, lambda l: None))
