@@ -357,6 +357,8 @@ def rms_norm_pair_conv(x: torch.Tensor, w1: torch.Tensor, w2: torch.Tensor, eps:
     _check(state, "state", out1.dtype, (None, max(1, taps.shape[1] - 1), H))
     _check(ctx.token_req, "token_req", torch.int32, (N,))
     _check(ctx.state_slots, "state_slots", torch.int32, (ctx.num_requests,))
+    if getattr(ctx, "max_q_len", 0) != 1:
+        raise ValueError("every request of the step must have one token")
     dcode = 0
     if delta is not None:
         _check(delta, "delta", None, (N, H))

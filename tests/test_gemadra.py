@@ -729,3 +729,14 @@ def test_decoding_with_norms_and_convolutions_at_any_place(shape, part, names):
     same bits."""
     moved = _decoded(shape, lambda l: getattr(l, part) is not None and _aside(getattr(l, part), names, 1))
     assert torch.equal(moved, _decoded(shape, lambda l: None))
+
+
+def test_a_norm_pair_with_a_convolution_is_for_steps_of_single_tokens(monkeypatch):
+    """One block a token moves its request's state on: two tokens of a request in one step are refused before the launch."""
+    from llm_infrence_engine_amd.kernels import ops
+
+    monkeypatch.setattr(ops, "_check", lambda *a, **k: None)
+    monkeypatch.setattr(ops, "_call", lambda *a: pytest.fail("launched"))
+    x, w, h = torch.zeros(3, 8), torch.ones(8), torch.zeros(3, 8, dtype=torch.bfloat16)
+    with pytest.raises(ValueError, match="one token"):
+        ops.rms_norm_pair_conv(x, w, w, 1e-6, torch.zeros(8, 2), torch.zeros(4, 1, 8, dtype=torch.bfloat16), _Ctx([2, 1], [0, 1], dev="cpu"), h, h)
