@@ -1547,7 +1547,8 @@ def gated_delta(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, a: torch.Tens
 
 def gated_delta_step_ok(proj: torch.Tensor, w_a2: torch.Tensor, w_g2: torch.Tensor, dim: int, vdim: int) -> bool:
     """Whether ``gated_delta_step`` takes these."""
-    return (proj.dtype == w_a2.dtype == w_g2.dtype == torch.bfloat16 and w_a2.data_ptr() % 16 == 0 and w_g2.data_ptr() % 16 == 0
+    return (proj.dtype == w_a2.dtype == w_g2.dtype == torch.bfloat16 and w_a2.is_contiguous() and w_g2.is_contiguous()
+            and w_a2.data_ptr() % 16 == 0 and w_g2.data_ptr() % 16 == 0
             and bool(_get("ms_gated_delta_step_takes")(dim, vdim, w_a2.shape[1], w_g2.shape[1])))
 
 

@@ -731,6 +731,27 @@ def test_decoding_with_norms_and_convolutions_at_any_place(shape, part, names):
     assert torch.equal(moved, _decoded(shape, lambda l: None))
 
 
+@gpu
+@pytest.mark.parametrize("strided", [False, True])
+def test_decoding_with_low_rank_maps_at_any_place(shape, strided):
+    """The second matrices of the decay's and the gate's low-rank maps off 16 bytes, or as columns of a wider matrix, which the products
+    have a kernel for: the parts of the delta rule's step one by one.  They round the gate's input, the whole step does not."""
+    def change(l):
+        if not hasattr(l.mixer, "w_g2"):
+            return
+        for n in ("w_a", "w_g2"):
+            w = getattr(l.mixer, n)
+            if strided:
+                setattr(l.mixer, n, torch.cat([w, w], dim=1)[:, :w.shape[1]])
+                assert not getattr(l.mixer, n).is_contiguous()
+            else:
+                _aside(l.mixer, [n], 1)
+
+    name, cfg, folder, reqs, want, noise = shape
+    moved, usual = _decoded(shape, change), _decoded(shape, lambda l: None)
+    assert (moved - usual).abs().max() < BF16_NOISE * max(max(noise.values()), 0.02)
+
+
 def test_a_norm_pair_with_a_convolution_is_for_steps_of_single_tokens(monkeypatch):
     """One block a token moves its request's state on: two tokens of a request in one step are refused before the launch."""
     from llm_infrence_engine_amd.kernels import ops
