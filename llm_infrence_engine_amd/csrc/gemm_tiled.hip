@@ -324,7 +324,7 @@ gemm_tiled_kernel(const bf16* __restrict__ A, size_t lda, const bf16* __restrict
   }
   auto last_steps = [&](auto self, auto left_c) -> void {
     constexpr int LEFT = decltype(left_c)::value;
-    if (steps - at > LEFT) {      // (fewer steps than slots: the pipeline never fills)
+    if (LEFT == 0 || steps - at > LEFT) {      // (fewer steps than slots: the pipeline never fills; the last one there always is)
       step(left_c, at, sw, after_w(sw), before_w(sw), sa, after_a(sa));
       sw = after_w(sw);
       sa = after_a(sa);
