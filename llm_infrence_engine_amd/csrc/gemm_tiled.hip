@@ -524,19 +524,42 @@ constexpr TileKind KINDS[] = {{T256, 256, 256, 1, 0.06, 5.93, 0.98, 0.52},     {
                               {T128X256, 128, 256, 1, 1.04, 3.31, 0.58, 0.31}, {T96X128, 96, 128, 1, 1.58, 2.21, 0.32, 0.16},
                               {T64X128, 64, 128, 1, 1.62, 1.64, 0.25, 0.13}};
 
+struct TileChoice { int tile, features, tokens; double us; long long tiles, slots; };
+
+// Of the tiles with two steps ahead alone, by what they were measured to take (a start and end of 3 us and a step by its tile, rounds over the CUs).
+TileChoice choose_older(int M, int N, int K) {
+  const long long cus = ms_compute_units();
+  const double steps = (double)((K + BK - 1) / BK);
+  const long long small = (long long)((N + 127) / 128) * ((M + 127) / 128);
+  if (small < cus) return {T64, 64, 64, 0.0, (long long)((N + 63) / 64) * ((M + 63) / 64), 4 * cus};
+  TileChoice best{T128, 128, 128, ((double)small / (double)(2 * cus) + 0.3) * 1.15 * steps, small, (small + 2 * cus - 1) / (2 * cus) * 2 * cus};
+  const struct { int tile, features; double step_us; } wide[] = {{T256, 256, 1.60}, {T192X256, 192, 1.30}, {T160X256, 160, 1.30}};
+  for (const auto& w : wide) {
+    const long long tiles = (long long)((N + w.features - 1) / w.features) * ((M + 255) / 256), rounds = (tiles + cus - 1) / cus;
+    const double us = (double)rounds * (3.0 + steps * w.step_us);
+    if (us < best.us) best = {w.tile, w.features, 256, us, tiles, rounds * cus};
+  }
+  return best;
+}
+
 // The tile that takes the least time by a model of the measurements: 200 sizes (65 to 4,096 tokens, 1,152 to 37,888 features,
 // 256 to 3,584 columns), every tile timed at each, every product by a W that lies in no cache.  Its times lie within 0.77 and 1.28 of the measured
 // ones (tiles with a CU to themselves 0.81 to 1.14), and the tile it takes is 0.4 % behind the best one on average, 12 % at worst; with 1 to 5 alone
 // the best is 9 % behind on average and up to 42 (0.5B gate/up, 9,728 x 896: 128 tokens 11.1 -> 9.3 us, 256 13.9 -> 10.9, 512 18.4 -> 13.6, 768 17.7 ->
 // 16.3, from 1,024 on the same; 5,632 x 2,048 at 256 tokens 20.8 -> 15.8, 37,888 x 3,584 at 128 80 -> 56).
-struct TileChoice { int tile, features, tokens; double us; long long tiles, slots; };
-
 TileChoice choose_tile(int M, int N, int K) {
+  // What the model was measured at ends here.  Taken there all the same it was 0.71 to 1.13 times as fast as those below up to 192 columns and 0.62 to 1.2
+  // beyond 4,096 tokens (146 sizes): 12,558 x 128 at 1,188 tokens 23.9 and 28.5 us, 980 x 128 at 10,455 15.4 and 22.4.
+  if (K < 256 || M >= 6144) return choose_older(M, N, K);
   const long long cus = ms_compute_units();
   const double steps = (double)((K + BK - 1) / BK);
+  const int xm = choose_xcd_split(M);
   TileChoice best{0, 0, 0, 1e30, 0, 0};
   for (const TileKind& k : KINDS) {
-    const long long tiles = (long long)((N + k.features - 1) / k.features) * ((M + k.tokens - 1) / k.tokens), rounds = (tiles + cus - 1) / cus;
+    const long long n_tiles = (N + k.features - 1) / k.features, m_tiles = (M + k.tokens - 1) / k.tokens;
+    // (laid over the XCDs in whole rows, as many as the XCD with the most has, eight times: 512 x 768 at 4,926 tokens took 96 x 128, 15.2 us, and
+    // takes 128 x 128, 9.5; 26 sizes from 4,096 tokens on 0.94 -> 1.10 times as fast as by choose_older)
+    const long long tiles = xm == 1 ? n_tiles * m_tiles : 8 * ((n_tiles + 8 / xm - 1) / (8 / xm)) * ((m_tiles + xm - 1) / xm), rounds = (tiles + cus - 1) / cus;
     if (k.tile == T64 ? tiles <= 2 * cus : k.tile == T64_DEEP && tiles > 2 * cus) continue;      // (two of the deep ones share a CU)
     const double share = (double)tiles / (double)cus;
     const double us = k.fixed + (double)rounds * (k.round + steps * k.step) + steps * k.busy * (k.to_a_cu == 1 ? share : std::min(1.0, share));
@@ -580,6 +603,7 @@ SumsChoice choose_sums(int M, int N, int K) {
 }  // namespace
 
 extern "C" void ms_gemm_tiled_force(int tile) { g_tile = tile; }
+extern "C" int ms_gemm_tiled_tile(int M, int N, int K) { return choose_tile(M, N, K).tile; }
 extern "C" void ms_gemm_tiled_force_xcd_split(int xm) { g_xcd_split = xm; }
 
 // What of the tiles' places the product fills: tiles in whole rounds over the CUs.
@@ -598,20 +622,6 @@ static double full_in_rows(int M, int N, const TileChoice& c) {
 // the library is expected to be faster now.  Of 1.4 million sizes (65 to 8,192 tokens) that is 11 % of the gated ones, most of them by more than
 // 5,120 columns, 2 % of the squared relu's and 0.02 % of the sums'; time of the library and the next kernel over this one's at 125 of them, W in no
 // cache: 0.84 to 1.63, 1.05 on average, 0.67 to 1.30, 0.95, and 0.82 to 1.88, 1.05.
-static TileChoice choose_older(int M, int N, int K) {
-  const long long cus = ms_compute_units();
-  const double steps = (double)((K + BK - 1) / BK);
-  const long long small = (long long)((N + 127) / 128) * ((M + 127) / 128);
-  if (small < cus) return {T64, 64, 64, 0.0, (long long)((N + 63) / 64) * ((M + 63) / 64), 4 * cus};
-  TileChoice best{T128, 128, 128, ((double)small / (double)(2 * cus) + 0.3) * 1.15 * steps, small, (small + 2 * cus - 1) / (2 * cus) * 2 * cus};
-  const struct { int tile, features; double step_us; } wide[] = {{T256, 256, 1.60}, {T192X256, 192, 1.30}, {T160X256, 160, 1.30}};
-  for (const auto& w : wide) {
-    const long long tiles = (long long)((N + w.features - 1) / w.features) * ((M + 255) / 256), rounds = (tiles + cus - 1) / cus;
-    const double us = (double)rounds * (3.0 + steps * w.step_us);
-    if (us < best.us) best = {w.tile, w.features, 256, us, tiles, rounds * cus};
-  }
-  return best;
-}
 static bool rounds_full(int M, const TileChoice& older) { return older.tile != T64 && M <= 2048 && older.tiles * 10 >= older.slots * 9; }
 static bool gate_in_float(int M, int N, int K) {
   const TileChoice c = choose_older(M, N, K);

@@ -798,3 +798,16 @@ def test_products_held_in_32_bits_up_to_their_reader_stay_so(ops, M, N, K, kind)
     them to bfloat16, is expected to be as fast or a little faster."""
     rule = {"gated": "ms_gemm_tiled_pays", "relu2": "ms_gemm_tiled_relu2_pays", "sums": "ms_gemm_tiled_sums_parts"}[kind]
     assert ops._get(rule)(M, N, K) > 0
+
+
+@pytest.mark.parametrize("M,N,K,tile", [
+    # us of the tiles of 256 x 256, 128 x 128, 64 x 64, 192 and 160 x 256, 64 x 64 deep, 96 x 128
+    (4926, 512, 768, 2), (5069, 472, 768, 2), (4402, 460, 1280, 2),         # 19.3 9.5 9.6 16.2 15.7 12.2 15.2;  23.9 10.7 10.9 .. 15.2;  35.0 15.7 15.7 .. 21.1
+    (5370, 1496, 1536, 2),                                                  # as 128 x 256 46.5, as 192 x 256 29.7
+    (10455, 980, 128, 2), (8403, 1906, 768, 2), (1188, 12558, 128, 2),      # 21.7 15.4 15.9 22.2 13.2;  62.3 45.6 49.6 47.0 39.7;  28.8 21.0 21.1 27.5 21.2
+    (13607, 4864, 1024, 4), (352, 2000, 128, 3),                            # 133 150 276 131 142;  .. 3.99 3.22 .. 3.36
+    # the measured range of the model
+    (300, 9728, 896, 2), (512, 9728, 896, 7), (2048, 9728, 896, 5), (157, 224, 1280, 6), (4096, 9728, 896, 1), (4096, 37888, 3584, 1)])
+def test_tiles_by_the_model_within_what_it_was_measured_at(ops, M, N, K, tile):
+    """Beyond 6,143 tokens and below 256 columns the choice is the older tiles'; from 4,096 tokens on rounds are counted as the tiles lie."""
+    assert ops._get("ms_gemm_tiled_tile")(M, N, K) == tile
