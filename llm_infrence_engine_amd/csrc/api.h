@@ -123,6 +123,7 @@ int ms_gemm_tiled_plain_pays(int M, int N, int K);   // the same question for a 
 // The q/k/v product of many tokens with bias, rotation (whole heads, pairs (j, j + d/2)) and the store of k and v
 // into the cache pages as its epilogue: A [M, lda] bfloat16, W [(nh + 2 nkv) d, ldw], q_out [M, nh d] bfloat16;
 // head_dim 64 or 128; rope_table float [M, d / 2, 2] from ms_rope_table.  Pages as in ms_rope_store.  ms_gemm_tiled_qkv_pays: where it beats product + rotation kernel.
+int ms_gemm_tiled_qkv_tile(int M, int K, int heads, int head_dim);   // the tile that it takes by itself
 int ms_gemm_tiled_qkv(const void* A, long long lda, const void* W, long long ldw, const float* bias,
                       const float* rope_table, const int* slot_mapping, void* q_out, void* k_pages, void* v_pages, int M,
                       int K, int nh, int nkv, int head_dim, int page_size, int v_transposed, hipStream_t stream);

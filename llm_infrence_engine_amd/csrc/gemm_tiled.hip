@@ -859,6 +859,20 @@ extern "C" int ms_gemm_tiled_qkv_pays(int M, int N, int K, int head_dim) {
   return M > 0 && N > 0 && K > 0 && K % BK == 0 && K <= 1024 && N <= 2048 && (head_dim == 64 || head_dim == 128);
 }
 
+// A wave's features are a head.  As long as a tile of 64 tokens (then of 128) to every head is not more than a CU's worth, these with as many slots
+// as LDS holds; then tiles that share a CU.  Heads of 64 (18 of them by 896, us of the tiles of 64 | the taken one): 512 tokens 10.3 | 8.9, 1,024
+// 11.5 | 10.7, 1,536 12.6 | 10.9, 2,048 19.7 in a second round, 15.3 in tiles of 64.  Of many tiles of 64 a CU those of 128 x 128 have less to read:
+// from 8 on by more than 960 columns and from 14 on by 768 and more 0.76 to 1.02 of the time (32 heads by 1,024 at 8,192 tokens 62 us, 79 in tiles of 64;
+// 18 by 896 at 16,384 78 and 84); below 0.95 to 2.2 (8 heads to 32, 1,024 to 16,384 tokens, 128 to 1,024 columns), by 512 columns 1.06 to 2.1.
+// Heads of 128 (12 by 1,024; 256 features by 128 tokens before; with 256 tokens the epilogue does not fit the registers): 100 to 1,024 tokens 32
+// to 34 | 16, 2,048 35 | 24, 4,096 36.
+extern "C" int ms_gemm_tiled_qkv_tile(int M, int K, int heads, int head_dim) {
+  const long long cus = ms_compute_units(), of_64 = (long long)heads * ((M + 63) / 64);
+  if (of_64 <= cus) return T64_DEEP;
+  if ((long long)heads * ((M + 127) / 128) <= cus) return T64X128;
+  return head_dim == 64 && (K <= 960 ? K < 768 || of_64 < 14 * cus : of_64 < 8 * cus) ? T64 : T128;
+}
+
 extern "C" int ms_gemm_tiled_qkv(const void* A, long long lda, const void* W, long long ldw, const float* bias,
                                  const float* rope_table, const int* slot_mapping, void* q_out,
                                  void* k_pages, void* v_pages, int M, int K, int nh, int nkv, int head_dim, int page_size,
@@ -877,14 +891,8 @@ extern "C" int ms_gemm_tiled_qkv(const void* A, long long lda, const void* W, lo
   bf16* o = (bf16*)q_out;
   const size_t ldo = (size_t)nh * head_dim;
 #define GO(WF, WT, FT, TT, SW, SA) return launch<WF, WT, FT, TT, SW, SA, EPI_QKV, bf16>(a, lda, w, ldw, o, ldo, M, N, K, stream, e)
-  // A wave's features are a head.  As long as a tile of 64 tokens (then of 128) to every head is not more than a CU's worth, these with
-  // as many slots as LDS holds; then tiles that share a CU.  Heads of 64 (18 of them by 896, us of the tiles of 64 | the taken one; the
-  // epilogue's inputs asked for early have taken 1 from either): 512 tokens 10.3 | 8.9, 1,024 11.5 | 10.7, 1,536 12.6 | 10.9, 2,048 19.7 in a second round, 15.3 in tiles of
-  // 64, 4,096 24.9 of 128 and 24.5 of 64.  Heads of 128 (12 by 1,024; 256 features by 128 tokens before; with 256 tokens the epilogue does not fit the
-  // registers): 100 to 1,024 tokens 32 to 34 | 16, 2,048 35 | 24, 4,096 36.
-  const long long cus = ms_compute_units(), heads = nh + 2 * nkv;
   int tile = g_tile;
-  if (tile == 0) tile = heads * ((M + 63) / 64) <= cus ? T64_DEEP : heads * ((M + 127) / 128) <= cus ? T64X128 : T64;
+  if (tile == 0) tile = ms_gemm_tiled_qkv_tile(M, K, nh + 2 * nkv, head_dim);
   if (head_dim == 128) {
     if (tile == T64_DEEP) GO(1, 4, 8, 1, 5, 4);
     if (tile == T64X128) GO(1, 8, 8, 1, 3, 3);

@@ -811,3 +811,12 @@ def test_products_held_in_32_bits_up_to_their_reader_stay_so(ops, M, N, K, kind)
 def test_tiles_by_the_model_within_what_it_was_measured_at(ops, M, N, K, tile):
     """Beyond 6,143 tokens and below 256 columns the choice is the older tiles'; from 4,096 tokens on rounds are counted as the tiles lie."""
     assert ops._get("ms_gemm_tiled_tile")(M, N, K) == tile
+
+
+@pytest.mark.parametrize("M,K,heads,d,tile", [
+    # time in tiles of 128 x 128 over that in tiles of 64 x 64
+    (4096, 896, 18, 64, 3), (8192, 512, 32, 64, 3), (4000, 1024, 32, 64, 3), (11000, 896, 18, 64, 3),            # 1.0 1.1 0.95 1.05
+    (8192, 1024, 32, 64, 2), (4096, 1024, 32, 64, 2), (16384, 896, 18, 64, 2), (8192, 768, 32, 64, 2),           # 0.79 0.95 0.92 0.97
+    (896, 896, 18, 64, 6), (1024, 896, 18, 64, 11), (1800, 1024, 14, 64, 11), (70, 512, 12, 128, 6), (4096, 1024, 12, 128, 2)])
+def test_tiles_of_the_qkv_product(ops, M, K, heads, d, tile):
+    assert ops._get("ms_gemm_tiled_qkv_tile")(M, K, heads, d) == tile
