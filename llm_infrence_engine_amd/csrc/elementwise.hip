@@ -107,13 +107,19 @@ extern "C" int ms_rms_norm(float* x, const void* delta, int delta_dtype, int n_p
   if (delta && (n_partials < 1 || partial_stride < 0)) return MS_BAD_ARG;
   if (hidden <= 0) return MS_BAD_ARG;
   dim3 grid(n_rows), block(hidden >= 1024 ? 256 : 128);
-  // bfloat16 results: a thread for every four values where that is no more threads than the chip takes at once, one round of loads instead of
-  // two and more (512 rows of 896 with four partial sums 4.15 -> 3.93 us, 64 of 3,584 4.77 -> 4.13, 512 6.3 -> 5.9, 1,024 of 896 4.6 -> 4.5; with 1,024 rows
-  // of 3,584 8.0 either way, 2,048 of 896 5.7 and 5.9).  (32-bit rows keep one order of sums, whatever their number.)
   const size_t out_quad = dtype == MS_BF16 ? 8 : 16, delta_quad = dtype == MS_BF16 && delta_dtype == MS_BF16 ? 8 : 16;
   const int quads = hidden % 4 == 0 && ((uintptr_t)x | (uintptr_t)weight) % 16 == 0 && (uintptr_t)out % out_quad == 0 &&
                     (!delta || ((uintptr_t)delta % delta_quad == 0 && (n_partials == 1 || partial_stride % 4 == 0)));
-  if (dtype == MS_BF16 && quads && (n_rows <= 512 || (n_rows <= 1024 && hidden <= 1024))) block = dim3(std::min(448, (hidden / 4 + 63) / 64 * 64));
+  // Several sums to add up and a CU for every row: a thread for every four values, one round of loads (64 rows of 2,048 with two sums 3.8 us with 448
+  // threads, 3.2 so; of 8,192 5.9 and 4.8).  Else, for bfloat16 results and no more threads than the chip takes at once, 448 threads where these save a
+  // round (512 rows of 896 with four sums 4.15 -> 3.93 us, 64 of 3,584 with one 4.5 -> 3.8, 512 6.8 -> 6.1, 200 of 8,192 8.7 -> 7.2; 2,048 values are two
+  // rounds either way, 3.5 and 3.6; with 1,024 rows of 3,584 8.8 either way) and, beyond 256 rows, something is added (300 of 1,536 with nothing to add 3.2
+  // and 3.3).  So the order of a bfloat16 row's squares goes by how many rows there are; 32-bit rows with one addend keep one order.
+  const int pieces = hidden / 4, wide = std::min(448, (pieces + 63) / 64 * 64), threads = (int)block.x;
+  if (n_partials > 1 && quads && n_rows <= ms_compute_units()) block = dim3(std::min(1024, (pieces + 63) / 64 * 64));
+  else if (dtype == MS_BF16 && quads && (n_rows <= 512 || (n_rows <= 1024 && hidden <= 1024)) && (n_rows <= 256 || delta || hidden > 2048) &&
+           (pieces + wide - 1) / wide < (pieces + threads - 1) / threads)
+    block = dim3(wide);
   // the row is staged in LDS while it fits what a launch may ask for without more ado (64 KB with the 64 bytes
   // of the reduction); a wider row is read from memory a second time instead
   const int staged = (size_t)hidden * sizeof(float) + 64 <= 65536 ? 1 : 0;
