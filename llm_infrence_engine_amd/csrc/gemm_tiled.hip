@@ -667,8 +667,10 @@ static int sums_in_float(int M, int N, int K) {
 // this kernel's, a different W every call, with silu (the gelu and the clamped gate, whose kernels cost more: 1.08 times that), at 190 sizes
 // of up to 2,048 tokens (65 on, 5,632 to 55,296 rows, 1,600 to 5,120 columns) and with the larger tiles at 687 of up to 4,096:
 //   up to 1,536 columns 1.02 to 2 (65 to 8,192 tokens);
-//   up to 2,048 tokens by up to 2,560 columns 0.94 to 1.8, 1.2 on average;
-//   by up to 3,584 columns up to 192 tokens 1.14 to 1.53; by up to 5,120 where the model expects 0.81
+//   up to 2,048 tokens by up to 2,560 columns and up to 192 tokens by up to 3,584 1.03 to 2.1 (128 to 11,008 rows, 65 to 2,048 tokens, 2,300 sizes);
+//     not: 2,304 columns and more that are a multiple of 256, by so few rows and tokens that the library splits them, products of up to 131,072 values,
+//     from 2,816 columns on 262,144 of up to 2,048 rows (2,560 for 96 tokens): 0.75 to 1.06 (512 x 3,584 at 192 tokens 18.7 us and 14.0);
+//   by up to 5,120 where the model expects 0.81
 //     PFLOP/s and more, or by up to 4,096 with tiles that are 0.72 full, 0.94 to 1.44, 1.11 on average (37,888 x 3,584 at 512 tokens 1.17, 900 1.23);
 //     not: tiles of 128 beyond 512 tokens at less than 0.92 PFLOP/s (0.84 to 1.0: what the library takes for 513 to 580 tokens is little more
 //     than for 512); beyond 1,024 tokens by more than 4,096 columns less full than 0.8 (0.95 to 1.12);
@@ -680,7 +682,9 @@ extern "C" int ms_gemm_tiled_pays(int M, int N, int K) {
   if (M <= 0 || N <= 0 || K <= 0 || K % BK) return 0;
   if (K <= 1536 || gate_in_float(M, N, K)) return 1;
   if (K > 5120) return 0;
-  if (M <= 2048 && (K <= 2560 || (K <= 3584 && M <= 192))) return 1;
+  if (M <= 2048 && (K <= 2560 || (K <= 3584 && M <= 192)))
+    return !(K > 2048 && K % 256 == 0 &&
+             (K <= 2560 ? (long long)M * N <= 1 << 17 : (long long)M * N <= 1 << 18 && N <= (M <= 96 ? 2560 : 2048)));
   const TileChoice c = choose_tile(M, N, K);
   if (M <= 2048) {
     const double rate = 2e-9 * M * N * K / c.us;       // PFLOP/s

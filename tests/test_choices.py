@@ -820,3 +820,12 @@ def test_tiles_by_the_model_within_what_it_was_measured_at(ops, M, N, K, tile):
     (896, 896, 18, 64, 6), (1024, 896, 18, 64, 11), (1800, 1024, 14, 64, 11), (70, 512, 12, 128, 6), (4096, 1024, 12, 128, 2)])
 def test_tiles_of_the_qkv_product(ops, M, K, heads, d, tile):
     assert ops._get("ms_gemm_tiled_qkv_tile")(M, K, heads, d) == tile
+
+
+@pytest.mark.parametrize("M,N,K,gated", [
+    # times of the library and the silu's kernel over the tiled kernel's
+    (78, 850, 3584, 0), (192, 512, 3584, 0), (128, 2048, 3584, 0), (160, 1536, 3072, 0), (72, 270, 2560, 0), (192, 512, 2304, 0),     # 0.86 0.75 0.79 0.92 0.98 0.87
+    (160, 2048, 3584, 1), (192, 1400, 2816, 1), (65, 3072, 3584, 1), (100, 2560, 3584, 1), (78, 850, 3456, 1), (192, 512, 2688, 1), (256, 1024, 2560, 1),  # 1.24 1.13 1.26 1.23 1.2 1.07 1.08
+    (65, 128, 2048, 1), (192, 1024, 2304, 1)])                                                                                  # 1.25 1.15
+def test_few_rows_and_tokens_by_long_rows_are_left_to_the_library(ops, M, N, K, gated):
+    assert ops._get("ms_gemm_tiled_pays")(M, N, K) == gated
