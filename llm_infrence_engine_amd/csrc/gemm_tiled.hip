@@ -698,13 +698,11 @@ extern "C" int ms_gemm_tiled_pays(int M, int N, int K) {
 }
 
 // The same question for the squared relu, whose product is written whole and whose own kernel costs little: the sizes that the
-// gated product takes beyond 2,048 tokens or with rounds not full are 0.69 to 1.4 here, a quarter of them below 0.97.
+// gated product takes beyond 2,048 tokens or with rounds not full are 0.69 to 1.4 here, a quarter of them below 0.97.  The narrower tiles
+// move few of them: 11 sizes that their rounds would fill were 0.84 to 1.36, half of them below 0.97 (4,694 x 3,072 at 1,212 tokens 54 us and 46).
 extern "C" int ms_gemm_tiled_relu2_pays(int M, int N, int K) {
   if (M <= 0 || N <= 0 || K <= 0 || K % BK) return 0;
-  if (K <= 1536) return 1;
-  if (rounds_full(M, choose_older(M, N, K))) return 1;
-  const TileChoice c = choose_tile(M, N, K);
-  return M <= 2048 && c.tiles * 10 >= c.slots * 9 && (M > 512 || full(M, N, c) >= 0.9);
+  return K <= 1536 || rounds_full(M, choose_older(M, N, K));
 }
 
 // A bfloat16 [M, lda], W bfloat16 [N, ldw] (rows of K, K a multiple of 64), out bfloat16.

@@ -829,3 +829,8 @@ def test_tiles_of_the_qkv_product(ops, M, K, heads, d, tile):
     (65, 128, 2048, 1), (192, 1024, 2304, 1)])                                                                                  # 1.25 1.15
 def test_few_rows_and_tokens_by_long_rows_are_left_to_the_library(ops, M, N, K, gated):
     assert ops._get("ms_gemm_tiled_pays")(M, N, K) == gated
+
+
+@pytest.mark.parametrize("M,N,K", [(1212, 4694, 3072), (565, 12434, 5120), (1837, 9378, 1600), (608, 10862, 2048)])     # 0.84 0.87 0.88 0.93
+def test_squared_relus_that_the_library_is_faster_at(ops, M, N, K):
+    assert ops._get("ms_gemm_tiled_relu2_pays")(M, N, K) == 0
