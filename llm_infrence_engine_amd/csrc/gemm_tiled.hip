@@ -584,6 +584,9 @@ SumsChoice choose_sums(int M, int N, int K) {
       {T256, 256, 1, 0.19, 5.74, 1.15, 0.00, 0.00, 0.24, 1.40, 0.33},     {T128, 128, 2, 7.16, 0.15, 0.48, 0.61, 0.20, 0.23, 1.13, 0.04},
       {T64, 64, 4, 5.44, 0.00, 0.30, 2.24, 0.00, 0.10, 1.78, 0.02},       {T64_DEEP, 64, 2, 5.87, 0.03, 0.28, 0.48, 0.54, 0.06, 1.39, 0.04},
       {T128_DEEP, 128, 1, 7.12, 0.37, 0.43, 0.00, 0.00, 0.09, 1.52, 0.02}};
+  // More parts than W is read in save nothing (8,072 x 10,880 at 123 tokens 8 parts 62 us, 4 57), and sums in rows that do not begin on four values go out
+  // and come back one by one (7,749 x 10,240 at 127 tokens 8 parts 140 us, 4 103; 103 such sizes 13 % behind the best parts without, 2.5 % so).
+  const double reading = 2e-6 * N * K / 5.5, apart = N % 4 ? 5. : 1.;
   SumsChoice best{0, 1, 1e30, 0};
   for (const auto& k : kinds) {
     if (k.tile == T128_DEEP && M <= 128 && (long long)N * K >= 40000000) continue;
@@ -593,7 +596,7 @@ SumsChoice choose_sums(int M, int N, int K) {
       const double share = (double)blocks / (double)cus;
       const double rounds = k.to_a_cu == 1 ? (double)deep : blocks <= places ? 1. : share / k.to_a_cu + k.over;
       const double step = k.step * (1. + k.beside * (double)(std::min<long long>(deep, k.to_a_cu) - 1)) + k.busy * std::min(1., share);
-      const double us = k.start + rounds * (k.round + (steps + p - 1) / p * step) + (k.sums * p + k.result) * M * N * 8 / 5e6;
+      const double us = k.start + std::max(rounds * (k.round + (steps + p - 1) / p * step), reading) + (k.sums * p * apart + k.result) * M * N * 8 / 5e6;
       if (us < best.us) best = {k.tile, p, us, blocks};
     }
   }
@@ -760,7 +763,9 @@ extern "C" int ms_gemm_tiled(const void* A, long long lda, const void* W, long l
 //     else 0.88 to 2.0, 1.08 on average (8,192 columns 0.89 to 1.17);
 //   up to 1,000 tokens by 4,096 to 8,192 columns for up to 2,048 features, in three parts and more or, from 5,600 columns on, in two of
 //     the tiles of 128, 0.94 to 1.35, 1.08 on average (300 sizes with the norm; 896 x 4,864 by 640 and 768 tokens 24.3 -> 20.6 and 24.9 ->
-//     22.6 us).  Not: whole columns (0.81 to 0.83), two parts of fewer columns (0.95 to 1.06) or of tiles of 64 (0.95 to 1.02);
+//     22.6 us).  Not: whole columns (0.81 to 0.83), two parts of fewer columns (0.95 to 1.06) or of tiles of 64 (0.95 to 1.02), rows that do not begin on four values (1,710 x 7,936
+//     at 711 tokens 0.93); 1,000 is where this was
+//     measured up to (1,001 to 1,100 tokens are 0.95 to 1.5, too);
 //   in all 12 of 3,416 below 0.97;
 //   beyond, by 16,384 columns and more where one round of blocks in parts fills 5/6 of the CUs, but not all: 0.96 to 2.0, 1.4 on
 //     average (3,584 x 18,944 at 1,281 to 1,536 tokens and at 1,793 to 2,304).  With every CU taken 0.96 to 1.02 (4,096 x 28,672 at 2,048
@@ -777,7 +782,7 @@ extern "C" int ms_gemm_tiled_sums_parts(int M, int N, int K) {
   const bool slower =
       (M > 256 && M <= 512 && K > 4096 && K <= 8192 &&
        (c.parts == 1 || c.blocks > 2 * cus || (c.tile != T64_DEEP && c.blocks > cus && c.parts <= 3 && 2e-9 * M * N * K < 0.485 * c.us))) ||
-      (M > 512 && M <= 1024 && K <= 8192 && c.parts < 3 && (c.parts == 1 || K < 5600 || c.tile == T64 || c.tile == T64_DEEP)) ||
+      (M > 512 && M <= 1024 && K <= 8192 && (N % 4 || (c.parts < 3 && (c.parts == 1 || K < 5600 || c.tile == T64 || c.tile == T64_DEEP)))) ||
       (M > 1024 && (c.tile != T256 || c.parts == 1 || c.blocks >= cus || c.blocks * 6 < cus * 5));
   return slower ? sums_in_float(M, N, K) : c.parts;
 }

@@ -834,3 +834,11 @@ def test_few_rows_and_tokens_by_long_rows_are_left_to_the_library(ops, M, N, K, 
 @pytest.mark.parametrize("M,N,K", [(1212, 4694, 3072), (565, 12434, 5120), (1837, 9378, 1600), (608, 10862, 2048)])     # 0.84 0.87 0.88 0.93
 def test_squared_relus_that_the_library_is_faster_at(ops, M, N, K):
     assert ops._get("ms_gemm_tiled_relu2_pays")(M, N, K) == 0
+
+
+@pytest.mark.parametrize("M,N,K,parts", [
+    # us by the parts of a model that counts neither the reading of W nor rows of sums that begin anywhere, and by these
+    (84, 7327, 11456, 4), (127, 7749, 10240, 2), (402, 827, 9088, 2), (77, 7473, 21248, 4),                  # 123 87; 140 103; 47 38; 151 119
+    (123, 8072, 10880, 4), (87, 8192, 7360, 4), (112, 6284, 21888, 5), (69, 6552, 7808, 4), (711, 1710, 7936, 0)])   # 62 57; 43 36; 96 86; 38 34; 54 50
+def test_parts_of_sums_by_what_reading_w_and_odd_rows_cost(ops, M, N, K, parts):
+    assert ops._get("ms_gemm_tiled_sums_parts")(M, N, K) == parts
