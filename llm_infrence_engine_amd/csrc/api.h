@@ -66,7 +66,8 @@ int ms_gemm_skinny(const void* A, long long lda, const void* W, long long ldw, c
 void ms_gemm_skinny_force(int ntile, int waves, int token_groups);
 void ms_attention_mfma_force(int nt, int waves, int dim_shares);
 void ms_attention_generic_force(int waves);      // measurements: 1 or 4 waves to a (token, query head); 0 leaves the choice
-void ms_gemm_f32_force(int kernel);              // measurements: 1 few rows, 2 and 3 tiles of 64 and 32, 4 and 5 up to 8 rows; 0 leaves the choice
+void ms_gemm_f32_force(int kernel);              // measurements: 1 few rows, 2 and 3 tiles of 64 and 32, 4 and 5 up to 8 rows, 6 to 8 slices of 16, 32 and 48 tokens; 0 leaves the choice
+int ms_gemm_f32_kernel(int M, int N, int K);     // the kernel (as forced) that a product of rows K apart takes by itself
 
 int ms_gemm_stream(const void* A, long long lda, const int* rows, const float* norm_w, float eps, const void* W,
                    long long ldw, const float* bias, void* out, long long ldo, int M, int N, int K, int epilogue,

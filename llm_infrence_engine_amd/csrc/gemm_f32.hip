@@ -4,7 +4,7 @@
 // The order of a sum is the same whatever M is, so a token's result does not depend on what else is in the batch: K is
 // cut into at most 16 slices (from K alone, `slice_steps`), a slice is summed 16 values at a time from its start, and the
 // slices are added in order.  All kernels keep that order:
-//   rows     up to 64 rows (a decode step; against very many rows of W up to 16): all waves of a block on the same 4 to 16
+//   rows     up to 64 rows, by less than 512 columns and where `choose` takes it: all waves of a block on the same 4 to 16
 //            rows of W, the slices dealt out over them and added through LDS.  Bound by reading W.
 //   few      up to 8 rows, of these: loads that take four steps at a time.
 //   diagonal up to 8 rows: an instruction takes a step of two or four slices; also with the norm of A's rows, the gate, or the rotation
@@ -493,15 +493,18 @@ gemm_f32_tiled_kernel(const float* __restrict__ A, const float* __restrict__ W, 
 
 int g_kernel = 0;      // measurements: 1 the kernel of up to 64 rows, 2 and 3 the tiled one with tiles of 64 and 32, 4 and 5 that of up to 8 with blocks of 4 and 8 rows of W, 6 to 8 the slices of 16, 32 and 48 tokens; 0 leaves the choice
 
-// Rows of W to a block of the kernel of slices side by side, for a plain product; 0: another kernel is as fast or faster.  us with four steps
-// to a load | so, at 3 and 8 tokens: 896 x 896 4.6 | 4.4 (8: 5.0 | 5.1), 896 x 4,864 11.4 | 8.5 and 12.9 | 12.3; 8 rows: 2,048 x 2,048
-// 7.5 | 7.0 and 8.0 | 7.8, 6,144 x 1,536 15.0 | 12.1 and 15.7 | 15.2, 4,608 x 3,584 26.3 | 22.3 but at 8 26.3 | 28.7; 3,584 x 18,944 62 | 71;
-// 384 x 192 3.1 | 3.3; 9,728 x 896 11.4 | 11.0 and 12.4 | 14.3.
+// Rows of W to a block of the kernel of slices side by side, for a plain product; 0: another kernel is as fast or faster.  Time with four steps to a
+// load over that so, W in no cache (64 to 64,000 rows, 256 to 18,944 columns).  4 rows a block, a block a CU: up to 4 tokens from 692 columns on 0.97 to 1.5
+// (896 x 4,864 with 3 tokens 11.4 | 8.5 us; 512 columns 0.94 to 1.0), 5 to 8 tokens by 1,028 to 4,864 0.94 to 1.2 (4,992 on 0.9 to 1.1, up to 1,024 0.9 to
+// 1.02).  8 rows, up to 4 tokens by 1,028 to 4,864 columns 0.98 to 1.24 (4,992 on 0.88 to 1.08), 5 to 8 by up to 1,536 0.95 to 1.2 (2,048 0.93 to 1.05): a
+// block a CU, or where 16 rows a block would be more than one; between these (2,049 to 4,096 rows) 0.67 to 1.0.  Up to three blocks a CU (9,728 rows 0.9 to
+// 1.2 up to 4 tokens, 0.86 to 1.1 with 8).
 int diagonal_rows(int M, int N, int K) {
   const int cus = ms_compute_units();
-  if (M > 8 || K < 512 || K > (M <= 4 ? 5120 : 4992)) return 0;
-  if ((N + 3) / 4 <= cus) return M <= 4 || K > 1024 ? 4 : 0;
-  return (N + 7) / 8 <= 3 * cus && K > 1024 && (M <= 4 || K <= 2048) ? 8 : 0;
+  if (M > 8) return 0;
+  if ((N + 3) / 4 <= cus) return M <= 4 ? (K > 640 ? 4 : 0) : K > 1024 && K <= 4864 ? 4 : 0;
+  const int blocks = (N + 7) / 8;
+  return (blocks <= cus || ((N + 15) / 16 > cus && blocks <= 3 * cus)) && K > 1024 && K <= (M <= 4 ? 4864 : 1536) ? 8 : 0;
 }
 
 // Floats of LDS.
@@ -622,27 +625,40 @@ int slices_of(int K) { const int steps = (K + STEP - 1) / STEP, per = slice_step
 // bytes: two stages of 32 columns a wave, or the slices' sums
 int slices_lds(int TM, int slices) { return std::max((slices + 1) / 2 * 2 * (32 + TM) * 32, slices * TM * (32 + 4)) * (int)sizeof(float); }
 
-// The kernel for more rows than the first two take, by what each was seen to take on 150 sizes (128 to 151,936 by 512 to 18,944, 13 to
-// 2,048 rows; 256 CUs): us = start + (begin + step * K / 1,000) * rounds.  `slices` runs in whole rounds of blocks, one or two to a CU by
-// its LDS; of the tiled one's blocks several lie on a CU, and up to one a CU they take as long as one.  The kernel so chosen is within
-// 0.3 % of the fastest on average (4 % at most, but for 7 sizes).  Before, by the number of tiles alone and with tiled kernels alone
-// | now: 896 x 4,864 at 17, 64, 350, 512 and 2,048 rows 24 | 18, 47 | 18, 81 | 45, 82 | 56, 224 | 192 us; 896 x 896 at 64 and 350
-// 12.5 | 6.9, 18.0 | 13.1; 1,152 x 896 at 350 18.1 | 16.8; 4,608 x 3,584 at 17 and 128 41 | 25, 80 | 65; 9,728 x 896 as before.
-enum { ROWS16 = 16, ROWS32 = 32, ROWS48 = 48, TILE32 = 1, TILE64 = 2 };
-int choose(int M, int N, int K, int cus) {
+// The kernel for more than 8 rows by 512 columns and more, by what each was seen to take at 4,600 sizes (64 to 64,000 by 512 to 18,944, 9 to 2,048
+// rows; 256 CUs, W in no cache): a start, the reading of W by the MB, and rounds.  `slices` is bound by what a CU reads however many blocks it has at once;
+// only their beginnings overlap, one to four to a CU by its LDS.  Of the tiled one's blocks several lie on a CU, and up to one a CU they take as long
+// as one.  Rows that are no multiple of 128 bytes cost `slices` 1.1 to 1.45 times the time (`apart`), the first kernel 1.13, the tiles nothing.  The kernel so
+// chosen is 0.8 % behind the fastest on average, 21 % at worst (by tiles and slices as if the blocks of a CU did not share it, and W's rows lay on 128 bytes,
+// 2.5 % and 7.8 % behind with rows that do and that do not, and twice the time at worst: 9 rows of 401 x 13,188 38 -> 72 -> 38 us, 512 of 64,000 x 512 331 ->
+// 571 -> 331, 1,000 of 3,072 x 768 50 -> 76 -> 50).  Before, by the number of tiles alone and with tiled kernels alone | now: 896 x 4,864 at 17, 64, 350, 512 and
+// 2,048 rows 24 | 18, 47 | 18, 81 | 45, 82 | 56, 224 | 192 us; 896 x 896 at 64 and 350 12.5 | 6.9, 18.0 | 13.1; 1,152 x 896 at 350 18.1 | 16.8; 4,608 x 3,584 at
+// 17 and 128 41 | 25, 80 | 65; 9,728 x 896 as before.
+enum { ROWS16 = 16, ROWS32 = 32, ROWS48 = 48, TILE32 = 1, TILE64 = 2, ROWS = 3 };
+int rows_a_block(int N, int cus) { return (N + 3) / 4 <= cus ? 4 : (N + 7) / 8 <= cus ? 8 : 16; }
+int choose(int M, int N, int K, bool apart, int cus) {
   int best = 0;
   float least = 0.f;
   auto offer = [&](int kind, float us) { if (best == 0 || us < least) { best = kind; least = us; } };
   auto tiles = [&](int T) { return (float)((long long)((N + T - 1) / T) * ((M + T - 1) / T)) / cus; };
-  const float k = K * 1e-3f, t64 = tiles(64), t32 = tiles(32);
-  offer(TILE64, 2.f + (1.7f + 24.2f * k) * (t64 <= 1.f ? 1.f : std::max(1.55f, 0.45f + 0.75f * t64)));
-  offer(TILE32, 2.f + (0.8f + 13.f * k) * (t32 <= 1.f ? 1.f : std::max(1.25f, 0.65f + 0.45f * t32)));
-  const float begin[] = {2.2f, 3.3f, 4.f}, step[] = {3.f, 5.1f, 7.8f};
+  const float k = K * 1e-3f, mb = k * N * 4e-3f, t64 = tiles(64), t32 = tiles(32);
+  offer(TILE64, 2.6f + 0.05f * mb + (2.6f + 23.2f * k) * (t64 <= 1.f ? 1.f : std::max(1.63f, 0.43f + 0.73f * t64)));
+  offer(TILE32, 2.1f + 0.09f * mb + (1.f + 14.1f * k) * (t32 <= 1.f ? 1.f : std::max(1.19f, 0.44f + 0.433f * t32)));
+  const struct { float begin, step, whole, read, begin_apart, step_apart; } kinds[] = {
+      {1.7f, 3.09f, 0.71f, 0.169f, 1.29f, 1.39f}, {2.88f, 4.83f, 0.9f, 0.117f, 1.36f, 1.2f}, {3.33f, 7.57f, 0.94f, 0.088f, 1.45f, 1.1f}};
   for (int i = 0; i < 3; ++i) {
-    const int TM = 16 * (i + 1), room = cus * std::min(4, LDS_BYTES / slices_lds(TM, slices_of(K)));
+    const auto& t = kinds[i];
+    const int TM = 16 * (i + 1), at_once = cus * std::min(4, LDS_BYTES / slices_lds(TM, slices_of(K)));
     const long long blocks = (long long)((N + 31) / 32) * ((M + TM - 1) / TM);
     if ((M + TM - 1) / TM > 65535) continue;
-    offer(TM, 1.5f + (begin[i] + step[i] * k) * (0.95f * ((blocks + room - 1) / room) + 0.05f * std::max(1.f, (float)blocks / room)));
+    const float begin = t.begin * (apart ? t.begin_apart : 1.f), step = t.step * k * (apart ? t.step_apart : 1.f);
+    offer(TM, 2.2f + t.read * mb + begin * ((blocks + at_once - 1) / at_once) +
+                  step * (t.whole * ((blocks + cus - 1) / cus) + (1.f - t.whole) * std::max(1.f, (float)blocks / cus)));
+  }
+  if (M <= 64) {
+    const int R = rows_a_block(N, cus), nt = M <= 16 ? 1 : M <= 32 ? 2 : 4;
+    const float share = (float)((N + R - 1) / R) / cus;
+    offer(ROWS, 2.7f + 0.41f * nt + (1.4f + 0.14f * R + 0.111f * M + 0.028f * R * nt) * k * (apart ? 1.13f : 1.f) * (share <= 1.f ? 1.f : 0.72f + 0.9f * share));
   }
   return best;
 }
@@ -683,28 +699,41 @@ int ms_gemm_f32_normed(const float* x, const float* W, const float* bias, float*
 #undef GO
 }
 
+namespace {
+
+// Below 512 columns, which writing C bounds: the tiles, the larger ones from two a CU on, but few rows against few of W in the first kernel (of more than 16
+// rows every block of it reads all of A, a tile its part once through LDS; 24 rows of 20,000 x 512 17.2 us there, 15.3 in tiles, 32 of 152,064 x 3,584 1,010 and
+// 519, 64 of 151,936 x 896 405 and 220, of 6,144 x 2,048 43 and 40, but 33 of them 33 and 40).
+int kind_of(int M, int N, int K, bool apart, int cus) {
+  if (M <= 8) return ROWS;
+  if (K >= 512) return choose(M, N, K, apart, cus);
+  if (M <= 16 || (M <= 32 ? N < 64 * cus : M <= 64 && N < 32 * cus)) return ROWS;
+  return M > 32 && (long long)((N + 63) / 64) * ((M + 63) / 64) >= 2 * cus ? TILE64 : TILE32;
+}
+
+}  // namespace
+
 extern "C" void ms_gemm_f32_force(int kernel) { g_kernel = kernel; }
+extern "C" int ms_gemm_f32_kernel(int M, int N, int K) {
+  const int side_by_side = diagonal_rows(M, N, K), kind = side_by_side ? 0 : kind_of(M, N, K, K % 32 != 0, ms_compute_units());
+  return side_by_side ? 3 + side_by_side / 4 : kind == ROWS ? 1 : kind == TILE64 ? 2 : kind == TILE32 ? 3 : 5 + kind / 16;
+}
 
 // The caller has checked sizes; K, lda and ldw are multiples of 4 and A and W lie on 16 bytes.
 int ms_gemm_f32_launch(const float* A, const float* W, const float* bias, float* C, int M, int N, int K, size_t lda,
                        size_t ldw, size_t ldc, int accumulate, hipStream_t stream) {
   const int cus = ms_compute_units();
-  // More than 16 rows against many: every block of the first kernel reads all of A, a tile its part once through LDS.  17 to 32
-  // rows from 64 features a CU on (24 rows of 20,000 x 512 17.2 us there, 15.3 in tiles; 32 of 152,064 x 3,584 1,010 and 519;
-  // of 9,728 x 896 19.3 and 19.1), 33 to 64 from 32 a CU on (64 of 9,728 x 896 33 and 24, of 151,936 x 896 405 and 220, of
-  // 6,144 x 2,048 43 and 40, but 33 of them 33 and 40).
-  // From 13 rows on (9 by rows of more than 1,024 columns) the choice is another one from 512 columns on (12 rows of 896 x 896 6.3 us
-  // in the first kernel, 6.5 as slices, 16 of them 6.8 and 6.5; 9 rows of 4,608 x 3,584 32 and 18, of 2,048 x 2,048 9.5 and 9.9).
-  const bool few = M <= 8 || (M <= 12 && K <= 1024) || (K < 512 && (M <= 16 || (M <= 32 ? N < 64 * cus : M <= 64 && N < 32 * cus)));
   const int side_by_side = M > 8 ? 0 : g_kernel == 4 ? 4 : g_kernel == 5 ? 8 : g_kernel == 0 ? diagonal_rows(M, N, K) : 0;
   if (side_by_side)
     return launch_diagonal<F32_STORE, 0>(side_by_side, A, W, bias, C, M, N, K, lda, ldw, ldc, accumulate, F32Norm{}, F32Front{}, stream);
-  if (g_kernel == 1 ? M <= 64 : g_kernel == 0 && few) {
+  const int kind = g_kernel == 1 && M <= 64 ? ROWS : g_kernel == 2 ? TILE64 : g_kernel == 3 ? TILE32 : g_kernel >= 6 ? 16 * (g_kernel - 5)
+                   : kind_of(M, N, K, lda % 32 || ldw % 32, cus);
+  if (kind == ROWS) {
     // Rows a block: as few as keep the blocks within the CUs, because a CU reads at a rate of its own and 16 bytes a lane
     // fill 64-byte pieces from 4 rows as from 16 (3 rows of 896 x 4,864: 18.3 us as 56 blocks of 16, 17.2 as 224 of 4;
     // q/k/v 6.5 and 6.3).  More tiles than CUs: blocks of four waves, several of them on a CU, instead of one that has a
     // wave for every slice (9,728 x 896: 19.6 us, now 11.9; the head 161, now 100).
-    const int R = (N + 3) / 4 <= cus ? 4 : (N + 7) / 8 <= cus ? 8 : 16;
+    const int R = rows_a_block(N, cus);
     const int steps = (K + STEP - 1) / STEP, per = slice_steps(K), slices = (steps + per - 1) / per;
     const int waves = (N + R - 1) / R > cus && slices > 4 ? 4 : slices;
     dim3 grid((N + R - 1) / R), block(waves * MS_WAVE);
@@ -727,9 +756,6 @@ int ms_gemm_f32_launch(const float* A, const float* W, const float* bias, float*
 #undef ROWS
     return ms_launch_status();
   }
-  // K below 512 is bound by writing C and stays with the tiled kernel, the larger tiles from two a CU on
-  const int kind = g_kernel == 2 ? TILE64 : g_kernel == 3 ? TILE32 : g_kernel >= 6 ? 16 * (g_kernel - 5) : K >= 512 ? choose(M, N, K, cus)
-                   : M > 32 && (long long)((N + 63) / 64) * ((M + 63) / 64) >= 2 * cus ? TILE64 : TILE32;
   const int runs = ldc % 4 == 0 && (uintptr_t)C % 16 == 0;
 #define SLICES(TM) return launch_slices<TM>(A, W, bias, C, M, N, K, lda, ldw, ldc, accumulate, runs, stream)
   if (kind == ROWS16) SLICES(16);

@@ -81,6 +81,7 @@ _SIGNATURES = {
     "ms_gemm_tiled_force_xcd_split": [_c_int],
     "ms_gemm_tiled_pays": [_c_int, _c_int, _c_int],
     "ms_gemm_tiled_tile": [_c_int, _c_int, _c_int],
+    "ms_gemm_f32_kernel": [_c_int, _c_int, _c_int],
     "ms_gemm_tiled_qkv_tile": [_c_int, _c_int, _c_int, _c_int],
     "ms_gemm_tiled_relu2_pays": [_c_int, _c_int, _c_int],
     "ms_gemm_tiled_plain_pays": [_c_int, _c_int, _c_int],

@@ -842,3 +842,18 @@ def test_squared_relus_that_the_library_is_faster_at(ops, M, N, K):
     (123, 8072, 10880, 4), (87, 8192, 7360, 4), (112, 6284, 21888, 5), (69, 6552, 7808, 4), (711, 1710, 7936, 0)])   # 62 57; 43 36; 96 86; 38 34; 54 50
 def test_parts_of_sums_by_what_reading_w_and_odd_rows_cost(ops, M, N, K, parts):
     assert ops._get("ms_gemm_tiled_sums_parts")(M, N, K) == parts
+
+
+@pytest.mark.parametrize("M,N,K,kernel", [
+    # us of the first kernel, tiles of 64 and 32, slices of 16, 32 and 48 tokens
+    (9, 401, 13188, 1), (16, 896, 9008, 1), (13, 3129, 764, 1),                     # 37.8 .. .. 72.7;  30 .. .. 46;  5.4 .. .. 7.1
+    (512, 64000, 512, 2), (1000, 3072, 768, 2), (1000, 20000, 512, 2), (350, 9728, 13188, 2),     # 331 .. 571;  50.3 .. 75.8;  207 .. 348;  990 .. .. 1,587
+    (17, 896, 4864, 6), (64, 896, 896, 6), (350, 896, 4864, 8), (24, 9728, 512, 6), (2048, 9728, 896, 2),
+    # below 512 columns
+    (16, 896, 132, 1), (20, 64000, 256, 3), (100, 64000, 256, 2), (100, 896, 256, 3),
+    # up to 8 rows: four steps to a load, slices side by side with 4 and with 8 rows of W a block
+    (8, 2563, 2048, 1), (4, 2563, 5120, 1), (4, 4608, 4992, 1), (8, 2048, 2048, 1), (3, 9728, 896, 1), (2, 896, 512, 1),       # 11.4 .. 14.2;  25.2 .. 29.9;  41.6 .. 44.6
+    (3, 896, 4864, 4), (4, 1024, 18944, 4), (8, 896, 4864, 4), (8, 896, 896, 1), (4, 2048, 4864, 5), (8, 6144, 1536, 5), (4, 4608, 3584, 5)])
+def test_kernels_of_32_bit_products(ops, M, N, K, kernel):
+    """All of them have the same bits."""
+    assert ops._get("ms_gemm_f32_kernel")(M, N, K) == kernel

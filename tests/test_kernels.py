@@ -2252,7 +2252,7 @@ def test_splits_are_put_together(ops, nh, nkv, d, keys, cap):
     assert (out[1] == 7.0).all()
 
 
-@pytest.mark.parametrize("N,K", [(4, 512), (90, 896), (896, 4864), (1031, 1028), (2053, 1100), (1500, 2052), (2048, 16)])
+@pytest.mark.parametrize("N,K", [(4, 512), (90, 896), (896, 4864), (1031, 1028), (2053, 1100), (1500, 2052), (2048, 16), (1021, 13188)])
 def test_32_bit_products_of_up_to_8_rows_have_the_bits_of_the_kernel_for_64(ops, N, K):
     """Blocks of 4 and of 8 rows of W whose instructions hold two or four slices side by side, for one to eight tokens: columns that
     end within a slice, a step or a piece, slices that are not a whole number of instructions, rows past the last; with bias and
@@ -2480,7 +2480,7 @@ def test_logits_of_17_to_64_tokens_by_very_many_rows(ops, M, N, K):
     assert torch.equal(got, ops.gemm_tiled_sums(a[:M], w, 1)[0])
 
 
-@pytest.mark.parametrize("M,N,K", [(9, 31, 512), (13, 64, 516), (17, 97, 560), (33, 33, 896), (48, 130, 1100), (49, 65, 2052), (97, 896, 4864), (5, 7, 64), (20, 36, 20)])
+@pytest.mark.parametrize("M,N,K", [(9, 31, 512), (13, 64, 516), (17, 97, 560), (33, 33, 896), (48, 130, 1100), (49, 65, 2052), (97, 896, 4864), (5, 7, 64), (20, 36, 20), (16, 401, 9008), (64, 130, 516), (33, 1026, 692)])
 def test_32_bit_products_by_slices_have_the_bits_of_the_tiles(ops, M, N, K):
     """Blocks whose waves have two slices each: one, an odd number and all sixteen of them, columns that end within a slice, a step or a
     piece, tokens and rows of W past the last, rows of C at any address; with bias and added onto what is there.  The tiled kernel sums in
