@@ -324,7 +324,9 @@ gemm_tiled_kernel(const bf16* __restrict__ A, size_t lda, const bf16* __restrict
   }
   auto last_steps = [&](auto self, auto left_c) -> void {
     constexpr int LEFT = decltype(left_c)::value;
-    if (LEFT == 0 || steps - at > LEFT) {      // (fewer steps than slots: the pipeline never fills; the last one there always is)
+    // Fewer steps than slots: the pipeline never fills.  (The last step there always is.  Said so to the compiler, the loop of small tiles is 64 to 68
+    // instructions; not, it has two copies of their sums and moves all of them over in every step, 99.  Large tiles it makes wait for registers when told.)
+    if ((LEFT == 0 && FT * TT <= 4) || steps - at > LEFT) {
       step(left_c, at, sw, after_w(sw), before_w(sw), sa, after_a(sa));
       sw = after_w(sw);
       sa = after_a(sa);
