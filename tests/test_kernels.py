@@ -1017,13 +1017,13 @@ def test_gemm_skinny_refuses_what_it_cannot_take(ops):
         ops.gemm_skinny(a[:4, :60], w[:, :60].contiguous())
 
 
-@pytest.mark.parametrize("tile", [1, 2, 3, 4, 5])
+@pytest.mark.parametrize("tile", [1, 2, 3, 4, 5, 6, 7, 8, 9, 10, 11])
 @pytest.mark.parametrize("M,N,K", [(65, 662, 64), (300, 2 * 331, 192), (257, 130, 896), (1000, 2 * 4864, 896), (2051, 1026, 128),
                                    (130, 16, 64), (513, 4100, 1536), (4100, 2 * 331, 64), (6200, 1300, 128), (70, 700, 256),
                                    (390, 258, 320)])
 def test_gemm_tiled(ops, M, N, K, tile):
-    """The many-rows product and its gated epilogue with every tile shape (256, 128, 64, 192 and 160 features wide:
-    the last two store a lane's results in pieces of 8 and 4 bytes): rows and features that fill no whole tile, rows
+    """The many-rows product and its gated epilogue with every tile shape (256, 128, 64, 192 and 160 features wide and those with
+    more steps ahead; 192, 160 and 96 store a lane's results in pieces of 8 and 4 bytes): rows and features that fill no whole tile, rows
     of the result that start at odd addresses, one to five steps of 64 columns and many, and so many tokens that the tiles are
     laid over the XCDs in two and in four rows."""
     force = ops._get("ms_gemm_tiled_force")
@@ -1046,9 +1046,12 @@ def test_gemm_tiled(ops, M, N, K, tile):
     assert torch.equal(ops.gemm_tiled(a[M - 70:], w), out[M - 70:])
 
 
-@pytest.mark.parametrize("M,N,K", [(640, 6528, 576), (640, 6530, 576), (65, 32640, 64), (129, 16386, 128)])
-def test_gemm_tiled_on_both_sides_of_its_small_tiles(ops, M, N, K):
-    """Where the choice goes from tiles of 64 x 64 to wider ones (as many tiles of 128 x 128 as CUs): the same bits as with either."""
+@pytest.mark.parametrize("M,N,K,taken", [(411, 4670, 384, 6), (411, 4674, 384, 2), (146, 19200, 256, 7), (146, 19246, 256, 3), (65, 32640, 64, 3),
+                                         (129, 16386, 128, 2), (6143, 1300, 256, 4), (6144, 1300, 256, 2), (640, 6528, 576, 2), (640, 6530, 576, 7)])
+def test_gemm_tiled_on_both_sides_of_its_small_tiles(ops, M, N, K, taken):
+    """Where the choice goes from deep tiles of 64 x 64 (two a CU) to wider ones, and to shallow ones where these are more; below 256 columns
+    from shallow ones to wider (as many tiles of 128 x 128 as CUs); at the ends of the model: the same bits as with either."""
+    assert ops._get("ms_gemm_tiled_tile")(M, N, K) == taken
     force = ops._get("ms_gemm_tiled_force")
     force.restype = None
     g = torch.Generator().manual_seed(M + N)
@@ -1056,7 +1059,7 @@ def test_gemm_tiled_on_both_sides_of_its_small_tiles(ops, M, N, K):
     w = (torch.randn(N, K, generator=g) / math.sqrt(K)).bfloat16().to(DEV)
     out, act = ops.gemm_tiled(a, w), ops.gemm_tiled(a, w, ops.EPI_SWIGLU)
     torch.testing.assert_close(out.double(), a.double() @ w.double().T, **tol(torch.bfloat16))
-    for tile in (2, 3):
+    for tile in (2, 3, 6):
         force(tile)
         try:
             assert torch.equal(out, ops.gemm_tiled(a, w)) and torch.equal(act, ops.gemm_tiled(a, w, ops.EPI_SWIGLU))
@@ -1065,9 +1068,10 @@ def test_gemm_tiled_on_both_sides_of_its_small_tiles(ops, M, N, K):
 
 
 def test_gemm_tiled_of_long_rows_is_not_taken_for_small_tiles(ops):
-    """Four tiles of 64 x 64 to nearly every CU, which the library's product is faster than: rows that begin on 8 bytes and
+    """A tile of 128 x 128 to nearly every CU, which the library's product is faster than: rows that begin on 8 bytes and
     rows that do not."""
     for n in (15360, 15362):
+        assert ops._get("ms_gemm_tiled_tile")(256, n, 4096) == 2
         assert ops._get("ms_gemm_tiled_pays")(256, n, 4096) == 0
 
 
