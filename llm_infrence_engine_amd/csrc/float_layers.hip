@@ -1,5 +1,6 @@
-// All layers of a 32-bit step by one call, to the same bits as when every part is asked for by itself: its nine kernels a layer, or,
-// up to 8 tokens, five.  A decode step of the 32-bit path was as slow as its launches were made: 219 of them took 2.62 ms from
+// All layers of a 32-bit step by one call, to the same bits as when every part is asked for by itself: its nine kernels a layer, or, up to 8
+// tokens where the products take the norms, the rotation and the gate (ms_gemm_f32_normed: hidden sizes up to 2,048, matrices up to 32 million
+// values, rows that fit 64 KB of LDS), five; the q/k/v and the gated product each for itself.  A decode step of the 32-bit path was as slow as its launches were made: 219 of them took 2.62 ms from
 // Python (12 us each, of which the launch itself is 4) where the GPU has 1.7 ms of work; with five it has 1.2 (0.5B sizes, 3 tokens behind
 // 130: two norms, the rotation and the activation were 15.6 us of a layer's 70, and are 1 to 2 of the products' that took them in).
 #include "common.h"

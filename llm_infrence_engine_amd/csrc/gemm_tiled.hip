@@ -2,10 +2,11 @@
 // matrix cores (v_mfma_f32_16x16x32_bf16), with the gated activation as an epilogue: the product of the
 // interleaved gate/up weight never goes to memory, which saves the write of [M, 2I], its read and a kernel.
 //
-// A block of 8 waves owns a tile of BN features by BM tokens, as large as registers allow (256 x 256: a byte
-// loaded does 128 multiply-adds).  Per step of 64 columns the tile's rows of W and A go from memory straight to LDS
-// (global_load_lds, 16 bytes a lane: no registers, no LDS write instructions), A one step and W two steps before they are
-// multiplied; the 256 x 256 tile's three slots for W and two for A are all of the CU's 160 KB.  LDS rows are 128 bytes
+// A block of 4 or 8 waves owns a tile of BN features by BM tokens: as large as registers allow where there are enough of them (256 x 256: a byte
+// loaded does 128 multiply-adds), narrower where CUs would be left without one.  Per step of 64 columns the tile's rows of W and A go from memory
+// straight to LDS (global_load_lds, 16 bytes a lane: no registers, no LDS write instructions) into SW slots for W and SA for A, SW - 1 and SA steps
+// before they are multiplied: with three slots and two the 256 x 256 tile's are all of the CU's 160 KB, tiles of 64 and 96 have up to five of each,
+// since a step of theirs is over before its successor's rows have come.  LDS rows are 128 bytes
 // with their eight 16-byte pieces permuted by the row number (piece c at place c ^ (row & 7)): fragment reads then run at
 // the full LDS rate (measured 237 bytes a clock; rows 144 bytes apart give 116).
 //
@@ -548,7 +549,8 @@ TileChoice choose_older(int M, int N, int K) {
 // 256 to 3,584 columns), every tile timed at each, every product by a W that lies in no cache.  Its times lie within 0.77 and 1.28 of the measured
 // ones (tiles with a CU to themselves 0.81 to 1.14), and the tile it takes is 0.4 % behind the best one on average, 12 % at worst; with 1 to 5 alone
 // the best is 9 % behind on average and up to 42 (0.5B gate/up, 9,728 x 896: 128 tokens 11.1 -> 9.3 us, 256 13.9 -> 10.9, 512 18.4 -> 13.6, 768 17.7 ->
-// 16.3, from 1,024 on the same; 5,632 x 2,048 at 256 tokens 20.8 -> 15.8, 37,888 x 3,584 at 128 80 -> 56).
+// 16.3, from 1,024 on the same; 5,632 x 2,048 at 256 tokens 20.8 -> 15.8, 37,888 x 3,584 at 128 80 -> 56).  (The tiles of 64 x 64 have become a
+// little faster since, 0.1 to 0.8 us a product; at 171 sizes down to 64 features it is 2.2 % behind the best one.)
 TileChoice choose_tile(int M, int N, int K) {
   // What the model was measured at ends here.  Taken there all the same it was 0.71 to 1.13 times as fast as those below up to 192 columns and 0.62 to 1.2
   // beyond 4,096 tokens (146 sizes): 12,558 x 128 at 1,188 tokens 23.9 and 28.5 us, 980 x 128 at 10,455 15.4 and 22.4.

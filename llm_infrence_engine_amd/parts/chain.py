@@ -138,7 +138,8 @@ class _Addresses:
 
 class FloatLayers:
     """The layers of a step in float32, launched kernel by kernel, by one call (``ops.float_layers``): the kernels that the parts
-    would launch one by one, in their order, or up to 8 tokens five a layer that take several of them together, to the same bits."""
+    would launch one by one, in their order, or, up to 8 tokens of up to 2,048 values, five a layer that take several of them together, to the
+    same bits."""
 
     def __init__(self, model, sizes: tuple, caches):
         self.sizes, self.layers = sizes, [model.layers[run.layer] for run in model.spec.order]
