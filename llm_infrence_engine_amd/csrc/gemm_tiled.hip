@@ -626,9 +626,9 @@ static double full_in_rows(int M, int N, const TileChoice& c) {
 // Products whose result has to stay in 32 bits up to what reads it.  Where gate and up, or the addend of a norm, have been held in float by this
 // kernel, the library's product in its place would round them to bfloat16 first, which nobody asked for: so the sizes below, which the tiles
 // with two steps ahead (256, 192 or 160 features by 256 tokens, 128 x 128, 64 x 64) were given by their own measurements, stay here also where
-// the library is expected to be faster now.  Of 1.4 million sizes (65 to 8,192 tokens) that is 11 % of the gated ones, most of them by more than
-// 5,120 columns, 2 % of the squared relu's and 0.02 % of the sums'; time of the library and the next kernel over this one's at 125 of them, W in no
-// cache: 0.84 to 1.63, 1.05 on average, 0.67 to 1.30, 0.95, and 0.82 to 1.88, 1.05.
+// the library is expected to be faster now (and the squared relu's are these alone).  Of 1.4 million sizes (65 to 8,192 tokens) that is 11 % of the gated
+// ones, most of them by more than 5,120 columns, and 0.02 % of the sums'; time of the library and the next kernel over this one's at 65 of them, W in
+// no cache: 0.84 to 1.63, 1.05 on average, and 0.82 to 1.88, 1.05.
 static bool rounds_full(int M, const TileChoice& older) { return older.tile != T64 && M <= 2048 && older.tiles * 10 >= older.slots * 9; }
 static bool gate_in_float(int M, int N, int K) {
   const TileChoice c = choose_older(M, N, K);
@@ -674,11 +674,10 @@ static int sums_in_float(int M, int N, int K) {
 // this kernel's, a different W every call, with silu (the gelu and the clamped gate, whose kernels cost more: 1.08 times that), at 190 sizes
 // of up to 2,048 tokens (65 on, 5,632 to 55,296 rows, 1,600 to 5,120 columns) and with the larger tiles at 687 of up to 4,096:
 //   up to 1,536 columns 1.02 to 2 (65 to 8,192 tokens);
-//   up to 2,048 tokens by up to 2,560 columns and up to 192 tokens by up to 3,584 1.03 to 2.1 (128 to 11,008 rows, 65 to 2,048 tokens, 2,300 sizes);
-//     not: 2,304 columns and more that are a multiple of 256, by so few rows and tokens that the library splits them, products of up to 131,072 values,
+//   up to 2,048 tokens by up to 2,560 columns and up to 192 tokens by up to 3,584 1.03 to 2.1 (128 to 11,008 rows, 65 to 2,048 tokens, 2,300
+//     sizes); not: 2,304 columns and more that are a multiple of 256, by so few rows and tokens that the library splits them, products of up to 131,072 values,
 //     from 2,816 columns on 262,144 of up to 2,048 rows (2,560 for 96 tokens): 0.75 to 1.06 (512 x 3,584 at 192 tokens 18.7 us and 14.0);
-//   by up to 5,120 where the model expects 0.81
-//     PFLOP/s and more, or by up to 4,096 with tiles that are 0.72 full, 0.94 to 1.44, 1.11 on average (37,888 x 3,584 at 512 tokens 1.17, 900 1.23);
+//   by up to 5,120 where the model expects 0.81 PFLOP/s and more, or by up to 4,096 with tiles that are 0.72 full, 0.94 to 1.44, 1.11 on average (37,888 x 3,584 at 512 tokens 1.17, 900 1.23);
 //     not: tiles of 128 beyond 512 tokens at less than 0.92 PFLOP/s (0.84 to 1.0: what the library takes for 513 to 580 tokens is little more
 //     than for 512); beyond 1,024 tokens by more than 4,096 columns less full than 0.8 (0.95 to 1.12);
 //   in all 0.6 % behind the better way on average (250 sizes), 7 % by the tiles' fill alone;
@@ -767,9 +766,8 @@ extern "C" int ms_gemm_tiled(const void* A, long long lda, const void* W, long l
 //     else 0.88 to 2.0, 1.08 on average (8,192 columns 0.89 to 1.17);
 //   up to 1,000 tokens by 4,096 to 8,192 columns for up to 2,048 features, in three parts and more or, from 5,600 columns on, in two of
 //     the tiles of 128, 0.94 to 1.35, 1.08 on average (300 sizes with the norm; 896 x 4,864 by 640 and 768 tokens 24.3 -> 20.6 and 24.9 ->
-//     22.6 us).  Not: whole columns (0.81 to 0.83), two parts of fewer columns (0.95 to 1.06) or of tiles of 64 (0.95 to 1.02), rows that do not begin on four values (1,710 x 7,936
-//     at 711 tokens 0.93); 1,000 is where this was
-//     measured up to (1,001 to 1,100 tokens are 0.95 to 1.5, too);
+//     22.6 us).  Not: whole columns (0.81 to 0.83), two parts of fewer columns (0.95 to 1.06) or of tiles of 64 (0.95 to 1.02), rows that do not
+//     begin on four values (1,710 x 7,936 at 711 tokens 0.93); 1,000 is where this was measured up to (1,001 to 1,100 tokens are 0.95 to 1.5, too);
 //   in all 12 of 3,416 below 0.97;
 //   beyond, by 16,384 columns and more where one round of blocks in parts fills 5/6 of the CUs, but not all: 0.96 to 2.0, 1.4 on
 //     average (3,584 x 18,944 at 1,281 to 1,536 tokens and at 1,793 to 2,304).  With every CU taken 0.96 to 1.02 (4,096 x 28,672 at 2,048

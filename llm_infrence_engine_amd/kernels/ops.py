@@ -764,7 +764,7 @@ def gemm_slab_qkv(a: torch.Tensor, w_qkv: torch.Tensor, bias: Optional[torch.Ten
 
 def gemm_tiled_pays(a: torch.Tensor, w: torch.Tensor, epilogue: int = EPI_SWIGLU) -> bool:
     """Whether ``gemm_tiled(a, w, epilogue)`` takes these sizes and is the faster way to the gated product (one of the three
-    gates) or to the squared relu's."""
+    gates) or to the squared relu's, or holds in float what the library would round before the activation, as it always has there."""
     pays = _get("ms_gemm_tiled_relu2_pays" if epilogue == EPI_RELU2 else "ms_gemm_tiled_pays")
     return (a.dtype == torch.bfloat16 and w.dtype == torch.bfloat16 and a.dim() == 2 and a.is_contiguous()
             and w.is_contiguous() and a.data_ptr() % 16 == 0 and w.data_ptr() % 16 == 0
